@@ -29,6 +29,11 @@ int lk_silu_mul(bf16_t* out, const bf16_t* x, long rows, int I, long xs, long os
 int lk_activation(bf16_t* x, const bf16_t* bias, long rows, int N, long xs, int kind,
                   hipStream_t st);
 
+// rows_gemm.hip (M <= 64, one launch, every epilogue)
+bool lk_rows_gemm_supported(int M, int N, int K, int epi);
+int lk_rows_gemm(const void* x, const void* w, const void* b, void* y, int M, int N, int K, long ldx, long ldy, int epi,
+                 hipStream_t st);
+
 // skinny_gemm.hip (decode-regime linear, optional fused SwiGLU)
 int lk_skinny_splits(int M, int N, int K, int swiglu);
 int lk_skinny_gemm(const bf16_t* x, long ldx, const bf16_t* w, int M, int N, int K, int S, int swiglu,

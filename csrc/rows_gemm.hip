@@ -1,0 +1,192 @@
+// K2 / K3, few rows: Y[M,N] = act(X[M,K] . W[N,K]^T + bias) for M <= 64 rows in ONE launch, bf16 in, f32
+// sums, one rounding (bias / bias + GELU / bias + ReLU / SwiGLU in the epilogue).
+//
+// What bounds it: at these sizes neither HBM (a 2048 x 2048 weight is 1.4 us of it) nor the matrix cores
+// but the serial chain of a launch: a tiled kernel with a barrier per K stage waits for each of them, and
+// a split-K one pays a second launch for its sum.  Here no wave waits for another inside the K walk:
+//   * a workgroup of 4 waves owns 16 output columns (SwiGLU: 16 gate and the 16 up columns) and all rows;
+//     the waves split K, so each element of X and W reaches the workgroup once;
+//   * every wave streams its own K range through a private LDS ring by 16-byte LDS-DMA (8 rows x one whole
+//     128-byte line per instruction; loads straight into the fragment layout, 16 rows x 64 bytes, ran at a
+//     quarter of the rate: 12.0 us against 7.7 at 64 x 2048 x 2048, 8.4 against 5.7 at 32 rows), counted vmcnt, no barrier; the
+//     chunk order in a row is XORed with the row so that the fragment reads meet no bank twice;
+//   * the waves' sums meet once in LDS, then the epilogue stores 4 columns per lane;
+//   * 16 columns per workgroup give N / 16 workgroups, which is what fills 256 CUs at N 2048-4096.  X is
+//     re-read by each of them out of L2: what bounds the large end, and why more than 64 rows and long K
+//     stay on the kernels with wider column tiles.
+#include "common.h"
+#include "kernels.h"
+
+namespace {
+
+constexpr int kRgWaves = 4;
+
+enum { RG_NONE = 0, RG_SWIGLU = 1, RG_BIAS = 2, RG_GELU = 3, RG_RELU = 4 };
+
+typedef __attribute__((address_space(3))) void* rg_lptr;
+typedef const __attribute__((address_space(1))) void* rg_gptr;
+
+template <int N>
+LK_DEVICE void rg_wait() {
+  static_assert(N >= 0 && N < 64, "vmcnt range");
+  __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
+}
+template <int L, int AHEAD>
+LK_DEVICE void rg_wait_ahead(int ahead) {  // all but the newest `ahead` stages of L loads have landed
+  if constexpr (AHEAD > 0) {
+    if (ahead >= AHEAD) {
+      rg_wait<L * AHEAD>();
+      return;
+    }
+    rg_wait_ahead<L, AHEAD - 1>(ahead);
+  } else {
+    rg_wait<0>();
+  }
+}
+
+// 64 K columns of (MT + NT) 16-row tiles: one stage of a wave's ring
+constexpr int rg_stage(int MT, int NT) { return (MT + NT) * 2048; }
+constexpr int rg_lds(int MT, int NT, int NS) {
+  const int ring = kRgWaves * NS * rg_stage(MT, NT), sums = kRgWaves * MT * NT * 1024;
+  return ring > sums ? ring : sums;
+}
+
+template <int MT, int NT, int NS, int EPI>
+__global__ __launch_bounds__(64 * kRgWaves, 1) void rows_gemm_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
+                                                                     const bf16_t* __restrict__ bias, bf16_t* __restrict__ Y, int M,
+                                                                     int N, int K, long ldx, long ldy) {
+  constexpr int SB = rg_stage(MT, NT), L = (MT + NT) * 2;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, g = lane >> 4;
+  const int all = K / 64, first = wave * all / kRgWaves, nst = (wave + 1) * all / kRgWaves - first;  // stages of this wave
+  const long k0 = (long)first * 64;
+  const int n0 = blockIdx.x * 16;  // first output column
+  unsigned char* const ring = smem + wave * NS * SB;
+
+  // LDS row `row` holds the eight 16-byte chunks of its 128 bytes in the order chunk ^ (row & 7)
+  const int lrow = lane >> 3, lcol = ((lane & 7) ^ lrow) * 8;
+  const bf16_t* xs[2 * MT];
+  const bf16_t* ws[2 * NT];
+#pragma unroll
+  for (int i = 0; i < 2 * MT; ++i) xs[i] = X + (long)min(8 * i + lrow, M - 1) * ldx + k0 + lcol;  // rows past M repeat the last one
+#pragma unroll
+  for (int i = 0; i < 2 * NT; ++i) ws[i] = W + ((long)(i >> 1) * (N >> 1) + n0 + 8 * (i & 1) + lrow) * K + k0 + lcol;
+
+  auto issue = [&](int st) {
+    unsigned char* base = ring + (st % NS) * SB;
+#pragma unroll
+    for (int i = 0; i < 2 * NT; ++i)
+      __builtin_amdgcn_global_load_lds((rg_gptr)(ws[i] + st * 64), (rg_lptr)(base + (2 * MT + i) * 1024), 16, 0, 2);
+#pragma unroll
+    for (int i = 0; i < 2 * MT; ++i)
+      __builtin_amdgcn_global_load_lds((rg_gptr)(xs[i] + st * 64), (rg_lptr)(base + i * 1024), 16, 0, 0);
+  };
+
+  floatx4 acc[MT][NT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int n = 0; n < NT; ++n) acc[m][n] = (floatx4){0.f, 0.f, 0.f, 0.f};
+
+#pragma unroll
+  for (int p = 0; p < NS - 1; ++p)
+    if (p < nst) issue(p);
+  for (int st = 0; st < nst; ++st) {
+    rg_wait_ahead<L, NS - 2>(min(NS - 2, nst - 1 - st));
+    __builtin_amdgcn_sched_barrier(0);
+    if (st + NS - 1 < nst) issue(st + NS - 1);  // into the slot whose fragments the last stage's products have consumed
+    __builtin_amdgcn_sched_barrier(0);
+    const unsigned char* base = ring + (st % NS) * SB;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int at = r16 * 128 + (((4 * h + g) ^ (r16 & 7)) << 4);
+      short8 a[MT], b[NT];
+#pragma unroll
+      for (int n = 0; n < NT; ++n) b[n] = *reinterpret_cast<const short8*>(base + (MT + n) * 2048 + at);
+#pragma unroll
+      for (int m = 0; m < MT; ++m) a[m] = *reinterpret_cast<const short8*>(base + m * 2048 + at);
+      // W as the A operand: the lane ends with one output row and 4 consecutive columns
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[n], a[m], acc[m][n], 0, 0, 0);
+    }
+  }
+
+  // lane l: row l & 15 of tile m, columns 4 (l >> 4) ..; partials as [wave][tile][lane] float4
+  __syncthreads();  // every wave's ring is read
+  floatx4* part = reinterpret_cast<floatx4*>(smem);
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int n = 0; n < NT; ++n) part[(wave * MT * NT + m * NT + n) * 64 + lane] = acc[m][n];
+  __syncthreads();
+#pragma unroll
+  for (int m = wave; m < MT; m += kRgWaves) {  // one row tile per wave
+    floatx4 t[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      t[n] = part[(m * NT + n) * 64 + lane];
+#pragma unroll
+      for (int w = 1; w < kRgWaves; ++w) t[n] += part[((w * MT + m) * NT + n) * 64 + lane];
+    }
+    const int row = m * 16 + r16;
+    if (row >= M) continue;
+    float y[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if constexpr (EPI == RG_SWIGLU) {  // rounded as the projection and the activation apart round
+        y[j] = bf2f(f2bf(lk_silu(bf2f(f2bf(t[0][j]))))) * bf2f(f2bf(t[NT - 1][j]));
+      } else {
+        y[j] = t[0][j];
+        if constexpr (EPI >= RG_BIAS) y[j] += bf2f(bias[n0 + 4 * g + j]);
+        if constexpr (EPI == RG_GELU) y[j] = lk_gelu_erf(y[j]);
+        if constexpr (EPI == RG_RELU) y[j] = fmaxf(y[j], 0.f);
+      }
+    }
+    uint2 pk;
+    pk.x = pack_bf2(y[0], y[1]);
+    pk.y = pack_bf2(y[2], y[3]);
+    *reinterpret_cast<uint2*>(Y + (long)row * ldy + n0 + 4 * g) = pk;
+  }
+}
+
+template <int MT, int NT, int NS, int EPI>
+int launch(const void* x, const void* w, const void* b, void* y, int M, int N, int K, long ldx, long ldy, hipStream_t st) {
+  constexpr int lds = rg_lds(MT, NT, NS);
+  LK_SET_MAX_LDS((rows_gemm_kernel<MT, NT, NS, EPI>), lds);
+  rows_gemm_kernel<MT, NT, NS, EPI><<<N / (16 * NT), 64 * kRgWaves, lds, st>>>((const bf16_t*)x, (const bf16_t*)w, (const bf16_t*)b,
+                                                                              (bf16_t*)y, M, N, K, ldx, ldy);
+  LK_CHECK_LAUNCH();
+  return 0;
+}
+
+template <int EPI>
+int by_rows(const void* x, const void* w, const void* b, void* y, int M, int N, int K, long ldx, long ldy, hipStream_t st) {
+  constexpr int NT = EPI == RG_SWIGLU ? 2 : 1;
+  if (M <= 16) return launch<1, NT, NT == 1 ? 5 : 4, EPI>(x, w, b, y, M, N, K, ldx, ldy, st);
+  if (M <= 32) return launch<2, NT, 4, EPI>(x, w, b, y, M, N, K, ldx, ldy, st);
+  if (M <= 48) return launch<3, NT, 4, EPI>(x, w, b, y, M, N, K, ldx, ldy, st);
+  return launch<4, NT, NT == 1 ? 4 : 3, EPI>(x, w, b, y, M, N, K, ldx, ldy, st);
+}
+
+}  // namespace
+
+// (the epilogue stores 8-byte groups of 4 columns: ldy is a multiple of 4, y 8-byte aligned)
+bool lk_rows_gemm_supported(int M, int N, int K, int epi) {
+  return M >= 1 && M <= 64 && K >= 64 && K % 64 == 0 && N >= 16 && N % (epi == RG_SWIGLU ? 32 : 16) == 0;
+}
+
+int lk_rows_gemm(const void* x, const void* w, const void* b, void* y, int M, int N, int K, long ldx, long ldy, int epi,
+                 hipStream_t st) {
+  if (!lk_rows_gemm_supported(M, N, K, epi) || ldy % 4) return -1;
+  switch (epi) {
+    case RG_NONE: return by_rows<RG_NONE>(x, w, b, y, M, N, K, ldx, ldy, st);
+    case RG_SWIGLU: return by_rows<RG_SWIGLU>(x, w, b, y, M, N, K, ldx, ldy, st);
+    case RG_BIAS: return by_rows<RG_BIAS>(x, w, b, y, M, N, K, ldx, ldy, st);
+    case RG_GELU: return by_rows<RG_GELU>(x, w, b, y, M, N, K, ldx, ldy, st);
+    case RG_RELU: return by_rows<RG_RELU>(x, w, b, y, M, N, K, ldx, ldy, st);
+    default: return -1;
+  }
+}

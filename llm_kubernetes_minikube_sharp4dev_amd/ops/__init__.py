@@ -375,12 +375,48 @@ def _decode_bucket(M: int) -> Optional[int]:
     return None
 
 
+# Few rows (csrc/rows_gemm.hip, M <= 64, one launch with any epilogue) or the kernels with wider column
+# tiles.  A workgroup of the few-row kernel reads 16 columns of W (SwiGLU 2 x 16) and ALL of X, so its time
+# is 2.6 us + (bytes per workgroup x rounds of 256 workgroups) / 58 KB/us (a further 1.3 when there is more
+# than one round); the weight-streaming kernel takes ~9.5 us for its two launches + 0.14 us per MB of W + M / 32.
+# Equating the two gives the line below.  Measured in hipGraphs, weights cold, few-row / streaming (us):
+#   64 x 2048 x 2048  7.7 / 10.9    32 x 2048 x 5632 11.9 / 13.2    16 x 10368 x 2048 10.9 / 14.1
+#   64 x 3072 x 2048  8.0 / 11.3    64 x 2048 x 5632 17.0 / 14.3    48 x 10368 x 2048 18.5 / 16.0
+#   64 x 4096 x 4096 14.1 / 14.0    32 x 6144 x 4096 17.5 / 16.5    32 x 4096 x 14336 34.0 / 28.6
+# (past K 8192 more than 16 rows of X no longer stay in L2, and a weight past 100 MB is bound by HBM either
+# way.)  SwiGLU costs the streaming side another 3.5 us in its second launch (64 x 11264 x 2048: 18.2 / 19.5);
+# with a bias or an activation the other side is the prefill GEMM, 15-19 us at K 768-3072.
+ROWS_MAX_M = 64
+_ROWS_RULE: dict = {}
+
+
+def _rows_rule(M: int, N: int, K: int, epi: int) -> bool:
+    key = ((M + 15) // 16, N, K, epi)
+    ok = _ROWS_RULE.get(key)
+    if ok is None:
+        mt, nt = key[0], 2 if epi == 1 else 1
+        rounds = -(-N // (16 * nt * 256))
+        q = rounds * (mt + nt) * K / 32 * (1.3 if rounds > 1 else 1.0)     # KB
+        mb = N * K * 2 / 1e6
+        ok = (1 <= M <= ROWS_MAX_M and (K <= 8192 or mt == 1) and q <= (600 if epi == 1 else 400) + 8 * min(mb, 100) + 29 * mt
+              and lib().rows_supported(M, N, K, epi))
+        _ROWS_RULE[key] = ok
+    return ok
+
+
+def _rows_ok(x, w, epi: int) -> bool:
+    return (x.dim() == 2 and w.dim() == 2 and 1 <= x.shape[0] <= ROWS_MAX_M and _gemm_ok(x, w) and w.data_ptr() % 16 == 0
+            and _rows_rule(x.shape[0], w.shape[0], w.shape[1], epi))
+
+
 def _decode_gemm_kind(x, w, swiglu: bool) -> Optional[str]:
     if not (use_hip(x) and x.dim() == 2 and w.dim() == 2 and x.dtype == torch.bfloat16
             and w.dtype == torch.bfloat16):
         return None
     M = x.shape[0]
     N, K = w.shape
+    if M > SKINNY_MAX_M and _rows_ok(x, w, 1 if swiglu else 0):
+        return "rows"
     if M < 1 or K % 256 or x.stride(1) != 1 or x.stride(0) % 8 or not w.is_contiguous():
         return None
     if swiglu:
@@ -701,7 +737,7 @@ def apply_ws_variants(table: dict):
             L.ws_set_variant(M, N, K, sw, v)
 
 
-def tune_decode(weights, ms: Sequence[int] = DECODE_TUNE_MS, iters: int = 5, cold_bytes: int = 640 << 20) -> dict:
+def tune_decode(weights, ms: Sequence[int] = DECODE_TUNE_MS, iters: int = 3, cold_bytes: int = 640 << 20) -> dict:
     """For each decode-sized M bucket and each (weight, swiglu) pair, time the weight-streaming
     kernel against the prefill GEMM with the weights arriving from HBM (each launch reads the
     next of enough copies to overflow the 256 MB MALL, back-to-back launches as in a decode
@@ -711,22 +747,35 @@ def tune_decode(weights, ms: Sequence[int] = DECODE_TUNE_MS, iters: int = 5, col
 
     L = lib()
     out = {}
+    side = torch.cuda.Stream() if len(weights) else None
     for w, swiglu in weights:
         N, K = w.shape
         swiglu = bool(swiglu)
         copies = [w] + [w.clone() for _ in range(max(1, -(-cold_bytes // (N * K * 2)) - 1))]
 
         def timed(fns):
-            ts = {k: [] for k in fns}
+            # as decode steps run: launches of a hipGraph (eager ones of a few microseconds are bound by the
+            # host, which favoured the arm with fewer launches: 64 x 2048 x 2048 went to the prefill GEMM,
+            # 18.5 us against 10.9 in a graph, and SwiGLU 64 x 11264 x 2048 at random, 32.5 against 19.5)
+            ts, graphs = {k: [] for k in fns}, {}
             for fn in fns.values():  # warm-up (and first-launch attributes)
                 fn(copies[0])
             torch.cuda.synchronize()
-            for _ in range(iters):
+            # (inference mode, as the engine's own captures: the generator's graph state may be an inference tensor by now)
+            with torch.inference_mode(), torch.cuda.stream(side):
                 for k, fn in fns.items():
+                    graphs[k] = torch.cuda.CUDAGraph()
+                    graphs[k].capture_begin(capture_error_mode="thread_local")
+                    try:
+                        for c in copies[1:] + copies[:1]:
+                            fn(c)
+                    finally:
+                        graphs[k].capture_end()
+            for _ in range(iters):
+                for k, g in graphs.items():
                     a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
                     a.record()
-                    for c in copies[1:] + copies[:1]:
-                        fn(c)
+                    g.replay()
                     b.record()
                     b.synchronize()
                     ts[k].append(a.elapsed_time(b) * 1e3 / len(copies))
@@ -736,7 +785,7 @@ def tune_decode(weights, ms: Sequence[int] = DECODE_TUNE_MS, iters: int = 5, col
         # ring vs loader waves (csrc/skinny_gemm.hip wsgemm_lw_kernel), measured at the tile's
         # largest M, before the routing below times the ws arm with it
         if WS_VARIANT_TUNE and _decode_static_ok(N, K, swiglu):
-            for M in [m for m in (64, 128, 192, 256) if m in ms]:
+            for M in [m for m in (64, 128, 192, 256) if m in ms and not _rows_rule(m, N, K, int(swiglu))]:
                 x = torch.randn(M, K, device=w.device, dtype=torch.bfloat16)
                 fns = {}
                 for v in (0, 1):
@@ -747,6 +796,8 @@ def tune_decode(weights, ms: Sequence[int] = DECODE_TUNE_MS, iters: int = 5, col
                 _WS_VARIANTS[(M, N, K, swiglu)] = best
                 out[(M, N, K, swiglu, "ws_variant")] = {("ring", "loader")[v]: round(t, 1) for v, t in med.items()}
         for M in ms:
+            if _rows_rule(M, N, K, int(swiglu)):  # routed by the rule, not by this table
+                continue
             x = torch.randn(M, K, device=w.device, dtype=torch.bfloat16)
             arms = {}
             if M <= 256 and _decode_static_ok(N, K, swiglu):
@@ -771,9 +822,9 @@ def _decode_static_ok(N: int, K: int, swiglu: bool) -> bool:
 
 
 def linear(x, w, b=None, act: Optional[str] = None):
-    """Projection GEMM (+ bias, + GELU / ReLU): decode-sized batches without an epilogue on
-    the weight-streaming MFMA kernels (skinny / ws), everything else on the prefill kernel
-    with the epilogue fused."""
+    """Projection GEMM (+ bias, + GELU / ReLU): few rows on the one-launch kernel with any epilogue,
+    decode-sized batches without an epilogue on the weight-streaming MFMA kernels (skinny / ws),
+    everything else on the prefill kernel with the epilogue fused."""
     if not use_hip(x):
         y = torch.nn.functional.linear(x, w, b)
         if act is not None:
@@ -783,6 +834,8 @@ def linear(x, w, b=None, act: Optional[str] = None):
         if _gemv_ok(x, w, 0):
             return lib().gemv_decode(0, x, w)
         kind = _decode_gemm_kind(x, w, False)
+        if kind == "rows":
+            return lib().rows_linear(x, w)
         if kind == "skinny":
             return lib().skinny_linear(x, w)
         if kind == "ws":
@@ -792,6 +845,8 @@ def linear(x, w, b=None, act: Optional[str] = None):
         b = torch.zeros(w.shape[0], device=x.device, dtype=x.dtype)
         epi = EPI[act]
     lib_arm = GEMM_LIBRARY == 1 or (GEMM_LIBRARY == 2 and epi == 0 and x.shape[0] > WS_MAX_M)
+    if epi >= 2 and not lib_arm and b.dtype == torch.bfloat16 and b.is_contiguous() and b.numel() == w.shape[0] and _rows_ok(x, w, epi):
+        return lib().rows_linear(x, w, b, epi)
     y = gemm(x, w, b, epi) if _gemm_ok(x, w) and not lib_arm else None
     if y is None:
         y = _library(x, w, b, act, (x.shape[0] > WS_MAX_M, w.shape[0], w.shape[1], epi))
@@ -806,6 +861,8 @@ def linear_swiglu(x, w_gate_up):
     if _gemv_ok(x, w_gate_up, 2):
         return lib().gemv_decode(2, x, w_gate_up)
     kind = _decode_gemm_kind(x, w_gate_up, True)
+    if kind == "rows":
+        return lib().rows_linear(x, w_gate_up, None, 1)
     if kind == "skinny":
         return lib().skinny_linear(x, w_gate_up, True)
     if kind == "ws":
