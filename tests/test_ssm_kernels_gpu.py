@@ -1,0 +1,62 @@
+"""State-space kernels (csrc/ssm.hip) against a float64 recurrence: single-token steps, token runs and chunks at the
+edges of the 64-token tiles, state sizes that fill their lanes and not, padding slots, first and later portions, and
+shapes that only the general kernels take."""
+import pytest
+import torch
+
+from llm_kubernetes_minikube_sharp4dev_amd import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _run(lens, H, P, N, G, dtype, max_len, later):
+    g = torch.Generator(device=DEV).manual_seed(H * P + N)
+    rn = lambda *s: torch.randn(*s, device=DEV, generator=g)  # noqa: E731
+    T, S, C = sum(lens), len(lens), H * P + 2 * G * N
+    xbc = rn(T, -(-C // 8) * 8 + 8).to(dtype)[:, :C]
+    d = rn(T, H + 3).to(dtype)[:, :H]
+    state, b, A, D = rn(S + 1, H, P, N), rn(H) * 0.5 - 1, rn(H) * 0.3, rn(H)
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32, device=DEV)
+    slots = torch.arange(S, 0, -1, device=DEV).to(torch.int32)
+    slots[1] = -1
+    pos = torch.cat([torch.arange(n) + later * (i % 2 == 0) for i, n in enumerate(lens)]).to(torch.int32).to(DEV)
+    want = state.double()
+    y = ops.ssm_scan(xbc, d, H, P, N, G, b, A, D, state, cu, slots, pos, max_len=max_len)
+    ref, X = torch.zeros(T, H * P, dtype=torch.float64, device=DEV), xbc.double()
+    for s in range(S):
+        sl = int(slots[s])
+        if sl < 0:
+            continue
+        r0, r1 = int(cu[s]), int(cu[s + 1])
+        st = want[sl].clone() if int(pos[r0]) > 0 else torch.zeros_like(want[sl])
+        for t in range(r0, r1):
+            x = X[t, :H * P].view(H, P)
+            B, Cc = (X[t, H * P + i * G * N:H * P + (i + 1) * G * N].view(G, N).repeat_interleave(H // G, 0) for i in (0, 1))
+            dt = torch.nn.functional.softplus(d[t].double() + b.double(), threshold=30.0)
+            st = torch.exp(-torch.exp(A.double()) * dt)[:, None, None] * st + (dt[:, None] * x)[:, :, None] * B[:, None, :]
+            ref[t] = ((st * Cc[:, None, :]).sum(-1) + D.double()[:, None] * x).reshape(-1)
+        want[sl] = st
+    return y, ref, state, want
+
+
+@pytest.mark.parametrize("H,P,N,G", [(4, 64, 128, 2), (6, 20, 16, 3), (2, 33, 24, 1), (4, 16, 64, 4), (2, 72, 256, 1), (2, 16, 200, 2),
+                                     (3, 8, 30, 1)])
+@pytest.mark.parametrize("lens,max_len", [([1, 1, 1, 1, 1], 1), ([3, 2, 1], 1), ([130, 9, 64, 65, 63, 1], 130)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_scan(hip, H, P, N, G, lens, max_len, dtype):
+    y, ref, state, want = _run(lens, H, P, N, G, dtype, max_len, 5)
+    # f32 arithmetic on the same inputs: sums of N terms and decays multiplied along a sequence, a few 2^-24 each
+    assert (y.double() - ref).norm() <= 1e-6 * ref.norm()
+    assert (state.double() - want).norm() <= 1e-6 * want.norm()
+
+
+@pytest.mark.parametrize("rows,inner,ng", [(1, 4096, 8), (77, 1536, 1), (5, 120, 3), (9, 2048, 1), (3, 2304, 1), (6, 44, 2)])
+def test_gated_group_norm(hip, rows, inner, ng):
+    torch.manual_seed(inner)
+    y, w = torch.randn(rows, inner, device=DEV), torch.randn(inner, device=DEV)
+    z = torch.randn(rows, inner + 8, device=DEV).to(torch.bfloat16)[:, :inner]
+    v = (y.double() * torch.nn.functional.silu(z.double())).view(rows, ng, -1)
+    r = (v / (v.pow(2).mean(-1, keepdim=True) + 1e-5).sqrt()).reshape(rows, inner) * w.double()
+    o = ops.gated_group_rmsnorm(y, z, w, ng, 1e-5).double()
+    assert ((o - r).abs() <= 2.0 ** -8 * r.abs() + 1e-6).all()   # one bf16 rounding of an f32 value
