@@ -14,6 +14,7 @@
 // rms(v) = v / sqrt(mean(v^2) + eps).
 #include "common.h"
 #include "kernels.h"
+#include "kv_rows.h"
 
 namespace {
 
@@ -247,6 +248,88 @@ __global__ __launch_bounds__(256) void rot_kv_write_kernel(RotParams p) {
   }
 }
 
+// The same for bf16 rows whose head sizes and strides are whole 16-byte pieces: R rows and a part of their heads per
+// workgroup (kv_rows.h).  grid (rows / R, q / k parts + value parts).  4,096 rows of 16 query and 16 key heads of 192 with
+// 16 x 128 values: 77 us with one workgroup per row (2-byte accesses, values in 64 sectors per store) -> 35 us; 64
+// decode rows 20 -> 6.4 us.
+template <int R, int LPH>
+__global__ __launch_bounds__(256) void rot_file_kernel(RotParams p, long rows, int qk_parts) {
+  using KT = KvTile<R, LPH>;
+  constexpr int SV = R == 1 ? 1 : R;
+  __shared__ float2 sct[R][kRotMaxHead / 2];
+  __shared__ __attribute__((aligned(16))) bf16_t sv[SV][KT::VCOLS + 2];
+  const long t0 = (long)blockIdx.x * R;
+  const int tl = (int)min((long)R, rows - t0), part = blockIdx.y;
+  if (part >= qk_parts) {
+    const int n = p.G * p.VD, c0 = (part - qk_parts) * KT::VCOLS;
+    kv_file_values<R, KT::VCOLS>(p.slots, t0, tl, c0, min(n, c0 + KT::VCOLS), p.G, p.VD, p.BS, reinterpret_cast<bf16_t*>(p.vc), sv,
+                                 [&](long t, int gh, int d, float (&f)[8]) {
+      if (d >= p.vdim) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] = 0.f;
+        return;
+      }
+      load8(reinterpret_cast<const bf16_t*>(p.v) + t * p.vs + (long)gh * p.vdim + d, f);
+      if (p.v2) {
+        float f2[8];
+        load8(reinterpret_cast<const bf16_t*>(p.v2) + t * p.v2s + (long)gh * p.vdim + d, f2);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] = (1.f - p.blend) * f[e] + p.blend * f2[e];
+      }
+    });
+    return;
+  }
+  const int np = p.rot / 2;
+  for (int i = threadIdx.x; i < tl * np; i += 256) {
+    const int r = i / np, k = i % np;
+    float sn, cs;
+    sincosf((float)p.positions[t0 + r] * p.freq[k], &sn, &cs);
+    sct[r][k] = make_float2(cs * p.mag, sn * p.mag);
+  }
+  __syncthreads();
+  const int h0 = part * KT::HEADS, nh = min(KT::HEADS, p.H + p.G - h0);
+  const int c = (threadIdx.x % LPH) * 8;
+  for (int i = threadIdx.x / LPH; i < tl * nh; i += 256 / LPH) {
+    const int r = i / nh, job = h0 + i % nh;
+    const long t = t0 + r;
+    const bool isq = job < p.H;
+    const int kh = job - p.H, hd = isq ? p.qdim : p.KD, slot = isq ? 0 : p.slots[t];
+    if (c >= hd || slot < 0) continue;
+    bf16_t* dst;
+    float f[8];
+    if (isq) {
+      dst = reinterpret_cast<bf16_t*>(p.q) + t * p.qs + (long)job * p.qdim + c;
+      load8(dst, f);
+    } else {
+      dst = reinterpret_cast<bf16_t*>(p.kc) + (((long)(slot / p.BS) * p.G + kh) * p.BS + slot % p.BS) * p.KD + c;
+      if (c < p.kdim) load8(reinterpret_cast<const bf16_t*>(p.k) + t * p.ks + (long)kh * p.kdim + c, f);
+      else if (c < p.kdim + p.sdim) load8(reinterpret_cast<const bf16_t*>(p.sh) + t * p.shs + (c - p.kdim), f);
+      else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] = 0.f;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+      const int k = c + e - p.rot_off;
+      if (k >= 0 && k < p.rot) {
+        const float2 cs = sct[r][k >> 1];
+        const float a = f[e], b = f[e + 1];
+        f[e] = a * cs.x - b * cs.y;
+        f[e + 1] = b * cs.x + a * cs.y;
+      }
+    }
+    store8(dst, f);
+  }
+}
+
+template <int R, int LPH>
+void launch_rot_file(const RotParams& p, long T, hipStream_t st) {
+  using KT = KvTile<R, LPH>;
+  const int qk = (p.H + p.G + KT::HEADS - 1) / KT::HEADS, vp = (p.G * p.VD + KT::VCOLS - 1) / KT::VCOLS;
+  rot_file_kernel<R, LPH><<<dim3((unsigned)((T + R - 1) / R), qk + vp), 256, 0, st>>>(p, T, qk);
+}
+
 // grid (blocks a sequence may complete in this step, G, sequences).  Sequence s holds ctx cached tokens, the last
 // qlen of them new: the blocks past / P .. ctx / P - 1 end on a new position.
 template <typename T>
@@ -339,7 +422,16 @@ int lk_rot_kv_write(void* q, long qs, int H, int qdim, const void* k, long ks, i
   p.sdim = sdim; p.v = v; p.vs = vs; p.vdim = vdim; p.rot_off = rot_off; p.rot = rot; p.freq = freq; p.mag = mag;
   p.positions = positions; p.kc = kc; p.vc = vc; p.slots = slots; p.BS = BS; p.KD = KD; p.VD = VD;
   p.v2 = v2; p.v2s = v2s; p.blend = blend;
-  if (esz == 2) rot_kv_write_kernel<bf16_t><<<(unsigned)T, 256, 0, st>>>(p);
+  const auto rows16 = [](const void* x, long stride) { return !x || ((reinterpret_cast<uintptr_t>(x) & 15) == 0 && stride % 8 == 0); };
+  if (esz == 2 && qdim % 8 == 0 && kdim % 8 == 0 && sdim % 8 == 0 && vdim % 8 == 0 && KD % 8 == 0 && VD % 8 == 0 && rot_off % 2 == 0 &&
+      rows16(q, qs) && rows16(kdim > 0 ? k : nullptr, ks) && rows16(p.sh, shs) && rows16(v, vs) && rows16(v2, v2s) && rows16(kc, 0) &&
+      (H + G) <= 32768 && (long)G * VD <= 1 << 24) {
+    const int lph = kv_lanes(qdim > KD ? qdim : KD);
+    const bool few = T < kFileFewRows;
+    if (lph == 8) few ? launch_rot_file<1, 8>(p, T, st) : launch_rot_file<kFileRows, 8>(p, T, st);
+    else if (lph == 16) few ? launch_rot_file<1, 16>(p, T, st) : launch_rot_file<kFileRows, 16>(p, T, st);
+    else few ? launch_rot_file<1, 32>(p, T, st) : launch_rot_file<kFileRows, 32>(p, T, st);
+  } else if (esz == 2) rot_kv_write_kernel<bf16_t><<<(unsigned)T, 256, 0, st>>>(p);
   else rot_kv_write_kernel<float><<<(unsigned)T, 256, 0, st>>>(p);
   LK_CHECK_LAUNCH();
   return 0;
