@@ -18,6 +18,7 @@
 #include "common.h"
 #include "kernels.h"
 #include "attn_frag.h"
+#include "row_ring.h"
 
 namespace {
 
@@ -315,6 +316,67 @@ int launch_moe(const void* x, long xs, const int* order, const int* seg, int E, 
   return 0;
 }
 
+// The same product for decode-sized steps of bf16 rows: a stream of the experts' weights, each read once.  One workgroup
+// takes 16 columns (act: 16 gate and their up columns; else 2 x 16) of ONE expert and all of its pairs, MT x 16 at a
+// time (more than that is a second walk over the same weight rows, out of L2); the four waves split K through private
+// LDS rings (row_ring.h), so up to 64 KB of weight rows are on their way per CU and no wave waits for another inside the walk.
+// 64 tokens x 2 of 16 experts of 2048 x 2816: gate / up 110 us (3.4 TB/s) -> 56 us (6.6 TB/s), down 67 us (2.7 TB/s) -> 30 us.
+template <bool ACT, int MT>
+__global__ __launch_bounds__(256) void moe_rows_kernel(const bf16_t* __restrict__ x, long xs, const int* __restrict__ order,
+                                                       const int* __restrict__ seg, int top, const bf16_t* __restrict__ w, int N, int K,
+                                                       bf16_t* __restrict__ out, long os, int blocks) {
+  constexpr int NT = 2, NS = 3;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int e = blockIdx.x / blocks, cb = blockIdx.x % blocks;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int end = seg[e + 1], F = ACT ? N / 2 : N, c0 = cb * (ACT ? 16 : 32);
+  const int all = K / 64, first = wave * all / kRgWaves, nst = (wave + 1) * all / kRgWaves - first;
+  const int lrow = lane >> 3;
+  const long k = (long)first * 64 + rg_lane_col(lane);
+  const bf16_t* ws[2 * NT];
+#pragma unroll
+  for (int i = 0; i < 2 * NT; ++i)
+    ws[i] = w + ((long)e * N + (ACT ? (long)(i >> 1) * F : (i >> 1) * 16) + c0 + 8 * (i & 1) + lrow) * K + k;
+  for (int place0 = seg[e]; place0 < end; place0 += 16 * MT) {
+    const bf16_t* xp[2 * MT];
+#pragma unroll
+    for (int i = 0; i < 2 * MT; ++i) {
+      const int place = min(place0 + 8 * i + lrow, end - 1);  // rows past the expert's last pair repeat it
+      xp[i] = x + (long)(ACT ? order[place] / top : place) * xs + k;
+    }
+    floatx4 acc[MT][NT];
+    rg_walk<MT, NT, NS>(xp, ws, nst, smem + wave * NS * rg_stage(MT, NT), acc);
+    rg_sums<MT, NT>(smem, acc, [&](int m, const floatx4 (&t)[NT]) {
+      const int place = place0 + m * 16 + (lane & 15), col = c0 + 4 * (lane >> 4);
+      if (place >= end) return;
+      bf16_t* dst = out + (long)(ACT ? place : order[place]) * os + col;
+#pragma unroll
+      for (int n = 0; n < (ACT ? 1 : NT); ++n) {
+        float y[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) y[j] = ACT ? t[0][j] * __builtin_amdgcn_rcpf(1.f + __expf(-t[0][j])) * t[1][j] : t[n][j];
+        uint2 pk;
+        pk.x = pack_bf2(y[0], y[1]);
+        pk.y = pack_bf2(y[2], y[3]);
+        *reinterpret_cast<uint2*>(dst + 16 * n) = pk;
+      }
+    });
+    __syncthreads();  // the sums are read: the rings are free again
+  }
+}
+
+template <bool ACT, int MT>
+int launch_moe_rows(const void* x, long xs, const int* order, const int* seg, int E, int top, const void* w, int N, int K, void* out,
+                    long os, hipStream_t st) {
+  const int blocks = N / 32;  // 16 output columns of two weight rows each, or 32
+  constexpr int lds = rg_lds(MT, 2, 3);
+  LK_SET_MAX_LDS((moe_rows_kernel<ACT, MT>), lds);
+  moe_rows_kernel<ACT, MT><<<(unsigned)((long)E * blocks), 256, lds, st>>>((const bf16_t*)x, xs, order, seg, top, (const bf16_t*)w, N, K,
+                                                                          (bf16_t*)out, os, blocks);
+  LK_CHECK_LAUNCH();
+  return 0;
+}
+
 template <typename T>
 int moe_gemm_t(const void* x, long xs, const int* order, const int* seg, int E, int top, long pairs, const void* w, int N, int K,
                int act, void* out, long os, int vec, hipStream_t st) {
@@ -323,6 +385,18 @@ int moe_gemm_t(const void* x, long xs, const int* order, const int* seg, int E, 
   if (wide && vec) {   // 128-pair tiles staged in LDS (256-pair tiles, RT = 8, measured slower: 575 us against 365 us)
     return act ? launch_moe_lds<T, true, 4>(x, xs, order, seg, E, top, pairs, w, N, K, out, os, st)
                : launch_moe_lds<T, false, 4>(x, xs, order, seg, E, top, pairs, w, N, K, out, os, st);
+  }
+  if constexpr (sizeof(T) == 2) {
+    // whole 64-column stages and 16-column blocks, 8-byte stores; rows per walk by the pairs an expert has on average (a third
+    // more than the mean keeps a second walk rare)
+    if (vec && K % 64 == 0 && N % 32 == 0 && os % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0 && (long)E * (N / 32) <= 2147483647L) {
+      const long avg = pairs / E;
+#define LK_MOE_ROWS(MT)                                                                           \
+  (act ? launch_moe_rows<true, MT>(x, xs, order, seg, E, top, w, N, K, out, os, st)               \
+       : launch_moe_rows<false, MT>(x, xs, order, seg, E, top, w, N, K, out, os, st))
+      return avg <= 10 ? LK_MOE_ROWS(1) : avg <= 22 ? LK_MOE_ROWS(2) : LK_MOE_ROWS(4);
+#undef LK_MOE_ROWS
+    }
   }
   if (act) return wide ? launch_moe<T, true, 4>(x, xs, order, seg, E, top, pairs, w, N, K, out, os, vec, st)
                        : launch_moe<T, true, 1>(x, xs, order, seg, E, top, pairs, w, N, K, out, os, vec, st);

@@ -16,123 +16,33 @@
 //     stay on the kernels with wider column tiles.
 #include "common.h"
 #include "kernels.h"
+#include "row_ring.h"
 
 namespace {
 
-constexpr int kRgWaves = 4;
-
 enum { RG_NONE = 0, RG_SWIGLU = 1, RG_BIAS = 2, RG_GELU = 3, RG_RELU = 4 };
-
-typedef __attribute__((address_space(3))) void* rg_lptr;
-typedef const __attribute__((address_space(1))) void* rg_gptr;
-
-template <int N>
-LK_DEVICE void rg_wait() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
-}
-template <int L, int AHEAD>
-LK_DEVICE void rg_wait_ahead(int ahead) {  // all but the newest `ahead` stages of L loads have landed
-  if constexpr (AHEAD > 0) {
-    if (ahead >= AHEAD) {
-      rg_wait<L * AHEAD>();
-      return;
-    }
-    rg_wait_ahead<L, AHEAD - 1>(ahead);
-  } else {
-    rg_wait<0>();
-  }
-}
-
-// 64 K columns of (MT + NT) 16-row tiles: one stage of a wave's ring
-constexpr int rg_stage(int MT, int NT) { return (MT + NT) * 2048; }
-constexpr int rg_lds(int MT, int NT, int NS) {
-  const int ring = kRgWaves * NS * rg_stage(MT, NT), sums = kRgWaves * MT * NT * 1024;
-  return ring > sums ? ring : sums;
-}
 
 template <int MT, int NT, int NS, int EPI>
 __global__ __launch_bounds__(64 * kRgWaves, 1) void rows_gemm_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                                                                      const bf16_t* __restrict__ bias, bf16_t* __restrict__ Y, int M,
                                                                      int N, int K, long ldx, long ldy) {
-  constexpr int SB = rg_stage(MT, NT), L = (MT + NT) * 2;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int r16 = lane & 15, g = lane >> 4;
   const int all = K / 64, first = wave * all / kRgWaves, nst = (wave + 1) * all / kRgWaves - first;  // stages of this wave
-  const long k0 = (long)first * 64;
   const int n0 = blockIdx.x * 16;  // first output column
-  unsigned char* const ring = smem + wave * NS * SB;
-
-  // LDS row `row` holds the eight 16-byte chunks of its 128 bytes in the order chunk ^ (row & 7)
-  const int lrow = lane >> 3, lcol = ((lane & 7) ^ lrow) * 8;
+  const int lrow = lane >> 3;
+  const long k = (long)first * 64 + rg_lane_col(lane);
   const bf16_t* xs[2 * MT];
   const bf16_t* ws[2 * NT];
 #pragma unroll
-  for (int i = 0; i < 2 * MT; ++i) xs[i] = X + (long)min(8 * i + lrow, M - 1) * ldx + k0 + lcol;  // rows past M repeat the last one
+  for (int i = 0; i < 2 * MT; ++i) xs[i] = X + (long)min(8 * i + lrow, M - 1) * ldx + k;  // rows past M repeat the last one
 #pragma unroll
-  for (int i = 0; i < 2 * NT; ++i) ws[i] = W + ((long)(i >> 1) * (N >> 1) + n0 + 8 * (i & 1) + lrow) * K + k0 + lcol;
-
-  auto issue = [&](int st) {
-    unsigned char* base = ring + (st % NS) * SB;
-#pragma unroll
-    for (int i = 0; i < 2 * NT; ++i)
-      __builtin_amdgcn_global_load_lds((rg_gptr)(ws[i] + st * 64), (rg_lptr)(base + (2 * MT + i) * 1024), 16, 0, 2);
-#pragma unroll
-    for (int i = 0; i < 2 * MT; ++i)
-      __builtin_amdgcn_global_load_lds((rg_gptr)(xs[i] + st * 64), (rg_lptr)(base + i * 1024), 16, 0, 0);
-  };
-
+  for (int i = 0; i < 2 * NT; ++i) ws[i] = W + ((long)(i >> 1) * (N >> 1) + n0 + 8 * (i & 1) + lrow) * K + k;
   floatx4 acc[MT][NT];
-#pragma unroll
-  for (int m = 0; m < MT; ++m)
-#pragma unroll
-    for (int n = 0; n < NT; ++n) acc[m][n] = (floatx4){0.f, 0.f, 0.f, 0.f};
-
-#pragma unroll
-  for (int p = 0; p < NS - 1; ++p)
-    if (p < nst) issue(p);
-  for (int st = 0; st < nst; ++st) {
-    rg_wait_ahead<L, NS - 2>(min(NS - 2, nst - 1 - st));
-    __builtin_amdgcn_sched_barrier(0);
-    if (st + NS - 1 < nst) issue(st + NS - 1);  // into the slot whose fragments the last stage's products have consumed
-    __builtin_amdgcn_sched_barrier(0);
-    const unsigned char* base = ring + (st % NS) * SB;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int at = r16 * 128 + (((4 * h + g) ^ (r16 & 7)) << 4);
-      short8 a[MT], b[NT];
-#pragma unroll
-      for (int n = 0; n < NT; ++n) b[n] = *reinterpret_cast<const short8*>(base + (MT + n) * 2048 + at);
-#pragma unroll
-      for (int m = 0; m < MT; ++m) a[m] = *reinterpret_cast<const short8*>(base + m * 2048 + at);
-      // W as the A operand: the lane ends with one output row and 4 consecutive columns
-#pragma unroll
-      for (int m = 0; m < MT; ++m)
-#pragma unroll
-        for (int n = 0; n < NT; ++n) acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[n], a[m], acc[m][n], 0, 0, 0);
-    }
-  }
-
-  // lane l: row l & 15 of tile m, columns 4 (l >> 4) ..; partials as [wave][tile][lane] float4
-  __syncthreads();  // every wave's ring is read
-  floatx4* part = reinterpret_cast<floatx4*>(smem);
-#pragma unroll
-  for (int m = 0; m < MT; ++m)
-#pragma unroll
-    for (int n = 0; n < NT; ++n) part[(wave * MT * NT + m * NT + n) * 64 + lane] = acc[m][n];
-  __syncthreads();
-#pragma unroll
-  for (int m = wave; m < MT; m += kRgWaves) {  // one row tile per wave
-    floatx4 t[NT];
-#pragma unroll
-    for (int n = 0; n < NT; ++n) {
-      t[n] = part[(m * NT + n) * 64 + lane];
-#pragma unroll
-      for (int w = 1; w < kRgWaves; ++w) t[n] += part[((w * MT + m) * NT + n) * 64 + lane];
-    }
-    const int row = m * 16 + r16;
-    if (row >= M) continue;
+  rg_walk<MT, NT, NS>(xs, ws, nst, smem + wave * NS * rg_stage(MT, NT), acc);
+  rg_sums<MT, NT>(smem, acc, [&](int m, const floatx4 (&t)[NT]) {
+    const int row = m * 16 + (lane & 15), col = n0 + 4 * (lane >> 4);
+    if (row >= M) return;
     float y[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -140,7 +50,7 @@ __global__ __launch_bounds__(64 * kRgWaves, 1) void rows_gemm_kernel(const bf16_
         y[j] = bf2f(f2bf(lk_silu(bf2f(f2bf(t[0][j]))))) * bf2f(f2bf(t[NT - 1][j]));
       } else {
         y[j] = t[0][j];
-        if constexpr (EPI >= RG_BIAS) y[j] += bf2f(bias[n0 + 4 * g + j]);
+        if constexpr (EPI >= RG_BIAS) y[j] += bf2f(bias[col + j]);
         if constexpr (EPI == RG_GELU) y[j] = lk_gelu_erf(y[j]);
         if constexpr (EPI == RG_RELU) y[j] = fmaxf(y[j], 0.f);
       }
@@ -148,8 +58,8 @@ __global__ __launch_bounds__(64 * kRgWaves, 1) void rows_gemm_kernel(const bf16_
     uint2 pk;
     pk.x = pack_bf2(y[0], y[1]);
     pk.y = pack_bf2(y[2], y[3]);
-    *reinterpret_cast<uint2*>(Y + (long)row * ldy + n0 + 4 * g) = pk;
-  }
+    *reinterpret_cast<uint2*>(Y + (long)row * ldy + col) = pk;
+  });
 }
 
 template <int MT, int NT, int NS, int EPI>

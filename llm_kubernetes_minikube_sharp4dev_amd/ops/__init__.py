@@ -385,7 +385,8 @@ def _decode_bucket(M: int) -> Optional[int]:
 #   64 x 4096 x 4096 14.1 / 14.0    32 x 6144 x 4096 17.5 / 16.5    32 x 4096 x 14336 34.0 / 28.6
 # (past K 8192 more than 16 rows of X no longer stay in L2, and a weight past 100 MB is bound by HBM either
 # way.)  SwiGLU costs the streaming side another 3.5 us in its second launch (64 x 11264 x 2048: 18.2 / 19.5);
-# with a bias or an activation the other side is the prefill GEMM, 15-19 us at K 768-3072.
+# with a bias or an activation the other side is the prefill GEMM, 15-19 us at K 768-3072.  Where the streaming
+# kernel's sum rides in its consumer (linear_add_rmsnorm, linear_rope_kv) the two are level, and those stay as they are.
 ROWS_MAX_M = 64
 _ROWS_RULE: dict = {}
 
@@ -415,8 +416,6 @@ def _decode_gemm_kind(x, w, swiglu: bool) -> Optional[str]:
         return None
     M = x.shape[0]
     N, K = w.shape
-    if M > SKINNY_MAX_M and _rows_ok(x, w, 1 if swiglu else 0):
-        return "rows"
     if M < 1 or K % 256 or x.stride(1) != 1 or x.stride(0) % 8 or not w.is_contiguous():
         return None
     if swiglu:
@@ -785,7 +784,7 @@ def tune_decode(weights, ms: Sequence[int] = DECODE_TUNE_MS, iters: int = 3, col
         # ring vs loader waves (csrc/skinny_gemm.hip wsgemm_lw_kernel), measured at the tile's
         # largest M, before the routing below times the ws arm with it
         if WS_VARIANT_TUNE and _decode_static_ok(N, K, swiglu):
-            for M in [m for m in (64, 128, 192, 256) if m in ms and not _rows_rule(m, N, K, int(swiglu))]:
+            for M in [m for m in (64, 128, 192, 256) if m in ms]:
                 x = torch.randn(M, K, device=w.device, dtype=torch.bfloat16)
                 fns = {}
                 for v in (0, 1):
@@ -796,8 +795,6 @@ def tune_decode(weights, ms: Sequence[int] = DECODE_TUNE_MS, iters: int = 3, col
                 _WS_VARIANTS[(M, N, K, swiglu)] = best
                 out[(M, N, K, swiglu, "ws_variant")] = {("ring", "loader")[v]: round(t, 1) for v, t in med.items()}
         for M in ms:
-            if _rows_rule(M, N, K, int(swiglu)):  # routed by the rule, not by this table
-                continue
             x = torch.randn(M, K, device=w.device, dtype=torch.bfloat16)
             arms = {}
             if M <= 256 and _decode_static_ok(N, K, swiglu):
@@ -833,9 +830,9 @@ def linear(x, w, b=None, act: Optional[str] = None):
     if b is None and act is None:
         if _gemv_ok(x, w, 0):
             return lib().gemv_decode(0, x, w)
-        kind = _decode_gemm_kind(x, w, False)
-        if kind == "rows":
+        if x.shape[0] > SKINNY_MAX_M and _rows_ok(x, w, 0):
             return lib().rows_linear(x, w)
+        kind = _decode_gemm_kind(x, w, False)
         if kind == "skinny":
             return lib().skinny_linear(x, w)
         if kind == "ws":
@@ -860,9 +857,9 @@ def linear_swiglu(x, w_gate_up):
         return silu_mul(linear(x, w_gate_up))
     if _gemv_ok(x, w_gate_up, 2):
         return lib().gemv_decode(2, x, w_gate_up)
-    kind = _decode_gemm_kind(x, w_gate_up, True)
-    if kind == "rows":
+    if x.shape[0] > SKINNY_MAX_M and _rows_ok(x, w_gate_up, 1):
         return lib().rows_linear(x, w_gate_up, None, 1)
+    kind = _decode_gemm_kind(x, w_gate_up, True)
     if kind == "skinny":
         return lib().skinny_linear(x, w_gate_up, True)
     if kind == "ws":
