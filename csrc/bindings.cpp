@@ -801,6 +801,22 @@ std::vector<at::Tensor> knn_topk(const at::Tensor& corpus, const at::Tensor& cno
   if (N == 0 || nq == 0) return {at::full({nq, (long)K}, -INFINITY, fo), at::full({nq, (long)K}, -1, io)};
   at::Tensor out_s = at::empty({nq, (long)K}, fo);
   at::Tensor out_i = at::empty({nq, (long)K}, io);
+  const auto a16 = [](const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
+  if (const int nb = force_fused || !a16(corpus) || !a16(queries) ? 0 : lk_knn_scan_blocks(N, D, nq, kk)) {
+    at::Tensor ps = at::empty({nq, nb, kk}, fo), pi = at::empty({nq, nb, kk}, io);
+    if (kk < K) {
+      out_s.fill_(-INFINITY);
+      out_i.fill_(-1);
+    }
+    at::Tensor ks = kk < K ? at::empty({nq, kk}, fo) : out_s, ki = kk < K ? at::empty({nq, kk}, io) : out_i;
+    CHECK_RC(lk_knn_scan(bp(corpus), cnorm.data_ptr<float>(), N, D, bp(queries), qnorm.data_ptr<float>(), nq, kk, ps.data_ptr<float>(),
+                         pi.data_ptr<int>(), ks.data_ptr<float>(), ki.data_ptr<int>(), cur_stream()), "knn_scan");
+    if (kk < K) {
+      out_s.slice(1, 0, kk).copy_(ks);
+      out_i.slice(1, 0, kk).copy_(ki);
+    }
+    return {out_s, out_i};
+  }
   if (D % 64 == 0 && nq <= 256 && !force_fused) {
     // corpus streamed once by the LDS-DMA weight-streaming GEMM (dots in f32), then a
     // normalise + chunked top-k pass and the shared merge
@@ -828,6 +844,26 @@ std::vector<at::Tensor> knn_topk(const at::Tensor& corpus, const at::Tensor& cno
                     out_i.data_ptr<int>(), cur_stream());
   CHECK_RC(rc, "knn_merge");
   return {out_s, out_i};
+}
+
+// The one-pass search with both results in one buffer, int32 [2, nq, K] (score bits, then row numbers), for a caller that copies
+// them to the host in one piece; an empty tensor where the one-pass search does not take the shape.
+at::Tensor knn_packed(const at::Tensor& corpus, const at::Tensor& cnorm, const at::Tensor& queries, int64_t K) {
+  CHECK_CUDA(corpus); CHECK_BF16(corpus); CHECK_CONTIG(corpus); CHECK_F32(cnorm); CHECK_CONTIG(cnorm);
+  CHECK_CUDA(queries); CHECK_BF16(queries); CHECK_CONTIG(queries);
+  TORCH_CHECK(corpus.dim() == 2 && queries.dim() == 2 && corpus.size(1) == queries.size(1), "dimension mismatch");
+  const long N = corpus.size(0);
+  const int D = corpus.size(1), nq = queries.size(0);
+  TORCH_CHECK(cnorm.numel() == N, "norm shapes");
+  auto io = corpus.options().dtype(at::kInt);
+  const auto a16 = [](const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
+  const int nb = K <= N && a16(corpus) && a16(queries) ? lk_knn_scan_blocks(N, D, nq, (int)std::min<int64_t>(K, 64)) : 0;
+  if (!nb) return at::empty({0}, io);
+  at::Tensor out = at::empty({2, nq, K}, io), part = at::empty({2, nq, nb, K}, io);
+  int *o = out.data_ptr<int>(), *p = part.data_ptr<int>();
+  CHECK_RC(lk_knn_scan(bp(corpus), cnorm.data_ptr<float>(), N, D, bp(queries), nullptr, nq, (int)K, reinterpret_cast<float*>(p),
+                       p + (long)nq * nb * K, reinterpret_cast<float*>(o), o + (long)nq * K, cur_stream()), "knn_scan");
+  return out;
 }
 
 std::vector<at::Tensor> knn_merge(const at::Tensor& cand_s, const at::Tensor& cand_i, int64_t K) {
@@ -2272,6 +2308,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("flash_prefill", &flash_prefill, "", py::arg("q"), py::arg("k"), py::arg("v"), py::arg("block_tables"), py::arg("cu_q"), py::arg("ctx_lens"), py::arg("tile_seq"), py::arg("tile_q0"), py::arg("Hq"), py::arg("Hkv"), py::arg("D"), py::arg("scale"), py::arg("causal"), py::arg("out") = py::none(), py::arg("part_o") = py::none(), py::arg("part_ml") = py::none(), py::arg("q_past") = py::none());
   m.def("knn_topk", &knn_topk, "", py::arg("corpus"), py::arg("cnorm"), py::arg("queries"), py::arg("qnorm"),
         py::arg("K"), py::arg("force_fused") = false);
+  m.def("knn_packed", &knn_packed);
   m.def("knn_merge", &knn_merge);
   m.def("pool_normalize", &pool_normalize, "", py::arg("hidden"), py::arg("cu"), py::arg("mode"), py::arg("normalize"),
         py::arg("out") = py::none());

@@ -12,11 +12,14 @@
 // 4 k-steps (the reduction order of a dot product is free).  Scores are staged in
 // LDS and each wave extracts the block-local top-k of 8 queries by k rounds of
 // wave-wide (score, index) argmax.
+// Few queries (lk_knn_scan, <= 16 queries, K <= 8, the serving path): one persistent pass over the corpus that
+// keeps its best rows as it goes, and a merge of its workgroups' lists; see knn_scan_kernel.
 // Pass 2 (lk_knn_merge): one workgroup per query merges nblocks*k candidates with
 // the same tie rule.  Sharded (multi-GPU) search reuses pass 2 on all-gathered
 // candidates.
 #include "common.h"
 #include "kernels.h"
+#include "row_ring.h"
 
 namespace {
 
@@ -31,6 +34,19 @@ LK_DEVICE bool better(float s1, int i1, float s2, int i2) {
 LK_DEVICE void wave_argmax(float& s, int& i) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
+    const float s2 = __shfl_xor(s, o, 64);
+    const int i2 = __shfl_xor(i, o, 64);
+    if (better(s2, i2, s, i)) {
+      s = s2;
+      i = i2;
+    }
+  }
+}
+
+template <int W>  // over groups of W lanes
+LK_DEVICE void group_argmax(float& s, int& i) {
+#pragma unroll
+  for (int o = W / 2; o > 0; o >>= 1) {
     const float s2 = __shfl_xor(s, o, 64);
     const int i2 = __shfl_xor(i, o, 64);
     if (better(s2, i2, s, i)) {
@@ -252,6 +268,218 @@ __global__ __launch_bounds__(256) void knn_merge_kernel(const float* __restrict_
   (void)last;
 }
 
+// One pass for up to 16 queries and K <= 8.  The corpus is read once (746 MB at 485,620 x 768) and nothing of its size is
+// written: the two-pass form wrote and re-read f32 scores of every row (31 MB at 16 queries) and paid two more launches.
+// 4 waves per CU, each with the queries' fragments in registers (D / 32 of them) and a private LDS ring of 16 stages of
+// 16 rows x 128 bytes (row_ring.h), walk 16-row tiles round robin without a barrier, so 120 KB of corpus are on their way
+// per CU.  A lane sees 4 rows of one query per tile and keeps its 8 best in order (rows come in ascending order, so an
+// equal score never displaces: the stable order); 16 lists per query meet in LDS at the end.
+// 16 x 485,620 x 768: scan 158 + top-k 26 + merge 10 us -> 130 + 6 (5.7 TB/s); 1 x 20,011: 11 + 12 + 5 -> 15 + 5.
+constexpr int kScanK = 8, kScanQ = 16, kScanStages = 16;
+
+// ls / li descending: s, i enters behind everything that is not smaller
+LK_DEVICE void list_insert(float s, int i, float (&ls)[kScanK], int (&li)[kScanK]) {
+#pragma unroll
+  for (int j = kScanK - 1; j >= 1; --j) {
+    const bool here = s > ls[j], above = s > ls[j - 1];
+    ls[j] = here ? (above ? ls[j - 1] : s) : ls[j];
+    li[j] = here ? (above ? li[j - 1] : i) : li[j];
+  }
+  if (s > ls[0]) {
+    ls[0] = s;
+    li[0] = i;
+  }
+}
+
+// the head leaves (of the padding behind a short list, all heads do: nothing follows it)
+LK_DEVICE void list_pop(float (&ls)[kScanK], int (&li)[kScanK]) {
+#pragma unroll
+  for (int j = 0; j + 1 < kScanK; ++j) {
+    ls[j] = ls[j + 1];
+    li[j] = li[j + 1];
+  }
+  ls[kScanK - 1] = -INFINITY;
+  li[kScanK - 1] = 0x7fffffff;
+}
+
+template <int SEG>
+__global__ __launch_bounds__(256, 1) void knn_scan_kernel(const bf16_t* __restrict__ corpus, const float* __restrict__ cnorm, long N,
+                                                          const bf16_t* __restrict__ queries, const float* __restrict__ qnorm, int nq,
+                                                          int K, float* __restrict__ part_s, int* __restrict__ part_i) {
+  constexpr int D = SEG * 64, NS = kScanStages;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, g = lane >> 4;
+  short8 qf[2 * SEG];
+  {
+    const bf16_t* q = queries + (long)min(r16, nq - 1) * D + 8 * g;
+#pragma unroll
+    for (int k = 0; k < 2 * SEG; ++k) qf[k] = *reinterpret_cast<const short8*>(q + 32 * k);
+  }
+  float qn;
+  if (qnorm) {
+    qn = qnorm[min(r16, nq - 1)];
+  } else {
+    float p[2 * SEG], ss = 0.f;  // (eight at a time: one chain of D / 4 additions would cost the norm its last bits)
+#pragma unroll
+    for (int k = 0; k < 2 * SEG; ++k) {
+      p[k] = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float v = bf2f((bf16_t)qf[k][e]);
+        p[k] += v * v;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 2 * SEG; k += 4) ss += (p[k] + p[k + 1]) + (2 * SEG - k >= 4 ? p[k + 2] + p[k + 3] : 0.f);
+    ss += __shfl_xor(ss, 16, 64);
+    ss += __shfl_xor(ss, 32, 64);
+    qn = sqrtf(ss);
+  }
+  const long tiles = (N + 15) / 16, first = (long)blockIdx.x * 4 + w, step = (long)gridDim.x * 4;
+  const long mine = first < tiles ? (tiles - 1 - first) / step + 1 : 0, total = mine * SEG;  // this wave's tiles and stages
+  unsigned char* const ring = smem + w * NS * 2048;
+  const int lrow = lane >> 3, lcol = rg_lane_col(lane);
+  long it = first, ist = 0;  // the next stage to request: its tile and number
+  int iseg = 0;
+  auto issue = [&]() {
+    unsigned char* base = ring + (ist % NS) * 2048;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const long row = min(it * 16 + 8 * i + lrow, N - 1);
+      __builtin_amdgcn_global_load_lds((rg_gptr)(corpus + row * D + iseg * 64 + lcol), (rg_lptr)(base + i * 1024), 16, 0, 2);
+    }
+    ++ist;
+    if (++iseg == SEG) {
+      iseg = 0;
+      it += step;
+    }
+  };
+#pragma unroll
+  for (int p = 0; p < NS - 1; ++p)
+    if (p < total) issue();
+  float ls[kScanK];
+  int li[kScanK];
+#pragma unroll
+  for (int j = 0; j < kScanK; ++j) {
+    ls[j] = -INFINITY;
+    li[j] = 0x7fffffff;
+  }
+  long st = 0;
+  for (long t = first; t < tiles; t += step) {
+    const long d0 = t * 16 + 4 * g;
+    float cn[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) cn[j] = cnorm[min(d0 + j, N - 1)];
+    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int seg = 0; seg < SEG; ++seg, ++st) {
+      rg_wait_ahead<2, NS - 2>((int)min((long)(NS - 2), total - 1 - st));
+      __builtin_amdgcn_sched_barrier(0);
+      if (ist < total) issue();
+      __builtin_amdgcn_sched_barrier(0);
+      const unsigned char* base = ring + (st % NS) * 2048;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const short8 a = *reinterpret_cast<const short8*>(base + r16 * 128 + (((4 * h + g) ^ (r16 & 7)) << 4));
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qf[2 * seg + h], acc, 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float s = d0 + j < N ? acc[j] / (qn * cn[j] + 1e-9f) : -INFINITY;
+      if (s > ls[kScanK - 1]) list_insert(s, (int)(d0 + j), ls, li);
+    }
+  }
+  // [query][4 waves x 4 lane groups][kScanK]
+  __syncthreads();
+  float* ms = reinterpret_cast<float*>(smem);
+  int* mi = reinterpret_cast<int*>(smem) + kScanQ * 16 * kScanK;
+#pragma unroll
+  for (int j = 0; j < kScanK; ++j) {
+    ms[(r16 * 16 + w * 4 + g) * kScanK + j] = ls[j];
+    mi[(r16 * 16 + w * 4 + g) * kScanK + j] = li[j];
+  }
+  __syncthreads();
+  // a wave takes four queries at once, a lane one of their 16 lists: K rounds over the lists' heads
+  {
+    const int q = w * 4 + g;
+    float v[kScanK];
+    int id[kScanK];
+#pragma unroll
+    for (int j = 0; j < kScanK; ++j) {
+      v[j] = ms[(q * 16 + r16) * kScanK + j];
+      id[j] = mi[(q * 16 + r16) * kScanK + j];
+    }
+    for (int k = 0; k < K; ++k) {
+      float bs = v[0];
+      int bi = id[0];
+      group_argmax<16>(bs, bi);
+      if (r16 == 0 && q < nq) {
+        const long o = ((long)q * gridDim.x + blockIdx.x) * K + k;
+        part_s[o] = bs;
+        part_i[o] = bs == -INFINITY ? -1 : bi;
+      }
+      if (id[0] == bi) list_pop(v, id);
+    }
+  }
+}
+
+// merge of at most 256 lists of K <= 8, each in order: one workgroup per query, a list per thread; every 16 lanes take the
+// K best of their lists by the lists' heads, then 16 lanes those of the 16 groups
+__global__ __launch_bounds__(256) void knn_merge_lists_kernel(const float* __restrict__ cs, const int* __restrict__ ci, int lists, int K,
+                                                              float* __restrict__ out_s, int* __restrict__ out_i) {
+  __shared__ float rs[16][kScanK];
+  __shared__ int ri[16][kScanK];
+  const int q = blockIdx.x, tid = threadIdx.x, l16 = tid & 15, grp = tid >> 4;
+  float s[kScanK];
+  int i[kScanK];
+#pragma unroll
+  for (int j = 0; j < kScanK; ++j) {
+    const long o = ((long)q * lists + tid) * K + j;
+    const bool on = tid < lists && j < K;
+    s[j] = on ? cs[o] : -INFINITY;
+    const int v = on ? ci[o] : -1;
+    i[j] = v < 0 ? 0x7fffffff : v;
+  }
+  for (int k = 0; k < K; ++k) {
+    float bs = s[0];
+    int bi = i[0];
+    group_argmax<16>(bs, bi);
+    if (l16 == 0) {
+      rs[grp][k] = bs;
+      ri[grp][k] = bi;
+    }
+    if (i[0] == bi) list_pop(s, i);
+  }
+  __syncthreads();
+  if (grp) return;
+#pragma unroll
+  for (int j = 0; j < kScanK; ++j) {
+    s[j] = j < K ? rs[l16][j] : -INFINITY;
+    i[j] = j < K ? ri[l16][j] : 0x7fffffff;
+  }
+  for (int k = 0; k < K; ++k) {
+    float bs = s[0];
+    int bi = i[0];
+    group_argmax<16>(bs, bi);
+    if (l16 == 0) {
+      out_s[(long)q * K + k] = bs;
+      out_i[(long)q * K + k] = bs == -INFINITY ? -1 : bi;
+    }
+    if (i[0] == bi) list_pop(s, i);
+  }
+}
+
+template <int SEG>
+int launch_scan(const bf16_t* corpus, const float* cnorm, long N, const bf16_t* queries, const float* qnorm, int nq, int K, int nb,
+                float* part_s, int* part_i, hipStream_t st) {
+  constexpr int lds = 4 * kScanStages * 2048;  // (the lists at the end need 16 KB of it)
+  LK_SET_MAX_LDS((knn_scan_kernel<SEG>), lds);
+  knn_scan_kernel<SEG><<<nb, 256, lds, st>>>(corpus, cnorm, N, queries, qnorm, nq, K, part_s, part_i);
+  LK_CHECK_LAUNCH();
+  return 0;
+}
+
 }  // namespace
 
 int lk_knn_nblocks(long N) { return (int)((N + ROWS - 1) / ROWS); }
@@ -290,5 +518,33 @@ int lk_knn_merge(const float* cand_s, const int* cand_i, int nq, int ncand, int 
                  int* out_i, hipStream_t st) {
   if (nq <= 0) return 0;
   knn_merge_kernel<<<nq, 256, 0, st>>>(cand_s, cand_i, ncand, K, out_s, out_i);
+  return 0;
+}
+
+// workgroups of the one-pass scan (0: it does not take this shape): one per CU, a tile of 16 rows per wave at least
+int lk_knn_scan_blocks(long N, int D, int nq, int K) {
+  if (N <= 0 || N >= 0x7fffffffL - 16 || nq < 1 || nq > kScanQ || K < 1 || K > kScanK) return 0;
+  if (D != 128 && D != 256 && D != 384 && D != 512 && D != 768 && D != 1024) return 0;
+  const long b = ((N + 15) / 16 + 3) / 4;
+  return (int)(b < 256 ? b : 256);
+}
+
+// out_s / out_i [nq, K]; qnorm null: the queries' norms are taken here; part_*: [nq, blocks, K]
+int lk_knn_scan(const bf16_t* corpus, const float* cnorm, long N, int D, const bf16_t* queries, const float* qnorm, int nq, int K,
+                float* part_s, int* part_i, float* out_s, int* out_i, hipStream_t st) {
+  const int nb = lk_knn_scan_blocks(N, D, nq, K);
+  if (!nb) return -1;
+  int rc;
+  switch (D) {
+    case 128: rc = launch_scan<2>(corpus, cnorm, N, queries, qnorm, nq, K, nb, part_s, part_i, st); break;
+    case 256: rc = launch_scan<4>(corpus, cnorm, N, queries, qnorm, nq, K, nb, part_s, part_i, st); break;
+    case 384: rc = launch_scan<6>(corpus, cnorm, N, queries, qnorm, nq, K, nb, part_s, part_i, st); break;
+    case 512: rc = launch_scan<8>(corpus, cnorm, N, queries, qnorm, nq, K, nb, part_s, part_i, st); break;
+    case 768: rc = launch_scan<12>(corpus, cnorm, N, queries, qnorm, nq, K, nb, part_s, part_i, st); break;
+    default: rc = launch_scan<16>(corpus, cnorm, N, queries, qnorm, nq, K, nb, part_s, part_i, st); break;
+  }
+  if (rc) return rc;
+  knn_merge_lists_kernel<<<nq, 256, 0, st>>>(part_s, part_i, nb, K, out_s, out_i);
+  LK_CHECK_LAUNCH();
   return 0;
 }

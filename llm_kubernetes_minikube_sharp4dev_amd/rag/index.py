@@ -202,6 +202,13 @@ class RagIndex:
             # host queries are cast on the host (a few KB) and copied once: no device cast kernel
             qt = (qt.to(torch.bfloat16).to(self.device) if qt.device.type == "cpu"
                   else qt.to(self.device, torch.bfloat16)).reshape(-1, corpus.shape[1]).contiguous()
+            both = ops.knn_packed(corpus, norms, qt, min(k, 64)) if qt.is_cuda else None
+            if both is not None:
+                host = torch.empty(both.shape, dtype=both.dtype, pin_memory=True)
+                host.copy_(both, non_blocking=True)
+                ev = torch.cuda.Event()
+                ev.record()
+                return PendingSearch(host=(host[0].view(torch.float32), host[1], min(k, n)), event=ev)
             qn = ops.row_norms(qt) if qt.is_cuda else qt.float().norm(dim=-1)
             s, i = ops.knn_topk(corpus, norms, qt, qn, min(k, 64))
         if not s.is_cuda:

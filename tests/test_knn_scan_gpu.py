@@ -1,0 +1,47 @@
+"""The one-pass search (csrc/knn.hip knn_scan_kernel) against float64 cosines in stable order: corpora of less than a tile to
+more tiles than waves, every width, the most queries and hits it takes, equal rows, and the shapes around it."""
+import pytest
+import torch
+
+from llm_kubernetes_minikube_sharp4dev_amd import ops
+from llm_kubernetes_minikube_sharp4dev_amd.rag.index import RagChunk, RagIndex
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("N,D,nq,K", [(1, 128, 1, 1), (15, 256, 16, 8), (17, 384, 3, 5), (65, 512, 16, 8), (4097, 1024, 7, 3),
+                                      (20011, 768, 1, 5), (70003, 768, 16, 8), (300, 768, 17, 8), (300, 768, 4, 9), (300, 192, 4, 4), (5, 768, 2, 8)])
+def test_scan(hip, N, D, nq, K):
+    g = torch.Generator(device=DEV).manual_seed(N)
+    c = torch.randn(N, D, device=DEV, generator=g).to(torch.bfloat16)
+    c[N // 2:] = c[:N - N // 2].clone()                     # every row of the first half again
+    q = torch.randn(nq, D, device=DEV, generator=g).to(torch.bfloat16)
+    cn, qn = ops.row_norms(c), ops.row_norms(q)
+    ref = (q.double() @ c.double().t()) / (q.double().norm(dim=1)[:, None] * c.double().norm(dim=1)[None] + 1e-9)
+    s, i = ops.knn_topk(c, cn, q, qn, K)
+    k = min(K, N)
+    want = ref.sort(dim=1, descending=True, stable=True)
+    # f32 sums of D products and one division: a few 2^-24 of the products' sizes (rows are unit after the division)
+    assert ((s[:, :k].double() - want[0][:, :k]).abs() <= 1e-6).all()
+    assert ((ref.gather(1, i[:, :k].long()) - want[0][:, :k]).abs() <= 1e-6).all()
+    same = s[:, 1:k] == s[:, :k - 1]
+    assert (i[:, 1:k][same] > i[:, :k - 1][same]).all()     # equal scores: the lower row first
+    assert (i[:, k:] == -1).all() and (s[:, k:] == float("-inf")).all()
+    both = ops.knn_packed(c, cn, q, K)
+    assert (both is not None) == (nq <= 16 and K <= 8 and D != 192 and K <= N)
+    if both is not None:
+        assert torch.equal(both[1], i) and ((both[0].view(torch.float32) - s).abs() <= 1e-6).all()
+
+
+def test_index_search_agrees(hip):
+    """RagIndex gives the same hits whether or not the one-pass search takes the shape."""
+    g = torch.Generator(device=DEV).manual_seed(3)
+    c = torch.randn(3000, 768, device=DEV, generator=g).to(torch.bfloat16)
+    q = torch.randn(20, 768, device=DEV, generator=g)
+    index = RagIndex(None, backend="gpu", device=DEV)
+    index.chunks = [RagChunk("d#0", "d", "")] * 3000
+    index.set_gpu_corpus(c)
+    many, few = index.search_vectors(q, 6), [index.search_vectors(q[j:j + 1], 6)[0] for j in range(20)]
+    assert [[i for i, _ in h] for h in many] == [[i for i, _ in h] for h in few]
+    assert max(abs(a - b) for x, y in zip(many, few) for (_, a), (_, b) in zip(x, y)) <= 1e-6
