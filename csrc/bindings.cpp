@@ -181,20 +181,20 @@ at::Tensor ws_linear(const at::Tensor& x, const at::Tensor& w, bool swiglu, int6
 
 // few-row GEMM (csrc/rows_gemm.hip): M <= 64 rows, any epilogue, one launch.  epi: 0 none, 1 SwiGLU, 2 bias, 3 bias + GELU,
 // 4 bias + ReLU
-at::Tensor rows_linear(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, int64_t epi) {
+at::Tensor rows_linear(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, int64_t epi, bool wide) {
   CHECK_CUDA(x); CHECK_BF16(x); CHECK_BF16(w); CHECK_LASTDIM(x); CHECK_CONTIG(w);
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1), "x [M,K], w [N,K]");
   check_rows16(x, "x"); check_rows16(w, "w");
   const int M = x.size(0), K = x.size(1), N = w.size(0);
   TORCH_CHECK(epi >= 0 && epi <= 4 && lk_rows_gemm_supported(M, N, K, (int)epi),
-              "rows_linear: M in [1, 64], K a multiple of 64, N of 16 (32 with SwiGLU)");
+              "rows_linear: M in [1, 4096], K a multiple of 64, N of 16 (32 with SwiGLU)");
   TORCH_CHECK((epi >= 2) == bias.has_value(), "rows_linear: a bias goes with epilogues 2-4");
   if (bias) {
     CHECK_CUDA((*bias)); CHECK_BF16((*bias)); CHECK_CONTIG((*bias));
     TORCH_CHECK(bias->numel() == N, "bias shape");
   }
   at::Tensor out = at::empty({M, epi == 1 ? N / 2 : N}, x.options());
-  int rc = lk_rows_gemm(bp(x), bp(w), bias ? bp(*bias) : nullptr, bp(out), M, N, K, x.stride(0), out.stride(0), (int)epi,
+  int rc = lk_rows_gemm(bp(x), bp(w), bias ? bp(*bias) : nullptr, bp(out), M, N, K, x.stride(0), out.stride(0), (int)epi, wide ? 1 : 0,
                         cur_stream());
   CHECK_RC(rc, "rows_linear");
   return out;
@@ -2233,7 +2233,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_linear", &skinny_linear, "", py::arg("x"), py::arg("w"), py::arg("swiglu") = false,
         py::arg("splits") = 0, py::arg("out") = py::none());
   m.def("skinny_splits", &skinny_splits);
-  m.def("rows_linear", &rows_linear, py::arg("x"), py::arg("w"), py::arg("bias") = py::none(), py::arg("epi") = 0);
+  m.def("rows_linear", &rows_linear, py::arg("x"), py::arg("w"), py::arg("bias") = py::none(), py::arg("epi") = 0, py::arg("wide") = false);
   m.def("rows_supported", [](int64_t M, int64_t N, int64_t K, int64_t epi) { return lk_rows_gemm_supported((int)M, (int)N, (int)K, (int)epi); });
   m.def("ws_linear", &ws_linear, "", py::arg("x"), py::arg("w"), py::arg("swiglu") = false, py::arg("bn") = 0,
         py::arg("splits") = 0, py::arg("out") = py::none());

@@ -31,7 +31,7 @@ int lk_activation(bf16_t* x, const bf16_t* bias, long rows, int N, long xs, int 
 
 // rows_gemm.hip (M <= 64, one launch, every epilogue)
 bool lk_rows_gemm_supported(int M, int N, int K, int epi);
-int lk_rows_gemm(const void* x, const void* w, const void* b, void* y, int M, int N, int K, long ldx, long ldy, int epi,
+int lk_rows_gemm(const void* x, const void* w, const void* b, void* y, int M, int N, int K, long ldx, long ldy, int epi, int wide,
                  hipStream_t st);
 
 // skinny_gemm.hip (decode-regime linear, optional fused SwiGLU)

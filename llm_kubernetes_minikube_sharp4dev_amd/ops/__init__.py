@@ -384,39 +384,63 @@ def _decode_bucket(M: int) -> Optional[int]:
     return None
 
 
-# Few rows (csrc/rows_gemm.hip, M <= 64, one launch with any epilogue) or the kernels with wider column
-# tiles.  A workgroup of the few-row kernel reads 16 columns of W (SwiGLU 2 x 16) and ALL of X, so its time
-# is 2.6 us + (bytes per workgroup x rounds of 256 workgroups) / 58 KB/us (a further 1.3 when there is more
-# than one round); the weight-streaming kernel takes ~9.5 us for its two launches + 0.14 us per MB of W + M / 32.
-# Equating the two gives the line below.  Measured in hipGraphs, weights cold, few-row / streaming (us):
-#   64 x 2048 x 2048  7.7 / 10.9    32 x 2048 x 5632 11.9 / 13.2    16 x 10368 x 2048 10.9 / 14.1
-#   64 x 3072 x 2048  8.0 / 11.3    64 x 2048 x 5632 17.0 / 14.3    48 x 10368 x 2048 18.5 / 16.0
-#   64 x 4096 x 4096 14.1 / 14.0    32 x 6144 x 4096 17.5 / 16.5    32 x 4096 x 14336 34.0 / 28.6
-# (past K 8192 more than 16 rows of X no longer stay in L2, and a weight past 100 MB is bound by HBM either
-# way.)  SwiGLU costs the streaming side another 3.5 us in its second launch (64 x 11264 x 2048: 18.2 / 19.5);
-# with a bias or an activation the other side is the prefill GEMM, 15-19 us at K 768-3072.  Where the streaming
-# kernel's sum rides in its consumer (linear_add_rmsnorm, linear_rope_kv) the two are level, and those stay as they are.
-ROWS_MAX_M = 64
+# Few rows (csrc/rows_gemm.hip, one launch with any epilogue) or the kernels with larger tiles.  A workgroup of the few-row
+# kernel reads 16 (wide: 32) columns of W -- SwiGLU 2 x 16 -- and up to 64 rows of X, so its time is
+#   2.6 us + rounds of 256 workgroups x (their bytes / 58 KB/us) + 1 us per round behind the first,
+# and not below W at 4.2 TB/s.  The other side: up to 256 rows without a bias the weight-streaming kernel (its two launches,
+# 0.14 us per MB of W, M / 22; 3.5 us for SwiGLU's second launch), else the prefill GEMM (a chain of K / 64 stages
+# whatever M is, as long as its tiles are fewer than CUs).  Measured in hipGraphs, weights cold, few-row / other (us):
+#    64 x  2048 x 2048  7.7 / 11.0    256 x 2048 x 2048  8.8 / 19.7    768 x 2048 x 2048 22.8 / 28.6   1024: 30.3 / 30.2
+#    64 x 10368 x 2048 17.9 / 16.7    128 x 4096 x 4096 15.7 / 18.4    192 x 4096 x 4096 28.6 / 20.9
+#    64 x 11264 x 2048 (SwiGLU) 18.3 / 19.6             512 x 2048 x 5632 38.6 / 43.9    768: 57.8 / 45.1
+#   bias:  19 x  768 x  768  3.5 / 15.6    512 x 2304 x 768 12.1 / 19.7    768 x 3072 x 768 18.6 / 23.5    2048: 48 / 24.7
+# (past K 8192 more than 16 rows of X do not stay in L2.)  Where the streaming kernel's sum rides in its consumer
+# (linear_add_rmsnorm, linear_rope_kv) the two are level at decode sizes, and those stay as they are.
+ROWS_MAX_M = 1024
 _ROWS_RULE: dict = {}
 
 
-def _rows_rule(M: int, N: int, K: int, epi: int) -> bool:
-    key = ((M + 15) // 16, N, K, epi)
-    ok = _ROWS_RULE.get(key)
-    if ok is None:
-        mt, nt = key[0], 2 if epi == 1 else 1
-        rounds = -(-N // (16 * nt * 256))
-        q = rounds * (mt + nt) * K / 32 * (1.3 if rounds > 1 else 1.0)     # KB
-        mb = N * K * 2 / 1e6
-        ok = (1 <= M <= ROWS_MAX_M and (K <= 8192 or mt == 1) and q <= (600 if epi == 1 else 400) + 8 * min(mb, 100) + 29 * mt
-              and lib().rows_supported(M, N, K, epi))
-        _ROWS_RULE[key] = ok
-    return ok
+def _rows_rule(M: int, N: int, K: int, epi: int) -> Optional[bool]:
+    """None: not the few-row kernel; else its ``wide`` argument."""
+    mt = (M + 15) // 16 if M <= 64 else 4 * ((M + 63) // 64)   # 16-row tiles of X
+    key = (mt, N, K, epi)
+    if key in _ROWS_RULE:
+        return _ROWS_RULE[key]
+    pick = None
+    if 1 <= M <= ROWS_MAX_M and (K <= 8192 or mt == 1) and lib().rows_supported(M, N, K, epi):
+        mb, rows = N * K * 2 / 1e6, 16 * mt
+
+        def cost(nt, wide):
+            m = min(mt, 4) if not wide else (2 if mt <= 2 else 4)
+            wgs = -(-mt // 4) * (N // (16 * nt))
+            rounds = -(-wgs // 256)
+            return max(2.6 + rounds * (m + nt) * K / 32 / 58 + (rounds - 1), mb / 4.2)
+
+        if epi == 1:
+            t, wide = cost(2, False), False
+        else:
+            t, wide = cost(1, False), False
+            if N % 32 == 0 and cost(2, True) < t:
+                t, wide = cost(2, True), True
+        if epi < 2 and rows <= 256:
+            other = min(7.5, 2 + K / 340) + 0.14 * mb + rows / 22 + (3.5 if epi == 1 else 0)
+        elif epi < 2:
+            other = min(20 + K / 256, 4 + K / 64)
+        else:
+            other = min(17 + 3 * K / 1024, 6 + K / 64)
+        if t < other:
+            pick = wide
+    _ROWS_RULE[key] = pick
+    return pick
 
 
-def _rows_ok(x, w, epi: int) -> bool:
-    return (x.dim() == 2 and w.dim() == 2 and 1 <= x.shape[0] <= ROWS_MAX_M and _gemm_ok(x, w) and w.data_ptr() % 16 == 0
-            and _rows_rule(x.shape[0], w.shape[0], w.shape[1], epi))
+def _rows(x, w, b, epi: int):
+    """The product on the few-row kernel, or None where the rule or the operands' layout say otherwise."""
+    if not (x.dim() == 2 and w.dim() == 2 and SKINNY_MAX_M < x.shape[0] <= (WS_MAX_M if GEMM_LIBRARY else ROWS_MAX_M)
+            and _gemm_ok(x, w) and w.data_ptr() % 16 == 0):
+        return None
+    wide = _rows_rule(x.shape[0], w.shape[0], w.shape[1], epi)
+    return None if wide is None else lib().rows_linear(x, w, b, epi, wide)
 
 
 def _decode_gemm_kind(x, w, swiglu: bool) -> Optional[str]:
@@ -839,8 +863,9 @@ def linear(x, w, b=None, act: Optional[str] = None):
     if b is None and act is None:
         if _gemv_ok(x, w, 0):
             return lib().gemv_decode(0, x, w)
-        if x.shape[0] > SKINNY_MAX_M and _rows_ok(x, w, 0):
-            return lib().rows_linear(x, w)
+        y = _rows(x, w, None, 0)
+        if y is not None:
+            return y
         kind = _decode_gemm_kind(x, w, False)
         if kind == "skinny":
             return lib().skinny_linear(x, w)
@@ -851,8 +876,10 @@ def linear(x, w, b=None, act: Optional[str] = None):
         b = torch.zeros(w.shape[0], device=x.device, dtype=x.dtype)
         epi = EPI[act]
     lib_arm = GEMM_LIBRARY == 1 or (GEMM_LIBRARY == 2 and epi == 0 and x.shape[0] > WS_MAX_M)
-    if epi >= 2 and not lib_arm and b.dtype == torch.bfloat16 and b.is_contiguous() and b.numel() == w.shape[0] and _rows_ok(x, w, epi):
-        return lib().rows_linear(x, w, b, epi)
+    if epi >= 2 and not lib_arm and b.dtype == torch.bfloat16 and b.is_contiguous() and b.numel() == w.shape[0]:
+        y = _rows(x, w, b, epi)
+        if y is not None:
+            return y
     y = gemm(x, w, b, epi) if _gemm_ok(x, w) and not lib_arm else None
     if y is None:
         y = _library(x, w, b, act, (x.shape[0] > WS_MAX_M, w.shape[0], w.shape[1], epi))
@@ -866,8 +893,9 @@ def linear_swiglu(x, w_gate_up):
         return silu_mul(linear(x, w_gate_up))
     if _gemv_ok(x, w_gate_up, 2):
         return lib().gemv_decode(2, x, w_gate_up)
-    if x.shape[0] > SKINNY_MAX_M and _rows_ok(x, w_gate_up, 1):
-        return lib().rows_linear(x, w_gate_up, None, 1)
+    y = _rows(x, w_gate_up, None, 1)
+    if y is not None:
+        return y
     kind = _decode_gemm_kind(x, w_gate_up, True)
     if kind == "skinny":
         return lib().skinny_linear(x, w_gate_up, True)

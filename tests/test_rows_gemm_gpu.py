@@ -19,15 +19,16 @@ def _ref(x, w, b, epi):
     return torch.nn.functional.gelu(y) if epi == 3 else torch.relu(y) if epi == 4 else y
 
 
-@pytest.mark.parametrize("M", [1, 15, 16, 17, 33, 48, 49, 64])
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("M", [1, 15, 16, 17, 33, 48, 49, 64, 65, 130, 257])
 @pytest.mark.parametrize("N,K,epi", [(16, 64, 0), (48, 128, 2), (2048, 2048, 0), (160, 320, 1), (768, 768, 2), (3072, 768, 3),
                                      (96, 832, 4), (64, 14336, 0), (2048, 5632, 1)])
-def test_rows_linear(hip, M, N, K, epi):
+def test_rows_linear(hip, M, N, K, epi, wide):
     torch.manual_seed(M + N + K)
     x = torch.randn(M + 1, K + 8, device=DEV).to(torch.bfloat16)[1:, :K]   # rows of a wider tensor
     w = (torch.randn(N, K, device=DEV) / K ** 0.5).to(torch.bfloat16)
     b = torch.randn(N, device=DEV).to(torch.bfloat16) if epi >= 2 else None
-    y, r = hip.rows_linear(x, w, b, epi), _ref(x, w, b, epi)
+    y, r = hip.rows_linear(x, w, b, epi, wide), _ref(x, w, b, epi)
     # one bf16 rounding (half a step: 2^-8 of the value) of an f32 sum of K products.  SwiGLU: the rounding of the
     # result and of silu(g), and a step (2^-7) of u and of g (silu's relative slope is below 1.3) where a sum
     # lies so near a rounding edge that f32 and f64 fall on different sides: below 7 half steps
@@ -36,13 +37,14 @@ def test_rows_linear(hip, M, N, K, epi):
 
 def test_rows_linear_refuses():
     lib = ops.lib()
-    x, w = torch.zeros(65, 128, device=DEV, dtype=torch.bfloat16), torch.zeros(32, 128, device=DEV, dtype=torch.bfloat16)
+    x, w = torch.zeros(4097, 128, device=DEV, dtype=torch.bfloat16), torch.zeros(32, 128, device=DEV, dtype=torch.bfloat16)
     for bad in ((x, w, None, 0), (x[:4], w[:24], None, 0), (x[:4], w, None, 2), (x[:4, :96], w[:, :96].contiguous(), None, 0)):
         with pytest.raises(RuntimeError):
             lib.rows_linear(*bad)
 
 
-@pytest.mark.parametrize("M,N,K", [(19, 2304, 768), (64, 2048, 2048), (3, 10368, 2048), (64, 10368, 2048), (20, 4096, 14336), (40, 1152, 384)])
+@pytest.mark.parametrize("M,N,K", [(19, 2304, 768), (64, 2048, 2048), (3, 10368, 2048), (64, 10368, 2048), (20, 4096, 14336), (40, 1152, 384),
+                                   (200, 2048, 2048), (700, 2048, 2048), (1000, 768, 768), (1100, 768, 768), (333, 2304, 768)])
 def test_routes_agree(M, N, K):
     """ops.linear / linear_swiglu give the same product whichever kernel the rule names."""
     torch.manual_seed(N)
