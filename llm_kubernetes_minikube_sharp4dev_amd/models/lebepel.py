@@ -65,8 +65,10 @@ class LebepelLayer(nn.Module):
             self.r1, self.r2, self.pb = P(a.heads, **f), P(a.heads, **f), P(a.heads, **f)
         else:
             s = self.spec = Mamba2Spec.from_dict(spec.mixer)
-            # rows [z | x B C | dt], padded with zero rows to the decode GEMMs' 128-column tiles
-            self.in_proj = P(-(-s.proj_out // 128) * 128, W, **e)
+            # rows [z | x B C | dt], padded with zero rows to the GEMMs' 256-column tiles where that adds few (10,368 -> 10,496 rows:
+            # 184 -> 150 us at 4,096 x 2,048), else to the decode GEMMs' 128
+            r128 = -(-s.proj_out // 128) * 128
+            self.in_proj = P(-(-r128 // 256) * 256 if r128 >= 4096 else r128, W, **e)
             self.conv_w, self.conv_b = P(s.conv_channels, s.conv, **f), P(s.conv_channels, **f)
             self.dt_bias, self.A_log, self.D = P(s.heads, **f), P(s.heads, **f), P(s.heads, **f)
             self.mix_norm = P(s.inner, **f)
@@ -107,7 +109,8 @@ class LebepelModel(nn.Module):
     def random_init(self, seed: int = 0, std: float = 0.02):
         gen_dev = self.device if self.device.type == "cuda" else torch.device("cpu")
 
-        def rnd(p, i, scale, shift=0.0):
+        def rnd(p, i, scale, shift=0.0, rows=None):
+            p = p if rows is None else p[:rows]
             g = torch.Generator(device=gen_dev).manual_seed(seed * 7919 + i * 104729)
             p.copy_((torch.randn(p.shape, generator=g, device=gen_dev) * scale + shift).to(p.dtype))
 
@@ -133,8 +136,9 @@ class LebepelModel(nn.Module):
                 rnd(p, i, 0.3)
             elif leaf in ("embed", "pos"):
                 rnd(p, i, 0.5)
-            else:  # projections: unit-variance outputs for unit-variance inputs
-                rnd(p, i, 1.0 / math.sqrt(p.shape[1]))
+            else:  # projections: unit-variance outputs for unit-variance inputs (in_proj: drawn for its rows in whole 128s)
+                L = self.layers[int(name.split(".")[1])] if leaf == "in_proj" else None
+                rnd(p, i, 1.0 / math.sqrt(p.shape[1]), rows=-(-L.spec.proj_out // 128) * 128 if L is not None else None)
         for L in self.layers:
             if L.type == "attention" and (L.spec.dim != L.true.dim or L.spec.vdim != L.true.vdim):
                 a, t = L.spec, L.true

@@ -1147,7 +1147,50 @@ def _cfg_of(M: int, N: int, K: int, epi: int):
             cfg = None
         elif cfg is not None and not SPLIT_ON and cfg[0] in GEMM1W_SPLIT:
             cfg = (3, 256, 1)
-    return cfg if cfg is not None else _gemm_default(M, N, K, epi)
+    return cfg if cfg is not None else _tile_rule(M, N, K, epi)
+
+
+# Shapes without a measured entry, more than 256 rows: gemm1w.hip's 128 / 192 / 256-row tiles against the fallback.  Its
+# one wave of tiles costs 5 us + 0.6 / 0.78 / 1.0 us per 64 columns of K (past K 4096 1.33 / 1.2 / 1.0 of that) however few the
+# tiles are, and the output's stores 0.5 / 0.3 / 0.38 us per MB; gemm.hip's split-K with its reduction 19 + 8 f us and
+# 0.8 + 0.8 f us per 64 columns of a range (f: how much of the chip its workgroups fill), unsplit 8 us + 1.35 us per wave and
+# 64 columns.  Measured, weights cold, fallback / the rule's pick (us):
+#   2048 x 2048: M 640 27.8 / 24.3 (128-row tiles)   M 2048 40.4 / 25.6   M 4096 51.9 / 33.4      3072 x 1024: M 949 27.8 / 15.6
+#   2048 x 5632: M 949 48.1 / same   M 2048 63.0 / same (128-row: 75.5)   M 4096 98.2 / 83.0       3072 x 2048: M 4096 51.1 / 46.7
+#   11264 x 2048 SwiGLU: M 1500 91.6 / 78.1 (192-row tiles)   M 2900 144.8 / 123.3   M 4096 154.6 / same (256-row tiles)
+_TILE_COST = {5: (128, 0.6, 1.33, 0.5), 4: (192, 0.78, 1.2, 0.3), 3: (256, 1.0, 1.0, 0.38)}
+_TILE_RULE: dict = {}
+
+
+def _tile_rule(M: int, N: int, K: int, epi: int):
+    d = _gemm_default(M, N, K, epi)
+    # (past the measured rows a launch is many waves of any tile, where the fallback's larger tiles lead: the encoder's
+    # 62,500-row batches ran 1.6 % longer on this rule's pick)
+    if not GEMM1W or not 256 < M <= 4608 or epi > 4 or K // 64 < 3 or N % 256 or d is None:
+        return d
+    key = (M, N, K, epi, d)
+    if key not in _TILE_RULE:
+        cus, steps = device_cus(), K / 64
+        out_mb = M * (N // 2 if epi == 1 else N) * 2 / 1e6
+
+        def cost(v):
+            bm, c, deep, store = _TILE_COST[v]
+            waves = -(-(-(-M // bm) * (N // 256)) // cus)
+            return 5 + waves * c * (deep if K > 4096 else 1.0) * steps + store * out_mb
+
+        if d[0] in _TILE_COST:
+            other = cost(d[0])
+        elif d[2] > 1:
+            f = min(1.0, -(-M // 256) * (N // d[1]) * d[2] / cus)
+            other = 19 + 8 * f + (0.8 + 0.8 * f) * steps / d[2]
+        else:
+            cols = N // 256 if epi == 1 else N // d[1]
+            other = 8 + 1.35 * steps * -(-(-(-M // 256) * cols) // cus)
+        best = min(_TILE_COST, key=cost)
+        if len(_TILE_RULE) > 4096:
+            _TILE_RULE.clear()
+        _TILE_RULE[key] = (best, 256, 1) if cost(best) < 0.97 * other else d
+    return _TILE_RULE[key]
 
 
 def _resid_cfg(M: int, N: int, K: int):
