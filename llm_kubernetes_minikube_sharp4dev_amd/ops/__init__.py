@@ -783,7 +783,9 @@ def tune_decode(weights, ms: Sequence[int] = DECODE_TUNE_MS, iters: int = 3, col
     for w, swiglu in weights:
         N, K = w.shape
         swiglu = bool(swiglu)
-        copies = [w] + [w.clone() for _ in range(max(1, -(-cold_bytes // (N * K * 2)) - 1))]
+        # (at most 96 launches per graph: weights below 7 MB are then read from the MALL in part, where a launch's chain
+        # and not the memory decides; a thousand captured launches per arm took seconds)
+        copies = [w] + [w.clone() for _ in range(min(95, max(1, -(-cold_bytes // (N * K * 2)) - 1)))]
 
         def timed(fns):
             # as decode steps run: launches of a hipGraph (eager ones of a few microseconds are bound by the
