@@ -2085,30 +2085,42 @@ LatShapes lat_check(const at::Tensor& qa, const at::Tensor& cache, const at::Ten
   return {(int)qa.size(1), (int)qa.size(2), (int)rp, (int)cache.size(1), esz_of(qa, "qa"), fpo(sink, qa.size(1), "sink")};
 }
 
+// sigmoid(gate[row][head]) on a row's averages: rows of H columns aligned with qa's
+void lat_gate_check(const c10::optional<at::Tensor>& gate, const at::Tensor& qa) {
+  if (!gate) return;
+  CHECK_CUDA(*gate); CHECK_LASTDIM((*gate)); same_type(*gate, qa, "gate");
+  TORCH_CHECK(gate->dim() == 2 && gate->size(0) >= qa.size(0) && gate->size(1) >= qa.size(1), "gate [rows, H]");
+}
+
 void latent_attn_prefill(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor& bt, const at::Tensor& cu_q, const at::Tensor& ctx,
-                         int64_t window, double scale, const c10::optional<at::Tensor>& sink, int64_t rp, at::Tensor& out, int64_t max_len) {
+                         int64_t window, double scale, const c10::optional<at::Tensor>& sink, int64_t rp, at::Tensor& out, int64_t max_len,
+                         const c10::optional<at::Tensor>& gate) {
   const LatShapes s = lat_check(qa, cache, bt, ctx, sink, rp, out);
+  lat_gate_check(gate, qa);
   CHECK_CUDA(cu_q); CHECK_I32(cu_q); CHECK_CONTIG(cu_q);
   TORCH_CHECK(cu_q.numel() == ctx.numel() + 1, "cu_q");
   CHECK_RC(lk_latent_attn_prefill(qa.data_ptr(), qa.stride(0), cache.data_ptr(), ip(bt), (int)bt.stride(0), ip(cu_q), ip(ctx), (int)ctx.numel(),
-                                  qa.size(0), s.BS, s.H, s.KD, s.RP, (int)window, (float)scale, s.sink, out.data_ptr(), out.stride(0), s.esz,
+                                  qa.size(0), s.BS, s.H, s.KD, s.RP, (int)window, (float)scale, s.sink, gate ? gate->data_ptr() : nullptr,
+                                  gate ? gate->stride(0) : 0, out.data_ptr(), out.stride(0), s.esz,
                                   cur_stream()), "latent_attn_prefill");
 }
 
 void latent_attn_decode(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor& bt, const at::Tensor& ctx, int64_t window, double scale,
-                        const c10::optional<at::Tensor>& sink, int64_t rp, at::Tensor& out, int64_t splits) {
+                        const c10::optional<at::Tensor>& sink, int64_t rp, at::Tensor& out, int64_t splits, const c10::optional<at::Tensor>& gate) {
   const LatShapes s = lat_check(qa, cache, bt, ctx, sink, rp, out);
+  lat_gate_check(gate, qa);
   TORCH_CHECK(ctx.numel() == qa.size(0) && splits >= 1, "one row per sequence");
   at::Tensor part;
   if (splits > 1) part = at::empty({qa.size(0) * s.H * splits * (rp + 2)}, qa.options().dtype(at::kFloat));
   CHECK_RC(lk_latent_attn_decode(qa.data_ptr(), qa.stride(0), cache.data_ptr(), ip(bt), (int)bt.stride(0), ip(ctx), (int)qa.size(0), (int)splits, s.BS,
-                                 s.H, s.KD, s.RP, (int)window, (float)scale, s.sink, out.data_ptr(), out.stride(0),
+                                 s.H, s.KD, s.RP, (int)window, (float)scale, s.sink, gate ? gate->data_ptr() : nullptr,
+                                 gate ? gate->stride(0) : 0, out.data_ptr(), out.stride(0),
                                  splits > 1 ? part.data_ptr<float>() : nullptr, s.esz, cur_stream()), "latent_attn_decode");
 }
 
 at::Tensor latent_prep(const at::Tensor& u, int64_t dq, int64_t qr, const at::Tensor& wq, int64_t dkv, int64_t R, const c10::optional<at::Tensor>& wkv,
                        int64_t rd, const at::Tensor& freq, const at::Tensor& positions, double eps, at::Tensor& cache, const at::Tensor& slots,
-                       int64_t rp) {
+                       int64_t rp, bool adjacent, double mag) {
   CHECK_CUDA(u); CHECK_LASTDIM(u); CHECK_CUDA(positions); CHECK_I32(positions); CHECK_CUDA(slots); CHECK_I32(slots);
   CHECK_CUDA(cache); CHECK_CONTIG(cache); same_type(cache, u, "cache");
   const long T = u.size(0);
@@ -2118,19 +2130,27 @@ at::Tensor latent_prep(const at::Tensor& u, int64_t dq, int64_t qr, const at::Te
   at::Tensor cq = at::empty({T, qr}, u.options());
   CHECK_RC(lk_latent_prep(u.data_ptr(), u.stride(0), (int)dq, (int)qr, fp(wq, qr, "dq norm"), (int)dkv, (int)R, fpo(wkv, R, "dkv norm"), (int)rd,
                           fp(freq, std::max<int64_t>(rd / 2, 1), "freq"), ip(positions), (float)eps, cache.data_ptr(), ip(slots), (int)rp,
-                          (int)cache.size(2), cq.data_ptr(), cq.stride(0), T, esz_of(u, "u"), cur_stream()), "latent_prep");
+                          (int)cache.size(2), cq.data_ptr(), cq.stride(0), T, adjacent ? 1 : 0, (float)mag,
+                          esz_of(u, "u"), cur_stream()), "latent_prep");
   return cq;
 }
 
-void latent_query_rot(const at::Tensor& q, at::Tensor& qa, int64_t H, int64_t qdim, int64_t dim, int64_t rd, const at::Tensor& freq,
-                      const at::Tensor& positions, int64_t rp) {
+// qa [T, H, KD]: columns rp .. of every row from q's rotated part; with w [H, rp, K] also the columns before, w[h] times the first K of
+// a head's part of q
+void latent_query(const at::Tensor& q, const c10::optional<at::Tensor>& w, at::Tensor& qa, int64_t H, int64_t qdim, int64_t dim, int64_t rd,
+                  const at::Tensor& freq, const at::Tensor& positions, int64_t rp, bool adjacent, double mag) {
   CHECK_CUDA(q); CHECK_LASTDIM(q); CHECK_CUDA(qa); CHECK_LASTDIM(qa); same_type(qa, q, "qa");
   CHECK_CUDA(positions); CHECK_I32(positions);
   TORCH_CHECK(q.dim() == 2 && qa.dim() == 3 && qa.size(0) == q.size(0) && qa.size(1) == H && qa.stride(1) == qa.size(2) && q.size(1) >= H * qdim &&
-                  positions.numel() >= q.size(0), "q [T, H qdim], qa [T, H, KD]");
-  CHECK_RC(lk_latent_query_rot(q.data_ptr(), q.stride(0), qa.data_ptr(), qa.stride(0), (int)H, (int)qdim, (int)dim, (int)rd,
-                               fp(freq, std::max<int64_t>(rd / 2, 1), "freq"), ip(positions), (int)rp, (int)qa.size(2), q.size(0), esz_of(q, "q"),
-                               cur_stream()), "latent_query_rot");
+                  positions.numel() >= q.size(0) && rp >= 0 && rp <= qa.size(2), "q [T, H qdim], qa [T, H, KD]");
+  if (w) {
+    CHECK_CUDA((*w)); CHECK_CONTIG((*w)); same_type(*w, q, "w");
+    TORCH_CHECK(w->dim() == 3 && w->size(0) == H && w->size(1) == rp && w->size(2) <= qdim && w->size(2) > 0, "w [H, rp, K], K <= qdim");
+  }
+  CHECK_RC(lk_latent_query(q.data_ptr(), q.stride(0), qdim, w ? w->data_ptr() : nullptr, (int)H, w ? (int)rp : 0, w ? (int)w->size(2) : 1, q.size(0),
+                           qa.data_ptr(), qa.stride(0), qa.stride(1), (int)qdim, (int)dim, (int)rd, fp(freq, std::max<int64_t>(rd / 2, 1), "freq"),
+                           ip(positions), (int)rp, (int)(qa.size(2) - rp), adjacent ? 1 : 0, (float)mag, esz_of(q, "q"), cur_stream()),
+           "latent_query");
 }
 
 }  // namespace
@@ -2192,7 +2212,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("latent_attn_prefill", &latent_attn_prefill);
   m.def("latent_attn_decode", &latent_attn_decode);
   m.def("latent_prep", &latent_prep);
-  m.def("latent_query_rot", &latent_query_rot);
+  m.def("latent_query", &latent_query);
   m.def("window_mark", [](int64_t id) { CHECK_RC(lk_window_mark((int)id, cur_stream()), "window_mark"); });
   m.def("debug_invalid_launch", []() { CHECK_RC(lk_debug_invalid_launch(cur_stream()), "debug_invalid_launch"); });
   // a HIP stream restricted to the CUs of a bit mask (32 CUs per word): two kernels that

@@ -7,12 +7,17 @@
 //
 // Many rows: a workgroup owns 128 tokens x 128 columns of a head, its 4 waves 64 x 64 quarters; both operands of a 128-byte step of
 // the contraction are fetched once per workgroup (the next step's under this step's products) and staged in LDS, rows padded to
-// 144 bytes.  Few rows, and sizes the vector loads do not divide: fragments straight from memory, a wave owns 16 tokens x 64 columns.
+// 144 bytes.  Few rows, and sizes the vector loads do not divide: head_linear_few_kernel.
+//
+// Rows that are attention queries over a cached latent also get their rotated part (RotTail): few rows in workgroups of the products'
+// launch behind the columns' (they read nothing that it writes), many in a launch of its own.
 #include "common.h"
 #include "kernels.h"
 #include "attn_frag.h"
 
 namespace {
+
+constexpr int kRotMax = 1024;   // rotated elements per head
 
 // the 4 adjacent columns n .. n + 3 of a token's row
 template <typename T>
@@ -30,6 +35,67 @@ LK_DEVICE void store4(T* row, int n, int N, int vst, const floatx4& v) {
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       if (n + j < N) El<T>::st(row + n + j, v[j]);
+  }
+}
+
+// The rotated part of an output row behind its rp columns: the rd elements of the token's input row behind a head's first dim, turned
+// by position (pairs i and i + rd / 2, or neighbours), zeros up to RDP.
+struct RotTail {
+  int dim, rd, rp, RDP, adj;
+  float mag;   // times cos and sin
+  const float* freq;
+  const int* positions;
+};
+
+// the pair d of one row and head, by its angle's cos and sin times the magnitude
+template <typename T>
+LK_DEVICE void rot_pair(const RotTail& p, const T* s, T* o, int d, float cs, float sn) {
+  const int ia = p.adj ? 2 * d : d, ib = p.adj ? 2 * d + 1 : p.rd / 2 + d;
+  const float a = El<T>::ld(s + ia), b = El<T>::ld(s + ib);
+  El<T>::st(o + ia, a * cs - b * sn);
+  El<T>::st(o + ib, b * cs + a * sn);
+}
+
+LK_DEVICE void rot_angle(const RotTail& p, long t, int d, float& cs, float& sn) {
+  sincosf((float)p.positions[t] * p.freq[d], &sn, &cs);
+  cs *= p.mag;
+  sn *= p.mag;
+}
+
+// 16 rows of one head by one workgroup
+template <typename T>
+LK_DEVICE void rot_tail(const RotTail& p, const T* x, long xs, long xh, T* out, long os, long oh, int h, long t0, long rows) {
+  const int half = p.rd / 2, n = half + p.RDP - p.rd;
+  for (int i = threadIdx.x; i < 16 * n; i += 256) {
+    const long t = t0 + i / n;
+    const int d = i % n;
+    if (t >= rows) return;
+    T* o = out + t * os + h * oh + p.rp;
+    if (d >= half) {
+      El<T>::st(o + half + d, 0.f);
+      continue;
+    }
+    float cs, sn;
+    rot_angle(p, t, d, cs, sn);
+    rot_pair<T>(p, x + t * xs + h * xh + p.dim, o, d, cs, sn);
+  }
+}
+
+// Many rows: one workgroup per token, its angles once for all heads (with an angle per head in the products' launch, 4,096 rows of 16
+// heads took 52 us with the products instead of 33.5 + 8.6).
+template <typename T>
+__global__ __launch_bounds__(256) void latent_rot_kernel(const T* __restrict__ x, long xs, long xh, T* __restrict__ out, long os, long oh, int H,
+                                                         RotTail p) {
+  __shared__ float cs[kRotMax / 2], sn[kRotMax / 2];
+  const long t = blockIdx.x;
+  const int half = p.rd / 2, n = half + p.RDP - p.rd;
+  for (int i = threadIdx.x; i < half; i += 256) rot_angle(p, t, i, cs[i], sn[i]);
+  __syncthreads();
+  for (int i = threadIdx.x; i < H * n; i += 256) {
+    const int h = i / n, d = i % n;
+    T* o = out + t * os + (long)h * oh + p.rp;
+    if (d >= half) El<T>::st(o + half + d, 0.f);
+    else rot_pair<T>(p, x + t * xs + (long)h * xh + p.dim, o, d, cs[d], sn[d]);
   }
 }
 
@@ -106,14 +172,24 @@ __global__ __launch_bounds__(256) void head_linear_lds_kernel(const T* __restric
   }
 }
 
-template <typename T, int RT, int WT>
-__global__ __launch_bounds__(256) void head_linear_kernel(const T* __restrict__ x, long xs, long xh, const T* __restrict__ w, int N, int K,
-                                                          long rows, T* __restrict__ out, long os, long oh, int vec, int vst) {
-  constexpr int EV = El<T>::V, STEP = 4 * EV, NT = 4, U = 2;
+// Few rows: a workgroup owns 16 RT tokens x 32 columns of a head, its 4 waves a quarter of the contraction each (steps of 64 bytes in
+// turn), up to 4 steps' fragments requested together straight from memory; the quarters meet in LDS.  At 64 rows the 2 MB of weights are
+// a microsecond of bandwidth, so what counts is the chain of waits per wave: one for K 128, one for K 512 (bf16).  A wave over the whole
+// contraction of 64 columns waited 8 times at K 512 and left 3 of 4 waves idle below 17 rows: 8.8 -> 5.5 us on average over
+// K 128 -> 512 and K 512 -> 128 columns, 16 heads, the rotated part included.
+template <typename T, int RT>
+__global__ __launch_bounds__(256) void head_linear_few_kernel(const T* __restrict__ x, long xs, long xh, const T* __restrict__ w, int N, int K,
+                                                              long rows, T* __restrict__ out, long os, long oh, int vec, int vst, int ncol,
+                                                              RotTail rot) {
+  constexpr int EV = El<T>::V, STEP = 4 * EV, NT = 2, U = 4;
+  __shared__ floatx4 part[4][RT * NT][64];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, n16 = lane & 15, g = lane >> 4;
-  const int h = blockIdx.x, c0 = (blockIdx.y * (4 / WT) + wv / WT) * 16 * NT;
-  const long t0 = ((long)blockIdx.z * WT + wv % WT) * 16 * RT;
-  if (t0 >= rows || c0 >= N) return;   // no barrier in this kernel
+  const int h = blockIdx.x, c0 = blockIdx.y * 16 * NT;
+  const long t0 = (long)blockIdx.z * 16 * RT;
+  if ((int)blockIdx.y >= ncol) {   // the whole workgroup
+    rot_tail<T>(rot, x, xs, xh, out, os, oh, h, t0 + 16 * ((int)blockIdx.y - ncol), rows);
+    return;
+  }
   const T* xr[RT];
 #pragma unroll
   for (int r = 0; r < RT; ++r) xr[r] = x + min(t0 + 16 * r + n16, rows - 1) * xs + h * xh;
@@ -125,42 +201,28 @@ __global__ __launch_bounds__(256) void head_linear_kernel(const T* __restrict__ 
   for (int r = 0; r < RT; ++r)
 #pragma unroll
     for (int c = 0; c < NT; ++c) acc[r][c] = floatx4{0.f, 0.f, 0.f, 0.f};
-  // whole steps as plain vector loads, U of them requested together, the next group's ahead of this group's products
-  int kb = 0;
-  const int groups = vec ? K / (U * STEP) : 0;
-  if (groups > 0) {
-    uint4_t a[2][U][NT], b[2][U][RT];
-    auto load = [&](int p, int k0) {
+  // step i of this wave: elements (4 i + wv) STEP ..; groups of U whole steps as plain vector loads, then one at a time
+  const int whole = vec ? K / STEP : 0, steps = (K + STEP - 1) / STEP;
+  int s = wv;
+  for (; s + 4 * (U - 1) < whole; s += 4 * U) {
+    uint4_t a[U][NT], b[U][RT];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int k = k0 + (4 * u + g) * EV;
+    for (int u = 0; u < U; ++u) {
+      const int k = (s + 4 * u) * STEP + g * EV;
 #pragma unroll
-        for (int c = 0; c < NT; ++c) a[p][u][c] = ld16(wr[c] + k);
+      for (int c = 0; c < NT; ++c) a[u][c] = ld16(wr[c] + k);
 #pragma unroll
-        for (int r = 0; r < RT; ++r) b[p][u][r] = ld16(xr[r] + k);
-      }
-    };
-    auto mul = [&](int p) {
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-#pragma unroll
-        for (int r = 0; r < RT; ++r)
-#pragma unroll
-          for (int c = 0; c < NT; ++c) acc[r][c] = mma_qk<T>(a[p][u][c], b[p][u][r], acc[r][c]);
-    };
-    load(0, 0);
-    for (int i = 0; i < groups; i += 2) {
-      if (i + 1 < groups) load(1, (i + 1) * U * STEP);
-      mul(0);
-      if (i + 1 < groups) {
-        if (i + 2 < groups) load(0, (i + 2) * U * STEP);
-        mul(1);
-      }
+      for (int r = 0; r < RT; ++r) b[u][r] = ld16(xr[r] + k);
     }
-    kb = groups * U * STEP;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int c = 0; c < NT; ++c) acc[r][c] = mma_qk<T>(a[u][c], b[u][r], acc[r][c]);
   }
-  for (; kb < K; kb += STEP) {
-    const int k = kb + g * EV;
+  for (; s < steps; s += 4) {
+    const int k = s * STEP + g * EV;
     uint4_t a[NT], b[RT];
 #pragma unroll
     for (int c = 0; c < NT; ++c) a[c] = frag<T>(wr[c], k, K, vec);
@@ -171,32 +233,51 @@ __global__ __launch_bounds__(256) void head_linear_kernel(const T* __restrict__ 
 #pragma unroll
       for (int c = 0; c < NT; ++c) acc[r][c] = mma_qk<T>(a[c], b[r], acc[r][c]);
   }
-  // accumulator j of this lane: output column 16 c + 4 g + j of token 16 r + n16
 #pragma unroll
-  for (int r = 0; r < RT; ++r) {
-    const long t = t0 + 16 * r + n16;
-    if (t >= rows) continue;
-    T* orow = out + t * os + h * oh;
+  for (int r = 0; r < RT; ++r)
 #pragma unroll
-    for (int c = 0; c < NT; ++c) store4<T>(orow, c0 + 16 * c + 4 * g, N, vst, acc[r][c]);
+    for (int c = 0; c < NT; ++c) part[wv][r * NT + c][lane] = acc[r][c];
+  __syncthreads();
+  // tile i = (r, c): accumulator j of a lane is output column 16 c + 4 g + j of token 16 r + n16
+  for (int i = wv; i < RT * NT; i += 4) {
+    floatx4 v = part[0][i][lane];
+#pragma unroll
+    for (int q = 1; q < 4; ++q) {
+      const floatx4 o = part[q][i][lane];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] += o[j];
+    }
+    const long t = t0 + 16 * (i / NT) + n16;
+    if (t < rows) store4<T>(out + t * os + h * oh, c0 + 16 * (i % NT) + 4 * g, N, vst, v);
   }
 }
 
 template <typename T>
 int head_linear_t(const void* x, long xs, long xh, const void* w, int H, int N, int K, long rows, void* out, long os, long oh, int vec, int vst,
-                  hipStream_t st) {
-  if (rows > 65535L * 64) return -1;
-#define LK_HEAD(RT, WT)                                                                                                                      \
-  head_linear_kernel<T, RT, WT><<<dim3((unsigned)H, (unsigned)((N + 64 * (4 / WT) - 1) / (64 * (4 / WT))),                                   \
-                                       (unsigned)((rows + 16 * RT * WT - 1) / (16 * RT * WT))), 256, 0, st>>>(                              \
-      (const T*)x, xs, xh, (const T*)w, N, K, rows, (T*)out, os, oh, vec, vst)
-  if (rows > 128 && vec)
+                  const RotTail& rot, hipStream_t st) {
+  if (N > 0 && rows > 65535L * 64) return -1;
+  const bool fused = rot.RDP > 0 && N > 0 && rows <= 128;
+  const int tail = fused ? 1 : 0;   // workgroups of 16 rows each behind the columns'
+#define LK_HEAD(RT)                                                                                                                          \
+  head_linear_few_kernel<T, RT><<<dim3((unsigned)H, (unsigned)((N + 31) / 32 + tail * RT), (unsigned)((rows + 16 * RT - 1) / (16 * RT))),    \
+                                  256, 0, st>>>((const T*)x, xs, xh, (const T*)w, N, K, rows, (T*)out, os, oh, vec, vst, (N + 31) / 32, rot)
+  if (N == 0)
+    ;
+  else if (rows > 128 && vec)
     head_linear_lds_kernel<T><<<dim3((unsigned)H, (unsigned)((N + 127) / 128), (unsigned)((rows + 127) / 128)), 256, 0, st>>>(
         (const T*)x, xs, xh, (const T*)w, N, K, rows, (T*)out, os, oh, vst);
+  else if (rows <= 16)
+    LK_HEAD(1);
+  else if (rows <= 32)
+    LK_HEAD(2);
   else
-    LK_HEAD(1, 4);
+    LK_HEAD(4);
 #undef LK_HEAD
   LK_CHECK_LAUNCH();
+  if (rot.RDP > 0 && !fused) {
+    latent_rot_kernel<T><<<(unsigned)rows, 256, 0, st>>>((const T*)x, xs, xh, (T*)out, os, oh, H, rot);
+    LK_CHECK_LAUNCH();
+  }
   return 0;
 }
 
@@ -204,12 +285,21 @@ int head_linear_t(const void* x, long xs, long xh, const void* w, int H, int N, 
 
 int lk_head_linear(const void* x, long xs, long xh, const void* w, int H, int N, int K, long rows, void* out, long os, long oh, int esz,
                    hipStream_t st) {
+  if (N < 1 || K < 1) return rows <= 0 ? 0 : -1;
+  return lk_latent_query(x, xs, xh, w, H, N, K, rows, out, os, oh, 0, 0, 0, nullptr, nullptr, 0, 0, 0, 1.f, esz, st);
+}
+
+// N 0: the rotated part alone
+int lk_latent_query(const void* x, long xs, long xh, const void* w, int H, int N, int K, long rows, void* out, long os, long oh, int qdim, int dim,
+                    int rd, const float* freq, const int* positions, int rp, int RDP, int adj, float mag, int esz, hipStream_t st) {
   if (rows <= 0) return 0;
-  if (H < 1 || H > 65535 || N < 1 || K < 1 || (N + 63) / 64 > 65535) return -1;
+  if (H < 1 || H > 65535 || N < 0 || (N > 0 && K < 1) || (N + 31) / 32 > 65000) return -1;
+  if (rd < 0 || rd % 2 || rd > kRotMax || dim < 0 || dim + rd > qdim || rd > RDP || N > (RDP > 0 ? rp : N) || (rd > 0 && (!freq || !positions))) return -1;
   const int ev = 16 / esz;
   const auto a16 = [](const void* p, int b) { return reinterpret_cast<uintptr_t>(p) % b == 0; };
   const int vec = K % ev == 0 && xs % ev == 0 && xh % ev == 0 && a16(x, 16) && a16(w, 16);
   const int vst = os % 4 == 0 && oh % 4 == 0 && a16(out, 4 * esz);
-  return esz == 2 ? head_linear_t<bf16_t>(x, xs, xh, w, H, N, K, rows, out, os, oh, vec, vst, st)
-                  : head_linear_t<float>(x, xs, xh, w, H, N, K, rows, out, os, oh, vec, vst, st);
+  const RotTail rot{dim, rd, rp, RDP, adj, mag, freq, positions};
+  return esz == 2 ? head_linear_t<bf16_t>(x, xs, xh, w, H, N, K, rows, out, os, oh, vec, vst, rot, st)
+                  : head_linear_t<float>(x, xs, xh, w, H, N, K, rows, out, os, oh, vec, vst, rot, st);
 }

@@ -384,16 +384,19 @@ int lk_mlstm_chunk_min();
 // csrc/head_linear.hip: out[t, h, :N] = w[h] x[t, h xh : h xh + K]
 int lk_head_linear(const void* x, long xs, long xh, const void* w, int H, int N, int K, long rows, void* out, long os, long oh, int esz,
                    hipStream_t st);
+// the same, and behind column rp of every output row RDP columns: x's rd elements behind a head's first dim, rotated, then zeros
+// (N 0: only those)
+int lk_latent_query(const void* x, long xs, long xh, const void* w, int H, int N, int K, long rows, void* out, long os, long oh, int qdim, int dim,
+                    int rd, const float* freq, const int* positions, int rp, int RDP, int adj, float mag, int esz, hipStream_t st);
 
 // csrc/latent_attn.hip: attention over a cached latent shared by all heads (cache [blocks, BS, KD], row = latent | rotated part) and
 // the preparation of its operands
 int lk_latent_attn_prefill(const void* q, long qs, const void* cache, const int* bt, int bt_stride, const int* cu_q, const int* ctx_lens, int nseq,
-                           long rows, int BS, int H, int KD, int RP, int window, float scale, const float* sink, void* out, long os, int esz,
-                           hipStream_t st);
+                           long rows, int BS, int H, int KD, int RP, int window, float scale, const float* sink, const void* gate, long gs,
+                           void* out, long os, int esz, hipStream_t st);
 int lk_latent_attn_decode(const void* q, long qs, const void* cache, const int* bt, int bt_stride, const int* ctx_lens, int B, int Z, int BS, int H,
-                          int KD, int RP, int window, float scale, const float* sink, void* out, long os, float* part, int esz, hipStream_t st);
+                          int KD, int RP, int window, float scale, const float* sink, const void* gate, long gs, void* out, long os,
+                          float* part, int esz, hipStream_t st);
 int lk_latent_prep(const void* u, long us, int dq, int qr, const float* wq, int dkv, int R, const float* wkv, int rd, const float* freq,
-                   const int* positions, float eps, void* cache, const int* slots, int RP, int KD, void* cq, long cqs, long rows, int esz,
-                   hipStream_t st);
-int lk_latent_query_rot(const void* q, long qs, void* qa, long as, int H, int qdim, int dim, int rd, const float* freq, const int* positions, int RP,
-                        int KD, long rows, int esz, hipStream_t st);
+                   const int* positions, float eps, void* cache, const int* slots, int RP, int KD, void* cq, long cqs, long rows, int adj, float mag,
+                   int esz, hipStream_t st);

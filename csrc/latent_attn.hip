@@ -20,7 +20,7 @@
 //
 // Masks are taken from absolute positions: a prompt cut anywhere, a decode row and a whole prompt are the same sums.
 //
-// lk_latent_prep / lk_latent_query_rot prepare the operands (norms, rotation in halves, the cache row) in f32.
+// lk_latent_prep prepares the operands (norms, rotation, the cache row) in f32; the queries come from head_linear.hip.
 #include <type_traits>
 
 #include "common.h"
@@ -47,7 +47,16 @@ struct LatParams {
   const float* sink;   // [H] or null
   void* out;           // [rows, H, RP]
   long os;
+  const void* gate;    // rows aligned with q's: the averages of head h times sigmoid(column h); null: none
+  long gs;
 };
+
+template <typename T>
+LK_DEVICE float lat_gate(const LatParams& p, long row, int head) {
+  if (!p.gate) return 1.f;
+  const float g = El<T>::ld(reinterpret_cast<const T*>(p.gate) + row * p.gs + head);
+  return sizeof(T) == 4 ? 1.f / (1.f + expf(-g)) : __builtin_amdgcn_rcpf(1.f + __expf(-g));
+}
 
 LK_DEVICE int first_key(int qpos, int window) { return window > 0 ? max(0, qpos - window + 1) : 0; }
 
@@ -311,7 +320,7 @@ __global__ __launch_bounds__(pre_waves<RP>() * 64, RP >= 256 ? 1 : 2) void lat_p
     const int c = 16 * (CG * w + x) + n16, qi = q0 + c / p.HC, head = blockIdx.y * p.HC + c % p.HC;
     if (qpos[x] >= 0) {
       if (p.sink) l[x] += __builtin_amdgcn_exp2f(p.sink[head] * kLog2e - m[x]);   // one more term without a value
-      const float f = l[x] > 0.f ? 1.f / l[x] : 0.f;
+      const float f = l[x] > 0.f ? lat_gate<bf16_t>(p, qbeg + qi, head) / l[x] : 0.f;
       bf16_t* orow = reinterpret_cast<bf16_t*>(p.out) + (long)(qbeg + qi) * p.os + (long)head * RP + 4 * g;
 #pragma unroll
       for (int vt = 0; vt < VT; ++vt) {
@@ -392,7 +401,7 @@ __global__ __launch_bounds__(256) void lat_decode_kernel(LatParams p, const int*
 #pragma unroll
   for (int vt = 0; vt < VT; ++vt) ob[vt * 64 + lane] = floatx4{o[0][vt][0] * f, o[0][vt][1] * f, o[0][vt][2] * f, o[0][vt][3] * f};
   __syncthreads();
-  const float inv = L > 0.f ? 1.f / L : 0.f;
+  const float inv = L > 0.f ? lat_gate<bf16_t>(p, b, min(head, p.H - 1)) / L : 0.f;
 #pragma unroll
   for (int i = 0; i < VT / 4; ++i) {
     const int vt = 4 * i + w;
@@ -423,17 +432,30 @@ __global__ __launch_bounds__(256) void lat_decode_kernel(LatParams p, const int*
   }
 }
 
+// One workgroup per (sequence, head), two columns per thread.  A chain of three waits (maxima, sums, averages): the splits' maxima and
+// sums are read by the lanes side by side and the averages four splits at a time; one split after the other it took 6.5 us at 64 x 16
+// rows of 512 columns in 4 splits, 4.7 now.
 __global__ __launch_bounds__(256) void lat_reduce_kernel(LatParams p, const float* __restrict__ part, int Z) {
-  const int b = blockIdx.x, head = blockIdx.y, RP = p.RP;
+  const int b = blockIdx.x, head = blockIdx.y, RP = p.RP, lane = threadIdx.x & 63;
   const float* pp = part + ((long)b * p.H + head) * Z * (RP + 2);
+  const float gate = lat_gate<bf16_t>(p, b, head);
   float M = kNegBig, L = 0.f;
-  for (int z = 0; z < Z; ++z) M = fmaxf(M, pp[(long)z * (RP + 2) + RP]);
-  for (int z = 0; z < Z; ++z) L += pp[(long)z * (RP + 2) + RP + 1] * __builtin_amdgcn_exp2f(pp[(long)z * (RP + 2) + RP] - M);
-  const float inv = L > 0.f ? 1.f / L : 0.f;
-  for (int d = threadIdx.x; d < RP; d += 256) {
-    float s = 0.f;
-    for (int z = 0; z < Z; ++z) s += pp[(long)z * (RP + 2) + d] * __builtin_amdgcn_exp2f(pp[(long)z * (RP + 2) + RP] - M);
-    reinterpret_cast<bf16_t*>(p.out)[(long)b * p.os + (long)head * RP + d] = f2bf(s * inv);
+  for (int z = lane; z < Z; z += 64) M = fmaxf(M, pp[(long)z * (RP + 2) + RP]);
+  M = wave_max(M);
+  for (int z = lane; z < Z; z += 64) L += pp[(long)z * (RP + 2) + RP + 1] * __builtin_amdgcn_exp2f(pp[(long)z * (RP + 2) + RP] - M);
+  L = wave_sum(L);
+  const float inv = L > 0.f ? gate / L : 0.f;
+  for (int d = 2 * threadIdx.x; d < RP; d += 512) {
+    float s0 = 0.f, s1 = 0.f;
+#pragma unroll 4
+    for (int z = 0; z < Z; ++z) {
+      const float* q = pp + (long)z * (RP + 2);
+      const float2 v = *reinterpret_cast<const float2*>(q + d);
+      const float e = __builtin_amdgcn_exp2f(q[RP] - M);
+      s0 += v.x * e;
+      s1 += v.y * e;
+    }
+    *reinterpret_cast<unsigned*>(reinterpret_cast<bf16_t*>(p.out) + (long)b * p.os + (long)head * RP + d) = pack_bf2(s0 * inv, s1 * inv);
   }
 }
 
@@ -505,7 +527,7 @@ __global__ __launch_bounds__(256) void lat_plain_kernel(LatParams p, const int* 
       }
     }
   }
-  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const float inv = l > 0.f ? lat_gate<T>(p, row, head) / l : 0.f;
 #pragma unroll
   for (int i = 0; i < kPlainDims; ++i) {
     const int d = tid + 256 * i;
@@ -530,6 +552,8 @@ struct PrepParams {
   int RP, KD;
   void* cq;
   long cqs;
+  int adj;             // pairs (2 i, 2 i + 1) instead of (i, i + rd / 2)
+  float mag;           // times cos and sin
 };
 
 // One workgroup per token: both root mean squares in one pass over the row, the normed query latent, the cache row.
@@ -565,36 +589,14 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(PrepParams p) {
   for (int i = tid; i < half; i += 256) {
     float sn, cs;
     sincosf(pos * p.freq[i], &sn, &cs);
-    const float a = El<T>::ld(ukv + p.R + i), b = El<T>::ld(ukv + p.R + half + i);
-    El<T>::st(row + p.RP + i, a * cs - b * sn);
-    El<T>::st(row + p.RP + half + i, b * cs + a * sn);
+    cs *= p.mag;
+    sn *= p.mag;
+    const int ia = p.adj ? 2 * i : i, ib = p.adj ? 2 * i + 1 : half + i;
+    const float a = El<T>::ld(ukv + p.R + ia), b = El<T>::ld(ukv + p.R + ib);
+    El<T>::st(row + p.RP + ia, a * cs - b * sn);
+    El<T>::st(row + p.RP + ib, b * cs + a * sn);
   }
   for (int c = p.RP + p.rd + tid; c < p.KD; c += 256) El<T>::st(row + c, 0.f);
-}
-
-constexpr int kRotMax = 1024;
-
-// One workgroup per token: cos and sin once per pair, then every head's rotated columns.
-template <typename T>
-__global__ __launch_bounds__(256) void latent_query_rot_kernel(const T* __restrict__ q, long qs, T* __restrict__ qa, long as, int H, int qdim,
-                                                               int dim, int rd, const float* __restrict__ freq,
-                                                               const int* __restrict__ positions, int RP, int KD) {
-  __shared__ float cs[kRotMax / 2], sn[kRotMax / 2];
-  const long t = blockIdx.x;
-  const int half = rd / 2, RDP = KD - RP;
-  const float pos = (float)positions[t];
-  for (int i = threadIdx.x; i < half; i += 256) sincosf(pos * freq[i], &sn[i], &cs[i]);
-  __syncthreads();
-  for (int x = threadIdx.x; x < H * RDP; x += 256) {
-    const int h = x / RDP, d = x % RDP;
-    float v = 0.f;
-    if (d < rd) {
-      const T* s = q + t * qs + (long)h * qdim + dim;
-      v = d < half ? El<T>::ld(s + d) * cs[d] - El<T>::ld(s + half + d) * sn[d]
-                   : El<T>::ld(s + d) * cs[d - half] + El<T>::ld(s + d - half) * sn[d - half];
-    }
-    El<T>::st(qa + t * as + (long)h * KD + RP + d, v);
-  }
 }
 
 bool mfma_shape(int RP, int KD) {
@@ -655,7 +657,8 @@ int run_plain(const LatParams& p, const int* cu_q, const int* ctx, int nseq, lon
 }
 
 bool make_params(LatParams& p, const void* q, long qs, const void* cache, const int* bt, int bt_stride, int BS, int H, int KD, int RP, int window,
-                 float scale, const float* sink, void* out, long os, int esz) {
+                 float scale, const float* sink, const void* gate, long gs, void* out, long os, int esz) {
+  p.gate = gate; p.gs = gs;
   p.q = q; p.qs = qs; p.cache = cache; p.bt = bt; p.bt_stride = bt_stride; p.BS = BS; p.H = H; p.KD = KD; p.RP = RP; p.window = window;
   p.scale = scale; p.sink = sink; p.out = out; p.os = os;
   const int blocks = (H + 15) / 16;
@@ -668,20 +671,21 @@ bool make_params(LatParams& p, const void* q, long qs, const void* cache, const 
 }  // namespace
 
 int lk_latent_attn_prefill(const void* q, long qs, const void* cache, const int* bt, int bt_stride, const int* cu_q, const int* ctx_lens, int nseq,
-                           long rows, int BS, int H, int KD, int RP, int window, float scale, const float* sink, void* out, long os, int esz,
-                           hipStream_t st) {
+                           long rows, int BS, int H, int KD, int RP, int window, float scale, const float* sink, const void* gate, long gs,
+                           void* out, long os, int esz, hipStream_t st) {
   if (rows <= 0 || nseq <= 0) return 0;
   LatParams p;
-  if (!make_params(p, q, qs, cache, bt, bt_stride, BS, H, KD, RP, window, scale, sink, out, os, esz)) return -1;
+  if (!make_params(p, q, qs, cache, bt, bt_stride, BS, H, KD, RP, window, scale, sink, gate, gs, out, os, esz)) return -1;
   if (esz == 2 && mfma_shape(RP, KD)) return run_prefill(p, cu_q, ctx_lens, nseq, rows, st);
   return esz == 2 ? run_plain<bf16_t>(p, cu_q, ctx_lens, nseq, rows, st) : run_plain<float>(p, cu_q, ctx_lens, nseq, rows, st);
 }
 
 int lk_latent_attn_decode(const void* q, long qs, const void* cache, const int* bt, int bt_stride, const int* ctx_lens, int B, int Z, int BS, int H,
-                          int KD, int RP, int window, float scale, const float* sink, void* out, long os, float* part, int esz, hipStream_t st) {
+                          int KD, int RP, int window, float scale, const float* sink, const void* gate, long gs, void* out, long os,
+                          float* part, int esz, hipStream_t st) {
   if (B <= 0) return 0;
   LatParams p;
-  if (!make_params(p, q, qs, cache, bt, bt_stride, BS, H, KD, RP, window, scale, sink, out, os, esz)) return -1;
+  if (!make_params(p, q, qs, cache, bt, bt_stride, BS, H, KD, RP, window, scale, sink, gate, gs, out, os, esz)) return -1;
   if (esz == 2 && mfma_shape(RP, KD)) {
     if (Z < 1 || Z > 65535 || (Z > 1 && !part)) return -1;
     return run_decode(p, ctx_lens, B, Z, part, st);
@@ -690,27 +694,15 @@ int lk_latent_attn_decode(const void* q, long qs, const void* cache, const int* 
 }
 
 int lk_latent_prep(const void* u, long us, int dq, int qr, const float* wq, int dkv, int R, const float* wkv, int rd, const float* freq,
-                   const int* positions, float eps, void* cache, const int* slots, int RP, int KD, void* cq, long cqs, long rows, int esz,
-                   hipStream_t st) {
+                   const int* positions, float eps, void* cache, const int* slots, int RP, int KD, void* cq, long cqs, long rows, int adj, float mag,
+                   int esz, hipStream_t st) {
   if (rows <= 0) return 0;
   if (qr < 1 || !wq || (wkv && (R < 1 || R > RP || rd < 0 || rd % 2 || RP + rd > KD || !cache || !slots || (rd > 0 && !freq)))) return -1;
   PrepParams p;
   p.u = u; p.us = us; p.dq = dq; p.qr = qr; p.wq = wq; p.dkv = dkv; p.R = R; p.wkv = wkv; p.rd = rd; p.freq = freq; p.positions = positions;
-  p.eps = eps; p.cache = cache; p.slots = slots; p.RP = RP; p.KD = KD; p.cq = cq; p.cqs = cqs;
+  p.eps = eps; p.cache = cache; p.slots = slots; p.RP = RP; p.KD = KD; p.cq = cq; p.cqs = cqs; p.adj = adj; p.mag = mag;
   if (esz == 2) latent_prep_kernel<bf16_t><<<(unsigned)rows, 256, 0, st>>>(p);
   else latent_prep_kernel<float><<<(unsigned)rows, 256, 0, st>>>(p);
-  LK_CHECK_LAUNCH();
-  return 0;
-}
-
-int lk_latent_query_rot(const void* q, long qs, void* qa, long as, int H, int qdim, int dim, int rd, const float* freq, const int* positions, int RP,
-                        int KD, long rows, int esz, hipStream_t st) {
-  if (rows <= 0) return 0;
-  if (H < 1 || rd < 0 || rd % 2 || rd > kRotMax || dim < 0 || dim + rd > qdim || RP + rd > KD || (rd > 0 && !freq)) return -1;
-  if (esz == 2)
-    latent_query_rot_kernel<bf16_t><<<(unsigned)rows, 256, 0, st>>>((const bf16_t*)q, qs, (bf16_t*)qa, as, H, qdim, dim, rd, freq, positions, RP, KD);
-  else
-    latent_query_rot_kernel<float><<<(unsigned)rows, 256, 0, st>>>((const float*)q, qs, (float*)qa, as, H, qdim, dim, rd, freq, positions, RP, KD);
   LK_CHECK_LAUNCH();
   return 0;
 }

@@ -85,10 +85,24 @@ class _LatentAttention(nn.Module):
         self.o = _p(W, H * s.vdim_p, **e)
         self.freq = _p(max(s.rot_dim // 2, 1), **f)
         self.hscale = _p(H, **f)
+        s.absorbed = s.absorb(e["dtype"], e["device"])
+        # the up projections by head, for attention on the cached latent; derived from w_ukv by init_constants
+        rp = ops.latent_row(s.kv_rank, s.rot_dim)[0]
+        self.register_buffer("w_uk_t", torch.zeros(H, rp, _pad8(s.dim), **e) if s.absorbed else None, persistent=False)
+        self.register_buffer("w_uv_h", torch.zeros(H, s.vdim_p, rp, **e) if s.absorbed else None, persistent=False)
 
     def init_constants(self):
-        self.freq.copy_(self.spec.rot.freq_tensor(self.freq.device))
-        self.hscale.fill_(self.spec.scale)
+        s = self.spec
+        self.freq.copy_(s.rot.freq_tensor(self.freq.device))
+        self.hscale.fill_(s.scale)
+        if s.absorbed:
+            uv = self.up_rows.off["uv"]
+            self.w_uk_t[:, :s.kv_rank, :s.dim].copy_(self.w_ukv[:s.heads * s.dim].view(s.heads, s.dim, s.kv_rank).transpose(1, 2))
+            self.w_uv_h[:, :, :s.kv_rank].copy_(self.w_ukv[uv:uv + s.heads * s.vdim_p].view(s.heads, s.vdim_p, s.kv_rank))
+
+    @property
+    def w_heads(self):
+        return self.w_uk_t, self.w_uv_h
 
 
 class _TableExperts(nn.Module):
@@ -272,7 +286,10 @@ class FusasunModel(nn.Module):
         seen, out = set(), []
         for L in self.layers:
             M = L.mix
-            ws = [L.rg1, M.w_in, M.o] + ([M.w_uq, M.w_ukv] if L.type == "latent_attention" else []) + ([L.rg2] if L.mlp is not None else [])
+            ws = [L.rg1, M.w_in, M.o]
+            if L.type == "latent_attention":
+                ws += [M.w_uq] if M.spec.absorbed else [M.w_uq, M.w_ukv]
+            ws += [L.rg2] if L.mlp is not None else []
             for w in ws:
                 if tuple(w.shape) not in seen:
                     seen.add(tuple(w.shape))
@@ -317,7 +334,7 @@ class FusasunModel(nn.Module):
             att = pooled_window_attention(u, cache, meta, M.spec, M.freq, M.hscale)
         else:
             att = latent_window_attention(u, M.rows, M.up_rows.off["uv"], M.w_uq, M.w_ukv, M.dq_norm, M.dkv_norm, cache, meta, M.spec, M.freq,
-                                          M.hscale, self.cfg.norm_eps)
+                                          M.hscale, self.cfg.norm_eps, w_heads=M.w_heads)
         return ops.linear(att, M.o)
 
     def forward(self, ids: torch.Tensor, meta: AttnMeta, caches, taps: list = None) -> torch.Tensor:

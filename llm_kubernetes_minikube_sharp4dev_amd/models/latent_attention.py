@@ -94,8 +94,7 @@ def cached_latent_attention(h, w_in, rows: FusedRows, w_uq, w_uk, w_uv, dq_norm,
                          meta.positions, eps, cache, meta.slots, rp)
     q = ops.linear(cq, w_uq)
     qa = torch.empty(T, H, rp + rdp, dtype=u.dtype, device=u.device)
-    ops.head_linear(q, w_uk, spec.qdim, qa)
-    ops.latent_query_rot(q, qa, H, spec.qdim, spec.dim, spec.rot_dim, freq, meta.positions, rp)
+    ops.latent_query(q, w_uk, qa, spec.qdim, spec.dim, spec.rot_dim, freq, meta.positions, rp)
     lat = torch.empty(T, H, rp, dtype=u.dtype, device=u.device)
     Tp, Bd = meta.num_prefill_tokens, meta.num_decode
     if Tp:

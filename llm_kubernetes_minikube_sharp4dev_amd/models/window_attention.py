@@ -246,8 +246,7 @@ class LatentAttnSpec:
     rotated key segment common to the heads; per head key ``[W_uk c | common segment]``, value ``W_uv c``; sliding
     window (``window`` 0: causal); the output times ``sigmoid(W_g h)``, one gate per head or (``gate_elem``) one
     per output element.  The cache holds the expanded keys and values
-    (``heads`` key / value heads): a sliding window bounds what a decoded token reads, and scores against
-    the latent would cost ``kv_rank / dim`` times the products."""
+    (``heads`` key / value heads), or with ``absorbed`` (:meth:`absorb`) one latent row per token for all heads."""
     heads: int
     dim: int
     rot_dim: int
@@ -258,6 +257,20 @@ class LatentAttnSpec:
     window: int
     rot: RotarySpec = field(default_factory=RotarySpec)
     gate_elem: bool = False
+    absorbed: bool = False
+
+    def absorb(self, dtype, device) -> bool:
+        """Whether scores and averages run on the cached latent (``ops.latent``; queries through ``W_uk^T`` once, the averages
+        through ``W_uv`` afterwards): bf16 on the GPU, where its matrix kernels take the row's size, for a sliding window (prompt rows
+        then cost alike at every length), where a token's row is at most a quarter of its expanded heads and the products per key at
+        most 3.5 times theirs.  One mixer, expanded -> cached latent, at 1,024 positions, in us for 4,096 prompt rows / 64 / 4
+        decoded: 16 heads of 128 + 64 / 128, rank 512 (3.4 times the products), window 512: 336 / 138 / 41 -> 314 / 61 / 39; 32 heads,
+        window 2,048: 732 / 401 / 67 -> 593 / 78 / 47; 16 heads of 64 + 32 / 64, rank 128 (2 times): 155 / 47 / 29 -> 137 / 35 / 27;
+        rank 256 (3.6 times, beyond the line): 193 / 70 / 32 -> 205 / 47 / 32."""
+        rp, rdp = ops.latent_row(self.kv_rank, self.rot_dim)
+        return (dtype == torch.bfloat16 and torch.device(device).type == "cuda" and self.window > 0 and not self.gate_elem
+                and self.rot_dim > 0 and rp in (128, 256, 512) and rdp in (64, 128)
+                and self.heads * (self.kdim + self.vdim_p) >= 4 * (rp + rdp) and 2 * (2 * rp + rdp) <= 7 * (self.kdim + self.vdim_p))
 
     @classmethod
     def from_dict(cls, m: dict, gate_elem: bool = False, causal_ok: bool = False) -> "LatentAttnSpec":
@@ -286,22 +299,53 @@ class LatentAttnSpec:
         return _pad8(self.vdim)
 
     def make_caches(self, num_blocks: int, block_size: int, dtype, device) -> tuple:
+        if self.absorbed:
+            return (torch.zeros(num_blocks, block_size, sum(ops.latent_row(self.kv_rank, self.rot_dim)), dtype=dtype, device=device),)
         return _cache_pair(num_blocks, self.heads, block_size, self.kdim, self.vdim_p, dtype, device)
 
     def bytes_per_token(self, dtype) -> int:
+        if self.absorbed:
+            return sum(ops.latent_row(self.kv_rank, self.rot_dim)) * torch.tensor([], dtype=dtype).element_size()
         return self.heads * (self.kdim + self.vdim_p) * torch.tensor([], dtype=dtype).element_size()
 
 
+def _absorbed_attention(u, rows, w_uq, w_heads, dq_norm, dkv_norm, cache, meta: AttnMeta, spec: LatentAttnSpec, freq, eps: float, out):
+    """:func:`latent_window_attention` on a cached latent."""
+    H, T = spec.heads, u.shape[0]
+    rp, rdp = ops.latent_row(spec.kv_rank, spec.rot_dim)
+    mag = spec.rot.magnitude
+    cq = ops.latent_prep(u, rows.off["dq"], spec.q_rank, dq_norm, rows.off["dkv"], spec.kv_rank, dkv_norm, spec.rot_dim, freq, meta.positions,
+                         eps, cache, meta.slots, rp, adjacent=True, mag=mag)
+    q = ops.linear(cq, w_uq)
+    qa = torch.empty(T, H, rp + rdp, dtype=u.dtype, device=u.device)
+    ops.latent_query(q, w_heads[0], qa, spec.kdim, spec.dim, spec.rot_dim, freq, meta.positions, rp, adjacent=True, mag=mag)
+    lat = torch.empty(T, H, rp, dtype=u.dtype, device=u.device)
+    gate = u[:, rows.off["g"]:rows.off["g"] + H]
+    Tp, Bd = meta.num_prefill_tokens, meta.num_decode
+    if Tp:
+        ops.latent_attention_prefill(qa[:Tp], cache, meta.block_tables_p, meta.cu_q, meta.ctx_lens_p, spec.window, spec.scale, None, rp,
+                                     lat[:Tp], max(meta.q_lens_cpu), gate=gate[:Tp])
+    if Bd:
+        span = meta.block_tables_d.shape[1] * cache.shape[1]
+        ops.latent_attention_decode(qa[Tp:Tp + Bd], cache, meta.block_tables_d, meta.ctx_lens_d, spec.window, spec.scale, None, rp,
+                                    lat[Tp:Tp + Bd], splits=ops.latent_decode_splits(Bd, H, min(span, spec.window)), gate=gate[Tp:Tp + Bd])
+    ops.head_linear(lat.view(T, H * rp), w_heads[1], rp, out.view(T, H, spec.vdim_p))
+    return out
+
+
 def latent_window_attention(u, rows, uv_col: int, w_uq, w_ukv, dq_norm, dkv_norm, caches, meta: AttnMeta, spec: LatentAttnSpec, freq, hscale,
-                            eps: float, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+                            eps: float, out: Optional[torch.Tensor] = None, w_heads=None) -> torch.Tensor:
     """u [T, dq | dkv | g] = the fused down projections of the mixer's input (``rows``: their column layout).
     ``w_uq`` [H kdim, q_rank] (zero rows behind every head's dim + rot_dim), ``w_ukv`` = [W_uk ; W_uv] with
-    the value rows starting at row ``uv_col`` (a multiple of 8)."""
+    the value rows starting at row ``uv_col`` (a multiple of 8); an absorbed ``spec`` takes ``w_heads`` = (W_uk transposed
+    per head [H, RP, dim padded to 8], W_uv [H, vdim_p, RP]) instead."""
     H, dim, rd, vdim = spec.heads, spec.dim, spec.rot_dim, spec.vdim
     kd, vd = spec.kdim, spec.vdim_p
     T = u.shape[0]
     if out is None:
         out = torch.empty(T, H * vd, dtype=u.dtype, device=u.device)
+    if spec.absorbed:
+        return _absorbed_attention(u, rows, w_uq, w_heads, dq_norm, dkv_norm, caches[0], meta, spec, freq, eps, out)
     cq = ops.rms_cols(u, rows.off["dq"], spec.q_rank, dq_norm, eps)
     q = ops.linear(cq, w_uq)                                            # [T, H kdim]
     c = ops.rms_cols(u, rows.off["dkv"], spec.kv_rank, dkv_norm, eps)

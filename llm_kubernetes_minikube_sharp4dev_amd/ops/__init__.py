@@ -25,7 +25,7 @@ from .routed import clamped_glu, routed_experts, router_topk, sigmoid_mul_, silu
 from .hyper import (GROUP_MAX, GROUP_TOP2, MAX_STREAMS, SCORE_SIGMOID, SCORE_SOFTMAX, gate_proj, relu_sq_, router_choice,  # noqa: F401
                     stream_hyper_norm)
 from .latent import (head_linear, latent_attention_decode, latent_attention_prefill, latent_decode_splits, latent_prep,  # noqa: F401
-                     latent_query_rot, latent_row)
+                     latent_query, latent_query_rot, latent_row)
 from .diff import (diff_attention_decode, diff_attention_prefill, diff_attention_supported, diff_prefill_rows, qkv_file, row_tiles,  # noqa: F401
                    tile_attention_prefill, tile_attention_rows, tile_attention_supported)
 from .head_delta import head_delta, head_delta_supported  # noqa: F401

@@ -15,7 +15,7 @@ import torch
 
 from ._ext import lib, use_hip
 
-__all__ = ["latent_row", "latent_prep", "latent_query_rot", "head_linear", "latent_attention_prefill", "latent_attention_decode",
+__all__ = ["latent_row", "latent_prep", "latent_query_rot", "latent_query", "head_linear", "latent_attention_prefill", "latent_attention_decode",
            "latent_decode_splits"]
 
 
@@ -26,23 +26,26 @@ def latent_row(kv_rank: int, rot_dim: int) -> tuple:
     return rp, rdp
 
 
-def _rotate_halves(x, positions, freq, rd: int):
-    """x f32 [T, ..., rd]: dimension i pairs with i + rd / 2, angle position * freq[i]."""
+def _rotate_pairs(x, positions, freq, rd: int, adjacent: bool = False, mag: float = 1.0):
+    """x f32 [T, ..., rd]: dimension i pairs with i + rd / 2 (``adjacent``: 2 i with 2 i + 1), angle position * freq[i], cos and sin
+    times ``mag``."""
     half = rd // 2
     ang = positions.float().view(-1, *([1] * (x.dim() - 1))) * freq.float()[:half]
-    c, s = torch.cos(ang), torch.sin(ang)
-    u, v = x[..., :half], x[..., half:rd]
-    return torch.cat([u * c - v * s, v * c + u * s], -1)
+    c, s = torch.cos(ang) * mag, torch.sin(ang) * mag
+    u, v = (x[..., 0:rd:2], x[..., 1:rd:2]) if adjacent else (x[..., :half], x[..., half:rd])
+    y = (u * c - v * s, v * c + u * s)
+    return torch.stack(y, -1).flatten(-2) if adjacent else torch.cat(y, -1)
 
 
 def latent_prep(u, dq_col: int, q_rank: int, dq_norm, dkv_col: int, kv_rank: int, dkv_norm, rot_dim: int, freq, positions, eps: float,
-                cache, slots, rp: int):
+                cache, slots, rp: int, adjacent: bool = False, mag: float = 1.0):
     """cq [T, q_rank] = the columns ``[dq_col, dq_col + q_rank)`` of ``u`` divided by their RMS times ``dq_norm`` (f32 arithmetic).
     With ``dkv_norm`` (None: this layer reads another layer's cache) also the token's cache row at ``slots`` (< 0: none): the
-    normed latent of the columns behind ``dkv_col`` and the ``rot_dim`` columns that follow, rotated by position."""
+    normed latent of the columns behind ``dkv_col`` and the ``rot_dim`` columns that follow, rotated by position (``adjacent`` pairs or halves; cos and
+    sin times ``mag``)."""
     if use_hip(u):
         return lib().latent_prep(u, int(dq_col), int(q_rank), dq_norm, int(dkv_col), int(kv_rank), dkv_norm, int(rot_dim), freq, positions,
-                                 float(eps), cache, slots, int(rp))
+                                 float(eps), cache, slots, int(rp), bool(adjacent), float(mag))
     T = u.shape[0]
 
     def rms(x, w):
@@ -53,7 +56,7 @@ def latent_prep(u, dq_col: int, q_rank: int, dq_norm, dkv_col: int, kv_rank: int
         row = torch.zeros(T, cache.shape[2], dtype=torch.float32, device=u.device)
         row[:, :kv_rank] = rms(u[:, dkv_col:dkv_col + kv_rank].float(), dkv_norm)
         kr = u[:, dkv_col + kv_rank:dkv_col + kv_rank + rot_dim].float()
-        row[:, rp:rp + rot_dim] = _rotate_halves(kr, positions[:T], freq, rot_dim)
+        row[:, rp:rp + rot_dim] = _rotate_pairs(kr, positions[:T], freq, rot_dim, adjacent, mag)
         BS = cache.shape[1]
         sl = slots[:T].long()
         ok = sl >= 0
@@ -61,16 +64,16 @@ def latent_prep(u, dq_col: int, q_rank: int, dq_norm, dkv_col: int, kv_rank: int
     return cq
 
 
-def latent_query_rot(q, qa, H: int, qdim: int, dim: int, rot_dim: int, freq, positions, rp: int):
+def latent_query_rot(q, qa, H: int, qdim: int, dim: int, rot_dim: int, freq, positions, rp: int, adjacent: bool = False, mag: float = 1.0):
     """Rotated parts of the queries: ``q`` rows hold H heads of ``qdim`` columns, ``[dim plain | rot_dim | padding]``; their rotated
     columns go to ``qa[..., rp : rp + rot_dim]`` (``qa`` [T, H, KD]), zeros behind them."""
     if use_hip(q):
-        lib().latent_query_rot(q, qa, int(H), int(qdim), int(dim), int(rot_dim), freq, positions, int(rp))
+        lib().latent_query(q, None, qa, int(H), int(qdim), int(dim), int(rot_dim), freq, positions, int(rp), bool(adjacent), float(mag))
         return qa
     T = q.shape[0]
     r = q[:, : H * qdim].view(T, H, qdim)[..., dim:dim + rot_dim].float()
     qa[..., rp:] = 0
-    qa[..., rp:rp + rot_dim] = _rotate_halves(r, positions[:T], freq, rot_dim).to(qa.dtype)
+    qa[..., rp:rp + rot_dim] = _rotate_pairs(r, positions[:T], freq, rot_dim, adjacent, mag).to(qa.dtype)
     return qa
 
 
@@ -85,6 +88,16 @@ def head_linear(x, w, x_head: int, out):
     xs = torch.stack([x[:, h * x_head:h * x_head + K] for h in range(H)], 0).float()           # [H, T, K]
     out[..., :N] = torch.bmm(xs, w.float().transpose(1, 2).contiguous()).transpose(0, 1).to(out.dtype)
     return out
+
+
+def latent_query(q, w, qa, qdim: int, dim: int, rot_dim: int, freq, positions, rp: int, adjacent: bool = False, mag: float = 1.0):
+    """Attention queries over a cached latent in one launch: ``qa[t, h, :rp] = w[h] q[t, h * qdim : h * qdim + K]`` for ``w`` [H, rp, K]
+    (:func:`head_linear`) and the rotated part behind them (:func:`latent_query_rot`)."""
+    if use_hip(q):
+        lib().latent_query(q, w, qa, int(w.shape[0]), int(qdim), int(dim), int(rot_dim), freq, positions, int(rp), bool(adjacent), float(mag))
+        return qa
+    head_linear(q, w, qdim, qa)
+    return latent_query_rot(q, qa, w.shape[0], qdim, dim, rot_dim, freq, positions, rp, adjacent, mag)
 
 
 def latent_decode_splits(B: int, H: int, span: int) -> int:
@@ -114,30 +127,31 @@ def _gather(cache, table, n):
     return cache[table[: (n + BS - 1) // BS].long()].reshape(-1, cache.shape[2])[:n].float()
 
 
-def latent_attention_prefill(qa, cache, block_tables, cu_q, ctx_lens, window: int, scale: float, sink, rp: int, out, max_len: int):
+def latent_attention_prefill(qa, cache, block_tables, cu_q, ctx_lens, window: int, scale: float, sink, rp: int, out, max_len: int, gate=None):
     """Query chunks over their sequences' cached rows (their own included).  ``qa`` [T, H, KD]; ``sink`` f32 [H] or None; ``window`` 0:
-    causal; ``out`` [T, H, rp] receives the averaged latents."""
+    causal; ``out`` [T, H, rp] receives the averaged latents (head h times ``sigmoid(gate[:, h])`` with a ``gate`` [T, H])."""
     if use_hip(qa):
-        lib().latent_attn_prefill(qa, cache, block_tables, cu_q, ctx_lens, int(window), float(scale), sink, int(rp), out, int(max_len))
+        lib().latent_attn_prefill(qa, cache, block_tables, cu_q, ctx_lens, int(window), float(scale), sink, int(rp), out, int(max_len), gate)
         return out
     cu = cu_q.tolist()
     for b in range(len(cu) - 1):
         s0, s1 = cu[b], cu[b + 1]
         n = int(ctx_lens[b])
-        out[s0:s1] = _rows(qa[s0:s1].float(), _gather(cache, block_tables[b], n), torch.arange(n - (s1 - s0), n, device=qa.device), window,
-                           scale, sink, rp).to(out.dtype)
+        r = _rows(qa[s0:s1].float(), _gather(cache, block_tables[b], n), torch.arange(n - (s1 - s0), n, device=qa.device), window, scale,
+                  sink, rp)
+        out[s0:s1] = (r if gate is None else r * torch.sigmoid(gate[s0:s1, : r.shape[1], None].float())).to(out.dtype)
     return out
 
 
-def latent_attention_decode(qa, cache, block_tables, ctx_lens, window: int, scale: float, sink, rp: int, out, splits: int = 1):
-    """One query row per sequence at its last position (ctx - 1)."""
+def latent_attention_decode(qa, cache, block_tables, ctx_lens, window: int, scale: float, sink, rp: int, out, splits: int = 1, gate=None):
+    """One query row per sequence at its last position (ctx - 1).  ``gate``: as in :func:`latent_attention_prefill`."""
     if use_hip(qa):
-        lib().latent_attn_decode(qa, cache, block_tables, ctx_lens, window, float(scale), sink, int(rp), out, int(splits))
+        lib().latent_attn_decode(qa, cache, block_tables, ctx_lens, window, float(scale), sink, int(rp), out, int(splits), gate)
         return out
     for b in range(qa.shape[0]):
         n = int(ctx_lens[b])
         if n < 1:
             continue
-        out[b:b + 1] = _rows(qa[b:b + 1].float(), _gather(cache, block_tables[b], n), torch.tensor([n - 1], device=qa.device), window, scale,
-                             sink, rp).to(out.dtype)
+        r = _rows(qa[b:b + 1].float(), _gather(cache, block_tables[b], n), torch.tensor([n - 1], device=qa.device), window, scale, sink, rp)
+        out[b:b + 1] = (r if gate is None else r * torch.sigmoid(gate[b:b + 1, : r.shape[1], None].float())).to(out.dtype)
     return out
