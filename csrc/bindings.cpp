@@ -2196,6 +2196,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sigmoid_mul_", &sigmoid_mul_);
   m.def("gemm_grouped", &gemm_grouped);
   m.def("gemm_grouped_supported", [](int64_t N, int64_t K, bool swiglu) { return lk_gemm_grouped_supported((int)N, (int)K, swiglu ? 1 : 0) != 0; });
+  m.def("gemm_grouped_fine", [](int64_t rows, int64_t x_rows, int64_t N, int64_t K, bool swiglu) {
+    return lk_gemm1w_grouped_supported(rows, K, x_rows, (int)N, (int)K, swiglu ? 1 : 0, swiglu ? N / 2 : N) != 0;
+  });
   m.def("moe_gemm", &moe_gemm);
   m.def("stream_hyper_norm", &stream_hyper_norm);
   m.def("relu_sq_", &relu_sq_);

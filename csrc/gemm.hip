@@ -44,6 +44,7 @@
 //     of the same columns in a lane;
 //   * tiles are visited in an XCD-aware order (bijective remap, 4 row tiles x all column
 //     tiles per group), so an XCD's ~32 concurrent tiles share their X / W K-slices in L2.
+#include <cmath>
 #include <cstdlib>
 #include <map>
 #include <mutex>
@@ -921,6 +922,34 @@ int launch_grouped(const bf16_t* x, long ldx, const bf16_t* w, const int* seg, i
   return 0;
 }
 
+int cu_count();
+
+// Row tile of the grouped form: 256 (gemm_grouped_kernel) or 192 / 128 rows (gemm1w.hip's).  The experts' counts are on the device, so
+// the number of tiles is what counts spread around the mean like random ones give; a tile's time per K-tile of 64 is a + b * (share of
+// the CUs at work beside it), as measured with 16 experts of 2048 x 2816, in us: 1.02 + 0.68 / 0.80 + 0.70 / 0.64 + 0.50.  A smaller
+// tile is taken where that predicts 5 % less, which is where 256 rows leave a round of tiles nearly empty or most of a tile without
+// rows.  Two of 16 experts per token, gate and up / down product in us, 256 rows -> the rule's: 600 tokens 112 / 58 -> 104 / 40,
+// 1,024: 105 / 61 -> 97 / 51, 1,400: 121 / 60 -> 111 / 54, 2,500: 172 / 74 -> 144 / 72, 4,096: 213 / 126 -> 213 / 104 (the rule keeps
+// 256 for the wider product; 192 measured 209), 2,048, 3,000 and 3,500: 256 as before (192 up to 35 % slower).
+int grouped_tile_rows(long rows, int E, int TN) {
+  struct Cost { int bm; double a, b; };
+  constexpr Cost costs[] = {{256, 1.02, 0.68}, {192, 0.80, 0.70}, {128, 0.64, 0.50}};
+  const double mean = (double)rows / E, sd = sqrt(mean), cus = cu_count();
+  int best = 256;
+  double least = 0;
+  for (const Cost& c : costs) {
+    double per = 0;   // expected row tiles of an expert: the sum over k of P(count > k bm)
+    for (int k = 0; k * c.bm < mean + 5 * sd; ++k) per += k == 0 ? 1.0 : 0.5 * erfc((k * c.bm - mean) / (sd * M_SQRT2));
+    const double rounds = E * per * TN / cus, whole = floor(rounds), part = rounds - whole;
+    const double t = (whole * (c.a + c.b) + c.a * fmin(1.0, part * cus) + c.b * part) * (c.bm == 256 ? 0.95 : 1.0);
+    if (c.bm == 256 || t < least) {
+      best = c.bm;
+      least = t;
+    }
+  }
+  return best;
+}
+
 int cu_count() {
   static const int cus = [] {
     int dev = 0, n = 256;
@@ -1119,6 +1148,10 @@ int lk_gemm_grouped(const bf16_t* x, long ldx, const bf16_t* w, const int* seg, 
   if (E < 1 || (gather && x_rows < 1) || !lk_gemm_grouped_supported(N, K, swiglu) || ldx % 8 || ldo % 8 || reinterpret_cast<uintptr_t>(out) % 16 ||
       reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(w) % 16)
     return -1;
+  if (lk_gemm1w_grouped_supported(rows, ldx, gather ? x_rows : rows, N, K, swiglu, ldo)) {
+    const int bm = grouped_tile_rows(rows, E, N / 256);
+    if (bm != kBM) return lk_gemm1w_grouped(x, ldx, w, seg, E, rows, N, K, swiglu, out, ldo, st, gather, x_rows, scatter, bm);
+  }
   if (swiglu) return launch_grouped<4, EPI_SWIGLU>(x, ldx, w, seg, E, rows, N, K, N / 2, out, ldo, N / 256, st, gather, x_rows, scatter);
   if (N % 256 == 0) return launch_grouped<4, EPI_NONE>(x, ldx, w, seg, E, rows, N, K, 0, out, ldo, N / 256, st, gather, x_rows, scatter);
   return launch_grouped<3, EPI_NONE>(x, ldx, w, seg, E, rows, N, K, 0, out, ldo, N / 192, st, gather, x_rows, scatter);

@@ -127,7 +127,8 @@ constexpr bool persistable(int e) { return e == E_NONE || e == E_BIAS || e == E_
 // blockIdx.x, + gridDim.x, ...; the next tile's first two K-tiles are DMA'd during the current
 // tile's last two, so its load ramp hides behind the current epilogue (short-K shapes: the
 // encoder's K = 768 projections, 12 K-tiles per tile)
-template <int EPI, int SCP, int BM, bool PERSIST = false>
+// GS (grouped form, lk_gemm1w_grouped): rows sorted by expert, sources gathered and results scattered through LkEpi
+template <int EPI, int SCP, int BM, bool PERSIST = false, bool GS = false>
 __global__ __launch_bounds__(256, 1) void gemm1w_kernel(const bf16_t* __restrict__ X, long ldx,
                                                         const bf16_t* __restrict__ W,
                                                         const bf16_t* __restrict__ bias, int M, int K, int I,
@@ -145,6 +146,29 @@ __global__ __launch_bounds__(256, 1) void gemm1w_kernel(const bf16_t* __restrict
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wr = w >> 1, wc = w & 1;
   const int r = lane & 15, g = lane >> 4;
+  int tile = blockIdx.x;
+  if constexpr (GS) {  // the expert of this tile, its rows and weights
+    static_assert(!PERSIST && !SC && (EPI == E_NONE || EPI == E_SWIGLU), "grouped form");
+    int e = -1, t0 = 0, r0 = 0, acc_t = 0;
+    for (int i = 0; i < ea.experts; ++i) {
+      const int a = ea.seg[i], m = ea.seg[i + 1] - a, nt = ((m + BM - 1) / BM) * TN;
+      if (e < 0 && (int)blockIdx.x < acc_t + nt) {
+        e = i;
+        t0 = acc_t;
+        r0 = a;
+        M = m;
+      }
+      acc_t += nt;
+    }
+    if (e < 0) return;  // the whole workgroup: the grid is an upper bound
+    tile -= t0;
+    TM = (M + BM - 1) / BM;
+    W += (long)e * (EPI == E_SWIGLU ? 2 * I : TN * kBN) * K;
+    if (ea.gather) ea.gather += r0;
+    else X += (long)r0 * ldx;
+    if (ea.scatter) ea.scatter += r0;
+    else out += (long)r0 * ldo;
+  }
   const int nwg = TM * TN;
   const int nkt = K / kBK, kz = blockIdx.y, ks = gridDim.y;
   const int kt0 = kz * nkt / ks, nk = (kz + 1) * nkt / ks - kt0;  // >= 3 (host check)
@@ -157,7 +181,7 @@ __global__ __launch_bounds__(256, 1) void gemm1w_kernel(const bf16_t* __restrict
     tm = first + (L % per_group) % gm;
     tn = tn0 + (L % per_group) / gm;  // (tn0: a column-split launch's first column tile)
   };
-  const u32x4_t xsrd = srd(X, (long)M * ldx * 2);
+  const u32x4_t xsrd = srd(X, (long)(GS && ea.gather ? ea.x_rows : M) * ldx * 2);
   const u32x4_t wsrd = srd(W, (long)(EPI == E_SWIGLU ? 2 * I : (tn0 + TN) * kBN) * K * 2);
   const unsigned lds0 = static_cast<unsigned>(reinterpret_cast<uintptr_t>((lds_ptr_t)smem));
   const unsigned ldsx = rfl(lds0 + (BM / 4) * w * kRowB), ldsw = rfl(lds0 + kOpX + 64 * w * kRowB);
@@ -181,7 +205,15 @@ __global__ __launch_bounds__(256, 1) void gemm1w_kernel(const bf16_t* __restrict
                                         : (unsigned)(tn * kBN + 64 * w + lanew);
     const unsigned wb = wl * kb;
 #pragma unroll
-    for (int i = 0; i < PX; ++i) xo[i] = xb + (unsigned)(8 * i) * ldxb + (ch0 ^ (unsigned)((i & 1) << 6));
+    for (int i = 0; i < PX; ++i) {
+      if constexpr (GS) {  // rows past the expert's end point behind the descriptor's range: zeros
+        const int tr = tm * BM + (BM / 4) * w + lr8 + 8 * i;
+        const int src = tr < M ? (ea.gather ? ea.gather[tr] : tr) : -1;
+        xo[i] = src >= 0 ? (unsigned)src * ldxb + (ch0 ^ (unsigned)((i & 1) << 6)) : 0xFFFFFF00u;
+      } else {
+        xo[i] = xb + (unsigned)(8 * i) * ldxb + (ch0 ^ (unsigned)((i & 1) << 6));
+      }
+    }
 #pragma unroll
     for (int i = 0; i < 8; ++i)
       wo[i] = wb + (unsigned)(32 * (i >> 2) + 16 * (i & 1) + 4 * ((i >> 1) & 1)) * kb + (ch0 ^ (unsigned)((i & 1) << 6));
@@ -285,7 +317,6 @@ __global__ __launch_bounds__(256, 1) void gemm1w_kernel(const bf16_t* __restrict
   // ---- one tile per workgroup by default (for long K a persistent walk measured 1-3 % slower: the
   // hardware already starts the next workgroup on a CU while the finished one's stores drain --
   // profiles/r5_gemm1w/); PERSIST for short K, where the load ramp is a third of a tile
-  int tile = blockIdx.x;
   int tm, tn;
   coords(tile, tm, tn);
   offsets(tm, tn, xo, wo);
@@ -359,6 +390,17 @@ __global__ __launch_bounds__(256, 1) void gemm1w_kernel(const bf16_t* __restrict
 #pragma unroll
       for (int m = 0; m < MB; ++m) scm[m] = scl[wr * WM + m * 16 + r];
     }
+    // the first byte of an output row's columns at c (grouped: the scattered row, or behind the range)
+    const long orows = GS && ea.scatter ? ea.out_rows : M;
+    auto row_at = [&](int m, int c) -> unsigned {
+      const long row = (long)tm * BM + wr * WM + m * 16 + r;
+      if constexpr (GS) {
+        if (row >= M) return 0xFFFFFE00u;
+        return (unsigned)((ea.scatter ? ea.scatter[row] : row) * ldo + c) * 2;
+      } else {
+        return (unsigned)(row * ldo + c) * 2;
+      }
+    };
     auto pk8 = [](const float (&y)[8]) {
       return u32x4_t{pack_bf2(y[0], y[1]), pack_bf2(y[2], y[3]), pack_bf2(y[4], y[5]), pack_bf2(y[6], y[7])};
     };
@@ -374,10 +416,10 @@ __global__ __launch_bounds__(256, 1) void gemm1w_kernel(const bf16_t* __restrict
                                                  rb + (unsigned)((32 * (n >> 1) + 8 * g + 4 * (n & 1)) * 4), 0, 0);
       }
     } else if constexpr (EPI == E_SWIGLU) {
-      const auto os = __builtin_amdgcn_make_buffer_rsrc(out, 0, (int)min((long)M * ldo * 2, 0x7FFFFFF0L), 0x00020000);
+      const auto os = __builtin_amdgcn_make_buffer_rsrc(out, 0, (int)min(orows * ldo * 2, 0x7FFFFFF0L), 0x00020000);
 #pragma unroll
       for (int m = 0; m < MB; ++m) {
-        const unsigned rb = (unsigned)(((long)tm * BM + wr * WM + m * 16 + r) * ldo + tn * 128 + wc * 64 + 8 * g) * 2;
+        const unsigned rb = row_at(m, tn * 128 + wc * 64 + 8 * g);
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
           float y[8];
@@ -385,7 +427,8 @@ __global__ __launch_bounds__(256, 1) void gemm1w_kernel(const bf16_t* __restrict
           for (int h = 0; h < 2; ++h)
 #pragma unroll
             for (int v = 0; v < 4; ++v)
-              y[4 * h + v] = rbf(lk_silu(rbf(acc[m][2 * p + h][v] * scm[m]))) * rbf(acc[m][4 + 2 * p + h][v] * scm[m]);
+              y[4 * h + v] = GS ? lk_silu(acc[m][2 * p + h][v]) * acc[m][4 + 2 * p + h][v]   // f32 up to the result
+                                : rbf(lk_silu(rbf(acc[m][2 * p + h][v] * scm[m]))) * rbf(acc[m][4 + 2 * p + h][v] * scm[m]);
           __builtin_amdgcn_raw_buffer_store_b128(pk8(y), os, rb + 64 * p, 0, 0);
         }
       }
@@ -510,7 +553,7 @@ __global__ __launch_bounds__(256, 1) void gemm1w_kernel(const bf16_t* __restrict
         }
       }
     } else {  // NONE / BIAS / BIAS_GELU / BIAS_RELU
-      const auto os = __builtin_amdgcn_make_buffer_rsrc(out, 0, (int)min((long)M * ldo * 2, 0x7FFFFFF0L), 0x00020000);
+      const auto os = __builtin_amdgcn_make_buffer_rsrc(out, 0, (int)min(orows * ldo * 2, 0x7FFFFFF0L), 0x00020000);
       float bv[8][4];
 #pragma unroll
       for (int n = 0; n < 8; ++n)
@@ -536,7 +579,7 @@ __global__ __launch_bounds__(256, 1) void gemm1w_kernel(const bf16_t* __restrict
       };
 #pragma unroll
       for (int m = 0; m < MB; ++m) {
-        const unsigned rb = (unsigned)(((long)tm * BM + wr * WM + m * 16 + r) * ldo + tn * kBN + wc * 128 + 8 * g) * 2;
+        const unsigned rb = row_at(m, tn * kBN + wc * 128 + 8 * g);
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
           float y[8];
@@ -712,7 +755,42 @@ void launch1w_sc(int bm, const bf16_t* x, long ldx, const bf16_t* w, const bf16_
   launch1w_tiles<EPI, 0>(bm, x, ldx, w, bias, M, K, I, out, ldo, TN, ks, group_m, st, ea);
 }
 
+template <int EPI, int BM>
+int launch1w_grouped(const bf16_t* x, long ldx, const bf16_t* w, long rows, int K, int I, bf16_t* out, long ldo, int TN, hipStream_t st,
+                     const LkEpi& ea) {
+  constexpr int lds = Tile<BM>::kLds;
+  LK_SET_MAX_LDS((gemm1w_kernel<EPI, 0, BM, false, true>), lds);
+  const long grid = ((rows + BM - 1) / BM + ea.experts) * TN;
+  if (grid > 2147483647L) return -1;
+  gemm1w_kernel<EPI, 0, BM, false, true><<<dim3((unsigned)grid, 1), 256, lds, st>>>(x, ldx, w, nullptr, 0, K, I, out, ldo, 0, TN, 0,
+                                                                                    group1w(), ea);
+  LK_CHECK_LAUNCH();
+  return 0;
+}
+
 }  // namespace
+
+int lk_gemm1w_grouped_supported(long rows, long ldx, long x_rows, int N, int K, int swiglu, long ldo) {
+  if (K % kBK || K / kBK < 3 || (swiglu ? N % 2 || (N / 2) % 128 : N % kBN)) return 0;
+  return (long)N * K * 2 < 0x7FFFFFF0L && max(rows, x_rows) * ldx * 2 < 0x7FFFFFF0L && rows * ldo * 2 < 0x7FFFFFF0L;
+}
+
+int lk_gemm1w_grouped(const bf16_t* x, long ldx, const bf16_t* w, const int* seg, int E, long rows, int N, int K, int swiglu, bf16_t* out,
+                      long ldo, hipStream_t st, const int* gather, long x_rows, const int* scatter, int bm) {
+  if (!lk_gemm1w_grouped_supported(rows, ldx, gather ? x_rows : rows, N, K, swiglu, ldo)) return -1;
+  LkEpi ea{};
+  ea.seg = seg;
+  ea.experts = E;
+  ea.gather = gather;
+  ea.scatter = scatter;
+  ea.x_rows = x_rows;
+  ea.out_rows = rows;
+  if (swiglu)
+    return bm == 128 ? launch1w_grouped<E_SWIGLU, 128>(x, ldx, w, rows, K, N / 2, out, ldo, N / 256, st, ea)
+                     : launch1w_grouped<E_SWIGLU, 192>(x, ldx, w, rows, K, N / 2, out, ldo, N / 256, st, ea);
+  return bm == 128 ? launch1w_grouped<E_NONE, 128>(x, ldx, w, rows, K, 0, out, ldo, N / kBN, st, ea)
+                   : launch1w_grouped<E_NONE, 192>(x, ldx, w, rows, K, 0, out, ldo, N / kBN, st, ea);
+}
 
 int lk_gemm1w_split_cols(int M, int TN, int cus) {
   const int tm = (M + 255) / 256;

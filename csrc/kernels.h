@@ -129,6 +129,10 @@ struct LkEpi {
   const int* gather = nullptr;
   const int* scatter = nullptr;
   long x_rows = 0;
+  // gemm1w's grouped form: the experts' row offsets, rows of the output behind the scatter
+  const int* seg = nullptr;
+  int experts = 0;
+  long out_rows = 0;
 };
 // variant: K-loop schedule of gemm.hip (0 / 1 / 2), or 3 = gemm1w.hip (bn 256)
 int lk_gemm(const bf16_t* x, long ldx, const bf16_t* w, const bf16_t* bias, int M, int N, int K, int epi, int bn,
@@ -148,6 +152,10 @@ int lk_gemm_grouped(const bf16_t* x, long ldx, const bf16_t* w, const int* seg, 
 // Variants 6 / 7: a column split -- the column tiles that fill whole waves of the CUs on 256-row
 // tiles, the remaining (less than a wave) on 128 / 192-row tiles, as two launches.
 constexpr int LK_GEMM1W_SPLIT128 = 1, LK_GEMM1W_SPLIT192 = 2;
+// grouped form (lk_gemm_grouped's contract) on bm = 128 / 192-row tiles; supported: >= 3 K-tiles, 32-bit offsets
+int lk_gemm1w_grouped_supported(long rows, long ldx, long x_rows, int N, int K, int swiglu, long ldo);
+int lk_gemm1w_grouped(const bf16_t* x, long ldx, const bf16_t* w, const int* seg, int E, long rows, int N, int K, int swiglu, bf16_t* out,
+                      long ldo, hipStream_t st, const int* gather, long x_rows, const int* scatter, int bm);
 inline int lk_gemm1w_bm(int variant) {
   return variant == 3 ? 256 : variant == 4 ? 192 : variant == 5 ? 128 : variant == 6 ? LK_GEMM1W_SPLIT128
        : variant == 7 ? LK_GEMM1W_SPLIT192 : 0;

@@ -21,8 +21,9 @@ import torch.nn.functional as F
 
 from ._ext import lib, use_hip
 
-# from this many (token, choice) pairs per expert on average the experts run on the dense GEMM's 256-row tiles
+# from this many (token, choice) pairs per expert on average the experts run on the dense GEMM's tiles (_grouped)
 GROUPED_DENSE_MIN_ROWS = 128
+GROUPED_FINE_MIN_ROWS = 64
 
 __all__ = ["stream_gated_norm", "rms_cols", "rot_kv_write", "pool_kv_write", "table_experts", "run_experts", "moe_route"]
 
@@ -153,6 +154,16 @@ def table_experts(h, ids, table, w_gate_up, w_down, top: int):
     return run_experts(h, ids, table, w_gate_up, w_down, top)
 
 
+def _grouped(T: int, pairs: int, E: int, W: int, ffp: int) -> bool:
+    """Whether the expert products run as one dense product per expert (``gemm_grouped``): from GROUPED_DENSE_MIN_ROWS pairs per expert on,
+    and from GROUPED_FINE_MIN_ROWS where its 128 / 192-row tiles take both sizes (2 of 16 experts of 2048 x 2816: 600 tokens 203 -> 144
+    us, 800 tokens 225 -> 149 us, with the same f32 activation)."""
+    if pairs >= GROUPED_DENSE_MIN_ROWS * E:
+        return lib().gemm_grouped_supported(2 * ffp, W, True) and lib().gemm_grouped_supported(W, ffp, False)
+    return (pairs >= GROUPED_FINE_MIN_ROWS * E and lib().gemm_grouped_fine(pairs, T, 2 * ffp, W, True)
+            and lib().gemm_grouped_fine(pairs, pairs, W, ffp, False))
+
+
 def run_experts(h, ids, table, w_gate_up, w_down, top: int):
     """The expert products behind ``table_experts`` (``ids`` int32 [T] index the table's rows) and
     ``routed_experts`` (``ids`` None: ``table`` int32 [T, top] holds each row's own choice)."""
@@ -160,8 +171,7 @@ def run_experts(h, ids, table, w_gate_up, w_down, top: int):
     E, ffp = w_gate_up.shape[0], w_down.shape[2]
     if use_hip(h):
         seg, order = moe_route(ids, table, E)
-        if (h.dtype == torch.bfloat16 and T * top >= GROUPED_DENSE_MIN_ROWS * E and lib().gemm_grouped_supported(2 * ffp, W, True)
-                and lib().gemm_grouped_supported(W, ffp, False)):
+        if h.dtype == torch.bfloat16 and _grouped(T, T * top, E, W, ffp):
             # prompt-sized steps on the framework's dense GEMM tiles, one GEMM per expert inside one launch: the first
             # product reads each pair's token row in place, the second writes each result into its pair's row
             mid = lib().gemm_grouped(h, seg, w_gate_up, True, torch.div(order, top, rounding_mode="floor"), None)

@@ -1,0 +1,46 @@
+"""One product per expert over rows sorted by expert (the prompt form of the routed feed-forward): row counts on both sides of the row
+tiles (128, 192 and 256 rows, chosen by the mean), against float64; gathered sources, scattered results, SwiGLU."""
+import pytest
+import torch
+
+from llm_kubernetes_minikube_sharp4dev_amd import ops
+
+
+# whole rounds of tiles on 256 CUs: 192 rows (one tile per expert instead of two of 128), 256 rows
+FULL192, FULL256 = [150, 192, 191, 1, 129, 193, 185, 160, 190, 170, 175, 0, 180, 188, 65, 192], [256, 250, 193, 240, 255, 257, 230, 245] * 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("counts,swiglu,N,K", [(FULL192, True, 8192, 192), (FULL192, False, 4096, 192), (FULL256, True, 4096, 192),
+                                               (FULL256, False, 4096, 256)])
+def test_full_rounds(counts, swiglu, N, K):
+    test_rows_per_expert(counts, swiglu, N, K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("counts", [[1, 64, 65], [128, 0, 129, 192, 17], [193, 256, 257, 17], [130, 191, 192, 193, 0, 385], [319, 320, 321, 384, 385, 512, 513]])
+@pytest.mark.parametrize("swiglu,N,K", [(True, 512, 192), (True, 768, 256), (False, 256, 128), (False, 512, 320), (False, 192, 320)])
+def test_rows_per_expert(counts, swiglu, N, K):
+    g = torch.Generator().manual_seed(sum(counts))
+    E, R = len(counts), sum(counts)
+    x = torch.randn(R, K, generator=g).bfloat16()
+    w = (torch.randn(E, N, K, generator=g) * K ** -0.5).bfloat16()
+    seg = torch.tensor([0] + counts).cumsum(0).int()
+    perm = torch.randperm(R, generator=g).int()
+    cols = N // 2 if swiglu else N
+    want, tol = torch.zeros(R, cols, dtype=torch.float64), torch.zeros(R, cols, dtype=torch.float64)
+    for e in range(E):
+        a, b = int(seg[e]), int(seg[e + 1])
+        y = x[perm[a:b].long()].double() @ w[e].double().T
+        # half a bf16 step (2^-8 of the value) per rounding: the product; SwiGLU: gate (its slope in silu is at most 1.1), up, silu, result
+        if swiglu:
+            gate, up = y[:, :cols], y[:, cols:]
+            want[a:b] = gate * torch.sigmoid(gate) * up
+            tol[a:b] = 2 ** -8 * (3 * want[a:b].abs() + 1.1 * (gate * up).abs())
+        else:
+            want[a:b], tol[a:b] = y, 2 ** -8 * y.abs()
+    got = ops.lib().gemm_grouped(x.cuda(), seg.cuda(), w.cuda(), swiglu, perm.cuda(), None).double().cpu()
+    tol = 1.05 * tol + 1e-4      # second order terms, f32 sums of K products of standard deviation 1
+    assert bool(((got - want).abs() <= tol).all()), float(((got - want).abs() - tol).max())
+    back = ops.lib().gemm_grouped(x[perm.long()].cuda(), seg.cuda(), w.cuda(), swiglu, None, perm.cuda()).double().cpu()
+    assert torch.equal(back[perm.long()], got)
