@@ -1,0 +1,21 @@
+"""GELU on every bf16 value against float64: in the negative tail too it is off by the rounding of the result and a relative 2e-4 of
+the fitted tail only; infinities and NaN as from x Phi(x) in f32."""
+import pytest
+import torch
+
+from llm_kubernetes_minikube_sharp4dev_amd import ops
+
+
+@pytest.mark.gpu
+def test_every_bf16_value():
+    x = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16).clone().view(256, 256)
+    got = ops.gelu_(x.clone().cuda()).cpu().double()
+    d = x.double()
+    want = d * torch.special.ndtr(d)
+    fin = torch.isfinite(d)
+    inner = fin & (d > -5)
+    # half a bf16 step of the result and the tail's fit; results below bf16's smallest normal value may round to zero
+    tol = (2 ** -8 + 3e-4) * want.abs() + 2 ** -126
+    assert bool(((got - want).abs() <= tol)[inner].all())
+    assert bool((got.abs() <= 1e-5)[fin & (d <= -5)].all())
+    assert bool((got == d)[d == float("inf")].all()) and bool(torch.isnan(got)[torch.isnan(d)].all())
