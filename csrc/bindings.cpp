@@ -1677,7 +1677,7 @@ void pool_kv_write(const at::Tensor& kc, const at::Tensor& vc, at::Tensor& pkc, 
 // x [rows, K] sorted by expert -- or, with `gather` int32 [rows], any x whose row gather[r] is sorted row r's input; the
 // result's rows are sorted, or with `scatter` int32 [rows] sorted row r lands in out row scatter[r] (a permutation)
 at::Tensor gemm_grouped(const at::Tensor& x, const at::Tensor& seg, const at::Tensor& w, bool swiglu,
-                        const c10::optional<at::Tensor>& gather, const c10::optional<at::Tensor>& scatter) {
+                        const c10::optional<at::Tensor>& gather, const c10::optional<at::Tensor>& scatter, int64_t top) {
   CHECK_CUDA(x); CHECK_BF16(x); CHECK_LASTDIM(x); CHECK_CUDA(w); CHECK_BF16(w); CHECK_CONTIG(w); CHECK_CUDA(seg); CHECK_I32(seg);
   CHECK_CONTIG(seg);
   TORCH_CHECK(x.dim() == 2 && w.dim() == 3 && w.size(2) == x.size(1) && seg.numel() == w.size(0) + 1, "x [rows, K], w [E, N, K], seg [E + 1]");
@@ -1688,7 +1688,7 @@ at::Tensor gemm_grouped(const at::Tensor& x, const at::Tensor& seg, const at::Te
   if (scatter) { CHECK_CUDA(*scatter); CHECK_I32(*scatter); CHECK_CONTIG(*scatter); TORCH_CHECK(scatter->numel() == rows, "scatter rows"); }
   at::Tensor out = at::empty({rows, swiglu ? N / 2 : N}, x.options());
   CHECK_RC(lk_gemm_grouped(bp(x), x.stride(0), bp(w), ip(seg), (int)w.size(0), rows, N, K, swiglu ? 1 : 0, bp(out), out.stride(0),
-                           cur_stream(), ipo(gather), x.size(0), ipo(scatter)), "gemm_grouped");
+                           cur_stream(), ipo(gather), x.size(0), ipo(scatter), (int)top), "gemm_grouped");
   return out;
 }
 
@@ -2194,7 +2194,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("clamped_glu", &clamped_glu);
   m.def("silu_", &silu_);
   m.def("sigmoid_mul_", &sigmoid_mul_);
-  m.def("gemm_grouped", &gemm_grouped);
+  m.def("gemm_grouped", &gemm_grouped, py::arg("x"), py::arg("seg"), py::arg("w"), py::arg("swiglu"), py::arg("gather"), py::arg("scatter"),
+        py::arg("top") = 1);
   m.def("gemm_grouped_supported", [](int64_t N, int64_t K, bool swiglu) { return lk_gemm_grouped_supported((int)N, (int)K, swiglu ? 1 : 0) != 0; });
   m.def("gemm_grouped_fine", [](int64_t rows, int64_t x_rows, int64_t N, int64_t K, bool swiglu) {
     return lk_gemm1w_grouped_supported(rows, K, x_rows, (int)N, (int)K, swiglu ? 1 : 0, swiglu ? N / 2 : N) != 0;

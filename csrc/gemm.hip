@@ -206,7 +206,7 @@ __device__ __forceinline__ void gemm8_body(const bf16_t* __restrict__ X, long ld
       const int s = 16 * w + 8 * i + lr;
       if constexpr (GS) {  // a gathered source row; tile rows past the expert's end point behind the descriptor's range
         const int tr = tm * kBM + a_row(h, s);
-        const int src = tr < M ? (ea.gather ? ea.gather[tr] : tr) : -1;
+        const int src = tr < M ? (ea.gather ? ea.gather[tr] / ea.top : tr) : -1;
         aoff[h][i] = src >= 0 ? (unsigned)((long)src * ldx * 2) + ((lc ^ swz(s)) << 4) : 0xFFFFFF00u;
       } else {
         aoff[h][i] = (unsigned)(((long)tm * kBM + a_row(h, s)) * ldx * 2) + ((lc ^ swz(s)) << 4);
@@ -878,14 +878,14 @@ int group_rows() {
 // whose weights are W + e * N * K.  Every expert is an ordinary GEMM of its own row count on the body above; a workgroup
 // finds its (expert, tile) by walking seg[] on the device, so the launch needs nothing from the host: the grid is the
 // upper bound (rows / 256 + E) * TN and surplus workgroups leave at once.  Rows past an expert's end read zeros through
-// the buffer descriptor's range check and are not stored.  gather (or null): X row of every sorted row (the experts'
-// inputs are then read in place instead of from a sorted copy); scatter (or null): out row of every sorted row.
+// the buffer descriptor's range check and are not stored.  gather (or null): top times the X row of every sorted row, plus less
+// than top (the experts' inputs are then read in place instead of from a sorted copy); scatter (or null): out row of every sorted row.
 template <int NF, int EPI>
 __global__ __launch_bounds__(512, 1) void gemm_grouped_kernel(const bf16_t* __restrict__ X, long ldx,
                                                               const bf16_t* __restrict__ W, const int* __restrict__ seg,
                                                               int E, int N, int K, int I, bf16_t* __restrict__ out, long ldo,
                                                               int TN, int group_m, const int* __restrict__ gather, long x_rows,
-                                                              const int* __restrict__ scatter) {
+                                                              const int* __restrict__ scatter, int top) {
   int e = -1, tile = 0, r0 = 0, rows = 0, acc = 0;
   for (int i = 0; i < E; ++i) {
     const int a = seg[i], m = seg[i + 1] - a, nt = ((m + kBM - 1) / kBM) * TN;
@@ -903,6 +903,7 @@ __global__ __launch_bounds__(512, 1) void gemm_grouped_kernel(const bf16_t* __re
   ea.gather = gather ? gather + r0 : nullptr;     // indexed by the expert's own tile rows
   ea.scatter = scatter ? scatter + r0 : nullptr;
   ea.x_rows = x_rows;
+  ea.top = top;
   gemm8_body<NF, EPI, 4, 0, false, true>(gather ? X : X + (long)r0 * ldx, ldx, W + (long)e * N * K, nullptr, rows, K, I,
                                          scatter ? out : out + (long)r0 * ldo, ldo, (rows + kBM - 1) / kBM, TN, group_m, tile, 0,
                                          K / kBK, 0, SK_FULL, 0, sk, ea);
@@ -911,13 +912,13 @@ __global__ __launch_bounds__(512, 1) void gemm_grouped_kernel(const bf16_t* __re
 
 template <int NF, int EPI>
 int launch_grouped(const bf16_t* x, long ldx, const bf16_t* w, const int* seg, int E, long rows, int N, int K, int I, bf16_t* out,
-                   long ldo, int TN, hipStream_t st, const int* gather, long x_rows, const int* scatter) {
+                   long ldo, int TN, hipStream_t st, const int* gather, long x_rows, const int* scatter, int top) {
   constexpr int lds = 2 * Geo<NF>::BUF;
   LK_SET_MAX_LDS((gemm_grouped_kernel<NF, EPI>), lds);
   const long grid = ((rows + kBM - 1) / kBM + E) * TN;
   if (grid > 2147483647L) return -1;
   gemm_grouped_kernel<NF, EPI><<<dim3((unsigned)grid), 512, lds, st>>>(x, ldx, w, seg, E, N, K, I, out, ldo, TN, group_rows(),
-                                                                       gather, x_rows, scatter);
+                                                                       gather, x_rows, scatter, top);
   LK_CHECK_LAUNCH();
   return 0;
 }
@@ -1143,18 +1144,18 @@ int lk_gemm_grouped_supported(int N, int K, int swiglu) {
 // out[r] = epi(X[r] . W_e^T) for the rows r in [seg[e], seg[e + 1]) of every expert e: X [rows, K] sorted by expert (row
 // stride ldx), W [E, N, K] contiguous, out [rows, N] (SwiGLU: W_e = [gate rows | up rows], out [rows, N / 2]).
 int lk_gemm_grouped(const bf16_t* x, long ldx, const bf16_t* w, const int* seg, int E, long rows, int N, int K, int swiglu,
-                    bf16_t* out, long ldo, hipStream_t st, const int* gather, long x_rows, const int* scatter) {
+                    bf16_t* out, long ldo, hipStream_t st, const int* gather, long x_rows, const int* scatter, int top) {
   if (rows <= 0) return 0;
-  if (E < 1 || (gather && x_rows < 1) || !lk_gemm_grouped_supported(N, K, swiglu) || ldx % 8 || ldo % 8 || reinterpret_cast<uintptr_t>(out) % 16 ||
+  if (E < 1 || top < 1 || (gather && x_rows < 1) || !lk_gemm_grouped_supported(N, K, swiglu) || ldx % 8 || ldo % 8 || reinterpret_cast<uintptr_t>(out) % 16 ||
       reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(w) % 16)
     return -1;
   if (lk_gemm1w_grouped_supported(rows, ldx, gather ? x_rows : rows, N, K, swiglu, ldo)) {
     const int bm = grouped_tile_rows(rows, E, N / 256);
-    if (bm != kBM) return lk_gemm1w_grouped(x, ldx, w, seg, E, rows, N, K, swiglu, out, ldo, st, gather, x_rows, scatter, bm);
+    if (bm != kBM) return lk_gemm1w_grouped(x, ldx, w, seg, E, rows, N, K, swiglu, out, ldo, st, gather, x_rows, scatter, top, bm);
   }
-  if (swiglu) return launch_grouped<4, EPI_SWIGLU>(x, ldx, w, seg, E, rows, N, K, N / 2, out, ldo, N / 256, st, gather, x_rows, scatter);
-  if (N % 256 == 0) return launch_grouped<4, EPI_NONE>(x, ldx, w, seg, E, rows, N, K, 0, out, ldo, N / 256, st, gather, x_rows, scatter);
-  return launch_grouped<3, EPI_NONE>(x, ldx, w, seg, E, rows, N, K, 0, out, ldo, N / 192, st, gather, x_rows, scatter);
+  if (swiglu) return launch_grouped<4, EPI_SWIGLU>(x, ldx, w, seg, E, rows, N, K, N / 2, out, ldo, N / 256, st, gather, x_rows, scatter, top);
+  if (N % 256 == 0) return launch_grouped<4, EPI_NONE>(x, ldx, w, seg, E, rows, N, K, 0, out, ldo, N / 256, st, gather, x_rows, scatter, top);
+  return launch_grouped<3, EPI_NONE>(x, ldx, w, seg, E, rows, N, K, 0, out, ldo, N / 192, st, gather, x_rows, scatter, top);
 }
 
 int lk_gemm_supported(int M, int N, int K, int epi, int bn, int ks) {

@@ -208,7 +208,7 @@ __global__ __launch_bounds__(256, 1) void gemm1w_kernel(const bf16_t* __restrict
     for (int i = 0; i < PX; ++i) {
       if constexpr (GS) {  // rows past the expert's end point behind the descriptor's range: zeros
         const int tr = tm * BM + (BM / 4) * w + lr8 + 8 * i;
-        const int src = tr < M ? (ea.gather ? ea.gather[tr] : tr) : -1;
+        const int src = tr < M ? (ea.gather ? ea.gather[tr] / ea.top : tr) : -1;
         xo[i] = src >= 0 ? (unsigned)src * ldxb + (ch0 ^ (unsigned)((i & 1) << 6)) : 0xFFFFFF00u;
       } else {
         xo[i] = xb + (unsigned)(8 * i) * ldxb + (ch0 ^ (unsigned)((i & 1) << 6));
@@ -772,12 +772,13 @@ int lk_gemm1w_grouped_supported(long rows, long ldx, long x_rows, int N, int K, 
 }
 
 int lk_gemm1w_grouped(const bf16_t* x, long ldx, const bf16_t* w, const int* seg, int E, long rows, int N, int K, int swiglu, bf16_t* out,
-                      long ldo, hipStream_t st, const int* gather, long x_rows, const int* scatter, int bm) {
+                      long ldo, hipStream_t st, const int* gather, long x_rows, const int* scatter, int top, int bm) {
   if (!lk_gemm1w_grouped_supported(rows, ldx, gather ? x_rows : rows, N, K, swiglu, ldo)) return -1;
   LkEpi ea{};
   ea.seg = seg;
   ea.experts = E;
   ea.gather = gather;
+  ea.top = top;
   ea.scatter = scatter;
   ea.x_rows = x_rows;
   ea.out_rows = rows;

@@ -132,6 +132,7 @@ struct LkEpi {
   // gemm1w's grouped form: the experts' row offsets, rows of the output behind the scatter
   const int* seg = nullptr;
   int experts = 0;
+  int top = 1;                   // both grouped forms: gather holds (row, choice) pairs, the X row is gather[j] / top
   long out_rows = 0;
 };
 // variant: K-loop schedule of gemm.hip (0 / 1 / 2), or 3 = gemm1w.hip (bn 256)
@@ -143,7 +144,8 @@ int lk_gemm(const bf16_t* x, long ldx, const bf16_t* w, const bf16_t* bias, int 
 // none or SwiGLU.  Needs K % 64 == 0, K >= 128, N % 256 or N % 192 == 0 (SwiGLU: N/2 % 128 == 0)
 int lk_gemm_grouped_supported(int N, int K, int swiglu);
 int lk_gemm_grouped(const bf16_t* x, long ldx, const bf16_t* w, const int* seg, int E, long rows, int N, int K, int swiglu,
-                    bf16_t* out, long ldo, hipStream_t st, const int* gather = nullptr, long x_rows = 0, const int* scatter = nullptr);
+                    bf16_t* out, long ldo, hipStream_t st, const int* gather = nullptr, long x_rows = 0, const int* scatter = nullptr,
+                    int top = 1);
 
 // gemm1w.hip: the one-wave-per-SIMD bm x 256 prefill GEMM (hipBLASLt's gfx950 K-loop schedule,
 // every lk_gemm epilogue); lk_gemm routes variants 3 / 4 / 5 here (row tile bm = 256 / 192 / 128).
@@ -155,7 +157,7 @@ constexpr int LK_GEMM1W_SPLIT128 = 1, LK_GEMM1W_SPLIT192 = 2;
 // grouped form (lk_gemm_grouped's contract) on bm = 128 / 192-row tiles; supported: >= 3 K-tiles, 32-bit offsets
 int lk_gemm1w_grouped_supported(long rows, long ldx, long x_rows, int N, int K, int swiglu, long ldo);
 int lk_gemm1w_grouped(const bf16_t* x, long ldx, const bf16_t* w, const int* seg, int E, long rows, int N, int K, int swiglu, bf16_t* out,
-                      long ldo, hipStream_t st, const int* gather, long x_rows, const int* scatter, int bm);
+                      long ldo, hipStream_t st, const int* gather, long x_rows, const int* scatter, int top, int bm);
 inline int lk_gemm1w_bm(int variant) {
   return variant == 3 ? 256 : variant == 4 ? 192 : variant == 5 ? 128 : variant == 6 ? LK_GEMM1W_SPLIT128
        : variant == 7 ? LK_GEMM1W_SPLIT192 : 0;

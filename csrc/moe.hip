@@ -25,33 +25,66 @@ namespace {
 constexpr int kRouteThreads = 1024;
 constexpr int kMaxExperts = 1024;
 
+// One workgroup; its time is the chain of dependent loads (token id, then table), so a thread requests the ids of all its pairs and then
+// all their table entries, kRouteU at a time, and keeps the experts in registers for the second pass where they fit (8,192 pairs).
+// 8,192 pairs of 16 experts: one pair after the other, twice, 18.7 us, now 14.6 (the rest are the counters' atomics).
+constexpr int kRouteU = 8;
+
 __global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(const int* __restrict__ ids, const int* __restrict__ table, int vocab,
                                                                   int top, int E, int T, int* __restrict__ seg,
                                                                   int* __restrict__ order) {
   __shared__ int cnt[kMaxExperts];
   __shared__ int nxt[kMaxExperts];
-  const int n = T * top;
-  for (int e = threadIdx.x; e < E; e += kRouteThreads) cnt[e] = 0;
+  const int n = T * top, tid = threadIdx.x;
+  for (int e = tid; e < E; e += kRouteThreads) cnt[e] = 0;
   __syncthreads();
-  auto expert_of = [&](int p) {
-    int id = ids ? ids[p / top] : p / top;      // no ids: the table has one row per token of the step
-    id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);
-    const int e = table[(long)id * top + p % top];
-    return e < 0 ? 0 : (e >= E ? E - 1 : e);
-  };
-  for (int p = threadIdx.x; p < n; p += kRouteThreads) atomicAdd(&cnt[expert_of(p)], 1);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int acc = 0;
-    for (int e = 0; e < E; ++e) {
-      seg[e] = acc;
-      nxt[e] = acc;
-      acc += cnt[e];
+  int ex[kRouteU];
+  auto experts = [&](int p0) {   // of pairs p0 + tid + 1024 u (behind the end: the last pair's)
+    int id[kRouteU];
+#pragma unroll
+    for (int u = 0; u < kRouteU; ++u) {
+      const int t = (int)min((long)p0 + u * kRouteThreads + tid, (long)n - 1) / top;
+      id[u] = ids ? ids[t] : t;                 // no ids: the table has one row per token of the step
     }
-    seg[E] = acc;
+#pragma unroll
+    for (int u = 0; u < kRouteU; ++u) {
+      const int p = (int)min((long)p0 + u * kRouteThreads + tid, (long)n - 1);
+      ex[u] = table[(long)min(max(id[u], 0), vocab - 1) * top + p % top];
+    }
+#pragma unroll
+    for (int u = 0; u < kRouteU; ++u) ex[u] = min(max(ex[u], 0), E - 1);
+  };
+  for (long p0 = 0; p0 < n; p0 += kRouteU * kRouteThreads) {
+    experts((int)p0);
+#pragma unroll
+    for (int u = 0; u < kRouteU; ++u)
+      if (p0 + u * kRouteThreads + tid < n) atomicAdd(&cnt[ex[u]], 1);
   }
   __syncthreads();
-  for (int p = threadIdx.x; p < n; p += kRouteThreads) order[atomicAdd(&nxt[expert_of(p)], 1)] = p;
+  if (tid < 64) {   // running sums of the counts, 64 experts at a time
+    int acc = 0;
+    for (int e0 = 0; e0 < E; e0 += 64) {
+      const int c = e0 + tid < E ? cnt[e0 + tid] : 0;
+      int v = c;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int below = __shfl_up(v, o, 64);
+        if (tid >= o) v += below;
+      }
+      if (e0 + tid < E) seg[e0 + tid] = nxt[e0 + tid] = acc + v - c;
+      acc += __shfl(v, 63, 64);
+    }
+    if (tid == 0) seg[E] = acc;
+  }
+  __syncthreads();
+  for (long p0 = 0; p0 < n; p0 += kRouteU * kRouteThreads) {
+    if (n > kRouteU * kRouteThreads) experts((int)p0);
+#pragma unroll
+    for (int u = 0; u < kRouteU; ++u) {
+      const long p = p0 + u * kRouteThreads + tid;
+      if (p < n) order[atomicAdd(&nxt[ex[u]], 1)] = (int)p;
+    }
+  }
 }
 
 // grid (row tiles of 16 RT pairs: at most pairs / (16 RT) + E, column blocks): 4 waves side by side along the columns, each

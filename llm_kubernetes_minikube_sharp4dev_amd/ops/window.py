@@ -174,7 +174,7 @@ def run_experts(h, ids, table, w_gate_up, w_down, top: int):
         if h.dtype == torch.bfloat16 and _grouped(T, T * top, E, W, ffp):
             # prompt-sized steps on the framework's dense GEMM tiles, one GEMM per expert inside one launch: the first
             # product reads each pair's token row in place, the second writes each result into its pair's row
-            mid = lib().gemm_grouped(h, seg, w_gate_up, True, torch.div(order, top, rounding_mode="floor"), None)
+            mid = lib().gemm_grouped(h, seg, w_gate_up, True, order, None, int(top))
             return lib().gemm_grouped(mid, seg, w_down, False, None, order)
         mid = lib().moe_gemm(h, order, seg, w_gate_up, int(top), True)          # [T * top, ffp], sorted-pair order
         return lib().moe_gemm(mid, order, seg, w_down, int(top), False)         # [T * top, W], pair order

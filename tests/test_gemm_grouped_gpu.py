@@ -42,5 +42,21 @@ def test_rows_per_expert(counts, swiglu, N, K):
     got = ops.lib().gemm_grouped(x.cuda(), seg.cuda(), w.cuda(), swiglu, perm.cuda(), None).double().cpu()
     tol = 1.05 * tol + 1e-4      # second order terms, f32 sums of K products of standard deviation 1
     assert bool(((got - want).abs() <= tol).all()), float(((got - want).abs() - tol).max())
+    pairs = ops.lib().gemm_grouped(x.cuda(), seg.cuda(), w.cuda(), swiglu, (3 * perm + perm % 3).cuda(), None, 3).double().cpu()
+    assert torch.equal(pairs, got)
     back = ops.lib().gemm_grouped(x[perm.long()].cuda(), seg.cuda(), w.cuda(), swiglu, None, perm.cuda()).double().cpu()
     assert torch.equal(back[perm.long()], got)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,top,E,by_id", [(1, 1, 1, True), (4096, 2, 16, True), (4097, 2, 16, True), (3000, 3, 200, False), (20000, 2, 1024, True), (5, 8, 65, False)])
+def test_pairs_sorted_by_expert(T, top, E, by_id):
+    g = torch.Generator().manual_seed(T)
+    vocab = 50 if by_id else T
+    table = torch.randint(-1, E + 1, (vocab, top), generator=g, dtype=torch.int32)
+    ids = torch.randint(-2, vocab + 2, (T,), generator=g, dtype=torch.int32) if by_id else None
+    seg, order = ops.lib().moe_route(None if ids is None else ids.cuda(), table.cuda(), E)
+    e = (table[ids.long().clamp(0, vocab - 1)] if by_id else table).clamp(0, E - 1).reshape(-1)
+    assert torch.equal(seg.cpu()[1:].long(), torch.bincount(e, minlength=E).cumsum(0)) and int(seg[0]) == 0
+    order = order.cpu().long()
+    assert torch.equal(order.sort().values, torch.arange(T * top)) and torch.equal(e[order], e.sort().values)
