@@ -132,18 +132,20 @@ __global__ __launch_bounds__(256, LK_DECODE_WG_PER_CU) void paged_decode_kernel(
   short8 kr[2][KK], vr[NVL];
   // k_begin is block-aligned (split % BS == 0, k_start a multiple of BS): row rel of the
   // split sits at slot rel % BS of its block
+  // (non-temporal: a step reads every key once, and its weights and other layers pass through the caches before the next; 120 sequences
+  // of 950 keys, 8 kv heads of 128: 102 us (4.6 TB/s) -> 89 us (5.2 TB/s), a single sequence alike)
   auto load_chunk = [&](int c, short8 (&kd)[2][KK], short8 (&vd)[NVL]) {
     const int base = 32 * c;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       const bf16_t* kp = blk_base(kc, base + 16 * t) + (min(base + 16 * t + r16, nkeys - 1) % BS) * D + 8 * h4;
 #pragma unroll
-      for (int kk = 0; kk < KK; ++kk) kd[t][kk] = *reinterpret_cast<const short8*>(kp + 32 * kk);
+      for (int kk = 0; kk < KK; ++kk) kd[t][kk] = __builtin_nontemporal_load(reinterpret_cast<const short8*>(kp + 32 * kk));
     }
 #pragma unroll
     for (int i = 0; i < NVL; ++i) {
       const int rel = min(base + i * RPL + lane / CPR, nkeys - 1);
-      vd[i] = *reinterpret_cast<const short8*>(blk_base(vc, base + i * RPL) + (rel % BS) * D + (lane % CPR) * 8);
+      vd[i] = __builtin_nontemporal_load(reinterpret_cast<const short8*>(blk_base(vc, base + i * RPL) + (rel % BS) * D + (lane % CPR) * 8));
     }
   };
 
