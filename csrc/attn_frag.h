@@ -23,6 +23,12 @@ struct El<float> {
 };
 
 LK_DEVICE uint4_t ld16(const void* p) { return *reinterpret_cast<const uint4_t*>(p); }
+// NT: read once (the keys and values of a decode step; 64 sequences of 950 keys, 4 kv heads: sigmoid attention 34.1 -> 32.9 us, windowed
+// softmax 21.9 -> 20.9 us)
+template <bool NT>
+LK_DEVICE uint4_t ld16_kv(const void* p) {
+  return NT ? __builtin_nontemporal_load(reinterpret_cast<const uint4_t*>(p)) : ld16(p);
+}
 
 // S^T += A(16 keys x one 16-byte fragment of dims) . B(the columns' same dims)
 template <typename T>

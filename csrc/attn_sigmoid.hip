@@ -65,7 +65,7 @@ LK_DEVICE float sig_weight(float s, float r1, float r2, float pb, int d) {
 // bf16: the next step's K fragments are requested as soon as this step's Q.K MFMAs have
 // consumed the current ones, and this step's V fragments before the weights are computed, so
 // both fly under the transcendental-heavy weight arithmetic.
-template <typename T, int PAD>
+template <typename T, int PAD, bool NT = false>
 LK_DEVICE void sig_run(const SigParams& p, const uint4_t (&qf)[PAD / (4 * El<T>::V)], int kvh, const int* bt, int k0,
                        int k1, int step0, int stride, bool cvalid, int qpos, float r1, float r2, float pb,
                        floatx4 (&o)[PAD / 16]) {
@@ -83,7 +83,7 @@ LK_DEVICE void sig_run(const SigParams& p, const uint4_t (&qf)[PAD / (4 * El<T>:
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
         const int d0 = s * 4 * EV + g * EV;
-        kf[t][s] = d0 < p.dim ? ld16(kr + d0) : uint4_t{0u, 0u, 0u, 0u};
+        kf[t][s] = d0 < p.dim ? ld16_kv<NT>(kr + d0) : uint4_t{0u, 0u, 0u, 0u};
       }
     }
   };
@@ -108,7 +108,7 @@ LK_DEVICE void sig_run(const SigParams& p, const uint4_t (&qf)[PAD / (4 * El<T>:
 #pragma unroll
       for (int vt = 0; vt < VT; ++vt) {
         const int vd = vt * 16 + n16;
-        vf[vt] = (vt * 16 < p.vdim && vd < p.vdim) ? ld16(vrow + (long)vd * p.BS) : uint4_t{0u, 0u, 0u, 0u};
+        vf[vt] = (vt * 16 < p.vdim && vd < p.vdim) ? ld16_kv<NT>(vrow + (long)vd * p.BS) : uint4_t{0u, 0u, 0u, 0u};
       }
       const int kn = kb + 32 * stride;
       if (kn < k1) load_k(kn, kf);
@@ -246,7 +246,7 @@ __global__ __launch_bounds__(256) void sigattn_decode_kernel(SigParams p, const 
   const int nsteps = (ctx + 31) / 32, spz = (nsteps + Z - 1) / Z;
   const int s0 = z * spz, s1 = min(nsteps, s0 + spz);
   if (s0 < s1)
-    sig_run<T, PAD>(p, qf, kvh, p.bt + (long)b * p.bt_stride, 32 * s0, min(ctx, 32 * s1), w, 4, cvalid, ctx - 1,
+    sig_run<T, PAD, true>(p, qf, kvh, p.bt + (long)b * p.bt_stride, 32 * s0, min(ctx, 32 * s1), w, 4, cvalid, ctx - 1,
                     p.r1[head], p.r2[head], p.pb[head], o);
   sum_waves<VT>(o, red);
   if (w == 0 && cvalid) {

@@ -90,7 +90,7 @@ LK_DEVICE float cap_f(float s, float cap, float icap) {
 // running maximum (equal in the four lane groups of a column), this lane group's share of the sum, and
 // the O^T accumulators.  Key order inside a step: see attn_sigmoid.hip (lane group g holds the weights
 // of the 8 consecutive keys 8g .. 8g + 7).
-template <typename T, int PAD>
+template <typename T, int PAD, bool NT = false>
 LK_DEVICE void sink_run(const SinkParams& p, const void* kcache, const void* vcache, const uint4_t (&qf)[PAD / (4 * El<T>::V)], int kvh,
                         const int* bt, int k0, int k1, int step0, int stride, bool cvalid, int qpos, int klo, float hs, float& m,
                         float& l, floatx4 (&o)[PAD / 16]) {
@@ -110,7 +110,7 @@ LK_DEVICE void sink_run(const SinkParams& p, const void* kcache, const void* vca
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
         const int d0 = s * 4 * EV + g * EV;
-        kf[t][s] = d0 < p.dim ? ld16(kr + d0) : uint4_t{0u, 0u, 0u, 0u};
+        kf[t][s] = d0 < p.dim ? ld16_kv<NT>(kr + d0) : uint4_t{0u, 0u, 0u, 0u};
       }
     }
   };
@@ -134,7 +134,7 @@ LK_DEVICE void sink_run(const SinkParams& p, const void* kcache, const void* vca
 #pragma unroll
       for (int vt = 0; vt < VT; ++vt) {
         const int vd = vt * 16 + n16;
-        vf[vt] = (vt * 16 < p.vdim && vd < p.vdim) ? ld16(vrow + (long)vd * p.BS) : uint4_t{0u, 0u, 0u, 0u};
+        vf[vt] = (vt * 16 < p.vdim && vd < p.vdim) ? ld16_kv<NT>(vrow + (long)vd * p.BS) : uint4_t{0u, 0u, 0u, 0u};
       }
       const int kn = kb + 32 * stride;
       if (kn < k1) load_k(kn, kf);
@@ -360,10 +360,10 @@ __global__ __launch_bounds__(256) void sinkattn_decode_kernel(SinkParams p, cons
   const int nwin = (ctx - k0 + 31) / 32, nsteps = nwin + (n1 + 31) / 32, spz = (nsteps + Z - 1) / Z;
   const int s0 = z * spz, s1 = min(nsteps, s0 + spz);
   if (s0 < min(s1, nwin))
-    sink_run<T, PAD>(p, p.kc, p.vc, qf, kvh, p.bt + (long)b * p.bt_stride, k0 + 32 * s0, min(ctx, k0 + 32 * min(s1, nwin)), w, 4, cvalid,
+    sink_run<T, PAD, true>(p, p.kc, p.vc, qf, kvh, p.bt + (long)b * p.bt_stride, k0 + 32 * s0, min(ctx, k0 + 32 * min(s1, nwin)), w, 4, cvalid,
                      ctx - 1, klo, p.hscale[head], m, l, o);
   if (max(s0, nwin) < s1)
-    sink_run<T, PAD>(p, pooled ? p.pkc : p.kc, pooled ? p.pvc : p.vc, qf, kvh, p.bt + (long)b * p.bt_stride, 32 * (max(s0, nwin) - nwin),
+    sink_run<T, PAD, true>(p, pooled ? p.pkc : p.kc, pooled ? p.pvc : p.vc, qf, kvh, p.bt + (long)b * p.bt_stride, 32 * (max(s0, nwin) - nwin),
                      min(n1, 32 * (s1 - nwin)), w, 4, cvalid, n1 - 1, 0, p.hscale[head], m, l, o);
   merge_waves<EXACT, VT>(m, l, o, red, ml);
   if (w == 0 && cvalid) {
