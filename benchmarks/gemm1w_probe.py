@@ -8,11 +8,8 @@ plus a numerics check of the new kernel against an fp32 torch matmul.
 
 ``--build`` compiles the probe library from the tracked ``csrc/gemm1w.hip`` (its ``extern "C"
 lk_gemm1w_c`` entry) into ``benchmarks/probes/bin/libgemm1w.so`` with hipcc first -- the
-library is a build product (git-ignored), the source is the serving kernel itself.  The
-schedule-sweep arms of ``profiles/r5_gemm1w/`` (``libgemm1w_c7`` / ``_n2``...) were builds of
-intermediate versions of that file; the kept schedule is the one in its history
-(``git log -- csrc/gemm1w.hip``), so rebuilding a sweep arm means checking out that commit's
-``csrc/gemm1w.hip`` and passing ``--build --so <name>``.
+library is a build product (git-ignored), the source is the serving kernel itself.  A sweep of its
+slots (``profiles/gemm1w_slots.md``) builds copies with other constants in ``Tile<BM>`` and passes them as ``--so a.so,b.so``.
 """
 from __future__ import annotations
 
@@ -38,6 +35,7 @@ def build_probe(out: str) -> str:
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     os.makedirs(os.path.dirname(os.path.abspath(out)), exist_ok=True)
     cmd = ["/opt/rocm/bin/hipcc", "--offload-arch=gfx950", "-O3", "-std=c++17", "-shared", "-fPIC", "-ffp-contract=fast",
+           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
            "-Wno-inline-asm", "-I", os.path.join(root, "csrc"), os.path.join(root, "csrc", "gemm1w.hip"), "-o", out]
     subprocess.run(cmd, check=True)
     return out

@@ -1,39 +1,39 @@
 // K2, prefill regime, one wave per SIMD: Y[M, N] = epilogue(X[M, K] . W[N, K]^T).
 //
-// A 256 x 256-tile, one-wave-per-SIMD schedule (MT256x256x64, 16x16 MFMA, direct-to-LDS loads of
-// both operands, two-deep global prefetch, one-deep local prefetch) written in HIP for our
-// K-contiguous operands and
-// extended with the fused serving epilogues of gemm.hip and with 192 / 128-row tiles:
-//   * 256 threads = 4 waves, ONE per SIMD, as 2 (M) x 2 (N); each wave owns (BM / 2) x 128 outputs =
-//     MB x 8 v_mfma_f32_16x16x32_bf16 accumulators (MB = BM / 32: 8 / 6 / 4) pinned to AGPRs by
-//     inline-asm MFMAs ("+a"); the first K-tile's MFMAs take an inline 0 as C (no zeroing pass);
-//   * BK = 64, two LDS stages of (BM + 256) x 128 B (X rows | W rows, (row >> 1) & 7 chunk XOR
-//     applied on the DMA SOURCE: lane-linear LDS image, conflict-free ds_read_b128);
-//   * a full K-tile of fragments lives in registers (kk 0 and kk 1 sets); every LDS read, LDS-DMA
-//     issue and wait is inline asm placed by hand among the NM = 16 MB MFMAs of a K-tile (BM 256:
-//     positions below; 192 / 128: Tile<BM>):
-//       top          : lgkmcnt(0) -- the (t, kk 0) fragments read at the end of K-tile t-1
-//       MFMA  0..15  : the 16 fragment reads of (t, kk 1), one per MFMA
-//       MFMA 26      : lgkmcnt(0) + s_barrier -- every wave is done with stage t & 1
-//       MFMA 28..103 : the 16 LDS-DMA pieces (1 KB each) of K-tile t+2 into stage t & 1, one per
-//                      5 MFMAs, M0 for the next piece written 2 MFMAs after each issue (no s_nop)
-//       MFMA 108     : vmcnt(16) + s_barrier -- K-tile t+1 (issued one K-tile ago) has landed
-//       MFMA 108..123: the 16 fragment reads of (t+1, kk 0)
-//     (probe sweeps of these positions, the wait placement and the M0 lag:
-//     benchmarks/gemm1w_probe.py, profiles/r5_gemm1w/);
-//   * row tiles of 192 / 128 fill the 256 CUs where 256-row tiles leave most of a wave idle (the
-//     serving bench's mixed steps: M = prefill chunk + ~105 decode rows); the dispatch picks the
-//     row tile per M bucket from measurements (ops.tune_gemm, benchmarks/gemm_tiles.py);
-//   * one tile per workgroup: the hardware starts the next workgroup on a CU while the finished
-//     one's epilogue stores drain (a persistent walk with the next tile's first K-tiles DMA'd
-//     during the last one measured 1-3 % slower);
-//   * operands swapped in the MFMA (A <- W rows, B <- X rows) and the W rows of every 32-row
-//     block permuted (pair_col) so a lane ends with one output row and 8 consecutive columns
-//     per fragment pair: 16-B epilogue stores; SwiGLU pairs gate / up of the same columns;
-//   * epilogues (same contracts and rounding as gemm.hip): NONE, SWIGLU, BIAS, BIAS_GELU,
-//     BIAS_RELU, PARTIAL (split-K fp32 slabs), RESID (r += acc in place + per-row partial sums of
-//     squares), QKV (RoPE + paged-KV scatter); NONE / SWIGLU / QKV take the folded-RMSNorm row
-//     scale (LkEpi::ss_in); rows past M are dropped by the buffer descriptors' range checks.
+// A workgroup of 4 waves, one per SIMD, owns a BM x 256 tile (BM = 256 / 192 / 128), a wave (BM / 2) x 128 of it as MB x 8
+// v_mfma_f32_16x16x32_bf16 accumulators (MB = BM / 32), which fill the AGPRs at BM 256.  K advances by 64 (whole 128-byte lines).
+//
+// What a K-tile costs at BM 256, in cycles of a CU: 128 MFMAs of 16 per SIMD = 2,048; 32 fragment reads of 1 KB per wave, 128 KB at
+// 128 bytes = 1,024 of LDS; 64 KB of LDS-DMA writes = 512.  LDS is busy three quarters of the time, so its work has to be spread over the
+// K-tile, and a load takes longer than a K-tile to arrive, so a piece of LDS must be refilled as soon as it has been read.  Hence:
+//   * X is resident, W streams.  All X fragments of a K-tile (2 MB of them) sit in registers, those of the next in a second set.  A W
+//     fragment serves MB MFMAs in a row and is read WA fragments ahead into a ring of 4; the order is n-major, both halves of K of a
+//     column fragment together, so LDS gets one W read per MB MFMAs all along.
+//   * A K-tile is two phases, each opened by one barrier that both hands over what has landed and frees what has been read:
+//       phase A (W columns 0-63 of a wave's 128 are being read): X's stage is free, its fragments being in registers, and so is the
+//         second half of W's stage of the K-tile before: refill W half 2 of t + 1, then X of t + 2;
+//       phase B (W columns 64-127): W half 1 of t is free: refill it with t + 2; X fragments of t + 1 are read.
+//     Every refill is requested between 1 and 1.5 K-tiles before the barrier that needs it, and the same NP newer requests are in flight
+//     at both barriers (s_waitcnt vmcnt(NP)), without draining.
+//   * The reads are plain loads, so the compiler counts lgkmcnt per fragment; the order is pinned by scheduling fences.  The LDS-DMA is
+//     inline asm (no register results) with M0 written one MFMA before.  The slots within a phase (Tile<BM>) are free parameters within
+//     the asserted limits; they were swept (profiles/gemm1w_slots.md).
+// One tile per workgroup: the hardware starts the next workgroup on a CU while the finished one's stores drain.  PERSIST, for short K
+// where the load ramp is a third of a tile, and an even number of K-tiles (K-tile t lies in stage t & 1 of every tile): one workgroup per
+// CU walks the tiles, and the last two K-tiles' refills are the next tile's first ones.
+//
+// Measured with cold weights: 4096 x 4096 x 4096 on 256-row tiles 91 us (1,500 TFLOP/s; MFMAs alone about 80, with the reads 86 - 89),
+// M 2664 on 192-row tiles 69 us, 2664 x 6144 x 4096 on 128-row tiles 107 us; 62500 x 3072 x 768 persistent 257 us.
+//
+// Layout: two stages of (BM + 256) rows x 128 bytes (X rows | W rows), the 16-byte chunk c of a row at c ^ ((row >> 1) & 7), applied to
+// the DMA's SOURCE: the LDS image is lane-linear and the fragment reads meet no bank twice.  The operands are swapped in the MFMA (A <- W
+// rows, B <- X rows) and the W rows of every 32-row block permuted so that a lane ends with one output row and 8 consecutive columns per
+// fragment pair: 16-byte stores; SwiGLU pairs gate (half 1) and up (half 2) of the same columns.
+//
+// Row tiles of 192 / 128 fill the 256 CUs where 256-row tiles leave most of a wave idle; the dispatch picks the row tile per M bucket
+// from measurements (ops.tune_gemm) or a cost rule.  Epilogues (same contracts and rounding as gemm.hip): NONE, SWIGLU, BIAS, BIAS_GELU,
+// BIAS_RELU, PARTIAL (split-K fp32 slabs), RESID (r += acc in place + per-row partial sums of squares), QKV (RoPE + paged-KV scatter);
+// NONE / SWIGLU / QKV take the folded-RMSNorm row scale (LkEpi::ss_in); rows past M are dropped by the buffer descriptors' range checks.
 #include <type_traits>
 #include <utility>
 
@@ -44,32 +44,30 @@ namespace {
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
-typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
+typedef const __attribute__((address_space(3))) short8* lds_frag_t;
 
 constexpr int kBN = 256, kBK = 64;
 constexpr int kRowB = kBK * 2;          // 128-B LDS rows
 constexpr int kLdsEpi = 8192;           // epilogue scratch above the stages (row scales, RESID sums)
 
-// Row-tile height BM (256, 192 or 128; the column tile is always 256): the 4 waves sit 2 (M) x 2 (N),
-// each owning (BM / 2) x 128 outputs = MB x 8 accumulators of 16 x 16.  A K-tile is NM = 16 MB
-// MFMAs, NR = MB + 8 fragment reads per kk set and NP = BM / 32 + 8 LDS-DMA pieces per wave.
-// Smaller row tiles fill the 256 CUs where 256-row tiles leave most of a wave idle (M 2664,
-// N 4096: 176 tiles of 256 rows, 224 of 192 rows -- the row tile hipBLASLt picks there).
+// A K-tile is NM MFMA slots of a wave; slot i multiplies X fragment m = i % MB with W fragment f = i / MB = 2 n + kk.  Barrier S1 opens
+// phase B, S0 phase A of the next K-tile, both 8 MB slots apart and WA fragments ahead of the MFMAs that use what they hand over.
 template <int BM>
 struct Tile {
-  static constexpr int MB = BM / 32, NM = 16 * MB, NR = MB + 8, PX = BM / 32, NP = PX + 8;
+  static constexpr int MB = BM / 32, NM = 16 * MB, PX = BM / 32, NP = PX + 8;  // PX / 8: LDS-DMA pieces (1 KB) of X / W per wave
   static constexpr int kOpX = BM * kRowB;                // X rows of one stage
   static constexpr int kStage = kOpX + 256 * kRowB;      // X rows then W rows
   static constexpr int kLdsStages = 2 * kStage;          // 128 / 112 / 96 KB
   static constexpr int kLds = kLdsStages + kLdsEpi;
-  // K-loop schedule (MFMA indices within the NM of a K-tile): barrier 1, first DMA piece, DMA
-  // spacing, M0 lag, barrier 2
-  static constexpr int B1 = BM == 256 ? 26 : BM == 192 ? 24 : 14;
-  static constexpr int D0 = B1 + 2;
-  static constexpr int DS = BM == 256 ? 5 : BM == 192 ? 4 : 2;
-  static constexpr int LAG = BM == 128 ? 1 : 2;
-  static constexpr int B2 = BM == 256 ? 108 : BM == 192 ? 82 : 48;
-  static_assert(NR - 1 < B1 && B1 < D0 && LAG < DS && D0 + DS * (NP - 1) + LAG < B2 && B2 + NR <= NM, "schedule");
+  static constexpr int WA = 3;                           // W fragments read ahead
+  static constexpr int S1 = (8 - WA) * MB, S0 = (16 - WA) * MB, PH = 8 * MB;
+  // slots within a phase: phase A's 4 W pieces, then its PX X pieces; phase B's 4 W pieces and its 2 MB X reads.  (first, step); chosen
+  // so that few of them fall on the slots of the W reads (multiples of MB): one wave issues everything, and a slot is four issues long
+  static constexpr int AW0 = 1, AWS = BM == 128 ? 2 : BM == 192 ? 3 : 4, AX0 = WA * MB + 1, AXS = 5;
+  static constexpr int BW0 = BM == 192 ? 4 : 2, BWS = MB, XR0 = BM == 192 ? 2 : 1, XRS = BM == 192 ? 3 : 2;
+  static_assert(WA >= 1 && WA <= 3, "ring of 4");
+  static_assert(AW0 >= 1 && AW0 + 3 * AWS < WA * MB && AX0 > WA * MB && AX0 + AXS * (PX - 1) < PH, "phase A");
+  static_assert(BW0 >= 1 && BW0 + 3 * BWS < PH && XR0 + XRS * (2 * MB - 1) < PH, "phase B");
 };
 
 enum { E_NONE = 0, E_SWIGLU = 1, E_BIAS = 2, E_BIAS_GELU = 3, E_BIAS_RELU = 4, E_PARTIAL = 5, E_RESID = 6,
@@ -110,11 +108,15 @@ LK_DEVICE void mfma(floatx4& acc, const short8& a, const short8& b) {
 LK_DEVICE void mfma0(floatx4& acc, const short8& a, const short8& b) {
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(acc) : "v"(a), "v"(b));
 }
-LK_DEVICE void set_m0(unsigned v) { asm volatile("s_mov_b32 m0, %0" ::"s"(v) : "memory", "m0"); }
+template <int OFF>
+LK_DEVICE void set_m0(unsigned base) { asm volatile("s_add_u32 m0, %0, %1" ::"s"(base), "i"(OFF) : "memory", "m0", "scc"); }
 LK_DEVICE u32x4_t srd(const void* p, long bytes) {  // buffer descriptor words, wave-uniform
   const unsigned long a = reinterpret_cast<unsigned long>(p);
   return u32x4_t{rfl((unsigned)a), rfl((unsigned)(a >> 32)), (unsigned)min(bytes, 0x7FFFFFF0L), 0x00020000u};
 }
+
+// the number of the event at slot u of a phase (n of them from slot `first` on, `step` apart), or -1
+constexpr int every(int u, int first, int step, int n) { return u >= first && (u - first) % step == 0 && (u - first) / step < n ? (u - first) / step : -1; }
 
 // vector-memory operations per lane of the plain / bias epilogues (bias loads, then stores): the
 // persistent walk's counted wait for the next tile's first K-tile skips them
@@ -124,8 +126,8 @@ constexpr bool persistable(int e) { return e == E_NONE || e == E_BIAS || e == E_
 
 // SCP: partial-sum planes of the folded-RMSNorm row scale loaded per row (0: no row scale; 16 covers
 // a 4096-wide producer, 32 an 8192-wide one).  PERSIST: one workgroup per CU walks the tiles
-// blockIdx.x, + gridDim.x, ...; the next tile's first two K-tiles are DMA'd during the current
-// tile's last two, so its load ramp hides behind the current epilogue (short-K shapes: the
+// blockIdx.x, + gridDim.x, ...; the next tile's first refills are requested during the current
+// tile's last two K-tiles, so its load ramp hides behind the current epilogue (short-K shapes: the
 // encoder's K = 768 projections, 12 K-tiles per tile)
 // GS (grouped form, lk_gemm1w_grouped): rows sorted by expert, sources gathered and results scattered through LkEpi
 template <int EPI, int SCP, int BM, bool PERSIST = false, bool GS = false>
@@ -138,7 +140,7 @@ __global__ __launch_bounds__(256, 1) void gemm1w_kernel(const bf16_t* __restrict
   static_assert(!SC || scalable(EPI), "row scale");
   static_assert(!PERSIST || (persistable(EPI) && !SC), "persistent walk: plain / bias epilogues");
   using TL = Tile<BM>;
-  constexpr int MB = TL::MB, NM = TL::NM, NR = TL::NR, PX = TL::PX, NP = TL::NP, WM = BM / 2;
+  constexpr int MB = TL::MB, NM = TL::NM, PX = TL::PX, NP = TL::NP, WM = BM / 2;
   constexpr int kOpX = TL::kOpX, kStage = TL::kStage, kLdsStages = TL::kLdsStages;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
@@ -181,191 +183,191 @@ __global__ __launch_bounds__(256, 1) void gemm1w_kernel(const bf16_t* __restrict
     tm = first + (L % per_group) % gm;
     tn = tn0 + (L % per_group) / gm;  // (tn0: a column-split launch's first column tile)
   };
-  const u32x4_t xsrd = srd(X, (long)(GS && ea.gather ? ea.x_rows : M) * ldx * 2);
-  const u32x4_t wsrd = srd(W, (long)(EPI == E_SWIGLU ? 2 * I : (tn0 + TN) * kBN) * K * 2);
+  u32x4_t xsrd = srd(X, (long)(GS && ea.gather ? ea.x_rows : M) * ldx * 2);
+  u32x4_t wsrd = srd(W, (long)(EPI == E_SWIGLU ? 2 * I : (tn0 + TN) * kBN) * K * 2);
   const unsigned lds0 = static_cast<unsigned>(reinterpret_cast<uintptr_t>((lds_ptr_t)smem));
-  const unsigned ldsx = rfl(lds0 + (BM / 4) * w * kRowB), ldsw = rfl(lds0 + kOpX + 64 * w * kRowB);
+  const int wrow = 128 * (w >> 1) + 32 * (w & 1);  // first W row of this wave's pieces of half 1; half 2: + 64
+  const unsigned ldsx = rfl(lds0 + (BM / 4) * w * kRowB), ldsw = rfl(lds0 + kOpX + wrow * kRowB);
 
-  // ---- LDS-DMA piece i (0..NP-1) of a K-tile: rows BM/4 w + 8 i + (lane >> 3) of X (i < PX) or
-  // 64 w + 8 (i - PX) + (lane >> 3) of W, 16-B chunk lane & 7 (source chunk swizzled); per-lane
-  // row offsets of the tile
+  // ---- LDS-DMA pieces of a K-tile, 8 rows each: X piece i covers rows BM/4 w + 8 i .., W piece 4 h + j rows wrow + 64 h + 8 j ..;
+  // lane l brings the 16-byte chunk of slot l & 7 of row l >> 3.  Byte offsets of this lane's sources at column 0 (32-bit: the host
+  // keeps every operand under 2^31 bytes).  A piece's rows are 8 apart, so
+  // (row >> 1) & 7 = (lr8 >> 1) ^ 4 (piece & 1); LDS row 8 j + lr8 of a 32-row block of W holds column
+  // 8 (lr8 >> 2) + (lr8 & 3) + 16 (j & 1) + 4 (j >> 1) of it.
   const int lr8 = lane >> 3, lc8 = lane & 7;
-  unsigned xo[PX], wo[8], xo2[PX], wo2[8];  // this tile's / (PERSIST) the next tile's
-  int par = 0;  // stage of tile-relative K-tile t: (t + par) & 1 (a persistent walk carries it on)
-  // (32-bit: the host keeps every operand under 2^31 bytes).  Closed forms with the piece index
-  // i in immediates only -- per-i lane constants held across the tile loop spill:
-  //   row = BM/4 w + 8 i + lr8;  swz(row) = (lr8 >> 1) ^ 4 (i & 1)  (BM/8 w is a multiple of 8);
-  //   W row = lane part + 32 (i >> 2) + 16 (i & 1) + 4 ((i >> 1) & 1)   (pair_col of row & 31)
+  unsigned xo[PX], wo[8];
   const unsigned ldxb = (unsigned)ldx * 2, kb = (unsigned)K * 2;
   const unsigned ch0 = (unsigned)((lc8 ^ (lr8 >> 1)) << 4);
   auto offsets = [&](int tm, int tn, unsigned (&xo)[PX], unsigned (&wo)[8]) {
-    const unsigned xb = (unsigned)(tm * BM + (BM / 4) * w + lr8) * ldxb;
-    const int lanew = 8 * (lr8 >> 2) + (lr8 & 3);
-    const unsigned wl = EPI == E_SWIGLU ? (unsigned)((w & 1) * I + tn * 128 + (w >> 1) * 64 + lanew)
-                                        : (unsigned)(tn * kBN + 64 * w + lanew);
-    const unsigned wb = wl * kb;
+    const int xr = tm * BM + (BM / 4) * w + lr8;
 #pragma unroll
     for (int i = 0; i < PX; ++i) {
       if constexpr (GS) {  // rows past the expert's end point behind the descriptor's range: zeros
-        const int tr = tm * BM + (BM / 4) * w + lr8 + 8 * i;
+        const int tr = xr + 8 * i;
         const int src = tr < M ? (ea.gather ? ea.gather[tr] / ea.top : tr) : -1;
         xo[i] = src >= 0 ? (unsigned)src * ldxb + (ch0 ^ (unsigned)((i & 1) << 6)) : 0xFFFFFF00u;
       } else {
-        xo[i] = xb + (unsigned)(8 * i) * ldxb + (ch0 ^ (unsigned)((i & 1) << 6));
+        xo[i] = (unsigned)(xr + 8 * i) * ldxb + (ch0 ^ (unsigned)((i & 1) << 6));
       }
     }
+    // SwiGLU: half 1 holds the gate rows of 64 output columns per column half, half 2 the up rows of the same
+    const unsigned wl = (EPI == E_SWIGLU ? (unsigned)(tn * 128 + (w >> 1) * 64 + 32 * (w & 1)) : (unsigned)(tn * kBN + wrow)) +
+                        (unsigned)(8 * (lr8 >> 2) + (lr8 & 3));
+    const unsigned half = EPI == E_SWIGLU ? (unsigned)I : 64u;
 #pragma unroll
     for (int i = 0; i < 8; ++i)
-      wo[i] = wb + (unsigned)(32 * (i >> 2) + 16 * (i & 1) + 4 * ((i >> 1) & 1)) * kb + (ch0 ^ (unsigned)((i & 1) << 6));
+      wo[i] = (wl + (i >> 2) * half + (unsigned)(16 * (i & 1) + 4 * ((i >> 1) & 1))) * kb + (ch0 ^ (unsigned)((i & 1) << 6));
   };
-  auto piece_m0 = [&](int t, int i) -> unsigned {  // LDS base of piece i of (tile-relative) K-tile t
-    return i < PX ? ldsx + (unsigned)(((t + par) & 1) * kStage + 8 * i * kRowB)
-                  : ldsw + (unsigned)(((t + par) & 1) * kStage + 8 * (i - PX) * kRowB);
+  // M0 = LDS address of piece i of the K-tile in stage P (one scalar instruction)
+  auto m0_x = [&](auto p_t, auto i_t) { set_m0<decltype(p_t)::value * kStage + 8 * decltype(i_t)::value * kRowB>(ldsx); };
+  auto m0_w = [&](auto p_t, auto i_t) {
+    constexpr int i = decltype(i_t)::value;
+    set_m0<decltype(p_t)::value * kStage + (64 * (i >> 2) + 8 * (i & 3)) * kRowB>(ldsw);
   };
-  // issue piece i of K-tile t (M0 already holds its LDS base); NEXT: K-tile t - nk of the next tile
-  auto dma = [&](bool NEXT, int t, int i) {  // (NEXT is a constant at every call: folded when inlined)
-    const unsigned so = rfl((unsigned)(NEXT ? t - nk : kt0 + t) * (kBK * 2));
-    const unsigned xv = NEXT ? xo2[i < PX ? i : 0] : xo[i < PX ? i : 0];
-    const unsigned wv = NEXT ? wo2[i < PX ? 0 : i - PX] : wo[i < PX ? 0 : i - PX];
-    if (i < PX) asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(xv), "s"(xsrd), "s"(so) : "memory");
-    else asm volatile("buffer_load_dwordx4 %0, %1, %2 offen sc0 sc1 lds" ::"v"(wv), "s"(wsrd), "s"(so) : "memory");
-  };
+  // the piece at column offset so (M0 holds its LDS base)
+  auto dma_x = [&](unsigned so, int i) { asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(xo[i]), "s"(xsrd), "s"(so) : "memory"); };
+  auto dma_w = [&](unsigned so, int i) { asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(wo[i]), "s"(wsrd), "s"(so) : "memory"); };
 
-  // ---- fragments: lane reads stage row (16-row base + r), 16-B chunk 4 kk + g, from per-(kk,
-  // operand) base VGPRs with the fragment offset as immediate
+  // ---- fragments: lane reads row (16-row base + r) of the stage, 16-byte chunk 4 kk + g
   const int rs = swz(r);
-  unsigned bx[2], bw[2];
+  unsigned bx[2][2], bw[2][2];  // [stage][kk], opaque so that the rest of every address stays the instruction's immediate
 #pragma unroll
   for (int kk = 0; kk < 2; ++kk) {
     const unsigned b = lds0 + (((4 * kk + g) ^ rs) << 4) + r * kRowB;
-    bx[kk] = b + wr * WM * kRowB;
-    bw[kk] = b + kOpX + wc * 128 * kRowB;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      bx[p][kk] = b + p * kStage + wr * WM * kRowB;
+      bw[p][kk] = b + p * kStage + kOpX + wc * 128 * kRowB;
+      asm volatile("" : "+v"(bx[p][kk]), "+v"(bw[p][kk]));
+    }
   }
-  short8 fx0[MB], fw0[8], fx1[MB], fw1[8];
-  // read j in the consumption order of the MFMA loop: fw[0], fx[0..MB-1], fw[1..7]
-  auto rd = [](unsigned bxv, unsigned bwv, auto j_t, short8(&fx)[MB], short8(&fw)[8]) {
-    constexpr int j = decltype(j_t)::value;
-    if constexpr (j == 0)
-      asm volatile("ds_read_b128 %0, %1" : "=v"(fw[0]) : "v"(bwv));
-    else if constexpr (j <= MB)
-      asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fx[j - 1]) : "v"(bxv), "i"((j - 1) * 16 * kRowB));
-    else
-      asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fw[j - MB]) : "v"(bwv), "i"((j - MB) * 16 * kRowB));
-  };
+  short8 fx[2][2][MB], fw[4];  // X fragments [stage][kk][m], the ring of W fragments
+  auto lds_rd = [](unsigned a, unsigned off) { return *reinterpret_cast<lds_frag_t>(a + off); };
+  auto rd_x = [&](int p, int j) { fx[p][j / MB][j % MB] = lds_rd(bx[p][j / MB], (j % MB) * 16 * kRowB); };
+  auto rd_w = [&](int p, int f) { fw[f & 3] = lds_rd(bw[p][f & 1], (f >> 1) * 16 * kRowB); };
   floatx4 acc[MB][8];
   using T = std::true_type;
   using F = std::false_type;
 
-  // ---- folded RMSNorm, consumer side: thread tid sums the ss_nt partials of tile row tid.  The
-  // loads are inline asm issued BEFORE the prologue's LDS-DMA, so the prologue's counted wait
-  // retires them and they are summed right after it (hipcc would otherwise wait for them with
-  // a vmcnt(0) in the middle of the K loop, draining the LDS-DMA pipeline)
+  // ---- folded RMSNorm, consumer side: thread tid sums the ss_nt partials of tile row tid.  Requested before everything else and
+  // summed behind the K loop, where the compiler's wait for them drains nothing
   float* scl = reinterpret_cast<float*>(smem + kLdsStages);  // [256] row scales
   float ssp[SC ? SCP : 1];
-  float ssum = 0.f;
-  auto ss_issue = [&](int tm_) {
-    if constexpr (SC) {
-      const u32x4_t s = srd(ea.ss_in, (long)ea.ss_nt * ea.ss_ld * 4);
-      const unsigned base = (unsigned)((tm_ * BM + tid) * 4);
-#pragma unroll
-      for (int p = 0; p < SCP; ++p)  // planes >= ss_nt read past the range: 0
-        asm volatile("buffer_load_dword %0, %1, %2, %3 offen" : "=v"(ssp[p]) : "v"(base), "s"(s), "s"(rfl((unsigned)(p * ea.ss_ld * 4))) : "memory");
-    }
-  };
 
-  // K-tile t: NM MFMAs (kk 0 set: n-major 0..NM/2-1, kk 1 set: the rest) with the reads / DMA /
-  // barriers of the file comment (positions: Tile<BM>).  FIRST: C = 0.  DMA: K-tile t+2 exists
-  // (NEXT: it is K-tile t+2-nk of the next tile of a persistent walk).  NXT: K-tile t+1 exists.
-  auto ktile = [&](auto first_t, auto dma_t, auto nxt_t, auto next_t, int t) {
-    constexpr bool FIRST = decltype(first_t)::value, DMA = decltype(dma_t)::value;
-    constexpr bool NXT = decltype(nxt_t)::value;
-    const unsigned so = (unsigned)((t + par) & 1) * kStage, sn = (unsigned)kStage - so;  // this / next stage
+  // K-tile t in stage P = t & 1; its refills are K-tile t + 2's, at column offset so2 of its operands.  FIRST: C = 0, and in a persistent
+  // walk's later tiles (later) the epilogue's memory operations lie among the requests.
+  auto ktile = [&](auto first_t, auto stage_t, unsigned so2, bool later) {
+    constexpr bool FIRST = decltype(first_t)::value;
+    constexpr int P = decltype(stage_t)::value, S1 = TL::S1, S0 = TL::S0, WA = TL::WA;
+    auto landed = [&]() {  // everything but the newest NP refills
+      if constexpr (FIRST && PERSIST) {
+        if (later) wait_vm<NP + epi_vm_ops<EPI, MB>()>();
+        else wait_vm<NP>();
+      } else {
+        wait_vm<NP>();
+      }
+    };
     unroll<NM>([&](auto i_t) {
-      constexpr int i = decltype(i_t)::value;
-      constexpr int B1 = TL::B1, D0 = TL::D0, DS = TL::DS, LAG = TL::LAG, B2 = TL::B2;
-      if constexpr (i == 0) lgkm0();
-      if constexpr (i < NR) rd(bx[1] + so, bw[1] + so, std::integral_constant<int, i>{}, fx1, fw1);
-      if constexpr (i == B1) {
+      constexpr int i = decltype(i_t)::value, f = i / MB, m = i % MB;
+      constexpr int ph = i < S1 ? 0 : i < S0 ? 1 : 2;                            // phase A, B, A of t + 1
+      constexpr int u = ph == 0 ? i + WA * MB : ph == 1 ? i - S1 : i - S0;       // slot within the phase
+      fence();
+      if constexpr (i == S1 || i == S0) {
+        // S1: W half 2 of t and X of t + 1 have landed, W half 1 of t has been read;
+        // S0: W half 1 of t + 1 has landed, W half 2 of t and X of t + 1 have been read
         lgkm0();
+        landed();
         barrier_raw();
       }
-      if constexpr (DMA && i >= D0 && i < D0 + DS * NP && (i - D0) % DS == 0) {
-        fence();
-        dma(decltype(next_t)::value, t + 2, (i - D0) / DS);
-        fence();
-      }
-      if constexpr (DMA && i >= D0 + LAG && i < D0 + LAG + DS * NP && (i - D0 - LAG) % DS == 0) {
-        constexpr int k = (i - D0 - LAG) / DS;
-        fence();
-        set_m0(k < NP - 1 ? piece_m0(t + 2, k + 1) : piece_m0(t + 3, 0));
-        fence();
-      }
-      if constexpr (NXT && i == B2) {
-        if constexpr (DMA) wait_vm<NP>();
-        else wait_vm<0>();
-        barrier_raw();
-      }
-      if constexpr (NXT && i >= B2 && i < B2 + NR)
-        rd(bx[0] + sn, bw[0] + sn, std::integral_constant<int, i - B2>{}, fx0, fw0);
-      constexpr int kk = i / (NM / 2), n = (i % (NM / 2)) / MB, m = i % MB;
-      if constexpr (kk == 0 && FIRST) mfma0(acc[m][n], fw0[n], fx0[m]);
-      else if constexpr (kk == 0) mfma(acc[m][n], fw0[n], fx0[m]);
-      else mfma(acc[m][n], fw1[n], fx1[m]);
+      if constexpr (m == 0) rd_w(f + WA < 16 ? P : P ^ 1, (f + WA) & 15);
+      if constexpr (ph == 1 && every(u, TL::XR0, TL::XRS, 2 * MB) >= 0) rd_x(P ^ 1, every(u, TL::XR0, TL::XRS, 2 * MB));
+      // the refill of this slot, then M0 for the next slot's
+      constexpr int aw = ph == 2 ? every(u, TL::AW0, TL::AWS, 4) : -1, aw1 = ph == 2 ? every(u + 1, TL::AW0, TL::AWS, 4) : -1;
+      constexpr int ax = ph == 0 ? every(u, TL::AX0, TL::AXS, PX) : -1, ax1 = ph == 0 ? every(u + 1, TL::AX0, TL::AXS, PX) : -1;
+      constexpr int bw_ = ph == 1 ? every(u, TL::BW0, TL::BWS, 4) : -1, bw1 = ph == 1 ? every(u + 1, TL::BW0, TL::BWS, 4) : -1;
+      if constexpr (aw >= 0) dma_w(so2, 4 + aw);
+      if constexpr (ax >= 0) dma_x(so2, ax);
+      if constexpr (bw_ >= 0) dma_w(so2, bw_);
+      if constexpr (aw1 >= 0) m0_w(stage_t, std::integral_constant<int, 4 + aw1>{});
+      if constexpr (ax1 >= 0) m0_x(stage_t, std::integral_constant<int, ax1>{});
+      if constexpr (bw1 >= 0) m0_w(stage_t, std::integral_constant<int, bw1>{});
+      fence();
+      if constexpr (FIRST && (f & 1) == 0) mfma0(acc[m][f >> 1], fw[f & 3], fx[P][f & 1][m]);
+      else mfma(acc[m][f >> 1], fw[f & 3], fx[P][f & 1][m]);
     });
   };
 
-  // ---- one tile per workgroup by default (for long K a persistent walk measured 1-3 % slower: the
-  // hardware already starts the next workgroup on a CU while the finished one's stores drain --
-  // profiles/r5_gemm1w/); PERSIST for short K, where the load ramp is a third of a tile
   int tm, tn;
   coords(tile, tm, tn);
   offsets(tm, tn, xo, wo);
-  ss_issue(tm);
-  // prologue: K-tiles 0 and 1 (the row-scale loads are older: retired with K-tile 0)
+  if constexpr (SC) {
+    const auto ssr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(ea.ss_in), 0, (int)min((long)ea.ss_nt * ea.ss_ld * 4, 0x7FFFFFF0L), 0x00020000);
 #pragma unroll
-  for (int q = 0; q < 2 * NP; ++q) {
-    set_m0(piece_m0(q / NP, q % NP));
-    asm volatile("s_nop 0");
-    dma(false, q / NP, q % NP);
+    for (int p = 0; p < SCP; ++p)  // (planes >= ss_nt lie past the range: 0)
+      ssp[p] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ssr, (unsigned)(tm * BM + tid + p * ea.ss_ld) * 4, 0, 0));
   }
-  set_m0(piece_m0(2, 0));
+  // prologue: what the refills of the two K-tiles before would have brought, in their order: X 0, W 0 half 1, W 0 half 2, X 1, W 1 half 1
+  const unsigned sof = rfl((unsigned)kt0 * kRowB);
+  unroll<2 * PX + 12>([&](auto q_t) {
+    constexpr int q = decltype(q_t)::value, t = q < PX + 8 ? 0 : 1;
+    constexpr bool x = q < PX || (q >= PX + 8 && q < 2 * PX + 8);
+    constexpr int i = q < PX ? q : q < PX + 8 ? q - PX : x ? q - PX - 8 : q - 2 * PX - 8;
+    constexpr std::integral_constant<int, i> i_t{};
+    constexpr std::integral_constant<int, t> t_t{};
+    if constexpr (x) m0_x(t_t, i_t);
+    else m0_w(t_t, i_t);
+    asm volatile("s_nop 0");
+    if constexpr (x) dma_x(sof + t * kRowB, i);
+    else dma_w(sof + t * kRowB, i);
+  });
   wait_vm<NP>();
-  for (;;) {
+  barrier_raw();
+  unroll<4>([&](auto j_t) {
+    m0_w(std::integral_constant<int, 1>{}, std::integral_constant<int, 4 + decltype(j_t)::value>{});
+    asm volatile("s_nop 0");
+    dma_w(sof + kRowB, 4 + decltype(j_t)::value);
+  });
+  for (bool later = false;; later = true) {
     int nxt = 0, tm2 = 0, tn2 = 0;
     bool has_next = false;
     if constexpr (PERSIST) {
-      // opaque per tile: keeps hipcc from hoisting the unrolled K-tiles' per-piece / per-fragment
-      // addresses out of the tile loop into hundreds of live registers (it spills them otherwise)
-      asm volatile("" : "+v"(bx[0]), "+v"(bx[1]), "+v"(bw[0]), "+v"(bw[1]));
-#pragma unroll
-      for (int i = 0; i < PX; ++i) asm volatile("" : "+v"(xo[i]));
-#pragma unroll
-      for (int i = 0; i < 8; ++i) asm volatile("" : "+v"(wo[i]));
       nxt = tile + (int)gridDim.x;
       has_next = nxt < nwg;
-      // the last tile of the walk DMAs its own first K-tiles again (harmless, never read): one
-      // straight-line tail instead of two
+      // the last tile of the walk requests its own first K-tiles again (never read)
       coords(has_next ? nxt : tile, tm2, tn2);
-      offsets(tm2, tn2, xo2, wo2);
     }
-    barrier_raw();
-    if constexpr (SC) {
+    fence();
 #pragma unroll
-      for (int p = 0; p < SCP; ++p) ssum += ssp[p];
-    }
-    {
-      const unsigned s0 = (unsigned)(par & 1) * kStage;
-      unroll<NR>([&](auto j_t) { rd(bx[0] + s0, bw[0] + s0, j_t, fx0, fw0); });
-    }
-    ktile(T{}, T{}, T{}, F{}, 0);
-    int t = 1;
-    for (; t + 2 < nk; ++t) ktile(F{}, T{}, T{}, F{}, t);
-    if constexpr (PERSIST) {  // the next tile's K-tiles 0 and 1 into the stages these two free
-      ktile(F{}, T{}, T{}, T{}, t);
-      ktile(F{}, T{}, F{}, T{}, t + 1);
-    } else {
-      ktile(F{}, F{}, T{}, F{}, t);
-      ktile(F{}, F{}, F{}, F{}, t + 1);
+    for (int j = 0; j < 2 * MB; ++j) rd_x(0, j);
+#pragma unroll
+    for (int f = 0; f < TL::WA; ++f) rd_w(0, f);
+    lgkm0();
+    barrier_raw();  // X's stage 0 is free
+    unsigned so2 = sof + 2 * kRowB;
+    // before K-tile t: the refills of the last two K-tiles are the next tile's first ones, or zeros that nobody reads (a descriptor
+    // without range), so that every K-tile is the same code
+    auto refills = [&](int t) {
+      if (t + 2 == nk) {
+        if constexpr (PERSIST) {
+          offsets(tm2, tn2, xo, wo);
+          so2 = sof;
+        } else {
+          xsrd.z = wsrd.z = 0;
+        }
+      }
+    };
+    constexpr std::integral_constant<int, 0> even{};
+    constexpr std::integral_constant<int, 1> odd{};
+    ktile(T{}, even, so2, later);
+    for (int t = 1;; t += 2) {
+      so2 += kRowB;
+      refills(t);
+      ktile(F{}, odd, so2, false);
+      if (t + 1 >= nk) break;
+      so2 += kRowB;
+      refills(t + 1);
+      ktile(F{}, even, so2, false);
+      if (t + 2 >= nk) break;
     }
     // the asm MFMAs are invisible to hipcc's hazard recognizer: wait out MFMA -> accumulator read,
     // and pin every accumulator behind that wait (hipcc otherwise schedules some v_accvgpr_read of
@@ -376,6 +378,8 @@ __global__ __launch_bounds__(256, 1) void gemm1w_kernel(const bf16_t* __restrict
 #pragma unroll
       for (int n = 0; n < 8; ++n) asm volatile("" : "+a"(acc[m][n]));
 
+    if constexpr (!PERSIST) wait_vm<0>();  // the last refills land before the workgroup's LDS is released
+
     // ================= epilogue of tile (tm, tn)
     // lane holds row tm*256 + wr*128 + 16m + r; fragment pair (2p, 2p+1) the 8 consecutive
     // columns 32p + 8g .. +7 of the wave's 128 (SwiGLU: gate pairs 0, 1 and up pairs 2, 3 of
@@ -384,6 +388,9 @@ __global__ __launch_bounds__(256, 1) void gemm1w_kernel(const bf16_t* __restrict
 #pragma unroll
     for (int m = 0; m < MB; ++m) scm[m] = 1.f;
     if constexpr (SC) {
+      float ssum = 0.f;
+#pragma unroll
+      for (int p = 0; p < SCP; ++p) ssum += ssp[p];
       scl[tid] = rsqrtf(ssum * ea.inv_h + ea.eps);
       lgkm0();
       barrier_raw();
@@ -605,14 +612,6 @@ __global__ __launch_bounds__(256, 1) void gemm1w_kernel(const bf16_t* __restrict
       tile = nxt;
       tm = tm2;
       tn = tn2;
-#pragma unroll
-      for (int i = 0; i < PX; ++i) xo[i] = xo2[i];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) wo[i] = wo2[i];
-      par ^= nk & 1;
-      // the next tile's K-tile 0 has landed: younger than it are K-tile 1's NP pieces and the
-      // epilogue's bias loads and stores (the counter retires in issue order)
-      wait_vm<NP + epi_vm_ops<EPI, MB>()>();
     }
   }
 }
@@ -705,7 +704,7 @@ void launch1w(const bf16_t* x, long ldx, const bf16_t* w, const bf16_t* bias, in
               long ldo, int TN, int tn0, int ks, int group_m, hipStream_t st, const LkEpi& ea) {
   if constexpr (persistable(EPI) && SCP == 0 && BM == 256) {
     const int tiles = ((M + BM - 1) / BM) * TN;
-    if (ks == 1 && K / kBK <= persist_kt() && tiles > 2 * cu_count()) {
+    if (ks == 1 && K / kBK <= persist_kt() && K / kBK % 2 == 0 && tiles > 2 * cu_count()) {
       launch1w_p<EPI, SCP, BM, true>(x, ldx, w, bias, M, K, I, out, ldo, TN, tn0, ks, group_m, st, ea);
       return;
     }

@@ -147,7 +147,7 @@ int lk_gemm_grouped(const bf16_t* x, long ldx, const bf16_t* w, const int* seg, 
                     bf16_t* out, long ldo, hipStream_t st, const int* gather = nullptr, long x_rows = 0, const int* scatter = nullptr,
                     int top = 1);
 
-// gemm1w.hip: the one-wave-per-SIMD bm x 256 prefill GEMM (hipBLASLt's gfx950 K-loop schedule,
+// gemm1w.hip: the one-wave-per-SIMD bm x 256 prefill GEMM (X resident in registers, W streamed;
 // every lk_gemm epilogue); lk_gemm routes variants 3 / 4 / 5 here (row tile bm = 256 / 192 / 128).
 // Needs K % 64 == 0 and >= 3 K-tiles per split, N % 256 == 0 (SwiGLU: N/2 % 128).
 // group_m <= 0: LK_GEMM_GROUP_M (4).

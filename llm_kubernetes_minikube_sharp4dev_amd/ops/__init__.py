@@ -567,13 +567,9 @@ def _gemm_key(M: int, N: int, K: int, epi: int):
     return ((M + 255) // 256, N, K, epi)
 
 
-# Variants 3 / 4 / 5 = csrc/gemm1w.hip, the one-wave-per-SIMD kernel on hipBLASLt's gfx950 K-loop
-# schedule, 256-wide column tiles and 256 / 192 / 128-row tiles: 1.04-1.09x gemm.hip and
-# 0.95-1.10x hipBLASLt on the Llama-3-8B projections at 256 rows (profiles/r5_gemm1w/).  The
-# smaller row tiles fill the 256 CUs where 256-row tiles leave most of a wave idle: at the
-# serving bench's mixed-step sizes (prefill chunk + ~105 decode rows) they are 1.2-1.4x the
-# round-4 dispatch (M 2664: QKV on 128-row tiles 109.5 vs 151.6 us, O / down on 192-row tiles
-# 66.7 / 220.8 vs 82.3 / 295.5 us; benchmarks/gemm_tiles.py, profiles/r5_gemm_tiles/).
+# Variants 3 / 4 / 5 = csrc/gemm1w.hip, the one-wave-per-SIMD kernel with 256-wide column tiles and
+# 256 / 192 / 128-row tiles.  The smaller row tiles fill the 256 CUs where 256-row tiles leave most of a
+# wave idle (M 2664: QKV on 128-row tiles 107 us, O on 192-row tiles 69 us; profiles/gemm1w_slots.md).
 # Which tile wins depends on M through the wave quantisation AND the chip's clocks (a partly
 # filled wave runs at a higher clock), so the choice is MEASURED: ``tune_gemm`` times every
 # candidate per 256-row M bucket, and a table of those measurements for the shipped models
