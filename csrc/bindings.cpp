@@ -2061,15 +2061,17 @@ at::Tensor mlstm_scan(const at::Tensor& q, const at::Tensor& k, const at::Tensor
   return o;
 }
 
-void head_linear(const at::Tensor& x, const at::Tensor& w, int64_t x_head, at::Tensor& out) {
+// parts 2: x holds K columns per head and K more that add to them, both times the same w (bf16)
+void head_linear(const at::Tensor& x, const at::Tensor& w, int64_t x_head, at::Tensor& out, int64_t parts) {
   CHECK_CUDA(x); CHECK_LASTDIM(x); CHECK_CUDA(w); CHECK_CONTIG(w); CHECK_CUDA(out); CHECK_LASTDIM(out);
   same_type(w, x, "w"); same_type(out, x, "out");
   TORCH_CHECK(w.dim() == 3 && x.dim() == 2 && out.dim() == 3, "x [T, *], w [H, N, K], out [T, H, >= N]");
   const long H = w.size(0), N = w.size(1), K = w.size(2);
-  TORCH_CHECK(x_head >= 0 && x.size(1) >= (H - 1) * x_head + K, "x has too few columns");
+  TORCH_CHECK(x_head >= 0 && x.size(1) >= (H - 1) * x_head + parts * K, "x has too few columns");
+  TORCH_CHECK(parts == 1 || (parts == 2 && x.scalar_type() == at::kBFloat16), "parts: 1, or 2 for bf16");
   TORCH_CHECK(out.size(0) == x.size(0) && out.size(1) == H && out.size(2) >= N, "out must be [T, H, >= N]");
   CHECK_RC(lk_head_linear(x.data_ptr(), x.stride(0), x_head, w.data_ptr(), (int)H, (int)N, (int)K, x.size(0), out.data_ptr(), out.stride(0),
-                          out.stride(1), esz_of(x, "x"), cur_stream()), "head_linear");
+                          out.stride(1), esz_of(x, "x"), cur_stream(), (int)parts), "head_linear");
 }
 
 struct LatShapes { int H, KD, RP, BS, esz; const float* sink; };
@@ -2079,8 +2081,9 @@ LatShapes lat_check(const at::Tensor& qa, const at::Tensor& cache, const at::Ten
   CHECK_CUDA(ctx); CHECK_I32(ctx); CHECK_CONTIG(ctx);
   same_type(cache, qa, "cache"); same_type(out, qa, "out");
   TORCH_CHECK(qa.dim() == 3 && cache.dim() == 3 && out.dim() == 3 && cache.size(2) == qa.size(2), "qa [T, H, KD], cache [blocks, BS, KD]");
-  TORCH_CHECK(qa.stride(2) == 1 && qa.stride(1) == qa.size(2) && out.stride(2) == 1 && out.stride(1) == rp, "heads must be adjacent");
-  TORCH_CHECK(out.size(0) == qa.size(0) && out.size(1) == qa.size(1) && out.size(2) == rp && rp < qa.size(2), "out must be [T, H, rp]");
+  TORCH_CHECK(qa.stride(2) == 1 && qa.stride(1) == qa.size(2) && out.stride(2) == 1 && out.stride(1) == out.size(2), "heads must be adjacent");
+  TORCH_CHECK(out.size(0) == qa.size(0) && out.size(1) == qa.size(1) && (out.size(2) == rp || (out.size(2) == 2 * rp && out.scalar_type() == at::kBFloat16)) &&
+                  rp < qa.size(2), "out must be [T, H, rp], or [T, H, 2 rp] for two bf16 parts");
   TORCH_CHECK(bt.dim() == 2 && bt.size(0) == ctx.numel(), "block tables: one row per sequence");
   return {(int)qa.size(1), (int)qa.size(2), (int)rp, (int)cache.size(1), esz_of(qa, "qa"), fpo(sink, qa.size(1), "sink")};
 }
@@ -2101,7 +2104,7 @@ void latent_attn_prefill(const at::Tensor& qa, const at::Tensor& cache, const at
   TORCH_CHECK(cu_q.numel() == ctx.numel() + 1, "cu_q");
   CHECK_RC(lk_latent_attn_prefill(qa.data_ptr(), qa.stride(0), cache.data_ptr(), ip(bt), (int)bt.stride(0), ip(cu_q), ip(ctx), (int)ctx.numel(),
                                   qa.size(0), s.BS, s.H, s.KD, s.RP, (int)window, (float)scale, s.sink, gate ? gate->data_ptr() : nullptr,
-                                  gate ? gate->stride(0) : 0, out.data_ptr(), out.stride(0), s.esz,
+                                  gate ? gate->stride(0) : 0, out.data_ptr(), out.stride(0), (int)out.size(2), s.esz,
                                   cur_stream()), "latent_attn_prefill");
 }
 
@@ -2114,7 +2117,7 @@ void latent_attn_decode(const at::Tensor& qa, const at::Tensor& cache, const at:
   if (splits > 1) part = at::empty({qa.size(0) * s.H * splits * (rp + 2)}, qa.options().dtype(at::kFloat));
   CHECK_RC(lk_latent_attn_decode(qa.data_ptr(), qa.stride(0), cache.data_ptr(), ip(bt), (int)bt.stride(0), ip(ctx), (int)qa.size(0), (int)splits, s.BS,
                                  s.H, s.KD, s.RP, (int)window, (float)scale, s.sink, gate ? gate->data_ptr() : nullptr,
-                                 gate ? gate->stride(0) : 0, out.data_ptr(), out.stride(0),
+                                 gate ? gate->stride(0) : 0, out.data_ptr(), out.stride(0), (int)out.size(2),
                                  splits > 1 ? part.data_ptr<float>() : nullptr, s.esz, cur_stream()), "latent_attn_decode");
 }
 
@@ -2212,7 +2215,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("diff_attention_decode", &diff_attention_decode);
   m.def("tile_attention_prefill", &tile_attention_prefill);
   m.def("head_delta", &head_delta);
-  m.def("head_linear", &head_linear);
+  m.def("head_linear", &head_linear, py::arg("x"), py::arg("w"), py::arg("x_head"), py::arg("out"), py::arg("parts") = 1);
   m.def("latent_attn_prefill", &latent_attn_prefill);
   m.def("latent_attn_decode", &latent_attn_decode);
   m.def("latent_prep", &latent_prep);

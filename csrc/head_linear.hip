@@ -99,7 +99,8 @@ __global__ __launch_bounds__(256) void latent_rot_kernel(const T* __restrict__ x
   }
 }
 
-template <typename T>
+// PARTS 2: x holds K columns and K more that add to them (an operand in two bf16 parts), both times the same w; K in whole steps.
+template <typename T, int PARTS>
 __global__ __launch_bounds__(256) void head_linear_lds_kernel(const T* __restrict__ x, long xs, long xh, const T* __restrict__ w, int N, int K,
                                                               long rows, T* __restrict__ out, long os, long oh, int vst) {
   constexpr int EV = El<T>::V, KS = 8 * EV, TM = 128, TN = 128;
@@ -118,16 +119,16 @@ __global__ __launch_bounds__(256) void head_linear_lds_kernel(const T* __restric
   }
   uint4_t rx[4], rw[4];
   auto fetch = [&](int kb) {
-    const int k = kb + ps * EV;
-    const bool in = k < K;
+    const int k = kb + ps * EV, kw = PARTS == 2 && kb >= K ? k - K : k;
+    const bool in = k < PARTS * K;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       rx[i] = ld16(xp[i] + (in ? k : 0));
-      rw[i] = ld16(wp[i] + (in ? k : 0));
+      rw[i] = ld16(wp[i] + (in ? kw : 0));
     }
   };
   auto stage = [&](int buf, int kb) {
-    const bool in = kb + ps * EV < K;
+    const bool in = kb + ps * EV < PARTS * K;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       sx[buf][pr + 32 * i][ps] = in ? rx[i] : uint4_t{0u, 0u, 0u, 0u};
@@ -144,8 +145,8 @@ __global__ __launch_bounds__(256) void head_linear_lds_kernel(const T* __restric
   stage(0, 0);
   __syncthreads();
   int cur = 0;
-  for (int kb = 0; kb < K; kb += KS) {
-    const bool more = kb + KS < K;
+  for (int kb = 0; kb < PARTS * K; kb += KS) {
+    const bool more = kb + KS < PARTS * K;
     if (more) fetch(kb + KS);
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
@@ -177,11 +178,12 @@ __global__ __launch_bounds__(256) void head_linear_lds_kernel(const T* __restric
 // a microsecond of bandwidth, so what counts is the chain of waits per wave: one for K 128, one for K 512 (bf16).  A wave over the whole
 // contraction of 64 columns waited 8 times at K 512 and left 3 of 4 waves idle below 17 rows: 8.8 -> 5.5 us on average over
 // K 128 -> 512 and K 512 -> 128 columns, 16 heads, the rotated part included.
-template <typename T, int RT>
+template <typename T, int RT, int PARTS>
 __global__ __launch_bounds__(256) void head_linear_few_kernel(const T* __restrict__ x, long xs, long xh, const T* __restrict__ w, int N, int K,
                                                               long rows, T* __restrict__ out, long os, long oh, int vec, int vst, int ncol,
                                                               RotTail rot) {
   constexpr int EV = El<T>::V, STEP = 4 * EV, NT = 2, U = 4;
+  static_assert(PARTS == 1 || sizeof(T) == 2, "f32 operands are whole");
   __shared__ floatx4 part[4][RT * NT][64];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, n16 = lane & 15, g = lane >> 4;
   const int h = blockIdx.x, c0 = blockIdx.y * 16 * NT;
@@ -205,21 +207,25 @@ __global__ __launch_bounds__(256) void head_linear_few_kernel(const T* __restric
   const int whole = vec ? K / STEP : 0, steps = (K + STEP - 1) / STEP;
   int s = wv;
   for (; s + 4 * (U - 1) < whole; s += 4 * U) {
-    uint4_t a[U][NT], b[U][RT];
+    uint4_t a[U][NT], b[U][PARTS][RT];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int k = (s + 4 * u) * STEP + g * EV;
 #pragma unroll
       for (int c = 0; c < NT; ++c) a[u][c] = ld16(wr[c] + k);
 #pragma unroll
-      for (int r = 0; r < RT; ++r) b[u][r] = ld16(xr[r] + k);
+      for (int q = 0; q < PARTS; ++q)
+#pragma unroll
+        for (int r = 0; r < RT; ++r) b[u][q][r] = ld16(xr[r] + q * K + k);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int r = 0; r < RT; ++r)
+      for (int q = 0; q < PARTS; ++q)
 #pragma unroll
-        for (int c = 0; c < NT; ++c) acc[r][c] = mma_qk<T>(a[u][c], b[u][r], acc[r][c]);
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+          for (int c = 0; c < NT; ++c) acc[r][c] = mma_qk<T>(a[u][c], b[u][q][r], acc[r][c]);
   }
   for (; s < steps; s += 4) {
     const int k = s * STEP + g * EV;
@@ -227,11 +233,14 @@ __global__ __launch_bounds__(256) void head_linear_few_kernel(const T* __restric
 #pragma unroll
     for (int c = 0; c < NT; ++c) a[c] = frag<T>(wr[c], k, K, vec);
 #pragma unroll
-    for (int r = 0; r < RT; ++r) b[r] = frag<T>(xr[r], k, K, vec);
+    for (int q = 0; q < PARTS; ++q) {
 #pragma unroll
-    for (int r = 0; r < RT; ++r)
+      for (int r = 0; r < RT; ++r) b[r] = frag<T>(xr[r] + q * K, k, K, vec);
 #pragma unroll
-      for (int c = 0; c < NT; ++c) acc[r][c] = mma_qk<T>(a[c], b[r], acc[r][c]);
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int c = 0; c < NT; ++c) acc[r][c] = mma_qk<T>(a[c], b[r], acc[r][c]);
+    }
   }
 #pragma unroll
   for (int r = 0; r < RT; ++r)
@@ -252,19 +261,19 @@ __global__ __launch_bounds__(256) void head_linear_few_kernel(const T* __restric
   }
 }
 
-template <typename T>
+template <typename T, int PARTS>
 int head_linear_t(const void* x, long xs, long xh, const void* w, int H, int N, int K, long rows, void* out, long os, long oh, int vec, int vst,
                   const RotTail& rot, hipStream_t st) {
   if (N > 0 && rows > 65535L * 64) return -1;
   const bool fused = rot.RDP > 0 && N > 0 && rows <= 128;
   const int tail = fused ? 1 : 0;   // workgroups of 16 rows each behind the columns'
 #define LK_HEAD(RT)                                                                                                                          \
-  head_linear_few_kernel<T, RT><<<dim3((unsigned)H, (unsigned)((N + 31) / 32 + tail * RT), (unsigned)((rows + 16 * RT - 1) / (16 * RT))),    \
+  head_linear_few_kernel<T, RT, PARTS><<<dim3((unsigned)H, (unsigned)((N + 31) / 32 + tail * RT), (unsigned)((rows + 16 * RT - 1) / (16 * RT))),    \
                                   256, 0, st>>>((const T*)x, xs, xh, (const T*)w, N, K, rows, (T*)out, os, oh, vec, vst, (N + 31) / 32, rot)
   if (N == 0)
     ;
-  else if (rows > 128 && vec)
-    head_linear_lds_kernel<T><<<dim3((unsigned)H, (unsigned)((N + 127) / 128), (unsigned)((rows + 127) / 128)), 256, 0, st>>>(
+  else if (rows > 128 && vec && (PARTS == 1 || K % 64 == 0))
+    head_linear_lds_kernel<T, PARTS><<<dim3((unsigned)H, (unsigned)((N + 127) / 128), (unsigned)((rows + 127) / 128)), 256, 0, st>>>(
         (const T*)x, xs, xh, (const T*)w, N, K, rows, (T*)out, os, oh, vst);
   else if (rows <= 16)
     LK_HEAD(1);
@@ -281,17 +290,9 @@ int head_linear_t(const void* x, long xs, long xh, const void* w, int H, int N, 
   return 0;
 }
 
-}  // namespace
-
-int lk_head_linear(const void* x, long xs, long xh, const void* w, int H, int N, int K, long rows, void* out, long os, long oh, int esz,
-                   hipStream_t st) {
-  if (N < 1 || K < 1) return rows <= 0 ? 0 : -1;
-  return lk_latent_query(x, xs, xh, w, H, N, K, rows, out, os, oh, 0, 0, 0, nullptr, nullptr, 0, 0, 0, 1.f, esz, st);
-}
-
 // N 0: the rotated part alone
-int lk_latent_query(const void* x, long xs, long xh, const void* w, int H, int N, int K, long rows, void* out, long os, long oh, int qdim, int dim,
-                    int rd, const float* freq, const int* positions, int rp, int RDP, int adj, float mag, int esz, hipStream_t st) {
+int head_products(const void* x, long xs, long xh, const void* w, int H, int N, int K, long rows, void* out, long os, long oh, int qdim, int dim,
+                  int rd, const float* freq, const int* positions, int rp, int RDP, int adj, float mag, int esz, hipStream_t st, int parts) {
   if (rows <= 0) return 0;
   if (H < 1 || H > 65535 || N < 0 || (N > 0 && K < 1) || (N + 31) / 32 > 65000) return -1;
   if (rd < 0 || rd % 2 || rd > kRotMax || dim < 0 || dim + rd > qdim || rd > RDP || N > (RDP > 0 ? rp : N) || (rd > 0 && (!freq || !positions))) return -1;
@@ -300,6 +301,20 @@ int lk_latent_query(const void* x, long xs, long xh, const void* w, int H, int N
   const int vec = K % ev == 0 && xs % ev == 0 && xh % ev == 0 && a16(x, 16) && a16(w, 16);
   const int vst = os % 4 == 0 && oh % 4 == 0 && a16(out, 4 * esz);
   const RotTail rot{dim, rd, rp, RDP, adj, mag, freq, positions};
-  return esz == 2 ? head_linear_t<bf16_t>(x, xs, xh, w, H, N, K, rows, out, os, oh, vec, vst, rot, st)
-                  : head_linear_t<float>(x, xs, xh, w, H, N, K, rows, out, os, oh, vec, vst, rot, st);
+  if (esz != 2) return head_linear_t<float, 1>(x, xs, xh, w, H, N, K, rows, out, os, oh, vec, vst, rot, st);
+  return parts == 2 ? head_linear_t<bf16_t, 2>(x, xs, xh, w, H, N, K, rows, out, os, oh, vec, vst, rot, st)
+                    : head_linear_t<bf16_t, 1>(x, xs, xh, w, H, N, K, rows, out, os, oh, vec, vst, rot, st);
+}
+
+}  // namespace
+
+int lk_head_linear(const void* x, long xs, long xh, const void* w, int H, int N, int K, long rows, void* out, long os, long oh, int esz,
+                   hipStream_t st, int parts) {
+  if (N < 1 || K < 1 || parts < 1 || parts > 2 || (parts == 2 && esz != 2)) return rows <= 0 ? 0 : -1;
+  return head_products(x, xs, xh, w, H, N, K, rows, out, os, oh, 0, 0, 0, nullptr, nullptr, 0, 0, 0, 1.f, esz, st, parts);
+}
+
+int lk_latent_query(const void* x, long xs, long xh, const void* w, int H, int N, int K, long rows, void* out, long os, long oh, int qdim, int dim,
+                    int rd, const float* freq, const int* positions, int rp, int RDP, int adj, float mag, int esz, hipStream_t st) {
+  return head_products(x, xs, xh, w, H, N, K, rows, out, os, oh, qdim, dim, rd, freq, positions, rp, RDP, adj, mag, esz, st, 1);
 }

@@ -391,9 +391,9 @@ int lk_mlstm_scan(const void* q, long qs, const void* k, long ks, const void* v,
                   long os, int max_len, float* pre, hipStream_t st);
 int lk_mlstm_chunk_min();
 
-// csrc/head_linear.hip: out[t, h, :N] = w[h] x[t, h xh : h xh + K]
+// csrc/head_linear.hip: out[t, h, :N] = w[h] x[t, h xh : h xh + K], with parts 2 plus w[h] x[t, h xh + K : h xh + 2 K]
 int lk_head_linear(const void* x, long xs, long xh, const void* w, int H, int N, int K, long rows, void* out, long os, long oh, int esz,
-                   hipStream_t st);
+                   hipStream_t st, int parts = 1);
 // the same, and behind column rp of every output row RDP columns: x's rd elements behind a head's first dim, rotated, then zeros
 // (N 0: only those)
 int lk_latent_query(const void* x, long xs, long xh, const void* w, int H, int N, int K, long rows, void* out, long os, long oh, int qdim, int dim,
@@ -403,10 +403,10 @@ int lk_latent_query(const void* x, long xs, long xh, const void* w, int H, int N
 // the preparation of its operands
 int lk_latent_attn_prefill(const void* q, long qs, const void* cache, const int* bt, int bt_stride, const int* cu_q, const int* ctx_lens, int nseq,
                            long rows, int BS, int H, int KD, int RP, int window, float scale, const float* sink, const void* gate, long gs,
-                           void* out, long os, int esz, hipStream_t st);
+                           void* out, long os, int OH, int esz, hipStream_t st);
 int lk_latent_attn_decode(const void* q, long qs, const void* cache, const int* bt, int bt_stride, const int* ctx_lens, int B, int Z, int BS, int H,
                           int KD, int RP, int window, float scale, const float* sink, const void* gate, long gs, void* out, long os,
-                          float* part, int esz, hipStream_t st);
+                          int OH, float* part, int esz, hipStream_t st);
 int lk_latent_prep(const void* u, long us, int dq, int qr, const float* wq, int dkv, int R, const float* wkv, int rd, const float* freq,
                    const int* positions, float eps, void* cache, const int* slots, int RP, int KD, void* cq, long cqs, long rows, int adj, float mag,
                    int esz, hipStream_t st);

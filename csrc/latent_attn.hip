@@ -45,8 +45,9 @@ struct LatParams {
   int window;          // 0: causal
   float scale;
   const float* sink;   // [H] or null
-  void* out;           // [rows, H, RP]
+  void* out;           // [rows, H, OH]: the averages, or with OH = 2 RP their bf16 value and, RP columns on, the bf16 of the rest
   long os;
+  int OH;
   const void* gate;    // rows aligned with q's: the averages of head h times sigmoid(column h); null: none
   long gs;
 };
@@ -56,6 +57,19 @@ LK_DEVICE float lat_gate(const LatParams& p, long row, int head) {
   if (!p.gate) return 1.f;
   const float g = El<T>::ld(reinterpret_cast<const T*>(p.gate) + row * p.gs + head);
   return sizeof(T) == 4 ? 1.f / (1.f + expf(-g)) : __builtin_amdgcn_rcpf(1.f + __expf(-g));
+}
+
+// four averages of a row whose parts start at o: one rounding to bf16, or two parts that keep 16 bits
+LK_DEVICE void store_avg(const LatParams& p, bf16_t* o, const float (&v)[4]) {
+  short4_t hi, lo;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const bf16_t h = f2bf(v[j]);
+    hi[j] = (short)h;
+    lo[j] = (short)f2bf(v[j] - bf2f(h));
+  }
+  *reinterpret_cast<short4_t*>(o) = hi;
+  if (p.OH > p.RP) *reinterpret_cast<short4_t*>(o + p.RP) = lo;
 }
 
 LK_DEVICE int first_key(int qpos, int window) { return window > 0 ? max(0, qpos - window + 1) : 0; }
@@ -321,14 +335,9 @@ __global__ __launch_bounds__(pre_waves<RP>() * 64, RP >= 256 ? 1 : 2) void lat_p
     if (qpos[x] >= 0) {
       if (p.sink) l[x] += __builtin_amdgcn_exp2f(p.sink[head] * kLog2e - m[x]);   // one more term without a value
       const float f = l[x] > 0.f ? lat_gate<bf16_t>(p, qbeg + qi, head) / l[x] : 0.f;
-      bf16_t* orow = reinterpret_cast<bf16_t*>(p.out) + (long)(qbeg + qi) * p.os + (long)head * RP + 4 * g;
+      bf16_t* orow = reinterpret_cast<bf16_t*>(p.out) + (long)(qbeg + qi) * p.os + (long)head * p.OH + 4 * g;
 #pragma unroll
-      for (int vt = 0; vt < VT; ++vt) {
-        short4_t v;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = (short)f2bf(o[x][vt][j] * f);
-        *reinterpret_cast<short4_t*>(orow + 16 * vt) = v;
-      }
+      for (int vt = 0; vt < VT; ++vt) store_avg(p, orow + 16 * vt, {o[x][vt][0] * f, o[x][vt][1] * f, o[x][vt][2] * f, o[x][vt][3] * f});
     }
   }
 }
@@ -414,10 +423,8 @@ __global__ __launch_bounds__(256) void lat_decode_kernel(LatParams p, const int*
     }
     if (n16 < p.HC && head < p.H) {
       if (Z == 1) {
-        short4_t v;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = (short)f2bf(s[j] * inv);
-        *reinterpret_cast<short4_t*>(reinterpret_cast<bf16_t*>(p.out) + (long)b * p.os + (long)head * RP + 16 * vt + 4 * g) = v;
+        store_avg(p, reinterpret_cast<bf16_t*>(p.out) + (long)b * p.os + (long)head * p.OH + 16 * vt + 4 * g,
+                  {s[0] * inv, s[1] * inv, s[2] * inv, s[3] * inv});
       } else {
         float* pp = part + (((long)b * p.H + head) * Z + z) * (RP + 2) + 16 * vt + 4 * g;
 #pragma unroll
@@ -432,9 +439,9 @@ __global__ __launch_bounds__(256) void lat_decode_kernel(LatParams p, const int*
   }
 }
 
-// One workgroup per (sequence, head), two columns per thread.  A chain of three waits (maxima, sums, averages): the splits' maxima and
+// One workgroup per (sequence, head), four columns per thread.  A chain of three waits (maxima, sums, averages): the splits' maxima and
 // sums are read by the lanes side by side and the averages four splits at a time; one split after the other it took 6.5 us at 64 x 16
-// rows of 512 columns in 4 splits, 4.7 now.
+// rows of 512 columns in 4 splits, 4.7 side by side.
 __global__ __launch_bounds__(256) void lat_reduce_kernel(LatParams p, const float* __restrict__ part, int Z) {
   const int b = blockIdx.x, head = blockIdx.y, RP = p.RP, lane = threadIdx.x & 63;
   const float* pp = part + ((long)b * p.H + head) * Z * (RP + 2);
@@ -445,17 +452,19 @@ __global__ __launch_bounds__(256) void lat_reduce_kernel(LatParams p, const floa
   for (int z = lane; z < Z; z += 64) L += pp[(long)z * (RP + 2) + RP + 1] * __builtin_amdgcn_exp2f(pp[(long)z * (RP + 2) + RP] - M);
   L = wave_sum(L);
   const float inv = L > 0.f ? gate / L : 0.f;
-  for (int d = 2 * threadIdx.x; d < RP; d += 512) {
-    float s0 = 0.f, s1 = 0.f;
+  for (int d = 4 * threadIdx.x; d < RP; d += 1024) {
+    float s[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
     for (int z = 0; z < Z; ++z) {
-      const float* q = pp + (long)z * (RP + 2);
-      const float2 v = *reinterpret_cast<const float2*>(q + d);
+      const float* q = pp + (long)z * (RP + 2);   // (a row is RP + 2 long: 8-byte loads)
+      const float2 v = *reinterpret_cast<const float2*>(q + d), w = *reinterpret_cast<const float2*>(q + d + 2);
       const float e = __builtin_amdgcn_exp2f(q[RP] - M);
-      s0 += v.x * e;
-      s1 += v.y * e;
+      s[0] += v.x * e;
+      s[1] += v.y * e;
+      s[2] += w.x * e;
+      s[3] += w.y * e;
     }
-    *reinterpret_cast<unsigned*>(reinterpret_cast<bf16_t*>(p.out) + (long)b * p.os + (long)head * RP + d) = pack_bf2(s0 * inv, s1 * inv);
+    store_avg(p, reinterpret_cast<bf16_t*>(p.out) + (long)b * p.os + (long)head * p.OH + d, {s[0] * inv, s[1] * inv, s[2] * inv, s[3] * inv});
   }
 }
 
@@ -479,9 +488,9 @@ __global__ __launch_bounds__(256) void lat_plain_kernel(LatParams p, const int* 
   } else {
     qpos = ctx_lens[b] - 1;
   }
-  T* orow = reinterpret_cast<T*>(p.out) + (long)row * p.os + (long)head * p.RP;
+  T* orow = reinterpret_cast<T*>(p.out) + (long)row * p.os + (long)head * p.OH;
   if (qpos < 0) {
-    for (int d = tid; d < p.RP; d += 256) El<T>::st(orow + d, 0.f);
+    for (int d = tid; d < p.OH; d += 256) El<T>::st(orow + d, 0.f);
     return;
   }
   const T* qrow = reinterpret_cast<const T*>(p.q) + (long)row * p.qs + (long)head * p.KD;
@@ -531,7 +540,11 @@ __global__ __launch_bounds__(256) void lat_plain_kernel(LatParams p, const int* 
 #pragma unroll
   for (int i = 0; i < kPlainDims; ++i) {
     const int d = tid + 256 * i;
-    if (d < p.RP) El<T>::st(orow + d, acc[i] * inv);
+    if (d < p.RP) {
+      const float v = acc[i] * inv;
+      El<T>::st(orow + d, v);
+      if (p.OH > p.RP) El<T>::st(orow + p.RP + d, v - El<T>::ld(orow + d));   // (this thread's own store)
+    }
   }
 }
 
@@ -657,14 +670,14 @@ int run_plain(const LatParams& p, const int* cu_q, const int* ctx, int nseq, lon
 }
 
 bool make_params(LatParams& p, const void* q, long qs, const void* cache, const int* bt, int bt_stride, int BS, int H, int KD, int RP, int window,
-                 float scale, const float* sink, const void* gate, long gs, void* out, long os, int esz) {
-  p.gate = gate; p.gs = gs;
+                 float scale, const float* sink, const void* gate, long gs, void* out, long os, int OH, int esz) {
+  p.gate = gate; p.gs = gs; p.OH = OH;
   p.q = q; p.qs = qs; p.cache = cache; p.bt = bt; p.bt_stride = bt_stride; p.BS = BS; p.H = H; p.KD = KD; p.RP = RP; p.window = window;
   p.scale = scale; p.sink = sink; p.out = out; p.os = os;
   const int blocks = (H + 15) / 16;
   p.HC = blocks > 0 ? (H + blocks - 1) / blocks : 1;
   const auto a16 = [](const void* x) { return reinterpret_cast<uintptr_t>(x) % 16 == 0; };
-  return H >= 1 && H <= 65535 && BS >= 16 && BS % 16 == 0 && RP >= 16 && KD > RP && KD % 64 == 0 && RP % 64 == 0 && window >= 0 && a16(q) &&
+  return H >= 1 && H <= 65535 && BS >= 16 && BS % 16 == 0 && RP >= 16 && KD > RP && KD % 64 == 0 && RP % 64 == 0 && window >= 0 && (OH == RP || OH == 2 * RP) && a16(q) &&
          a16(cache) && a16(out) && qs % (16 / esz) == 0 && os % (16 / esz) == 0;
 }
 
@@ -672,20 +685,20 @@ bool make_params(LatParams& p, const void* q, long qs, const void* cache, const 
 
 int lk_latent_attn_prefill(const void* q, long qs, const void* cache, const int* bt, int bt_stride, const int* cu_q, const int* ctx_lens, int nseq,
                            long rows, int BS, int H, int KD, int RP, int window, float scale, const float* sink, const void* gate, long gs,
-                           void* out, long os, int esz, hipStream_t st) {
+                           void* out, long os, int OH, int esz, hipStream_t st) {
   if (rows <= 0 || nseq <= 0) return 0;
   LatParams p;
-  if (!make_params(p, q, qs, cache, bt, bt_stride, BS, H, KD, RP, window, scale, sink, gate, gs, out, os, esz)) return -1;
+  if (!make_params(p, q, qs, cache, bt, bt_stride, BS, H, KD, RP, window, scale, sink, gate, gs, out, os, OH, esz)) return -1;
   if (esz == 2 && mfma_shape(RP, KD)) return run_prefill(p, cu_q, ctx_lens, nseq, rows, st);
   return esz == 2 ? run_plain<bf16_t>(p, cu_q, ctx_lens, nseq, rows, st) : run_plain<float>(p, cu_q, ctx_lens, nseq, rows, st);
 }
 
 int lk_latent_attn_decode(const void* q, long qs, const void* cache, const int* bt, int bt_stride, const int* ctx_lens, int B, int Z, int BS, int H,
                           int KD, int RP, int window, float scale, const float* sink, const void* gate, long gs, void* out, long os,
-                          float* part, int esz, hipStream_t st) {
+                          int OH, float* part, int esz, hipStream_t st) {
   if (B <= 0) return 0;
   LatParams p;
-  if (!make_params(p, q, qs, cache, bt, bt_stride, BS, H, KD, RP, window, scale, sink, gate, gs, out, os, esz)) return -1;
+  if (!make_params(p, q, qs, cache, bt, bt_stride, BS, H, KD, RP, window, scale, sink, gate, gs, out, os, OH, esz)) return -1;
   if (esz == 2 && mfma_shape(RP, KD)) {
     if (Z < 1 || Z > 65535 || (Z > 1 && !part)) return -1;
     return run_decode(p, ctx_lens, B, Z, part, st);

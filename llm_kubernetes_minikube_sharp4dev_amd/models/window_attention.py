@@ -263,10 +263,11 @@ class LatentAttnSpec:
         """Whether scores and averages run on the cached latent (``ops.latent``; queries through ``W_uk^T`` once, the averages
         through ``W_uv`` afterwards): bf16 on the GPU, where its matrix kernels take the row's size, for a sliding window (prompt rows
         then cost alike at every length), where a token's row is at most a quarter of its expanded heads and the products per key at
-        most 3.5 times theirs.  One mixer, expanded -> cached latent, at 1,024 positions, in us for 4,096 prompt rows / 64 / 4
-        decoded: 16 heads of 128 + 64 / 128, rank 512 (3.4 times the products), window 512: 336 / 138 / 41 -> 314 / 61 / 39; 32 heads,
-        window 2,048: 732 / 401 / 67 -> 593 / 78 / 47; 16 heads of 64 + 32 / 64, rank 128 (2 times): 155 / 47 / 29 -> 137 / 35 / 27;
-        rank 256 (3.6 times, beyond the line): 193 / 70 / 32 -> 205 / 47 / 32."""
+        most 3.5 times theirs.  Its error is no larger than the expanded form's (the averages go into ``W_uv`` in two bf16 parts).
+        One mixer, expanded -> cached latent, at 1,024 positions, in us for 4,096 prompt rows / 64 / 4 decoded: 16 heads of 128 + 64 / 128,
+        rank 512 (3.4 times the products), window 512: 333 / 143 / 41 -> 343 / 66 / 40; 32 heads, window 2,048: 692 / 415 / 67 -> 645 / 83 /
+        48; 16 heads of 64 + 32 / 64, rank 128 (2 times): 153 / 47 / 30 -> 140 / 35 / 27; rank 256 (3.6 times, beyond the line): 192 / 74 /
+        33 -> 216 / 47 / 33."""
         rp, rdp = ops.latent_row(self.kv_rank, self.rot_dim)
         return (dtype == torch.bfloat16 and torch.device(device).type == "cuda" and self.window > 0 and not self.gate_elem
                 and self.rot_dim > 0 and rp in (128, 256, 512) and rdp in (64, 128)
@@ -319,7 +320,8 @@ def _absorbed_attention(u, rows, w_uq, w_heads, dq_norm, dkv_norm, cache, meta: 
     q = ops.linear(cq, w_uq)
     qa = torch.empty(T, H, rp + rdp, dtype=u.dtype, device=u.device)
     ops.latent_query(q, w_heads[0], qa, spec.kdim, spec.dim, spec.rot_dim, freq, meta.positions, rp, adjacent=True, mag=mag)
-    lat = torch.empty(T, H, rp, dtype=u.dtype, device=u.device)
+    # the averages in two bf16 parts: rounded to one they would add a rounding that expanded values, averaged in f32, do not have
+    lat = torch.empty(T, H, 2 * rp, dtype=u.dtype, device=u.device)
     gate = u[:, rows.off["g"]:rows.off["g"] + H]
     Tp, Bd = meta.num_prefill_tokens, meta.num_decode
     if Tp:
@@ -329,7 +331,7 @@ def _absorbed_attention(u, rows, w_uq, w_heads, dq_norm, dkv_norm, cache, meta: 
         span = meta.block_tables_d.shape[1] * cache.shape[1]
         ops.latent_attention_decode(qa[Tp:Tp + Bd], cache, meta.block_tables_d, meta.ctx_lens_d, spec.window, spec.scale, None, rp,
                                     lat[Tp:Tp + Bd], splits=ops.latent_decode_splits(Bd, H, min(span, spec.window)), gate=gate[Tp:Tp + Bd])
-    ops.head_linear(lat.view(T, H * rp), w_heads[1], rp, out.view(T, H, spec.vdim_p))
+    ops.head_linear(lat.view(T, 2 * H * rp), w_heads[1], 2 * rp, out.view(T, H, spec.vdim_p), parts=2)
     return out
 
 

@@ -77,15 +77,16 @@ def latent_query_rot(q, qa, H: int, qdim: int, dim: int, rot_dim: int, freq, pos
     return qa
 
 
-def head_linear(x, w, x_head: int, out):
+def head_linear(x, w, x_head: int, out, parts: int = 1):
     """Per-head products: ``out[t, h, :N] = w[h] x[t, h * x_head : h * x_head + K]`` for ``w`` [H, N, K] and ``out`` [T, H, >= N]
-    (a view whose last dimension is contiguous); f32 accumulation."""
+    (a view whose last dimension is contiguous); f32 accumulation.  ``parts`` 2 (bf16): the K columns behind those add to them, an
+    operand that is kept in two bf16 parts."""
     if use_hip(x):
-        lib().head_linear(x, w, int(x_head), out)
+        lib().head_linear(x, w, int(x_head), out, int(parts))
         return out
     H, N, K = w.shape
     T = x.shape[0]
-    xs = torch.stack([x[:, h * x_head:h * x_head + K] for h in range(H)], 0).float()           # [H, T, K]
+    xs = torch.stack([x[:, h * x_head:h * x_head + parts * K].float().view(T, parts, K).sum(1) for h in range(H)], 0)   # [H, T, K]
     out[..., :N] = torch.bmm(xs, w.float().transpose(1, 2).contiguous()).transpose(0, 1).to(out.dtype)
     return out
 
@@ -127,9 +128,16 @@ def _gather(cache, table, n):
     return cache[table[: (n + BS - 1) // BS].long()].reshape(-1, cache.shape[2])[:n].float()
 
 
+def _put(out, v, rp: int):
+    out[..., :rp] = v.to(out.dtype)
+    if out.shape[-1] > rp:
+        out[..., rp:] = (v - out[..., :rp].float()).to(out.dtype)
+
+
 def latent_attention_prefill(qa, cache, block_tables, cu_q, ctx_lens, window: int, scale: float, sink, rp: int, out, max_len: int, gate=None):
     """Query chunks over their sequences' cached rows (their own included).  ``qa`` [T, H, KD]; ``sink`` f32 [H] or None; ``window`` 0:
-    causal; ``out`` [T, H, rp] receives the averaged latents (head h times ``sigmoid(gate[:, h])`` with a ``gate`` [T, H])."""
+    causal; ``out`` [T, H, rp] receives the averaged latents (head h times ``sigmoid(gate[:, h])`` with a ``gate`` [T, H]).  With
+    ``out`` [T, H, 2 rp] (bf16) they come in two parts, the rounded value and the rest behind it."""
     if use_hip(qa):
         lib().latent_attn_prefill(qa, cache, block_tables, cu_q, ctx_lens, int(window), float(scale), sink, int(rp), out, int(max_len), gate)
         return out
@@ -139,12 +147,12 @@ def latent_attention_prefill(qa, cache, block_tables, cu_q, ctx_lens, window: in
         n = int(ctx_lens[b])
         r = _rows(qa[s0:s1].float(), _gather(cache, block_tables[b], n), torch.arange(n - (s1 - s0), n, device=qa.device), window, scale,
                   sink, rp)
-        out[s0:s1] = (r if gate is None else r * torch.sigmoid(gate[s0:s1, : r.shape[1], None].float())).to(out.dtype)
+        _put(out[s0:s1], r if gate is None else r * torch.sigmoid(gate[s0:s1, : r.shape[1], None].float()), rp)
     return out
 
 
 def latent_attention_decode(qa, cache, block_tables, ctx_lens, window: int, scale: float, sink, rp: int, out, splits: int = 1, gate=None):
-    """One query row per sequence at its last position (ctx - 1).  ``gate``: as in :func:`latent_attention_prefill`."""
+    """One query row per sequence at its last position (ctx - 1).  ``gate`` and an ``out`` in two parts: as in :func:`latent_attention_prefill`."""
     if use_hip(qa):
         lib().latent_attn_decode(qa, cache, block_tables, ctx_lens, window, float(scale), sink, int(rp), out, int(splits), gate)
         return out
@@ -153,5 +161,5 @@ def latent_attention_decode(qa, cache, block_tables, ctx_lens, window: int, scal
         if n < 1:
             continue
         r = _rows(qa[b:b + 1].float(), _gather(cache, block_tables[b], n), torch.tensor([n - 1], device=qa.device), window, scale, sink, rp)
-        out[b:b + 1] = (r if gate is None else r * torch.sigmoid(gate[b:b + 1, : r.shape[1], None].float())).to(out.dtype)
+        _put(out[b:b + 1], r if gate is None else r * torch.sigmoid(gate[b:b + 1, : r.shape[1], None].float()), rp)
     return out
