@@ -180,16 +180,16 @@ __global__ __launch_bounds__(256) void head_linear_lds_kernel(const T* __restric
 // K 128 -> 512 and K 512 -> 128 columns, 16 heads, the rotated part included.
 template <typename T, int RT, int PARTS>
 __global__ __launch_bounds__(256) void head_linear_few_kernel(const T* __restrict__ x, long xs, long xh, const T* __restrict__ w, int N, int K,
-                                                              long rows, T* __restrict__ out, long os, long oh, int vec, int vst, int ncol,
+                                                              long rows, T* __restrict__ out, long os, long oh, int vec, int vst, int H, int ncol,
                                                               RotTail rot) {
   constexpr int EV = El<T>::V, STEP = 4 * EV, NT = 2, U = 4;
   static_assert(PARTS == 1 || sizeof(T) == 2, "f32 operands are whole");
   __shared__ floatx4 part[4][RT * NT][64];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, n16 = lane & 15, g = lane >> 4;
-  const int h = blockIdx.x, c0 = blockIdx.y * 16 * NT;
+  const int h = blockIdx.x % H, cb = blockIdx.x / H, c0 = cb * 16 * NT;
   const long t0 = (long)blockIdx.z * 16 * RT;
-  if ((int)blockIdx.y >= ncol) {   // the whole workgroup
-    rot_tail<T>(rot, x, xs, xh, out, os, oh, h, t0 + 16 * ((int)blockIdx.y - ncol), rows);
+  if (cb >= ncol) {   // the whole workgroup
+    rot_tail<T>(rot, x, xs, xh, out, os, oh, h, t0 + 16 * (cb - ncol), rows);
     return;
   }
   const T* xr[RT];
@@ -268,8 +268,8 @@ int head_linear_t(const void* x, long xs, long xh, const void* w, int H, int N, 
   const bool fused = rot.RDP > 0 && N > 0 && rows <= 128;
   const int tail = fused ? 1 : 0;   // workgroups of 16 rows each behind the columns'
 #define LK_HEAD(RT)                                                                                                                          \
-  head_linear_few_kernel<T, RT, PARTS><<<dim3((unsigned)H, (unsigned)((N + 31) / 32 + tail * RT), (unsigned)((rows + 16 * RT - 1) / (16 * RT))),    \
-                                  256, 0, st>>>((const T*)x, xs, xh, (const T*)w, N, K, rows, (T*)out, os, oh, vec, vst, (N + 31) / 32, rot)
+  head_linear_few_kernel<T, RT, PARTS><<<dim3((unsigned)((long)H * ((N + 31) / 32 + tail * RT)), 1, (unsigned)((rows + 16 * RT - 1) / (16 * RT))),  \
+                                  256, 0, st>>>((const T*)x, xs, xh, (const T*)w, N, K, rows, (T*)out, os, oh, vec, vst, H, (N + 31) / 32, rot)
   if (N == 0)
     ;
   else if (rows > 128 && vec && (PARTS == 1 || K % 64 == 0))
@@ -294,7 +294,7 @@ int head_linear_t(const void* x, long xs, long xh, const void* w, int H, int N, 
 int head_products(const void* x, long xs, long xh, const void* w, int H, int N, int K, long rows, void* out, long os, long oh, int qdim, int dim,
                   int rd, const float* freq, const int* positions, int rp, int RDP, int adj, float mag, int esz, hipStream_t st, int parts) {
   if (rows <= 0) return 0;
-  if (H < 1 || H > 65535 || N < 0 || (N > 0 && K < 1) || (N + 31) / 32 > 65000) return -1;
+  if (H < 1 || H > 65535 || N < 0 || (N > 0 && K < 1) || (N + 63) / 64 > 65535 || (long)H * ((N + 31) / 32 + 4) > 2147483647L) return -1;
   if (rd < 0 || rd % 2 || rd > kRotMax || dim < 0 || dim + rd > qdim || rd > RDP || N > (RDP > 0 ? rp : N) || (rd > 0 && (!freq || !positions))) return -1;
   const int ev = 16 / esz;
   const auto a16 = [](const void* p, int b) { return reinterpret_cast<uintptr_t>(p) % b == 0; };

@@ -189,3 +189,16 @@ def test_head_products_of_two_parts(rows, H, N, K):
     want = torch.einsum("thk,hnk->thn", hi.double() + lo.double(), w)
     # half a step of the result, f32 sums of 2 K terms
     assert bool(((out.double().cpu() - want).abs() <= 2 ** -8 * want.abs() + 1e-5).all())
+
+
+@pytest.mark.gpu
+def test_head_products_of_many_columns():
+    """More 32-column workgroups than a grid's second dimension has places."""
+    from llm_kubernetes_minikube_sharp4dev_amd import ops
+    N, K = 32 * 65536 + 40, 8
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x, w = torch.randn(2, K, generator=g, device="cuda").bfloat16(), torch.randn(1, N, K, generator=g, device="cuda").bfloat16()
+    out = torch.empty(2, 1, N, dtype=torch.bfloat16, device="cuda")
+    ops.head_linear(x, w, K, out)
+    want = x.double() @ w[0].double().T
+    assert bool(((out[:, 0].double() - want).abs() <= 2 ** -8 * want.abs() + 1e-5).all())
