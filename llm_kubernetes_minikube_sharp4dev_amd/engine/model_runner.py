@@ -177,7 +177,7 @@ class ModelRunner:
 
     @staticmethod
     def _tune_decode(model) -> dict:
-        """Weight-streaming kernel vs prefill GEMM per decode M bucket and projection
+        """Weight-streaming, few-row or prefill kernel per decode M bucket and projection
         (ops.tune_decode, ~1 s).  Under TP the leader's measurements are used by every rank, so
         the ranks of a group run the same kernels."""
         tp = getattr(model, "tp", None)
@@ -186,15 +186,17 @@ class ModelRunner:
         if tp is not None and tp.enabled and not getattr(tp, "simulated", False):
             import torch.distributed as dist
 
-            box = [(dict(ops._DECODE_TABLE), dict(ops._WS_VARIANTS)) if lead else None]
+            box = [(dict(ops._DECODE_TABLE), dict(ops._WS_VARIANTS), dict(ops._ROWS_TABLE)) if lead else None]
             dist.broadcast_object_list(box, src=tp.ranks[0] if tp.ranks else 0, group=tp.ctrl or tp.group)
             ops._DECODE_TABLE.clear()
             ops._DECODE_TABLE.update(box[0][0])
+            ops._ROWS_TABLE.clear()
+            ops._ROWS_TABLE.update(box[0][2])
             if not lead:
                 ops.apply_ws_variants(box[0][1])
         picks = {}
-        for (m, n, k, sw), arm in sorted(ops._DECODE_TABLE.items()):
-            picks.setdefault(f"N{n} K{k}{' swiglu' if sw else ''}", []).append(f"{m}:{arm}")
+        for m, n, k, sw in sorted(set(ops._DECODE_TABLE) | set(ops._ROWS_TABLE)):
+            picks.setdefault(f"N{n} K{k}{' swiglu' if sw else ''}", []).append(f"{m}:{ops.decode_route(m, n, k, sw)}")
         log.info("decode GEMM routing (M bucket: kernel): %s", "; ".join(f"{k} {' '.join(v)}" for k, v in picks.items()))
         if ops._WS_VARIANTS:
             log.info("weight-streaming kernel per row tile (1 = loader waves): %s",

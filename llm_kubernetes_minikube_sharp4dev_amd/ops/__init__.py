@@ -400,13 +400,13 @@ ROWS_MAX_M = 1024
 _ROWS_RULE: dict = {}
 
 
-def _rows_rule(M: int, N: int, K: int, epi: int) -> Optional[bool]:
-    """None: not the few-row kernel; else its ``wide`` argument."""
+def _rows_cost(M: int, N: int, K: int, epi: int):
+    """(us of the few-row kernel, its ``wide`` argument, us of the other kernels), or None where it does not take the shape."""
     mt = (M + 15) // 16 if M <= 64 else 4 * ((M + 63) // 64)   # 16-row tiles of X
     key = (mt, N, K, epi)
     if key in _ROWS_RULE:
         return _ROWS_RULE[key]
-    pick = None
+    est = None
     if 1 <= M <= ROWS_MAX_M and (K <= 8192 or mt == 1) and lib().rows_supported(M, N, K, epi):
         mb, rows = N * K * 2 / 1e6, 16 * mt
 
@@ -428,18 +428,42 @@ def _rows_rule(M: int, N: int, K: int, epi: int) -> Optional[bool]:
             other = min(20 + K / 256, 4 + K / 64)
         else:
             other = min(17 + 3 * K / 1024, 6 + K / 64)
-        if t < other:
-            pick = wide
-    _ROWS_RULE[key] = pick
-    return pick
+        est = (t, wide, other)
+    _ROWS_RULE[key] = est
+    return est
+
+
+def _rows_rule(M: int, N: int, K: int, epi: int) -> Optional[bool]:
+    """None: not the few-row kernel; else its ``wide`` argument."""
+    est = _rows_cost(M, N, K, epi)
+    return est[1] if est is not None and est[0] < est[2] else None
+
+
+# What ``tune_decode`` measured of the few-row kernel for a plain or SwiGLU projection, {(M bucket, N, K, swiglu): wide, or None
+# where another kernel (``_DECODE_TABLE``) was faster}; the rule above holds for shapes and rows that were not measured.
+_ROWS_TABLE: dict = {}
+
+
+def _rows_choice(M: int, N: int, K: int, epi: int) -> Optional[bool]:
+    if epi < 2 and M > LM_HEAD_SKINNY_MAX_M and _ROWS_TABLE:
+        key = (_decode_bucket(M), N, K, epi == 1)
+        if key in _ROWS_TABLE:
+            return _ROWS_TABLE[key]
+    return _rows_rule(M, N, K, epi)
+
+
+def decode_route(M: int, N: int, K: int, swiglu: bool) -> str:
+    """The kernel that :func:`linear` / :func:`linear_swiglu` run for M rows of a tuned projection: "rows", "rows wide", "ws" or "gemm"."""
+    wide = _rows_choice(M, N, K, 1 if swiglu else 0)
+    return _DECODE_TABLE.get((_decode_bucket(M), N, K, swiglu), "ws") if wide is None else "rows wide" if wide else "rows"
 
 
 def _rows(x, w, b, epi: int):
-    """The product on the few-row kernel, or None where the rule or the operands' layout say otherwise."""
+    """The product on the few-row kernel, or None where the measured table, the rule or the operands' layout say otherwise."""
     if not (x.dim() == 2 and w.dim() == 2 and SKINNY_MAX_M < x.shape[0] <= (WS_MAX_M if GEMM_LIBRARY else ROWS_MAX_M)
             and _gemm_ok(x, w) and w.data_ptr() % 16 == 0):
         return None
-    wide = _rows_rule(x.shape[0], w.shape[0], w.shape[1], epi)
+    wide = _rows_choice(x.shape[0], w.shape[0], w.shape[1], epi)
     return None if wide is None else lib().rows_linear(x, w, b, epi, wide)
 
 
@@ -767,10 +791,14 @@ def apply_ws_variants(table: dict):
 
 def tune_decode(weights, ms: Sequence[int] = DECODE_TUNE_MS, iters: int = 3, cold_bytes: int = 640 << 20) -> dict:
     """For each decode-sized M bucket and each (weight, swiglu) pair, time the weight-streaming
-    kernel against the prefill GEMM with the weights arriving from HBM (each launch reads the
-    next of enough copies to overflow the 256 MB MALL, back-to-back launches as in a decode
-    graph) and record the faster in the dispatch table.  Returns {(M, N, K, swiglu): {arm: us}}
-    plus, per measured row tile, {(M, N, K, swiglu, "ws_variant"): {"ring" / "loader": us}}."""
+    kernel, the prefill GEMM and the few-row kernel in a hipGraph, each launch on the next copy
+    of the weight (enough to overflow the 256 MB MALL for weights of 4 MB and more; below, 64 copies
+    lie in it whole), and record the faster of the first two (`_DECODE_TABLE`: what
+    steps with a fused consumer choose by) and whether the few-row kernel is faster still
+    (`_ROWS_TABLE`: what `linear` chooses by).  The few-row rule's answer stands unless another arm is 5 %
+    faster, so that near ties do not change from one start to the next.  Returns
+    {(M, N, K, swiglu): {"ws" / "gemm": us}}, {(M, N, K, swiglu, "few", "rows"): {arm: us}} of all arms and,
+    per measured row tile, {(M, N, K, swiglu, "ws_variant"): {"ring" / "loader": us}}."""
     import statistics
 
     L = lib()
@@ -779,9 +807,9 @@ def tune_decode(weights, ms: Sequence[int] = DECODE_TUNE_MS, iters: int = 3, col
     for w, swiglu in weights:
         N, K = w.shape
         swiglu = bool(swiglu)
-        # (at most 96 launches per graph: weights below 7 MB are then read from the MALL in part, where a launch's chain
-        # and not the memory decides; a thousand captured launches per arm took seconds)
-        copies = [w] + [w.clone() for _ in range(min(95, max(1, -(-cold_bytes // (N * K * 2)) - 1)))]
+        # (at most 64 launches per graph: a thousand captured launches per arm took seconds, and for small weights a launch's
+        # chain and not the memory decides)
+        copies = [w] + [w.clone() for _ in range(min(63, max(1, -(-cold_bytes // (N * K * 2)) - 1)))]
 
         def timed(fns):
             # as decode steps run: launches of a hipGraph (eager ones of a few microseconds are bound by the
@@ -834,11 +862,26 @@ def tune_decode(weights, ms: Sequence[int] = DECODE_TUNE_MS, iters: int = 3, col
             cfg = _gemm_default(M, N, K, epi)
             if cfg is not None and L.gemm_supported(M, N, K, epi, cfg[1], cfg[2], cfg[0]):
                 arms["gemm"] = lambda c, x=x, cfg=cfg: L.gemm(x, c, None, epi, cfg[1], None, cfg[0], cfg[2])
-            if len(arms) < 2:
+            # the few-row kernel in the form that the rule prefers, unless the rule has it beyond 1.5 times the others (its
+            # estimates are good to 30 %)
+            est = _rows_cost(M, N, K, epi)
+            rows = {}
+            if (est is not None and est[0] < 1.5 * est[2] and SKINNY_MAX_M < M <= (WS_MAX_M if GEMM_LIBRARY else ROWS_MAX_M)
+                    and w.data_ptr() % 16 == 0):
+                rows["rows wide" if est[1] else "rows"] = lambda c, x=x, wide=est[1]: L.rows_linear(x, c, None, epi, wide)
+            if len(arms) + len(rows) < 2:
                 continue
-            med = timed(arms)
-            _DECODE_TABLE[(M, N, K, swiglu)] = min(med, key=med.get)
-            out[(M, N, K, swiglu)] = {k: round(v, 1) for k, v in med.items()}
+            med = timed({**arms, **rows})
+            key = (M, N, K, swiglu)
+            if len(arms) > 1:
+                _DECODE_TABLE[key] = min(arms, key=med.get)
+                out[key] = {k: round(med[k], 1) for k in arms}
+            if rows and arms:
+                best = min(med, key=med.get)
+                stay = next(iter(rows)) if est[0] < est[2] else min(arms, key=med.get)
+                pick = best if med[best] < 0.95 * med[stay] else stay
+                _ROWS_TABLE[key] = {"rows": False, "rows wide": True}.get(pick)
+                out[key + ("few", "rows")] = {k: round(v, 1) for k, v in med.items()}
         del copies
     return out
 

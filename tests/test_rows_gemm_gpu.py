@@ -54,3 +54,59 @@ def test_routes_agree(M, N, K):
     for y, r in ((ops.linear(x, w), _ref(x, w, None, 0)), (ops.linear(x, w, b), _ref(x, w, b, 2)),
                  (ops.linear(x, w, b, act="gelu"), _ref(x, w, b, 3)), (ops.linear_swiglu(x, w), _ref(x, w, None, 1))):
         assert ((y.double() - r).norm() / r.norm()) < 4e-3
+
+
+@pytest.fixture(autouse=True)
+def tables():
+    """The measured decode tables, put back behind a test that fills them."""
+    saved = [(t, dict(t)) for t in (ops._DECODE_TABLE, ops._ROWS_TABLE, ops._WS_VARIANTS)]
+    for t, _ in saved[:2]:
+        t.clear()
+    yield
+    for t, v in saved:
+        t.clear()
+        t.update(v)
+    ops.apply_ws_variants(saved[2][1])
+
+
+class Spy:
+    """The kernel library with the names of the products that ran."""
+
+    def __init__(self, lib):
+        self.lib, self.ran = lib, []
+
+    def __getattr__(self, name):
+        f = getattr(self.lib, name)
+        if name in ("rows_linear", "ws_linear", "gemm", "skinny_linear", "gemv_decode"):
+            return lambda *a, **k: (self.ran.append(name), f(*a, **k))[1]
+        return f
+
+
+@pytest.mark.parametrize("N,K,swiglu", [(2048, 2048, False), (1024, 1024, False), (4096, 1024, True), (10368, 2048, False)])
+def test_measured_routes_win(monkeypatch, N, K, swiglu):
+    """What start-up measured is what linear runs: each bucket's choice, also against the rule; shapes without an entry take the rule."""
+    w = torch.randn(N, K, device="cuda").bfloat16() * K ** -0.5
+    ms = (32, 64, 256)
+    res = ops.tune_decode([(w, swiglu)], ms=ms)
+    ms = [m for m in ms if (m, N, K, swiglu) in ops._ROWS_TABLE]
+    assert ms
+    spy = Spy(ops.lib())
+    monkeypatch.setattr(ops, "lib", lambda: spy)
+    run = ops.linear_swiglu if swiglu else ops.linear
+    for m in ms:
+        key = (m, N, K, swiglu)
+        us = res[key + ("few", "rows")]
+        assert {"ws", "gemm"} < set(us)
+        route = ops.decode_route(m, N, K, swiglu)
+        assert us[route] <= min(us.values()) / 0.94 + 0.1   # within the margin of a near tie (times rounded to 0.1 us)
+        x = torch.randn(m - 3, K, device="cuda").bfloat16()
+        for choice in (ops._ROWS_TABLE[key], None, False):      # the measured one, then both others forced
+            ops._ROWS_TABLE[key] = choice
+            spy.ran.clear()
+            run(x, w)
+            want = {None: "ws_linear" if ops._DECODE_TABLE[key] == "ws" else "gemm"}.get(choice, "rows_linear")
+            assert spy.ran == [want]
+        del ops._ROWS_TABLE[key]
+        spy.ran.clear()
+        run(x, w)
+        assert (spy.ran == ["rows_linear"]) == (ops._rows_rule(m - 3, N, K, 1 if swiglu else 0) is not None)
