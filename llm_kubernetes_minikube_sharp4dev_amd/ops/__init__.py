@@ -386,7 +386,7 @@ def _decode_bucket(M: int) -> Optional[int]:
 
 # Few rows (csrc/rows_gemm.hip, one launch with any epilogue) or the kernels with larger tiles.  A workgroup of the few-row
 # kernel reads 16 (wide: 32) columns of W -- SwiGLU 2 x 16 -- and up to 64 rows of X, so its time is
-#   2.6 us + rounds of 256 workgroups x (their bytes / 58 KB/us) + 1 us per round behind the first,
+#   2.6 us + rounds of workgroups (one per CU) x (their bytes / 58 KB/us) + 1 us per round behind the first,
 # and not below W at 4.2 TB/s.  The other side: up to 256 rows without a bias the weight-streaming kernel (its two launches,
 # 0.14 us per MB of W, M / 22; 3.5 us for SwiGLU's second launch), else the prefill GEMM (a chain of K / 64 stages
 # whatever M is, as long as its tiles are fewer than CUs).  Measured in hipGraphs, weights cold, few-row / other (us):
@@ -408,12 +408,12 @@ def _rows_cost(M: int, N: int, K: int, epi: int):
         return _ROWS_RULE[key]
     est = None
     if 1 <= M <= ROWS_MAX_M and (K <= 8192 or mt == 1) and lib().rows_supported(M, N, K, epi):
-        mb, rows = N * K * 2 / 1e6, 16 * mt
+        mb, rows, cus = N * K * 2 / 1e6, 16 * mt, device_cus()
 
         def cost(nt, wide):
             m = min(mt, 4) if not wide else (2 if mt <= 2 else 4)
             wgs = -(-mt // 4) * (N // (16 * nt))
-            rounds = -(-wgs // 256)
+            rounds = -(-wgs // cus)
             return max(2.6 + rounds * (m + nt) * K / 32 / 58 + (rounds - 1), mb / 4.2)
 
         if epi == 1:

@@ -392,6 +392,20 @@ def test_gemm1w_default_policy(monkeypatch):
     assert all(c[0] not in ops.GEMM1W_BM for c in ops._gemm_configs(4096, 0))
 
 
+def test_few_row_rule_counts_the_devices_cus(monkeypatch):
+    """The few-row kernel's rounds are of the device's CUs: what it wins on a whole chip (128 workgroups in half a round) it loses on a
+    partition of 32 CUs, where they are four rounds."""
+    from types import SimpleNamespace
+
+    from llm_kubernetes_minikube_sharp4dev_amd import ops
+
+    monkeypatch.setattr(ops, "lib", lambda: SimpleNamespace(rows_supported=lambda *a: True))
+    for cus, pick in ((256, False), (32, None)):
+        monkeypatch.setattr(ops, "_CUS", cus)
+        monkeypatch.setattr(ops, "_ROWS_RULE", {})
+        assert ops._rows_rule(64, 2048, 2048, 0) is pick
+
+
 def test_static_gemm_table_is_well_formed(monkeypatch):
     """The shipped measured dispatch table (benchmarks/gemm_table.py on an MI355X): every entry a
     kernel / tile / split the dispatch knows, looked up by _cfg_of before the fallback policy,
