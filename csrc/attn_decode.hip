@@ -62,7 +62,11 @@ LK_DEVICE void merge_splits(int b, int qh, int d, int Hq, int max_splits, int ns
 //         XOR-swizzled LDS image of the chunk.
 // The 4 waves' (m, l, O) are merged through LDS at the end; splits > 1 emit
 // partials for lk_decode_reduce (flash-decoding).
-template <int D, int G>
+// NT: the cache is read non-temporally, for batches whose sequences share no block (a step then reads every key once, and its weights
+// and other layers pass through the caches before the next).  Rows that share blocks read them from L2 instead, which the hint would
+// give up.  8 kv heads of 128, plain -> non-temporal, us: 120 sequences of 950 own keys 85.5 -> 79.4, 32: 30.7 -> 28.8, 120 of 400: 42.4 -> 39.5;
+// 700 of 950 keys shared by 8: 54.9 -> 60.4, by 2: 62.5 -> 71.0; 64 of 3,000 with 2,800 shared by 4: 83 -> 112.
+template <int D, int G, bool NT>
 __global__ __launch_bounds__(256, LK_DECODE_WG_PER_CU) void paged_decode_kernel(
     const bf16_t* __restrict__ q, long qs, const bf16_t* __restrict__ kc,
     const bf16_t* __restrict__ vc, const int* __restrict__ block_tables, int bt_stride,
@@ -132,20 +136,19 @@ __global__ __launch_bounds__(256, LK_DECODE_WG_PER_CU) void paged_decode_kernel(
   short8 kr[2][KK], vr[NVL];
   // k_begin is block-aligned (split % BS == 0, k_start a multiple of BS): row rel of the
   // split sits at slot rel % BS of its block
-  // (non-temporal: a step reads every key once, and its weights and other layers pass through the caches before the next; 120 sequences
-  // of 950 keys, 8 kv heads of 128: 102 us (4.6 TB/s) -> 89 us (5.2 TB/s), a single sequence alike)
+  auto ld = [](const bf16_t* p) { return NT ? __builtin_nontemporal_load(reinterpret_cast<const short8*>(p)) : *reinterpret_cast<const short8*>(p); };
   auto load_chunk = [&](int c, short8 (&kd)[2][KK], short8 (&vd)[NVL]) {
     const int base = 32 * c;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       const bf16_t* kp = blk_base(kc, base + 16 * t) + (min(base + 16 * t + r16, nkeys - 1) % BS) * D + 8 * h4;
 #pragma unroll
-      for (int kk = 0; kk < KK; ++kk) kd[t][kk] = __builtin_nontemporal_load(reinterpret_cast<const short8*>(kp + 32 * kk));
+      for (int kk = 0; kk < KK; ++kk) kd[t][kk] = ld(kp + 32 * kk);
     }
 #pragma unroll
     for (int i = 0; i < NVL; ++i) {
       const int rel = min(base + i * RPL + lane / CPR, nkeys - 1);
-      vd[i] = __builtin_nontemporal_load(reinterpret_cast<const short8*>(blk_base(vc, base + i * RPL) + (rel % BS) * D + (lane % CPR) * 8));
+      vd[i] = ld(blk_base(vc, base + i * RPL) + (rel % BS) * D + (lane % CPR) * 8);
     }
   };
 
@@ -348,14 +351,15 @@ int lk_paged_decode(const bf16_t* q, long qs, const bf16_t* kc, const bf16_t* vc
                     const int* block_tables, int bt_stride, const int* ctx_lens, bf16_t* out,
                     long os, float* part_o, float* part_ml, int B, int Hq, int Hkv, int D, int BS,
                     int max_splits, int split, float scale, const int* k_start, const float* pp_o,
-                    const float* pp_ml, hipStream_t st, int* tickets, int reduce) {
+                    const float* pp_ml, hipStream_t st, int* tickets, int reduce, int own_blocks) {
   if (B == 0) return 0;
   if (Hq % Hkv || BS % 16 || split % 32 || split > kMaxSplit || split % BS) return -1;
   const int G = Hq / Hkv;
   const float scale_log2 = scale * 1.4426950408889634f;
   dim3 grid(B * Hkv, max_splits);
-#define LAUNCH(DD, GG)                                                                        \
-  paged_decode_kernel<DD, GG><<<grid, 256, 0, st>>>(q, qs, kc, vc, block_tables, bt_stride,   \
+#define LAUNCH(DD, GG) do { if (own_blocks) LAUNCH_NT(DD, GG, true); else LAUNCH_NT(DD, GG, false); } while (0)
+#define LAUNCH_NT(DD, GG, NT)                                                                 \
+  paged_decode_kernel<DD, GG, NT><<<grid, 256, 0, st>>>(q, qs, kc, vc, block_tables, bt_stride,   \
                                                     ctx_lens, out, os, part_o, part_ml, Hkv, \
                                                     BS, max_splits, split, scale_log2, k_start, \
                                                     pp_o != nullptr, pp_o, pp_ml, tickets)
@@ -372,6 +376,7 @@ int lk_paged_decode(const bf16_t* q, long qs, const bf16_t* kc, const bf16_t* vc
   else return -3;
 #undef BY_G
 #undef LAUNCH
+#undef LAUNCH_NT
   LK_CHECK_LAUNCH();
   // (fused: the last split merges; reduce == 0: the consumer merges -- the O projection's
   // weight-streaming prologue, lk_wsgemm_pro kind 2)

@@ -685,7 +685,7 @@ at::Tensor paged_decode(const at::Tensor& q, const at::Tensor& k_cache, const at
                         const c10::optional<at::Tensor>& part_ml, const c10::optional<at::Tensor>& out_,
                         const c10::optional<at::Tensor>& k_start, const c10::optional<at::Tensor>& pp_o,
                         const c10::optional<at::Tensor>& pp_ml, const c10::optional<at::Tensor>& tickets,
-                        bool reduce) {
+                        bool reduce, bool own_blocks) {
   CHECK_CUDA(q); CHECK_BF16(q); CHECK_BF16(k_cache); CHECK_BF16(v_cache);
   CHECK_I32(block_tables); CHECK_I32(ctx_lens); CHECK_CONTIG(ctx_lens);
   TORCH_CHECK(q.dim() == 3 && q.stride(2) == 1 && q.stride(1) == q.size(2), "q must be [B, Hq, D] (row-strided)");
@@ -724,7 +724,7 @@ at::Tensor paged_decode(const at::Tensor& q, const at::Tensor& k_cache, const at
                            parts ? pm.data_ptr<float>() : nullptr, B, Hq, Hkv, D, BS, (int)max_splits,
                            (int)split, (float)scale, cascade ? ip(*k_start) : nullptr,
                            cascade ? pp_o->data_ptr<float>() : nullptr, cascade ? pp_ml->data_ptr<float>() : nullptr,
-                           cur_stream(), tickets ? tickets->data_ptr<int>() : nullptr, reduce ? 1 : 0);
+                           cur_stream(), tickets ? tickets->data_ptr<int>() : nullptr, reduce ? 1 : 0, own_blocks ? 1 : 0);
   CHECK_RC(rc, "paged_decode");
   return out;
 }
@@ -2298,7 +2298,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("kv_write", &kv_write);
   m.def("decode_splits", &decode_splits);
   m.def("decode_split_size", &decode_split_size);
-  m.def("paged_decode", &paged_decode, "", py::arg("q"), py::arg("k_cache"), py::arg("v_cache"), py::arg("block_tables"), py::arg("ctx_lens"), py::arg("max_splits"), py::arg("split"), py::arg("scale"), py::arg("part_o") = py::none(), py::arg("part_ml") = py::none(), py::arg("out") = py::none(), py::arg("k_start") = py::none(), py::arg("pp_o") = py::none(), py::arg("pp_ml") = py::none(), py::arg("tickets") = py::none(), py::arg("reduce") = true);
+  m.def("paged_decode", &paged_decode, "", py::arg("q"), py::arg("k_cache"), py::arg("v_cache"), py::arg("block_tables"), py::arg("ctx_lens"), py::arg("max_splits"), py::arg("split"), py::arg("scale"), py::arg("part_o") = py::none(), py::arg("part_ml") = py::none(), py::arg("out") = py::none(), py::arg("k_start") = py::none(), py::arg("pp_o") = py::none(), py::arg("pp_ml") = py::none(), py::arg("tickets") = py::none(), py::arg("reduce") = true, py::arg("own_blocks") = false);
   m.def("prefill_rows_per_tile", &prefill_rows_per_tile);
   m.def("ws_pro", &ws_pro, "", py::arg("x"), py::arg("w"), py::arg("swiglu"), py::arg("bn"), py::arg("splits"),
         py::arg("kind"), py::arg("reduce") = false, py::arg("pp") = py::none(), py::arg("res_in") = py::none(),

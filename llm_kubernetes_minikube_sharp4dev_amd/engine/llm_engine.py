@@ -74,6 +74,7 @@ class LLMEngine:
         # state after the shared prefix is not kept.  Its sequences hold a state slot while they run.
         stateful = bool(getattr(model, "stateful", False))
         self.allocator = make_allocator(self.runner.num_blocks, block_size, enable_prefix_caching and not stateful)
+        self.runner.own_blocks = not (enable_prefix_caching and not stateful)
         self.state_pool = StateSlotPool(max_num_seqs) if stateful else None
         self._replay: dict = {}  # replay_step: request id -> its sequence
         if prefill_hold is None:

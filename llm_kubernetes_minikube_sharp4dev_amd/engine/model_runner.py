@@ -92,6 +92,7 @@ class ModelRunner:
         self.model = model
         self.device = model.device
         self.bs = block_size
+        self.own_blocks = False  # set by the engine: no prefix reuse, so no cache block belongs to two sequences
         self.max_model_len = max_model_len
         self.max_blocks = (max_model_len + block_size - 1) // block_size
         self.max_num_seqs = max_num_seqs
@@ -455,7 +456,7 @@ class ModelRunner:
             host.update(seq_cu=seq_cu, state_slots=si.state_slots)
         d = self._upload(host)
         meta = AttnMeta(positions=d["pos"], slots=d["slots"], num_prefill_tokens=Tp,
-                        num_prefill_seqs=len(si.q_lens), num_decode=si.num_decode)
+                        num_prefill_seqs=len(si.q_lens), num_decode=si.num_decode, own_blocks=self.own_blocks)
         if si.q_lens:
             meta.cu_q, meta.ctx_lens_p, meta.block_tables_p = d["cu"], d["ctx_p"], d["bt_p"]
             meta.q_lens_cpu, meta.ctx_lens_cpu = list(si.q_lens), list(si.ctx_lens)
@@ -572,7 +573,7 @@ class ModelRunner:
         split, ms = self.decode_split(B)
         st["meta"] = AttnMeta(positions=st["pos"], slots=st["slots"], num_decode=B,
                               block_tables_d=st["bt"], ctx_lens_d=st["ctx"], max_splits=ms,
-                              decode_split=split, part_o=po, part_ml=pm)
+                              decode_split=split, part_o=po, part_ml=pm, own_blocks=self.own_blocks)
         if self.stateful:
             st["meta"].seq_cu = torch.arange(B + 1, dtype=torch.int32, device=dev)
             st["meta"].state_slots = st["state_slots"]

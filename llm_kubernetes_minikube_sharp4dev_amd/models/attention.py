@@ -61,6 +61,7 @@ class AttnMeta:
     ctx_lens_d: Optional[torch.Tensor] = None
     max_splits: Optional[int] = None
     decode_split: Optional[int] = None
+    own_blocks: bool = False                 # no cache block belongs to two sequences (no prefix reuse)
     part_o: Optional[torch.Tensor] = None
     part_ml: Optional[torch.Tensor] = None
     # cascade decode: the first shared_len (device int32 [1]) keys of every decode row are
@@ -140,7 +141,7 @@ def paged_attention(qkv: torch.Tensor, k_cache, v_cache, meta: AttnMeta, Hq: int
             prefix = (meta.pp_o, meta.pp_ml)
         ops.paged_decode(q, k_cache, v_cache, meta.block_tables_d, meta.ctx_lens_d, scale,
                          meta.max_splits, meta.part_o, meta.part_ml, out=o, split=meta.decode_split,
-                         k_start=meta.shared_len, prefix=prefix)
+                         k_start=meta.shared_len, prefix=prefix, own_blocks=meta.own_blocks)
 
     def prefill():
         meta.ensure_tiles(Hq, Hkv, qkv.device, D)

@@ -277,7 +277,7 @@ class LlamaModel(nn.Module):
                                                                               device=res.device)
                 ops.paged_decode(qkv[:, : hq * D].view(M, hq, D), kc, vc, meta.block_tables_d, meta.ctx_lens_d,
                                  self.scale, meta.max_splits, po, pml, out=attn_out.view(M, hq, D),
-                                 split=meta.decode_split, reduce=False)
+                                 split=meta.decode_split, reduce=False, own_blocks=meta.own_blocks)
                 ops.gemv_decode(1, attn_out, L.o, res=res, po=po, pml=pml, ctx=meta.ctx_lens_d,
                                 max_splits=meta.max_splits, split=meta.decode_split, Hq=hq, D=D)
             else:
@@ -354,7 +354,8 @@ class LlamaModel(nn.Module):
             qkv = ops.splitk_rope_kv(qp, meta.positions, self.cos_sin, hq, hkv, D, kc, vc, meta.slots, self.rope_neox)
             attn = torch.empty(M, hq * D, dtype=res.dtype, device=res.device)
             ops.paged_decode(qkv[:, : hq * D].view(M, hq, D), kc, vc, meta.block_tables_d, meta.ctx_lens_d, self.scale,
-                             meta.max_splits, po, pml, out=attn.view(M, hq, D), split=meta.decode_split, reduce=False)
+                             meta.max_splits, po, pml, out=attn.view(M, hq, D), split=meta.decode_split, reduce=False,
+                             own_blocks=meta.own_blocks)
             op = ops.ws_pro(attn, L.o, p_o, 2, po=po, pml=pml, ctx=meta.ctx_lens_d, split=meta.decode_split,
                             max_splits=meta.max_splits, Hq=hq)
             x2 = torch.empty_like(res)

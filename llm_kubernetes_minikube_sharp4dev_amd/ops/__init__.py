@@ -157,7 +157,7 @@ def decode_tickets(device, n: int):
 
 def paged_decode(q, k_cache, v_cache, block_tables, ctx_lens, scale: float, max_splits: Optional[int] = None,
                  part_o=None, part_ml=None, out=None, split: Optional[int] = None, k_start=None, prefix=None,
-                 reduce: bool = True):
+                 reduce: bool = True, own_blocks: bool = False):
     """q [B, Hq, D] -> [B, Hq, D].  ``split`` keys per workgroup (default from
     :func:`decode_split_size`), ``max_splits`` = splits covering the block-table width —
     both static, so the launch is hipGraph-capturable.
@@ -167,7 +167,8 @@ def paged_decode(q, k_cache, v_cache, block_tables, ctx_lens, scale: float, max_
     into ``prefix`` = (o [B, Hq, D], ml [B, Hq, 2]); this call attends the rest and
     merges (the CPU reference attends everything directly).  ``reduce=False`` (GPU, no
     tickets): rows with more than one split keep their partials in ``part_o`` / ``part_ml`` for
-    the consumer to merge (:func:`ws_pro` kind 2)."""
+    the consumer to merge (:func:`ws_pro` kind 2).  ``own_blocks``: no cache block belongs to two rows (their
+    reads then pass the caches by; the result is the same)."""
     if use_hip(q):
         BS = k_cache.shape[2]
         if split is None:
@@ -179,7 +180,7 @@ def paged_decode(q, k_cache, v_cache, block_tables, ctx_lens, scale: float, max_
         fused = reduce and (DECODE_FUSED_REDUCE == 2 or (DECODE_FUSED_REDUCE == 1 and bh >= 512))
         tickets = decode_tickets(q.device, bh) if fused else None
         return lib().paged_decode(q, k_cache, v_cache, block_tables, ctx_lens, max_splits, split, scale,
-                                  part_o, part_ml, out, k_start, pp_o, pp_ml, tickets, reduce)
+                                  part_o, part_ml, out, k_start, pp_o, pp_ml, tickets, reduce, own_blocks)
     y = ref.paged_decode(q, k_cache, v_cache, block_tables, ctx_lens, scale)
     if out is not None:
         out.copy_(y)

@@ -147,6 +147,21 @@ def test_paged_decode(hip, G, D):
             assert int(tickets.abs().sum()) == 0
 
 
+@pytest.mark.parametrize("G,D", [(1, 64), (4, 128), (8, 128)])
+def test_paged_decode_own_blocks(hip, G, D):
+    """Reading the cache past the caches changes no bit, with blocks of one row each and (not promised, but safe) shared ones."""
+    torch.manual_seed(8)
+    Hkv, ctx = 2, [1, 17, 511, 700, 700]
+    kc, vc, bt = _paged_setup(len(ctx), ctx, Hkv, D, 16)
+    q = torch.randn(len(ctx), Hkv * G, D, device=DEV, dtype=torch.bfloat16)
+    cl = torch.tensor(ctx, dtype=torch.int32, device=DEV)
+    for _ in range(2):
+        for split in (128, 2048):
+            a, b = (ops.paged_decode(q, kc, vc, bt, cl, D ** -0.5, split=split, own_blocks=own) for own in (False, True))
+            assert torch.equal(a, b)
+        bt[4] = bt[3]
+
+
 def test_paged_decode_fused_merge_empty_rows(hip):
     """Rows without keys (graph-bucket padding, ctx 0) get zeros from split 0 when no reduce
     kernel runs (the separate reduce kernel leaves such rows unwritten: nobody reads them); the

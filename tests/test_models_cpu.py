@@ -368,6 +368,20 @@ def test_gemm_split_k_policy():
     assert ops._gemm_default(256, 768, 768, 2)[2] == 1  # 12 K-tiles: < 8 per split at S 2
 
 
+@pytest.mark.parametrize("prefix_caching", [True, False])
+def test_decode_reads_past_the_caches_only_without_prefix_reuse(monkeypatch, prefix_caching):
+    """Decode attention is told that no cache block belongs to two sequences exactly where prefixes are not reused."""
+    from llm_kubernetes_minikube_sharp4dev_amd import ops
+
+    hf, cfg = _hf_llama()
+    m = build_decoder(cfg, dtype=torch.float32)
+    m.load_hf_state_dict(hf.state_dict())
+    eng, told, fn = _engine(m, enable_prefix_caching=prefix_caching), [], ops.paged_decode
+    monkeypatch.setattr(ops, "paged_decode", lambda *a, own_blocks=None, **k: told.append(own_blocks) or fn(*a, own_blocks=own_blocks, **k))
+    eng.generate([[5, 17, 99, 3] * 5, [5, 17, 99, 3] * 5 + [7]], SamplingParams(max_tokens=3, temperature=0.0))
+    assert told and all(t is (not prefix_caching) for t in told)
+
+
 def test_gemm1w_default_policy(monkeypatch):
     """Fallback policy (shapes without a measured entry): 256-wide prefill tiles go to the
     one-wave-per-SIMD kernel (variant 3, csrc/gemm1w.hip) once they fill a wave of 256 CUs, its
