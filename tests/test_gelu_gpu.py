@@ -17,5 +17,7 @@ def test_every_bf16_value():
     # half a bf16 step of the result and the tail's fit; results below bf16's smallest normal value may round to zero
     tol = (2 ** -8 + 3e-4) * want.abs() + 2 ** -126
     assert bool(((got - want).abs() <= tol)[inner].all())
-    assert bool((got.abs() <= 1e-5)[fin & (d <= -5)].all())
+    # behind the fit (x <= -5, |GELU| at most 1.5e-6): the rounding of the result and 1e-9 (measured of the polynomial in f32: 5.0e-10)
+    assert bool(((got - want).abs() <= 2 ** -8 * want.abs() + 1e-9)[fin & (d <= -5)].all())
     assert bool((got == d)[d == float("inf")].all()) and bool(torch.isnan(got)[torch.isnan(d)].all())
+    assert bool(torch.isnan(got)[d == float("-inf")].all())   # -inf x 0
