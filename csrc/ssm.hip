@@ -868,9 +868,14 @@ __global__ __launch_bounds__(256, 1) void ssm_chunk_bf16_kernel(const bf16_t* __
       for (int tt = 0; tt < 4; ++tt) ya[tt] *= sec[16 * tt + r16];
     }
     __syncthreads();  // M is complete
-    short8 xf[2];
+    // (xe: without the second tile of a 32-step, whose M rows are zeros for an even token tile: an infinity or NaN among its x would
+    // reach outputs up to 31 tokens before it, not only those of its own 16 as in chunks of 16)
+    short8 xf[2], xe[2];
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk) xf[kk] = *reinterpret_cast<const short8*>(sXt + (16 * w + r16) * LT + 32 * kk + 8 * g);
+    for (int kk = 0; kk < 2; ++kk) {
+      xf[kk] = *reinterpret_cast<const short8*>(sXt + (16 * w + r16) * LT + 32 * kk + 8 * g);
+      xe[kk] = g < 2 ? xf[kk] : (short8){0, 0, 0, 0, 0, 0, 0, 0};
+    }
 #pragma unroll
     for (int tt = 0; tt < 4; ++tt) {
 #pragma unroll
@@ -878,7 +883,7 @@ __global__ __launch_bounds__(256, 1) void ssm_chunk_bf16_kernel(const bf16_t* __
 #pragma unroll
         for (int k = 2; k >= 0; --k) {
           const short8 m = *reinterpret_cast<const short8*>(sM + (k * L + 16 * tt + r16) * LT + 32 * kk + 8 * g);
-          ya[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[kk], m, ya[tt], 0, 0, 0);
+          ya[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(2 * kk == tt ? xe[kk] : xf[kk], m, ya[tt], 0, 0, 0);
         }
       const int t = 16 * tt + r16, p = p0 + 16 * w + 4 * g;
       if (t < tl && p < P) *reinterpret_cast<floatx4*>(y + (long)(row0 + t0 + t) * ys + (long)h * P + p) = ya[tt];
@@ -973,7 +978,9 @@ __global__ __launch_bounds__(256) void gated_group_rmsnorm_wave_kernel(const flo
   }
 }
 
-// prompt portions (some sequence of the step has >= kChunkMin rows): the chunked MFMA kernel
+// prompt portions (some sequence of the step has >= kChunkMin rows): the chunked MFMA kernel, for the step's other sequences too.  What
+// decides in short portions and decode rows is the pass over the state, so the 64-token chunks lead there as well; us, chunks of 16 ->
+// of 64, 64 heads of [64, 128]: 512 rows and 64 decode rows 322 -> 212, 8 and 64 177 -> 157, 64 portions of 8 170 -> 153, one of 8 14.4 -> 11.4.
 constexpr int kChunkMin = 8;
 
 template <typename T>

@@ -60,3 +60,21 @@ def test_gated_group_norm(hip, rows, inner, ng):
     r = (v / (v.pow(2).mean(-1, keepdim=True) + 1e-5).sqrt()).reshape(rows, inner) * w.double()
     o = ops.gated_group_rmsnorm(y, z, w, ng, 1e-5).double()
     assert ((o - r).abs() <= 2.0 ** -8 * r.abs() + 1e-6).all()   # one bf16 rounding of an f32 value
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("at", [20, 50, 95, 118])
+def test_non_finite_rows_reach_no_earlier_tile(bad, at):
+    """An infinity or NaN among one token's x leaves the outputs of the 16-token tiles before its own as they are without it."""
+    H, P, N, G, T = 2, 64, 128, 1, 130
+    g = torch.Generator().manual_seed(1)
+    r = lambda *s: torch.randn(*s, generator=g).cuda()
+    xbc, dt, db, A, D = (0.5 * r(T, H * P + 2 * G * N)).bfloat16(), r(T, H).bfloat16(), 0.3 * r(H), 0.3 * r(H), 0.3 * r(H)
+    cu, slots = torch.tensor([0, T], dtype=torch.int32).cuda(), torch.zeros(1, dtype=torch.int32).cuda()
+    pos = torch.arange(T, dtype=torch.int32).cuda()
+    run = lambda x: ops.ssm_scan(x, dt, H, P, N, G, db, A, D, torch.zeros(1, H, P, N).cuda(), cu, slots, pos, T)
+    want = run(xbc)
+    xbc = xbc.clone()
+    xbc[at, 3] = bad
+    got = run(xbc)
+    assert torch.equal(got[:at // 16 * 16], want[:at // 16 * 16]) and not bool(torch.isfinite(got[at, 3]))
