@@ -86,23 +86,30 @@ class _LatentAttention(nn.Module):
         self.freq = _p(max(s.rot_dim // 2, 1), **f)
         self.hscale = _p(H, **f)
         s.absorbed = s.absorb(e["dtype"], e["device"])
-        # the up projections by head, for attention on the cached latent; derived from w_ukv by init_constants
+        # the up projections by head, for attention on the cached latent; derived from w_ukv by init_constants, whenever weights were
+        # loaded.  W_uv lies in w_ukv as it is used unless the latent's row is padded.
         rp = ops.latent_row(s.kv_rank, s.rot_dim)[0]
         self.register_buffer("w_uk_t", torch.zeros(H, rp, _pad8(s.dim), **e) if s.absorbed else None, persistent=False)
-        self.register_buffer("w_uv_h", torch.zeros(H, s.vdim_p, rp, **e) if s.absorbed else None, persistent=False)
+        self.register_buffer("w_uv_h", torch.zeros(H, s.vdim_p, rp, **e) if s.absorbed and rp != s.kv_rank else None, persistent=False)
+        self.register_load_state_dict_post_hook(lambda module, keys: module.init_constants())
 
+    @torch.no_grad()
     def init_constants(self):
         s = self.spec
         self.freq.copy_(s.rot.freq_tensor(self.freq.device))
         self.hscale.fill_(s.scale)
-        if s.absorbed:
-            uv = self.up_rows.off["uv"]
+        if self.w_uk_t is not None:
             self.w_uk_t[:, :s.kv_rank, :s.dim].copy_(self.w_ukv[:s.heads * s.dim].view(s.heads, s.dim, s.kv_rank).transpose(1, 2))
-            self.w_uv_h[:, :, :s.kv_rank].copy_(self.w_ukv[uv:uv + s.heads * s.vdim_p].view(s.heads, s.vdim_p, s.kv_rank))
+        if self.w_uv_h is not None:
+            self.w_uv_h[:, :, :s.kv_rank].copy_(self._w_uv())
+
+    def _w_uv(self):
+        s, uv = self.spec, self.up_rows.off["uv"]
+        return self.w_ukv[uv:uv + s.heads * s.vdim_p].view(s.heads, s.vdim_p, s.kv_rank)
 
     @property
     def w_heads(self):
-        return self.w_uk_t, self.w_uv_h
+        return self.w_uk_t, self._w_uv() if self.w_uv_h is None else self.w_uv_h
 
 
 class _TableExperts(nn.Module):

@@ -321,7 +321,8 @@ def _absorbed_attention(u, rows, w_uq, w_heads, dq_norm, dkv_norm, cache, meta: 
     qa = torch.empty(T, H, rp + rdp, dtype=u.dtype, device=u.device)
     ops.latent_query(q, w_heads[0], qa, spec.kdim, spec.dim, spec.rot_dim, freq, meta.positions, rp, adjacent=True, mag=mag)
     # the averages in two bf16 parts: rounded to one they would add a rounding that expanded values, averaged in f32, do not have
-    lat = torch.empty(T, H, 2 * rp, dtype=u.dtype, device=u.device)
+    parts = 2 if u.dtype == torch.bfloat16 else 1
+    lat = torch.empty(T, H, parts * rp, dtype=u.dtype, device=u.device)
     gate = u[:, rows.off["g"]:rows.off["g"] + H]
     Tp, Bd = meta.num_prefill_tokens, meta.num_decode
     if Tp:
@@ -331,7 +332,7 @@ def _absorbed_attention(u, rows, w_uq, w_heads, dq_norm, dkv_norm, cache, meta: 
         span = meta.block_tables_d.shape[1] * cache.shape[1]
         ops.latent_attention_decode(qa[Tp:Tp + Bd], cache, meta.block_tables_d, meta.ctx_lens_d, spec.window, spec.scale, None, rp,
                                     lat[Tp:Tp + Bd], splits=ops.latent_decode_splits(Bd, H, min(span, spec.window)), gate=gate[Tp:Tp + Bd])
-    ops.head_linear(lat.view(T, 2 * H * rp), w_heads[1], 2 * rp, out.view(T, H, spec.vdim_p), parts=2)
+    ops.head_linear(lat.view(T, parts * H * rp), w_heads[1], parts * rp, out.view(T, H, spec.vdim_p), parts=parts)
     return out
 
 

@@ -202,3 +202,17 @@ def test_head_products_of_many_columns():
     ops.head_linear(x, w, K, out)
     want = x.double() @ w[0].double().T
     assert bool(((out[:, 0].double() - want).abs() <= 2 ** -8 * want.abs() + 1e-5).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kv_rank", [128, 100])
+def test_weights_of_another_model(kv_rank):
+    """A model that took another's weights by ``load_state_dict`` attends with them: the projections by head follow."""
+    mx = mixer(16, 50, 10, 40, 32, kv_rank, 33)
+    h = q16(rnd(torch.Generator().manual_seed(3), 40, 64))
+    a, _ = one_layer("latent_attention", mx, 64, "cuda", torch.bfloat16, seed=5)
+    b, _ = one_layer("latent_attention", mx, 64, "cuda", torch.bfloat16, seed=6)
+    assert a.layers[0].mix.spec.absorbed
+    b.load_state_dict(a.state_dict())
+    assert torch.equal(run_mixer(a, h, [30], "cuda", torch.bfloat16), run_mixer(b, h, [30], "cuda", torch.bfloat16))
+    assert (a.layers[0].mix.w_uv_h is None) == (kv_rank == 128)
