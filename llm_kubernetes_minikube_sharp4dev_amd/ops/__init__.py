@@ -1193,21 +1193,26 @@ def _cfg_of(M: int, N: int, K: int, epi: int):
 
 
 # Shapes without a measured entry, more than 256 rows: gemm1w.hip's 128 / 192 / 256-row tiles against the fallback.  Its
-# one wave of tiles costs 5 us + 0.6 / 0.78 / 1.0 us per 64 columns of K (past K 4096 1.33 / 1.2 / 1.0 of that) however few the
-# tiles are, and the output's stores 0.5 / 0.3 / 0.38 us per MB; gemm.hip's split-K with its reduction 19 + 8 f us and
-# 0.8 + 0.8 f us per 64 columns of a range (f: how much of the chip its workgroups fill), unsplit 8 us + 1.35 us per wave and
-# 64 columns.  Measured, weights cold, fallback / the rule's pick (us):
-#   2048 x 2048: M 640 27.8 / 24.3 (128-row tiles)   M 2048 40.4 / 25.6   M 4096 51.9 / 33.4      3072 x 1024: M 949 27.8 / 15.6
-#   2048 x 5632: M 949 48.1 / same   M 2048 63.0 / same (128-row: 75.5)   M 4096 98.2 / 83.0       3072 x 2048: M 4096 51.1 / 46.7
-#   11264 x 2048 SwiGLU: M 1500 91.6 / 78.1 (192-row tiles)   M 2900 144.8 / 123.3   M 4096 154.6 / same (256-row tiles)
-_TILE_COST = {5: (128, 0.6, 1.33, 0.5), 4: (192, 0.78, 1.2, 0.3), 3: (256, 1.0, 1.0, 0.38)}
+# waves of tiles cost 0.6 / 0.78 / 1.0 us per 64 columns of K each (128-row tiles from K 4096 on 1.1 of that) however few the tiles are, its
+# start and end 4 / 5.5 / 6.5 us (GELU 2 / 3.5 / 4.5 more), and the output's stores 0.5 / 0.3 / 0.38 us per MB; gemm.hip's split-K with its
+# reduction 16 + 8 f us and 0.8 + 0.8 f us per 64 columns of a range and 256 of N's tile (f: how much of the chip its workgroups
+# fill), unsplit 8 us + 1.35 us per wave and 64 columns.  Measured, weights cold, fallback / the rule's pick (us):
+#   3072 x 2048: M 320 26.5 / 27.2 (128-row tiles)   M 949 31.3 / 26.9   M 2048 41.5 / 29.9   M 2900 43.0 / 34.7 (192)   M 4096 47.8 / 46.3 (256)
+#   2048 x 5632: M 1500 52.7 / same (128-row: 72.4)   M 2900 77.1 / 74.8 (128)   M 4096 96.9 / 79.4
+#   1536 x 4096: M 1500 38.3 / same (128-row: 50.6)   M 2048 41.3 / same (51.8)   M 2900 54.4 / 51.1 (128)   M 4096 59.8 / 54.2
+#   3072 x 768 GELU: M 949 22.4 / 15.0 (128)   M 2048 23.6 / 17.0   M 2900 25.7 / 22.7 (192)   768 x 3072: M 2048 30.6 / same (34.8)
+#   11264 x 2048 SwiGLU: M 640 35.9 / 33.3 (128)   M 2048 99.7 / 81.6 (192)   M 2900 141.6 / 119.5   M 4096 156.9 / same (256)
+# Over those and eight more widths its picks are 0.4 % behind the best of the four on average, 8 % at most (768 x 3072 at M 4096).
+# v: (rows, start and end, per 64 columns, from K 4096 on, stores per MB, GELU)
+_TILE_COST = {5: (128, 4.0, 0.6, 1.1, 0.5, 2.0), 4: (192, 5.5, 0.78, 1.0, 0.3, 3.5), 3: (256, 6.5, 1.0, 1.0, 0.38, 4.5)}
 _TILE_RULE: dict = {}
 
 
 def _tile_rule(M: int, N: int, K: int, epi: int):
     d = _gemm_default(M, N, K, epi)
-    # (past the measured rows a launch is many waves of any tile, where the fallback's larger tiles lead: the encoder's
-    # 62,500-row batches ran 1.6 % longer on this rule's pick)
+    # (past the rows it was fitted on a launch is many waves, whose stores overlap and which this cost does not describe: the encoder's
+    # 62,500-row batches ran 1.6 % longer on its pick.  The fallback stays there, also at 4,608 - 8,192 rows, where the best tiles
+    # measured up to 1.5 times faster than it: 768 x 768 GELU at M 6500 22.9 / 15.1, 3072 x 2048 at M 5500 88.7 / 68.9)
     if not GEMM1W or not 256 < M <= 4608 or epi > 4 or K // 64 < 3 or N % 256 or d is None:
         return d
     key = (M, N, K, epi, d)
@@ -1216,22 +1221,23 @@ def _tile_rule(M: int, N: int, K: int, epi: int):
         out_mb = M * (N // 2 if epi == 1 else N) * 2 / 1e6
 
         def cost(v):
-            bm, c, deep, store = _TILE_COST[v]
+            bm, ends, c, deep, store, gelu = _TILE_COST[v]
             waves = -(-(-(-M // bm) * (N // 256)) // cus)
-            return 5 + waves * c * (deep if K > 4096 else 1.0) * steps + store * out_mb
+            return ends + (gelu if epi == 3 else 0) + waves * c * (deep if K >= 4096 else 1.0) * steps + store * out_mb
 
         if d[0] in _TILE_COST:
             other = cost(d[0])
         elif d[2] > 1:
             f = min(1.0, -(-M // 256) * (N // d[1]) * d[2] / cus)
-            other = 19 + 8 * f + (0.8 + 0.8 * f) * steps / d[2]
+            other = 16 + 8 * f + (0.8 + 0.8 * f) * d[1] / 256 * steps / d[2]
         else:
             cols = N // 256 if epi == 1 else N // d[1]
             other = 8 + 1.35 * steps * -(-(-(-M // 256) * cols) // cus)
         best = min(_TILE_COST, key=cost)
         if len(_TILE_RULE) > 4096:
             _TILE_RULE.clear()
-        _TILE_RULE[key] = (best, 256, 1) if cost(best) < 0.97 * other else d
+        # (between two of these tiles the pick has to be clear: 3 % of the estimate)
+        _TILE_RULE[key] = (best, 256, 1) if cost(best) < (0.97 if d[0] in _TILE_COST else 1.0) * other else d
     return _TILE_RULE[key]
 
 

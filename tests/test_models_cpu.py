@@ -406,6 +406,21 @@ def test_gemm1w_default_policy(monkeypatch):
     assert all(c[0] not in ops.GEMM1W_BM for c in ops._gemm_configs(4096, 0))
 
 
+@pytest.mark.parametrize("M,N,K,epi,pick", [
+    (1500, 1536, 4096, 0, None), (2048, 1536, 4096, 0, None), (2048, 768, 3072, 2, None), (2900, 768, 3072, 2, None), (1500, 2048, 5632, 0, None),
+    (2900, 1536, 4096, 0, 5), (949, 3072, 2048, 0, 5), (2048, 3072, 768, 3, 5), (2900, 2304, 768, 2, 5), (2900, 3072, 2048, 0, 4), (2048, 11264, 2048, 1, 4),
+    (4096, 3072, 2048, 0, 3), (4096, 11264, 2048, 1, None), (5500, 3072, 2048, 0, None)])
+def test_tile_rule_takes_what_measured_fastest(monkeypatch, M, N, K, epi, pick):
+    """Tiles of shapes without a measured entry, on both sides of the lines between split-K, the fallback and the three row tiles (None: the
+    fallback's own choice)."""
+    from llm_kubernetes_minikube_sharp4dev_amd import ops
+
+    monkeypatch.setattr(ops, "GEMM1W", True)
+    monkeypatch.setattr(ops, "_CUS", 256)
+    monkeypatch.setattr(ops, "_TILE_RULE", {})
+    assert ops._tile_rule(M, N, K, epi) == (ops._gemm_default(M, N, K, epi) if pick is None else (pick, 256, 1))
+
+
 def test_few_row_rule_counts_the_devices_cus(monkeypatch):
     """The few-row kernel's rounds are of the device's CUs: what it wins on a whole chip (128 workgroups in half a round) it loses on a
     partition of 32 CUs, where they are four rounds."""
