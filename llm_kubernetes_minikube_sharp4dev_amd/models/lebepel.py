@@ -44,6 +44,14 @@ from .ssm import Mamba2Spec, mamba2_mixer
 FUSE_QKV_BIAS = True
 
 
+def _pad_in_proj(layer, sd, prefix, *_):
+    """A state dict whose ``in_proj`` is padded to whole 128s of rows loads into a model that pads to 256s."""
+    key = prefix + "in_proj"
+    w = sd.get(key)
+    if w is not None and w.dim() == 2 and w.shape[0] == -(-layer.spec.proj_out // 128) * 128:
+        sd[key] = torch.nn.functional.pad(w, (0, 0, 0, layer.in_proj.shape[0] - w.shape[0]))
+
+
 class LebepelLayer(nn.Module):
     def __init__(self, cfg: LebepelConfig, spec, dtype, device):
         super().__init__()
@@ -69,6 +77,7 @@ class LebepelLayer(nn.Module):
             # 184 -> 150 us at 4,096 x 2,048), else to the decode GEMMs' 128
             r128 = -(-s.proj_out // 128) * 128
             self.in_proj = P(-(-r128 // 256) * 256 if r128 >= 4096 else r128, W, **e)
+            self.register_load_state_dict_pre_hook(_pad_in_proj)
             self.conv_w, self.conv_b = P(s.conv_channels, s.conv, **f), P(s.conv_channels, **f)
             self.dt_bias, self.A_log, self.D = P(s.heads, **f), P(s.heads, **f), P(s.heads, **f)
             self.mix_norm = P(s.inner, **f)

@@ -353,3 +353,19 @@ def test_pipelined_generation_on_captured_graphs():
         for i, tid in enumerate(sq.output_ids):
             gap = float(lg[i].max() - lg[i, tid])
             assert gap <= 0.25 * float(lg[i].max() - lg[i].min()), (i, gap)
+
+
+def test_state_dict_with_fewer_padding_rows():
+    """``in_proj`` of 4,144 rows is kept in 4,352; a state dict that pads it to 4,224 loads all the same, other sizes are refused."""
+    cfg = LebepelConfig.from_json(config([ff(ssm(16, 128, 16, 1, 4, 1), 32)], 64))
+    a, b = LebepelModel(cfg).random_init(1), LebepelModel(cfg).random_init(2)
+    sd = a.state_dict()
+    assert sd["layers.0.in_proj"].shape[0] == 4352
+    sd["layers.0.in_proj"] = sd["layers.0.in_proj"][:4224].clone()
+    b.load_state_dict(sd)
+    assert sd["layers.0.in_proj"].shape[0] == 4224
+    for k, v in a.state_dict().items():
+        assert torch.equal(v, b.state_dict()[k]), k
+    for rows in (4100, 4144, 4351):
+        with pytest.raises(RuntimeError):
+            b.load_state_dict({**sd, "layers.0.in_proj": a.layers[0].in_proj[:rows]})
