@@ -29,7 +29,7 @@ int lk_silu_mul(bf16_t* out, const bf16_t* x, long rows, int I, long xs, long os
 int lk_activation(bf16_t* x, const bf16_t* bias, long rows, int N, long xs, int kind,
                   hipStream_t st);
 
-// rows_gemm.hip (M <= 64, one launch, every epilogue)
+// rows_gemm.hip (few rows, up to 4,096; one launch, every epilogue)
 bool lk_rows_gemm_supported(int M, int N, int K, int epi);
 int lk_rows_gemm(const void* x, const void* w, const void* b, void* y, int M, int N, int K, long ldx, long ldy, int epi, int wide,
                  hipStream_t st);

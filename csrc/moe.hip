@@ -421,7 +421,9 @@ int moe_gemm_t(const void* x, long xs, const int* order, const int* seg, int E, 
   }
   if constexpr (sizeof(T) == 2) {
     // whole 64-column stages and 16-column blocks, 8-byte stores; rows per walk by the pairs an expert has on average (a third
-    // more than the mean keeps a second walk rare)
+    // more than the mean keeps a second walk rare).  A skewed table's further walks come one after the other, out of caches: both
+    // products of 64 tokens, 12 pairs in the fullest of 16 experts / 40 / 64 in each of two: 93 / 109 / 85 us (tiles of 16 pairs over
+    // the chip, moe_gemm_kernel: 183 / 195 / 92); of 300 tokens, 46 / 173 / 300: 148 / 179 / 138 us (329 / 324 / 268).
     if (vec && K % 64 == 0 && N % 32 == 0 && os % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0 && (long)E * (N / 32) <= 2147483647L) {
       const long avg = pairs / E;
 #define LK_MOE_ROWS(MT)                                                                           \

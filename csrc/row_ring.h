@@ -1,6 +1,6 @@
 // The K walk of the few-row products: a wave multiplies MT x 16 rows of X by NT x 16 rows of W over its own range of K,
 // both streamed through a private LDS ring by 16-byte LDS-DMA (8 rows x one whole 128-byte line per instruction), counted
-// vmcnt, no barrier.  The four waves of a workgroup split K; row_sums() joins them.
+// vmcnt, no barrier.  The four waves of a workgroup split K; rg_sums() joins them.
 #pragma once
 #include "common.h"
 
