@@ -395,6 +395,9 @@ def _decode_bucket(M: int) -> Optional[int]:
 #    64 x 10368 x 2048 17.9 / 16.7    128 x 4096 x 4096 15.7 / 18.4    192 x 4096 x 4096 28.6 / 20.9
 #    64 x 11264 x 2048 (SwiGLU) 18.3 / 19.6             512 x 2048 x 5632 38.6 / 43.9    768: 57.8 / 45.1
 #   bias:  19 x  768 x  768  3.5 / 15.6    512 x 2304 x 768 12.1 / 19.7    768 x 3072 x 768 18.6 / 23.5    2048: 48 / 24.7
+# Widths that neither tiles (N no multiple of 192 or 256) go to the vendor's kernels, which split K for narrow outputs: fitted to
+# within 25 % for N 48 - 11,280, K 256 - 8,192, 17 - 1,024 rows, and taken 10 % lower, since an even choice is worth nothing (few-row / vendor):
+#    64 x  400 x 1024  4.2 / 6.7      64 x 2064 x 1024  5.5 / 8.8     512 x   48 x 8192 24.9 / 9.1     400 x 2064 x 1024 17.4 / 9.4
 # (past K 8192 more than 16 rows of X do not stay in L2.)  Where the streaming kernel's sum rides in its consumer
 # (linear_add_rmsnorm, linear_rope_kv) the two are level at decode sizes, and those stay as they are.
 ROWS_MAX_M = 1024
@@ -429,6 +432,10 @@ def _rows_cost(M: int, N: int, K: int, epi: int):
             other = min(20 + K / 256, 4 + K / 64)
         else:
             other = min(17 + 3 * K / 1024, 6 + K / 64)
+        tiled = N % 256 == 0 or (epi != 1 and N % 192 == 0)
+        if not tiled and not (epi < 2 and rows <= 256 and _decode_static_ok(N, K, epi == 1)):
+            vendor = 5.2 + K / 2048 + 3.1e-9 * rows * N * K + 0.19 * mb + 2.8e-7 * rows * (N + K) + (0 if epi in (0, 2) else 2.7)
+            other = min(other, 0.9 * vendor)
         est = (t, wide, other)
     _ROWS_RULE[key] = est
     return est

@@ -435,6 +435,21 @@ def test_few_row_rule_counts_the_devices_cus(monkeypatch):
         assert ops._rows_rule(64, 2048, 2048, 0) is pick
 
 
+@pytest.mark.parametrize("M,N,K,epi,rows", [(512, 48, 8192, 0, False), (128, 96, 8192, 2, False), (400, 2064, 1024, 0, False),
+                                            (400, 2064, 1024, 3, False), (512, 96, 8192, 1, False), (64, 2064, 1024, 0, True),
+                                            (64, 400, 1024, 0, True), (192, 48, 256, 2, True), (512, 48, 256, 3, True)])
+def test_few_row_rule_where_no_tile_takes_the_width(monkeypatch, M, N, K, epi, rows):
+    """Widths that go to the vendor's kernels otherwise: those are the other side of the comparison, not the tiles."""
+    from types import SimpleNamespace
+
+    from llm_kubernetes_minikube_sharp4dev_amd import ops
+
+    monkeypatch.setattr(ops, "lib", lambda: SimpleNamespace(rows_supported=lambda *a: True))
+    monkeypatch.setattr(ops, "_CUS", 256)
+    monkeypatch.setattr(ops, "_ROWS_RULE", {})
+    assert (ops._rows_rule(M, N, K, epi) is not None) == rows
+
+
 def test_static_gemm_table_is_well_formed(monkeypatch):
     """The shipped measured dispatch table (benchmarks/gemm_table.py on an MI355X): every entry a
     kernel / tile / split the dispatch knows, looked up by _cfg_of before the fallback policy,
