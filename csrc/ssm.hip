@@ -981,6 +981,8 @@ __global__ __launch_bounds__(256) void gated_group_rmsnorm_wave_kernel(const flo
 // prompt portions (some sequence of the step has >= kChunkMin rows): the chunked MFMA kernel, for the step's other sequences too.  What
 // decides in short portions and decode rows is the pass over the state, so the 64-token chunks lead there as well; us, chunks of 16 ->
 // of 64, 64 heads of [64, 128]: 512 rows and 64 decode rows 322 -> 212, 8 and 64 177 -> 157, 64 portions of 8 170 -> 153, one of 8 14.4 -> 11.4.
+// With up to 32 state columns that pass is short and a chunk's own work decides: there portions of up to 16 tokens stay with chunks of 16
+// (16 heads of [128, 16]: 32 portions of 16 10.3 against 15.0, 8 and 64 decode rows 17.4 / 24.8; 17 tokens 7.5 / 7.1).
 constexpr int kChunkMin = 8;
 
 template <typename T>
@@ -992,7 +994,7 @@ int scan_t(const T* xbc, long xs, const T* dtp, long dts, int S, int heads, int 
     if constexpr (sizeof(T) == 2) {
       // 16-byte loads of B, C and the state's rows, 8-byte ones of x, 16-byte stores of y
       const auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-      if (N % 8 == 0 && N <= 256 && P % 4 == 0 && ((long)heads * P) % 8 == 0 && xs % 8 == 0 && ys % 4 == 0 && a16(xbc) && a16(state) && a16(y)) {
+      if (!(N <= 32 && max_len <= 16) && N % 8 == 0 && N <= 256 && P % 4 == 0 && ((long)heads * P) % 8 == 0 && xs % 8 == 0 && ys % 4 == 0 && a16(xbc) && a16(state) && a16(y)) {
 #define LK_CHUNK64(NR)                                                                                                             \
   do {                                                                                                                             \
     LK_SET_MAX_LDS((ssm_chunk_bf16_kernel<NR>), (ssm_chunk_lds<NR>()));                                                            \
@@ -1026,11 +1028,21 @@ int scan_t(const T* xbc, long xs, const T* dtp, long dts, int S, int heads, int 
 #define LK_STEP(LPR, RB)                                                                                                  \
   ssm_step_kernel<T, LPR, RB><<<sgrid, 256, 0, st>>>(xbc, xs, dtp, dts, heads, P, N, groups, dt_bias, A_log, D, state, cu, \
                                                      slots, positions, y, ys)
-    if (N <= 16) LK_STEP(4, 4);
-    else if (N <= 32) LK_STEP(8, 8);
-    else if (N <= 64) LK_STEP(16, 8);
-    else if (N <= 128) LK_STEP(32, 8);
-    else LK_STEP(64, 8);
+    // rows per lane group of a pass: 8, or what gives all four waves a part of P.  One sequence, 32 heads of [64, 32] / [64, 64]:
+    // 5.2 / 5.5 us with 8 (one and two of the four waves at work) -> 3.6 / 4.3; 16 sequences 6.1 / 7.1 -> 4.5 / 5.9
+#define LK_STEPS(LPR)                                       \
+  do {                                                      \
+    if (P * LPR > 1024) LK_STEP(LPR, (LPR > 4 ? 8 : 4));    \
+    else if (P * LPR > 512) LK_STEP(LPR, 4);                \
+    else if (P * LPR > 256) LK_STEP(LPR, 2);                \
+    else LK_STEP(LPR, 1);                                   \
+  } while (0)
+    if (N <= 16) LK_STEPS(4);
+    else if (N <= 32) LK_STEPS(8);
+    else if (N <= 64) LK_STEPS(16);
+    else if (N <= 128) LK_STEPS(32);
+    else LK_STEPS(64);
+#undef LK_STEPS
 #undef LK_STEP
     LK_CHECK_LAUNCH();
     return 0;

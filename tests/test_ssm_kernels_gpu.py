@@ -51,6 +51,24 @@ def test_scan(hip, H, P, N, G, lens, max_len, dtype):
     assert (state.double() - want).norm() <= 1e-6 * want.norm()
 
 
+@pytest.mark.parametrize("P,N", [(100, 16), (160, 16), (31, 28), (96, 32), (136, 32), (24, 64), (40, 40), (129, 64), (5, 128), (12, 128),
+                                 (3, 256), (6, 256), (64, 64), (64, 32)])
+def test_step_rows_per_lane_group(hip, P, N):
+    """Single tokens where a pass takes 1, 2, 4 or 8 rows per lane group, P whole passes and not."""
+    y, ref, state, want = _run([1, 1, 1], 3, P, N, 1, torch.bfloat16, 1, 5)
+    assert (y.double() - ref).norm() <= 1e-6 * ref.norm()   # as above
+    assert (state.double() - want).norm() <= 1e-6 * want.norm()
+
+
+@pytest.mark.parametrize("lens,max_len", [([16, 9, 1, 8], 16), ([17, 1, 8], 17)])
+@pytest.mark.parametrize("P,N", [(128, 16), (64, 32), (20, 24), (64, 40)])
+def test_short_portions(hip, P, N, lens, max_len):
+    """Portions of up to 16 tokens and one more, with few state columns (chunks of 16 tokens, of 64 behind the line) and more."""
+    y, ref, state, want = _run(lens, 4, P, N, 2, torch.bfloat16, max_len, 5)
+    assert (y.double() - ref).norm() <= 1e-6 * ref.norm()
+    assert (state.double() - want).norm() <= 1e-6 * want.norm()
+
+
 @pytest.mark.parametrize("rows,inner,ng", [(1, 4096, 8), (77, 1536, 1), (5, 120, 3), (9, 2048, 1), (3, 2304, 1), (6, 44, 2)])
 def test_gated_group_norm(hip, rows, inner, ng):
     torch.manual_seed(inner)
