@@ -27,9 +27,23 @@ constexpr int kMaxExperts = 1024;
 
 // One workgroup; its time is the chain of dependent loads (token id, then table), so a thread requests the ids of all its pairs and then
 // all their table entries, kRouteU at a time, and keeps the experts in registers for the second pass where they fit (8,192 pairs).
-// 8,192 pairs of 16 experts: one pair after the other, twice, 18.7 us, now 14.6 (the rest are the counters' atomics).
+// 8,192 pairs of 16 experts: one pair after the other, twice, 18.7 us, now 14.6 (the rest are the counters' atomics).  Up to 1,024 pairs
+// take the form of one pair per thread (U = 1: eight divisions by top cost a decode step more than its loads:
+// 64 tokens x 2 of 16 experts 4.3 -> 2.0 us).
 constexpr int kRouteU = 8;
 
+// inclusive sums over the wave's lanes
+LK_DEVICE int wave_sums(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr 1, 2, 4, 8: inside 16 lanes
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast 15 to the second and fourth 16
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast 31 to the upper half
+  return v;
+}
+
+template <int U>
 __global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(const int* __restrict__ ids, const int* __restrict__ table, int vocab,
                                                                   int top, int E, int T, int* __restrict__ seg,
                                                                   int* __restrict__ order) {
@@ -38,26 +52,31 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(const int* __r
   const int n = T * top, tid = threadIdx.x;
   for (int e = tid; e < E; e += kRouteThreads) cnt[e] = 0;
   __syncthreads();
-  int ex[kRouteU];
+  int ex[U];
   auto experts = [&](int p0) {   // of pairs p0 + tid + 1024 u (behind the end: the last pair's)
-    int id[kRouteU];
+    int id[U], at[U];
 #pragma unroll
-    for (int u = 0; u < kRouteU; ++u) {
-      const int t = (int)min((long)p0 + u * kRouteThreads + tid, (long)n - 1) / top;
+    for (int u = 0; u < U; ++u) {
+      if ((long)p0 + u * kRouteThreads >= n) break;   // (no division for pairs that are not there)
+      const int p = (int)min((long)p0 + u * kRouteThreads + tid, (long)n - 1), t = p / top;
+      at[u] = p - t * top;
       id[u] = ids ? ids[t] : t;                 // no ids: the table has one row per token of the step
     }
 #pragma unroll
-    for (int u = 0; u < kRouteU; ++u) {
-      const int p = (int)min((long)p0 + u * kRouteThreads + tid, (long)n - 1);
-      ex[u] = table[(long)min(max(id[u], 0), vocab - 1) * top + p % top];
+    for (int u = 0; u < U; ++u) {
+      if ((long)p0 + u * kRouteThreads >= n) break;
+      ex[u] = table[(long)min(max(id[u], 0), vocab - 1) * top + at[u]];
     }
 #pragma unroll
-    for (int u = 0; u < kRouteU; ++u) ex[u] = min(max(ex[u], 0), E - 1);
+    for (int u = 0; u < U; ++u) {
+      if ((long)p0 + u * kRouteThreads >= n) break;
+      ex[u] = min(max(ex[u], 0), E - 1);
+    }
   };
-  for (long p0 = 0; p0 < n; p0 += kRouteU * kRouteThreads) {
+  for (long p0 = 0; p0 < n; p0 += U * kRouteThreads) {
     experts((int)p0);
 #pragma unroll
-    for (int u = 0; u < kRouteU; ++u)
+    for (int u = 0; u < U; ++u)
       if (p0 + u * kRouteThreads + tid < n) atomicAdd(&cnt[ex[u]], 1);
   }
   __syncthreads();
@@ -65,22 +84,17 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(const int* __r
     int acc = 0;
     for (int e0 = 0; e0 < E; e0 += 64) {
       const int c = e0 + tid < E ? cnt[e0 + tid] : 0;
-      int v = c;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int below = __shfl_up(v, o, 64);
-        if (tid >= o) v += below;
-      }
+      const int v = wave_sums(c);
       if (e0 + tid < E) seg[e0 + tid] = nxt[e0 + tid] = acc + v - c;
-      acc += __shfl(v, 63, 64);
+      acc += __builtin_amdgcn_readlane(v, 63);
     }
     if (tid == 0) seg[E] = acc;
   }
   __syncthreads();
-  for (long p0 = 0; p0 < n; p0 += kRouteU * kRouteThreads) {
-    if (n > kRouteU * kRouteThreads) experts((int)p0);
+  for (long p0 = 0; p0 < n; p0 += U * kRouteThreads) {
+    if (n > U * kRouteThreads) experts((int)p0);
 #pragma unroll
-    for (int u = 0; u < kRouteU; ++u) {
+    for (int u = 0; u < U; ++u) {
       const long p = p0 + u * kRouteThreads + tid;
       if (p < n) order[atomicAdd(&nxt[ex[u]], 1)] = (int)p;
     }
@@ -444,7 +458,8 @@ int moe_gemm_t(const void* x, long xs, const int* order, const int* seg, int E, 
 int lk_moe_route(const int* ids, const int* table, int vocab, int top, int E, int T, int* seg, int* order, hipStream_t st) {
   if (T <= 0) return 0;
   if (E < 1 || E > kMaxExperts || top < 1 || vocab < 1) return -1;
-  moe_route_kernel<<<1, kRouteThreads, 0, st>>>(ids, table, vocab, top, E, T, seg, order);
+  if ((long)T * top <= kRouteThreads) moe_route_kernel<1><<<1, kRouteThreads, 0, st>>>(ids, table, vocab, top, E, T, seg, order);
+  else moe_route_kernel<kRouteU><<<1, kRouteThreads, 0, st>>>(ids, table, vocab, top, E, T, seg, order);
   LK_CHECK_LAUNCH();
   return 0;
 }

@@ -49,7 +49,9 @@ def test_rows_per_expert(counts, swiglu, N, K):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("T,top,E,by_id", [(1, 1, 1, True), (4096, 2, 16, True), (4097, 2, 16, True), (3000, 3, 200, False), (20000, 2, 1024, True), (5, 8, 65, False)])
+@pytest.mark.parametrize("T,top,E,by_id", [(1, 1, 1, True), (4096, 2, 16, True), (4097, 2, 16, True), (3000, 3, 200, False), (20000, 2, 1024, True), (5, 8, 65, False),
+                                             (1024, 1, 64, True), (341, 3, 128, False), (1025, 1, 7, False), (512, 2, 63, True),
+                                             (8192, 1, 129, True)])
 def test_pairs_sorted_by_expert(T, top, E, by_id):
     g = torch.Generator().manual_seed(T)
     vocab = 50 if by_id else T
