@@ -1211,7 +1211,9 @@ def _cfg_of(M: int, N: int, K: int, epi: int):
 #   1536 x 4096: M 1500 38.3 / same (128-row: 50.6)   M 2048 41.3 / same (51.8)   M 2900 54.4 / 51.1 (128)   M 4096 59.8 / 54.2
 #   3072 x 768 GELU: M 949 22.4 / 15.0 (128)   M 2048 23.6 / 17.0   M 2900 25.7 / 22.7 (192)   768 x 3072: M 2048 30.6 / same (34.8)
 #   11264 x 2048 SwiGLU: M 640 35.9 / 33.3 (128)   M 2048 99.7 / 81.6 (192)   M 2900 141.6 / 119.5   M 4096 156.9 / same (256)
-# Over those and eight more widths its picks are 0.4 % behind the best of the four on average, 8 % at most (768 x 3072 at M 4096).
+#   8192 x 14336: M 640 159 / same (128-row: 195)   7168 x 6144: M 640 69.6 / same (87.4)   11264 x 512 GELU: M 2500 41.7 / 50.1 (192)
+# Over 132 widths (N 768 - 11,264, K 512 - 14,336) at 12 row counts with three epilogues it takes 0.861 of the fallback's time, and 0.8 % more than
+# the best of the four; 18 of the 4,752 picks are more than 8 % slower than the fallback, 20 % at most (the last shape above).
 # v: (rows, start and end, per 64 columns, from K 4096 on, stores per MB, GELU)
 _TILE_COST = {5: (128, 4.0, 0.6, 1.1, 0.5, 2.0), 4: (192, 5.5, 0.78, 1.0, 0.3, 3.5), 3: (256, 6.5, 1.0, 1.0, 0.38, 4.5)}
 _TILE_RULE: dict = {}
@@ -1245,8 +1247,13 @@ def _tile_rule(M: int, N: int, K: int, epi: int):
         best = min(_TILE_COST, key=cost)
         if len(_TILE_RULE) > 4096:
             _TILE_RULE.clear()
-        # (between two of these tiles the pick has to be clear: 3 % of the estimate)
-        _TILE_RULE[key] = (best, 256, 1) if cost(best) < (0.97 if d[0] in _TILE_COST else 1.0) * other else d
+        # (the pick has to be clear where the estimates are least sure: between two of these tiles 3 % of them, at K up to 1,024 7 %, and
+        # against split-K 20 % from K 5,632 on, where 100 - 200 tiles of deep K run up to a quarter longer than estimated)
+        if d[0] in _TILE_COST:
+            clear = 0.93 if K <= 1024 else 0.97
+        else:
+            clear = 0.8 if d[2] > 1 and K >= 5632 else 1.0
+        _TILE_RULE[key] = (best, 256, 1) if cost(best) < clear * other else d
     return _TILE_RULE[key]
 
 

@@ -409,7 +409,7 @@ def test_gemm1w_default_policy(monkeypatch):
 @pytest.mark.parametrize("M,N,K,epi,pick", [
     (1500, 1536, 4096, 0, None), (2048, 1536, 4096, 0, None), (2048, 768, 3072, 2, None), (2900, 768, 3072, 2, None), (1500, 2048, 5632, 0, None),
     (2900, 1536, 4096, 0, 5), (949, 3072, 2048, 0, 5), (2048, 3072, 768, 3, 5), (2900, 2304, 768, 2, 5), (2900, 3072, 2048, 0, 4), (2048, 11264, 2048, 1, 4),
-    (4096, 3072, 2048, 0, 3), (4096, 11264, 2048, 1, None), (5500, 3072, 2048, 0, None)])
+    (4096, 3072, 2048, 0, 3), (4096, 11264, 2048, 1, None), (5500, 3072, 2048, 0, None), (640, 8192, 14336, 0, None), (640, 7168, 6144, 0, None)])
 def test_tile_rule_takes_what_measured_fastest(monkeypatch, M, N, K, epi, pick):
     """Tiles of shapes without a measured entry, on both sides of the lines between split-K, the fallback and the three row tiles (None: the
     fallback's own choice)."""
