@@ -441,12 +441,47 @@ __global__ __launch_bounds__(256) void lat_decode_kernel(LatParams p, const int*
 
 // One workgroup per (sequence, head), four columns per thread.  A chain of three waits (maxima, sums, averages): the splits' maxima and
 // sums are read by the lanes side by side and the averages four splits at a time; one split after the other it took 6.5 us at 64 x 16
-// rows of 512 columns in 4 splits, 4.7 side by side.
+// rows of 512 columns in 4 splits, 4.7 side by side.  Up to four splits every thread takes them all, requested together: the lanes' sums
+// cost a step of few splits more than they save (whole decode attention, 64 x 32 rows of 256 columns in 2 splits of 512 keys: 13.8 -> 12.9).
+constexpr int kLatFew = 4;
+
 __global__ __launch_bounds__(256) void lat_reduce_kernel(LatParams p, const float* __restrict__ part, int Z) {
   const int b = blockIdx.x, head = blockIdx.y, RP = p.RP, lane = threadIdx.x & 63;
   const float* pp = part + ((long)b * p.H + head) * Z * (RP + 2);
   const float gate = lat_gate<bf16_t>(p, b, head);
+  bf16_t* const orow = reinterpret_cast<bf16_t*>(p.out) + (long)b * p.os + (long)head * p.OH;
   float M = kNegBig, L = 0.f;
+  if (Z <= kLatFew) {
+    float e[kLatFew], l[kLatFew];
+#pragma unroll
+    for (int z = 0; z < kLatFew; ++z) {
+      e[z] = z < Z ? pp[(long)z * (RP + 2) + RP] : kNegBig;
+      l[z] = z < Z ? pp[(long)z * (RP + 2) + RP + 1] : 0.f;
+    }
+#pragma unroll
+    for (int z = 0; z < kLatFew; ++z) M = fmaxf(M, e[z]);
+#pragma unroll
+    for (int z = 0; z < kLatFew; ++z) {
+      e[z] = __builtin_amdgcn_exp2f(e[z] - M);
+      if (z < Z) L += l[z] * e[z];
+    }
+    const float inv = L > 0.f ? gate / L : 0.f;
+    for (int d = 4 * threadIdx.x; d < RP; d += 1024) {
+      float s[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int z = 0; z < kLatFew; ++z) {
+        if (z >= Z) break;
+        const float* q = pp + (long)z * (RP + 2) + d;   // (a row is RP + 2 long: 8-byte loads)
+        const float2 v = *reinterpret_cast<const float2*>(q), w = *reinterpret_cast<const float2*>(q + 2);
+        s[0] += v.x * e[z];
+        s[1] += v.y * e[z];
+        s[2] += w.x * e[z];
+        s[3] += w.y * e[z];
+      }
+      store_avg(p, orow + d, {s[0] * inv, s[1] * inv, s[2] * inv, s[3] * inv});
+    }
+    return;
+  }
   for (int z = lane; z < Z; z += 64) M = fmaxf(M, pp[(long)z * (RP + 2) + RP]);
   M = wave_max(M);
   for (int z = lane; z < Z; z += 64) L += pp[(long)z * (RP + 2) + RP + 1] * __builtin_amdgcn_exp2f(pp[(long)z * (RP + 2) + RP] - M);
@@ -456,7 +491,7 @@ __global__ __launch_bounds__(256) void lat_reduce_kernel(LatParams p, const floa
     float s[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
     for (int z = 0; z < Z; ++z) {
-      const float* q = pp + (long)z * (RP + 2);   // (a row is RP + 2 long: 8-byte loads)
+      const float* q = pp + (long)z * (RP + 2);
       const float2 v = *reinterpret_cast<const float2*>(q + d), w = *reinterpret_cast<const float2*>(q + d + 2);
       const float e = __builtin_amdgcn_exp2f(q[RP] - M);
       s[0] += v.x * e;
@@ -464,7 +499,7 @@ __global__ __launch_bounds__(256) void lat_reduce_kernel(LatParams p, const floa
       s[2] += w.x * e;
       s[3] += w.y * e;
     }
-    store_avg(p, reinterpret_cast<bf16_t*>(p.out) + (long)b * p.os + (long)head * p.OH + d, {s[0] * inv, s[1] * inv, s[2] * inv, s[3] * inv});
+    store_avg(p, orow + d, {s[0] * inv, s[1] * inv, s[2] * inv, s[3] * inv});
   }
 }
 
