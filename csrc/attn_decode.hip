@@ -14,6 +14,8 @@
 //  combines (flash-decoding).  The grid is sized for the *maximum* context so the
 //  launch shape is static and the whole step can be captured in a hipGraph;
 //  splits beyond a sequence's length exit immediately.
+#include <type_traits>
+
 #include "common.h"
 #include "kernels.h"
 
@@ -62,18 +64,24 @@ LK_DEVICE void merge_splits(int b, int qh, int d, int Hq, int max_splits, int ns
 //         XOR-swizzled LDS image of the chunk.
 // The 4 waves' (m, l, O) are merged through LDS at the end; splits > 1 emit
 // partials for lk_decode_reduce (flash-decoding).
-// NT: the cache is read non-temporally, for batches whose sequences share no block (a step then reads every key once, and its weights
-// and other layers pass through the caches before the next).  Rows that share blocks read them from L2 instead, which the hint would
-// give up.  8 kv heads of 128, plain -> non-temporal, us: 120 sequences of 950 own keys 85.5 -> 79.4, 32: 30.7 -> 28.8, 120 of 400: 42.4 -> 39.5;
-// 700 of 950 keys shared by 8: 54.9 -> 60.4, by 2: 62.5 -> 71.0; 64 of 3,000 with 2,800 shared by 4: 83 -> 112.
-template <int D, int G, bool NT>
+// READ_ONCE: keys and values are read non-temporally, for batches whose sequences share no block (a step then reads every key once, and
+// its weights and other layers pass through the caches before the next).  Rows that share a block read it from L2 instead, which
+// the hint would give up, so with prefix reuse (READ_SHARED) every split looks whether its rows are shared: plain loads from a third of
+// its keys on, where the two are level.  Behind a pass over 768 MB, 8 kv heads of 128, plain / non-temporal / by the look, us: 120 sequences of 950
+// own keys 89.9 / 85.3 / 85.9, 250 of them shared by all 76.5 / 75.8 / 76.7, 700 shared by 8 58.1 / 75.0 / 59.8, by 2 69.0 / 79.6 / 70.4;
+// 64 of 3,000 with 2,800 shared by 4 86.3 / 118.1 / 88.1; 240 of 950 172 / 161 / 162.  The look costs 0.5 us, which steps of few rows do
+// not get back (2 rows of 950 keys 13.4 / 13.9 / 14.3, 8 rows 16.2 / 16.3 / 16.7): READ_PLAIN below kShareRows.
+enum { READ_PLAIN = 0, READ_ONCE = 1, READ_SHARED = 2 };
+constexpr int kShareRows = 16;
+
+template <int D, int G, int READ>
 __global__ __launch_bounds__(256, LK_DECODE_WG_PER_CU) void paged_decode_kernel(
     const bf16_t* __restrict__ q, long qs, const bf16_t* __restrict__ kc,
     const bf16_t* __restrict__ vc, const int* __restrict__ block_tables, int bt_stride,
     const int* __restrict__ ctx_lens, bf16_t* __restrict__ out, long os,
     float* __restrict__ part_o, float* __restrict__ part_ml, int Hkv, int BS, int max_splits,
     int split, float scale_log2, const int* __restrict__ k_start, int has_prefix,
-    const float* __restrict__ pp_o, const float* __restrict__ pp_ml, int* __restrict__ tickets) {
+    const float* __restrict__ pp_o, const float* __restrict__ pp_ml, int* __restrict__ tickets, int rows) {
   constexpr int KK = D / 32;     // QK k-steps (16x16x32)
   constexpr int ND = D / 16;     // PV output tiles of 16 d
   constexpr int CPR = D / 8;     // 16-B chunks per V row
@@ -111,7 +119,17 @@ __global__ __launch_bounds__(256, LK_DECODE_WG_PER_CU) void paged_decode_kernel(
     blk[i] = block_tables[(long)b * bt_stride + k_begin / BS + i];
     LK_DASSERT(blk[i] >= 0);
   }
-  __syncthreads();
+  // is a third of the split's keys or more in blocks that some other row's table holds too?  (shared blocks are prefixes: they lie at
+  // the same place of both tables, so one place tells; a thread looks at one row)
+  bool shared = READ == READ_PLAIN;
+  if constexpr (READ == READ_SHARED) {
+    const int* col = block_tables + k_begin / BS + nblk / 3;
+    const int mine = col[(long)b * bt_stride];
+    for (int r = threadIdx.x; r < rows; r += 256) shared |= r != b && col[(long)r * bt_stride] == mine;
+    shared = __syncthreads_or(shared);
+  } else {
+    __syncthreads();
+  }
 
   // A wave's 16 K rows (16t + r16) and the 4 V rows of one load (i * RPL + lane / CPR) lie in
   // one cache block (BS >= 16, splits and chunks block-aligned: checked on the host), so the
@@ -136,9 +154,10 @@ __global__ __launch_bounds__(256, LK_DECODE_WG_PER_CU) void paged_decode_kernel(
   short8 kr[2][KK], vr[NVL];
   // k_begin is block-aligned (split % BS == 0, k_start a multiple of BS): row rel of the
   // split sits at slot rel % BS of its block
-  auto ld = [](const bf16_t* p) { return NT ? __builtin_nontemporal_load(reinterpret_cast<const short8*>(p)) : *reinterpret_cast<const short8*>(p); };
-  auto load_chunk = [&](int c, short8 (&kd)[2][KK], short8 (&vd)[NVL]) {
+  auto load_chunk = [&](auto nt_t, int c, short8 (&kd)[2][KK], short8 (&vd)[NVL]) {
     const int base = 32 * c;
+    constexpr bool NT = decltype(nt_t)::value;
+    auto ld = [](const bf16_t* p) { return NT ? __builtin_nontemporal_load(reinterpret_cast<const short8*>(p)) : *reinterpret_cast<const short8*>(p); };
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       const bf16_t* kp = blk_base(kc, base + 16 * t) + (min(base + 16 * t + r16, nkeys - 1) % BS) * D + 8 * h4;
@@ -158,76 +177,85 @@ __global__ __launch_bounds__(256, LK_DECODE_WG_PER_CU) void paged_decode_kernel(
   float m_run = -INFINITY, l_run = 0.f;
   bf16_t* vw = vlds[w];
 
-  int c = w;
-  if (c < nch) load_chunk(c, kr, vr);
-  for (; c < nch; c += 4) {
-    // stage this chunk's V into the wave-private LDS image (row-major, 16-B chunk
-    // index XOR ((row & 7) << 1) so the transposed reads below are conflict-free)
+  // (two loops, not two loads in one: the compiler makes one plain load of both)
+  auto walk = [&](auto nt_t) {
+    int c = w;
+    if (c < nch) load_chunk(nt_t, c, kr, vr);
+    for (; c < nch; c += 4) {
+      // stage this chunk's V into the wave-private LDS image (row-major, 16-B chunk
+      // index XOR ((row & 7) << 1) so the transposed reads below are conflict-free)
 #pragma unroll
-    for (int i = 0; i < NVL; ++i) {
-      const int row = i * RPL + lane / CPR, ch = lane % CPR;
-      *reinterpret_cast<short8*>(vw + row * D + ((ch ^ ((row & 7) << 1)) & (CPR - 1)) * 8) = vr[i];
-    }
-    // S^T tiles: lane (q = r16) holds keys 16t + 4*h4 + i
-    floatx4 sc[2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      sc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int kk = 0; kk < KK; ++kk)
-        sc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kr[t][kk], qf[kk], sc[t], 0, 0, 0);
-    }
-    // K consumed, V already in LDS: the next chunk's loads fly under softmax + PV (no
-    // second register set: 32 VGPRs fewer, three workgroups per CU)
-    if (c + 4 < nch) load_chunk(c + 4, kr, vr);
-    float mx = -INFINITY;
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int rel = 32 * c + 16 * t + 4 * h4 + i;
-        const float x = rel < nkeys ? sc[t][i] * scale_log2 : -INFINITY;
-        sc[t][i] = x;
-        mx = fmaxf(mx, x);
+      for (int i = 0; i < NVL; ++i) {
+        const int row = i * RPL + lane / CPR, ch = lane % CPR;
+        *reinterpret_cast<short8*>(vw + row * D + ((ch ^ ((row & 7) << 1)) & (CPR - 1)) * 8) = vr[i];
       }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float m_new = fmaxf(m_run, mx);  // finite: every chunk has >= 1 valid key
-    const float alpha = exp2f(m_run - m_new);
-    float rs = 0.f;
-    short8 pa;
+      // S^T tiles: lane (q = r16) holds keys 16t + 4*h4 + i
+      floatx4 sc[2];
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < 2; ++t) {
+        sc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float e = exp2f(sc[t][i] - m_new);
-        rs += e;
-        pa[4 * t + i] = (short)f2bf(e);
+        for (int kk = 0; kk < KK; ++kk)
+          sc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kr[t][kk], qf[kk], sc[t], 0, 0, 0);
       }
-    rs += __shfl_xor(rs, 16, 64);
-    rs += __shfl_xor(rs, 32, 64);
-    l_run = l_run * alpha + rs;
-    m_run = m_new;
-    // O rows are q = 4*h4 + reg: fetch alpha of those query rows (lanes 0..15 hold q = lane)
+      // K consumed, V already in LDS: the next chunk's loads fly under softmax + PV (no
+      // second register set: 32 VGPRs fewer, three workgroups per CU)
+      if (c + 4 < nch) load_chunk(nt_t, c + 4, kr, vr);
+      float mx = -INFINITY;
 #pragma unroll
-    for (int rr = 0; rr < 4; ++rr) {
-      const float a = __shfl(alpha, 4 * h4 + rr, 64);
+      for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int n = 0; n < ND; ++n) o[n][rr] *= a;
+        for (int i = 0; i < 4; ++i) {
+          const int rel = 32 * c + 16 * t + 4 * h4 + i;
+          const float x = rel < nkeys ? sc[t][i] * scale_log2 : -INFINITY;
+          sc[t][i] = x;
+          mx = fmaxf(mx, x);
+        }
+      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      const float m_new = fmaxf(m_run, mx);  // finite: every chunk has >= 1 valid key
+      const float alpha = exp2f(m_run - m_new);
+      float rs = 0.f;
+      short8 pa;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float e = exp2f(sc[t][i] - m_new);
+          rs += e;
+          pa[4 * t + i] = (short)f2bf(e);
+        }
+      rs += __shfl_xor(rs, 16, 64);
+      rs += __shfl_xor(rs, 32, 64);
+      l_run = l_run * alpha + rs;
+      m_run = m_new;
+      // O rows are q = 4*h4 + reg: fetch alpha of those query rows (lanes 0..15 hold q = lane)
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) {
+        const float a = __shfl(alpha, 4 * h4 + rr, 64);
+#pragma unroll
+        for (int n = 0; n < ND; ++n) o[n][rr] *= a;
+      }
+      // PV: B = V^T fragment of k-step = keys {4*h4 + j} u {16 + 4*h4 + j}, column 16n + r16
+      const int qq = r16 >> 2, pp = r16 & 3;
+#pragma unroll
+      for (int n = 0; n < ND; ++n) {
+        const int col = 16 * n + 4 * pp;
+        const int r0 = 4 * h4 + qq, r1 = 16 + 4 * h4 + qq;
+        const bf16_t* a0 = vw + r0 * D + (((col >> 3) ^ ((r0 & 7) << 1)) & (CPR - 1)) * 8 + (col & 7);
+        const bf16_t* a1 = vw + r1 * D + (((col >> 3) ^ ((r1 & 7) << 1)) & (CPR - 1)) * 8 + (col & 7);
+        const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4_ptr)(a0));
+        const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4_ptr)(a1));
+        const short8 vb = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        o[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa, vb, o[n], 0, 0, 0);
+      }
     }
-    // PV: B = V^T fragment of k-step = keys {4*h4 + j} u {16 + 4*h4 + j}, column 16n + r16
-    const int qq = r16 >> 2, pp = r16 & 3;
-#pragma unroll
-    for (int n = 0; n < ND; ++n) {
-      const int col = 16 * n + 4 * pp;
-      const int r0 = 4 * h4 + qq, r1 = 16 + 4 * h4 + qq;
-      const bf16_t* a0 = vw + r0 * D + (((col >> 3) ^ ((r0 & 7) << 1)) & (CPR - 1)) * 8 + (col & 7);
-      const bf16_t* a1 = vw + r1 * D + (((col >> 3) ^ ((r1 & 7) << 1)) & (CPR - 1)) * 8 + (col & 7);
-      const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4_ptr)(a0));
-      const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4_ptr)(a1));
-      const short8 vb = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-      o[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa, vb, o[n], 0, 0, 0);
-    }
+  };
+  if constexpr (READ == READ_SHARED) {
+    if (shared) walk(std::false_type{});
+    else walk(std::true_type{});
+  } else {
+    walk(std::integral_constant<bool, READ == READ_ONCE>{});
   }
 
   // ---- merge the 4 waves: (m, l) per query row (lanes 0..15 hold q = lane), O rows
@@ -357,12 +385,17 @@ int lk_paged_decode(const bf16_t* q, long qs, const bf16_t* kc, const bf16_t* vc
   const int G = Hq / Hkv;
   const float scale_log2 = scale * 1.4426950408889634f;
   dim3 grid(B * Hkv, max_splits);
-#define LAUNCH(DD, GG) do { if (own_blocks) LAUNCH_NT(DD, GG, true); else LAUNCH_NT(DD, GG, false); } while (0)
-#define LAUNCH_NT(DD, GG, NT)                                                                 \
-  paged_decode_kernel<DD, GG, NT><<<grid, 256, 0, st>>>(q, qs, kc, vc, block_tables, bt_stride,   \
+#define LAUNCH(DD, GG)                                            \
+  do {                                                            \
+    if (own_blocks) LAUNCH_READ(DD, GG, READ_ONCE);               \
+    else if (B < kShareRows) LAUNCH_READ(DD, GG, READ_PLAIN);     \
+    else LAUNCH_READ(DD, GG, READ_SHARED);                        \
+  } while (0)
+#define LAUNCH_READ(DD, GG, READ)                                                                \
+  paged_decode_kernel<DD, GG, READ><<<grid, 256, 0, st>>>(q, qs, kc, vc, block_tables, bt_stride,   \
                                                     ctx_lens, out, os, part_o, part_ml, Hkv, \
                                                     BS, max_splits, split, scale_log2, k_start, \
-                                                    pp_o != nullptr, pp_o, pp_ml, tickets)
+                                                    pp_o != nullptr, pp_o, pp_ml, tickets, B)
 #define BY_G(DD)                          \
   switch (G) {                            \
     case 1: LAUNCH(DD, 1); break;         \
@@ -376,7 +409,7 @@ int lk_paged_decode(const bf16_t* q, long qs, const bf16_t* kc, const bf16_t* vc
   else return -3;
 #undef BY_G
 #undef LAUNCH
-#undef LAUNCH_NT
+#undef LAUNCH_READ
   LK_CHECK_LAUNCH();
   // (fused: the last split merges; reduce == 0: the consumer merges -- the O projection's
   // weight-streaming prologue, lk_wsgemm_pro kind 2)

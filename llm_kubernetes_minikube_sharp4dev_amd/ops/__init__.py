@@ -168,7 +168,7 @@ def paged_decode(q, k_cache, v_cache, block_tables, ctx_lens, scale: float, max_
     merges (the CPU reference attends everything directly).  ``reduce=False`` (GPU, no
     tickets): rows with more than one split keep their partials in ``part_o`` / ``part_ml`` for
     the consumer to merge (:func:`ws_pro` kind 2).  ``own_blocks``: no cache block belongs to two rows (their
-    reads then pass the caches by; the result is the same)."""
+    reads then pass the caches by; without it every split looks whether its rows are shared; the result is the same)."""
     if use_hip(q):
         BS = k_cache.shape[2]
         if split is None:

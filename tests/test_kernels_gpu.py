@@ -162,6 +162,25 @@ def test_paged_decode_own_blocks(hip, G, D):
         bt[4] = bt[3]
 
 
+@pytest.mark.parametrize("rows", [15, 16, 300])
+@pytest.mark.parametrize("shared", [0, 16, 320, 700])
+def test_paged_decode_shared_prefixes(hip, rows, shared):
+    """From 16 rows on every split looks for rows that share its blocks and reads accordingly: no bit changes, whatever is shared and by whom."""
+    torch.manual_seed(rows + shared)
+    Hkv, D = 2, 128
+    ctx = [(1, 16, 400, 701, 950)[i % 5] for i in range(rows)]
+    kc, vc, bt = _paged_setup(rows, ctx, Hkv, D, 16)
+    for i in range(rows):   # every third row has the prefix of the row two before it, as far as both go
+        if i % 3 == 2:
+            n = min(shared, ctx[i], ctx[i - 2]) // 16
+            bt[i, :n] = bt[i - 2, :n]
+    q = torch.randn(rows, Hkv * 4, D, device=DEV, dtype=torch.bfloat16)
+    cl = torch.tensor(ctx, dtype=torch.int32, device=DEV)
+    for split in (128, 512, 2048):
+        a, b = (ops.paged_decode(q, kc, vc, bt, cl, D ** -0.5, split=split, own_blocks=own) for own in (False, True))
+        assert torch.equal(a, b)
+
+
 def test_paged_decode_fused_merge_empty_rows(hip):
     """Rows without keys (graph-bucket padding, ctx 0) get zeros from split 0 when no reduce
     kernel runs (the separate reduce kernel leaves such rows unwritten: nobody reads them); the
