@@ -261,12 +261,26 @@ __global__ __launch_bounds__(256) void head_linear_few_kernel(const T* __restric
   }
 }
 
+int cu_count() {
+  static const int cus = [] {
+    int dev = 0, n = 256;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 256;
+    return n;
+  }();
+  return cus;
+}
+
 template <typename T, int PARTS>
 int head_linear_t(const void* x, long xs, long xh, const void* w, int H, int N, int K, long rows, void* out, long os, long oh, int vec, int vst,
                   const RotTail& rot, hipStream_t st) {
   if (N > 0 && rows > 65535L * 64) return -1;
   const bool fused = rot.RDP > 0 && N > 0 && rows <= 128;
   const int tail = fused ? 1 : 0;   // workgroups of 16 rows each behind the columns'
+  // 16-row tiles of a workgroup: up to 4, fewer while that leaves no more than one workgroup per CU (a workgroup's rows come at the rate of
+  // its CU; the weights, read once more per halving, out of L2).  16 heads of 128 columns on K 512 in two parts at 64 rows: 4, 2, 1 tiles 8.3,
+  // 5.6, 4.7 us, at 128 rows 8.4, 5.7, 6.3; 32 heads at 128 rows (2 tiles: 512 workgroups) 8.8, 8.4, 10.0; in one part at 64 rows 6.0, 4.7, 4.1.
+  int rt = rows <= 16 ? 1 : rows <= 32 ? 2 : 4;
+  while (rt > 1 && (long)H * ((N + 31) / 32) * ((rows + 8 * rt - 1) / (8 * rt)) <= cu_count()) rt /= 2;
 #define LK_HEAD(RT)                                                                                                                          \
   head_linear_few_kernel<T, RT, PARTS><<<dim3((unsigned)((long)H * ((N + 31) / 32 + tail * RT)), 1, (unsigned)((rows + 16 * RT - 1) / (16 * RT))),  \
                                   256, 0, st>>>((const T*)x, xs, xh, (const T*)w, N, K, rows, (T*)out, os, oh, vec, vst, H, (N + 31) / 32, rot)
@@ -275,9 +289,9 @@ int head_linear_t(const void* x, long xs, long xh, const void* w, int H, int N, 
   else if (rows > 128 && vec && (PARTS == 1 || K % 64 == 0))
     head_linear_lds_kernel<T, PARTS><<<dim3((unsigned)H, (unsigned)((N + 127) / 128), (unsigned)((rows + 127) / 128)), 256, 0, st>>>(
         (const T*)x, xs, xh, (const T*)w, N, K, rows, (T*)out, os, oh, vst);
-  else if (rows <= 16)
+  else if (rt == 1)
     LK_HEAD(1);
-  else if (rows <= 32)
+  else if (rt == 2)
     LK_HEAD(2);
   else
     LK_HEAD(4);

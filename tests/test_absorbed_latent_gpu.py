@@ -192,6 +192,22 @@ def test_head_products_of_two_parts(rows, H, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows", [16, 33, 63, 64, 65, 127, 128])
+@pytest.mark.parametrize("H,N", [(16, 128), (40, 128), (130, 128)])   # one, two and four 16-row tiles per workgroup among the rows
+@pytest.mark.parametrize("parts", [1, 2])
+def test_head_products_row_tiles(rows, H, N, parts):
+    from llm_kubernetes_minikube_sharp4dev_amd import ops
+    K = 64
+    g = torch.Generator().manual_seed(rows + H)
+    x, w = q16(rnd(g, rows, H, parts, K)), q16(rnd(g, H, N, K, scale=K ** -0.5))
+    buf = torch.full((rows + 1, H, N), 7.0, dtype=torch.bfloat16, device="cuda")
+    ops.head_linear(x.reshape(rows, -1).bfloat16().cuda(), w.bfloat16().cuda(), parts * K, buf[:rows], parts=parts)
+    want = torch.bmm(x.double().sum(2).transpose(0, 1), w.double().transpose(1, 2).contiguous()).transpose(0, 1)
+    assert bool(((buf[:rows].double().cpu() - want).abs() <= 2 ** -8 * want.abs() + 1e-5).all())   # as above
+    assert bool((buf[rows] == 7.0).all())
+
+
+@pytest.mark.gpu
 def test_head_products_of_many_columns():
     """More 32-column workgroups than a grid's second dimension has places."""
     from llm_kubernetes_minikube_sharp4dev_amd import ops
