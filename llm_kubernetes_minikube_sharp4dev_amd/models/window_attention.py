@@ -265,8 +265,8 @@ class LatentAttnSpec:
         then cost alike at every length), where a token's row is at most a quarter of its expanded heads and the products per key at
         most 3.5 times theirs.  Its error is no larger than the expanded form's (the averages go into ``W_uv`` in two bf16 parts).
         One mixer, expanded -> cached latent, at 1,024 positions, in us for 4,096 prompt rows / 64 / 4 decoded: 16 heads of 128 + 64 / 128,
-        rank 512 (3.4 times the products), window 512: 333 / 143 / 41 -> 343 / 66 / 40; 32 heads, window 2,048: 692 / 415 / 67 -> 645 / 83 /
-        48; 16 heads of 64 + 32 / 64, rank 128 (2 times): 153 / 47 / 30 -> 140 / 35 / 27; rank 256 (3.6 times, beyond the line): 192 / 74 /
+        rank 512 (3.4 times the products), window 512: 333 / 143 / 41 -> 343 / 59 / 40; 32 heads, window 2,048: 692 / 415 / 67 -> 645 / 77 /
+        48; 16 heads of 64 + 32 / 64, rank 128 (2 times): 153 / 47 / 30 -> 140 / 34 / 27; rank 256 (3.6 times, beyond the line): 192 / 74 /
         33 -> 216 / 47 / 33."""
         rp, rdp = ops.latent_row(self.kv_rank, self.rot_dim)
         return (dtype == torch.bfloat16 and torch.device(device).type == "cuda" and self.window > 0 and not self.gate_elem
