@@ -181,21 +181,27 @@ at::Tensor ws_linear(const at::Tensor& x, const at::Tensor& w, bool swiglu, int6
 
 // few-row GEMM (csrc/rows_gemm.hip): M <= 4,096 rows, any epilogue, one launch.  epi: 0 none, 1 SwiGLU, 2 bias, 3 bias + GELU,
 // 4 bias + ReLU
-at::Tensor rows_linear(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, int64_t epi, bool wide) {
+at::Tensor rows_linear(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, int64_t epi, int64_t wide,
+                       const c10::optional<at::Tensor>& residual) {
   CHECK_CUDA(x); CHECK_BF16(x); CHECK_BF16(w); CHECK_LASTDIM(x); CHECK_CONTIG(w);
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1), "x [M,K], w [N,K]");
   check_rows16(x, "x"); check_rows16(w, "w");
   const int M = x.size(0), K = x.size(1), N = w.size(0);
-  TORCH_CHECK(epi >= 0 && epi <= 4 && lk_rows_gemm_supported(M, N, K, (int)epi),
+  TORCH_CHECK(epi >= 0 && epi <= 5 && lk_rows_gemm_supported(M, N, K, (int)epi),
               "rows_linear: M in [1, 4096], K a multiple of 64, N of 16 (32 with SwiGLU)");
-  TORCH_CHECK((epi >= 2) == bias.has_value(), "rows_linear: a bias goes with epilogues 2-4");
+  TORCH_CHECK((epi >= 2) == bias.has_value(), "rows_linear: a bias goes with epilogues 2-5");
+  TORCH_CHECK((epi == 5) == residual.has_value(), "rows_linear: a residual goes with epilogue 5");
   if (bias) {
     CHECK_CUDA((*bias)); CHECK_BF16((*bias)); CHECK_CONTIG((*bias));
     TORCH_CHECK(bias->numel() == N, "bias shape");
   }
+  if (residual) {
+    CHECK_CUDA((*residual)); CHECK_BF16((*residual)); CHECK_LASTDIM((*residual));
+    TORCH_CHECK(residual->dim() == 2 && residual->size(0) == M && residual->size(1) == N, "residual [M, N]");
+  }
   at::Tensor out = at::empty({M, epi == 1 ? N / 2 : N}, x.options());
-  int rc = lk_rows_gemm(bp(x), bp(w), bias ? bp(*bias) : nullptr, bp(out), M, N, K, x.stride(0), out.stride(0), (int)epi, wide ? 1 : 0,
-                        cur_stream());
+  int rc = lk_rows_gemm(bp(x), bp(w), bias ? bp(*bias) : nullptr, residual ? bp(*residual) : nullptr, residual ? residual->stride(0) : 0, bp(out),
+                        M, N, K, x.stride(0), out.stride(0), (int)epi, (int)wide, cur_stream());
   CHECK_RC(rc, "rows_linear");
   return out;
 }
@@ -2260,7 +2266,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_linear", &skinny_linear, "", py::arg("x"), py::arg("w"), py::arg("swiglu") = false,
         py::arg("splits") = 0, py::arg("out") = py::none());
   m.def("skinny_splits", &skinny_splits);
-  m.def("rows_linear", &rows_linear, py::arg("x"), py::arg("w"), py::arg("bias") = py::none(), py::arg("epi") = 0, py::arg("wide") = false);
+  m.def("rows_linear", &rows_linear, py::arg("x"), py::arg("w"), py::arg("bias") = py::none(), py::arg("epi") = 0, py::arg("wide") = 0,
+        py::arg("residual") = py::none());
   m.def("rows_supported", [](int64_t M, int64_t N, int64_t K, int64_t epi) { return lk_rows_gemm_supported((int)M, (int)N, (int)K, (int)epi); });
   m.def("ws_linear", &ws_linear, "", py::arg("x"), py::arg("w"), py::arg("swiglu") = false, py::arg("bn") = 0,
         py::arg("splits") = 0, py::arg("out") = py::none());

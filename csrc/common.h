@@ -37,16 +37,28 @@ LK_DEVICE unsigned pack_bf2(float lo, float hi) {
   return __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2_t){lo, hi}, bf16x2_t));
 }
 
-LK_DEVICE float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+// Butterflies over the 64 lanes in the order 32, 16, 8, 4, 2, 1 (every lane ends with the same bits), by lane swaps and row rotations
+// of the vector unit: __shfl_xor goes through the LDS unit, whose latency was most of a short row's reduction.
+template <int STEP>
+LK_DEVICE float wave_partner(float v) {  // the value of lane ^ STEP or of another lane that holds the same partial result
+  return __uint_as_float((unsigned)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), 0x120 + STEP, 0xf, 0xf, true));  // row_ror
 }
-
+template <typename F>
+LK_DEVICE float wave_all(float v, F f) {
+  auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(h[0]), __uint_as_float(h[1]));
+  auto q = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(q[0]), __uint_as_float(q[1]));
+  v = f(v, wave_partner<8>(v));
+  v = f(v, wave_partner<4>(v));
+  v = f(v, wave_partner<2>(v));
+  return f(v, wave_partner<1>(v));
+}
+LK_DEVICE float wave_sum(float v) {
+  return wave_all(v, [](float a, float b) { return a + b; });
+}
 LK_DEVICE float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
+  return wave_all(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // block-wide sum for blockDim.x = NW*64; `red` must hold NW floats.

@@ -31,8 +31,9 @@ int lk_activation(bf16_t* x, const bf16_t* bias, long rows, int N, long xs, int 
 
 // rows_gemm.hip (few rows, up to 4,096; one launch, every epilogue)
 bool lk_rows_gemm_supported(int M, int N, int K, int epi);
-int lk_rows_gemm(const void* x, const void* w, const void* b, void* y, int M, int N, int K, long ldx, long ldy, int epi, int wide,
-                 hipStream_t st);
+// epi: 0 none, 1 SwiGLU, 2 bias, 3 bias + GELU, 4 bias + ReLU, 5 bf16(bias) + the residual rows r (elsewhere null)
+int lk_rows_gemm(const void* x, const void* w, const void* b, const void* r, long ldr, void* y, int M, int N, int K, long ldx, long ldy, int epi,
+                 int wide, hipStream_t st);
 
 // skinny_gemm.hip (decode-regime linear, optional fused SwiGLU)
 int lk_skinny_splits(int M, int N, int K, int swiglu);

@@ -14,6 +14,7 @@ LK_DEVICE void rg_wait() {
   static_assert(N >= 0 && N < 64, "vmcnt range");
   __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
 }
+LK_DEVICE void rg_wait_lds() { __builtin_amdgcn_s_waitcnt(0xF | (0x3 << 14) | (0x7 << 4)); }  // lgkmcnt(0) alone
 template <int L, int AHEAD>
 LK_DEVICE void rg_wait_ahead(int ahead) {  // all but the newest `ahead` stages of L loads have landed
   if constexpr (AHEAD > 0) {
@@ -59,28 +60,36 @@ LK_DEVICE void rg_walk(const bf16_t* const (&xs)[2 * MT], const bf16_t* const (&
 #pragma unroll
     for (int n = 0; n < NT; ++n) acc[m][n] = (floatx4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int p = 0; p < NS - 1; ++p)
+  for (int p = 0; p < NS; ++p)
     if (p < nst) issue(p);
   for (int st = 0; st < nst; ++st) {
-    rg_wait_ahead<L, NS - 2>(min(NS - 2, nst - 1 - st));
+    rg_wait_ahead<L, NS - 1>(min(NS - 1, nst - 1 - st));
     __builtin_amdgcn_sched_barrier(0);
-    if (st + NS - 1 < nst) issue(st + NS - 1);  // into the slot whose fragments the last stage's products have consumed
-    __builtin_amdgcn_sched_barrier(0);
+    // the whole stage into registers, so that its slot is free for the loads of stage st + NS before the products
     const unsigned char* base = ring + (st % NS) * SB;
+    short8 a[2][MT], b[2][NT];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int at = r16 * 128 + (((4 * h + g) ^ (r16 & 7)) << 4);
-      short8 a[MT], b[NT];
 #pragma unroll
-      for (int n = 0; n < NT; ++n) b[n] = *reinterpret_cast<const short8*>(base + (MT + n) * 2048 + at);
+      for (int n = 0; n < NT; ++n) b[h][n] = *reinterpret_cast<const short8*>(base + (MT + n) * 2048 + at);
 #pragma unroll
-      for (int m = 0; m < MT; ++m) a[m] = *reinterpret_cast<const short8*>(base + m * 2048 + at);
+      for (int m = 0; m < MT; ++m) a[h][m] = *reinterpret_cast<const short8*>(base + m * 2048 + at);
+    }
+    if (st + NS < nst) {
+      __builtin_amdgcn_sched_barrier(0);
+      rg_wait_lds();   // the reads are done before a load may write there
+      __builtin_amdgcn_sched_barrier(0);
+      issue(st + NS);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
       // W as the A operand: the lane ends with one output row and 4 consecutive columns
 #pragma unroll
       for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int n = 0; n < NT; ++n) acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[n], a[m], acc[m][n], 0, 0, 0);
-    }
+        for (int n = 0; n < NT; ++n) acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[h][n], a[h][m], acc[m][n], 0, 0, 0);
   }
 }
 

@@ -4,36 +4,42 @@
 // What bounds it: at these sizes neither HBM (a 2048 x 2048 weight is 1.4 us of it) nor the matrix cores
 // but the serial chain of a launch: a tiled kernel with a barrier per K stage waits for each of them, and
 // a split-K one pays a second launch for its sum.  Here no wave waits for another inside the K walk:
-//   * a workgroup of 4 waves owns 16 output columns (wide: 32; SwiGLU: 16 gate and the 16 up columns) and up
+//   * a workgroup of 4 waves owns 16 output columns (wide: 32 or 64; SwiGLU: half of them gate and half the up columns) and up
 //     to 64 rows; the waves split K, so each element of X and W reaches the workgroup once;
 //   * every wave streams its own K range through a private LDS ring by LDS-DMA (row_ring.h; loads straight into
 //     the fragment layout, 16 rows x 64 bytes, ran at a quarter of the rate: 12.0 us against 7.7 at
 //     64 x 2048 x 2048, 8.4 against 5.7 at 32 rows);
 //   * the waves' sums meet once in LDS, then the epilogue stores 4 columns per lane;
-//   * 16 columns per workgroup give N / 16 workgroups, which is what fills 256 CUs at N 2048-4096; with more
-//     rows or columns than that, 32 columns halve the re-reading of X out of L2 (256 x 2048 x 2048: 13.3 -> 8.8 us).
-//     That re-reading bounds the large end, where the tiled kernels take over (ops: _rows_rule).
+//   * what a CU loads into LDS is then the time: 58 - 68 KB/us, with three stages of the ring in flight or with four.  So the
+//     tile is the one with the fewest bytes per CU: 16 columns and few rows where that fills 256 CUs (64 x 2048 x 2048: 64 rows
+//     6.9 us, 32 rows 6.0; K 5632: 15.6 -> 12.0; 64 x 768 x 3072: 16 rows 8.5 -> 5.2), 64 columns where N is large (64 x 10496 x
+//     2048: 17.9 -> 14.3, SwiGLU 64 x 11264 x 2048: 17.2 -> 14.6; 32 columns need a second round of workgroups).
+//     With many rows the re-reading of X out of L2 bounds it and the tiled kernels take over (ops: _rows_rule).
 #include "common.h"
 #include "kernels.h"
 #include "row_ring.h"
 
 namespace {
 
-constexpr int kRgRows = 64;  // rows of a workgroup
-
-enum { RG_NONE = 0, RG_SWIGLU = 1, RG_BIAS = 2, RG_GELU = 3, RG_RELU = 4 };
+enum { RG_NONE = 0, RG_SWIGLU = 1, RG_BIAS = 2, RG_GELU = 3, RG_RELU = 4, RG_ADD = 5 };
 
 template <int MT, int NT, int NS, int EPI>
 __global__ __launch_bounds__(64 * kRgWaves, 1) void rows_gemm_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
-                                                                     const bf16_t* __restrict__ bias, bf16_t* __restrict__ Y, int M,
-                                                                     int N, int K, long ldx, long ldy) {
+                                                                     const bf16_t* __restrict__ bias, const bf16_t* __restrict__ R,
+                                                                     long ldr, bf16_t* __restrict__ Y, int M, int N, int K, long ldx,
+                                                                     long ldy) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int all = K / 64, first = wave * all / kRgWaves, nst = (wave + 1) * all / kRgWaves - first;  // stages of this wave
-  const int n0 = blockIdx.x * (EPI == RG_SWIGLU ? 16 : 16 * NT), m0 = blockIdx.y * kRgRows;  // first output column and row
+  // grid (8 XCDs, row tiles, column tiles / 8): the row tiles of a column tile follow one another on one XCD, whose L2 then has the
+  // weight rows
+  const int cols = EPI == RG_SWIGLU ? N / 2 : N;
+  const int n0 = (blockIdx.z * 8 + blockIdx.x) * (EPI == RG_SWIGLU ? 8 * NT : 16 * NT), m0 = blockIdx.y * (16 * MT);  // first output column and row
+  if (n0 >= cols) return;   // the whole workgroup: the grid holds whole eights of column tiles
   X += (long)m0 * ldx;
   Y += (long)m0 * ldy;
-  M = min(M - m0, kRgRows);
+  if constexpr (EPI == RG_ADD) R += (long)m0 * ldr;
+  M = min(M - m0, 16 * MT);
   const int lrow = lane >> 3;
   const long k = (long)first * 64 + rg_lane_col(lane);
   const bf16_t* xs[2 * MT];
@@ -41,24 +47,30 @@ __global__ __launch_bounds__(64 * kRgWaves, 1) void rows_gemm_kernel(const bf16_
 #pragma unroll
   for (int i = 0; i < 2 * MT; ++i) xs[i] = X + (long)min(8 * i + lrow, M - 1) * ldx + k;  // rows past M repeat the last one
 #pragma unroll
-  for (int i = 0; i < 2 * NT; ++i) ws[i] = W + ((EPI == RG_SWIGLU ? (long)(i >> 1) * (N >> 1) : (i >> 1) * 16) + n0 + 8 * (i & 1) + lrow) * K + k;
+  for (int i = 0; i < 2 * NT; ++i) {
+    const int t = i >> 1;   // W tile; SwiGLU: the second half are the up rows of the first half's columns
+    constexpr int HT = NT > 1 ? NT / 2 : 1;
+    const long row = EPI == RG_SWIGLU ? (long)(t / HT) * cols + t % HT * 16 : t * 16;
+    ws[i] = W + (row + n0 + 8 * (i & 1) + lrow) * K + k;
+  }
   floatx4 acc[MT][NT];
   rg_walk<MT, NT, NS>(xs, ws, nst, smem + wave * NS * rg_stage(MT, NT), acc);
   rg_sums<MT, NT>(smem, acc, [&](int m, const floatx4 (&t)[NT]) {
     const int row = m * 16 + (lane & 15), col = n0 + 4 * (lane >> 4);
     if (row >= M) return;
 #pragma unroll
-    for (int n = 0; n < (EPI == RG_SWIGLU ? 1 : NT); ++n) {
+    for (int n = 0; n < (EPI == RG_SWIGLU ? NT / 2 : NT); ++n) {
       float y[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         if constexpr (EPI == RG_SWIGLU) {  // rounded as the projection and the activation apart round
-          y[j] = bf2f(f2bf(lk_silu(bf2f(f2bf(t[0][j]))))) * bf2f(f2bf(t[NT - 1][j]));
+          y[j] = bf2f(f2bf(lk_silu(bf2f(f2bf(t[n][j]))))) * bf2f(f2bf(t[n + NT / 2][j]));
         } else {
           y[j] = t[n][j];
           if constexpr (EPI >= RG_BIAS) y[j] += bf2f(bias[col + 16 * n + j]);
           if constexpr (EPI == RG_GELU) y[j] = lk_gelu_erf(y[j]);
           if constexpr (EPI == RG_RELU) y[j] = fmaxf(y[j], 0.f);
+          if constexpr (EPI == RG_ADD) y[j] = bf2f(f2bf(y[j])) + bf2f(R[(long)row * ldr + col + 16 * n + j]);  // rounded as the product and the sum apart
         }
       }
       uint2 pk;
@@ -69,29 +81,61 @@ __global__ __launch_bounds__(64 * kRgWaves, 1) void rows_gemm_kernel(const bf16_
   });
 }
 
-template <int MT, int NT, int NS, int EPI>
-int launch(const void* x, const void* w, const void* b, void* y, int M, int N, int K, long ldx, long ldy, hipStream_t st) {
-  constexpr int lds = rg_lds(MT, NT, NS);
+template <int MT, int NT, int EPI>
+int launch(const void* x, const void* w, const void* b, const void* r, long ldr, void* y, int M, int N, int K, long ldx, long ldy, hipStream_t st) {
+  constexpr int NS0 = 20 / (MT + NT), NS = NS0 > 5 ? 5 : NS0, lds = rg_lds(MT, NT, NS);   // stages: as many as 160 KB hold
   LK_SET_MAX_LDS((rows_gemm_kernel<MT, NT, NS, EPI>), lds);
-  rows_gemm_kernel<MT, NT, NS, EPI><<<dim3(N / (16 * NT), (M + kRgRows - 1) / kRgRows), 64 * kRgWaves, lds, st>>>((const bf16_t*)x, (const bf16_t*)w, (const bf16_t*)b,
-                                                                              (bf16_t*)y, M, N, K, ldx, ldy);
+  const int cols = N / (16 * NT), tiles = (M + 16 * MT - 1) / (16 * MT);
+  rows_gemm_kernel<MT, NT, NS, EPI><<<dim3(8, tiles, (cols + 7) / 8), 64 * kRgWaves, lds, st>>>(
+      (const bf16_t*)x, (const bf16_t*)w, (const bf16_t*)b, (const bf16_t*)r, ldr, (bf16_t*)y, M, N, K, ldx, ldy);
   LK_CHECK_LAUNCH();
   return 0;
 }
 
-template <int EPI>
-int by_rows(const void* x, const void* w, const void* b, void* y, int M, int N, int K, long ldx, long ldy, int wide, hipStream_t st) {
-  constexpr int NT = EPI == RG_SWIGLU ? 2 : 1;
-  if constexpr (EPI != RG_SWIGLU) {
-    if (wide && N % 32 == 0) {
-      if (M <= 32) return launch<2, 2, 3, EPI>(x, w, b, y, M, N, K, ldx, ldy, st);
-      return launch<4, 2, 3, EPI>(x, w, b, y, M, N, K, ldx, ldy, st);
+int device_cus() {
+  static const int n = [] {
+    int dev = 0, v = 0;
+    return hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0 ? v : 256;
+  }();
+  return n;
+}
+
+// Row tiles per workgroup: its time is its bytes, 16 (MT + NT) rows of K, times the rounds of workgroups.  Where column tiles leave CUs
+// free, fewer rows per workgroup read the same weight rows out of L2 again and end sooner.
+int row_tiles(int M, int cols, int nt) {
+  const int m16 = (M + 15) / 16, cus = device_cus();
+  int best = 4, cost = 1 << 30;
+  for (int mt = m16 < 4 ? m16 : 4; mt >= 1; --mt) {
+    const int rounds = ((m16 + mt - 1) / mt * cols + cus - 1) / cus, c = rounds * (mt + nt);
+    if (c < cost) {
+      cost = c;
+      best = mt;
     }
   }
-  if (M <= 16) return launch<1, NT, NT == 1 ? 5 : 4, EPI>(x, w, b, y, M, N, K, ldx, ldy, st);
-  if (M <= 32) return launch<2, NT, 4, EPI>(x, w, b, y, M, N, K, ldx, ldy, st);
-  if (M <= 48) return launch<3, NT, 4, EPI>(x, w, b, y, M, N, K, ldx, ldy, st);
-  return launch<4, NT, NT == 1 ? 4 : 3, EPI>(x, w, b, y, M, N, K, ldx, ldy, st);
+  return best;
+}
+
+template <int NT, int EPI>
+int by_rows(const void* x, const void* w, const void* b, const void* r, long ldr, void* y, int M, int N, int K, long ldx, long ldy, hipStream_t st) {
+  switch (row_tiles(M, N / (16 * NT), NT)) {
+    case 1: return launch<1, NT, EPI>(x, w, b, r, ldr, y, M, N, K, ldx, ldy, st);
+    case 2: return launch<2, NT, EPI>(x, w, b, r, ldr, y, M, N, K, ldx, ldy, st);
+    case 3: return launch<3, NT, EPI>(x, w, b, r, ldr, y, M, N, K, ldx, ldy, st);
+    default: return launch<4, NT, EPI>(x, w, b, r, ldr, y, M, N, K, ldx, ldy, st);
+  }
+}
+
+// wide: 0: 16 columns per workgroup (SwiGLU: 16 gate and 16 up), 1: 32 (SwiGLU: as 0), 2: 64 (SwiGLU: 32 and 32), where N divides
+template <int EPI>
+int by_cols(const void* x, const void* w, const void* b, const void* r, long ldr, void* y, int M, int N, int K, long ldx, long ldy, int wide,
+            hipStream_t st) {
+  if (wide == 2 && N % 64 == 0) return by_rows<4, EPI>(x, w, b, r, ldr, y, M, N, K, ldx, ldy, st);
+  if constexpr (EPI == RG_SWIGLU) {
+    return by_rows<2, EPI>(x, w, b, r, ldr, y, M, N, K, ldx, ldy, st);
+  } else {
+    if (wide && N % 32 == 0) return by_rows<2, EPI>(x, w, b, r, ldr, y, M, N, K, ldx, ldy, st);
+    return by_rows<1, EPI>(x, w, b, r, ldr, y, M, N, K, ldx, ldy, st);
+  }
 }
 
 }  // namespace
@@ -101,15 +145,16 @@ bool lk_rows_gemm_supported(int M, int N, int K, int epi) {
   return M >= 1 && M <= 4096 && K >= 64 && K % 64 == 0 && N >= 16 && N % (epi == RG_SWIGLU ? 32 : 16) == 0;
 }
 
-int lk_rows_gemm(const void* x, const void* w, const void* b, void* y, int M, int N, int K, long ldx, long ldy, int epi, int wide,
-                 hipStream_t st) {
+int lk_rows_gemm(const void* x, const void* w, const void* b, const void* r, long ldr, void* y, int M, int N, int K, long ldx, long ldy, int epi,
+                 int wide, hipStream_t st) {
   if (!lk_rows_gemm_supported(M, N, K, epi) || ldy % 4) return -1;
   switch (epi) {
-    case RG_NONE: return by_rows<RG_NONE>(x, w, b, y, M, N, K, ldx, ldy, wide, st);
-    case RG_SWIGLU: return by_rows<RG_SWIGLU>(x, w, b, y, M, N, K, ldx, ldy, wide, st);
-    case RG_BIAS: return by_rows<RG_BIAS>(x, w, b, y, M, N, K, ldx, ldy, wide, st);
-    case RG_GELU: return by_rows<RG_GELU>(x, w, b, y, M, N, K, ldx, ldy, wide, st);
-    case RG_RELU: return by_rows<RG_RELU>(x, w, b, y, M, N, K, ldx, ldy, wide, st);
+    case RG_NONE: return by_cols<RG_NONE>(x, w, b, r, ldr, y, M, N, K, ldx, ldy, wide, st);
+    case RG_SWIGLU: return by_cols<RG_SWIGLU>(x, w, b, r, ldr, y, M, N, K, ldx, ldy, wide, st);
+    case RG_BIAS: return by_cols<RG_BIAS>(x, w, b, r, ldr, y, M, N, K, ldx, ldy, wide, st);
+    case RG_GELU: return by_cols<RG_GELU>(x, w, b, r, ldr, y, M, N, K, ldx, ldy, wide, st);
+    case RG_RELU: return by_cols<RG_RELU>(x, w, b, r, ldr, y, M, N, K, ldx, ldy, wide, st);
+    case RG_ADD: return by_cols<RG_ADD>(x, w, b, r, ldr, y, M, N, K, ldx, ldy, wide, st);
     default: return -1;
   }
 }

@@ -386,15 +386,17 @@ def _decode_bucket(M: int) -> Optional[int]:
 
 
 # Few rows (csrc/rows_gemm.hip, one launch with any epilogue) or the kernels with larger tiles.  A workgroup of the few-row
-# kernel reads 16 (wide: 32) columns of W -- SwiGLU 2 x 16 -- and up to 64 rows of X, so its time is
+# kernel reads 16 (``wide`` True: 32, 2: 64) columns of W -- SwiGLU 2 x 16 or 2 x 32 -- and 16 to 64 rows of X, as many as need the
+# fewest bytes per CU, so its time is
 #   2.6 us + rounds of workgroups (one per CU) x (their bytes / 58 KB/us) + 1 us per round behind the first,
-# and not below W at 4.2 TB/s.  The other side: up to 256 rows without a bias the weight-streaming kernel (its two launches,
+# and not below W at 4.2 TB/s (a CU's loads into LDS run at 58 - 68 KB/us whatever the depth of the ring).  64 columns only from
+# N 3072 on: below, the narrower forms fill the chip in one round.  The other side: up to 256 rows without a bias the weight-streaming kernel (its two launches,
 # 0.14 us per MB of W, M / 22; 3.5 us for SwiGLU's second launch), else the prefill GEMM (a chain of K / 64 stages
 # whatever M is, as long as its tiles are fewer than CUs).  Measured in hipGraphs, weights cold, few-row / other (us):
-#    64 x  2048 x 2048  7.7 / 11.0    256 x 2048 x 2048  8.8 / 19.7    768 x 2048 x 2048 22.8 / 28.6   1024: 30.3 / 30.2
-#    64 x 10368 x 2048 17.9 / 16.7    128 x 4096 x 4096 15.7 / 18.4    192 x 4096 x 4096 28.6 / 20.9
-#    64 x 11264 x 2048 (SwiGLU) 18.3 / 19.6             512 x 2048 x 5632 38.6 / 43.9    768: 57.8 / 45.1
-#   bias:  19 x  768 x  768  3.5 / 15.6    512 x 2304 x 768 12.1 / 19.7    768 x 3072 x 768 18.6 / 23.5    2048: 48 / 24.7
+#    64 x  2048 x 2048  6.0 / 10.9    256 x 2048 x 2048  8.8 / 19.7    768 x 2048 x 2048 22.8 / 28.6   1024: 30.3 / 30.2
+#    64 x  2048 x 5632 12.0 / 14.5     64 x 10496 x 2048 14.3 / 18.3   120 x 4096 x 4096 15.5 / 18.1   192: 28.6 / 20.9
+#    64 x 11264 x 2048 (SwiGLU) 14.6 / 18.9             512 x 2048 x 5632 38.6 / 43.9    768: 57.8 / 45.1
+#   bias:  19 x  768 x  768  3.0 / 15.6    512 x 2304 x 768 12.1 / 19.7    768 x 3072 x 768 18.6 / 23.5    2048: 48 / 24.7
 # Widths that neither tiles (N no multiple of 192 or 256) go to the vendor's kernels, which split K for narrow outputs: fitted to
 # within 25 % for N 48 - 11,280, K 256 - 8,192, 17 - 1,024 rows, and taken 10 % lower, since an even choice is worth nothing (few-row / vendor):
 #    64 x  400 x 1024  4.2 / 6.7      64 x 2064 x 1024  5.5 / 8.8     512 x   48 x 8192 24.9 / 9.1     400 x 2064 x 1024 17.4 / 9.4
@@ -407,25 +409,21 @@ _ROWS_RULE: dict = {}
 def _rows_cost(M: int, N: int, K: int, epi: int):
     """(us of the few-row kernel, its ``wide`` argument, us of the other kernels), or None where it does not take the shape."""
     mt = (M + 15) // 16 if M <= 64 else 4 * ((M + 63) // 64)   # 16-row tiles of X
-    key = (mt, N, K, epi)
+    key = ((M + 15) // 16, N, K, epi)
     if key in _ROWS_RULE:
         return _ROWS_RULE[key]
     est = None
     if 1 <= M <= ROWS_MAX_M and (K <= 8192 or mt == 1) and lib().rows_supported(M, N, K, epi):
-        mb, rows, cus = N * K * 2 / 1e6, 16 * mt, device_cus()
+        mb, rows, cus, mt16 = N * K * 2 / 1e6, 16 * mt, device_cus(), (M + 15) // 16
 
-        def cost(nt, wide):
-            m = min(mt, 4) if not wide else (2 if mt <= 2 else 4)
-            wgs = -(-mt // 4) * (N // (16 * nt))
-            rounds = -(-wgs // cus)
-            return max(2.6 + rounds * (m + nt) * K / 32 / 58 + (rounds - 1), mb / 4.2)
+        def cost(nt):   # (the row tiles of a workgroup: as csrc/rows_gemm.hip takes them)
+            units, rounds = min((r * (m + nt), r) for m in range(1, min(mt16, 4) + 1) for r in [-(-(-(-mt16 // m) * (N // (16 * nt))) // cus)])
+            return max(2.6 + units * K / 32 / 58 + (rounds - 1), mb / 4.2)
 
-        if epi == 1:
-            t, wide = cost(2, False), False
-        else:
-            t, wide = cost(1, False), False
-            if N % 32 == 0 and cost(2, True) < t:
-                t, wide = cost(2, True), True
+        t, wide = (cost(2), False) if epi == 1 else (cost(1), False)
+        for nt, form in ((2, True), (4, 2)):
+            if N % (16 * nt) == 0 and (nt == 2 or N >= 3072) and not (nt == 2 and epi == 1) and cost(nt) < t:
+                t, wide = cost(nt), form
         if epi < 2 and rows <= 256:
             other = min(7.5, 2 + K / 340) + 0.14 * mb + rows / 22 + (3.5 if epi == 1 else 0)
         elif epi < 2:
@@ -890,7 +888,7 @@ def tune_decode(weights, ms: Sequence[int] = DECODE_TUNE_MS, iters: int = 3, col
                 best = min(med, key=med.get)
                 stay = next(iter(rows)) if est[0] < est[2] else min(arms, key=med.get)
                 pick = best if med[best] < 0.95 * med[stay] else stay
-                _ROWS_TABLE[key] = {"rows": False, "rows wide": True}.get(pick)
+                _ROWS_TABLE[key] = est[1] if pick in rows else None
                 out[key + ("few", "rows")] = {k: round(v, 1) for k, v in med.items()}
         del copies
     return out
