@@ -206,6 +206,43 @@ at::Tensor rows_linear(const at::Tensor& x, const at::Tensor& w, const c10::opti
   return out;
 }
 
+// (y, h): h = LN(s), y = act(h w^T + bias) in one launch
+std::tuple<at::Tensor, at::Tensor> ln_linear(const at::Tensor& s, const at::Tensor& ln_w, const at::Tensor& ln_b, double eps, const at::Tensor& w,
+                                             const at::Tensor& bias, bool gelu) {
+  CHECK_CUDA(s); CHECK_BF16(s); CHECK_LASTDIM(s); check_rows16(s, "rows");
+  TORCH_CHECK(s.dim() == 2, "rows [M, K]");
+  const int M = s.size(0), K = s.size(1), N = w.size(0);
+  for (const at::Tensor* t : {&ln_w, &ln_b, &w, &bias}) {
+    CHECK_CUDA((*t)); CHECK_BF16((*t)); CHECK_CONTIG((*t));
+    TORCH_CHECK(reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0, "weights must be 16-byte aligned");
+  }
+  TORCH_CHECK(w.dim() == 2 && w.size(1) == K && ln_w.numel() == K && ln_b.numel() == K && bias.numel() == N, "weight shapes");
+  TORCH_CHECK(lk_ln_rows_supported(M, N, K), "ln_linear: M in [1, 4096], K a multiple of 64 up to 768, N of 16");
+  at::Tensor y = at::empty({M, N}, s.options()), h = at::empty({M, K}, s.options());
+  CHECK_RC(lk_ln_rows(bp(s), s.stride(0), bp(ln_w), bp(ln_b), (float)eps, bp(h), bp(w), bp(bias), bp(y), M, N, K, gelu ? 1 : 0, cur_stream()),
+           "ln_linear");
+  return {y, h};
+}
+
+// attention of one text (rows [q | k | v], heads of 64), the projection behind it and the residual in one launch
+at::Tensor attn_linear(const at::Tensor& qkv, int64_t nh, double scale, const at::Tensor& w, const at::Tensor& bias, const at::Tensor& residual) {
+  CHECK_CUDA(qkv); CHECK_BF16(qkv); CHECK_LASTDIM(qkv); check_rows16(qkv, "qkv");
+  CHECK_CUDA(residual); CHECK_BF16(residual); CHECK_LASTDIM(residual);
+  for (const at::Tensor* t : {&w, &bias}) {
+    CHECK_CUDA((*t)); CHECK_BF16((*t)); CHECK_CONTIG((*t));
+    TORCH_CHECK(reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0, "weights must be 16-byte aligned");
+  }
+  TORCH_CHECK(qkv.dim() == 2 && w.dim() == 2, "qkv [M, 3 K], w [N, K]");
+  const int M = qkv.size(0), N = w.size(0);
+  TORCH_CHECK(nh >= 1 && qkv.size(1) == 3 * nh * 64 && w.size(1) == nh * 64 && bias.numel() == N, "attn_linear: shapes");
+  TORCH_CHECK(residual.dim() == 2 && residual.size(0) == M && residual.size(1) == N, "residual [M, N]");
+  TORCH_CHECK(lk_attn_rows_supported(M, (int)nh, N), "attn_linear: M in [1, 32], up to 12 heads of 64, N a multiple of 16");
+  at::Tensor y = at::empty({M, N}, qkv.options());
+  CHECK_RC(lk_attn_rows(bp(qkv), qkv.stride(0), (int)nh, (float)scale, bp(w), bp(bias), bp(residual), residual.stride(0), bp(y), M, N,
+                        cur_stream()), "attn_linear");
+  return y;
+}
+
 // Decode-step fusions (split-K weight-streaming GEMM whose reduction is done by the
 // consumer kernel): the partial slabs never become a bf16 tensor, one launch fewer each.
 namespace {
@@ -2266,6 +2303,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_linear", &skinny_linear, "", py::arg("x"), py::arg("w"), py::arg("swiglu") = false,
         py::arg("splits") = 0, py::arg("out") = py::none());
   m.def("skinny_splits", &skinny_splits);
+  m.def("ln_linear", &ln_linear);
+  m.def("ln_linear_supported", [](int64_t M, int64_t N, int64_t K) { return lk_ln_rows_supported((int)M, (int)N, (int)K); });
+  m.def("attn_linear", &attn_linear);
+  m.def("attn_linear_supported", [](int64_t M, int64_t nh, int64_t N) { return lk_attn_rows_supported((int)M, (int)nh, (int)N); });
   m.def("rows_linear", &rows_linear, py::arg("x"), py::arg("w"), py::arg("bias") = py::none(), py::arg("epi") = 0, py::arg("wide") = 0,
         py::arg("residual") = py::none());
   m.def("rows_supported", [](int64_t M, int64_t N, int64_t K, int64_t epi) { return lk_rows_gemm_supported((int)M, (int)N, (int)K, (int)epi); });

@@ -30,6 +30,12 @@ int lk_activation(bf16_t* x, const bf16_t* bias, long rows, int N, long xs, int 
                   hipStream_t st);
 
 // rows_gemm.hip (few rows, up to 4,096; one launch, every epilogue)
+bool lk_ln_rows_supported(int M, int N, int K);
+int lk_ln_rows(const void* s, long ss, const void* lw, const void* lb, float eps, void* h, const void* w, const void* b, void* y, int M, int N,
+               int K, int gelu, hipStream_t st);
+bool lk_attn_rows_supported(int M, int nh, int N);
+int lk_attn_rows(const void* qkv, long qs, int nh, float scale, const void* w, const void* b, const void* r, long rs, void* y, int M, int N,
+                 hipStream_t st);
 bool lk_rows_gemm_supported(int M, int N, int K, int epi);
 // epi: 0 none, 1 SwiGLU, 2 bias, 3 bias + GELU, 4 bias + ReLU, 5 bf16(bias) + the residual rows r (elsewhere null)
 int lk_rows_gemm(const void* x, const void* w, const void* b, const void* r, long ldr, void* y, int M, int N, int K, long ldx, long ldy, int epi,

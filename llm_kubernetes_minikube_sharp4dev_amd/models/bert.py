@@ -87,6 +87,8 @@ class EncoderModel(nn.Module):
         cfg, nh, D, H = self.cfg, self.nh, self.D, self.cfg.hidden
         h = ops.embed_layernorm(ids, None if cfg.rotary else positions, type_ids, self.tok, self.pos,
                                 self.typ, self.emb_ln_w, self.emb_ln_b, cfg.norm_eps)
+        if cfg.bias and cfg.activation == "gelu" and not cfg.rotary and ops.encoder_rows_ok(h, H, cfg.intermediate):
+            return self._few_rows(h, cu, lens_cpu, pool, out, tiles)
         for L in self.layers:
             qkv = ops.linear(h, L.qkv, L.qkv_b)
             if cfg.rotary:
@@ -101,6 +103,24 @@ class EncoderModel(nn.Module):
                 f = ops.linear(h, L.fc1, L.fc1_b, act="gelu")  # bias + GELU fused into the GEMM
             d = ops.linear(f, L.fc2, L.fc2_b)
             h = ops.layernorm(d, L.ln2_w, L.ln2_b, cfg.norm_eps, residual=h)
+        if not pool:
+            return h
+        return ops.pool_normalize(h, cu, 1 if cfg.pooling == "cls" else 0, cfg.normalize, out=out)
+
+    def _few_rows(self, h, cu, lens_cpu, pool, out, tiles):
+        """The layers with every norm inside the projection that reads it (and one text's attention inside its own)."""
+        cfg, prev, s = self.cfg, None, None
+        for L in self.layers:
+            if prev is None:
+                qkv = ops.linear(h, L.qkv, L.qkv_b)
+            else:
+                qkv, h = ops.ln_linear(s, prev.ln2_w, prev.ln2_b, cfg.norm_eps, L.qkv, L.qkv_b)
+            s = ops.attn_linear_add(qkv, cu, lens_cpu, self.nh, self.D, self.scale, L.o, L.o_b, h, tiles)
+            f, h = ops.ln_linear(s, L.ln1_w, L.ln1_b, cfg.norm_eps, L.fc1, L.fc1_b, act="gelu")
+            s = ops.linear_add(f, L.fc2, L.fc2_b, h)
+            prev = L
+        if prev is not None:
+            h = ops.layernorm(s, prev.ln2_w, prev.ln2_b, cfg.norm_eps)
         if not pool:
             return h
         return ops.pool_normalize(h, cu, 1 if cfg.pooling == "cls" else 0, cfg.normalize, out=out)

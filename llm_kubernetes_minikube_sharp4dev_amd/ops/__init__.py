@@ -935,6 +935,46 @@ def linear(x, w, b=None, act: Optional[str] = None):
     return y
 
 
+# Encoder passes of few rows: the layer norms and the attention run inside the projections behind them (csrc/encoder_rows.hip).  Up to
+# one row tile: a pass of bge-base, cold weights, 8 / 19 / 33 / 64 tokens 480 / 518 / 549 / 599 -> 360 / 410 / 469 / 527 us; 100 tokens
+# (two tiles, each normalised by all of its workgroups) took longer on the device than the norms apart.
+ENCODER_ROWS = 64
+
+
+def encoder_rows_ok(h, width: int, inner: int) -> bool:
+    """Whether :func:`ln_linear` takes these rows in the projections of an encoder layer (``width`` to 3 ``width`` and to ``inner``)."""
+    return (use_hip(h) and h.dtype == torch.bfloat16 and not GEMM_LIBRARY and 1 <= h.shape[0] <= ENCODER_ROWS
+            and all(lib().ln_linear_supported(h.shape[0], n, width) for n in (3 * width, inner)))
+
+
+def linear_add(x, w, b, residual):
+    """x w^T + b, then + residual (each rounded on its own, as the two operations apart round)."""
+    if use_hip(x) and b is not None:
+        est = _rows_cost(x.shape[0], w.shape[0], w.shape[1], 2) if _gemm_ok(x, w) and w.data_ptr() % 16 == 0 else None
+        if est is not None and not GEMM_LIBRARY:
+            return lib().rows_linear(x, w, b, 5, est[1], residual)
+    return linear(x, w, b) + residual
+
+
+def ln_linear(s, ln_w, ln_b, eps: float, w, b, act: Optional[str] = None):
+    """(act(h w^T + b), h) with h = LN(s); ``act``: None or "gelu"."""
+    if use_hip(s):
+        return lib().ln_linear(s, ln_w, ln_b, eps, w, b, act == "gelu")
+    h = layernorm(s, ln_w, ln_b, eps)
+    return linear(h, w, b, act=act), h
+
+
+def attn_linear_add(qkv, cu, lens_cpu, nh: int, head_dim: int, scale: float, w, b, residual, tiles=None):
+    """Bidirectional attention over packed rows [q | k | v], the projection of its output and the residual; one launch for one short
+    text."""
+    K = nh * head_dim
+    if (use_hip(qkv) and not GEMM_LIBRARY and head_dim == 64 and len(lens_cpu) == 1 and lens_cpu[0] == qkv.shape[0]
+            and lib().attn_linear_supported(qkv.shape[0], nh, w.shape[0])):
+        return lib().attn_linear(qkv, nh, scale, w, b, residual)
+    a = flash_prefill(qkv[:, :K], qkv[:, K:2 * K], qkv[:, 2 * K:], cu, nh, nh, head_dim, scale, False, q_lens_cpu=lens_cpu, tiles=tiles)
+    return linear_add(a, w, b, residual)
+
+
 def linear_swiglu(x, w_gate_up):
     """silu(x Wg^T) * (x Wu^T) for a fused [Wg; Wu] weight: one kernel (GEMM with the
     SwiGLU epilogue) in every regime."""
