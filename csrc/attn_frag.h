@@ -54,4 +54,23 @@ LK_DEVICE uint4_t frag(const T* r, int k, int K, bool vec) {
   return *reinterpret_cast<const uint4_t*>(tmp);
 }
 
+typedef void __attribute__((address_space(3))) * lds_void_ptr;
+
+// maximum over the four lane groups (lanes l, l ^ 16, l ^ 32, l ^ 48), in registers
+LK_DEVICE float max_groups(float v) {
+  // (the swapped pair is taken apart as integers: a bit cast of a vector's element reads element 0)
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  const unsigned a0 = a[0], a1 = a[1];
+  v = fmaxf(__uint_as_float(a0), __uint_as_float(a1));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  const unsigned b0 = b[0], b1 = b[1];
+  return fmaxf(__uint_as_float(b0), __uint_as_float(b1));
+}
+
+// one fragment: lane l's 16 bytes at src go to LDS byte off + 16 l (off wave-uniform).  As assembly: the compiler would wait for the
+// transfer before the next LDS read of the OTHER buffer; a kernel's loop waits for it itself, ahead of its barrier.
+LK_DEVICE void dma16(unsigned off, const void* src) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(off), "v"(src) : "memory", "m0");
+}
+
 }  // namespace

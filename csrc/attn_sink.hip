@@ -36,6 +36,7 @@
 #include "common.h"
 #include "kernels.h"
 #include "attn_frag.h"
+#include "attn_stage.h"
 
 namespace {
 
@@ -329,6 +330,114 @@ __global__ __launch_bounds__(256) void sinkattn_prefill_kernel(SinkParams p, con
   }
 }
 
+// ---- prefill, bf16, heads up to 128: keys and values staged in LDS (attn_stage.h).  4 prompts of 900 - 1,148 tokens, 16 heads of 128 over
+// 4 kv heads, window 512 and pooled blocks of 64: 113 us with the kernel above (one wave per tile), 48 us.  blockIdx.y walks the same list of 16-query tiles;
+// those that do not begin a workgroup's run of queries leave at once.  The running maximum (of scores times log2 e) moves only when a
+// score exceeds it by more than kDefer: until then weights are at most 2^kDefer, exact alike in bf16 and f32.
+constexpr float kDefer = 8.f, kLog2e = 1.4426950408889634f;
+
+template <int PAD>
+__global__ __launch_bounds__(256, 3) void sinkattn_stage_kernel(SinkParams p, int wh, int bs_shift, const int* __restrict__ cu_q,
+                                                                const int* __restrict__ ctx_lens, const int* __restrict__ tile_seq,
+                                                                const int* __restrict__ tile_q0, bf16_t* __restrict__ out, long os) {
+  constexpr int VT = PAD / 16;
+  extern __shared__ __attribute__((aligned(16))) bf16_t lds[];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n16 = lane & 15, g = lane >> 4;
+  const int b = tile_seq[blockIdx.y], q0 = tile_q0[blockIdx.y], rows = 16 * (4 / wh);
+  if (q0 % rows) return;   // the whole workgroup
+  const int rep = p.H / p.G, ngr = rep / wh, kvh = blockIdx.x / ngr, head = kvh * rep + blockIdx.x % ngr * wh + w % wh;
+  const int qbeg = cu_q[b], qlen = cu_q[b + 1] - qbeg, ctx = ctx_lens[b], past = ctx - qlen, qw = q0 + w / wh * 16, qi = qw + n16;
+  uint4_t qf[PAD / 32];
+  floatx4 o[VT];
+  float m = p.sink ? 0.f : kNegBig, l = 0.f;
+  int g0 = first_key(past + qw, p.mkind, p.msize) & ~31;   // first(i) never decreases with i
+  int g1 = qw < qlen ? min(ctx, past + qw + 16) : 0;       // (queries past the chunk's end see nothing)
+  stage_q<PAD>(reinterpret_cast<const bf16_t*>(p.q) + (long)(qbeg + min(qi, qlen - 1)) * p.qs + (long)head * p.dim, p.dim, qf);
+#pragma unroll
+  for (int vt = 0; vt < VT; ++vt) o[vt] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const float hs = p.hscale[head] * kLog2e, cs = p.cap > 0.f ? 2.f * hs / p.cap : 0.f, cap = p.cap * kLog2e;
+  int hi = past + qi, lo = first_key(hi, p.mkind, p.msize);   // this lane's column sees keys lo .. hi
+  auto weights = [&](int kb, const floatx4& s0, const floatx4& s1) {
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float s = e < 4 ? s0[e & 3] : s1[e & 3];
+      v[e] = p.cap > 0.f ? cap * (1.f - 2.f * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(s * cs))) : s * hs;
+    }
+    const int k = kb + 8 * g;
+    const bool edge = __any(hi < kb + 31 || lo > kb);
+    if (edge) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = k + e >= lo && k + e <= hi ? v[e] : kNegBig;
+    }
+    float mx = fmaxf(fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])), fmaxf(fmaxf(v[4], v[5]), fmaxf(v[6], v[7])));
+    mx = max_groups(mx);
+    const bool grow = mx > m + kDefer;
+    if (__any(grow)) {
+      const float mn = grow ? mx : m, alpha = __builtin_amdgcn_exp2f(m - mn);
+      m = mn;
+      l *= alpha;
+#pragma unroll
+      for (int vt = 0; vt < VT; ++vt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[vt][j] *= alpha;
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = __builtin_amdgcn_exp2f(v[e] - m);
+    if (edge) {   // (a column that has seen nothing yet would give its masked keys 2^0)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = k + e >= lo && k + e <= hi ? v[e] : 0.f;
+    }
+    uint4_t pk;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) l += v[e];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) pk[e] = pack_bf2(v[2 * e], v[2 * e + 1]);
+    return __builtin_bit_cast(short8, pk);
+  };
+  const int qlast = past + min(q0 + rows, qlen) - 1;   // the workgroup's last query
+  StageCache c = {reinterpret_cast<const bf16_t*>(p.kc), reinterpret_cast<const bf16_t*>(p.vc), p.bt + (long)b * p.bt_stride,
+                  p.G, kvh, p.dim, p.vdim, p.BS, bs_shift};
+  int k0 = first_key(past + q0, p.mkind, p.msize) & ~31, k1 = min(ctx, qlast + 1);
+  const bool pooled = p.pool > 0;
+  auto behind = [&](int q) { return pooled ? blocks_seen(q, p.msize, p.pool) : kept_keys(p, first_key(q, p.mkind, p.msize)); };
+  // the window (or chunk, or all), then what lies behind it: the pooled blocks, or (never both) the kept first positions
+#pragma unroll 1
+  for (int pass = 0;; ++pass) {
+    stage_walk<PAD>(c, lds, qf, k0, k1, g0, g1, o, weights);
+    if (pass || (!pooled && p.keep == 0)) break;
+    hi = behind(hi) - 1;
+    lo = 0;
+    g0 = 0;
+    g1 = g1 > 0 ? behind(g1 - 1) : 0;
+    if (pooled) {
+      c.kc = reinterpret_cast<const bf16_t*>(p.pkc);
+      c.vc = reinterpret_cast<const bf16_t*>(p.pvc);
+    }
+    k0 = 0;
+    k1 = behind(qlast);
+  }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (qi >= qlen) return;
+  const float den = l + (p.sink ? __builtin_amdgcn_exp2f(-m) : 0.f);
+  const float f = den > 0.f ? p.oscale * gate_of<bf16_t>(p, qbeg + qi, head) / den : 0.f;
+  bf16_t* orow = out + (long)(qbeg + qi) * os + (long)head * p.vdim;
+#pragma unroll
+  for (int vt = 0; vt < VT; ++vt) {
+    const int vd = vt * 16 + 4 * g;
+    if (vd < p.vdim) {   // (vdim is a multiple of 8)
+      float y[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) y[j] = o[vt][j] * f * gate_el<bf16_t>(p, qbeg + qi, head, vd + j);
+      uint2 pk;
+      pk.x = pack_bf2(y[0], y[1]);
+      pk.y = pack_bf2(y[2], y[3]);
+      *reinterpret_cast<uint2*>(orow + vd) = pk;
+    }
+  }
+}
+
 // ---- decode: workgroup = (sequence, up to 16 heads of one kv group, key split z) -----------------------
 // part: [B, H, Z, vdim + 2] f32 = O^T relative to m, then m, l
 template <typename T, int PAD>
@@ -520,6 +629,18 @@ int launch_prefill(const SinkParams& p, const int* cu_q, const int* ctx, const i
   return 0;
 }
 
+template <int PAD>
+int launch_stage(const SinkParams& p, const int* cu_q, const int* ctx, const int* ts, const int* tq, int ntiles, void* out, long os,
+                 hipStream_t st) {
+  if (ntiles > 65535) return -2;
+  const int wh = stage_heads(p.H / p.G), shift = (p.BS & (p.BS - 1)) == 0 ? __builtin_ctz(p.BS) : -1;
+  const dim3 grid(p.H / wh, ntiles);
+  LK_SET_MAX_LDS((sinkattn_stage_kernel<PAD>), stage_lds(PAD));
+  sinkattn_stage_kernel<PAD><<<grid, 256, stage_lds(PAD), st>>>(p, wh, shift, cu_q, ctx, ts, tq, (bf16_t*)out, os);
+  LK_CHECK_LAUNCH();
+  return 0;
+}
+
 template <typename T, int PAD>
 int launch_decode(const SinkParams& p, const int* ctx, int B, int Z, void* out, long os, float* part, hipStream_t st) {
   const int rep = p.H / p.G;
@@ -590,6 +711,14 @@ int lk_sinkattn_prefill(const void* q, long qs, const void* kc, const void* vc, 
   const SinkParams p = make_params(q, qs, kc, vc, bt, bt_stride, H, G, dim, vdim, BS, hscale, mkind, msize, sink, gate, gs, gcol, pkc, pvc,
                                    pool, keep, cap, gelem, oscale);
   if (!shape_ok(p, esz)) return -1;
+  const auto al = [](const void* x, int n) { return reinterpret_cast<uintptr_t>(x) % n == 0; };
+  if (esz == 2 && pad_of(dim, vdim) <= kStageMaxPad && qs % 8 == 0 && os % 4 == 0 && al(q, 16) && al(kc, 16) && al(vc, 16) && al(pkc, 16) &&
+      al(pvc, 16) && al(out, 8)) {
+    const int pad = pad_of(dim, vdim);
+    return pad == 64   ? launch_stage<64>(p, cu_q, ctx_lens, tile_seq, tile_q0, ntiles, out, os, st)
+           : pad == 96 ? launch_stage<96>(p, cu_q, ctx_lens, tile_seq, tile_q0, ntiles, out, os, st)
+                       : launch_stage<128>(p, cu_q, ctx_lens, tile_seq, tile_q0, ntiles, out, os, st);
+  }
   return esz == 2 ? prefill_t<bf16_t>(p, cu_q, ctx_lens, tile_seq, tile_q0, ntiles, out, os, st)
                   : prefill_t<float>(p, cu_q, ctx_lens, tile_seq, tile_q0, ntiles, out, os, st);
 }

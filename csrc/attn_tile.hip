@@ -25,8 +25,6 @@ constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kRows = 32;   // queries of a wave
 constexpr int CG = 2;       // column groups of 16 of a wave
 
-typedef void __attribute__((address_space(3))) * lds_void_ptr;
-
 struct TileParams {
   const bf16_t* q;
   long qs;
@@ -44,22 +42,6 @@ struct TileParams {
   long gs;
   int gcol;
 };
-
-// maximum over the four lane groups (lanes l, l ^ 16, l ^ 32, l ^ 48), in registers
-LK_DEVICE float max_groups(float v) {
-  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  const unsigned a0 = a[0], a1 = a[1];
-  v = fmaxf(__uint_as_float(a0), __uint_as_float(a1));
-  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  const unsigned b0 = b[0], b1 = b[1];
-  return fmaxf(__uint_as_float(b0), __uint_as_float(b1));
-}
-
-// one fragment: lane l's 16 bytes at src go to LDS byte off + 16 l (off wave-uniform).  As assembly: the compiler would wait for the
-// transfer before the next LDS read of the OTHER buffer; the loop below waits for it itself, ahead of its barrier.
-LK_DEVICE void dma16(unsigned off, const void* src) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(off), "v"(src) : "memory", "m0");
-}
 
 template <int KP, int VP, int NM, bool CAP>
 __global__ __launch_bounds__(256, (CG * NM * (VP / 16 + KP / 32) * 4 <= 160 ? 2 : 1)) void tile_attention_kernel(

@@ -29,7 +29,6 @@
 
 namespace {
 
-typedef __attribute__((address_space(3))) void* lds_void_ptr;
 typedef const __attribute__((address_space(1))) void* gbl_void_ptr;
 
 constexpr float kNegBig = -1e30f;
@@ -106,17 +105,6 @@ LK_DEVICE void static_for(F&& f) {
     f(std::integral_constant<int, I>{});
     static_for<N, I + 1>(f);
   }
-}
-
-// maximum over the four lane groups (lanes l, l ^ 16, l ^ 32, l ^ 48), in registers
-LK_DEVICE float max_groups(float v) {
-  // (the swapped pair is taken apart as integers: a bit cast of a vector's element reads element 0)
-  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  const unsigned a0 = a[0], a1 = a[1];
-  v = fmaxf(__uint_as_float(a0), __uint_as_float(a1));
-  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  const unsigned b0 = b[0], b1 = b[1];
-  return fmaxf(__uint_as_float(b0), __uint_as_float(b1));
 }
 
 template <int RP, int RDP, int CG, bool THIN>
