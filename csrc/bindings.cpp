@@ -4,6 +4,8 @@
 // reaches a kernel unchecked.  Kernels run on PyTorch's current HIP stream, so the
 // ops compose with torch.cuda.graphs (hipGraph capture) and stream semantics.
 #include <torch/extension.h>
+#include <ATen/core/CachingHostAllocator.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/hip/HIPStream.h>
 #include "kernels.h"
 
@@ -891,7 +893,7 @@ std::vector<at::Tensor> knn_topk(const at::Tensor& corpus, const at::Tensor& cno
 
 // The one-pass search with both results in one buffer, int32 [2, nq, K] (score bits, then row numbers), for a caller that copies
 // them to the host in one piece; an empty tensor where the one-pass search does not take the shape.
-at::Tensor knn_packed(const at::Tensor& corpus, const at::Tensor& cnorm, const at::Tensor& queries, int64_t K) {
+at::Tensor knn_packed(const at::Tensor& corpus, const at::Tensor& cnorm, const at::Tensor& queries, int64_t K, bool host) {
   CHECK_CUDA(corpus); CHECK_BF16(corpus); CHECK_CONTIG(corpus); CHECK_F32(cnorm); CHECK_CONTIG(cnorm);
   CHECK_CUDA(queries); CHECK_BF16(queries); CHECK_CONTIG(queries);
   TORCH_CHECK(corpus.dim() == 2 && queries.dim() == 2 && corpus.size(1) == queries.size(1), "dimension mismatch");
@@ -902,10 +904,14 @@ at::Tensor knn_packed(const at::Tensor& corpus, const at::Tensor& cnorm, const a
   const auto a16 = [](const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
   const int nb = K <= N && a16(corpus) && a16(queries) ? lk_knn_scan_blocks(N, D, nq, (int)std::min<int64_t>(K, 64)) : 0;
   if (!nb) return at::empty({0}, io);
-  at::Tensor out = at::empty({2, nq, K}, io), part = at::empty({2, nq, nb, K}, io);
+  // host: the merge writes the few hits straight into pinned memory (a copy behind it was one more launch in the caller's wait)
+  at::Tensor out = at::empty({2, nq, K}, host ? at::TensorOptions(at::kInt).pinned_memory(true) : io), part = at::empty({2, nq, nb, K}, io);
   int *o = out.data_ptr<int>(), *p = part.data_ptr<int>();
-  CHECK_RC(lk_knn_scan(bp(corpus), cnorm.data_ptr<float>(), N, D, bp(queries), nullptr, nq, (int)K, reinterpret_cast<float*>(p),
-                       p + (long)nq * nb * K, reinterpret_cast<float*>(o), o + (long)nq * K, cur_stream()), "knn_scan");
+  const int rc = lk_knn_scan(bp(corpus), cnorm.data_ptr<float>(), N, D, bp(queries), nullptr, nq, (int)K, reinterpret_cast<float*>(p),
+                             p + (long)nq * nb * K, reinterpret_cast<float*>(o), o + (long)nq * K, cur_stream());
+  if (host)   // the pinned block is not given out again before the stream has passed this point
+    at::getHostAllocator(at::kCUDA)->record_event(o, out.storage().data_ptr().get_context(), c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().unwrap());
+  CHECK_RC(rc, "knn_scan");
   return out;
 }
 
@@ -2383,7 +2389,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("flash_prefill", &flash_prefill, "", py::arg("q"), py::arg("k"), py::arg("v"), py::arg("block_tables"), py::arg("cu_q"), py::arg("ctx_lens"), py::arg("tile_seq"), py::arg("tile_q0"), py::arg("Hq"), py::arg("Hkv"), py::arg("D"), py::arg("scale"), py::arg("causal"), py::arg("out") = py::none(), py::arg("part_o") = py::none(), py::arg("part_ml") = py::none(), py::arg("q_past") = py::none());
   m.def("knn_topk", &knn_topk, "", py::arg("corpus"), py::arg("cnorm"), py::arg("queries"), py::arg("qnorm"),
         py::arg("K"), py::arg("force_fused") = false);
-  m.def("knn_packed", &knn_packed);
+  m.def("knn_packed", &knn_packed, "", py::arg("corpus"), py::arg("cnorm"), py::arg("queries"), py::arg("K"), py::arg("host") = false);
   m.def("knn_merge", &knn_merge);
   m.def("pool_normalize", &pool_normalize, "", py::arg("hidden"), py::arg("cu"), py::arg("mode"), py::arg("normalize"),
         py::arg("out") = py::none());

@@ -45,3 +45,19 @@ def test_index_search_agrees(hip):
     many, few = index.search_vectors(q, 6), [index.search_vectors(q[j:j + 1], 6)[0] for j in range(20)]
     assert [[i for i, _ in h] for h in many] == [[i for i, _ in h] for h in few]
     assert max(abs(a - b) for x, y in zip(many, few) for (_, a), (_, b) in zip(x, y)) <= 1e-6
+
+
+def test_hits_in_pinned_memory(hip):
+    """The form that leaves the hits on the host: the device form's, also when the result of a search before it was dropped unread."""
+    g = torch.Generator(device=DEV).manual_seed(4)
+    c = torch.randn(20011, 768, device=DEV, generator=g).to(torch.bfloat16)
+    cn = ops.row_norms(c)
+    for nq in (1, 5, 16):
+        q = torch.randn(nq, 768, device=DEV, generator=g).to(torch.bfloat16)
+        want = ops.knn_packed(c, cn, q, 5)
+        for _ in range(3):
+            ops.knn_packed(c, cn, q.flip(1).contiguous(), 5, host=True)
+            got = ops.knn_packed(c, cn, q, 5, host=True)
+            assert got.is_pinned() and not got.is_cuda
+            torch.cuda.current_stream().synchronize()
+            assert torch.equal(got, want.cpu())
