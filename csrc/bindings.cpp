@@ -208,6 +208,24 @@ at::Tensor rows_linear(const at::Tensor& x, const at::Tensor& w, const c10::opti
   return out;
 }
 
+// (x1 w1^T, x2 w2^T), two products of the same sizes in one launch
+std::tuple<at::Tensor, at::Tensor> rows_pair(const at::Tensor& x1, const at::Tensor& w1, const at::Tensor& x2, const at::Tensor& w2, int64_t wide) {
+  for (const at::Tensor* t : {&x1, &x2}) {
+    CHECK_CUDA((*t)); CHECK_BF16((*t)); CHECK_LASTDIM((*t)); check_rows16(*t, "x");
+  }
+  for (const at::Tensor* t : {&w1, &w2}) {
+    CHECK_CUDA((*t)); CHECK_BF16((*t)); CHECK_CONTIG((*t)); check_rows16(*t, "w");
+  }
+  TORCH_CHECK(x1.dim() == 2 && w1.dim() == 2 && x1.size(1) == w1.size(1) && x2.sizes() == x1.sizes() && w2.sizes() == w1.sizes(),
+              "rows_pair: x [M, K], w [N, K], both pairs alike");
+  const int M = x1.size(0), K = x1.size(1), N = w1.size(0);
+  TORCH_CHECK(lk_rows_gemm_supported(M, N, K, 0), "rows_pair: M in [1, 4096], K a multiple of 64, N of 16");
+  at::Tensor y1 = at::empty({M, N}, x1.options()), y2 = at::empty({M, N}, x1.options());
+  CHECK_RC(lk_rows_pair(bp(x1), x1.stride(0), bp(w1), bp(y1), bp(x2), x2.stride(0), bp(w2), bp(y2), M, N, K, (int)wide, cur_stream()),
+           "rows_pair");
+  return {y1, y2};
+}
+
 // (y, h): h = LN(s), y = act(h w^T + bias) in one launch
 std::tuple<at::Tensor, at::Tensor> ln_linear(const at::Tensor& s, const at::Tensor& ln_w, const at::Tensor& ln_b, double eps, const at::Tensor& w,
                                              const at::Tensor& bias, bool gelu) {
@@ -1742,17 +1760,30 @@ at::Tensor gemm_grouped(const at::Tensor& x, const at::Tensor& seg, const at::Te
 }
 
 // ids absent: the table has one row per token of the step (a router's choice)
-std::vector<at::Tensor> moe_route(const c10::optional<at::Tensor>& ids, const at::Tensor& table, int64_t E) {
-  CHECK_CUDA(table); CHECK_I32(table); CHECK_CONTIG(table);
+// seg [n, E + 1] and order [n, T * top] of n tables of the same sizes
+std::vector<at::Tensor> moe_routes(const c10::optional<at::Tensor>& ids, const std::vector<at::Tensor>& tables, int64_t E) {
   if (ids) { CHECK_CUDA(*ids); CHECK_I32(*ids); CHECK_CONTIG(*ids); }
-  TORCH_CHECK(table.dim() == 2 && E >= 1, "table must be int32 [vocab, top]");
-  const long T = ids ? ids->numel() : table.size(0);
-  const int top = table.size(1);
-  at::Tensor seg = at::empty({E + 1}, table.options());
-  at::Tensor order = at::empty({T * top}, table.options());
-  CHECK_RC(lk_moe_route(ipo(ids), ip(table), (int)table.size(0), top, (int)E, (int)T, seg.data_ptr<int>(), order.data_ptr<int>(),
+  const int n = tables.size();
+  TORCH_CHECK(n >= 1 && n <= kMaxRouteTables && E >= 1, "tables");
+  const int* ptr[kMaxRouteTables];
+  for (int i = 0; i < n; ++i) {
+    const at::Tensor& t = tables[i];
+    CHECK_CUDA(t); CHECK_I32(t); CHECK_CONTIG(t);
+    TORCH_CHECK(t.dim() == 2 && t.sizes() == tables[0].sizes(), "tables must be int32 [vocab, top], of the same sizes");
+    ptr[i] = ip(t);
+  }
+  const long T = ids ? ids->numel() : tables[0].size(0);
+  const int top = tables[0].size(1);
+  at::Tensor seg = at::empty({n, E + 1}, tables[0].options());
+  at::Tensor order = at::empty({n, T * top}, tables[0].options());
+  CHECK_RC(lk_moe_route(ipo(ids), ptr, n, (int)tables[0].size(0), top, (int)E, (int)T, seg.data_ptr<int>(), order.data_ptr<int>(),
                         cur_stream()), "moe_route");
   return {seg, order};
+}
+
+std::vector<at::Tensor> moe_route(const c10::optional<at::Tensor>& ids, const at::Tensor& table, int64_t E) {
+  const auto r = moe_routes(ids, {table}, E);
+  return {r[0][0], r[1][0]};
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -2241,6 +2272,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rot_kv_write", &rot_kv_write);
   m.def("pool_kv_write", &pool_kv_write);
   m.def("moe_route", &moe_route);
+  m.def("moe_routes", &moe_routes);
   m.def("stream_parallel_norm", &stream_parallel_norm);
   m.def("router_topk", &router_topk);
   m.def("clamped_glu", &clamped_glu);
@@ -2309,6 +2341,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_linear", &skinny_linear, "", py::arg("x"), py::arg("w"), py::arg("swiglu") = false,
         py::arg("splits") = 0, py::arg("out") = py::none());
   m.def("skinny_splits", &skinny_splits);
+  m.def("rows_pair", &rows_pair);
   m.def("ln_linear", &ln_linear);
   m.def("ln_linear_supported", [](int64_t M, int64_t N, int64_t K) { return lk_ln_rows_supported((int)M, (int)N, (int)K); });
   m.def("attn_linear", &attn_linear);

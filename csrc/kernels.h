@@ -36,6 +36,8 @@ int lk_ln_rows(const void* s, long ss, const void* lw, const void* lb, float eps
 bool lk_attn_rows_supported(int M, int nh, int N);
 int lk_attn_rows(const void* qkv, long qs, int nh, float scale, const void* w, const void* b, const void* r, long rs, void* y, int M, int N,
                  hipStream_t st);
+int lk_rows_pair(const void* x1, long ldx1, const void* w1, void* y1, const void* x2, long ldx2, const void* w2, void* y2, int M, int N, int K,
+                 int wide, hipStream_t st);
 bool lk_rows_gemm_supported(int M, int N, int K, int epi);
 // epi: 0 none, 1 SwiGLU, 2 bias, 3 bias + GELU, 4 bias + ReLU, 5 bf16(bias) + the residual rows r (elsewhere null)
 int lk_rows_gemm(const void* x, const void* w, const void* b, const void* r, long ldr, void* y, int M, int N, int K, long ldx, long ldy, int epi,
@@ -351,7 +353,8 @@ int lk_silu_(void* x, long xs, long rows, int n, int esz, hipStream_t st);
 int lk_sigmoid_mul_(void* x, long xs, const void* g, long gs, long rows, int n, int esz, hipStream_t st);
 
 // csrc/moe.hip: experts chosen by a table of token ids: pairs sorted by expert on the device, grouped MFMA products
-int lk_moe_route(const int* ids, const int* table, int vocab, int top, int E, int T, int* seg, int* order, hipStream_t st);
+constexpr int kMaxRouteTables = 64;
+int lk_moe_route(const int* ids, const int* const* tables, int n, int vocab, int top, int E, int T, int* seg, int* order, hipStream_t st);
 int lk_moe_gemm(const void* x, long xs, const int* order, const int* seg, int E, int top, long pairs, const void* w, int N, int K,
                 int act, void* out, long os, int esz, hipStream_t st);
 

@@ -43,10 +43,18 @@ LK_DEVICE int wave_sums(int v) {
   return v;
 }
 
+struct RouteTables {
+  const int* t[kMaxRouteTables];
+};
+
+// one workgroup per table (the layers of a model whose tables are indexed by the token ids know their routing at the step's start)
 template <int U>
-__global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(const int* __restrict__ ids, const int* __restrict__ table, int vocab,
+__global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(const int* __restrict__ ids, RouteTables tables, int vocab,
                                                                   int top, int E, int T, int* __restrict__ seg,
                                                                   int* __restrict__ order) {
+  const int* __restrict__ table = tables.t[blockIdx.x];
+  seg += (long)blockIdx.x * (E + 1);
+  order += (long)blockIdx.x * T * top;
   __shared__ int cnt[kMaxExperts];
   __shared__ int nxt[kMaxExperts];
   const int n = T * top, tid = threadIdx.x;
@@ -455,11 +463,14 @@ int moe_gemm_t(const void* x, long xs, const int* order, const int* seg, int E, 
 
 }  // namespace
 
-int lk_moe_route(const int* ids, const int* table, int vocab, int top, int E, int T, int* seg, int* order, hipStream_t st) {
+// seg [tables][E + 1], order [tables][T * top]
+int lk_moe_route(const int* ids, const int* const* tables, int n, int vocab, int top, int E, int T, int* seg, int* order, hipStream_t st) {
   if (T <= 0) return 0;
-  if (E < 1 || E > kMaxExperts || top < 1 || vocab < 1) return -1;
-  if ((long)T * top <= kRouteThreads) moe_route_kernel<1><<<1, kRouteThreads, 0, st>>>(ids, table, vocab, top, E, T, seg, order);
-  else moe_route_kernel<kRouteU><<<1, kRouteThreads, 0, st>>>(ids, table, vocab, top, E, T, seg, order);
+  if (E < 1 || E > kMaxExperts || top < 1 || vocab < 1 || n < 1 || n > kMaxRouteTables) return -1;
+  RouteTables rt = {};
+  for (int i = 0; i < n; ++i) rt.t[i] = tables[i];
+  if ((long)T * top <= kRouteThreads) moe_route_kernel<1><<<n, kRouteThreads, 0, st>>>(ids, rt, vocab, top, E, T, seg, order);
+  else moe_route_kernel<kRouteU><<<n, kRouteThreads, 0, st>>>(ids, rt, vocab, top, E, T, seg, order);
   LK_CHECK_LAUNCH();
   return 0;
 }

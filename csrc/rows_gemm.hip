@@ -24,17 +24,15 @@ namespace {
 enum { RG_NONE = 0, RG_SWIGLU = 1, RG_BIAS = 2, RG_GELU = 3, RG_RELU = 4, RG_ADD = 5 };
 
 template <int MT, int NT, int NS, int EPI>
-__global__ __launch_bounds__(64 * kRgWaves, 1) void rows_gemm_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
-                                                                     const bf16_t* __restrict__ bias, const bf16_t* __restrict__ R,
-                                                                     long ldr, bf16_t* __restrict__ Y, int M, int N, int K, long ldx,
-                                                                     long ldy) {
+LK_DEVICE void rows_tile(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W, const bf16_t* __restrict__ bias,
+                         const bf16_t* __restrict__ R, long ldr, bf16_t* __restrict__ Y, int M, int N, int K, long ldx, long ldy, int cz) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int all = K / 64, first = wave * all / kRgWaves, nst = (wave + 1) * all / kRgWaves - first;  // stages of this wave
-  // grid (8 XCDs, row tiles, column tiles / 8): the row tiles of a column tile follow one another on one XCD, whose L2 then has the
+  // (8 XCDs, row tiles, column tiles / 8): the row tiles of a column tile follow one another on one XCD, whose L2 then has the
   // weight rows
   const int cols = EPI == RG_SWIGLU ? N / 2 : N;
-  const int n0 = (blockIdx.z * 8 + blockIdx.x) * (EPI == RG_SWIGLU ? 8 * NT : 16 * NT), m0 = blockIdx.y * (16 * MT);  // first output column and row
+  const int n0 = (cz * 8 + blockIdx.x) * (EPI == RG_SWIGLU ? 8 * NT : 16 * NT), m0 = blockIdx.y * (16 * MT);  // first output column and row
   if (n0 >= cols) return;   // the whole workgroup: the grid holds whole eights of column tiles
   X += (long)m0 * ldx;
   Y += (long)m0 * ldy;
@@ -81,9 +79,30 @@ __global__ __launch_bounds__(64 * kRgWaves, 1) void rows_gemm_kernel(const bf16_
   });
 }
 
+template <int MT, int NT, int NS, int EPI>
+__global__ __launch_bounds__(64 * kRgWaves, 1) void rows_gemm_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
+                                                                     const bf16_t* __restrict__ bias, const bf16_t* __restrict__ R,
+                                                                     long ldr, bf16_t* __restrict__ Y, int M, int N, int K, long ldx,
+                                                                     long ldy) {
+  rows_tile<MT, NT, NS, EPI>(X, W, bias, R, ldr, Y, M, N, K, ldx, ldy, blockIdx.z);
+}
+
+// two plain products of the same sizes, the second in the upper half of the grid's z
+template <int MT, int NT, int NS>
+__global__ __launch_bounds__(64 * kRgWaves, 1) void rows_pair_kernel(const bf16_t* __restrict__ X1, long ldx1, const bf16_t* __restrict__ W1,
+                                                                     bf16_t* __restrict__ Y1, const bf16_t* __restrict__ X2, long ldx2,
+                                                                     const bf16_t* __restrict__ W2, bf16_t* __restrict__ Y2, int M, int N,
+                                                                     int K) {
+  const int half = gridDim.z >> 1, z = blockIdx.z;
+  const bool up = z >= half;
+  rows_tile<MT, NT, NS, RG_NONE>(up ? X2 : X1, up ? W2 : W1, nullptr, nullptr, 0, up ? Y2 : Y1, M, N, K, up ? ldx2 : ldx1, N, up ? z - half : z);
+}
+
+constexpr int ring_stages(int MT, int NT) { return 20 / (MT + NT) > 5 ? 5 : 20 / (MT + NT); }   // as many as 160 KB hold
+
 template <int MT, int NT, int EPI>
 int launch(const void* x, const void* w, const void* b, const void* r, long ldr, void* y, int M, int N, int K, long ldx, long ldy, hipStream_t st) {
-  constexpr int NS0 = 20 / (MT + NT), NS = NS0 > 5 ? 5 : NS0, lds = rg_lds(MT, NT, NS);   // stages: as many as 160 KB hold
+  constexpr int NS = ring_stages(MT, NT), lds = rg_lds(MT, NT, NS);
   LK_SET_MAX_LDS((rows_gemm_kernel<MT, NT, NS, EPI>), lds);
   const int cols = N / (16 * NT), tiles = (M + 16 * MT - 1) / (16 * MT);
   rows_gemm_kernel<MT, NT, NS, EPI><<<dim3(8, tiles, (cols + 7) / 8), 64 * kRgWaves, lds, st>>>(
@@ -138,6 +157,29 @@ int by_cols(const void* x, const void* w, const void* b, const void* r, long ldr
   }
 }
 
+template <int MT, int NT>
+int launch_pair(const void* x1, long ldx1, const void* w1, void* y1, const void* x2, long ldx2, const void* w2, void* y2, int M, int N, int K,
+                hipStream_t st) {
+  constexpr int NS = ring_stages(MT, NT), lds = rg_lds(MT, NT, NS);
+  LK_SET_MAX_LDS((rows_pair_kernel<MT, NT, NS>), lds);
+  const int cols = N / (16 * NT), tiles = (M + 16 * MT - 1) / (16 * MT);
+  rows_pair_kernel<MT, NT, NS><<<dim3(8, tiles, (cols + 7) / 8 * 2), 64 * kRgWaves, lds, st>>>(
+      (const bf16_t*)x1, ldx1, (const bf16_t*)w1, (bf16_t*)y1, (const bf16_t*)x2, ldx2, (const bf16_t*)w2, (bf16_t*)y2, M, N, K);
+  LK_CHECK_LAUNCH();
+  return 0;
+}
+
+template <int NT>
+int pair_by_rows(const void* x1, long ldx1, const void* w1, void* y1, const void* x2, long ldx2, const void* w2, void* y2, int M, int N, int K,
+                 hipStream_t st) {
+  switch (row_tiles(M, 2 * (N / (16 * NT)), NT)) {
+    case 1: return launch_pair<1, NT>(x1, ldx1, w1, y1, x2, ldx2, w2, y2, M, N, K, st);
+    case 2: return launch_pair<2, NT>(x1, ldx1, w1, y1, x2, ldx2, w2, y2, M, N, K, st);
+    case 3: return launch_pair<3, NT>(x1, ldx1, w1, y1, x2, ldx2, w2, y2, M, N, K, st);
+    default: return launch_pair<4, NT>(x1, ldx1, w1, y1, x2, ldx2, w2, y2, M, N, K, st);
+  }
+}
+
 }  // namespace
 
 // (the epilogue stores 8-byte groups of 4 columns: ldy is a multiple of 4, y 8-byte aligned)
@@ -157,4 +199,14 @@ int lk_rows_gemm(const void* x, const void* w, const void* b, const void* r, lon
     case RG_ADD: return by_cols<RG_ADD>(x, w, b, r, ldr, y, M, N, K, ldx, ldy, wide, st);
     default: return -1;
   }
+}
+
+// y1 = x1 w1^T and y2 = x2 w2^T of the same sizes in one launch (outputs contiguous).  A product of a few rows is mostly its launch and
+// its first loads: 64 x 2048 x 2048 is 6.1 us in a decode step, two of them here 8.7 us, and a launch's gap less.
+int lk_rows_pair(const void* x1, long ldx1, const void* w1, void* y1, const void* x2, long ldx2, const void* w2, void* y2, int M, int N, int K,
+                 int wide, hipStream_t st) {
+  if (!lk_rows_gemm_supported(M, N, K, RG_NONE)) return -1;
+  if (wide == 2 && N % 64 == 0) return pair_by_rows<4>(x1, ldx1, w1, y1, x2, ldx2, w2, y2, M, N, K, st);
+  if (wide && N % 32 == 0) return pair_by_rows<2>(x1, ldx1, w1, y1, x2, ldx2, w2, y2, M, N, K, st);
+  return pair_by_rows<1>(x1, ldx1, w1, y1, x2, ldx2, w2, y2, M, N, K, st);
 }

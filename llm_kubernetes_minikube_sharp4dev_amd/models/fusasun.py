@@ -331,18 +331,33 @@ class FusasunModel(nn.Module):
         return self.cache_block_bytes(1)
 
     # ------------------------------------------------------------------ forward
-    def _mixer(self, L: FusasunLayer, h, meta: AttnMeta, cache):
+    def _attended(self, L: FusasunLayer, h, meta: AttnMeta, cache):
+        """The mixer's heads, before its output projection."""
         W = self.cfg.hidden
         hc = ops.conv_silu(h, 0, W, L.canon, None, cache[-1], meta.seq_cu, meta.state_slots, meta.positions, meta.max_seq_len,
                            act=False)
         M = L.mix
         u = ops.linear(hc, M.w_in)
         if L.type == "attention":
-            att = pooled_window_attention(u, cache, meta, M.spec, M.freq, M.hscale)
-        else:
-            att = latent_window_attention(u, M.rows, M.up_rows.off["uv"], M.w_uq, M.w_ukv, M.dq_norm, M.dkv_norm, cache, meta, M.spec, M.freq,
-                                          M.hscale, self.cfg.norm_eps, w_heads=M.w_heads)
-        return ops.linear(att, M.o)
+            return pooled_window_attention(u, cache, meta, M.spec, M.freq, M.hscale)
+        return latent_window_attention(u, M.rows, M.up_rows.off["uv"], M.w_uq, M.w_ukv, M.dq_norm, M.dkv_norm, cache, meta, M.spec, M.freq,
+                                       M.hscale, self.cfg.norm_eps, w_heads=M.w_heads)
+
+    def _mixer(self, L: FusasunLayer, h, meta: AttnMeta, cache):
+        return ops.linear(self._attended(L, h, meta, cache), L.mix.o)
+
+    def _routes(self, ids) -> list:
+        """Every layer's expert routing (None: no experts), known from the token ids."""
+        out = [None] * len(self.layers)
+        if self.embed.is_cuda:
+            groups = {}
+            for i, L in enumerate(self.layers):
+                if L.mlp is not None:
+                    groups.setdefault((L.mlp.gate_up.shape[0], tuple(L.mlp.table.shape)), []).append(i)
+            for (experts, _), at in groups.items():
+                for i, r in zip(at, ops.moe_routes(ids, [self.layers[i].mlp.table for i in at], experts)):
+                    out[i] = r
+        return out
 
     def forward(self, ids: torch.Tensor, meta: AttnMeta, caches, taps: list = None) -> torch.Tensor:
         """-> normed hidden rows [R, W] that feed the LM head (``meta.logits_idx``, or every row).
@@ -351,16 +366,16 @@ class FusasunModel(nn.Module):
         eps = cfg.norm_eps
         x, _ = ops.embed_stream(ids, self.embed, self.dtype, cfg.embed_scale)
         h = ops.stream_rmsnorm(x, w=self.layers[0].norm1, eps=eps, out_dtype=self.dtype)
-        n = len(self.layers)
+        n, routes = len(self.layers), self._routes(ids)
         for i, L in enumerate(self.layers):
-            g = ops.linear(h, L.rg1)
-            y = self._mixer(L, h, meta, caches[i])
+            # the first gate reads h and is as large as the output projection: one launch for both
+            g, y = ops.linear_pair(h, L.rg1, self._attended(L, h, meta, caches[i]), L.mix.o)
             nxt = L.norm2 if L.mlp is not None else (self.layers[i + 1].norm1 if i + 1 < n else None)
             h = ops.stream_gated_norm(x, y, g, L.rg1_b, L.norm1b, nxt, eps, self.dtype)
             if L.mlp is not None:
                 X = L.mlp
                 g = ops.linear(h, L.rg2)
-                y = ops.table_experts(h, ids, X.table, X.gate_up, X.down, X.top)
+                y = ops.table_experts(h, ids, X.table, X.gate_up, X.down, X.top, routes[i])
                 nxt = self.layers[i + 1].norm1 if i + 1 < n else None
                 h = ops.stream_gated_norm(x, y, g, L.rg2_b, L.norm2b, nxt, eps, self.dtype, parts=X.top)
             if taps is not None:

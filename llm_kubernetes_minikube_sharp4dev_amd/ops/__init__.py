@@ -20,7 +20,7 @@ from .mixers import (conv_silu, embed_pos, gated_group_rmsnorm, linear_swiglu_an
                      softcap, ssm_scan, stream_rmsnorm, unitnorm_kv_write, embed_stream, stream_layernorm, gelu_tanh_mul,
                      dual_rmsnorm_mean, normrope_kv_write, sink_attention_prefill, sink_attention_decode, mask_first_key,
                      pooled_blocks_seen, stream_sandwich_layernorm, MASK_CAUSAL, MASK_CHUNK, MASK_WINDOW, SIG_TILE_ROWS)
-from .window import moe_route, pool_kv_write, rms_cols, rot_kv_write, run_experts, stream_gated_norm, table_experts  # noqa: F401
+from .window import moe_route, moe_routes, pool_kv_write, rms_cols, rot_kv_write, run_experts, stream_gated_norm, table_experts  # noqa: F401
 from .routed import clamped_glu, routed_experts, router_topk, sigmoid_mul_, silu_, stream_parallel_norm  # noqa: F401
 from .hyper import (GROUP_MAX, GROUP_TOP2, MAX_STREAMS, SCORE_SIGMOID, SCORE_SOFTMAX, gate_proj, relu_sq_, router_choice,  # noqa: F401
                     stream_hyper_norm)
@@ -440,8 +440,8 @@ def _rows_cost(M: int, N: int, K: int, epi: int):
     return est
 
 
-def _rows_rule(M: int, N: int, K: int, epi: int) -> Optional[bool]:
-    """None: not the few-row kernel; else its ``wide`` argument."""
+def _rows_rule(M: int, N: int, K: int, epi: int) -> Optional[int]:
+    """None: not the few-row kernel; else its ``wide`` argument (False, True or 2)."""
     est = _rows_cost(M, N, K, epi)
     return est[1] if est is not None and est[0] < est[2] else None
 
@@ -451,7 +451,7 @@ def _rows_rule(M: int, N: int, K: int, epi: int) -> Optional[bool]:
 _ROWS_TABLE: dict = {}
 
 
-def _rows_choice(M: int, N: int, K: int, epi: int) -> Optional[bool]:
+def _rows_choice(M: int, N: int, K: int, epi: int) -> Optional[int]:
     if epi < 2 and M > LM_HEAD_SKINNY_MAX_M and _ROWS_TABLE:
         key = (_decode_bucket(M), N, K, epi == 1)
         if key in _ROWS_TABLE:
@@ -934,6 +934,18 @@ def linear(x, w, b=None, act: Optional[str] = None):
     if y is None:
         y = _library(x, w, b, act, (x.shape[0] > WS_MAX_M, w.shape[0], w.shape[1], epi))
     return y
+
+
+def linear_pair(x1, w1, x2, w2):
+    """(x1 w1^T, x2 w2^T) of two products of the same sizes: one launch where both are the few-row kernel's."""
+    if use_hip(x1) and x1.dim() == 2 and x1.shape == x2.shape and w1.shape == w2.shape and not _gemv_ok(x1, w1, 0):
+        M, (N, K) = x1.shape[0], w1.shape
+        if (SKINNY_MAX_M < M <= (WS_MAX_M if GEMM_LIBRARY else ROWS_MAX_M) and _gemm_ok(x1, w1) and _gemm_ok(x2, w2)
+                and w1.data_ptr() % 16 == 0 and w2.data_ptr() % 16 == 0):
+            wide = _rows_choice(M, N, K, 0)
+            if wide is not None:
+                return lib().rows_pair(x1, w1, x2, w2, wide)
+    return linear(x1, w1), linear(x2, w2)
 
 
 # Encoder passes of few rows: the layer norms and the attention run inside the projections behind them (csrc/encoder_rows.hip).  Up to

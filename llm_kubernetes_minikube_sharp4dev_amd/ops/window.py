@@ -25,7 +25,7 @@ from ._ext import lib, use_hip
 GROUPED_DENSE_MIN_ROWS = 128
 GROUPED_FINE_MIN_ROWS = 64
 
-__all__ = ["stream_gated_norm", "rms_cols", "rot_kv_write", "pool_kv_write", "table_experts", "run_experts", "moe_route"]
+__all__ = ["stream_gated_norm", "rms_cols", "rot_kv_write", "pool_kv_write", "table_experts", "run_experts", "moe_route", "moe_routes"]
 
 
 def stream_gated_norm(x, y, g, g_bias, w_post, w_next, eps: float, out_dtype=torch.bfloat16, parts: int = 1):
@@ -145,13 +145,25 @@ def moe_route(ids, table, experts: int):
     return seg, order
 
 
-def table_experts(h, ids, table, w_gate_up, w_down, top: int):
+def moe_routes(ids, tables, experts: int) -> list:
+    """:func:`moe_route` of several layers' tables of the same sizes, [(seg, order)] in their order: on the GPU one launch per
+    64 of them (8 layers, 64 tokens x 2 of 16 experts: 8 launches of 4.5 us behind each other before)."""
+    if tables and use_hip(tables[0]):
+        out = []
+        for a in range(0, len(tables), 64):
+            seg, order = lib().moe_routes(ids, list(tables[a:a + 64]), int(experts))
+            out += list(zip(seg.unbind(0), order.unbind(0)))
+        return out
+    return [moe_route(ids, t, experts) for t in tables]
+
+
+def table_experts(h, ids, table, w_gate_up, w_down, top: int, route=None):
     """Feed-forward of table-routed experts: token t runs the experts ``table[ids[t]]`` (int32 [vocab, top]),
     each ``W_down (silu(W_gate h) * (W_up h))``.  ``w_gate_up`` [E, 2 * ffp, W] (gate rows, then up rows, each
     padded with zero rows to ffp), ``w_down`` [E, W, ffp].  Returns the experts' results un-summed,
     [T * top, W] in h's dtype with a token's ``top`` rows adjacent: the consumer averages them in f32
-    (``stream_gated_norm(parts=top)``)."""
-    return run_experts(h, ids, table, w_gate_up, w_down, top)
+    (``stream_gated_norm(parts=top)``).  ``route``: :func:`moe_route`'s result for these ids and this table."""
+    return run_experts(h, ids, table, w_gate_up, w_down, top, route)
 
 
 def _grouped(T: int, pairs: int, E: int, W: int, ffp: int) -> bool:
@@ -164,13 +176,13 @@ def _grouped(T: int, pairs: int, E: int, W: int, ffp: int) -> bool:
             and lib().gemm_grouped_fine(pairs, pairs, W, ffp, False))
 
 
-def run_experts(h, ids, table, w_gate_up, w_down, top: int):
+def run_experts(h, ids, table, w_gate_up, w_down, top: int, route=None):
     """The expert products behind ``table_experts`` (``ids`` int32 [T] index the table's rows) and
     ``routed_experts`` (``ids`` None: ``table`` int32 [T, top] holds each row's own choice)."""
     T, W = h.shape
     E, ffp = w_gate_up.shape[0], w_down.shape[2]
     if use_hip(h):
-        seg, order = moe_route(ids, table, E)
+        seg, order = route if route is not None else moe_route(ids, table, E)
         if h.dtype == torch.bfloat16 and _grouped(T, T * top, E, W, ffp):
             # prompt-sized steps on the framework's dense GEMM tiles, one GEMM per expert inside one launch: the first
             # product reads each pair's token row in place, the second writes each result into its pair's row

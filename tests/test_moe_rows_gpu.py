@@ -76,3 +76,43 @@ def test_route_to_the_grouped_product(monkeypatch, T, dense):
         want[p] = dn[e].double() @ mid
     # the result's rounding, and the middle's where its f32 value fell on the other side of a rounding boundary (2^-8 of single terms)
     assert float((got - want).norm() / want.norm()) < 2 ** -8
+
+
+@pytest.mark.parametrize("T,top,E,n", [(1, 1, 1, 1), (64, 2, 16, 8), (513, 2, 16, 3), (700, 3, 40, 65)])
+def test_routes_of_several_layers(hip, T, top, E, n):
+    """One launch for all tables sorts each as a launch for it alone (the order inside an expert's segment is free)."""
+    g = torch.Generator().manual_seed(T)
+    tables = [torch.randint(0, E, (50, top), generator=g, dtype=torch.int32).cuda() for _ in range(n)]
+    ids = torch.randint(0, 50, (T,), generator=g, dtype=torch.int32).cuda()
+    got = ops.moe_routes(ids, tables, E)
+    assert len(got) == n
+    for t, (seg, order) in zip(tables, got):
+        want, worder = ops.moe_route(ids, t, E)
+        assert torch.equal(seg, want)
+        for e in range(E):
+            a, b = int(seg[e]), int(seg[e + 1])
+            assert torch.equal(order[a:b].sort().values, worder[a:b].sort().values)
+
+
+@pytest.mark.parametrize("dim,vdim,P,BS", [(128, 128, 64, 16), (72, 40, 8, 16), (64, 96, 24, 48), (256, 8, 32, 32), (16, 200, 64, 128)])
+def test_pooled_means(hip, dim, vdim, P, BS):
+    """Blocks that end in the step, of sequences with and without a past, against the f32 means."""
+    G, lens = 2, [(5 * P, 5 * P), (3, 2 * P), (1, P - 1), (P + 1, 3 * P + 1), (1, 4 * P)]
+    g = torch.Generator().manual_seed(dim)
+    nb = [-(-c // BS) for _, c in lens]
+    bt = torch.zeros(len(lens), max(nb), dtype=torch.int32)
+    perm, at = torch.randperm(sum(nb), generator=g).to(torch.int32), 0
+    for s, n in enumerate(nb):
+        bt[s, :n] = perm[at:at + n]
+        at += n
+    kc, vc = torch.randn(sum(nb), G, BS, dim, generator=g).bfloat16(), torch.randn(sum(nb), G, vdim, BS, generator=g).bfloat16()
+    cu = torch.tensor([0] + [n for n, _ in lens]).cumsum(0).to(torch.int32)
+    ctx = torch.tensor([c for _, c in lens], dtype=torch.int32)
+    slots = torch.zeros(int(cu[-1]), dtype=torch.int32)
+    out = []
+    for dev in ("cpu", "cuda"):
+        pk, pv = torch.zeros_like(kc).to(dev), torch.zeros_like(vc).to(dev)
+        ops.pool_kv_write(kc.to(dev), vc.to(dev), pk, pv, P, bt.to(dev), ctx.to(dev), cu.to(dev), slots.to(dev), 0, max(n for n, _ in lens))
+        out.append((pk.cpu().float(), pv.cpu().float()))
+    for a, b in zip(*out):   # f32 means in another order may round to the other neighbour: one bf16 step
+        assert ((a - b).abs() <= 2.0 ** -7 * a.abs() + 1e-6).all() and ((a != 0) == (b != 0)).all()

@@ -24,3 +24,13 @@ def test_64_columns_per_workgroup(hip, M, N, K, epi):
     x, w = _r(g, M, K), _r(g, N, K, scale=K ** -0.5)
     b = _r(g, N) if epi >= 2 else None
     assert torch.equal(hip.rows_linear(x, w, b, epi, 2), hip.rows_linear(x, w, b, epi, 0))
+
+
+@pytest.mark.parametrize("wide", [0, 1, 2])
+@pytest.mark.parametrize("M,N,K", [(1, 16, 64), (17, 128, 128), (64, 2048, 2048), (65, 192, 832)])
+def test_two_products_in_one_launch(hip, M, N, K, wide):
+    g = torch.Generator("cuda").manual_seed(M)
+    x1, x2 = _r(g, M, K), _r(g, M, K + 8)[:, :K]
+    w1, w2 = _r(g, N, K, scale=K ** -0.5), _r(g, N, K, scale=K ** -0.5)
+    y1, y2 = hip.rows_pair(x1, w1, x2, w2, wide)
+    assert torch.equal(y1, hip.rows_linear(x1, w1, None, 0, wide)) and torch.equal(y2, hip.rows_linear(x2, w2, None, 0, wide))
