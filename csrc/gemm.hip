@@ -925,13 +925,16 @@ int launch_grouped(const bf16_t* x, long ldx, const bf16_t* w, const int* seg, i
 
 int cu_count();
 
-// Row tile of the grouped form: 256 (gemm_grouped_kernel) or 192 / 128 rows (gemm1w.hip's).  The experts' counts are on the device, so
+// Row tile of the grouped form in gemm1w.hip: 256, 192 or 128 rows.  The experts' counts are on the device, so
 // the number of tiles is what counts spread around the mean like random ones give; a tile's time per K-tile of 64 is a + b * (share of
-// the CUs at work beside it), as measured with 16 experts of 2048 x 2816, in us: 1.02 + 0.68 / 0.80 + 0.70 / 0.64 + 0.50.  A smaller
+// the CUs at work beside it), as measured with 16 experts of 2048 x 2816, in us: 1.02 + 0.68 / 0.80 + 0.70 / 0.64 + 0.50 (256 rows by the
+// kernel above; by gemm1w.hip's, which takes them now, 6 % less, but choices made with that are worse: 1,400 tokens 121 for 106 us).  A smaller
 // tile is taken where that predicts 5 % less, which is where 256 rows leave a round of tiles nearly empty or most of a tile without
 // rows.  Two of 16 experts per token, gate and up / down product in us, 256 rows -> the rule's: 600 tokens 112 / 58 -> 104 / 40,
-// 1,024: 105 / 61 -> 97 / 51, 1,400: 121 / 60 -> 111 / 54, 2,500: 172 / 74 -> 144 / 72, 4,096: 213 / 126 -> 213 / 104 (the rule keeps
-// 256 for the wider product; 192 measured 209), 2,048, 3,000 and 3,500: 256 as before (192 up to 35 % slower).
+// 1,024: 105 / 61 -> 97 / 51, 1,400: 121 / 60 -> 111 / 54, 2,500: 152 / 78 -> 135 / 68, 4,096: 196 / 128 -> 196 / 113 (the rule keeps
+// 256 for the wider product; 192 measured 202), 2,048, 3,000 and 3,500: 256 as before (192 up to 22 % slower).
+// The eight-wave kernel above, which had the 256-row tiles before, takes 5 - 8 % longer (3,500 and 4,096 tokens: 171 and 212 us instead
+// of 158 and 196); it is left with the widths and sizes that gemm1w.hip does not take.
 int grouped_tile_rows(long rows, int E, int TN) {
   struct Cost { int bm; double a, b; };
   constexpr Cost costs[] = {{256, 1.02, 0.68}, {192, 0.80, 0.70}, {128, 0.64, 0.50}};
@@ -1150,8 +1153,7 @@ int lk_gemm_grouped(const bf16_t* x, long ldx, const bf16_t* w, const int* seg, 
       reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(w) % 16)
     return -1;
   if (lk_gemm1w_grouped_supported(rows, ldx, gather ? x_rows : rows, N, K, swiglu, ldo)) {
-    const int bm = grouped_tile_rows(rows, E, N / 256);
-    if (bm != kBM) return lk_gemm1w_grouped(x, ldx, w, seg, E, rows, N, K, swiglu, out, ldo, st, gather, x_rows, scatter, top, bm);
+    return lk_gemm1w_grouped(x, ldx, w, seg, E, rows, N, K, swiglu, out, ldo, st, gather, x_rows, scatter, top, grouped_tile_rows(rows, E, N / 256));
   }
   if (swiglu) return launch_grouped<4, EPI_SWIGLU>(x, ldx, w, seg, E, rows, N, K, N / 2, out, ldo, N / 256, st, gather, x_rows, scatter, top);
   if (N % 256 == 0) return launch_grouped<4, EPI_NONE>(x, ldx, w, seg, E, rows, N, K, 0, out, ldo, N / 256, st, gather, x_rows, scatter, top);

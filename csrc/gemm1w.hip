@@ -781,11 +781,10 @@ int lk_gemm1w_grouped(const bf16_t* x, long ldx, const bf16_t* w, const int* seg
   ea.scatter = scatter;
   ea.x_rows = x_rows;
   ea.out_rows = rows;
-  if (swiglu)
-    return bm == 128 ? launch1w_grouped<E_SWIGLU, 128>(x, ldx, w, rows, K, N / 2, out, ldo, N / 256, st, ea)
-                     : launch1w_grouped<E_SWIGLU, 192>(x, ldx, w, rows, K, N / 2, out, ldo, N / 256, st, ea);
-  return bm == 128 ? launch1w_grouped<E_NONE, 128>(x, ldx, w, rows, K, 0, out, ldo, N / kBN, st, ea)
-                   : launch1w_grouped<E_NONE, 192>(x, ldx, w, rows, K, 0, out, ldo, N / kBN, st, ea);
+#define LK_G1W(EPI, BM) launch1w_grouped<EPI, BM>(x, ldx, w, rows, K, swiglu ? N / 2 : 0, out, ldo, N / kBN, st, ea)
+  if (swiglu) return bm == 128 ? LK_G1W(E_SWIGLU, 128) : bm == 192 ? LK_G1W(E_SWIGLU, 192) : LK_G1W(E_SWIGLU, 256);
+  return bm == 128 ? LK_G1W(E_NONE, 128) : bm == 192 ? LK_G1W(E_NONE, 192) : LK_G1W(E_NONE, 256);
+#undef LK_G1W
 }
 
 int lk_gemm1w_split_cols(int M, int TN, int cus) {
