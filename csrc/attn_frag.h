@@ -69,8 +69,10 @@ LK_DEVICE float max_groups(float v) {
 
 // one fragment: lane l's 16 bytes at src go to LDS byte off + 16 l (off wave-uniform).  As assembly: the compiler would wait for the
 // transfer before the next LDS read of the OTHER buffer; a kernel's loop waits for it itself, ahead of its barrier.
+template <bool NT = false>
 LK_DEVICE void dma16(unsigned off, const void* src) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(off), "v"(src) : "memory", "m0");
+  if constexpr (NT) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(off), "v"(src) : "memory", "m0");
+  else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(off), "v"(src) : "memory", "m0");
 }
 
 }  // namespace

@@ -287,12 +287,16 @@ __global__ __launch_bounds__(256, 3) void sigattn_stage_kernel(SigParams p, int 
 
 // ---- decode: workgroup = (sequence, up to 16 heads of one kv group, key split z); its 4 waves
 // take every fourth 32-key step of the split and are summed through LDS in wave order ------------
-template <typename T, int PAD>
-__global__ __launch_bounds__(256) void sigattn_decode_kernel(SigParams p, const int* __restrict__ ctx_lens, int Z,
+// STAGE (bf16, heads up to 128): through LDS-DMA (attn_stage.h).  64 sequences of 700 - 1,200 keys, 16 heads of 128 over 4: 32 us
+// with the fragments straight from the cache.
+template <typename T, int PAD, bool STAGE>
+__global__ __launch_bounds__(256) void sigattn_decode_kernel(SigParams p, int bs_shift, const int* __restrict__ ctx_lens, int Z,
                                                              T* __restrict__ out, long os,
                                                              float* __restrict__ part) {
   constexpr int VT = PAD / 16;
-  __shared__ float red[3][VT][64][4];
+  typedef float Red[3][VT][64][4];
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];   // the rings, then the waves' sums
+  Red& red = *reinterpret_cast<Red*>(smem);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, n16 = lane & 15, g = lane >> 4;
   const int rep = p.H / p.G, ngr = (rep + 15) / 16;
   const int b = blockIdx.x, kvh = blockIdx.y / ngr, sub = blockIdx.y % ngr, z = blockIdx.z;
@@ -308,7 +312,26 @@ __global__ __launch_bounds__(256) void sigattn_decode_kernel(SigParams p, const 
   for (int vt = 0; vt < VT; ++vt) o[vt] = floatx4{0.f, 0.f, 0.f, 0.f};
   const int nsteps = (ctx + 31) / 32, spz = (nsteps + Z - 1) / Z;
   const int s0 = z * spz, s1 = min(nsteps, s0 + spz);
-  if (s0 < s1)
+  if constexpr (STAGE) {
+    const StageCache c = {reinterpret_cast<const bf16_t*>(p.kc), reinterpret_cast<const bf16_t*>(p.vc), p.bt + (long)b * p.bt_stride,
+                          p.G, kvh, p.dim, p.vdim, p.BS, bs_shift};
+    const int k1 = min(ctx, 32 * s1);
+    const float r1 = p.r1[head], r2 = p.r2[head], hb = p.pb[head];
+    stage_wave<PAD>(c, reinterpret_cast<bf16_t*>(smem), qf, 32 * (s0 + w), k1, o, [&](int kb, const floatx4& c0, const floatx4& c1) {
+      float wt[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int key = kb + 8 * g + e;
+        const float wgt = sig_weight<false>((e < 4 ? c0[e & 3] : c1[e & 3]) * p.scale, r1, r2, hb, ctx - 1 - key);
+        wt[e] = cvalid && key < k1 ? wgt : 0.f;
+      }
+      uint4_t pk;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) pk[e] = pack_bf2(wt[2 * e], wt[2 * e + 1]);
+      return __builtin_bit_cast(short8, pk);
+    });
+    __syncthreads();   // all rings are read: the sums go there
+  } else if (s0 < s1)
     sig_run<T, PAD, true>(p, qf, kvh, p.bt + (long)b * p.bt_stride, 32 * s0, min(ctx, 32 * s1), w, 4, cvalid, ctx - 1,
                     p.r1[head], p.r2[head], p.pb[head], o);
   sum_waves<VT>(o, red);
@@ -476,7 +499,19 @@ template <typename T, int PAD>
 int launch_decode(const SigParams& p, const int* ctx, int B, int Z, void* out, long os, float* part, hipStream_t st) {
   const int rep = p.H / p.G;
   dim3 grid(B, p.G * ((rep + 15) / 16), Z);
-  sigattn_decode_kernel<T, PAD><<<grid, 256, 0, st>>>(p, ctx, Z, reinterpret_cast<T*>(out), os, part);
+  const auto al = [](const void* x) { return reinterpret_cast<uintptr_t>(x) % 16 == 0; };
+  constexpr int red = 3 * PAD * 64;   // floats of 3 waves' sums, in bytes: 3 (PAD / 16) 64 * 4 * 4
+  bool staged = false;
+  if constexpr (sizeof(T) == 2 && PAD <= kStageMaxPad) {
+    constexpr int lds = stage_wave_lds(PAD) > red ? stage_wave_lds(PAD) : red;
+    staged = p.qs % 8 == 0 && al(p.q) && al(p.kc) && al(p.vc);
+    if (staged) {
+      LK_SET_MAX_LDS((sigattn_decode_kernel<T, PAD, true>), lds);
+      const int shift = (p.BS & (p.BS - 1)) == 0 ? __builtin_ctz(p.BS) : -1;
+      sigattn_decode_kernel<T, PAD, true><<<grid, 256, lds, st>>>(p, shift, ctx, Z, reinterpret_cast<T*>(out), os, part);
+    }
+  }
+  if (!staged) sigattn_decode_kernel<T, PAD, false><<<grid, 256, red, st>>>(p, 0, ctx, Z, reinterpret_cast<T*>(out), os, part);
   LK_CHECK_LAUNCH();
   if (Z > 1) {
     sigattn_reduce_kernel<T><<<dim3(B, p.H), 256, 0, st>>>(part, Z, p.H, p.vdim, reinterpret_cast<T*>(out), os);

@@ -440,13 +440,18 @@ __global__ __launch_bounds__(256, 3) void sinkattn_stage_kernel(SinkParams p, in
 
 // ---- decode: workgroup = (sequence, up to 16 heads of one kv group, key split z) -----------------------
 // part: [B, H, Z, vdim + 2] f32 = O^T relative to m, then m, l
-template <typename T, int PAD>
-__global__ __launch_bounds__(256) void sinkattn_decode_kernel(SinkParams p, const int* __restrict__ ctx_lens, int Z,
+// STAGE (bf16, heads up to 128): through LDS-DMA (attn_stage.h).  64 sequences of 700 - 1,200 keys, 16 heads of 128 over 4, window 512 and
+// pooled blocks: 21 us with the fragments straight from the cache.
+template <typename T, int PAD, bool STAGE>
+__global__ __launch_bounds__(256) void sinkattn_decode_kernel(SinkParams p, int bs_shift, const int* __restrict__ ctx_lens, int Z,
                                                               T* __restrict__ out, long os, float* __restrict__ part) {
   constexpr int VT = PAD / 16;
   constexpr bool EXACT = sizeof(T) == 4;
-  __shared__ float red[3][VT][64][4];
-  __shared__ float ml[3][64][2];
+  typedef float Red[3][VT][64][4];
+  typedef float Ml[3][64][2];
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];   // the rings, then the waves' parts
+  Red& red = *reinterpret_cast<Red*>(smem);
+  Ml& ml = *reinterpret_cast<Ml*>(smem + sizeof(Red));
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, n16 = lane & 15, g = lane >> 4;
   const int rep = p.H / p.G, ngr = (rep + 15) / 16;
   const int b = blockIdx.x, kvh = blockIdx.y / ngr, sub = blockIdx.y % ngr, z = blockIdx.z;
@@ -468,12 +473,61 @@ __global__ __launch_bounds__(256) void sinkattn_decode_kernel(SinkParams p, cons
   const int n1 = pooled ? blocks_seen(ctx - 1, p.msize, p.pool) : kept_keys(p, klo);
   const int nwin = (ctx - k0 + 31) / 32, nsteps = nwin + (n1 + 31) / 32, spz = (nsteps + Z - 1) / Z;
   const int s0 = z * spz, s1 = min(nsteps, s0 + spz);
+  if constexpr (STAGE) {
+    StageCache c = {reinterpret_cast<const bf16_t*>(p.kc), reinterpret_cast<const bf16_t*>(p.vc), p.bt + (long)b * p.bt_stride,
+                    p.G, kvh, p.dim, p.vdim, p.BS, bs_shift};
+    const float hs = p.hscale[head], icap = p.cap > 0.f ? 1.f / p.cap : 0.f;
+    int lo = klo, hi = min(ctx, k0 + 32 * min(s1, nwin));   // keys lo .. hi - 1
+    auto weights = [&](int kb, const floatx4& c0, const floatx4& c1) {
+      float v[8], mx = kNegBig;
+      bool ok[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int key = kb + 8 * g + e;
+        ok[e] = cvalid && key >= lo && key < hi;
+        v[e] = (e < 4 ? c0[e & 3] : c1[e & 3]) * hs;
+        if (p.cap > 0.f) v[e] = cap_f<false>(v[e], p.cap, icap);
+        if (ok[e]) mx = fmaxf(mx, v[e]);
+      }
+      const float mn = fmaxf(m, max_groups(mx)), alpha = exp_f<false>(m - mn);   // (nothing seen yet, no sink: exp(0) on zeros)
+      m = mn;
+      l *= alpha;
+#pragma unroll
+      for (int vt = 0; vt < VT; ++vt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[vt][j] *= alpha;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        v[e] = ok[e] ? exp_f<false>(v[e] - mn) : 0.f;
+        l += v[e];
+      }
+      uint4_t pk;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) pk[e] = pack_bf2(v[2 * e], v[2 * e + 1]);
+      return __builtin_bit_cast(short8, pk);
+    };
+    int first = k0 + 32 * (s0 + w);
+#pragma unroll 1
+    for (int pass = 0;; ++pass) {   // the window's steps of this split, then those behind it
+      stage_wave<PAD>(c, reinterpret_cast<bf16_t*>(smem), qf, first, hi, o, weights);
+      if (pass || n1 <= 0) break;
+      if (pooled) {
+        c.kc = reinterpret_cast<const bf16_t*>(p.pkc);
+        c.vc = reinterpret_cast<const bf16_t*>(p.pvc);
+      }
+      lo = 0;
+      hi = min(n1, 32 * (s1 - nwin));
+      first = 32 * (max(s0, nwin) - nwin + w);
+    }
+    __syncthreads();   // all rings are read: the parts go there
+  } else {
   if (s0 < min(s1, nwin))
     sink_run<T, PAD, true>(p, p.kc, p.vc, qf, kvh, p.bt + (long)b * p.bt_stride, k0 + 32 * s0, min(ctx, k0 + 32 * min(s1, nwin)), w, 4, cvalid,
                      ctx - 1, klo, p.hscale[head], m, l, o);
   if (max(s0, nwin) < s1)
     sink_run<T, PAD, true>(p, pooled ? p.pkc : p.kc, pooled ? p.pvc : p.vc, qf, kvh, p.bt + (long)b * p.bt_stride, 32 * (max(s0, nwin) - nwin),
                      min(n1, 32 * (s1 - nwin)), w, 4, cvalid, n1 - 1, 0, p.hscale[head], m, l, o);
+  }
   merge_waves<EXACT, VT>(m, l, o, red, ml);
   if (w == 0 && cvalid) {
     if (Z == 1) {
@@ -644,7 +698,20 @@ int launch_stage(const SinkParams& p, const int* cu_q, const int* ctx, const int
 template <typename T, int PAD>
 int launch_decode(const SinkParams& p, const int* ctx, int B, int Z, void* out, long os, float* part, hipStream_t st) {
   const int rep = p.H / p.G;
-  sinkattn_decode_kernel<T, PAD><<<dim3(B, p.G * ((rep + 15) / 16), Z), 256, 0, st>>>(p, ctx, Z, reinterpret_cast<T*>(out), os, part);
+  const auto al = [](const void* x) { return reinterpret_cast<uintptr_t>(x) % 16 == 0; };
+  const dim3 grid(B, p.G * ((rep + 15) / 16), Z);
+  constexpr int red = 3 * PAD * 64 + 3 * 64 * 2 * 4;   // bytes of 3 waves' O, m and l
+  bool staged = false;
+  if constexpr (sizeof(T) == 2 && PAD <= kStageMaxPad) {
+    constexpr int lds = stage_wave_lds(PAD) > red ? stage_wave_lds(PAD) : red;
+    staged = p.qs % 8 == 0 && al(p.q) && al(p.kc) && al(p.vc) && al(p.pkc) && al(p.pvc);
+    if (staged) {
+      LK_SET_MAX_LDS((sinkattn_decode_kernel<T, PAD, true>), lds);
+      const int shift = (p.BS & (p.BS - 1)) == 0 ? __builtin_ctz(p.BS) : -1;
+      sinkattn_decode_kernel<T, PAD, true><<<grid, 256, lds, st>>>(p, shift, ctx, Z, reinterpret_cast<T*>(out), os, part);
+    }
+  }
+  if (!staged) sinkattn_decode_kernel<T, PAD, false><<<grid, 256, red, st>>>(p, 0, ctx, Z, reinterpret_cast<T*>(out), os, part);
   LK_CHECK_LAUNCH();
   if (Z > 1) {
     sinkattn_reduce_kernel<T><<<dim3(B, p.H), 256, 0, st>>>(p, part, Z, reinterpret_cast<T*>(out), os);

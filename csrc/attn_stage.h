@@ -158,4 +158,71 @@ LK_DEVICE void stage_walk(const StageCache& p, bf16_t* lds, uint4_t (&qf)[PAD / 
   }
 }
 
+// Decode: one wave alone with keys first, first + 128, .. (32 at a time) below k1, read once and therefore non-temporally, through its own
+// 1 / 4 of the workgroup's LDS without a barrier.  A step's fragments go to registers together, so that the next step's 16 KB (heads of 128)
+// are requested before this step's arithmetic.  As fragments straight from the cache, 16 rows x 64 bytes, a CU took 17 KB/us.
+constexpr int stage_wave_lds(int PAD) { return 4 * stage_frags(PAD) * 1024; }
+
+template <int PAD, typename F>
+LK_DEVICE void stage_wave(const StageCache& p, bf16_t* lds, uint4_t (&qf)[PAD / 32], int first, int k1, floatx4 (&o)[PAD / 16], F weights) {
+  constexpr int KS = PAD / 32, VT = PAD / 16, NK = 2 * KS, FR = NK + VT, CPR = PAD / 8;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n16 = lane & 15, g = lane >> 4;
+  const int krow = 8 * (n16 >> 2) + (n16 & 3);
+  bf16_t* fr = lds + w * FR * 512;
+  const unsigned lds0 = (unsigned)reinterpret_cast<uintptr_t>((lds_void_ptr)fr);
+  auto issue = [&](int kb) {
+    int pg[2], at[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int key = min(kb + 16 * h, k1 - 1), page = __builtin_amdgcn_readfirstlane(p.bs_shift >= 0 ? key >> p.bs_shift : key / p.BS);
+      pg[h] = ((const __attribute__((address_space(4))) int*)p.bt)[page];
+      at[h] = page * p.BS;
+    }
+#pragma unroll
+    for (int f = 0; f < FR; ++f) {
+      const unsigned off = lds0 + (unsigned)f * 1024u;
+      if (f < NK) {
+        const int q = 64 * f + lane, row = q / CPR, ch = stage_chunk<CPR>(q % CPR, row, -1), h = row >> 4;
+        const bf16_t* kr = p.kc + (((long)(h ? pg[1] : pg[0]) * p.G + p.kvh) * p.BS - (h ? at[1] : at[0]) + min(kb + row, k1 - 1)) * p.dim;
+        dma16<true>(off, kr + min(8 * ch, p.dim - 8));
+      } else {
+        const int h = (f - NK) / (VT / 2), vd = (f - NK) % (VT / 2) * 32 + (lane >> 1), c = (lane ^ (vd >> 2)) & 1;
+        const bf16_t* vr = p.vc + ((long)pg[h] * p.G + p.kvh) * p.vdim * p.BS + min(kb + 16 * h + 8 * c, (k1 - 1) & ~7) - at[h];
+        dma16<true>(off, vr + (long)min(vd, p.vdim - 1) * p.BS);
+      }
+    }
+  };
+  int kat[KS];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) kat[s] = (krow * CPR + stage_chunk<CPR>(4 * s + g, krow, 1)) * 8;
+  const int vat = NK * 512 + (g >> 1) * (VT / 2) * 512 + n16 * 16 + (((g & 1) ^ (n16 >> 2)) & 1) * 8;
+  // (a walk before this one has its last fragments in registers)
+  if (first < k1) issue(first);
+#pragma unroll
+  for (int i = 0; i < KS; ++i) asm volatile("" : "+v"(qf[i]));   // (q has arrived: the waits in the loop are for fragments alone)
+  for (int kb = first; kb < k1; kb += 128) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    uint4_t kf[2][KS], vf[VT];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int s = 0; s < KS; ++s) kf[t][s] = ld16(fr + kat[s] + t * (4 * CPR * 8));
+#pragma unroll
+    for (int vt = 0; vt < VT; ++vt) vf[vt] = ld16(fr + vat + vt * 256);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the fragments are read before a load may write there
+    __builtin_amdgcn_sched_barrier(0);
+    if (kb + 128 < k1) issue(kb + 128);
+    __builtin_amdgcn_sched_barrier(0);
+    floatx4 c[2];
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) c[t] = mma_qk<bf16_t>(kf[t][s], qf[s], s == 0 ? floatx4{0.f, 0.f, 0.f, 0.f} : c[t]);
+    const short8 pb = weights(kb, c[0], c[1]);
+#pragma unroll
+    for (int vt = 0; vt < VT; ++vt) o[vt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(short8, vf[vt]), pb, o[vt], 0, 0, 0);
+  }
+}
+
 }  // namespace
