@@ -59,37 +59,50 @@ LK_DEVICE void rg_walk(const bf16_t* const (&xs)[2 * MT], const bf16_t* const (&
   for (int m = 0; m < MT; ++m)
 #pragma unroll
     for (int n = 0; n < NT; ++n) acc[m][n] = (floatx4){0.f, 0.f, 0.f, 0.f};
+  // Three stages or more: the next is requested into the slot of the stage before, whose fragments its products have consumed.  Two: a
+  // stage's fragments go to registers together and its own slot is requested again before the products, which keeps both on their way
+  // (the wait for LDS in between costs 0.2 us of a walk of 8 stages, and a deeper ring gains nothing from it).
+  constexpr bool SELF = NS < 3;
+  constexpr int AHEAD = SELF ? NS : NS - 1;
 #pragma unroll
-  for (int p = 0; p < NS; ++p)
+  for (int p = 0; p < AHEAD; ++p)
     if (p < nst) issue(p);
   for (int st = 0; st < nst; ++st) {
-    rg_wait_ahead<L, NS - 1>(min(NS - 1, nst - 1 - st));
+    rg_wait_ahead<L, AHEAD - 1>(min(AHEAD - 1, nst - 1 - st));
     __builtin_amdgcn_sched_barrier(0);
-    // the whole stage into registers, so that its slot is free for the loads of stage st + NS before the products
+    if constexpr (!SELF) {
+      if (st + AHEAD < nst) issue(st + AHEAD);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     const unsigned char* base = ring + (st % NS) * SB;
     short8 a[2][MT], b[2][NT];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    auto read = [&](int h) {
       const int at = r16 * 128 + (((4 * h + g) ^ (r16 & 7)) << 4);
 #pragma unroll
       for (int n = 0; n < NT; ++n) b[h][n] = *reinterpret_cast<const short8*>(base + (MT + n) * 2048 + at);
 #pragma unroll
       for (int m = 0; m < MT; ++m) a[h][m] = *reinterpret_cast<const short8*>(base + m * 2048 + at);
-    }
-    if (st + NS < nst) {
-      __builtin_amdgcn_sched_barrier(0);
-      rg_wait_lds();   // the reads are done before a load may write there
-      __builtin_amdgcn_sched_barrier(0);
-      issue(st + NS);
-      __builtin_amdgcn_sched_barrier(0);
+    };
+    read(0);
+    if constexpr (SELF) {
+      read(1);
+      if (st + AHEAD < nst) {
+        __builtin_amdgcn_sched_barrier(0);
+        rg_wait_lds();   // the reads are done before a load may write there
+        __builtin_amdgcn_sched_barrier(0);
+        issue(st + AHEAD);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int h = 0; h < 2; ++h) {
+      if (!SELF && h == 1) read(1);
       // W as the A operand: the lane ends with one output row and 4 consecutive columns
 #pragma unroll
       for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int n = 0; n < NT; ++n) acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[h][n], a[h][m], acc[m][n], 0, 0, 0);
+    }
   }
 }
 
