@@ -650,7 +650,7 @@ __global__ __launch_bounds__(256) void ssm_chunk_kernel(const T* __restrict__ xb
 // enters a product as three bf16 parts (8 + 8 + 8 mantissa bits, an f32), summed in the f32 accumulators.  A sequence's chunks are a
 // serial chain, so what bounds the kernel is the time of one chunk: 64 tokens take 130 products of 16 cycles per wave instead of
 // 4 x 100 of 32 (16x16x4 f32), with two barriers instead of eight.  4 x 1,024 tokens, 64 heads of [64, 128]: 351 us (f32
-// products, chunks of 16) -> 129 us; y writes 67 MB and the rows read 50.  Error against f64 9e-8 (f32 products: 2.2e-7).
+// products, chunks of 16) -> 133 -> 126 us (operands filed and prefetched as below); y writes 67 MB and the rows read 50.  Error against f64 9e-8 (f32 products: 2.2e-7).
 // grid (sequence, head, P / 64): wave w owns state columns p0 + 16 w .. +15 (all N rows as accumulators S[n][p]: lane p = l & 15,
 // rows 16 nt + 4 (l >> 4) + j) and computes M's rows of token tile w for everybody.  y is accumulated transposed (lane: one token,
 // four adjacent columns).  The order of n inside a 32-step is (4g + j, 16 + 4g + j), so that the accumulators are operands as they lie.
@@ -685,6 +685,14 @@ LK_DEVICE float exp_f64sum(double c) {
 template <int NR>
 constexpr int ssm_chunk_lds() {
   return 2 * 64 * (NR * 16 + 8) * 2 + NR * 16 * 72 * 2 + 64 * 72 * 2 + 3 * 64 * 72 * 2 + 5 * 64 * 4;
+}
+
+// the lanes' doubles moved by one DPP control (0 where a lane has no source or its row is masked out)
+template <int CTRL, int ROWS>
+LK_DEVICE double dpp64(double v) {
+  const int2 a = __builtin_bit_cast(int2, v);
+  return __builtin_bit_cast(double, make_int2(__builtin_amdgcn_update_dpp(0, a.x, CTRL, ROWS, 0xf, ROWS == 0xf),
+                                              __builtin_amdgcn_update_dpp(0, a.y, CTRL, ROWS, 0xf, ROWS == 0xf)));
 }
 
 template <int NR>
@@ -731,7 +739,7 @@ __global__ __launch_bounds__(256, 1) void ssm_chunk_bf16_kernel(const bf16_t* __
   constexpr int NB = NP / 64 > 0 ? NP / 64 : 1, NC = NP / 32;
   short4_t fb[NB][4], fx[4];
   uint4_t fc[NC];
-  float fdt = 0.f;
+  bf16_t fdt = 0;
   const short4_t z4 = {0, 0, 0, 0};
   auto fetch = [&](int t0) {
     const int tl = len - t0;
@@ -751,8 +759,11 @@ __global__ __launch_bounds__(256, 1) void ssm_chunk_bf16_kernel(const bf16_t* __
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       fx[i] = (xt + i < tl && p0 + xp < P) ? *reinterpret_cast<const short4_t*>(bx + (long)(t0 + xt + i) * xs + xp) : z4;
-    fdt = lane < tl ? bf2f(dtp[(long)(row0 + t0 + lane) * dts + h]) : 0.f;
+    // (kept as it lies: converted here, every load above would be waited for at once, 2 us of a chunk)
+    fdt = dtp[(long)(row0 + t0 + min(lane, tl - 1)) * dts + h];
   };
+  // a transposed row's groups of 8 tokens are turned by the row: threads file rows four apart, which lay in the same banks (16 deep)
+  auto at_t = [&](int row, int t) { return row * LT + (((t >> 3) ^ ((row >> 3) & 7)) << 3) + (t & 7); };
   fetch(0);
   for (int t0 = 0; t0 < len; t0 += L) {
     const int tl = min(L, len - t0);
@@ -764,7 +775,7 @@ __global__ __launch_bounds__(256, 1) void ssm_chunk_bf16_kernel(const bf16_t* __
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           *reinterpret_cast<short4_t*>(sB + (t + i) * LN + n) = fb[k][i];
-          *reinterpret_cast<short4_t*>(sBt + (n + i) * LT + t) = (short4_t){fb[k][0][i], fb[k][1][i], fb[k][2][i], fb[k][3][i]};
+          *reinterpret_cast<short4_t*>(sBt + at_t(n + i, t)) = (short4_t){fb[k][0][i], fb[k][1][i], fb[k][2][i], fb[k][3][i]};
         }
       }
     }
@@ -777,22 +788,24 @@ __global__ __launch_bounds__(256, 1) void ssm_chunk_bf16_kernel(const bf16_t* __
       const int xp = (tid & 15) * 4, xt = (tid >> 4) * 4;
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        *reinterpret_cast<short4_t*>(sXt + (xp + i) * LT + xt) = (short4_t){fx[0][i], fx[1][i], fx[2][i], fx[3][i]};
+        *reinterpret_cast<short4_t*>(sXt + at_t(xp + i, xt)) = (short4_t){fx[0][i], fx[1][i], fx[2][i], fx[3][i]};
     }
     // lane = token: c, the running sum of the log-decays (every wave computes and files the same values)
     float dec;
     {
-      const float a = fdt + db;
+      const float a = bf2f(fdt) + db;
       const float dt = lane < tl ? (a > 20.f ? a : log1pf(expf(a))) : 0.f;
       // (the sum over 64 tokens in f64 and as two floats: a difference of two of them keeps an f32's relative error, as the
       // 16-token chunks' sums did)
       double c = (double)nA * dt;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const double v = __shfl_up(c, o, 64);
-        if (lane >= o) c += v;
-      }
-      const double cld = __shfl(c, 63, 64);
+      c += dpp64<0x111, 0xf>(c);   // row_shr 1, 2, 4, 8: inside 16 lanes (by the LDS unit, 14 exchanges deep, it was a tenth of a chunk)
+      c += dpp64<0x112, 0xf>(c);
+      c += dpp64<0x114, 0xf>(c);
+      c += dpp64<0x118, 0xf>(c);
+      c += dpp64<0x142, 0xa>(c);   // row_bcast 15 to the second and fourth 16, 31 to the upper half
+      c += dpp64<0x143, 0xc>(c);
+      const int2 last = __builtin_bit_cast(int2, c);
+      const double cld = __builtin_bit_cast(double, make_int2(__builtin_amdgcn_readlane(last.x, 63), __builtin_amdgcn_readlane(last.y, 63)));
       const float hi = (float)c;
       sc[lane] = hi;
       scl[lane] = (float)(c - hi);
@@ -811,33 +824,40 @@ __global__ __launch_bounds__(256, 1) void ssm_chunk_bf16_kernel(const bf16_t* __
       short8 cf[NR / 2];
 #pragma unroll
       for (int kk = 0; kk < NR / 2; ++kk) cf[kk] = *reinterpret_cast<const short8*>(sC + t * LN + 32 * kk + 8 * g);
-      for (int st = 0; st <= (w | 1); ++st) {
-        floatx4 m = {0.f, 0.f, 0.f, 0.f};
-        if (st <= w) {
+      // (all four tiles in every wave, side by side: those behind t's are zeros, and the wave with four of them is the one waited for)
+      floatx4 m[4];
 #pragma unroll
-          for (int kk = 0; kk < NR / 2; ++kk) {
-            const short8 a = *reinterpret_cast<const short8*>(sB + (16 * st + r16) * LN + 32 * kk + 8 * g);
-            m = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, cf[kk], m, 0, 0, 0);
-          }
-          const floatx4 cs = *reinterpret_cast<const floatx4*>(sc + 16 * st + 4 * g);
-          const floatx4 cw = *reinterpret_cast<const floatx4*>(scl + 16 * st + 4 * g);
-          const floatx4 ds = *reinterpret_cast<const floatx4*>(sdt + 16 * st + 4 * g);
+      for (int kk = 0; kk < NR / 2; ++kk)
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int sj = 16 * st + 4 * g + j;
-            m[j] = sj < t ? m[j] * expf((ct - cs[j]) + (ctl - cw[j])) * ds[j] : (sj == t ? m[j] * ds[j] + Dh : 0.f);  // the skip D x on the diagonal
-          }
+        for (int st = 0; st < 4; ++st) {
+          const short8 a = *reinterpret_cast<const short8*>(sB + (16 * st + r16) * LN + 32 * kk + 8 * g);
+          m[st] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, cf[kk], kk == 0 ? floatx4{0.f, 0.f, 0.f, 0.f} : m[st], 0, 0, 0);
         }
+#pragma unroll
+      for (int st = 0; st < 4; ++st) {
+        const floatx4 cs = *reinterpret_cast<const floatx4*>(sc + 16 * st + 4 * g);
+        const floatx4 cw = *reinterpret_cast<const floatx4*>(scl + 16 * st + 4 * g);
+        const floatx4 ds = *reinterpret_cast<const floatx4*>(sdt + 16 * st + 4 * g);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int sj = 16 * st + 4 * g + j;
+          m[st][j] = sj < t ? m[st][j] * expf((ct - cs[j]) + (ctl - cw[j])) * ds[j]
+                            : (sj == t ? m[st][j] * ds[j] + Dh : 0.f);  // the skip D x on the diagonal
+        }
+      }
+#pragma unroll
+      for (int st = 0; st < 4; ++st) {
+        if (st > (w | 1)) break;   // (the 32-steps behind t's are not read)
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
           uint2 u;
-          u.x = pack_bf2(m[0], m[1]);
-          u.y = pack_bf2(m[2], m[3]);
+          u.x = pack_bf2(m[st][0], m[st][1]);
+          u.y = pack_bf2(m[st][2], m[st][3]);
           *reinterpret_cast<uint2*>(sM + (k * L + t) * LT + 16 * st + 4 * g) = u;
-          m[0] -= __uint_as_float(u.x << 16);
-          m[1] -= __uint_as_float(u.x & 0xffff0000u);
-          m[2] -= __uint_as_float(u.y << 16);
-          m[3] -= __uint_as_float(u.y & 0xffff0000u);
+          m[st][0] -= __uint_as_float(u.x << 16);
+          m[st][1] -= __uint_as_float(u.x & 0xffff0000u);
+          m[st][2] -= __uint_as_float(u.y << 16);
+          m[st][3] -= __uint_as_float(u.y & 0xffff0000u);
         }
       }
     }
@@ -873,7 +893,7 @@ __global__ __launch_bounds__(256, 1) void ssm_chunk_bf16_kernel(const bf16_t* __
     short8 xf[2], xe[2];
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
-      xf[kk] = *reinterpret_cast<const short8*>(sXt + (16 * w + r16) * LT + 32 * kk + 8 * g);
+      xf[kk] = *reinterpret_cast<const short8*>(sXt + at_t(16 * w + r16, 32 * kk + 8 * g));
       xe[kk] = g < 2 ? xf[kk] : (short8){0, 0, 0, 0, 0, 0, 0, 0};
     }
 #pragma unroll
@@ -900,7 +920,7 @@ __global__ __launch_bounds__(256, 1) void ssm_chunk_bf16_kernel(const bf16_t* __
       const BfParts q = bf_split3(v);
 #pragma unroll
       for (int nt = 0; nt < NR; ++nt) {
-        const short8 b = *reinterpret_cast<const short8*>(sBt + (16 * nt + r16) * LT + 32 * kk + 8 * g);
+        const short8 b = *reinterpret_cast<const short8*>(sBt + at_t(16 * nt + r16, 32 * kk + 8 * g));
 #pragma unroll
         for (int k = 2; k >= 0; --k) S[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, q.p[k], S[nt], 0, 0, 0);
       }
