@@ -368,14 +368,47 @@ LK_DEVICE void ld4s(const T* p, bool on, bool vec, float (&f)[4]) {
   }
 }
 
+// the value of lane ^ O, by the vector unit's lane moves
+template <int O>
+LK_DEVICE float lane_xor(float v) {
+  static_assert(O == 1 || O == 2 || O == 4 || O == 8);
+  const int i = (int)__float_as_uint(v);
+  if constexpr (O == 4) {  // ^ 3, then ^ 7 (the half row mirrored)
+    const int q = __builtin_amdgcn_update_dpp(0, i, 0x1b, 0xf, 0xf, true);
+    return __uint_as_float((unsigned)__builtin_amdgcn_update_dpp(0, q, 0x141, 0xf, 0xf, true));
+  } else {  // quad_perm [1, 0, 3, 2], [2, 3, 0, 1]; row_ror 8
+    return __uint_as_float((unsigned)__builtin_amdgcn_update_dpp(0, i, O == 1 ? 0xb1 : O == 2 ? 0x4e : 0x128, 0xf, 0xf, true));
+  }
+}
+// butterfly over the distances O, 2 O, .. below END
+template <int O, int END>
+LK_DEVICE float group_sum(float v) {
+  if constexpr (O >= END) {
+    return v;
+  } else if constexpr (O < 16) {
+    return group_sum<2 * O, END>(v + lane_xor<O>(v));
+  } else {
+    const unsigned u = __float_as_uint(v);
+    if constexpr (O == 16) {
+      const auto h = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+      return group_sum<2 * O, END>(__uint_as_float(h[0]) + __uint_as_float(h[1]));
+    } else {
+      const auto h = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+      return __uint_as_float(h[0]) + __uint_as_float(h[1]);
+    }
+  }
+}
+
 // One token per sequence (decode): grid (sequence, head).  All a step does is pass over the state once
 // (read, decay, add, write: 8 bytes per element), so HBM is the bound and the kernel is laid out for it:
 // LPR = N / 4 lanes hold one state row [n] as 16-byte vectors, a wave covers 64 / LPR rows per access and
 // requests RB of them together.  y_p is the row's sum over its lanes: the RB rows' sums are halved against
 // each other first (log2 RB exchanges leave one row per lane group), then finished inside the group.
-// 64 sequences x 64 heads x [64, 128]: 143 us as a one-token run of ssm_scan_kernel (256 threads for 16
-// rows, positions before the state is requested) -> 67 us, 4.0 TB/s.
-template <typename T, int LPR, int RB>
+// FULL: N = 4 LPR, P whole passes, rows aligned.  Then nothing is tested per row, and a wave's rows lie at immediates from one address:
+// 69 registers instead of 142, so that 7 waves and not 3 per SIMD keep requests in flight; the exchanges are lane moves of the vector
+// unit instead of the LDS unit's.  64 sequences x 64 heads x [64, 128]: 143 us as a one-token run of ssm_scan_kernel (256 threads for 16
+// rows, positions before the state is requested) -> 67 us (without FULL) -> 48 us, 5.6 TB/s; a bare pass over the state takes 43.
+template <typename T, int LPR, int RB, bool FULL>
 __global__ __launch_bounds__(256) void ssm_step_kernel(const T* __restrict__ xbc, long xs, const T* __restrict__ dtp, long dts,
                                                        int heads, int P, int N, int groups, const float* __restrict__ dt_bias,
                                                        const float* __restrict__ A_log, const float* __restrict__ Dp,
@@ -393,11 +426,12 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(const T* __restrict__ xbc
     return;
   }
   const int inner = heads * P, grp = h / (heads / groups);
-  const bool nv = n0 < N;
+  const bool nv = FULL || n0 < N;
   bool past = positions[row0] > 0;
   const float nA = -expf(A_log[h]), db = dt_bias[h], Dh = Dp[h];
-  const bool vec = ((reinterpret_cast<uintptr_t>(xbc) | xs * sizeof(T) | inner * sizeof(T)) & (4 * sizeof(T) - 1)) == 0;
+  const bool vec = FULL || ((reinterpret_cast<uintptr_t>(xbc) | xs * sizeof(T) | inner * sizeof(T)) & (4 * sizeof(T) - 1)) == 0;
   float* sp = state + ((long)slot * heads + h) * P * N;
+  const int ld = FULL ? 4 * LPR : N;
   for (int row = row0; row < row1; ++row) {  // (a longer sequence comes back to the rows that this thread has written)
     const T* in = xbc + (long)row * xs;
     const T* xp = in + (long)h * P;
@@ -411,16 +445,17 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(const T* __restrict__ xbc
     for (int p0 = w * RPA * RB; p0 < P; p0 += 4 * RPA * RB) {
       floatx4 S[RB];
       float x[RB], acc[RB];
+      float* const s0 = sp + (long)(p0 + sub) * ld + n0;
+      const T* const x0 = xp + p0 + sub;
 #pragma unroll
       for (int i = 0; i < RB; ++i) {
-        const int p = p0 + i * RPA + sub;
+        const bool on = FULL || p0 + i * RPA + sub < P;
         // (requested whether the sequence has a past or not: the position is still on its way)
-        S[i] = (nv && p < P) ? __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(sp + (long)p * N + n0)) : (floatx4){0.f, 0.f, 0.f, 0.f};
-        x[i] = p < P ? ldf<T>(xp + p) : 0.f;
+        S[i] = nv && on ? __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(s0 + (long)i * RPA * ld)) : (floatx4){0.f, 0.f, 0.f, 0.f};
+        x[i] = on ? ldf<T>(x0 + i * RPA) : 0.f;
       }
 #pragma unroll
       for (int i = 0; i < RB; ++i) {
-        const int p = p0 + i * RPA + sub;
         const float dx = dt * x[i];
         acc[i] = 0.f;
 #pragma unroll
@@ -428,25 +463,27 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(const T* __restrict__ xbc
           S[i][e] = dA * (past ? S[i][e] : 0.f) + dx * B[e];
           acc[i] += S[i][e] * C[e];
         }
-        if (nv && p < P) __builtin_nontemporal_store(S[i], reinterpret_cast<floatx4*>(sp + (long)p * N + n0));
+        if (nv && (FULL || p0 + i * RPA + sub < P)) __builtin_nontemporal_store(S[i], reinterpret_cast<floatx4*>(s0 + (long)i * RPA * ld));
       }
       // halve the rows against the lanes of a group: an exchange at distance o leaves each lane with the half
       // of the rows that bit o of its number names
       int base = 0;  // first row of the block that acc[0] stands for
-#pragma unroll
-      for (int k = RB / 2, o = 1; k >= 1; k >>= 1, o <<= 1) {
+      auto halve = [&](auto k_t) {
+        constexpr int k = decltype(k_t)::value, o = RB / 2 / k;
         const bool up = nl & o;
 #pragma unroll
         for (int i = 0; i < k; ++i) {
           const float mine = up ? acc[i + k] : acc[i], give = up ? acc[i] : acc[i + k];
-          acc[i] = mine + __shfl_xor(give, o, 64);
+          acc[i] = mine + lane_xor<o>(give);
         }
         base += up ? k : 0;
-      }
-#pragma unroll
-      for (int o = RB; o < LPR; o <<= 1) acc[0] += __shfl_xor(acc[0], o, 64);
+      };
+      if constexpr (RB >= 8) halve(std::integral_constant<int, 4>{});
+      if constexpr (RB >= 4) halve(std::integral_constant<int, 2>{});
+      if constexpr (RB >= 2) halve(std::integral_constant<int, 1>{});
+      acc[0] = group_sum<RB, LPR>(acc[0]);
       const int p = p0 + base * RPA + sub;
-      if (nl < RB && p < P) yr[p] = acc[0] + Dh * ldf<T>(xp + p);
+      if (nl < RB && (FULL || p < P)) yr[p] = acc[0] + Dh * ldf<T>(xp + p);
     }
     past = true;
   }
@@ -650,7 +687,8 @@ __global__ __launch_bounds__(256) void ssm_chunk_kernel(const T* __restrict__ xb
 // enters a product as three bf16 parts (8 + 8 + 8 mantissa bits, an f32), summed in the f32 accumulators.  A sequence's chunks are a
 // serial chain, so what bounds the kernel is the time of one chunk: 64 tokens take 130 products of 16 cycles per wave instead of
 // 4 x 100 of 32 (16x16x4 f32), with two barriers instead of eight.  4 x 1,024 tokens, 64 heads of [64, 128]: 351 us (f32
-// products, chunks of 16) -> 133 -> 126 us (operands filed and prefetched as below); y writes 67 MB and the rows read 50.  Error against f64 9e-8 (f32 products: 2.2e-7).
+// products, chunks of 16) -> 133 -> 126 us (operands filed and prefetched as below); y writes 67 MB and the
+// rows read 50.  Error against f64 9e-8 (f32 products: 2.2e-7).
 // grid (sequence, head, P / 64): wave w owns state columns p0 + 16 w .. +15 (all N rows as accumulators S[n][p]: lane p = l & 15,
 // rows 16 nt + 4 (l >> 4) + j) and computes M's rows of token tile w for everybody.  y is accumulated transposed (lane: one token,
 // four adjacent columns).  The order of n inside a 32-step is (4g + j, 16 + 4g + j), so that the accumulators are operands as they lie.
@@ -1045,9 +1083,15 @@ int scan_t(const T* xbc, long xs, const T* dtp, long dts, int S, int heads, int 
   }
   if (max_len == 1 && N % 4 == 0 && N >= 16 && N <= 256 && (reinterpret_cast<uintptr_t>(state) & 15) == 0) {
     dim3 sgrid(S, heads);
-#define LK_STEP(LPR, RB)                                                                                                  \
-  ssm_step_kernel<T, LPR, RB><<<sgrid, 256, 0, st>>>(xbc, xs, dtp, dts, heads, P, N, groups, dt_bias, A_log, D, state, cu, \
-                                                     slots, positions, y, ys)
+    const bool vec = ((reinterpret_cast<uintptr_t>(xbc) | xs * sizeof(T) | (size_t)heads * P * sizeof(T)) & (4 * sizeof(T) - 1)) == 0;
+#define LK_STEP_(LPR, RB, FULL)                                                                                                  \
+  ssm_step_kernel<T, LPR, RB, FULL><<<sgrid, 256, 0, st>>>(xbc, xs, dtp, dts, heads, P, N, groups, dt_bias, A_log, D, state, cu, \
+                                                           slots, positions, y, ys)
+#define LK_STEP(LPR, RB)                                                       \
+  do {                                                                         \
+    if (vec && N == 4 * LPR && P % (64 / LPR * (RB)) == 0) LK_STEP_(LPR, (RB), true); \
+    else LK_STEP_(LPR, (RB), false);                                           \
+  } while (0)
     // rows per lane group of a pass: 8, or what gives all four waves a part of P.  One sequence, 32 heads of [64, 32] / [64, 64]:
     // 5.2 / 5.5 us with 8 (one and two of the four waves at work) -> 3.6 / 4.3; 16 sequences 6.1 / 7.1 -> 4.5 / 5.9
 #define LK_STEPS(LPR)                                       \
@@ -1064,6 +1108,7 @@ int scan_t(const T* xbc, long xs, const T* dtp, long dts, int S, int heads, int 
     else LK_STEPS(64);
 #undef LK_STEPS
 #undef LK_STEP
+#undef LK_STEP_
     LK_CHECK_LAUNCH();
     return 0;
   }

@@ -10,11 +10,11 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
-def _run(lens, H, P, N, G, dtype, max_len, later):
+def _run(lens, H, P, N, G, dtype, max_len, later, shift=0):
     g = torch.Generator(device=DEV).manual_seed(H * P + N)
     rn = lambda *s: torch.randn(*s, device=DEV, generator=g)  # noqa: E731
     T, S, C = sum(lens), len(lens), H * P + 2 * G * N
-    xbc = rn(T, -(-C // 8) * 8 + 8).to(dtype)[:, :C]
+    xbc = rn(T, -(-C // 8) * 8 + 8).to(dtype)[:, shift:C + shift]
     d = rn(T, H + 3).to(dtype)[:, :H]
     state, b, A, D = rn(S + 1, H, P, N), rn(H) * 0.5 - 1, rn(H) * 0.3, rn(H)
     cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32, device=DEV)
@@ -96,3 +96,14 @@ def test_non_finite_rows_reach_no_earlier_tile(bad, at):
     xbc[at, 3] = bad
     got = run(xbc)
     assert torch.equal(got[:at // 16 * 16], want[:at // 16 * 16]) and not bool(torch.isfinite(got[at, 3]))
+
+
+@pytest.mark.parametrize("N", [16, 32, 64, 128, 256])
+@pytest.mark.parametrize("P", [2, 16, 64, 66, 128])
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_step_whole_passes(hip, N, P, shift, dtype):
+    """State rows that fill their lanes: whole passes of rows and a rest, input rows aligned to four values and not, tokens in a run."""
+    y, ref, state, want = _run([1, 1, 2, 1], 4, P, N, 2, dtype, 1, 5, shift)
+    assert (y.double() - ref).norm() <= 1e-6 * ref.norm()   # as above
+    assert (state.double() - want).norm() <= 1e-6 * want.norm()
