@@ -226,6 +226,29 @@ std::tuple<at::Tensor, at::Tensor> rows_pair(const at::Tensor& x1, const at::Ten
   return {y1, y2};
 }
 
+// f32 parts [s, M, N] of x1 w1^T and x2 w2^T in one launch, and how many belong to the first (csrc/rows_gemm.hip)
+bool rows_sums_supported(int64_t M, int64_t N, int64_t K1, int64_t K2) {
+  int s1 = 0;
+  return M <= 64 && N < (1 << 24) && K1 < (1 << 24) && K2 < (1 << 24) && lk_rows_sums_parts((int)M, (int)N, (int)K1, (int)K2, &s1) > 0;
+}
+std::tuple<at::Tensor, int64_t> rows_sums(const at::Tensor& x1, const at::Tensor& w1, const at::Tensor& x2, const at::Tensor& w2) {
+  for (const at::Tensor* t : {&x1, &x2}) {
+    CHECK_CUDA((*t)); CHECK_BF16((*t)); CHECK_LASTDIM((*t)); check_rows16(*t, "x");
+  }
+  for (const at::Tensor* t : {&w1, &w2}) {
+    CHECK_CUDA((*t)); CHECK_BF16((*t)); CHECK_CONTIG((*t)); check_rows16(*t, "w");
+  }
+  TORCH_CHECK(x1.dim() == 2 && x2.dim() == 2 && w1.dim() == 2 && w2.dim() == 2 && x1.size(0) == x2.size(0) && w1.size(0) == w2.size(0) &&
+              x1.size(1) == w1.size(1) && x2.size(1) == w2.size(1), "rows_sums: x [M, K], w [N, K], outputs alike");
+  const int M = x1.size(0), N = w1.size(0), K1 = x1.size(1), K2 = x2.size(1);
+  int s1 = 0;
+  const int parts = lk_rows_sums_parts(M, N, K1, K2, &s1);
+  TORCH_CHECK(parts > 0, "rows_sums: 17 to 64 rows, N and K multiples of 64");
+  at::Tensor p = at::empty({parts, M, N}, x1.options().dtype(at::kFloat));
+  CHECK_RC(lk_rows_sums(bp(x1), x1.stride(0), bp(w1), K1, bp(x2), x2.stride(0), bp(w2), K2, p.data_ptr<float>(), M, N, cur_stream()), "rows_sums");
+  return {p, s1};
+}
+
 // (y, h): h = LN(s), y = act(h w^T + bias) in one launch
 std::tuple<at::Tensor, at::Tensor> ln_linear(const at::Tensor& s, const at::Tensor& ln_w, const at::Tensor& ln_b, double eps, const at::Tensor& w,
                                              const at::Tensor& bias, bool gelu) {
@@ -1244,6 +1267,23 @@ at::Tensor stream_rmsnorm(at::Tensor& x, const c10::optional<at::Tensor>& a, con
   return out;
 }
 
+// stream_rmsnorm with a and b as the parts of rows_sums
+at::Tensor stream_rmsnorm_sums(at::Tensor& x, const at::Tensor& parts, int64_t s1, const c10::optional<at::Tensor>& a_bias,
+                               const c10::optional<at::Tensor>& e, double mult, const c10::optional<at::Tensor>& w, double woff, double eps,
+                               const c10::optional<at::Tensor>& idx) {
+  CHECK_CUDA(x); CHECK_F32(x); CHECK_CONTIG(x); CHECK_CUDA(parts); CHECK_F32(parts); CHECK_CONTIG(parts);
+  TORCH_CHECK(x.dim() == 2 && parts.dim() == 3 && parts.size(1) == x.size(0) && parts.size(2) == x.size(1), "x [T, W], parts [n, T, W]");
+  const int W = x.size(1);
+  at::Tensor out = at::empty({idx ? idx->numel() : x.size(0), W}, x.options().dtype(at::kBFloat16));
+  if (e) { CHECK_CUDA(*e); CHECK_F32(*e); CHECK_CONTIG(*e); TORCH_CHECK(e->sizes() == x.sizes(), "e shape"); }
+  if (idx) { CHECK_CUDA(*idx); TORCH_CHECK(idx->scalar_type() == at::kLong && idx->is_contiguous(), "idx must be int64"); }
+  CHECK_RC(lk_stream_rmsnorm_sums(x.data_ptr<float>(), parts.data_ptr<float>(), (int)s1, (int)parts.size(0), x.size(0), fpo(a_bias, W, "a_bias"),
+                                  e ? e->data_ptr<float>() : nullptr, (float)mult, fpo(w, W, "w"), (float)woff, (float)eps,
+                                  idx ? idx->data_ptr<int64_t>() : nullptr, out.size(0), out.data_ptr(), out.stride(0), W, cur_stream()),
+           "stream_rmsnorm_sums");
+  return out;
+}
+
 at::Tensor softcap(const at::Tensor& z, double cap) {
   CHECK_CUDA(z); CHECK_LASTDIM(z);
   TORCH_CHECK(z.dim() == 2, "logits must be [R, V]");
@@ -2244,6 +2284,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("embed_pos", &embed_pos);
   m.def("stream_embed_errors", []() { return lk_stream_embed_errors(); });
   m.def("stream_rmsnorm", &stream_rmsnorm);
+  m.def("stream_rmsnorm_sums", &stream_rmsnorm_sums);
   m.def("softcap", &softcap);
   m.def("silu_mul_f32", &silu_mul_f32);
   m.def("sigattn_supported", [](int64_t H, int64_t G, int64_t dim, int64_t vdim, int64_t BS, int64_t esz) {
@@ -2342,6 +2383,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("splits") = 0, py::arg("out") = py::none());
   m.def("skinny_splits", &skinny_splits);
   m.def("rows_pair", &rows_pair);
+  m.def("rows_sums", &rows_sums);
+  m.def("rows_sums_supported", &rows_sums_supported);
   m.def("ln_linear", &ln_linear);
   m.def("ln_linear_supported", [](int64_t M, int64_t N, int64_t K) { return lk_ln_rows_supported((int)M, (int)N, (int)K); });
   m.def("attn_linear", &attn_linear);

@@ -38,6 +38,10 @@ int lk_attn_rows(const void* qkv, long qs, int nh, float scale, const void* w, c
                  hipStream_t st);
 int lk_rows_pair(const void* x1, long ldx1, const void* w1, void* y1, const void* x2, long ldx2, const void* w2, void* y2, int M, int N, int K,
                  int wide, hipStream_t st);
+constexpr int kMaxSums = 16;
+int lk_rows_sums_parts(int M, int N, int K1, int K2, int* s1);
+int lk_rows_sums(const void* x1, long ldx1, const void* w1, int K1, const void* x2, long ldx2, const void* w2, int K2, float* p, int M, int N,
+                 hipStream_t st);
 bool lk_rows_gemm_supported(int M, int N, int K, int epi);
 // epi: 0 none, 1 SwiGLU, 2 bias, 3 bias + GELU, 4 bias + ReLU, 5 bf16(bias) + the residual rows r (elsewhere null)
 int lk_rows_gemm(const void* x, const void* w, const void* b, const void* r, long ldr, void* y, int M, int N, int K, long ldx, long ldy, int epi,
@@ -262,6 +266,8 @@ int lk_stream_embed_errors();  // ids / positions outside their tables seen by l
 int lk_stream_rmsnorm(float* x, const void* a, long as, const float* a_bias, const void* b, long bs, const float* e, float m, const float* w,
                       float woff, float eps, const long* idx, long out_rows, void* out, long os, int W, int esz,
                       hipStream_t st);
+int lk_stream_rmsnorm_sums(float* x, const float* parts, int s1, int n, long rows, const float* a_bias, const float* e, float m, const float* w,
+                           float woff, float eps, const long* idx, long out_rows, void* out, long os, int W, hipStream_t st);
 int lk_silu_mul_f32(const float* x, long xs, float* out, long os, long rows, int I, hipStream_t st);
 int lk_softcap(const void* in, long is, float cap, float* out, long os, long rows, int V, int esz, hipStream_t st);
 

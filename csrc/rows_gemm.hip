@@ -99,6 +99,44 @@ __global__ __launch_bounds__(64 * kRgWaves, 1) void rows_pair_kernel(const bf16_
   rows_tile<MT, NT, NS, RG_NONE>(up ? X2 : X1, up ? W2 : W1, nullptr, nullptr, 0, up ? Y2 : Y1, M, N, K, up ? ldx2 : ldx1, N, up ? z - half : z);
 }
 
+// The f32 parts of two products with outputs of one shape, K split over workgroups: grid (8, s1 + s2, column tiles / 8), part z of
+// P [s1 + s2, M, N] is a range of K of the first product (z < s1) or the second.  One row tile.  What bounds a few-row product is the
+// bytes that each CU takes in, X's and W's rows of its tile: where N is narrow a whole-K tile for every CU is 16 or 32 columns, and X is most
+// of what comes.  Tiles of 64 columns over a part of K take half.  64 rows to 2,048 columns, K 4,096 (2,048) beside 5,632:
+// apart 9.5 us each on average -> 11.7 us for both, and the norm that adds the parts takes the 4.8 us it took before.
+template <int MT, int NT, int NS>
+__global__ __launch_bounds__(64 * kRgWaves, 1) void rows_sums_kernel(const bf16_t* __restrict__ X1, long ldx1, const bf16_t* __restrict__ W1,
+                                                                     int K1, const bf16_t* __restrict__ X2, long ldx2,
+                                                                     const bf16_t* __restrict__ W2, int K2, float* __restrict__ P, int M,
+                                                                     int N, int s1) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int z = blockIdx.y, n0 = (blockIdx.z * 8 + blockIdx.x) * (16 * NT);
+  asm volatile("" ::"s"(X1), "s"(W1), "s"(X2), "s"(W2), "s"(P), "s"(ldx1), "s"(ldx2));   // (as in rows_tile)
+  if (n0 >= N) return;
+  const bool second = z >= s1;
+  const bf16_t *const X = second ? X2 : X1, *const W = second ? W2 : W1;
+  const long ldx = second ? ldx2 : ldx1;
+  const int K = second ? K2 : K1, all = K / 64, waves = (second ? (int)gridDim.y - s1 : s1) * kRgWaves;
+  const int q = (second ? z - s1 : z) * kRgWaves + wave, first = q * all / waves, nst = (q + 1) * all / waves - first;
+  const int lrow = lane >> 3;
+  const long k = (long)first * 64 + rg_lane_col(lane);
+  const bf16_t* xs[2 * MT];
+  const bf16_t* ws[2 * NT];
+#pragma unroll
+  for (int i = 0; i < 2 * MT; ++i) xs[i] = X + (long)min(8 * i + lrow, M - 1) * ldx + k;  // rows past M repeat the last one
+#pragma unroll
+  for (int i = 0; i < 2 * NT; ++i) ws[i] = W + (long)(n0 + 8 * i + lrow) * K + k;
+  floatx4 acc[MT][NT];
+  rg_walk<MT, NT, NS>(xs, ws, nst, smem + wave * NS * rg_stage(MT, NT), acc);
+  rg_sums<MT, NT>(smem, acc, [&](int m, const floatx4 (&t)[NT]) {
+    const int row = m * 16 + (lane & 15);
+    if (row >= M) return;
+#pragma unroll
+    for (int n = 0; n < NT; ++n) *reinterpret_cast<floatx4*>(P + ((long)z * M + row) * N + n0 + 16 * n + 4 * (lane >> 4)) = t[n];
+  });
+}
+
 constexpr int ring_stages(int MT, int NT) { return 20 / (MT + NT) > 5 ? 5 : 20 / (MT + NT); }   // as many as 160 KB hold
 
 template <int MT, int NT, int EPI>
@@ -181,6 +219,17 @@ int pair_by_rows(const void* x1, long ldx1, const void* w1, void* y1, const void
   }
 }
 
+template <int MT>
+int launch_sums(const void* x1, long ldx1, const void* w1, int K1, const void* x2, long ldx2, const void* w2, int K2, float* p, int M, int N,
+                int s1, int parts, hipStream_t st) {
+  constexpr int NT = 4, NS = ring_stages(MT, NT), lds = rg_lds(MT, NT, NS);
+  LK_SET_MAX_LDS((rows_sums_kernel<MT, NT, NS>), lds);
+  rows_sums_kernel<MT, NT, NS><<<dim3(8, parts, (N / 64 + 7) / 8), 64 * kRgWaves, lds, st>>>(
+      (const bf16_t*)x1, ldx1, (const bf16_t*)w1, K1, (const bf16_t*)x2, ldx2, (const bf16_t*)w2, K2, p, M, N, s1);
+  LK_CHECK_LAUNCH();
+  return 0;
+}
+
 }  // namespace
 
 // (the epilogue stores 8-byte groups of 4 columns: ldy is a multiple of 4, y 8-byte aligned)
@@ -210,4 +259,32 @@ int lk_rows_pair(const void* x1, long ldx1, const void* w1, void* y1, const void
   if (wide == 2 && N % 64 == 0) return pair_by_rows<4>(x1, ldx1, w1, y1, x2, ldx2, w2, y2, M, N, K, st);
   if (wide && N % 32 == 0) return pair_by_rows<2>(x1, ldx1, w1, y1, x2, ldx2, w2, y2, M, N, K, st);
   return pair_by_rows<1>(x1, ldx1, w1, y1, x2, ldx2, w2, y2, M, N, K, st);
+}
+
+// Parts of x1 w1^T and x2 w2^T (as many as fill the chip's CUs once, split so that the longest K range is shortest): *s1 of the first.
+// 0: not taken.  Up to 16 rows the weights are what comes in and the products apart read them once too; beyond 64 a second row tile would
+// read them again; with less than two stages a wave the ring has nothing in flight.
+int lk_rows_sums_parts(int M, int N, int K1, int K2, int* s1) {
+  if (M < 17 || M > 64 || N < 64 || N > 8192 || N % 64 || K1 % 64 || K2 % 64 || K1 < 64 || K2 < 64) return 0;
+  const int parts = device_cus() / (N / 64);
+  if (parts < 2 || parts > kMaxSums || (K1 + K2) / 64 < 2 * parts * kRgWaves) return 0;   // (two stages a wave)
+  int least = 1 << 30;
+  for (int s = 1; s < parts; ++s) {
+    const auto longest = [](int K, int n) { return (K / 64 + n * kRgWaves - 1) / (n * kRgWaves); };
+    const int t = max(longest(K1, s), longest(K2, parts - s));
+    if (t < least) least = t, *s1 = s;
+  }
+  return parts;
+}
+
+int lk_rows_sums(const void* x1, long ldx1, const void* w1, int K1, const void* x2, long ldx2, const void* w2, int K2, float* p, int M, int N,
+                 hipStream_t st) {
+  int s1 = 0;
+  const int parts = lk_rows_sums_parts(M, N, K1, K2, &s1);
+  if (!parts) return -1;
+  switch ((M + 15) / 16) {
+    case 2: return launch_sums<2>(x1, ldx1, w1, K1, x2, ldx2, w2, K2, p, M, N, s1, parts, st);
+    case 3: return launch_sums<3>(x1, ldx1, w1, K1, x2, ldx2, w2, K2, p, M, N, s1, parts, st);
+    default: return launch_sums<4>(x1, ldx1, w1, K1, x2, ldx2, w2, K2, p, M, N, s1, parts, st);
+  }
 }

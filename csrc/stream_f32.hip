@@ -140,6 +140,60 @@ __global__ __launch_bounds__(256) void stream_rmsnorm_vec_kernel(float* __restri
   }
 }
 
+// The same where a and b are products that come as f32 parts [n, rows, W] (s1 of them a's): each is summed and rounded as the product
+// itself would be.  W % 4 == 0, W <= 1024 MAXV; SP >= n parts are requested together.
+template <int MAXV, int SP>
+__global__ __launch_bounds__(256) void stream_rmsnorm_sums_kernel(float* __restrict__ x, const float* __restrict__ parts, int s1, int n, long plane,
+                                                                  const float* __restrict__ ab, const float* __restrict__ e, float m,
+                                                                  const float* __restrict__ w, float woff, float eps,
+                                                                  const long* __restrict__ idx, bf16_t* __restrict__ out, long os, int W) {
+  // (weights in a larger tensor may lie anywhere)
+  const bool vec = ((reinterpret_cast<uintptr_t>(ab) | reinterpret_cast<uintptr_t>(w)) & 15) == 0;
+  auto ldf4 = [&](const float* p) { return vec ? *reinterpret_cast<const floatx4*>(p) : floatx4{p[0], p[1], p[2], p[3]}; };
+  __shared__ float red[4];
+  const long orow = blockIdx.x, row = idx ? idx[orow] : orow;
+  const int nv = W >> 2;
+  floatx4 v[MAXV];
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < MAXV; ++i) {
+    const int c = threadIdx.x + 256 * i;
+    if (c < nv) {
+      floatx4 p[SP], s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+      for (int k = 0; k < SP; ++k) p[k] = *reinterpret_cast<const floatx4*>(parts + min(k, n - 1) * plane + row * W + 4 * c);
+      floatx4 t = *reinterpret_cast<const floatx4*>(x + row * W + 4 * c), d;
+      const floatx4 z = {0.f, 0.f, 0.f, 0.f};
+      const floatx4 bias = ab ? ldf4(ab + 4 * c) : z;
+      const floatx4 again = e ? *reinterpret_cast<const floatx4*>(e + row * W + 4 * c) : z;
+#pragma unroll
+      for (int k = 0; k < SP; ++k) {
+        if (k < s1) s[0] += p[k];
+        else if (k < n) s[1] += p[k];
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) d[j] = (bf2f(f2bf(s[0][j])) + bias[j]) + bf2f(f2bf(s[1][j]));
+      t += m * d;
+      if (e) t += again;
+      if (!idx) *reinterpret_cast<floatx4*>(x + row * W + 4 * c) = t;
+      v[i] = t;
+      ss += t[0] * t[0] + t[1] * t[1] + t[2] * t[2] + t[3] * t[3];
+    }
+  }
+  ss = block_sum<4>(ss, red);
+  const float inv = 1.f / sqrtf(ss / (float)W + eps);
+#pragma unroll
+  for (int i = 0; i < MAXV; ++i) {
+    const int c = threadIdx.x + 256 * i;
+    if (c < nv) {
+      floatx4 g = {1.f, 1.f, 1.f, 1.f};
+      if (w) g = ldf4(w + 4 * c) + woff;
+      const floatx4 r = v[i] * inv * g;
+      *reinterpret_cast<uint2*>(out + orow * os + 4 * c) = make_uint2(pack_bf2(r[0], r[1]), pack_bf2(r[2], r[3]));
+    }
+  }
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void softcap_kernel(const T* __restrict__ in, long is, float cap, float* __restrict__ out,
                                                       long os, int V) {
@@ -214,6 +268,25 @@ int lk_stream_rmsnorm(float* x, const void* a, long as, const float* a_bias, con
   else
     stream_rmsnorm_kernel<float><<<(unsigned)out_rows, 256, 0, st>>>(x, (const float*)a, as, a_bias, (const float*)b, bs, e, m, w,
                                                                      woff, eps, idx, (float*)out, os, W);
+  LK_CHECK_LAUNCH();
+  return 0;
+}
+
+int lk_stream_rmsnorm_sums(float* x, const float* parts, int s1, int n, long rows, const float* a_bias, const float* e, float m, const float* w,
+                           float woff, float eps, const long* idx, long out_rows, void* out, long os, int W, hipStream_t st) {
+  if (out_rows <= 0) return 0;
+  const auto a16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  if (W < 4 || W % 4 || W > 8192 || n < 2 || n > kMaxSums || s1 < 1 || s1 >= n || !a16(x) || !a16(parts) || !a16(e) ||
+      os % 4 || reinterpret_cast<uintptr_t>(out) % 8)
+    return -1;
+#define LK_SUMS(MAXV, SP)                                                                                                                \
+  stream_rmsnorm_sums_kernel<MAXV, SP><<<(unsigned)out_rows, 256, 0, st>>>(x, parts, s1, n, rows * W, a_bias, e, m, w, woff, eps, idx, \
+                                                                           (bf16_t*)out, os, W)
+  if (W <= 2048 && n <= 8) LK_SUMS(2, 8);
+  else if (W <= 2048) LK_SUMS(2, 16);
+  else if (n <= 8) LK_SUMS(8, 8);
+  else LK_SUMS(8, 16);
+#undef LK_SUMS
   LK_CHECK_LAUNCH();
   return 0;
 }

@@ -7,7 +7,7 @@
 A configurable span of layers runs several times with the same weights; every pass has its own
 KV cache or recurrent state, and the embedding output is added to the stream once before each
 pass after the first.  Mixers: ``models.attention.sigmoid_paged_attention`` (paged K/V) and
-``models.ssm.mamba2_mixer`` (per-sequence state slots).
+``models.ssm.mamba2_mixed`` (per-sequence state slots).
 
 MI355X layout decisions:
   * the residual stream is f32 and never leaves one fused kernel per block: the scaled sum of the
@@ -36,7 +36,7 @@ from .. import ops
 from ..parallel.tp import SINGLE, TPGroup
 from .attention import AttnMeta, SigmoidAttnSpec, sigmoid_paged_attention
 from .configs import LebepelConfig, pad_vocab
-from .ssm import Mamba2Spec, mamba2_mixer
+from .ssm import Mamba2Spec, mamba2_mixed
 
 
 # The q|k|v bias either rides in the projection GEMM's epilogue (False) or is added in f32 by the
@@ -307,8 +307,8 @@ class LebepelModel(nn.Module):
         return self.cache_block_bytes(1)
 
     # ------------------------------------------------------------------ forward
-    def _mixer(self, L: LebepelLayer, h, meta: AttnMeta, cache):
-        """-> (mixer output without its output bias, that bias or None)."""
+    def _mixed(self, L: LebepelLayer, h, meta: AttnMeta, cache):
+        """-> (what the mixer's output projection L.o reads, the projection's bias or None)."""
         if L.type == "attention":
             # the output projection runs bias-free (decode-sized steps then take the weight-streaming GEMMs):
             # its bias is added by the stream update in f32; the q|k|v bias: see FUSE_QKV_BIAS
@@ -316,8 +316,8 @@ class LebepelModel(nn.Module):
             qkv = ops.linear(h, L.qkv) if fuse else ops.linear(h, L.qkv, L.qkv_b)
             att = sigmoid_paged_attention(qkv, cache[0], cache[1], meta, L.spec, L.r1, L.r2, L.pb, self.cfg.norm_eps,
                                           qkv_bias=L.qkv_b if fuse else None)
-            return ops.linear(att, L.o), L.o_b
-        return mamba2_mixer(h, L.in_proj, L.conv_w, L.conv_b, L.dt_bias, L.A_log, L.D, L.mix_norm, L.o, L.spec,
+            return att, L.o_b
+        return mamba2_mixed(h, L.in_proj, L.conv_w, L.conv_b, L.dt_bias, L.A_log, L.D, L.mix_norm, L.spec,
                             self.cfg.norm_eps, cache, meta), None
 
     def forward(self, ids: torch.Tensor, meta: AttnMeta, caches, taps: list = None) -> torch.Tensor:
@@ -327,20 +327,26 @@ class LebepelModel(nn.Module):
         cfg = self.cfg
         m, eps = cfg.residual_mult, cfg.norm_eps
         x, emb = ops.embed_pos(ids, meta.positions, self.embed, self.pos, keep_copy=self.reinject)
-        a = b = ab = None
+        a = b = ab = sums = None
         for run, (li, add_emb) in enumerate(self.runs):
             L = self.layers[li]
             h = ops.stream_rmsnorm(x, a, b, emb if add_emb else None, m, L.norm1, 1.0, eps, out_dtype=self.dtype,
-                                   a_bias=ab)
+                                   a_bias=ab, sums=sums)
             if taps is not None and run:  # the stream after the previous run, before this pass's re-injection
                 taps.append(x - emb if add_emb else x.clone())
-            a, ab = self._mixer(L, h, meta, caches[run])
-            b = ops.linear(ops.linear_swiglu_any(h, L.gate_up), L.down) if L.ff else None
+            y, ab = self._mixed(L, h, meta, caches[run])
+            f = ops.linear_swiglu_any(h, L.gate_up) if L.ff else None
+            # (decode-sized steps: both projections as f32 parts that the next norm adds up)
+            sums = ops.linear_sums(y, L.o, f, L.down) if L.ff and taps is None and self.dtype == torch.bfloat16 else None
+            if sums is None:
+                a, b = ops.linear(y, L.o), ops.linear(f, L.down) if L.ff else None
+            else:
+                a = b = None
         if taps is not None:
             d = a.float() if b is None else a.float() + b.float()
             taps.append(x + m * (d if ab is None else d + ab))
         return ops.stream_rmsnorm(x, a, b, None, m, self.final_norm, 1.0, eps, idx=meta.logits_idx, out_dtype=self.dtype,
-                                  a_bias=ab)
+                                  a_bias=ab, sums=sums)
 
     def head(self, hidden):
         return ops.linear(hidden, self.lm_head)[:, : self.cfg.vocab_size]

@@ -59,6 +59,11 @@ def mamba2_mixer(h, w_in, conv_w, conv_b, dt_bias, A_log, D, norm_w, w_out, spec
     """h [T, W] -> [T, W]: input projection, causal conv + SiLU over [x | B | C], the selective scan
     with an f32 state, gate, grouped RMS norm, output projection.  ``state`` = (conv, ssm) of this
     layer run; dt, the decay and the recurrence are f32."""
+    return ops.linear(mamba2_mixed(h, w_in, conv_w, conv_b, dt_bias, A_log, D, norm_w, spec, eps, state, meta), w_out)
+
+
+def mamba2_mixed(h, w_in, conv_w, conv_b, dt_bias, A_log, D, norm_w, spec: Mamba2Spec, eps: float, state, meta):
+    """The mixer up to its output projection."""
     conv_state, ssm_state = state
     u = ops.linear(h, w_in)
     inner, C = spec.inner, spec.conv_channels
@@ -66,5 +71,4 @@ def mamba2_mixer(h, w_in, conv_w, conv_b, dt_bias, A_log, D, norm_w, w_out, spec
                         meta.max_seq_len)
     y = ops.ssm_scan(xbc, u[:, inner + C:inner + C + spec.heads], spec.heads, spec.vdim, spec.state, spec.groups, dt_bias, A_log, D,
                      ssm_state, meta.seq_cu, meta.state_slots, meta.positions, max_len=meta.max_seq_len)
-    g = ops.gated_group_rmsnorm(y, u[:, :inner], norm_w, spec.norm_groups, eps)
-    return ops.linear(g, w_out)
+    return ops.gated_group_rmsnorm(y, u[:, :inner], norm_w, spec.norm_groups, eps)

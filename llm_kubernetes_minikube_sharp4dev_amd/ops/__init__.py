@@ -948,6 +948,16 @@ def linear_pair(x1, w1, x2, w2):
     return linear(x1, w1), linear(x2, w2)
 
 
+def linear_sums(x1, w1, x2, w2):
+    """(parts, s1): the f32 parts [n, M, N] of x1 w1^T (the first s1) and x2 w2^T in one launch, for ``stream_rmsnorm(sums=...)``;
+    None where the two products run apart."""
+    if use_hip(x1) and x1.dim() == 2 and x2.dim() == 2 and not GEMM_LIBRARY and x1.shape[0] == x2.shape[0] and w1.shape[0] == w2.shape[0]:
+        if (_gemm_ok(x1, w1) and _gemm_ok(x2, w2) and w1.data_ptr() % 16 == 0 and w2.data_ptr() % 16 == 0
+                and lib().rows_sums_supported(x1.shape[0], w1.shape[0], w1.shape[1], w2.shape[1])):
+            return lib().rows_sums(x1, w1, x2, w2)
+    return None
+
+
 # Encoder passes of few rows: the layer norms and the attention run inside the projections behind them (csrc/encoder_rows.hip).  Up to
 # one row tile: a pass of bge-base, cold weights, 8 / 19 / 33 / 64 tokens 480 / 518 / 549 / 599 -> 360 / 410 / 469 / 527 us; 100 tokens
 # (two tiles, each normalised by all of its workgroups) took longer on the device than the norms apart.

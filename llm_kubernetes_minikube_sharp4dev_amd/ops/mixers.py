@@ -44,11 +44,14 @@ def embed_pos(ids, positions, tok, pos, keep_copy: bool = False):
 
 
 def stream_rmsnorm(x, a=None, b=None, e=None, mult: float = 1.0, w=None, w_offset: float = 0.0, eps: float = 1e-5,
-                   idx=None, out_dtype=torch.bfloat16, a_bias=None):
+                   idx=None, out_dtype=torch.bfloat16, a_bias=None, sums=None):
     """``x += mult * (a + a_bias + b) + e`` in place (f32), then ``x / sqrt(mean(x^2) + eps) *
     (w_offset + w)`` in ``out_dtype``.  With ``idx`` (int64 rows) only those rows are computed and
     ``x`` is left as it was.  ``a_bias`` (f32 [W]): the bias of the projection that produced ``a``,
-    added here so that the projection itself runs on the bias-free GEMM kernels."""
+    added here so that the projection itself runs on the bias-free GEMM kernels.  ``sums``: what ``linear_sums`` returned, instead of
+    ``a`` and ``b`` (bf16)."""
+    if sums is not None:
+        return lib().stream_rmsnorm_sums(x, sums[0], sums[1], a_bias, e, float(mult), w, float(w_offset), float(eps), idx)
     if use_hip(x):
         return lib().stream_rmsnorm(x, a, a_bias if a is not None else None, b, e, float(mult), w, float(w_offset),
                                     float(eps), idx, out_dtype)

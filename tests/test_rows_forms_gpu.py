@@ -1,6 +1,10 @@
 """The few-row product's residual epilogue and its widest form."""
+import functools
+
 import pytest
 import torch
+
+from llm_kubernetes_minikube_sharp4dev_amd import ops
 
 pytestmark = pytest.mark.gpu
 
@@ -34,3 +38,36 @@ def test_two_products_in_one_launch(hip, M, N, K, wide):
     w1, w2 = _r(g, N, K, scale=K ** -0.5), _r(g, N, K, scale=K ** -0.5)
     y1, y2 = hip.rows_pair(x1, w1, x2, w2, wide)
     assert torch.equal(y1, hip.rows_linear(x1, w1, None, 0, wide)) and torch.equal(y2, hip.rows_linear(x2, w2, None, 0, wide))
+
+
+@pytest.mark.parametrize("M", [17, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize("N,K1,K2", [(2048, 4096, 5632), (2048, 2048, 5632), (1024, 4096, 4160), (4096, 1024, 1088), (8192, 512, 960)])
+@pytest.mark.parametrize("picked", [False, True])
+def test_sums_of_two_products(hip, M, N, K1, K2, picked):
+    """Two products as f32 parts and the norm that adds them up, against the same in float64 with each product rounded to bf16 once."""
+    g = torch.Generator(device="cuda").manual_seed(M + N + K2)
+    rn = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    x1, x2 = rn(M, K1 + 8).bfloat16()[:, :K1], rn(M, K2).bfloat16()
+    w1, w2 = (rn(N, K1) / K1 ** 0.5).bfloat16(), (rn(N, K2) / K2 ** 0.5).bfloat16()
+    sums = ops.linear_sums(x1, w1, x2, w2)
+    assert sums is not None and sums[0].shape[1:] == (M, N) and 1 <= sums[1] < sums[0].shape[0]
+    a, b = x1.double() @ w1.double().T, x2.double() @ w2.double().T
+    got1, got2 = (functools.reduce(torch.add, s.unbind(0)) for s in (sums[0][:sums[1]], sums[0][sums[1]:]))   # in the norm's order: the same bits
+    for got, want in ((got1, a), (got2, b)):
+        assert (got.double() - want).norm() <= 2 ** -21 * want.norm()   # f32 sums of exact products: some 2^-24 each
+    x, e, bias, w = rn(M, N), rn(M, N), rn(N), rn(N + 1)[1:]   # (weights that are not aligned to four)
+    idx = torch.arange(M - 1, -1, -3, device="cuda") if picked else None
+    want = x.double() + 0.5 * (got1.bfloat16().double() + bias.double() + got2.bfloat16().double()) + e.double()
+    out = want if idx is None else want[idx]
+    out = out / (out.pow(2).mean(-1, keepdim=True) + 1e-5).sqrt() * (1.0 + w.double())
+    x0 = x.clone()
+    y = ops.stream_rmsnorm(x, None, None, e, 0.5, w, 1.0, 1e-5, idx=idx, a_bias=bias, sums=sums)
+    # one bf16 rounding of the result; the stream itself a few f32 roundings of terms of its own size
+    assert (y.double() - out).norm() <= 2 ** -8 * out.norm()
+    assert torch.equal(x, x0) if picked else (x.double() - want).norm() <= 2 ** -18 * want.norm()
+
+
+@pytest.mark.parametrize("M,N,K1,K2", [(16, 2048, 2048, 5632), (65, 2048, 2048, 5632), (64, 2080, 2048, 2048), (64, 2048, 256, 256), (64, 64, 4096, 4096)])
+def test_sums_not_taken(hip, M, N, K1, K2):
+    z = lambda *s: torch.zeros(*s, device="cuda", dtype=torch.bfloat16)  # noqa: E731
+    assert ops.linear_sums(z(M, K1), z(N, K1), z(M, K2), z(N, K2)) is None
