@@ -229,7 +229,7 @@ std::tuple<at::Tensor, at::Tensor> rows_pair(const at::Tensor& x1, const at::Ten
 // f32 parts [s, M, N] of x1 w1^T and x2 w2^T in one launch, and how many belong to the first (csrc/rows_gemm.hip)
 bool rows_sums_supported(int64_t M, int64_t N, int64_t K1, int64_t K2) {
   int s1 = 0;
-  return M <= 64 && N < (1 << 24) && K1 < (1 << 24) && K2 < (1 << 24) && lk_rows_sums_parts((int)M, (int)N, (int)K1, (int)K2, &s1) > 0;
+  return M >= 1 && M <= 64 && N < (1 << 24) && K1 < (1 << 24) && K2 < (1 << 24) && lk_rows_sums_parts((int)M, (int)N, (int)K1, (int)K2, &s1) > 0;
 }
 std::tuple<at::Tensor, int64_t> rows_sums(const at::Tensor& x1, const at::Tensor& w1, const at::Tensor& x2, const at::Tensor& w2) {
   for (const at::Tensor* t : {&x1, &x2}) {
@@ -243,7 +243,7 @@ std::tuple<at::Tensor, int64_t> rows_sums(const at::Tensor& x1, const at::Tensor
   const int M = x1.size(0), N = w1.size(0), K1 = x1.size(1), K2 = x2.size(1);
   int s1 = 0;
   const int parts = lk_rows_sums_parts(M, N, K1, K2, &s1);
-  TORCH_CHECK(parts > 0, "rows_sums: 17 to 64 rows, N and K multiples of 64");
+  TORCH_CHECK(parts > 0, "rows_sums: 1 to 64 rows, N and K multiples of 64");
   at::Tensor p = at::empty({parts, M, N}, x1.options().dtype(at::kFloat));
   CHECK_RC(lk_rows_sums(bp(x1), x1.stride(0), bp(w1), K1, bp(x2), x2.stride(0), bp(w2), K2, p.data_ptr<float>(), M, N, cur_stream()), "rows_sums");
   return {p, s1};

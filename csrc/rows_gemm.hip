@@ -262,10 +262,11 @@ int lk_rows_pair(const void* x1, long ldx1, const void* w1, void* y1, const void
 }
 
 // Parts of x1 w1^T and x2 w2^T (as many as fill the chip's CUs once, split so that the longest K range is shortest): *s1 of the first.
-// 0: not taken.  Up to 16 rows the weights are what comes in and the products apart read them once too; beyond 64 a second row tile would
-// read them again; with less than two stages a wave the ring has nothing in flight.
+// 0: not taken.  Beyond 64 rows a second row tile would read the weights again; with less than two stages a wave the ring has nothing in
+// flight.  Few rows gain the second launch: four steps of a state-space hybrid (above), 1 / 4 / 16 sequences, 1,579 / 1,807 / 2,178 us
+// apart (weight-streaming kernels of up to 16 rows) -> 1,489 / 1,711 / 1,953.
 int lk_rows_sums_parts(int M, int N, int K1, int K2, int* s1) {
-  if (M < 17 || M > 64 || N < 64 || N > 8192 || N % 64 || K1 % 64 || K2 % 64 || K1 < 64 || K2 < 64) return 0;
+  if (M < 1 || M > 64 || N < 64 || N > 8192 || N % 64 || K1 % 64 || K2 % 64 || K1 < 64 || K2 < 64) return 0;
   const int parts = device_cus() / (N / 64);
   if (parts < 2 || parts > kMaxSums || (K1 + K2) / 64 < 2 * parts * kRgWaves) return 0;   // (two stages a wave)
   int least = 1 << 30;
@@ -283,6 +284,7 @@ int lk_rows_sums(const void* x1, long ldx1, const void* w1, int K1, const void* 
   const int parts = lk_rows_sums_parts(M, N, K1, K2, &s1);
   if (!parts) return -1;
   switch ((M + 15) / 16) {
+    case 1: return launch_sums<1>(x1, ldx1, w1, K1, x2, ldx2, w2, K2, p, M, N, s1, parts, st);
     case 2: return launch_sums<2>(x1, ldx1, w1, K1, x2, ldx2, w2, K2, p, M, N, s1, parts, st);
     case 3: return launch_sums<3>(x1, ldx1, w1, K1, x2, ldx2, w2, K2, p, M, N, s1, parts, st);
     default: return launch_sums<4>(x1, ldx1, w1, K1, x2, ldx2, w2, K2, p, M, N, s1, parts, st);

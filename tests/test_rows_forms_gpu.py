@@ -40,7 +40,7 @@ def test_two_products_in_one_launch(hip, M, N, K, wide):
     assert torch.equal(y1, hip.rows_linear(x1, w1, None, 0, wide)) and torch.equal(y2, hip.rows_linear(x2, w2, None, 0, wide))
 
 
-@pytest.mark.parametrize("M", [17, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize("M", [1, 2, 16, 17, 32, 33, 48, 49, 64])
 @pytest.mark.parametrize("N,K1,K2", [(2048, 4096, 5632), (2048, 2048, 5632), (1024, 4096, 4160), (4096, 1024, 1088), (8192, 512, 960)])
 @pytest.mark.parametrize("picked", [False, True])
 def test_sums_of_two_products(hip, M, N, K1, K2, picked):
@@ -67,7 +67,7 @@ def test_sums_of_two_products(hip, M, N, K1, K2, picked):
     assert torch.equal(x, x0) if picked else (x.double() - want).norm() <= 2 ** -18 * want.norm()
 
 
-@pytest.mark.parametrize("M,N,K1,K2", [(16, 2048, 2048, 5632), (65, 2048, 2048, 5632), (64, 2080, 2048, 2048), (64, 2048, 256, 256), (64, 64, 4096, 4096)])
+@pytest.mark.parametrize("M,N,K1,K2", [(0, 2048, 2048, 5632), (65, 2048, 2048, 5632), (64, 2080, 2048, 2048), (64, 2048, 256, 256), (64, 64, 4096, 4096)])
 def test_sums_not_taken(hip, M, N, K1, K2):
     z = lambda *s: torch.zeros(*s, device="cuda", dtype=torch.bfloat16)  # noqa: E731
     assert ops.linear_sums(z(M, K1), z(N, K1), z(M, K2), z(N, K2)) is None
