@@ -288,7 +288,7 @@ __global__ __launch_bounds__(256, 3) void sigattn_stage_kernel(SigParams p, int 
 // ---- decode: workgroup = (sequence, up to 16 heads of one kv group, key split z); its 4 waves
 // take every fourth 32-key step of the split and are summed through LDS in wave order ------------
 // STAGE (bf16, heads up to 128): through LDS-DMA (attn_stage.h).  64 sequences of 700 - 1,200 keys, 16 heads of 128 over 4: 32 us
-// with the fragments straight from the cache.
+// with the fragments straight from the cache (16 rows x 64 bytes a load), 27 us by whole lines.
 template <typename T, int PAD, bool STAGE>
 __global__ __launch_bounds__(256) void sigattn_decode_kernel(SigParams p, int bs_shift, const int* __restrict__ ctx_lens, int Z,
                                                              T* __restrict__ out, long os,
