@@ -64,6 +64,22 @@ LK_DEVICE void stage_q(const bf16_t* qrow, int dim, uint4_t (&qf)[PAD / 32]) {
   }
 }
 
+// K fragments as rows of dim columns: what lies past them in LDS (a row's last chunk again) must not meet the zeros of q as it is, since
+// an infinity or NaN there times zero would reach the scores.  Heads that fill PAD (the common ones) skip it by one scalar branch.
+template <int PAD>
+LK_DEVICE void stage_k_end(int dim, uint4_t (&kf)[2][PAD / 32]) {
+  if (dim == PAD) return;
+  const int g = (threadIdx.x & 63) >> 4;
+#pragma unroll
+  for (int s = 0; s < PAD / 32; ++s) {
+    const bool in = 32 * s + 8 * g < dim;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) kf[t][s][e] = in ? kf[t][s][e] : 0u;
+  }
+}
+
 // Keys [k0, k1) of the workgroup (k0 a multiple of 32); this wave takes part in tiles of [g0, g1) (g0 a multiple of 32; g1 <= g0: none).
 // weights(kb, s0, s1) gives the 8 weights of keys kb + 8 g .. + 7 for column lane & 15 from the raw scores (in
 // that order) as bf16.  Every wave of the workgroup calls this with the same k0 and k1.
@@ -97,7 +113,7 @@ LK_DEVICE void stage_walk(const StageCache& p, bf16_t* lds, uint4_t (&qf)[PAD / 
       if (f < NK) {
         const int q = 64 * f + lane, row = q / CPR, ch = stage_chunk<CPR>(q % CPR, row, -1), h = row >> 4;
         const bf16_t* kr = p.kc + (((long)(h ? pg[1] : pg[0]) * p.G + p.kvh) * p.BS - (h ? at[1] : at[0]) + min(kb + row, k1 - 1)) * p.dim;
-        dma16(off, kr + min(8 * ch, p.dim - 8));   // (columns past dim meet zero queries)
+        dma16(off, kr + min(8 * ch, p.dim - 8));   // (columns past dim are cleared when they are read)
       } else {
         const int h = (f - NK) / (VT / 2), vd = (f - NK) % (VT / 2) * 32 + (lane >> 1), c = (lane ^ (vd >> 2)) & 1;
         const bf16_t* vr = p.vc + ((long)(h ? pg[1] : pg[0]) * p.G + p.kvh) * p.vdim * p.BS + min(kb + 16 * h + 8 * c, (k1 - 1) & ~7) - (h ? at[1] : at[0]);
@@ -138,6 +154,7 @@ LK_DEVICE void stage_walk(const StageCache& p, bf16_t* lds, uint4_t (&qf)[PAD / 
 #pragma unroll
       for (int s = 0; s < KS; ++s) kf[t][s] = ld16(fr + kat[s] + t * (4 * CPR * 8));   // (rows krow and krow + 4 are placed alike)
     __builtin_amdgcn_sched_barrier(0);
+    stage_k_end<PAD>(p.dim, kf);
 #pragma unroll
     for (int s = 0; s < KS; ++s)
 #pragma unroll
@@ -214,6 +231,7 @@ LK_DEVICE void stage_wave(const StageCache& p, bf16_t* lds, uint4_t (&qf)[PAD / 
     __builtin_amdgcn_sched_barrier(0);
     if (kb + 128 < k1) issue(kb + 128);
     __builtin_amdgcn_sched_barrier(0);
+    stage_k_end<PAD>(p.dim, kf);
     floatx4 c[2];
 #pragma unroll
     for (int s = 0; s < KS; ++s)

@@ -90,3 +90,30 @@ def test_a_later_token_reaches_no_earlier_tile(hip, what):
     vc[blk, :, :, 40 % BS] = float("nan")
     bad = run(kc.cuda(), vc.cuda())
     assert torch.equal(bad[:32], clean[:32]) and torch.equal(bad[70:], clean[70:]) and bad[40:64].isnan().all()
+
+
+@pytest.mark.parametrize("dim", [40, 72, 80])
+@pytest.mark.parametrize("what", ["sigmoid", "window"])
+@pytest.mark.parametrize("decode", [False, True])
+def test_infinite_last_columns(hip, what, dim, decode):
+    """Infinities in the last columns of a key, of heads that do not fill their fragments: the sigmoid saturates and the softmax gives
+    minus infinity no weight, as for every other head size."""
+    H, G, BS = 8, 2, 16
+    lens = [(1, 30 + b) for b in range(20)] if decode else [(17, 17)] * 130   # (prompts: enough tiles for the staged form)
+    q, kc, vc, bt, cu, ctx, _ = _step(H, G, dim, dim, BS, lens, 7)
+    q = q.abs()   # (infinity's sign is then the score's)
+    kc[:, :, 3, -8:] = float("inf") if what == "sigmoid" else float("-inf")
+    kc[:, :, 5, -1] = float("-inf")
+    if what == "sigmoid":
+        one = torch.ones(H)
+        fn, extra = (ops.sigmoid_attention_decode if decode else ops.sigmoid_attention_prefill), (H, G, dim, dim, dim ** -0.5, one, one, one)
+    else:
+        fn, extra = (ops.sink_attention_decode if decode else ops.sink_attention_prefill), (
+            H, G, dim, dim, torch.full((H,), dim ** -0.5), ops.MASK_WINDOW, 24, True, None, 0)
+    if decode:
+        got, ref = _both(lambda q, kc, vc, bt, cu, ctx, *a: fn(q, kc, vc, bt, ctx, *a), q, kc, vc, bt, cu, ctx, H, dim, extra)
+    else:
+        got, ref = _both(fn, q, kc, vc, bt, cu, ctx, H, dim, extra)
+    assert ref.isfinite().all()
+    # as test_sigmoid and test_softmax (weights of at most 1, rounded to bf16)
+    assert ((got - ref).abs() <= 2.0 ** -8 * ref.abs() + 6 * 2.0 ** -9 * float(ctx.max()) ** 0.5).all()
