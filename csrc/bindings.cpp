@@ -255,9 +255,9 @@ std::tuple<at::Tensor, at::Tensor> ln_linear(const at::Tensor& s, const at::Tens
   CHECK_CUDA(s); CHECK_BF16(s); CHECK_LASTDIM(s); check_rows16(s, "rows");
   TORCH_CHECK(s.dim() == 2, "rows [M, K]");
   const int M = s.size(0), K = s.size(1), N = w.size(0);
-  for (const at::Tensor* t : {&ln_w, &ln_b, &w, &bias}) {
+  for (const at::Tensor* t : {&ln_w, &ln_b, &w, &bias}) {   // (the bias is read value by value: it may lie anywhere)
     CHECK_CUDA((*t)); CHECK_BF16((*t)); CHECK_CONTIG((*t));
-    TORCH_CHECK(reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0, "weights must be 16-byte aligned");
+    TORCH_CHECK(t == &bias || reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0, "weights must be 16-byte aligned");
   }
   TORCH_CHECK(w.dim() == 2 && w.size(1) == K && ln_w.numel() == K && ln_b.numel() == K && bias.numel() == N, "weight shapes");
   TORCH_CHECK(lk_ln_rows_supported(M, N, K), "ln_linear: M in [1, 4096], K a multiple of 64 up to 768, N of 16");
@@ -271,9 +271,9 @@ std::tuple<at::Tensor, at::Tensor> ln_linear(const at::Tensor& s, const at::Tens
 at::Tensor attn_linear(const at::Tensor& qkv, int64_t nh, double scale, const at::Tensor& w, const at::Tensor& bias, const at::Tensor& residual) {
   CHECK_CUDA(qkv); CHECK_BF16(qkv); CHECK_LASTDIM(qkv); check_rows16(qkv, "qkv");
   CHECK_CUDA(residual); CHECK_BF16(residual); CHECK_LASTDIM(residual);
-  for (const at::Tensor* t : {&w, &bias}) {
+  for (const at::Tensor* t : {&w, &bias}) {   // (the bias is read value by value)
     CHECK_CUDA((*t)); CHECK_BF16((*t)); CHECK_CONTIG((*t));
-    TORCH_CHECK(reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0, "weights must be 16-byte aligned");
+    TORCH_CHECK(t == &bias || reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0, "weights must be 16-byte aligned");
   }
   TORCH_CHECK(qkv.dim() == 2 && w.dim() == 2, "qkv [M, 3 K], w [N, K]");
   const int M = qkv.size(0), N = w.size(0);

@@ -970,18 +970,24 @@ def encoder_rows_ok(h, width: int, inner: int) -> bool:
             and all(lib().ln_linear_supported(h.shape[0], n, width) for n in (3 * width, inner)))
 
 
+def _fused_weight(w, *vectors) -> bool:
+    """Whether the fused encoder launches read a projection's weight and the vectors beside it as they lie: contiguous bf16, and the
+    weight on a 16-byte line."""
+    return all(t is not None and t.dtype == torch.bfloat16 and t.is_contiguous() for t in (w, *vectors)) and w.data_ptr() % 16 == 0
+
+
 def linear_add(x, w, b, residual):
     """x w^T + b, then + residual (each rounded on its own, as the two operations apart round)."""
-    if use_hip(x) and b is not None:
-        est = _rows_cost(x.shape[0], w.shape[0], w.shape[1], 2) if _gemm_ok(x, w) and w.data_ptr() % 16 == 0 else None
-        if est is not None and not GEMM_LIBRARY:
+    if use_hip(x) and not GEMM_LIBRARY and _fused_weight(w, b) and _gemm_ok(x, w):
+        est = _rows_cost(x.shape[0], w.shape[0], w.shape[1], 2)
+        if est is not None:
             return lib().rows_linear(x, w, b, 5, est[1], residual)
     return linear(x, w, b) + residual
 
 
 def ln_linear(s, ln_w, ln_b, eps: float, w, b, act: Optional[str] = None):
     """(act(h w^T + b), h) with h = LN(s); ``act``: None or "gelu"."""
-    if use_hip(s):
+    if use_hip(s) and _fused_weight(w, b, ln_w, ln_b) and ln_w.data_ptr() % 16 == 0 and ln_b.data_ptr() % 16 == 0:
         return lib().ln_linear(s, ln_w, ln_b, eps, w, b, act == "gelu")
     h = layernorm(s, ln_w, ln_b, eps)
     return linear(h, w, b, act=act), h
@@ -991,7 +997,7 @@ def attn_linear_add(qkv, cu, lens_cpu, nh: int, head_dim: int, scale: float, w, 
     """Bidirectional attention over packed rows [q | k | v], the projection of its output and the residual; one launch for one short
     text."""
     K = nh * head_dim
-    if (use_hip(qkv) and not GEMM_LIBRARY and head_dim == 64 and len(lens_cpu) == 1 and lens_cpu[0] == qkv.shape[0]
+    if (use_hip(qkv) and not GEMM_LIBRARY and head_dim == 64 and len(lens_cpu) == 1 and lens_cpu[0] == qkv.shape[0] and _fused_weight(w, b)
             and lib().attn_linear_supported(qkv.shape[0], nh, w.shape[0])):
         return lib().attn_linear(qkv, nh, scale, w, b, residual)
     a = flash_prefill(qkv[:, :K], qkv[:, K:2 * K], qkv[:, 2 * K:], cu, nh, nh, head_dim, scale, False, q_lens_cpu=lens_cpu, tiles=tiles)

@@ -63,3 +63,27 @@ def test_short_texts_take_the_fused_layers(hip):
         finally:
             ops.ENCODER_ROWS = keep
         assert torch.nn.functional.cosine_similarity(got, apart).min() > 0.9999
+
+
+@pytest.mark.parametrize("lens", [[9], [3, 9]])
+def test_parameters_anywhere(hip, lens):
+    """Biases that begin between two 16-byte lines (views of a larger tensor) are taken, as by the launches apart; the rows are the same."""
+    from llm_kubernetes_minikube_sharp4dev_amd.models import build_encoder
+
+    m = build_encoder("bert-tiny", device="cuda").random_init(3)
+    g = torch.Generator("cuda").manual_seed(1)
+    for L in m.layers:
+        for name in ("qkv_b", "o_b", "fc1_b", "fc2_b"):
+            getattr(L, name).copy_(_r(g, getattr(L, name).numel(), scale=0.1))
+    ids = torch.randint(1000, 30000, (sum(lens),), dtype=torch.int32, device="cuda")
+    pos = torch.cat([torch.arange(n, dtype=torch.int32) for n in lens]).cuda()
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32).cuda()
+    want = m(ids, cu, pos, lens)
+    for L in m.layers:
+        for name in ("qkv_b", "o_b", "fc1_b", "fc2_b"):
+            v = getattr(L, name)
+            wide = torch.empty(v.numel() + 1, dtype=v.dtype, device="cuda")
+            wide[1:] = v
+            setattr(L, name, torch.nn.Parameter(wide[1:], requires_grad=False))
+            assert getattr(L, name).data_ptr() % 16
+    assert torch.equal(m(ids, cu, pos, lens), want)
