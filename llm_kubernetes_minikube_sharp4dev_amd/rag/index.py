@@ -179,12 +179,12 @@ class RagIndex:
         if search_fn is not None:
             self._gpu = None
 
-    def search_vectors_async(self, q: np.ndarray | torch.Tensor, top_k: int, wait: bool = False) -> "PendingSearch":
+    def search_vectors_async(self, q: np.ndarray | torch.Tensor, top_k: int) -> "PendingSearch":
         """Launch a batched search without blocking the host: on the GPU the kNN kernels, which leave
-        (scores, ids) in pinned memory, are enqueued on the current stream before an event; :meth:`PendingSearch.result` waits for that event
-        only (an engine thread collects it after its next step, when it has long completed).
-        Elsewhere the search runs synchronously.  ``wait``: the caller asks for the result at once, so
-        the stream is waited for (38 us a search of 20,011 rows with an event behind it, 32 us without)."""
+        (scores, ids) in pinned memory, are enqueued on the current stream before an event;
+        :meth:`PendingSearch.result` waits for that event only (an engine thread collects it after its next
+        step, when it has long completed), not for what other threads enqueue on the stream behind it.
+        Elsewhere the search runs synchronously."""
         k = max(1, top_k)
         n = len(self.chunks)
         if n == 0 or not self._use_gpu():
@@ -204,9 +204,8 @@ class RagIndex:
                   else qt.to(self.device, torch.bfloat16)).reshape(-1, corpus.shape[1]).contiguous()
             host = ops.knn_packed(corpus, norms, qt, min(k, 64), host=True) if qt.is_cuda else None
             if host is not None:
-                ev = torch.cuda.current_stream() if wait else torch.cuda.Event()
-                if not wait:
-                    ev.record()
+                ev = torch.cuda.Event()
+                ev.record()
                 return PendingSearch(host=(host[0].view(torch.float32), host[1], min(k, n)), event=ev)
             qn = ops.row_norms(qt) if qt.is_cuda else qt.float().norm(dim=-1)
             s, i = ops.knn_topk(corpus, norms, qt, qn, min(k, 64))
@@ -227,7 +226,7 @@ class RagIndex:
         if n == 0:
             return [[] for _ in range(len(q))]
         if self._use_gpu():
-            return self.search_vectors_async(q, top_k, wait=True).result()
+            return self.search_vectors_async(q, top_k).result()
         mat = self.matrix()
         qa = np.asarray(q.float().cpu().numpy() if isinstance(q, torch.Tensor) else q, dtype=np.float32)
         if qa.ndim == 1:

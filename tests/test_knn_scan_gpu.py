@@ -4,7 +4,7 @@ import pytest
 import torch
 
 from llm_kubernetes_minikube_sharp4dev_amd import ops
-from llm_kubernetes_minikube_sharp4dev_amd.rag.index import RagChunk, RagIndex
+from llm_kubernetes_minikube_sharp4dev_amd.rag.index import PendingSearch, RagChunk, RagIndex
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -61,3 +61,28 @@ def test_hits_in_pinned_memory(hip):
             assert got.is_pinned() and not got.is_cuda
             torch.cuda.current_stream().synchronize()
             assert torch.equal(got, want.cpu())
+
+
+def test_a_search_waits_for_its_own_work(hip, monkeypatch):
+    """Work that another thread enqueues on the stream behind the search's kernels is not waited for."""
+    g = torch.Generator(device=DEV).manual_seed(6)
+    c, q = (torch.randn(n, 768, device=DEV, generator=g).to(torch.bfloat16) for n in (3000, 2))
+    index = RagIndex(None, backend="gpu", device=DEV)
+    index.chunks = [RagChunk("d#0", "d", "")] * 3000
+    index.set_gpu_corpus(c)
+    want, result = index.search_vectors(q, 5), PendingSearch.result
+    big, out, behind = torch.ones(8192, 8192, device=DEV).bfloat16(), torch.empty(8192, 8192, device=DEV).bfloat16(), torch.cuda.Event()
+    torch.mm(big, big, out=out)
+    torch.cuda.synchronize()
+
+    def work_before_the_wait(pending):
+        for _ in range(200):   # 1.1 TFLOP each: at least 0.08 s
+            torch.mm(big, big, out=out)
+        behind.record()
+        return result(pending)
+
+    monkeypatch.setattr(PendingSearch, "result", work_before_the_wait)
+    got = index.search_vectors(q, 5)
+    done = behind.query()
+    torch.cuda.synchronize()
+    assert got == want and not done
