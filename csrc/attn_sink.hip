@@ -779,7 +779,8 @@ int lk_sinkattn_prefill(const void* q, long qs, const void* kc, const void* vc, 
                                    pool, keep, cap, gelem, oscale);
   if (!shape_ok(p, esz)) return -1;
   const auto al = [](const void* x, int n) { return reinterpret_cast<uintptr_t>(x) % n == 0; };
-  if (esz == 2 && pad_of(dim, vdim) <= kStageMaxPad && qs % 8 == 0 && os % 4 == 0 && al(q, 16) && al(kc, 16) && al(vc, 16) && al(pkc, 16) &&
+  // (more tiles than a grid dimension holds: the kernel below with four tiles per workgroup still takes them)
+  if (esz == 2 && ntiles <= 65535 && pad_of(dim, vdim) <= kStageMaxPad && qs % 8 == 0 && os % 4 == 0 && al(q, 16) && al(kc, 16) && al(vc, 16) && al(pkc, 16) &&
       al(pvc, 16) && al(out, 8)) {
     const int pad = pad_of(dim, vdim);
     return pad == 64   ? launch_stage<64>(p, cu_q, ctx_lens, tile_seq, tile_q0, ntiles, out, os, st)

@@ -117,3 +117,34 @@ def test_infinite_last_columns(hip, what, dim, decode):
     assert ref.isfinite().all()
     # as test_sigmoid and test_softmax (weights of at most 1, rounded to bf16)
     assert ((got - ref).abs() <= 2.0 ** -8 * ref.abs() + 6 * 2.0 ** -9 * float(ctx.max()) ** 0.5).all()
+
+
+def test_more_tiles_than_a_grid_takes(hip):
+    """65,536 tiles of a window: more than one grid dimension holds of the staged kernel's, and a quarter of the other kernel's limit."""
+    H, G, dim, BS, long_, short = 1, 1, 64, 16, 65535 * 16, 40
+    g = torch.Generator("cuda").manual_seed(9)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)  # noqa: E731
+    nb = [long_ // BS, 3]
+    kc, vc, q = r(sum(nb), G, BS, dim), r(sum(nb), G, dim, BS), r(long_ + short, H * dim)
+    bt = torch.zeros(2, nb[0], dtype=torch.int32, device="cuda")
+    bt[0], bt[1, :3] = torch.arange(nb[0]), torch.arange(nb[0], sum(nb))
+    scale = torch.full((H,), dim ** -0.5, device="cuda")
+
+    def run(q, bt, lens):
+        out = torch.zeros(q.shape[0], H * dim, dtype=torch.bfloat16, device="cuda")
+        n = torch.tensor(lens, dtype=torch.int32, device="cuda")
+        cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32).cuda()
+        return ops.sink_attention_prefill(q, kc, vc, bt, cu, n, H, G, dim, dim, scale, ops.MASK_WINDOW, 16, False, None, 0, out, q_lens_cpu=lens)
+
+    got = run(q, bt, [long_, short])
+    tail, alone = run(q[:1600], bt, [1600]), run(q[long_:], bt[1:], [short])
+    # the two kernels round the same weights (2^-9 of each) against their f32 sum: as test_softmax
+    for a, b in ((got[:1600], tail), (got[long_:], alone)):
+        assert ((a.float() - b.float()).abs() <= 2.0 ** -7 * b.float().abs() + 5 * 2.0 ** -8).all()
+    last = got[long_ - 16:long_].float()   # the long sequence's last rows, with their keys alone
+    k = kc[nb[0] - 2:nb[0], 0].reshape(32, dim).float()
+    v = vc[nb[0] - 2:nb[0], 0].transpose(1, 2).reshape(32, dim).float()
+    s = q[long_ - 16:long_].float() @ k.T * dim ** -0.5
+    d = torch.arange(16, 32, device="cuda")[:, None] - torch.arange(32, device="cuda")[None]
+    want = torch.softmax(s.masked_fill((d < 0) | (d >= 16), float("-inf")), 1) @ v
+    assert ((last - want).abs() <= 2.0 ** -8 * want.abs() + 5 * 2.0 ** -9).all()
