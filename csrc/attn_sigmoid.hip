@@ -226,7 +226,7 @@ __global__ __launch_bounds__(256) void sigattn_prefill_kernel(SigParams p, const
 // ---- prefill, bf16, heads up to 128: keys and values staged in LDS (attn_stage.h).  4 prompts of 900 - 1,148 tokens, 16 heads of 128 over
 // 4 kv heads: 149 us with the kernel above (four waves over one tile's keys, fragments straight from the cache), 48 us.  blockIdx.y walks the same list of 16-query tiles;
 // those that do not begin a workgroup's run of queries leave at once.
-template <int PAD>
+template <int PAD, bool FULL>
 __global__ __launch_bounds__(256, 3) void sigattn_stage_kernel(SigParams p, int wh, int bs_shift, const int* __restrict__ cu_q,
                                                                const int* __restrict__ ctx_lens, const int* __restrict__ tile_seq,
                                                                const int* __restrict__ tile_q0, bf16_t* __restrict__ out, long os) {
@@ -250,7 +250,7 @@ __global__ __launch_bounds__(256, 3) void sigattn_stage_kernel(SigParams p, int 
   const StageCache c = {reinterpret_cast<const bf16_t*>(p.kc), reinterpret_cast<const bf16_t*>(p.vc), p.bt + (long)b * p.bt_stride,
                         p.G, kvh, p.dim, p.vdim, p.BS, bs_shift};
   // (queries past the chunk's end see nothing)
-  stage_walk<PAD>(c, lds, qf, 0, min(ctx, past + min(q0 + rows, qlen)), 0, qw < qlen ? min(ctx, past + qw + 16) : 0, o,
+  stage_walk<PAD, FULL>(c, lds, qf, 0, min(ctx, past + min(q0 + rows, qlen)), 0, qw < qlen ? min(ctx, past + qw + 16) : 0, o,
                   [&](int kb, const floatx4& s0, const floatx4& s1) {
     const int base = past + qw - kb, d0 = base + n16 - 8 * g;   // d0: distance of the run's first key
     pen[lane] = __builtin_fmaf(r1, __builtin_amdgcn_logf(__builtin_fmaf(r2, (float)max(base + 15 - lane, 0), 1.f)), pb);
@@ -289,7 +289,7 @@ __global__ __launch_bounds__(256, 3) void sigattn_stage_kernel(SigParams p, int 
 // take every fourth 32-key step of the split and are summed through LDS in wave order ------------
 // STAGE (bf16, heads up to 128): through LDS-DMA (attn_stage.h).  64 sequences of 700 - 1,200 keys, 16 heads of 128 over 4: 32 us
 // with the fragments straight from the cache (16 rows x 64 bytes a load), 27 us by whole lines.
-template <typename T, int PAD, bool STAGE>
+template <typename T, int PAD, bool STAGE, bool FULL>
 __global__ __launch_bounds__(256) void sigattn_decode_kernel(SigParams p, int bs_shift, const int* __restrict__ ctx_lens, int Z,
                                                              T* __restrict__ out, long os,
                                                              float* __restrict__ part) {
@@ -317,7 +317,7 @@ __global__ __launch_bounds__(256) void sigattn_decode_kernel(SigParams p, int bs
                           p.G, kvh, p.dim, p.vdim, p.BS, bs_shift};
     const int k1 = min(ctx, 32 * s1);
     const float r1 = p.r1[head], r2 = p.r2[head], hb = p.pb[head];
-    stage_wave<PAD>(c, reinterpret_cast<bf16_t*>(smem), qf, 32 * (s0 + w), k1, o, [&](int kb, const floatx4& c0, const floatx4& c1) {
+    stage_wave<PAD, FULL>(c, reinterpret_cast<bf16_t*>(smem), qf, 32 * (s0 + w), k1, o, [&](int kb, const floatx4& c0, const floatx4& c1) {
       float wt[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
@@ -482,15 +482,15 @@ int launch_prefill(const SigParams& p, const int* cu_q, const int* ctx, const in
   return 0;
 }
 
-template <int PAD>
+template <int PAD, bool FULL>
 int launch_stage(const SigParams& p, const int* cu_q, const int* ctx, const int* ts, const int* tq, int ntiles, void* out, long os,
                  hipStream_t st) {
   if (ntiles > 65535) return -2;
   const int wh = stage_heads(p.H / p.G), shift = (p.BS & (p.BS - 1)) == 0 ? __builtin_ctz(p.BS) : -1;
   const dim3 grid(p.H / wh, ntiles);
   constexpr int lds = stage_lds(PAD) + 4 * 64 * 4;
-  LK_SET_MAX_LDS((sigattn_stage_kernel<PAD>), lds);
-  sigattn_stage_kernel<PAD><<<grid, 256, lds, st>>>(p, wh, shift, cu_q, ctx, ts, tq, (bf16_t*)out, os);
+  LK_SET_MAX_LDS((sigattn_stage_kernel<PAD, FULL>), lds);
+  sigattn_stage_kernel<PAD, FULL><<<grid, 256, lds, st>>>(p, wh, shift, cu_q, ctx, ts, tq, (bf16_t*)out, os);
   LK_CHECK_LAUNCH();
   return 0;
 }
@@ -499,19 +499,21 @@ template <typename T, int PAD>
 int launch_decode(const SigParams& p, const int* ctx, int B, int Z, void* out, long os, float* part, hipStream_t st) {
   const int rep = p.H / p.G;
   dim3 grid(B, p.G * ((rep + 15) / 16), Z);
-  const auto al = [](const void* x) { return reinterpret_cast<uintptr_t>(x) % 16 == 0; };
   constexpr int red = 3 * PAD * 64;   // floats of 3 waves' sums, in bytes: 3 (PAD / 16) 64 * 4 * 4
-  bool staged = false;
   if constexpr (sizeof(T) == 2 && PAD <= kStageMaxPad) {
+    const auto al = [](const void* x) { return reinterpret_cast<uintptr_t>(x) % 16 == 0; };
+    if (p.qs % 8 || !al(p.q) || !al(p.kc) || !al(p.vc)) return -1;   // (refused by the bindings before)
     constexpr int lds = stage_wave_lds(PAD) > red ? stage_wave_lds(PAD) : red;
-    staged = p.qs % 8 == 0 && al(p.q) && al(p.kc) && al(p.vc);
-    if (staged) {
-      LK_SET_MAX_LDS((sigattn_decode_kernel<T, PAD, true>), lds);
-      const int shift = (p.BS & (p.BS - 1)) == 0 ? __builtin_ctz(p.BS) : -1;
-      sigattn_decode_kernel<T, PAD, true><<<grid, 256, lds, st>>>(p, shift, ctx, Z, reinterpret_cast<T*>(out), os, part);
-    }
+    const int shift = (p.BS & (p.BS - 1)) == 0 ? __builtin_ctz(p.BS) : -1;
+    const auto launch = [&](auto full) {
+      LK_SET_MAX_LDS((sigattn_decode_kernel<T, PAD, true, decltype(full)::value>), lds);
+      sigattn_decode_kernel<T, PAD, true, decltype(full)::value><<<grid, 256, lds, st>>>(p, shift, ctx, Z, reinterpret_cast<T*>(out), os, part);
+    };
+    if (p.dim == PAD) launch(std::true_type{});
+    else launch(std::false_type{});
+  } else {
+    sigattn_decode_kernel<T, PAD, false, false><<<grid, 256, red, st>>>(p, 0, ctx, Z, reinterpret_cast<T*>(out), os, part);
   }
-  if (!staged) sigattn_decode_kernel<T, PAD, false><<<grid, 256, red, st>>>(p, 0, ctx, Z, reinterpret_cast<T*>(out), os, part);
   LK_CHECK_LAUNCH();
   if (Z > 1) {
     sigattn_reduce_kernel<T><<<dim3(B, p.H), 256, 0, st>>>(part, Z, p.H, p.vdim, reinterpret_cast<T*>(out), os);
@@ -589,10 +591,12 @@ int lk_sigattn_prefill(const void* q, long qs, const void* kc, const void* vc, c
   const SigParams p = make_params(q, qs, kc, vc, bt, bt_stride, H, G, dim, vdim, BS, scale, r1, r2, pb);
   const auto al = [](const void* x, int n) { return reinterpret_cast<uintptr_t>(x) % n == 0; };
   if (esz == 2 && pad_of(dim, vdim) <= kStageMaxPad && qs % 8 == 0 && os % 4 == 0 && al(q, 16) && al(kc, 16) && al(vc, 16) && al(out, 8)) {
+#define LK_STAGE(PAD) \
+  (dim == PAD ? launch_stage<PAD, true>(p, cu_q, ctx_lens, tile_seq, tile_q0, ntiles, out, os, st) \
+              : launch_stage<PAD, false>(p, cu_q, ctx_lens, tile_seq, tile_q0, ntiles, out, os, st))
     const int pad = pad_of(dim, vdim);
-    return pad == 64   ? launch_stage<64>(p, cu_q, ctx_lens, tile_seq, tile_q0, ntiles, out, os, st)
-           : pad == 96 ? launch_stage<96>(p, cu_q, ctx_lens, tile_seq, tile_q0, ntiles, out, os, st)
-                       : launch_stage<128>(p, cu_q, ctx_lens, tile_seq, tile_q0, ntiles, out, os, st);
+    return pad == 64 ? LK_STAGE(64) : pad == 96 ? LK_STAGE(96) : LK_STAGE(128);
+#undef LK_STAGE
   }
   return esz == 2 ? prefill_t<bf16_t>(p, cu_q, ctx_lens, tile_seq, tile_q0, ntiles, out, os, st)
                   : prefill_t<float>(p, cu_q, ctx_lens, tile_seq, tile_q0, ntiles, out, os, st);

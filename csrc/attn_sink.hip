@@ -336,7 +336,7 @@ __global__ __launch_bounds__(256) void sinkattn_prefill_kernel(SinkParams p, con
 // score exceeds it by more than kDefer: until then weights are at most 2^kDefer, exact alike in bf16 and f32.
 constexpr float kDefer = 8.f, kLog2e = 1.4426950408889634f;
 
-template <int PAD>
+template <int PAD, bool FULL>
 __global__ __launch_bounds__(256, 3) void sinkattn_stage_kernel(SinkParams p, int wh, int bs_shift, const int* __restrict__ cu_q,
                                                                 const int* __restrict__ ctx_lens, const int* __restrict__ tile_seq,
                                                                 const int* __restrict__ tile_q0, bf16_t* __restrict__ out, long os) {
@@ -404,7 +404,7 @@ __global__ __launch_bounds__(256, 3) void sinkattn_stage_kernel(SinkParams p, in
   // the window (or chunk, or all), then what lies behind it: the pooled blocks, or (never both) the kept first positions
 #pragma unroll 1
   for (int pass = 0;; ++pass) {
-    stage_walk<PAD>(c, lds, qf, k0, k1, g0, g1, o, weights);
+    stage_walk<PAD, FULL>(c, lds, qf, k0, k1, g0, g1, o, weights);
     if (pass || (!pooled && p.keep == 0)) break;
     hi = behind(hi) - 1;
     lo = 0;
@@ -442,7 +442,7 @@ __global__ __launch_bounds__(256, 3) void sinkattn_stage_kernel(SinkParams p, in
 // part: [B, H, Z, vdim + 2] f32 = O^T relative to m, then m, l
 // STAGE (bf16, heads up to 128): through LDS-DMA (attn_stage.h).  64 sequences of 700 - 1,200 keys, 16 heads of 128 over 4, window 512 and
 // pooled blocks: 21 us with the fragments straight from the cache, 19 us by whole lines.
-template <typename T, int PAD, bool STAGE>
+template <typename T, int PAD, bool STAGE, bool FULL>
 __global__ __launch_bounds__(256) void sinkattn_decode_kernel(SinkParams p, int bs_shift, const int* __restrict__ ctx_lens, int Z,
                                                               T* __restrict__ out, long os, float* __restrict__ part) {
   constexpr int VT = PAD / 16;
@@ -509,7 +509,7 @@ __global__ __launch_bounds__(256) void sinkattn_decode_kernel(SinkParams p, int 
     int first = k0 + 32 * (s0 + w);
 #pragma unroll 1
     for (int pass = 0;; ++pass) {   // the window's steps of this split, then those behind it
-      stage_wave<PAD>(c, reinterpret_cast<bf16_t*>(smem), qf, first, hi, o, weights);
+      stage_wave<PAD, FULL>(c, reinterpret_cast<bf16_t*>(smem), qf, first, hi, o, weights);
       if (pass || n1 <= 0) break;
       if (pooled) {
         c.kc = reinterpret_cast<const bf16_t*>(p.pkc);
@@ -683,14 +683,14 @@ int launch_prefill(const SinkParams& p, const int* cu_q, const int* ctx, const i
   return 0;
 }
 
-template <int PAD>
+template <int PAD, bool FULL>
 int launch_stage(const SinkParams& p, const int* cu_q, const int* ctx, const int* ts, const int* tq, int ntiles, void* out, long os,
                  hipStream_t st) {
   if (ntiles > 65535) return -2;
   const int wh = stage_heads(p.H / p.G), shift = (p.BS & (p.BS - 1)) == 0 ? __builtin_ctz(p.BS) : -1;
   const dim3 grid(p.H / wh, ntiles);
-  LK_SET_MAX_LDS((sinkattn_stage_kernel<PAD>), stage_lds(PAD));
-  sinkattn_stage_kernel<PAD><<<grid, 256, stage_lds(PAD), st>>>(p, wh, shift, cu_q, ctx, ts, tq, (bf16_t*)out, os);
+  LK_SET_MAX_LDS((sinkattn_stage_kernel<PAD, FULL>), stage_lds(PAD));
+  sinkattn_stage_kernel<PAD, FULL><<<grid, 256, stage_lds(PAD), st>>>(p, wh, shift, cu_q, ctx, ts, tq, (bf16_t*)out, os);
   LK_CHECK_LAUNCH();
   return 0;
 }
@@ -698,20 +698,22 @@ int launch_stage(const SinkParams& p, const int* cu_q, const int* ctx, const int
 template <typename T, int PAD>
 int launch_decode(const SinkParams& p, const int* ctx, int B, int Z, void* out, long os, float* part, hipStream_t st) {
   const int rep = p.H / p.G;
-  const auto al = [](const void* x) { return reinterpret_cast<uintptr_t>(x) % 16 == 0; };
   const dim3 grid(B, p.G * ((rep + 15) / 16), Z);
   constexpr int red = 3 * PAD * 64 + 3 * 64 * 2 * 4;   // bytes of 3 waves' O, m and l
-  bool staged = false;
   if constexpr (sizeof(T) == 2 && PAD <= kStageMaxPad) {
+    const auto al = [](const void* x) { return reinterpret_cast<uintptr_t>(x) % 16 == 0; };
+    if (p.qs % 8 || !al(p.q) || !al(p.kc) || !al(p.vc) || !al(p.pkc) || !al(p.pvc)) return -1;   // (refused by the bindings before)
     constexpr int lds = stage_wave_lds(PAD) > red ? stage_wave_lds(PAD) : red;
-    staged = p.qs % 8 == 0 && al(p.q) && al(p.kc) && al(p.vc) && al(p.pkc) && al(p.pvc);
-    if (staged) {
-      LK_SET_MAX_LDS((sinkattn_decode_kernel<T, PAD, true>), lds);
-      const int shift = (p.BS & (p.BS - 1)) == 0 ? __builtin_ctz(p.BS) : -1;
-      sinkattn_decode_kernel<T, PAD, true><<<grid, 256, lds, st>>>(p, shift, ctx, Z, reinterpret_cast<T*>(out), os, part);
-    }
+    const int shift = (p.BS & (p.BS - 1)) == 0 ? __builtin_ctz(p.BS) : -1;
+    const auto launch = [&](auto full) {
+      LK_SET_MAX_LDS((sinkattn_decode_kernel<T, PAD, true, decltype(full)::value>), lds);
+      sinkattn_decode_kernel<T, PAD, true, decltype(full)::value><<<grid, 256, lds, st>>>(p, shift, ctx, Z, reinterpret_cast<T*>(out), os, part);
+    };
+    if (p.dim == PAD) launch(std::true_type{});
+    else launch(std::false_type{});
+  } else {
+    sinkattn_decode_kernel<T, PAD, false, false><<<grid, 256, red, st>>>(p, 0, ctx, Z, reinterpret_cast<T*>(out), os, part);
   }
-  if (!staged) sinkattn_decode_kernel<T, PAD, false><<<grid, 256, red, st>>>(p, 0, ctx, Z, reinterpret_cast<T*>(out), os, part);
   LK_CHECK_LAUNCH();
   if (Z > 1) {
     sinkattn_reduce_kernel<T><<<dim3(B, p.H), 256, 0, st>>>(p, part, Z, reinterpret_cast<T*>(out), os);
@@ -782,10 +784,12 @@ int lk_sinkattn_prefill(const void* q, long qs, const void* kc, const void* vc, 
   // (more tiles than a grid dimension holds: the kernel below with four tiles per workgroup still takes them)
   if (esz == 2 && ntiles <= 65535 && pad_of(dim, vdim) <= kStageMaxPad && qs % 8 == 0 && os % 4 == 0 && al(q, 16) && al(kc, 16) && al(vc, 16) && al(pkc, 16) &&
       al(pvc, 16) && al(out, 8)) {
+#define LK_STAGE(PAD) \
+  (dim == PAD ? launch_stage<PAD, true>(p, cu_q, ctx_lens, tile_seq, tile_q0, ntiles, out, os, st) \
+              : launch_stage<PAD, false>(p, cu_q, ctx_lens, tile_seq, tile_q0, ntiles, out, os, st))
     const int pad = pad_of(dim, vdim);
-    return pad == 64   ? launch_stage<64>(p, cu_q, ctx_lens, tile_seq, tile_q0, ntiles, out, os, st)
-           : pad == 96 ? launch_stage<96>(p, cu_q, ctx_lens, tile_seq, tile_q0, ntiles, out, os, st)
-                       : launch_stage<128>(p, cu_q, ctx_lens, tile_seq, tile_q0, ntiles, out, os, st);
+    return pad == 64 ? LK_STAGE(64) : pad == 96 ? LK_STAGE(96) : LK_STAGE(128);
+#undef LK_STAGE
   }
   return esz == 2 ? prefill_t<bf16_t>(p, cu_q, ctx_lens, tile_seq, tile_q0, ntiles, out, os, st)
                   : prefill_t<float>(p, cu_q, ctx_lens, tile_seq, tile_q0, ntiles, out, os, st);

@@ -29,6 +29,10 @@ struct StageCache {
   int G, kvh, dim, vdim, BS, bs_shift;   // bs_shift: log2(BS), -1 when BS is no power of two
 };
 
+// What the columns past a head that does not fill PAD hold: they meet zeros of q, and an infinity or NaN there (a piece of the key again)
+// times zero would reach the scores.
+__device__ __attribute__((aligned(16))) const bf16_t stage_zeros[8] = {};
+
 constexpr int kStageBufs = 3;
 constexpr int stage_frags(int PAD) { return 2 * (PAD / 32) + PAD / 16; }   // a multiple of 4: every wave fetches as many
 constexpr int stage_lds(int PAD) { return kStageBufs * stage_frags(PAD) * 1024; }
@@ -64,26 +68,11 @@ LK_DEVICE void stage_q(const bf16_t* qrow, int dim, uint4_t (&qf)[PAD / 32]) {
   }
 }
 
-// K fragments as rows of dim columns: what lies past them in LDS (a row's last chunk again) must not meet the zeros of q as it is, since
-// an infinity or NaN there times zero would reach the scores.  Heads that fill PAD (the common ones) skip it by one scalar branch.
-template <int PAD>
-LK_DEVICE void stage_k_end(int dim, uint4_t (&kf)[2][PAD / 32]) {
-  if (dim == PAD) return;
-  const int g = (threadIdx.x & 63) >> 4;
-#pragma unroll
-  for (int s = 0; s < PAD / 32; ++s) {
-    const bool in = 32 * s + 8 * g < dim;
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) kf[t][s][e] = in ? kf[t][s][e] : 0u;
-  }
-}
-
 // Keys [k0, k1) of the workgroup (k0 a multiple of 32); this wave takes part in tiles of [g0, g1) (g0 a multiple of 32; g1 <= g0: none).
 // weights(kb, s0, s1) gives the 8 weights of keys kb + 8 g .. + 7 for column lane & 15 from the raw scores (in
-// that order) as bf16.  Every wave of the workgroup calls this with the same k0 and k1.
-template <int PAD, typename F>
+// that order) as bf16.  Every wave of the workgroup calls this with the same k0 and k1.  FULL: dim is PAD (the test per request for others
+// took 5 % of a prompt's softmax).
+template <int PAD, bool FULL, typename F>
 LK_DEVICE void stage_walk(const StageCache& p, bf16_t* lds, uint4_t (&qf)[PAD / 32], int k0, int k1, int g0, int g1, floatx4 (&o)[PAD / 16],
                           F weights) {
   constexpr int KS = PAD / 32, VT = PAD / 16, NK = 2 * KS, FR = NK + VT, CPR = PAD / 8;   // CPR: 16-byte chunks of a key row
@@ -113,7 +102,7 @@ LK_DEVICE void stage_walk(const StageCache& p, bf16_t* lds, uint4_t (&qf)[PAD / 
       if (f < NK) {
         const int q = 64 * f + lane, row = q / CPR, ch = stage_chunk<CPR>(q % CPR, row, -1), h = row >> 4;
         const bf16_t* kr = p.kc + (((long)(h ? pg[1] : pg[0]) * p.G + p.kvh) * p.BS - (h ? at[1] : at[0]) + min(kb + row, k1 - 1)) * p.dim;
-        dma16(off, kr + min(8 * ch, p.dim - 8));   // (columns past dim are cleared when they are read)
+        dma16(off, FULL || 8 * ch < p.dim ? kr + 8 * ch : stage_zeros);
       } else {
         const int h = (f - NK) / (VT / 2), vd = (f - NK) % (VT / 2) * 32 + (lane >> 1), c = (lane ^ (vd >> 2)) & 1;
         const bf16_t* vr = p.vc + ((long)(h ? pg[1] : pg[0]) * p.G + p.kvh) * p.vdim * p.BS + min(kb + 16 * h + 8 * c, (k1 - 1) & ~7) - (h ? at[1] : at[0]);
@@ -154,7 +143,6 @@ LK_DEVICE void stage_walk(const StageCache& p, bf16_t* lds, uint4_t (&qf)[PAD / 
 #pragma unroll
       for (int s = 0; s < KS; ++s) kf[t][s] = ld16(fr + kat[s] + t * (4 * CPR * 8));   // (rows krow and krow + 4 are placed alike)
     __builtin_amdgcn_sched_barrier(0);
-    stage_k_end<PAD>(p.dim, kf);
 #pragma unroll
     for (int s = 0; s < KS; ++s)
 #pragma unroll
@@ -180,7 +168,7 @@ LK_DEVICE void stage_walk(const StageCache& p, bf16_t* lds, uint4_t (&qf)[PAD / 
 // are requested before this step's arithmetic.  As fragments straight from the cache, 16 rows x 64 bytes, a CU took 17 KB/us.
 constexpr int stage_wave_lds(int PAD) { return 4 * stage_frags(PAD) * 1024; }
 
-template <int PAD, typename F>
+template <int PAD, bool FULL, typename F>
 LK_DEVICE void stage_wave(const StageCache& p, bf16_t* lds, uint4_t (&qf)[PAD / 32], int first, int k1, floatx4 (&o)[PAD / 16], F weights) {
   constexpr int KS = PAD / 32, VT = PAD / 16, NK = 2 * KS, FR = NK + VT, CPR = PAD / 8;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n16 = lane & 15, g = lane >> 4;
@@ -201,7 +189,7 @@ LK_DEVICE void stage_wave(const StageCache& p, bf16_t* lds, uint4_t (&qf)[PAD / 
       if (f < NK) {
         const int q = 64 * f + lane, row = q / CPR, ch = stage_chunk<CPR>(q % CPR, row, -1), h = row >> 4;
         const bf16_t* kr = p.kc + (((long)(h ? pg[1] : pg[0]) * p.G + p.kvh) * p.BS - (h ? at[1] : at[0]) + min(kb + row, k1 - 1)) * p.dim;
-        dma16<true>(off, kr + min(8 * ch, p.dim - 8));
+        dma16<true>(off, FULL || 8 * ch < p.dim ? kr + 8 * ch : stage_zeros);
       } else {
         const int h = (f - NK) / (VT / 2), vd = (f - NK) % (VT / 2) * 32 + (lane >> 1), c = (lane ^ (vd >> 2)) & 1;
         const bf16_t* vr = p.vc + ((long)pg[h] * p.G + p.kvh) * p.vdim * p.BS + min(kb + 16 * h + 8 * c, (k1 - 1) & ~7) - at[h];
@@ -231,7 +219,6 @@ LK_DEVICE void stage_wave(const StageCache& p, bf16_t* lds, uint4_t (&qf)[PAD / 
     __builtin_amdgcn_sched_barrier(0);
     if (kb + 128 < k1) issue(kb + 128);
     __builtin_amdgcn_sched_barrier(0);
-    stage_k_end<PAD>(p.dim, kf);
     floatx4 c[2];
 #pragma unroll
     for (int s = 0; s < KS; ++s)
