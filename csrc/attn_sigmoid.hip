@@ -582,6 +582,11 @@ int lk_unitnorm_kv_write(void* qkv, long qs, long T, int H, int G, int dim, int 
   return 0;
 }
 
+bool lk_sigattn_staged(long ntiles, int H, int dim, int vdim) {
+  const int pad = pad_of(dim, vdim);
+  return pad && stage_pays(ntiles, H, pad, 0);
+}
+
 int lk_sigattn_prefill(const void* q, long qs, const void* kc, const void* vc, const int* bt, int bt_stride,
                        const int* cu_q, const int* ctx_lens, const int* tile_seq, const int* tile_q0, int ntiles, int H,
                        int G, int dim, int vdim, int BS, float scale, const float* r1, const float* r2, const float* pb,
@@ -590,7 +595,7 @@ int lk_sigattn_prefill(const void* q, long qs, const void* kc, const void* vc, c
   if (!shape_ok(H, G, dim, vdim, BS, esz)) return -1;
   const SigParams p = make_params(q, qs, kc, vc, bt, bt_stride, H, G, dim, vdim, BS, scale, r1, r2, pb);
   const auto al = [](const void* x, int n) { return reinterpret_cast<uintptr_t>(x) % n == 0; };
-  if (esz == 2 && pad_of(dim, vdim) <= kStageMaxPad && qs % 8 == 0 && os % 4 == 0 && al(q, 16) && al(kc, 16) && al(vc, 16) && al(out, 8)) {
+  if (esz == 2 && lk_sigattn_staged(ntiles, H, dim, vdim) && qs % 8 == 0 && os % 4 == 0 && al(q, 16) && al(kc, 16) && al(vc, 16) && al(out, 8)) {
 #define LK_STAGE(PAD) \
   (dim == PAD ? launch_stage<PAD, true>(p, cu_q, ctx_lens, tile_seq, tile_q0, ntiles, out, os, st) \
               : launch_stage<PAD, false>(p, cu_q, ctx_lens, tile_seq, tile_q0, ntiles, out, os, st))

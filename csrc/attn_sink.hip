@@ -772,6 +772,11 @@ int lk_normrope_kv_write(void* qkv, long qs, long T, int H, int G, int dim, int 
   return 0;
 }
 
+bool lk_sinkattn_staged(long ntiles, int H, int dim, int vdim, int window) {
+  const int pad = pad_of(dim, vdim);
+  return pad && stage_pays(ntiles, H, pad, window);
+}
+
 int lk_sinkattn_prefill(const void* q, long qs, const void* kc, const void* vc, const int* bt, int bt_stride, const int* cu_q,
                         const int* ctx_lens, const int* tile_seq, const int* tile_q0, int ntiles, int H, int G, int dim, int vdim,
                         int BS, const float* hscale, int mkind, int msize, int sink, const void* gate, long gs, int gcol, void* out,
@@ -781,9 +786,8 @@ int lk_sinkattn_prefill(const void* q, long qs, const void* kc, const void* vc, 
                                    pool, keep, cap, gelem, oscale);
   if (!shape_ok(p, esz)) return -1;
   const auto al = [](const void* x, int n) { return reinterpret_cast<uintptr_t>(x) % n == 0; };
-  // (more tiles than a grid dimension holds: the kernel below with four tiles per workgroup still takes them)
-  if (esz == 2 && ntiles <= 65535 && pad_of(dim, vdim) <= kStageMaxPad && qs % 8 == 0 && os % 4 == 0 && al(q, 16) && al(kc, 16) && al(vc, 16) && al(pkc, 16) &&
-      al(pvc, 16) && al(out, 8)) {
+  if (esz == 2 && lk_sinkattn_staged(ntiles, H, dim, vdim, mkind == 0 ? 0 : msize) && qs % 8 == 0 && os % 4 == 0 && al(q, 16) && al(kc, 16) &&
+      al(vc, 16) && al(pkc, 16) && al(pvc, 16) && al(out, 8)) {
 #define LK_STAGE(PAD) \
   (dim == PAD ? launch_stage<PAD, true>(p, cu_q, ctx_lens, tile_seq, tile_q0, ntiles, out, os, st) \
               : launch_stage<PAD, false>(p, cu_q, ctx_lens, tile_seq, tile_q0, ntiles, out, os, st))

@@ -45,6 +45,21 @@ LK_DEVICE void stage_wait(int ahead) {  // all but the newest `ahead` tiles of L
   }
   if constexpr (AHEAD > 0) stage_wait<L, AHEAD - 1>(ahead);
 }
+// Whether a step's prompt rows take the staged kernel (PAD: the padded head size; window: the keys that a query sees, 0 for all; the
+// pooled or kept keys behind a window are few).  Staged, a wave walks all keys of its 16 queries, so it needs (tile, head) pairs for
+// every CU, or short walks; else the kernel whose four waves split a tile's keys is faster.  The key counts are on the device: the line
+// is drawn by pairs alone.  Split / staged in us, sigmoid and causal softmax:
+//   16 heads of 128 over 4:  16 rows behind 8,000 keys 193 / 252 and 183 / 286, 512 rows (512 pairs) behind 2,000 66 / 80 and 65 / 94,
+//     1,024 rows 135 / 95 and 129 / 112, 2,048 rows 304 / 130 and 354 / 149;
+//   16 heads of 64:  1,024 rows (1,024 pairs) behind 2,000 keys 68 / 92 and 60 / 119, 2,048 rows 153 / 154 and 237 / 182;
+//   12 heads of 96:  1,536 pairs 0.6 - 1.0 and 0.7 - 1.4 of the time, 2,048 pairs 0.5 - 0.85 and 0.6 - 1.1.
+// At 1,024 pairs of 128 one causal prompt from its first token is slower still (16 heads, 1,024 rows 40 / 45; 8 heads, 2,048 rows 62 / 82),
+// several prompts or a longer past are faster (16 x 64 rows 17 / 10).  Windows of 512: 16 rows 44 / 26, 2,048 rows 68 / 31.
+// (65,535 tiles: the grid)
+inline bool stage_pays(long ntiles, int H, int PAD, int window) {
+  if (PAD > kStageMaxPad || ntiles > 65535) return false;
+  return (window > 0 && window <= 512) || ntiles * H >= (PAD > 96 ? 1024 : 2048);
+}
 inline int stage_heads(int rep) { return rep % 4 == 0 ? 4 : rep % 2 == 0 ? 2 : 1; }   // wh: the most that divide the heads of a kv group
 
 // The place of chunk c among the CPR of key row `row` (dir 1), or the chunk at place c (dir -1): turned by the row, so that the 16 rows

@@ -2287,6 +2287,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("stream_rmsnorm_sums", &stream_rmsnorm_sums);
   m.def("softcap", &softcap);
   m.def("silu_mul_f32", &silu_mul_f32);
+  m.def("sigattn_staged", [](int64_t tiles, int64_t H, int64_t dim, int64_t vdim) { return lk_sigattn_staged(tiles, (int)H, (int)dim, (int)vdim); });
+  m.def("sinkattn_staged", [](int64_t tiles, int64_t H, int64_t dim, int64_t vdim, int64_t window) {
+    return lk_sinkattn_staged(tiles, (int)H, (int)dim, (int)vdim, (int)window);
+  });
   m.def("sigattn_supported", [](int64_t H, int64_t G, int64_t dim, int64_t vdim, int64_t BS, int64_t esz) {
     return lk_sigattn_supported((int)H, (int)G, (int)dim, (int)vdim, (int)BS, (int)esz) != 0;
   });

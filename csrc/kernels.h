@@ -276,6 +276,7 @@ int lk_softcap(const void* in, long is, float cap, float* out, long os, long row
 int lk_sigattn_supported(int H, int G, int dim, int vdim, int BS, int esz);
 int lk_unitnorm_kv_write(void* qkv, long qs, long T, int H, int G, int dim, int vdim, int norm_dim, float eps, void* kc, void* vc,
                          const int* slots, int BS, const void* bias, int esz, hipStream_t st);
+bool lk_sigattn_staged(long ntiles, int H, int dim, int vdim);   // whether bf16 prompt rows go through LDS (attn_stage.h)
 int lk_sigattn_prefill(const void* q, long qs, const void* kc, const void* vc, const int* bt, int bt_stride,
                        const int* cu_q, const int* ctx_lens, const int* tile_seq, const int* tile_q0, int ntiles, int H,
                        int G, int dim, int vdim, int BS, float scale, const float* r1, const float* r2, const float* pb,
@@ -325,6 +326,7 @@ int lk_tanh_(void* x, long xs, long T, int n, int esz, hipStream_t st);
 int lk_normrope_kv_write(void* qkv, long qs, long T, int H, int G, int dim, int vdim, int norm_dim, int norm_vdim, const float* qw,
                          const float* kw, int rot, const float* inv_freq, const int* positions, float eps, void* kc, void* vc,
                          const int* slots, int BS, int v_unit, int esz, hipStream_t st);
+bool lk_sinkattn_staged(long ntiles, int H, int dim, int vdim, int window);
 int lk_sinkattn_prefill(const void* q, long qs, const void* kc, const void* vc, const int* bt, int bt_stride, const int* cu_q,
                         const int* ctx_lens, const int* tile_seq, const int* tile_q0, int ntiles, int H, int G, int dim, int vdim,
                         int BS, const float* hscale, int mkind, int msize, int sink, const void* gate, long gs, int gcol, void* out,

@@ -169,7 +169,8 @@ def _sig_rows(q, k, v, qpos, scale, r1, r2, pb):
 def sigmoid_attention_prefill(q, k_cache, v_cache, block_tables, cu_q, ctx_lens, H: int, G: int, dim: int, vdim: int,
                               scale: float, r1, r2, pb, out, tiles=None, q_lens_cpu=None):
     """Causal sigmoid attention of query chunks over their sequences' cached keys (the chunk's own
-    keys included).  q: rows whose first H * dim columns are the unit-RMS queries; out [T, H * vdim]."""
+    keys included).  q: rows whose first H * dim columns are the unit-RMS queries; out [T, H * vdim].
+    ``tiles``: what ``sig_prefill_tiles`` gives for these chunks (all of them), on the device."""
     if use_hip(q):
         if tiles is None:
             ql = q_lens_cpu if q_lens_cpu is not None else (cu_q[1:] - cu_q[:-1]).tolist()
@@ -507,7 +508,8 @@ def sink_attention_prefill(q, k_cache, v_cache, block_tables, cu_q, ctx_lens, H:
     ``pool_kv_write`` at the logical position b of the same block table.
     ``keep_first`` (window masks, no pooling): positions below it stay visible to every later query.  ``softcap`` >
     0: a score s becomes softcap * tanh(s / softcap) before the softmax.  ``gate_elem``: the gate has one column
-    per output element, ``gate_col + h * vdim + d``, instead of one per head.  ``out_scale``: the f32 result is multiplied by it."""
+    per output element, ``gate_col + h * vdim + d``, instead of one per head.  ``out_scale``: the f32 result is multiplied by it.
+    ``tiles``: what ``sig_prefill_tiles`` gives for these chunks (all of them), on the device."""
     _check_mask_options(mask_kind, pool, keep_first)
     if use_hip(q):
         if tiles is None:

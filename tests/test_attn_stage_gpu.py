@@ -148,3 +148,37 @@ def test_more_tiles_than_a_grid_takes(hip):
     d = torch.arange(16, 32, device="cuda")[:, None] - torch.arange(32, device="cuda")[None]
     want = torch.softmax(s.masked_fill((d < 0) | (d >= 16), float("-inf")), 1) @ v
     assert ((last - want).abs() <= 2.0 ** -8 * want.abs() + 5 * 2.0 ** -9).all()
+
+
+@pytest.mark.parametrize("lens", [[(17, 17)] * 130, [(16, 40), (33, 33), (1, 70)] * 40, [(2100, 2300)]])
+@pytest.mark.parametrize("what", ["sigmoid", "causal", "chunk", "kept"])
+@pytest.mark.parametrize("H,G,dim,vdim,BS", SHAPES[:4])
+def test_many_tiles(hip, H, G, dim, vdim, BS, lens, what):
+    """Steps with tiles enough for the staged kernel at every mask (the few of the tests above take it for short windows alone)."""
+    rows = sum(n for n, _ in lens)
+    if rows == 2100 and (dim, what) != (128, "sigmoid"):
+        pytest.skip("one long prompt: one head size (the reference is slow)")
+    q, kc, vc, bt, cu, ctx, _ = _step(H, G, dim, vdim, BS, lens, 11)
+    g = torch.Generator().manual_seed(12)
+    tiles = sum(-(-n // 16) for n, _ in lens)
+    if what == "sigmoid":
+        assert hip.sigattn_staged(tiles, H, dim, vdim) == (tiles * H >= (1024 if max(dim, vdim) > 96 else 2048))
+        r1, r2, pb = torch.rand(H, generator=g), torch.rand(H, generator=g), torch.randn(H, generator=g) * 0.1
+        got, ref = _both(ops.sigmoid_attention_prefill, q, kc, vc, bt, cu, ctx, H, vdim, (H, G, dim, vdim, dim ** -0.5, r1, r2, pb))
+        assert ((got - ref).abs() <= 2.0 ** -8 * ref.abs() + 6 * 2.0 ** -9 * float(ctx.max()) ** 0.5).all()   # as test_sigmoid
+    else:
+        kind, kw = {"causal": (ops.MASK_CAUSAL, {}), "chunk": (ops.MASK_CHUNK, {}), "kept": (ops.MASK_WINDOW, dict(keep_first=3))}[what]
+        size = 600 if what == "chunk" else 24
+        got, ref = _both(ops.sink_attention_prefill, q, kc, vc, bt, cu, ctx, H, vdim,
+                         (H, G, dim, vdim, torch.rand(H, generator=g) * dim ** -0.5, kind, size, False, None, 0), **kw)
+        assert ((got - ref).abs() <= 2.0 ** -8 * ref.abs() + 5 * 2.0 ** -9).all()   # as test_softmax
+
+
+@pytest.mark.parametrize("tiles,H,dim,window,staged", [
+    (1, 16, 128, 0, False), (32, 16, 128, 0, False), (64, 16, 128, 0, True), (63, 16, 128, 600, False), (1, 16, 128, 512, True), (65535, 1, 64, 512, True),
+    (65536, 16, 128, 512, False), (64, 16, 64, 0, False), (128, 16, 64, 0, True), (170, 12, 96, 513, False), (171, 12, 96, 513, True), (4096, 16, 192, 512, False)])
+def test_line_between_the_kernels(hip, tiles, H, dim, window, staged):
+    """Portions of few tiles over many keys keep the kernel that splits a tile's keys over four waves, on both sides of the measured line."""
+    assert hip.sinkattn_staged(tiles, H, dim, dim, window) == staged
+    if window == 0:
+        assert hip.sigattn_staged(tiles, H, dim, dim) == staged
