@@ -23,18 +23,30 @@ namespace {
 
 enum { RG_NONE = 0, RG_SWIGLU = 1, RG_BIAS = 2, RG_GELU = 3, RG_RELU = 4, RG_ADD = 5 };
 
+// Grid (8 XCDs, row tiles, column tiles / 8 rounded up): the row tiles of a column tile follow one another on one XCD, whose L2 then has the
+// weight rows.  From z = spread on (rows_spread: the last columns, fewer than 8) they go around over the XCDs instead.
+// False: a workgroup without work.
+LK_DEVICE bool rg_place(int z, int spread, int columns, int per, int& column, int& item) {
+  column = z * 8 + blockIdx.x;
+  item = blockIdx.y;
+  if (__builtin_expect(z < spread, 1)) return column < columns;
+  const int at = blockIdx.y * 8 + blockIdx.x, rest = columns - z * 8;
+  column = z * 8 + at % rest;
+  item = at / rest;
+  return item < per;
+}
+
 template <int MT, int NT, int NS, int EPI>
 LK_DEVICE void rows_tile(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W, const bf16_t* __restrict__ bias,
-                         const bf16_t* __restrict__ R, long ldr, bf16_t* __restrict__ Y, int M, int N, int K, long ldx, long ldy, int cz) {
+                         const bf16_t* __restrict__ R, long ldr, bf16_t* __restrict__ Y, int M, int N, int K, long ldx, long ldy, int cz, int spread) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int all = K / 64, first = wave * all / kRgWaves, nst = (wave + 1) * all / kRgWaves - first;  // stages of this wave
-  // (8 XCDs, row tiles, column tiles / 8): the row tiles of a column tile follow one another on one XCD, whose L2 then has the
-  // weight rows
   const int cols = EPI == RG_SWIGLU ? N / 2 : N;
-  const int n0 = (cz * 8 + blockIdx.x) * (EPI == RG_SWIGLU ? 8 * NT : 16 * NT), m0 = blockIdx.y * (16 * MT);  // first output column and row
   asm volatile("" ::"s"(X), "s"(W), "s"(Y), "s"(ldx), "s"(ldy));   // (all arguments are loaded before the branch: 0.2 us for a second wait behind it)
-  if (n0 >= cols) return;   // the whole workgroup: the grid holds whole eights of column tiles
+  int column, item;
+  if (!rg_place(cz, spread, N / (16 * NT), (M + 16 * MT - 1) / (16 * MT), column, item)) return;   // the whole workgroup
+  const int n0 = column * (EPI == RG_SWIGLU ? 8 * NT : 16 * NT), m0 = item * (16 * MT);  // first output column and row
   X += (long)m0 * ldx;
   Y += (long)m0 * ldy;
   if constexpr (EPI == RG_ADD) R += (long)m0 * ldr;
@@ -84,8 +96,8 @@ template <int MT, int NT, int NS, int EPI>
 __global__ __launch_bounds__(64 * kRgWaves, 1) void rows_gemm_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                                                                      const bf16_t* __restrict__ bias, const bf16_t* __restrict__ R,
                                                                      long ldr, bf16_t* __restrict__ Y, int M, int N, int K, long ldx,
-                                                                     long ldy) {
-  rows_tile<MT, NT, NS, EPI>(X, W, bias, R, ldr, Y, M, N, K, ldx, ldy, blockIdx.z);
+                                                                     long ldy, int spread) {
+  rows_tile<MT, NT, NS, EPI>(X, W, bias, R, ldr, Y, M, N, K, ldx, ldy, blockIdx.z, spread);
 }
 
 // two plain products of the same sizes, the second in the upper half of the grid's z
@@ -93,13 +105,14 @@ template <int MT, int NT, int NS>
 __global__ __launch_bounds__(64 * kRgWaves, 1) void rows_pair_kernel(const bf16_t* __restrict__ X1, long ldx1, const bf16_t* __restrict__ W1,
                                                                      bf16_t* __restrict__ Y1, const bf16_t* __restrict__ X2, long ldx2,
                                                                      const bf16_t* __restrict__ W2, bf16_t* __restrict__ Y2, int M, int N,
-                                                                     int K) {
+                                                                     int K, int spread) {
   const int half = gridDim.z >> 1, z = blockIdx.z;
   const bool up = z >= half;
-  rows_tile<MT, NT, NS, RG_NONE>(up ? X2 : X1, up ? W2 : W1, nullptr, nullptr, 0, up ? Y2 : Y1, M, N, K, up ? ldx2 : ldx1, N, up ? z - half : z);
+  rows_tile<MT, NT, NS, RG_NONE>(up ? X2 : X1, up ? W2 : W1, nullptr, nullptr, 0, up ? Y2 : Y1, M, N, K, up ? ldx2 : ldx1, N, up ? z - half : z,
+                                 spread);
 }
 
-// The f32 parts of two products with outputs of one shape, K split over workgroups: grid (8, s1 + s2, column tiles / 8), part z of
+// The f32 parts of two products with outputs of one shape, K split over workgroups (grid as above, parts for row tiles): part z of
 // P [s1 + s2, M, N] is a range of K of the first product (z < s1) or the second.  One row tile.  What bounds a few-row product is the
 // bytes that each CU takes in, X's and W's rows of its tile: where N is narrow a whole-K tile for every CU is 16 or 32 columns, and X is most
 // of what comes.  Tiles of 64 columns over a part of K take half.  64 rows to 2,048 columns, K 4,096 (2,048) beside 5,632:
@@ -108,12 +121,13 @@ template <int MT, int NT, int NS>
 __global__ __launch_bounds__(64 * kRgWaves, 1) void rows_sums_kernel(const bf16_t* __restrict__ X1, long ldx1, const bf16_t* __restrict__ W1,
                                                                      int K1, const bf16_t* __restrict__ X2, long ldx2,
                                                                      const bf16_t* __restrict__ W2, int K2, float* __restrict__ P, int M,
-                                                                     int N, int s1) {
+                                                                     int N, int s1, int spread) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int z = blockIdx.y, n0 = (blockIdx.z * 8 + blockIdx.x) * (16 * NT);
   asm volatile("" ::"s"(X1), "s"(W1), "s"(X2), "s"(W2), "s"(P), "s"(ldx1), "s"(ldx2));   // (as in rows_tile)
-  if (n0 >= N) return;
+  int column, z;
+  if (!rg_place(blockIdx.z, spread, N / (16 * NT), gridDim.y, column, z)) return;
+  const int n0 = column * (16 * NT);
   const bool second = z >= s1;
   const bf16_t *const X = second ? X2 : X1, *const W = second ? W2 : W1;
   const long ldx = second ? ldx2 : ldx1;
@@ -137,19 +151,6 @@ __global__ __launch_bounds__(64 * kRgWaves, 1) void rows_sums_kernel(const bf16_
   });
 }
 
-constexpr int ring_stages(int MT, int NT) { return 20 / (MT + NT) > 5 ? 5 : 20 / (MT + NT); }   // as many as 160 KB hold
-
-template <int MT, int NT, int EPI>
-int launch(const void* x, const void* w, const void* b, const void* r, long ldr, void* y, int M, int N, int K, long ldx, long ldy, hipStream_t st) {
-  constexpr int NS = ring_stages(MT, NT), lds = rg_lds(MT, NT, NS);
-  LK_SET_MAX_LDS((rows_gemm_kernel<MT, NT, NS, EPI>), lds);
-  const int cols = N / (16 * NT), tiles = (M + 16 * MT - 1) / (16 * MT);
-  rows_gemm_kernel<MT, NT, NS, EPI><<<dim3(8, tiles, (cols + 7) / 8), 64 * kRgWaves, lds, st>>>(
-      (const bf16_t*)x, (const bf16_t*)w, (const bf16_t*)b, (const bf16_t*)r, ldr, (bf16_t*)y, M, N, K, ldx, ldy);
-  LK_CHECK_LAUNCH();
-  return 0;
-}
-
 int device_cus() {
   static const int n = [] {
     int dev = 0, v = 0;
@@ -158,13 +159,39 @@ int device_cus() {
   return n;
 }
 
-// Row tiles per workgroup: its time is its bytes, 16 (MT + NT) rows of K, times the rounds of workgroups.  Where column tiles leave CUs
-// free, fewer rows per workgroup read the same weight rows out of L2 again and end sooner.
-int row_tiles(int M, int cols, int nt) {
-  const int m16 = (M + 15) / 16, cus = device_cus();
-  int best = 4, cost = 1 << 30;
+// rounds of workgroups, one per CU, where the fullest of the 8 XCDs has `most` of them
+int rounds_of(long most) { return (int)((most * 8 + device_cus() - 1) / device_cus()); }
+
+// z from which a launch's last columns (of n products with `per` workgroups a column tile) go around over the XCDs: only where some XCDs would
+// have a round more than the others (36 column tiles of 7 row tiles are 35 workgroups on four XCDs of 32 CUs and 28 on four: 400 x 576 x 1152
+// 8.4 -> 6.1 us); elsewhere the placement's division is 0.3 us for nothing.
+int rows_spread(int cols, int per, int n = 1) {
+  const long eights = (cols + 7) / 8, even = (cols / 8 * per + (cols % 8 * per + 7) / 8);
+  return rounds_of(eights * per * n) > rounds_of(even * n) ? cols / 8 : 1 << 30;
+}
+
+constexpr int ring_stages(int MT, int NT) { return 20 / (MT + NT) > 5 ? 5 : 20 / (MT + NT); }   // as many as 160 KB hold
+
+template <int MT, int NT, int EPI>
+int launch(const void* x, const void* w, const void* b, const void* r, long ldr, void* y, int M, int N, int K, long ldx, long ldy, hipStream_t st) {
+  constexpr int NS = ring_stages(MT, NT), lds = rg_lds(MT, NT, NS);
+  LK_SET_MAX_LDS((rows_gemm_kernel<MT, NT, NS, EPI>), lds);
+  const int cols = N / (16 * NT), tiles = (M + 16 * MT - 1) / (16 * MT);
+  rows_gemm_kernel<MT, NT, NS, EPI><<<dim3(8, tiles, (cols + 7) / 8), 64 * kRgWaves, lds, st>>>(
+      (const bf16_t*)x, (const bf16_t*)w, (const bf16_t*)b, (const bf16_t*)r, ldr, (bf16_t*)y, M, N, K, ldx, ldy, rows_spread(cols, tiles));
+  LK_CHECK_LAUNCH();
+  return 0;
+}
+
+// Row tiles per workgroup: a workgroup's time is its bytes, 16 (MT + NT) rows of K at 58 KB/us, and 1 us more for each one that its CU has had
+// before (its first loads and its sums; the rings leave one workgroup per CU).  Where column tiles leave CUs free, fewer rows per workgroup
+// read the same weight rows out of L2 again and end sooner.
+int row_tiles(int M, int cols, int nt, int K) {
+  const int m16 = (M + 15) / 16;
+  int best = 4;
+  double cost = 1e30;
   for (int mt = m16 < 4 ? m16 : 4; mt >= 1; --mt) {
-    const int rounds = ((m16 + mt - 1) / mt * cols + cus - 1) / cus, c = rounds * (mt + nt);
+    const double c = rounds_of(((long)((m16 + mt - 1) / mt) * cols + 7) / 8) * ((mt + nt) * (K / 32) / 58.0 + 1.0);
     if (c < cost) {
       cost = c;
       best = mt;
@@ -175,7 +202,7 @@ int row_tiles(int M, int cols, int nt) {
 
 template <int NT, int EPI>
 int by_rows(const void* x, const void* w, const void* b, const void* r, long ldr, void* y, int M, int N, int K, long ldx, long ldy, hipStream_t st) {
-  switch (row_tiles(M, N / (16 * NT), NT)) {
+  switch (row_tiles(M, N / (16 * NT), NT, K)) {
     case 1: return launch<1, NT, EPI>(x, w, b, r, ldr, y, M, N, K, ldx, ldy, st);
     case 2: return launch<2, NT, EPI>(x, w, b, r, ldr, y, M, N, K, ldx, ldy, st);
     case 3: return launch<3, NT, EPI>(x, w, b, r, ldr, y, M, N, K, ldx, ldy, st);
@@ -203,7 +230,7 @@ int launch_pair(const void* x1, long ldx1, const void* w1, void* y1, const void*
   LK_SET_MAX_LDS((rows_pair_kernel<MT, NT, NS>), lds);
   const int cols = N / (16 * NT), tiles = (M + 16 * MT - 1) / (16 * MT);
   rows_pair_kernel<MT, NT, NS><<<dim3(8, tiles, (cols + 7) / 8 * 2), 64 * kRgWaves, lds, st>>>(
-      (const bf16_t*)x1, ldx1, (const bf16_t*)w1, (bf16_t*)y1, (const bf16_t*)x2, ldx2, (const bf16_t*)w2, (bf16_t*)y2, M, N, K);
+      (const bf16_t*)x1, ldx1, (const bf16_t*)w1, (bf16_t*)y1, (const bf16_t*)x2, ldx2, (const bf16_t*)w2, (bf16_t*)y2, M, N, K, rows_spread(cols, tiles, 2));
   LK_CHECK_LAUNCH();
   return 0;
 }
@@ -211,7 +238,7 @@ int launch_pair(const void* x1, long ldx1, const void* w1, void* y1, const void*
 template <int NT>
 int pair_by_rows(const void* x1, long ldx1, const void* w1, void* y1, const void* x2, long ldx2, const void* w2, void* y2, int M, int N, int K,
                  hipStream_t st) {
-  switch (row_tiles(M, 2 * (N / (16 * NT)), NT)) {
+  switch (row_tiles(M, 2 * (N / (16 * NT)), NT, K)) {
     case 1: return launch_pair<1, NT>(x1, ldx1, w1, y1, x2, ldx2, w2, y2, M, N, K, st);
     case 2: return launch_pair<2, NT>(x1, ldx1, w1, y1, x2, ldx2, w2, y2, M, N, K, st);
     case 3: return launch_pair<3, NT>(x1, ldx1, w1, y1, x2, ldx2, w2, y2, M, N, K, st);
@@ -225,7 +252,7 @@ int launch_sums(const void* x1, long ldx1, const void* w1, int K1, const void* x
   constexpr int NT = 4, NS = ring_stages(MT, NT), lds = rg_lds(MT, NT, NS);
   LK_SET_MAX_LDS((rows_sums_kernel<MT, NT, NS>), lds);
   rows_sums_kernel<MT, NT, NS><<<dim3(8, parts, (N / 64 + 7) / 8), 64 * kRgWaves, lds, st>>>(
-      (const bf16_t*)x1, ldx1, (const bf16_t*)w1, K1, (const bf16_t*)x2, ldx2, (const bf16_t*)w2, K2, p, M, N, s1);
+      (const bf16_t*)x1, ldx1, (const bf16_t*)w1, K1, (const bf16_t*)x2, ldx2, (const bf16_t*)w2, K2, p, M, N, s1, rows_spread(N / 64, parts));
   LK_CHECK_LAUNCH();
   return 0;
 }

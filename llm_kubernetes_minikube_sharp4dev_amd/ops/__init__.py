@@ -387,62 +387,87 @@ def _decode_bucket(M: int) -> Optional[int]:
 
 
 # Few rows (csrc/rows_gemm.hip, one launch with any epilogue) or the kernels with larger tiles.  A workgroup of the few-row
-# kernel reads 16 (``wide`` True: 32, 2: 64) columns of W -- SwiGLU 2 x 16 or 2 x 32 -- and 16 to 64 rows of X, as many as need the
-# fewest bytes per CU, so its time is
-#   2.6 us + rounds of workgroups (one per CU) x (their bytes / 58 KB/us) + 1 us per round behind the first,
-# and not below W at 4.2 TB/s (a CU's loads into LDS run at 58 - 68 KB/us whatever the depth of the ring).  64 columns only from
-# N 3072 on: below, the narrower forms fill the chip in one round.  The other side: up to 256 rows without a bias the weight-streaming kernel (its two launches,
-# 0.14 us per MB of W, M / 22; 3.5 us for SwiGLU's second launch), else the prefill GEMM (a chain of K / 64 stages
-# whatever M is, as long as its tiles are fewer than CUs).  Measured in hipGraphs, weights cold, few-row / other (us):
-#    64 x  2048 x 2048  6.0 / 10.9    256 x 2048 x 2048  8.8 / 19.7    768 x 2048 x 2048 22.8 / 28.6   1024: 30.3 / 30.2
-#    64 x  2048 x 5632 12.0 / 14.5     64 x 10496 x 2048 14.3 / 18.3   120 x 4096 x 4096 15.5 / 18.1   192: 28.6 / 20.9
-#    64 x 11264 x 2048 (SwiGLU) 14.6 / 18.9             512 x 2048 x 5632 38.6 / 43.9    768: 57.8 / 45.1
-#   bias:  19 x  768 x  768  3.0 / 15.6    512 x 2304 x 768 12.1 / 19.7    768 x 3072 x 768 18.6 / 23.5    2048: 48 / 24.7
+# kernel reads 16 (``wide`` True: 32, 2: 64) columns of W -- SwiGLU 2 x 16 or 2 x 32 -- and 16 to 64 rows of X, so its time is
+#   2.1 us + rounds of workgroups (one per CU, the 8 XCDs alike) x (their bytes / 58 KB/us + 1 us),
+# and not below 2 us and W at 4.9 TB/s, 0.3 of it again for each further row tile (a weight of more than 96 MB, which no L2 keeps, 0.9 for
+# the second): within 10 % of 13,000 launches (30 shapes of W, 17 - 1,024 rows, all forms), GELU 0.3 us per round.  64 columns up to 64 rows only
+# from N 3072 on: below, the narrower forms fill the chip in one round.  The other side: the weight-streaming kernel (``_ws_cost``) where
+# it takes the step, else the prefill tiles (``_tiled_cost``; the choice is the tiles' where they come within 5 % and with SwiGLU, whose tiles
+# take longer than that estimate, the few-row kernel's up to 10 % more).  Measured in hipGraphs, weights cold, few-row / other (us):
+#    64 x  2048 x 2048  6.0 / 11.6    256 x 2048 x 2048  9.1 / 20.0    768 x 2048 x 2048 18.1 / 27.9     64 x 2048 x 5632 12.1 / 15.1
+#    64 x 10496 x 2048 14.4 / 19.3    128 x 4096 x 4096 16.1 / 19.4    192 x 4096 x 4096 18.1 / 21.6    512 x 2048 x 5632 28.3 / 43.8
+#   128 x 16384 x 1024 16.1 / 13.2    192 x 16384 x 1024 21.7 / 15.4   768 x 3072 x 768 15.7 / 11.8      65 x 8192 x 8192 52.8 / 42.0
+#   SwiGLU: 64 x 11264 x 2048 14.6 / 18.9   192 x 4096 x 5632 26.2 / 97   400 x 6144 x 768 17.6 / 12.8   96 x 32768 x 1024 27.2 / 18.1
+#   bias:   19 x  768 x  768  3.0 / 15.6    512 x 2304 x 768 11.4 / 18.0   400 x 576 x 1152 6.4 / 21.3   1000 x 3072 x 768 (GELU) 18.3 / 14.5
+# Over 1,200 of them (M x N x K and epilogue) the picks take 0.4 - 1.0 % more than the best of all forms and kernels, where a rule by bytes per CU
+# alone took 3.8 % more and up to 1.6 times as long as the other side.
 # Widths that neither tiles (N no multiple of 192 or 256) go to the vendor's kernels, which split K for narrow outputs: fitted to
-# within 25 % for N 48 - 11,280, K 256 - 8,192, 17 - 1,024 rows, and taken 10 % lower, since an even choice is worth nothing (few-row / vendor):
-#    64 x  400 x 1024  4.2 / 6.7      64 x 2064 x 1024  5.5 / 8.8     512 x   48 x 8192 24.9 / 9.1     400 x 2064 x 1024 17.4 / 9.4
+# within 25 % for N 48 - 11,280, K 256 - 8,192, 17 - 1,024 rows, and taken 5 % lower, since an even choice is worth nothing (few-row / vendor):
+#    64 x  400 x 1024  3.3 / 6.7      64 x 2064 x 1024  5.5 / 8.8     512 x   48 x 8192 24.9 / 9.1     400 x 2064 x 1024 17.4 / 9.4
 # (past K 8192 more than 16 rows of X do not stay in L2.)  Where the streaming kernel's sum rides in its consumer
 # (linear_add_rmsnorm, linear_rope_kv) the two are level at decode sizes, and those stay as they are.
 ROWS_MAX_M = 1024
 _ROWS_RULE: dict = {}
 
 
-def _rows_cost(M: int, N: int, K: int, epi: int):
-    """(us of the few-row kernel, its ``wide`` argument, us of the other kernels), or None where it does not take the shape."""
-    mt = (M + 15) // 16 if M <= 64 else 4 * ((M + 63) // 64)   # 16-row tiles of X
-    key = ((M + 15) // 16, N, K, epi)
+def _ws_cost(M: int, N: int, K: int, swiglu: bool) -> float:
+    """us of the weight-streaming kernel: its workgroups' bytes at 32 KB/us, 1.2 us for each further round of them, the weight at
+    5.1 TB/s at least, and the sum of its parts of K behind it.  Within 7 % of 600 measured products."""
+    def plan(bn):   # (filled share of the CUs, parts of K), as csrc/skinny_gemm.hip lays a launch out
+        cols, per = (N // 2, bn // 2) if swiglu else (N, bn)
+        if cols % per:
+            return -1.0, 1
+        s = 1
+        while cols // per * s * 2 <= 256 and K % (s * 128) == 0 and K // (s * 2) >= 1024:
+            s *= 2
+        return cols // per * s / (256 * -(-cols // per * s // 256)), s
+
+    full, half, mid = plan(128), plan(64), (-1.0, 1) if swiglu else plan(96)
+    (fill, parts), bn = (full, 128) if full[0] >= 0.7 or 0 <= half[0] <= full[0] else (half, 64)
+    if mid[0] > fill + 1e-9:
+        parts, bn = mid[1], 96
+    rounds = -(-(N // bn * parts) // 256)
+    chain = 3.1 + rounds * (K / parts) * 2 * (bn + 0.54 * 64 * -(-M // 64)) / 32300 + 1.25 * (rounds - 1)
+    return max(chain, 4 + N * K * 2 / 5.07e6) + (2.1 + 2.3e-6 * parts * M * N if parts > 1 else 0)
+
+
+def _rows_cost(M: int, N: int, K: int, epi: int, products: int = 1):
+    """(us of the few-row kernel, its ``wide`` argument, us of the other kernels), or None where it does not take the shape; of one
+    product or of ``products`` like it, in one launch or one after the other."""
+    mt = (M + 15) // 16   # 16-row tiles of X
+    key = (mt, N, K, epi, products)
     if key in _ROWS_RULE:
         return _ROWS_RULE[key]
     est = None
     if 1 <= M <= ROWS_MAX_M and (K <= 8192 or mt == 1) and lib().rows_supported(M, N, K, epi):
-        mb, rows, cus, mt16 = N * K * 2 / 1e6, 16 * mt, device_cus(), (M + 15) // 16
+        mb, cus = N * K * 2 / 1e6, device_cus()
 
         def cost(nt):   # (the row tiles of a workgroup: as csrc/rows_gemm.hip takes them)
-            units, rounds = min((r * (m + nt), r) for m in range(1, min(mt16, 4) + 1) for r in [-(-(-(-mt16 // m) * (N // (16 * nt))) // cus)])
-            return max(2.6 + units * K / 32 / 58 + (rounds - 1), mb / 4.2)
+            chain, rounds, tiles = min((r * ((m + nt) * (K // 32) / 58 + 1), r, t) for m in range(1, min(mt, 4) + 1) for t in [-(-mt // m)]
+                                       for r in [-(-(-(-(t * (N // (16 * nt)) * products) // 8)) * 8 // cus)])
+            again = 0.3 * (tiles - 1) + (0.6 if tiles > 1 and products * mb > 96 else 0)   # (the L2s hold 32 MB)
+            return max(2.1 + chain, 2 + products * mb * (1 + again) / 4.9) + 0.05 * chain + (0.3 * rounds if epi == 3 else 0)
 
         t, wide = (cost(2), False) if epi == 1 else (cost(1), False)
         for nt, form in ((2, True), (4, 2)):
-            if N % (16 * nt) == 0 and (nt == 2 or N >= 3072) and not (nt == 2 and epi == 1) and cost(nt) < t:
+            if N % (16 * nt) == 0 and (nt == 2 or N >= 3072 or M > 64) and not (nt == 2 and epi == 1) and cost(nt) < t:
                 t, wide = cost(nt), form
-        if epi < 2 and rows <= 256:
-            other = min(7.5, 2 + K / 340) + 0.14 * mb + rows / 22 + (3.5 if epi == 1 else 0)
-        elif epi < 2:
-            other = min(20 + K / 256, 4 + K / 64)
+        tiled = _tiled_cost(16 * mt, N, K, epi)
+        if epi < 2 and M <= (WS_SWIGLU_MAX_M if epi == 1 else WS_MAX_M) and _decode_static_ok(N, K, epi == 1):
+            other = _ws_cost(16 * mt, N, K, epi == 1)
+        elif tiled is not None:
+            other = tiled * (1.1 if epi == 1 else 0.95)
         else:
-            other = min(17 + 3 * K / 1024, 6 + K / 64)
-        tiled = N % 256 == 0 or (epi != 1 and N % 192 == 0)
-        if not tiled and not (epi < 2 and rows <= 256 and _decode_static_ok(N, K, epi == 1)):
-            vendor = 5.2 + K / 2048 + 3.1e-9 * rows * N * K + 0.19 * mb + 2.8e-7 * rows * (N + K) + (0 if epi in (0, 2) else 2.7)
-            other = min(other, 0.9 * vendor)
-        est = (t, wide, other)
+            rows = 16 * mt if M <= 64 else 64 * ((M + 63) // 64)
+            other = 0.95 * (5.2 + K / 2048 + 3.1e-9 * rows * N * K + 0.19 * mb + 2.8e-7 * rows * (N + K) + (0 if epi in (0, 2) else 2.7))
+        est = (t, wide, products * other)
     _ROWS_RULE[key] = est
     return est
 
 
-def _rows_rule(M: int, N: int, K: int, epi: int) -> Optional[int]:
+def _rows_rule(M: int, N: int, K: int, epi: int, products: int = 1) -> Optional[int]:
     """None: not the few-row kernel; else its ``wide`` argument (False, True or 2)."""
-    est = _rows_cost(M, N, K, epi)
+    est = _rows_cost(M, N, K, epi, products)
     return est[1] if est is not None and est[0] < est[2] else None
 
 
@@ -451,12 +476,12 @@ def _rows_rule(M: int, N: int, K: int, epi: int) -> Optional[int]:
 _ROWS_TABLE: dict = {}
 
 
-def _rows_choice(M: int, N: int, K: int, epi: int) -> Optional[int]:
+def _rows_choice(M: int, N: int, K: int, epi: int, products: int = 1) -> Optional[int]:
     if epi < 2 and M > LM_HEAD_SKINNY_MAX_M and _ROWS_TABLE:
         key = (_decode_bucket(M), N, K, epi == 1)
         if key in _ROWS_TABLE:
             return _ROWS_TABLE[key]
-    return _rows_rule(M, N, K, epi)
+    return _rows_rule(M, N, K, epi, products)
 
 
 def decode_route(M: int, N: int, K: int, swiglu: bool) -> str:
@@ -942,7 +967,7 @@ def linear_pair(x1, w1, x2, w2):
         M, (N, K) = x1.shape[0], w1.shape
         if (SKINNY_MAX_M < M <= (WS_MAX_M if GEMM_LIBRARY else ROWS_MAX_M) and _gemm_ok(x1, w1) and _gemm_ok(x2, w2)
                 and w1.data_ptr() % 16 == 0 and w2.data_ptr() % 16 == 0):
-            wide = _rows_choice(M, N, K, 0)
+            wide = _rows_choice(M, N, K, 0, 2)
             if wide is not None:
                 return lib().rows_pair(x1, w1, x2, w2, wide)
     return linear(x1, w1), linear(x2, w2)
@@ -1286,6 +1311,35 @@ _TILE_COST = {5: (128, 4.0, 0.6, 1.1, 0.5, 2.0), 4: (192, 5.5, 0.78, 1.0, 0.3, 3
 _TILE_RULE: dict = {}
 
 
+def _tile_times(M: int, N: int, K: int, epi: int, d):
+    """(us of a ``_TILE_COST`` variant, us of the fallback's choice ``d``), by the costs above."""
+    cus, steps = device_cus(), K / 64
+    out_mb = M * (N // 2 if epi == 1 else N) * 2 / 1e6
+
+    def cost(v):
+        bm, ends, c, deep, store, gelu = _TILE_COST[v]
+        waves = -(-(-(-M // bm) * (N // 256)) // cus)
+        return ends + (gelu if epi == 3 else 0) + waves * c * (deep if K >= 4096 else 1.0) * steps + store * out_mb
+
+    if d[0] in _TILE_COST:
+        return cost, cost(d[0])
+    if d[2] > 1:
+        f = min(1.0, -(-M // 256) * (N // d[1]) * d[2] / cus)
+        return cost, 16 + 8 * f + (0.8 + 0.8 * f) * d[1] / 256 * steps / d[2]
+    cols = N // 256 if epi == 1 else N // d[1]
+    return cost, 8 + 1.35 * steps * -(-(-(-M // 256) * cols) // cus)
+
+
+def _tiled_cost(M: int, N: int, K: int, epi: int) -> Optional[float]:
+    """us that :func:`gemm` is estimated to take, or None where no tile takes the width."""
+    d = _gemm_default(M, N, K, epi)
+    if d is None or not (N % 256 == 0 or (epi != 1 and N % 192 == 0)):
+        return None
+    cost, other = _tile_times(M, N, K, epi, d)
+    cfg = _cfg_of(M, N, K, epi)
+    return cost(cfg[0]) if cfg is not None and cfg != d and cfg[0] in _TILE_COST else other
+
+
 def _tile_rule(M: int, N: int, K: int, epi: int):
     d = _gemm_default(M, N, K, epi)
     # (past the rows it was fitted on a launch is many waves, whose stores overlap and which this cost does not describe: the encoder's
@@ -1295,22 +1349,7 @@ def _tile_rule(M: int, N: int, K: int, epi: int):
         return d
     key = (M, N, K, epi, d)
     if key not in _TILE_RULE:
-        cus, steps = device_cus(), K / 64
-        out_mb = M * (N // 2 if epi == 1 else N) * 2 / 1e6
-
-        def cost(v):
-            bm, ends, c, deep, store, gelu = _TILE_COST[v]
-            waves = -(-(-(-M // bm) * (N // 256)) // cus)
-            return ends + (gelu if epi == 3 else 0) + waves * c * (deep if K >= 4096 else 1.0) * steps + store * out_mb
-
-        if d[0] in _TILE_COST:
-            other = cost(d[0])
-        elif d[2] > 1:
-            f = min(1.0, -(-M // 256) * (N // d[1]) * d[2] / cus)
-            other = 16 + 8 * f + (0.8 + 0.8 * f) * d[1] / 256 * steps / d[2]
-        else:
-            cols = N // 256 if epi == 1 else N // d[1]
-            other = 8 + 1.35 * steps * -(-(-(-M // 256) * cols) // cus)
+        cost, other = _tile_times(M, N, K, epi, d)
         best = min(_TILE_COST, key=cost)
         if len(_TILE_RULE) > 4096:
             _TILE_RULE.clear()

@@ -586,3 +586,19 @@ def test_gemm1w_column_split_plan():
     assert not ops._split_applies(8192, 6144, 0)  # 32 x 24: three waves
     assert not ops._split_applies(1024, 4096, 0)  # under a wave: nothing to split
     assert ops.gemm1w_split_cols(600, 28672, 1) == 85  # SwiGLU: 3 x 112 tiles
+
+
+@pytest.mark.parametrize("M,N,K,epi,form", [
+    (768, 3072, 768, 0, None), (1000, 3072, 768, 3, None), (400, 6144, 768, 1, None), (128, 16384, 1024, 0, None), (192, 16384, 1024, 0, None),
+    (96, 32768, 1024, 1, None), (640, 6272, 1024, 1, None), (65, 8192, 8192, 0, None), (400, 1152, 384, 0, True), (400, 576, 1152, 0, True),
+    (192, 4096, 5632, 1, 2), (64, 10496, 2048, 0, 2), (33, 12288, 4096, 1, 2), (64, 2048, 2048, 0, False)])
+def test_few_row_rule_on_measured_shapes(monkeypatch, M, N, K, epi, form):
+    """Rounds of workgroups, weights read again by further row tiles, and what the weight-streaming and tiled kernels take: the measured faster side."""
+    from types import SimpleNamespace
+
+    from llm_kubernetes_minikube_sharp4dev_amd import ops
+
+    monkeypatch.setattr(ops, "lib", lambda: SimpleNamespace(rows_supported=lambda *a: True))
+    monkeypatch.setattr(ops, "_CUS", 256)
+    monkeypatch.setattr(ops, "_ROWS_RULE", {})
+    assert ops._rows_rule(M, N, K, epi) == form

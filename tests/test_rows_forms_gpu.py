@@ -71,3 +71,37 @@ def test_sums_of_two_products(hip, M, N, K1, K2, picked):
 def test_sums_not_taken(hip, M, N, K1, K2):
     z = lambda *s: torch.zeros(*s, device="cuda", dtype=torch.bfloat16)  # noqa: E731
     assert ops.linear_sums(z(M, K1), z(N, K1), z(M, K2), z(N, K2)) is None
+
+
+@pytest.mark.parametrize("M,N,K,epi,wide", [(400, 576, 1152, 3, 1), (400, 1152, 384, 0, 1), (320, 3136, 128, 1, 2), (257, 400, 64, 2, 0), (1000, 2112, 64, 0, 2),
+                                            (16, 16, 64, 0, 0), (4096, 48, 64, 0, 0)])
+def test_last_columns_over_all_xcds(hip, M, N, K, epi, wide):
+    """Column tiles that are no multiple of 8, of several row tiles: every row tile of the last columns is computed once."""
+    g = torch.Generator("cuda").manual_seed(M + N)
+    x, w = _r(g, M, K), _r(g, N, K, scale=K ** -0.5)
+    b = _r(g, N) if epi >= 2 else None
+    y = hip.rows_linear(x, w, b, epi, wide)
+    p = x.double() @ w.double().T
+    if epi == 1:
+        u, v = (t.to(torch.bfloat16).double() for t in p.chunk(2, 1))
+        p = torch.nn.functional.silu(u).to(torch.bfloat16).double() * v
+    elif epi >= 2:
+        p = p + b.double()
+        p = torch.nn.functional.gelu(p) if epi == 3 else p
+    # as tests/test_rows_gemm_gpu.py: one bf16 rounding of an f32 sum, SwiGLU below 7 half steps
+    assert ((y.double() - p).abs() <= (7 if epi == 1 else 1) * 2.0 ** -8 * p.abs() + 2e-5 * K ** 0.5).all()
+    if epi == 0:
+        x2, w2 = _r(g, M, K), _r(g, N, K, scale=K ** -0.5)
+        y1, y2 = hip.rows_pair(x, w, x2, w2, wide)
+        assert torch.equal(y1, y) and torch.equal(y2, hip.rows_linear(x2, w2, None, 0, wide))
+
+
+@pytest.mark.parametrize("M", [1, 64])
+def test_sums_of_odd_column_tiles(hip, M):
+    """33 column tiles of 7 parts: 35 of them on one XCD, unless the last column's parts go around."""
+    g = torch.Generator("cuda").manual_seed(M)
+    x1, x2, w1, w2 = _r(g, M, 2112), _r(g, M, 2816), _r(g, 2112, 2112, scale=2112 ** -0.5), _r(g, 2112, 2816, scale=2816 ** -0.5)
+    parts, s1 = hip.rows_sums(x1, w1, x2, w2)
+    assert parts.shape == (7, M, 2112)
+    for got, want in ((parts[:s1], x1.double() @ w1.double().T), (parts[s1:], x2.double() @ w2.double().T)):
+        assert (got.double().sum(0) - want).norm() <= 2 ** -21 * want.norm()
