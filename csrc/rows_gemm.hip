@@ -290,7 +290,8 @@ int lk_rows_pair(const void* x1, long ldx1, const void* w1, void* y1, const void
 
 // Parts of x1 w1^T and x2 w2^T (as many as fill the chip's CUs once, split so that the longest K range is shortest): *s1 of the first.
 // 0: not taken.  Beyond 64 rows a second row tile would read the weights again; with less than two stages a wave the ring has nothing in
-// flight.  Few rows gain the second launch: four steps of a state-space hybrid (above), 1 / 4 / 16 sequences, 1,579 / 1,807 / 2,178 us
+// flight; outputs of less than 1,024 columns would be more than 16 parts to add up (fewer parts leave CUs without work).  Whether the
+// launch is worth it where it is taken: ops.sums_pay.  Few rows gain the second launch: four steps of a state-space hybrid (above), 1 / 4 / 16 sequences, 1,579 / 1,807 / 2,178 us
 // apart (weight-streaming kernels of up to 16 rows) -> 1,489 / 1,711 / 1,953.
 int lk_rows_sums_parts(int M, int N, int K1, int K2, int* s1) {
   if (M < 1 || M > 64 || N < 64 || N > 8192 || N % 64 || K1 % 64 || K2 % 64 || K1 < 64 || K2 < 64) return 0;

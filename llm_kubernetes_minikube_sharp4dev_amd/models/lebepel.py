@@ -337,7 +337,9 @@ class LebepelModel(nn.Module):
             y, ab = self._mixed(L, h, meta, caches[run])
             f = ops.linear_swiglu_any(h, L.gate_up) if L.ff else None
             # (decode-sized steps: both projections as f32 parts that the next norm adds up)
-            sums = ops.linear_sums(y, L.o, f, L.down) if L.ff and taps is None and self.dtype == torch.bfloat16 else None
+            fused = (L.ff and taps is None and self.dtype == torch.bfloat16
+                     and ops.sums_pay(y.shape[0], L.o.shape[0], L.o.shape[1], L.down.shape[1]))
+            sums = ops.linear_sums(y, L.o, f, L.down) if fused else None
             if sums is None:
                 a, b = ops.linear(y, L.o), ops.linear(f, L.down) if L.ff else None
             else:

@@ -973,9 +973,27 @@ def linear_pair(x1, w1, x2, w2):
     return linear(x1, w1), linear(x2, w2)
 
 
+def sums_pay(M: int, N: int, K1: int, K2: int) -> bool:
+    """Whether :func:`linear_sums` of weights [N, K1] and [N, K2] is worth its launch.  What decides is the longest range of K that a
+    workgroup gets against the mean: where it is longer, part of the chip waits while the weights' stream runs on.  Launches apart and the
+    norm / the sums and theirs, us, weights cold, 1 / 4 / 16 / 64 rows (longest over mean):
+      2048 x (4096 | 5632)  1.07: 15.2 / 17.2 / 20.7 / 25.2 -> 12.4 / 12.8 / 13.1 / 17.3     5120 x (5120 | 5120)  1.5: 31 / 32 / 37 / 54 -> 31 / 31 / 33 / 43
+      4096 x (4096 | 8192)  1.33: 26.5 / 29.1 / 30.9 / 42.7 -> 27.3 / 27.9 / 28.5 / 33.8     8192 x (4096 | 6144)  1.2: 40 / 41 / 42 / 56 -> 42 / 42 / 44 / 53
+      6144 x (6144 | 16384) 1.45: 56 / 65 / 69 / 82 -> 68 / 69 / 73 / 96                     8192 x (8192 | 28672) 1.56: 107 / 118 / 120 / 128 -> 128 / 129 / 137 / 177
+      8192 x (8192 | 8192)  1.0:  57 / 72 / 73 / 81 -> 65 / 66 / 65 / 67 (one or two rows: the matrix-vector kernel at 4.7 TB/s)
+    Weights of up to 64 MB together gain the launch whatever the ranges (8192 x (512 | 960), 1.39: 17.1 / 17.8 / 18.5 / 22.1 -> 16.6 / 17.3 / 18.0 / 21.9)."""
+    if N * (K1 + K2) * 2 <= 64e6:
+        return True
+    parts = device_cus() // max(1, N // 64)
+    if parts < 2 or (parts == 2 and M <= 2):
+        return False
+    longest = min(max(-(-K1 // (256 * s)), -(-K2 // (256 * (parts - s)))) for s in range(1, parts))
+    return longest * 256 * parts <= (1.15 if parts == 2 else 1.3 if M <= 2 else 1.5) * (K1 + K2)
+
+
 def linear_sums(x1, w1, x2, w2):
     """(parts, s1): the f32 parts [n, M, N] of x1 w1^T (the first s1) and x2 w2^T in one launch, for ``stream_rmsnorm(sums=...)``;
-    None where the two products run apart."""
+    None where the two products run apart (a program asks :func:`sums_pay` too)."""
     if use_hip(x1) and x1.dim() == 2 and x2.dim() == 2 and not GEMM_LIBRARY and x1.shape[0] == x2.shape[0] and w1.shape[0] == w2.shape[0]:
         if (_gemm_ok(x1, w1) and _gemm_ok(x2, w2) and w1.data_ptr() % 16 == 0 and w2.data_ptr() % 16 == 0
                 and lib().rows_sums_supported(x1.shape[0], w1.shape[0], w1.shape[1], w2.shape[1])):

@@ -602,3 +602,15 @@ def test_few_row_rule_on_measured_shapes(monkeypatch, M, N, K, epi, form):
     monkeypatch.setattr(ops, "_CUS", 256)
     monkeypatch.setattr(ops, "_ROWS_RULE", {})
     assert ops._rows_rule(M, N, K, epi) == form
+
+
+@pytest.mark.parametrize("M,N,K1,K2,pay", [
+    (1, 2048, 4096, 5632, True), (64, 2048, 4096, 5632, True), (64, 8192, 512, 960, True), (1, 4096, 4096, 8192, False), (4, 4096, 4096, 8192, True),
+    (64, 5120, 5120, 5120, True), (64, 8192, 8192, 28672, False), (64, 6144, 6144, 16384, False), (64, 8192, 2048, 8192, False),
+    (2, 8192, 8192, 8192, False), (64, 8192, 8192, 8192, True)])
+def test_sums_of_two_products_where_they_pay(monkeypatch, M, N, K1, K2, pay):
+    """Ranges of K of different length leave CUs waiting: measured on both sides."""
+    from llm_kubernetes_minikube_sharp4dev_amd import ops
+
+    monkeypatch.setattr(ops, "_CUS", 256)
+    assert ops.sums_pay(M, N, K1, K2) == pay
