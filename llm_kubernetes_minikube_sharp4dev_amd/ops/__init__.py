@@ -1001,15 +1001,19 @@ def linear_sums(x1, w1, x2, w2):
     return None
 
 
-# Encoder passes of few rows: the layer norms and the attention run inside the projections behind them (csrc/encoder_rows.hip).  Up to
-# one row tile: a pass of bge-base, cold weights, 8 / 19 / 33 / 64 tokens 480 / 518 / 549 / 599 -> 360 / 410 / 469 / 527 us; 100 tokens
-# (two tiles, each normalised by all of its workgroups) took longer on the device than the norms apart.
-ENCODER_ROWS = 64
+# Encoder passes of few rows: the layer norms and the attention run inside the projections behind them (csrc/encoder_rows.hip).  Every
+# workgroup normalises all rows, so what a launch saves is lost again with more of them, sooner where the layers are narrow and each of
+# their launches is short: up to 32 rows at width 768, 16 below.  A captured pass, launches apart -> fused, us (cold: everything evicted before):
+#   12 layers of 768, one text of 8 / 16 / 19 / 32 / 48 / 64 tokens: 312 / 326 / 310 / 349 / 358 / 369 -> 256 / 278 / 300 / 337 / 389 / 415,
+#     cold 353 / 367 / 357 / 379 / 382 / 389 -> 281 / 302 / 323 / 356 / 397 / 423; 8 texts of 2 / of 4 tokens 325 / 351 -> 302 / 339
+#   6 layers of 384, one text of 8 / 16 / 22 / 32 / 64 tokens: 131 / 136 / 137 / 144 / 152 -> 127 / 137 / 145 / 152 / 196,
+#     cold 156 / 162 / 161 / 165 / 177 -> 143 / 154 / 160 / 168 / 211
+ENCODER_ROWS = 32
 
 
 def encoder_rows_ok(h, width: int, inner: int) -> bool:
     """Whether :func:`ln_linear` takes these rows in the projections of an encoder layer (``width`` to 3 ``width`` and to ``inner``)."""
-    return (use_hip(h) and h.dtype == torch.bfloat16 and not GEMM_LIBRARY and 1 <= h.shape[0] <= ENCODER_ROWS
+    return (use_hip(h) and h.dtype == torch.bfloat16 and not GEMM_LIBRARY and 1 <= h.shape[0] <= (ENCODER_ROWS if width >= 768 else ENCODER_ROWS // 2)
             and all(lib().ln_linear_supported(h.shape[0], n, width) for n in (3 * width, inner)))
 
 

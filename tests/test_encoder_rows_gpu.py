@@ -46,23 +46,96 @@ def test_attn_linear(hip, M, nh, N):
     assert ((y.double() - want - res.double()).abs() <= bound).all()
 
 
-def test_short_texts_take_the_fused_layers(hip):
-    """One text and several packed ones give the rows that the layers apart give, up to the order of the attention's sums."""
+def _double_forward(m, ids, pos, lens):
+    """The encoder's rows in float64, of the same bf16 weights and nothing rounded on the way."""
+    F, cfg = torch.nn.functional, m.cfg
+    d = lambda t: t.double()  # noqa: E731
+    ln = lambda x, w, b: F.layer_norm(x, (cfg.hidden,), d(w), d(b), cfg.norm_eps)  # noqa: E731
+    h = ln(d(m.tok)[ids.long()] + d(m.pos)[pos.long()] + d(m.typ)[0], m.emb_ln_w, m.emb_ln_b)
+    for L in m.layers:
+        q, k, v = (t.view(-1, m.nh, m.D).transpose(0, 1) for t in F.linear(h, d(L.qkv), d(L.qkv_b)).chunk(3, 1))
+        at, out = 0, []
+        for n in lens:
+            s = slice(at, at + n)
+            p = torch.softmax(q[:, s] @ k[:, s].transpose(1, 2).contiguous() * m.scale, -1)
+            out.append((p @ v[:, s]).transpose(0, 1).reshape(n, -1))
+            at += n
+        h = ln(F.linear(torch.cat(out), d(L.o), d(L.o_b)) + h, L.ln1_w, L.ln1_b)
+        h = ln(F.linear(F.gelu(F.linear(h, d(L.fc1), d(L.fc1_b))), d(L.fc2), d(L.fc2_b)) + h, L.ln2_w, L.ln2_b)
+    return h
+
+
+def _inputs(lens):
+    ids = torch.randint(1000, 30000, (sum(lens),), dtype=torch.int32, device="cuda")
+    pos = torch.cat([torch.arange(n, dtype=torch.int32) for n in lens]).cuda()
+    return ids, torch.tensor([0] + lens).cumsum(0).to(torch.int32).cuda(), pos
+
+
+class _Spy:
+    """The native library, counting calls by name."""
+
+    def __init__(self, lib):
+        self.lib, self.calls = lib, []
+
+    def __getattr__(self, name):
+        f = getattr(self.lib, name)
+
+        def call(*a, **k):
+            if not name.endswith("_supported"):
+                self.calls.append((name, a[3]) if name == "rows_linear" else name)
+            return f(*a, **k)
+        return call
+
+
+@pytest.mark.parametrize("name,lens,norms,attention", [
+    ("bge-base", [1], True, True), ("bge-base", [19], True, True), ("bge-base", [32], True, True), ("bge-base", [33], False, False),
+    ("bge-base", [64], False, False), ("bge-base", [5, 9, 17], True, False), ("bge-base", [5, 9, 33], False, False),
+    ("minilm-l6", [16], True, False), ("minilm-l6", [17], False, False), ("bert-tiny", [16], True, True), ("bert-tiny", [17], False, False), ("bert-tiny", [4, 12], True, False)])
+def test_short_texts_take_the_fused_layers(hip, monkeypatch, name, lens, norms, attention):
+    """Which passes run the norms, and the attention of one text, inside the projections; their rows against float64, no farther from it
+    than the layers apart."""
     from llm_kubernetes_minikube_sharp4dev_amd import ops
     from llm_kubernetes_minikube_sharp4dev_amd.models import build_encoder
 
-    m = build_encoder("bge-base", device="cuda").random_init(3)
-    for lens in ([19], [33], [64], [5, 9, 33]):
-        ids = torch.randint(1000, 30000, (sum(lens),), dtype=torch.int32, device="cuda")
-        pos = torch.cat([torch.arange(n, dtype=torch.int32) for n in lens]).cuda()
-        cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32).cuda()
-        got, keep = m(ids, cu, pos, lens), ops.ENCODER_ROWS
-        try:
-            ops.ENCODER_ROWS = 0
-            apart = m(ids, cu, pos, lens)
-        finally:
-            ops.ENCODER_ROWS = keep
-        assert torch.nn.functional.cosine_similarity(got, apart).min() > 0.9999
+    m = build_encoder(name, device="cuda").random_init(3)
+    ids, cu, pos = _inputs(lens)
+    spy = _Spy(hip)
+    monkeypatch.setattr(ops, "lib", lambda: spy)
+    got = m(ids, cu, pos, lens, pool=False)
+    n = m.cfg.num_layers
+    assert spy.calls.count("ln_linear") == (2 * n - 1 if norms else 0)
+    assert spy.calls.count("attn_linear") == (n if attention else 0)
+    assert spy.calls.count(("rows_linear", 5)) == ((n if attention else 2 * n) if norms else 0)
+    monkeypatch.setattr(ops, "ENCODER_ROWS", 0)
+    apart, want = m(ids, cu, pos, lens, pool=False), _double_forward(m, ids, pos, lens)
+    e, a = ((y.double() - want).norm() / want.norm() for y in (got, apart))
+    # each layer rounds eight tensors on the way to bf16, 2^-9 of a value at most and a third of that on average, alike on both ways
+    assert e <= (8 * n) ** 0.5 * 2.0 ** -9 and e <= 1.2 * a + 2.0 ** -12, (float(e), float(a))
+
+
+def test_product_plus_residual_routes(hip, monkeypatch):
+    """``linear_add`` and ``linear_pair``: one launch where the few-row kernel takes the operands, the same rows where it does not."""
+    from llm_kubernetes_minikube_sharp4dev_amd import ops
+
+    g = torch.Generator("cuda").manual_seed(5)
+    x, w, b, r = _r(g, 19, 768), _r(g, 768, 768, scale=768 ** -0.5), _r(g, 768), _r(g, 19, 768)
+    odd = torch.empty(19, 769, dtype=torch.bfloat16, device="cuda")[:, :768].copy_(x)   # rows that begin between two 16-byte lines
+    spy = _Spy(hip)
+    monkeypatch.setattr(ops, "lib", lambda: spy)
+    one = ops.linear_add(x, w, b, r)
+    assert spy.calls == [("rows_linear", 5)]
+    want = x.double() @ w.double().T + b.double()
+    for y in (one, ops.linear_add(odd, w, b, r), ops.linear_add(x, w, torch.stack([b, b], 1)[:, 0], r)):
+        # the product's and the sum's rounding
+        assert ((y.double() - want - r.double()).abs() <= EPS * (want.abs() + (want + r.double()).abs()) + 1e-4).all()
+    spy.calls.clear()
+    w2 = _r(g, 768, 768, scale=768 ** -0.5)
+    y1, y2 = ops.linear_pair(x, w, r, w2)
+    assert spy.calls == ["rows_pair"]
+    z1, z2 = ops.linear_pair(odd, w, r, w2)
+    assert spy.calls.count("rows_pair") == 1
+    for y, z, p in ((y1, z1, x.double() @ w.double().T), (y2, z2, r.double() @ w2.double().T)):
+        assert ((y.double() - p).abs() <= EPS * p.abs() + 1e-4).all() and ((z.double() - p).abs() <= EPS * p.abs() + 1e-4).all()
 
 
 @pytest.mark.parametrize("lens", [[9], [3, 9]])
