@@ -332,7 +332,7 @@ class FusasunModel(nn.Module):
 
     # ------------------------------------------------------------------ forward
     def _attended(self, L: FusasunLayer, h, meta: AttnMeta, cache):
-        """The mixer's heads, before its output projection."""
+        """The mixer's heads; its output projection runs beside the layer's first gate."""
         W = self.cfg.hidden
         hc = ops.conv_silu(h, 0, W, L.canon, None, cache[-1], meta.seq_cu, meta.state_slots, meta.positions, meta.max_seq_len,
                            act=False)
@@ -342,9 +342,6 @@ class FusasunModel(nn.Module):
             return pooled_window_attention(u, cache, meta, M.spec, M.freq, M.hscale)
         return latent_window_attention(u, M.rows, M.up_rows.off["uv"], M.w_uq, M.w_ukv, M.dq_norm, M.dkv_norm, cache, meta, M.spec, M.freq,
                                        M.hscale, self.cfg.norm_eps, w_heads=M.w_heads)
-
-    def _mixer(self, L: FusasunLayer, h, meta: AttnMeta, cache):
-        return ops.linear(self._attended(L, h, meta, cache), L.mix.o)
 
     def _routes(self, ids) -> list:
         """Every layer's expert routing (None: no experts), known from the token ids."""

@@ -86,6 +86,12 @@ def one_layer(kind, mixer, W, device, dtype, seed=5, eps=1e-5, taps=3, sd=None):
     return m, out
 
 
+def mixed(m, h, meta, cache):
+    """The first layer's mixer as the model's forward runs it: the output projection beside the layer's first gate."""
+    L = m.layers[0]
+    return ops.linear_pair(h, L.rg1, m._attended(L, h, meta, cache), L.mix.o)[1]
+
+
 def run_mixer(m, h, cuts, device, dtype, slot=1, blocks=None, nblocks=40, caches=None):
     """The layer's mixer over ``h`` [T, W] fed in portions of the sizes ``cuts`` (the rest as decode rows)."""
     T = h.shape[0]
@@ -97,7 +103,7 @@ def run_mixer(m, h, cuts, device, dtype, slot=1, blocks=None, nblocks=40, caches
         n = 1 if dec else min(sizes.pop(0), T - at)
         meta = step_meta([(at, n, blocks, slot, dec)], device)
         with torch.inference_mode():
-            y = m._mixer(m.layers[0], h[at:at + n].to(dtype).to(device).contiguous(), meta, caches[0])
+            y = mixed(m, h[at:at + n].to(dtype).to(device).contiguous(), meta, caches[0])
         out.append(y.float().cpu())
         at += n
     return torch.cat(out)
@@ -270,8 +276,8 @@ def test_used_pages_and_slots_do_not_leak(device, dtype):
         ta, tb = [5, 2, 9], [7, 1]
         dev = lambda t: t.to(dtype).to(device).contiguous()
         with torch.inference_mode():
-            y1 = m._mixer(m.layers[0], dev(torch.cat([ha[:30], hb[:20]])), step_meta([(0, 30, ta, 2, False), (0, 20, tb, 0, False)], device), caches[0])
-            y2 = m._mixer(m.layers[0], dev(torch.cat([ha[30:], hb[20:]])), step_meta([(30, 7, ta, 2, False), (20, 1, tb, 0, True)], device), caches[0])
+            y1 = mixed(m, dev(torch.cat([ha[:30], hb[:20]])), step_meta([(0, 30, ta, 2, False), (0, 20, tb, 0, False)], device), caches[0])
+            y2 = mixed(m, dev(torch.cat([ha[30:], hb[20:]])), step_meta([(30, 7, ta, 2, False), (20, 1, tb, 0, True)], device), caches[0])
         got_a = torch.cat([y1[:30], y2[:7]]).float().cpu()
         got_b = torch.cat([y1[30:], y2[7:]]).float().cpu()
         assert rel_err(got_a, wa) < tol(dtype) and rel_err(got_b, wb) < tol(dtype), kind
