@@ -11,8 +11,9 @@
 //
 // Layouts: K cache [blocks, G, BS, dim]; V cache TRANSPOSED per block [blocks, G, vdim, BS], so
 // that both MFMA operands are contiguous along their contraction index (dim for q.k, keys for
-// p.v) and every fragment is one 16-byte (K) or 8/16-byte (V) load straight from the cache: no
-// LDS staging, no barriers.  Waves of a workgroup that share a kv head hit the same lines in L1.
+// p.v) and a fragment is one 16-byte (K) or 8/16-byte (V) piece of a cache row.  f32, heads of more than 128 and prompt steps of few
+// tiles load the fragments straight from the cache, without LDS or barriers (waves of a workgroup that share a kv head hit the same
+// lines in L1); bf16 decode and prompt steps of many tiles bring whole lines into LDS first (attn_stage.h).
 //
 // One wave = 16 "columns" (queries) against a run of 16-key tiles:
 //   S^T (16 keys x 16 columns) = K . Q^T     A = K rows, B = the columns' q kept in registers

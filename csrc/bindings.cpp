@@ -182,7 +182,7 @@ at::Tensor ws_linear(const at::Tensor& x, const at::Tensor& w, bool swiglu, int6
 }
 
 // few-row GEMM (csrc/rows_gemm.hip): M <= 4,096 rows, any epilogue, one launch.  epi: 0 none, 1 SwiGLU, 2 bias, 3 bias + GELU,
-// 4 bias + ReLU
+// 4 bias + ReLU, 5 bias + residual; wide: columns of a workgroup, 0: 16, 1: 32, 2: 64
 at::Tensor rows_linear(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, int64_t epi, int64_t wide,
                        const c10::optional<at::Tensor>& residual) {
   CHECK_CUDA(x); CHECK_BF16(x); CHECK_BF16(w); CHECK_LASTDIM(x); CHECK_CONTIG(w);

@@ -927,12 +927,15 @@ int cu_count();
 
 // Row tile of the grouped form in gemm1w.hip: 256, 192 or 128 rows.  The experts' counts are on the device, so
 // the number of tiles is what counts spread around the mean like random ones give; a tile's time per K-tile of 64 is a + b * (share of
-// the CUs at work beside it), as measured with 16 experts of 2048 x 2816, in us: 1.02 + 0.68 / 0.80 + 0.70 / 0.64 + 0.50 (256 rows by the
-// kernel above; by gemm1w.hip's, which takes them now, 6 % less, but choices made with that are worse: 1,400 tokens 121 for 106 us).  A smaller
-// tile is taken where that predicts 5 % less, which is where 256 rows leave a round of tiles nearly empty or most of a tile without
-// rows.  Two of 16 experts per token, gate and up / down product in us, 256 rows -> the rule's: 600 tokens 112 / 58 -> 104 / 40,
-// 1,024: 105 / 61 -> 97 / 51, 1,400: 121 / 60 -> 111 / 54, 2,500: 152 / 78 -> 135 / 68, 4,096: 196 / 128 -> 196 / 113 (the rule keeps
-// 256 for the wider product; 192 measured 202), 2,048, 3,000 and 3,500: 256 as before (192 up to 22 % slower).
+// the CUs at work beside it), in us: 1.02 + 0.68 / 0.80 + 0.70 / 0.64 + 0.50.  These were the times of the eight-wave kernel above at 256 rows
+// and of gemm1w.hip's tiles at 192 and 128 (16 experts of 2048 x 2816); gemm1w.hip's 256 rows take 6 % less, so what the constants are
+// now is the line that its picks were checked at.  A smaller tile is taken where that predicts 5 % less, which is where 256 rows leave a
+// round of tiles nearly empty or most of a tile without rows.  Over 240 products (8 expert layouts, 64 - 1,100 rows an expert) the picks
+// take 2.1 % more than the best of the three, 39 % at most; 256 rows always, 13.4 % more.  Constants nearer to all three tiles' times (1.0 + 0.64 /
+// 0.74 + 0.62 / 0.62 + 0.48, no 5 %) take 1.2 % more, but of the 32 picks that change eight are 5 - 21 % slower than these.
+// Two of 16 experts per token, gate and up / down product in us, 256 rows -> the rule's: 600 tokens 110 / 58 -> 99 / 53,
+// 1,024: 115 / 62 -> 109 / 58, 1,400: 121 / 67 -> 108 / 57, 2,500: 165 / 78 -> 143 / 71, 4,096: 206 / 135 -> 206 / 118 (the rule keeps
+// 256 for the wider product; 192 measured 211), 2,048, 3,000 and 3,500: 256 (2,048 down: 192 measured 66 for 74).
 // The eight-wave kernel above, which had the 256-row tiles before, takes 5 - 8 % longer (3,500 and 4,096 tokens: 171 and 212 us instead
 // of 158 and 196); it is left with the widths and sizes that gemm1w.hip does not take.
 int grouped_tile_rows(long rows, int E, int TN) {

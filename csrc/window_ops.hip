@@ -506,8 +506,8 @@ int lk_pool_kv_write(const void* kc, const void* vc, void* pkc, void* pvc, int P
   // a run of max_len new positions ends at most (max_len + P - 1) / P blocks (+ 1 when it starts inside one)
   const dim3 grid((unsigned)((max_len + P - 1) / P + 1), (unsigned)G, (unsigned)S);
   const auto a16 = [](const void* x) { return reinterpret_cast<uintptr_t>(x) % 16 == 0; };
-  if (esz == 2 && dim % 8 == 0 && vdim % 8 == 0 && P % 8 == 0 && BS % 8 == 0 && dim <= 2048 && (long)(256 / (dim / 8)) * dim <= kPoolSums &&
-      (long)P / 8 * vdim <= kPoolSums && a16(kc) && a16(vc))
+  if (esz == 2 && dim % 8 == 0 && vdim % 8 == 0 && P % 8 == 0 && BS % 8 == 0 && dim <= 2048 && (long)P / 8 * vdim <= kPoolSums &&
+      a16(kc) && a16(vc))   // (the keys' partial sums, 256 / (dim / 8) rows of dim, are 2,048 floats at most)
     pool_kv_vec_kernel<<<dim3(2 * grid.x, grid.y, grid.z), 256, 0, st>>>((const bf16_t*)kc, (const bf16_t*)vc, (bf16_t*)pkc, (bf16_t*)pvc, P, bt,
                                                                         bt_stride, ctx_lens, cu_q, slots, row0, G, BS, dim, vdim);
   else if (esz == 2)
