@@ -30,9 +30,11 @@
 //   S^T (keys x columns) = K . Q^T,   O^T (vdim x columns) += V^T . P^T
 // with the same key permutation on both sides.  The softmax is the running-maximum form: per column a
 // maximum m >= 0 when there is a sink (its score bounds the maximum from below, so exp(-m) <= 1 is its
-// share of the denominator), the sum l of exp(s - m) and O^T scaled alike.  The four waves of a
-// workgroup take every fourth step and are merged through LDS in wave order; decode splits the key range
-// over workgroups as well and a second kernel merges the parts (m, l, O) and applies the gate.
+// share of the denominator), the sum l of exp(s - m) and O^T scaled alike.  Straight from the cache the four
+// waves of a workgroup take every fourth step and are merged through LDS in wave order (or each has a tile of
+// its own where the mask is short); staged prompts (attn_stage.h) give a wave 16 queries and all their steps.
+// Decode splits the key range over workgroups as well and a second kernel merges the parts (m, l, O) and
+// applies the gate.
 #include "common.h"
 #include "kernels.h"
 #include "attn_frag.h"
