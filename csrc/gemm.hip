@@ -925,32 +925,31 @@ int launch_grouped(const bf16_t* x, long ldx, const bf16_t* w, const int* seg, i
 
 int cu_count();
 
-// Row tile of the grouped form in gemm1w.hip: 256, 192 or 128 rows.  The experts' counts are on the device, so
-// the number of tiles is what counts spread around the mean like random ones give; a tile's time per K-tile of 64 is a + b * (share of
-// the CUs at work beside it), in us: 1.02 + 0.68 / 0.80 + 0.70 / 0.64 + 0.50.  These were the times of the eight-wave kernel above at 256 rows
-// and of gemm1w.hip's tiles at 192 and 128 (16 experts of 2048 x 2816); gemm1w.hip's 256 rows take 6 % less, so what the constants are
-// now is the line that its picks were checked at.  A smaller tile is taken where that predicts 5 % less, which is where 256 rows leave a
-// round of tiles nearly empty or most of a tile without rows.  Over 240 products (8 expert layouts, 64 - 1,100 rows an expert) the picks
-// take 2.1 % more than the best of the three, 39 % at most; 256 rows always, 13.4 % more.  Constants nearer to all three tiles' times (1.0 + 0.64 /
-// 0.74 + 0.62 / 0.62 + 0.48, no 5 %) take 1.2 % more, but of the 32 picks that change eight are 5 - 21 % slower than these.
-// Two of 16 experts per token, gate and up / down product in us, 256 rows -> the rule's: 600 tokens 110 / 58 -> 99 / 53,
-// 1,024: 115 / 62 -> 109 / 58, 1,400: 121 / 67 -> 108 / 57, 2,500: 165 / 78 -> 143 / 71, 4,096: 206 / 135 -> 206 / 118 (the rule keeps
-// 256 for the wider product; 192 measured 211), 2,048, 3,000 and 3,500: 256 (2,048 down: 192 measured 66 for 74).
-// The eight-wave kernel above, which had the 256-row tiles before, takes 5 - 8 % longer (3,500 and 4,096 tokens: 171 and 212 us instead
-// of 158 and 196); it is left with the widths and sizes that gemm1w.hip does not take.
+// Row tile of the grouped form in gemm1w.hip: 128, 192, 224, 256 or 288 rows.  The experts' counts are on the device, so the number of
+// tiles is what counts spread around the mean like random ones give.  A tile's time per K-tile of 64 is a + b * (share of the CUs at
+// work beside it), a = 1.41 f - 0.17 and b = 0.69 - 0.18 f us for f * 256 rows: the weights' stream is a part of both, so half a tile
+// costs more than half, and what decides is how many rounds of tiles the CUs take and how full the last one is.  288 rows are there for
+// the experts whose counts lie a little above whole 256-row tiles, about half of them wherever the mean is near such a multiple: each
+// would begin a tile for a few rows and stream all of its expert's weights again for it.  The constants minimise what the picks take over
+// the best tile: 1.2 % over 322 products (7 expert layouts, 40 - 1,150 rows an expert), 27 % at most (a product of few K-tiles and
+// barely one round); 256 rows always, 10.1 %.  Against the rule for 128 / 192 / 256 rows that was here before, 0.967 of its time; 314 of
+// the 322 within 3 % or faster.
+// Two of 16 experts of 2048 x 2816 per token, gate and up / down product in us, that rule -> this one: 1,024 tokens 110 / 56 -> 110 / 56,
+// 1,840: 125 / 70 -> 125 / 61, 2,048: 149 / 72 -> 133 / 63, 3,000: 156 / 77 -> 150 / 74, 3,840: 170 / 126 -> 166 / 86, 4,096: 204 / 116
+// -> 179 / 89, 8,192: 355 / 205 -> 341 / 161.
+// The eight-wave kernel above is left with the widths and sizes that gemm1w.hip does not take.
 int grouped_tile_rows(long rows, int E, int TN) {
-  struct Cost { int bm; double a, b; };
-  constexpr Cost costs[] = {{256, 1.02, 0.68}, {192, 0.80, 0.70}, {128, 0.64, 0.50}};
   const double mean = (double)rows / E, sd = sqrt(mean), cus = cu_count();
   int best = 256;
   double least = 0;
-  for (const Cost& c : costs) {
+  for (const int bm : {256, 128, 192, 224, 288}) {
+    const double a = 1.41 * bm / 256 - 0.17, b = 0.69 - 0.18 * bm / 256;
     double per = 0;   // expected row tiles of an expert: the sum over k of P(count > k bm)
-    for (int k = 0; k * c.bm < mean + 5 * sd; ++k) per += k == 0 ? 1.0 : 0.5 * erfc((k * c.bm - mean) / (sd * M_SQRT2));
+    for (int k = 0; k * bm < mean + 5 * sd; ++k) per += k == 0 ? 1.0 : 0.5 * erfc((k * bm - mean) / (sd * M_SQRT2));
     const double rounds = E * per * TN / cus, whole = floor(rounds), part = rounds - whole;
-    const double t = (whole * (c.a + c.b) + c.a * fmin(1.0, part * cus) + c.b * part) * (c.bm == 256 ? 0.95 : 1.0);
-    if (c.bm == 256 || t < least) {
-      best = c.bm;
+    const double t = whole * (a + b) + a * fmin(1.0, part * cus) + b * part;
+    if (bm == 256 || t < least) {
+      best = bm;
       least = t;
     }
   }

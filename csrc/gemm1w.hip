@@ -1,7 +1,7 @@
 // K2, prefill regime, one wave per SIMD: Y[M, N] = epilogue(X[M, K] . W[N, K]^T).
 //
-// A workgroup of 4 waves, one per SIMD, owns a BM x 256 tile (BM = 256 / 192 / 128), a wave (BM / 2) x 128 of it as MB x 8
-// v_mfma_f32_16x16x32_bf16 accumulators (MB = BM / 32), which fill the AGPRs at BM 256.  K advances by 64 (whole 128-byte lines).
+// A workgroup of 4 waves, one per SIMD, owns a BM x 256 tile (BM = 256 / 192 / 128; grouped also 288 / 224), a wave (BM / 2) x 128 of it
+// as MB x 8 v_mfma_f32_16x16x32_bf16 accumulators (MB = BM / 32), which fill the AGPRs at BM 256 (at 288 the ninth row block's are VGPRs).  K advances by 64 (whole 128-byte lines).
 //
 // What a K-tile costs at BM 256, in cycles of a CU: 128 MFMAs of 16 per SIMD = 2,048; 32 fragment reads of 1 KB per wave, 128 KB at
 // 128 bytes = 1,024 of LDS; 64 KB of LDS-DMA writes = 512.  LDS is busy three quarters of the time, so its work has to be spread over the
@@ -31,7 +31,8 @@
 // fragment pair: 16-byte stores; SwiGLU pairs gate (half 1) and up (half 2) of the same columns.
 //
 // Row tiles of 192 / 128 fill the 256 CUs where 256-row tiles leave most of a wave idle; the dispatch picks the row tile per M bucket
-// from measurements (ops.tune_gemm) or a cost rule.  Epilogues (same contracts and rounding as gemm.hip): NONE, SWIGLU, BIAS, BIAS_GELU,
+// from measurements (ops.tune_gemm) or a cost rule; the grouped form takes 128, 192, 224, 256 or 288 rows by the rounds that experts of the
+// expected sizes fill (grouped_tile_rows in gemm.hip).  Epilogues (same contracts and rounding as gemm.hip): NONE, SWIGLU, BIAS, BIAS_GELU,
 // BIAS_RELU, PARTIAL (split-K fp32 slabs), RESID (r += acc in place + per-row partial sums of squares), QKV (RoPE + paged-KV scatter);
 // NONE / SWIGLU / QKV take the folded-RMSNorm row scale (LkEpi::ss_in); rows past M are dropped by the buffer descriptors' range checks.
 #include <type_traits>
@@ -57,7 +58,7 @@ struct Tile {
   static constexpr int MB = BM / 32, NM = 16 * MB, PX = BM / 32, NP = PX + 8;  // PX / 8: LDS-DMA pieces (1 KB) of X / W per wave
   static constexpr int kOpX = BM * kRowB;                // X rows of one stage
   static constexpr int kStage = kOpX + 256 * kRowB;      // X rows then W rows
-  static constexpr int kLdsStages = 2 * kStage;          // 128 / 112 / 96 KB
+  static constexpr int kLdsStages = 2 * kStage;          // 128 / 112 / 96 KB (136 at 288 rows)
   static constexpr int kLds = kLdsStages + kLdsEpi;
   static constexpr int WA = 3;                           // W fragments read ahead
   static constexpr int S1 = (8 - WA) * MB, S0 = (16 - WA) * MB, PH = 8 * MB;
@@ -108,6 +109,13 @@ LK_DEVICE void mfma(floatx4& acc, const short8& a, const short8& b) {
 LK_DEVICE void mfma0(floatx4& acc, const short8& a, const short8& b) {
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(acc) : "v"(a), "v"(b));
 }
+// the same with the accumulator in ordinary registers: the ninth 16-row block of a 288-row tile, for which the 256 AGPRs are taken
+LK_DEVICE void mfma_v(floatx4& acc, const short8& a, const short8& b) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
+}
+LK_DEVICE void mfma0_v(floatx4& acc, const short8& a, const short8& b) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "v"(b));
+}
 template <int OFF>
 LK_DEVICE void set_m0(unsigned base) { asm volatile("s_add_u32 m0, %0, %1" ::"s"(base), "i"(OFF) : "memory", "m0", "scc"); }
 LK_DEVICE u32x4_t srd(const void* p, long bytes) {  // buffer descriptor words, wave-uniform
@@ -138,6 +146,7 @@ __global__ __launch_bounds__(256, 1) void gemm1w_kernel(const bf16_t* __restrict
                                                         int tn0, int group_m, LkEpi ea) {
   constexpr bool SC = SCP > 0;
   static_assert(!SC || scalable(EPI), "row scale");
+  static_assert(BM <= 256 || (!SC && EPI != E_RESID), "one thread per tile row");
   static_assert(!PERSIST || (persistable(EPI) && !SC), "persistent walk: plain / bias epilogues");
   using TL = Tile<BM>;
   constexpr int MB = TL::MB, NM = TL::NM, PX = TL::PX, NP = TL::NP, WM = BM / 2;
@@ -198,6 +207,7 @@ __global__ __launch_bounds__(256, 1) void gemm1w_kernel(const bf16_t* __restrict
   unsigned xo[PX], wo[8];
   const unsigned ldxb = (unsigned)ldx * 2, kb = (unsigned)K * 2;
   const unsigned ch0 = (unsigned)((lc8 ^ (lr8 >> 1)) << 4);
+  const unsigned chx = PX & w & 1 ? ch0 ^ 64u : ch0;  // (an odd number of pieces per wave: the odd waves' rows begin at an odd piece)
   auto offsets = [&](int tm, int tn, unsigned (&xo)[PX], unsigned (&wo)[8]) {
     const int xr = tm * BM + (BM / 4) * w + lr8;
 #pragma unroll
@@ -205,9 +215,9 @@ __global__ __launch_bounds__(256, 1) void gemm1w_kernel(const bf16_t* __restrict
       if constexpr (GS) {  // rows past the expert's end point behind the descriptor's range: zeros
         const int tr = xr + 8 * i;
         const int src = tr < M ? (ea.gather ? ea.gather[tr] / ea.top : tr) : -1;
-        xo[i] = src >= 0 ? (unsigned)src * ldxb + (ch0 ^ (unsigned)((i & 1) << 6)) : 0xFFFFFF00u;
+        xo[i] = src >= 0 ? (unsigned)src * ldxb + (chx ^ (unsigned)((i & 1) << 6)) : 0xFFFFFF00u;
       } else {
-        xo[i] = (unsigned)(xr + 8 * i) * ldxb + (ch0 ^ (unsigned)((i & 1) << 6));
+        xo[i] = (unsigned)(xr + 8 * i) * ldxb + (chx ^ (unsigned)((i & 1) << 6));
       }
     }
     // SwiGLU: half 1 holds the gate rows of 64 output columns per column half, half 2 the up rows of the same
@@ -292,8 +302,13 @@ __global__ __launch_bounds__(256, 1) void gemm1w_kernel(const bf16_t* __restrict
       if constexpr (ax1 >= 0) m0_x(stage_t, std::integral_constant<int, ax1>{});
       if constexpr (bw1 >= 0) m0_w(stage_t, std::integral_constant<int, bw1>{});
       fence();
-      if constexpr (FIRST && (f & 1) == 0) mfma0(acc[m][f >> 1], fw[f & 3], fx[P][f & 1][m]);
-      else mfma(acc[m][f >> 1], fw[f & 3], fx[P][f & 1][m]);
+      if constexpr (FIRST && (f & 1) == 0) {
+        if constexpr (m < 8) mfma0(acc[m][f >> 1], fw[f & 3], fx[P][f & 1][m]);
+        else mfma0_v(acc[m][f >> 1], fw[f & 3], fx[P][f & 1][m]);
+      } else {
+        if constexpr (m < 8) mfma(acc[m][f >> 1], fw[f & 3], fx[P][f & 1][m]);
+        else mfma_v(acc[m][f >> 1], fw[f & 3], fx[P][f & 1][m]);
+      }
     });
   };
 
@@ -376,7 +391,10 @@ __global__ __launch_bounds__(256, 1) void gemm1w_kernel(const bf16_t* __restrict
 #pragma unroll
     for (int m = 0; m < MB; ++m)
 #pragma unroll
-      for (int n = 0; n < 8; ++n) asm volatile("" : "+a"(acc[m][n]));
+      for (int n = 0; n < 8; ++n) {
+        if (m < 8) asm volatile("" : "+a"(acc[m][n]));
+        else asm volatile("" : "+v"(acc[m][n]));
+      }
 
     if constexpr (!PERSIST) wait_vm<0>();  // the last refills land before the workgroup's LDS is released
 
@@ -781,9 +799,18 @@ int lk_gemm1w_grouped(const bf16_t* x, long ldx, const bf16_t* w, const int* seg
   ea.scatter = scatter;
   ea.x_rows = x_rows;
   ea.out_rows = rows;
-#define LK_G1W(EPI, BM) launch1w_grouped<EPI, BM>(x, ldx, w, rows, K, swiglu ? N / 2 : 0, out, ldo, N / kBN, st, ea)
-  if (swiglu) return bm == 128 ? LK_G1W(E_SWIGLU, 128) : bm == 192 ? LK_G1W(E_SWIGLU, 192) : LK_G1W(E_SWIGLU, 256);
-  return bm == 128 ? LK_G1W(E_NONE, 128) : bm == 192 ? LK_G1W(E_NONE, 192) : LK_G1W(E_NONE, 256);
+#define LK_G1W(BM)                                                                                                  \
+  case BM:                                                                                                          \
+    return swiglu ? launch1w_grouped<E_SWIGLU, BM>(x, ldx, w, rows, K, N / 2, out, ldo, N / kBN, st, ea)            \
+                  : launch1w_grouped<E_NONE, BM>(x, ldx, w, rows, K, 0, out, ldo, N / kBN, st, ea)
+  switch (bm) {
+    LK_G1W(128);
+    LK_G1W(192);
+    LK_G1W(224);
+    LK_G1W(256);
+    LK_G1W(288);
+    default: return -1;
+  }
 #undef LK_G1W
 }
 

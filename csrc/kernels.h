@@ -167,7 +167,7 @@ int lk_gemm_grouped(const bf16_t* x, long ldx, const bf16_t* w, const int* seg, 
 // Variants 6 / 7: a column split -- the column tiles that fill whole waves of the CUs on 256-row
 // tiles, the remaining (less than a wave) on 128 / 192-row tiles, as two launches.
 constexpr int LK_GEMM1W_SPLIT128 = 1, LK_GEMM1W_SPLIT192 = 2;
-// grouped form (lk_gemm_grouped's contract) on bm = 128 / 192-row tiles; supported: >= 3 K-tiles, 32-bit offsets
+// grouped form (lk_gemm_grouped's contract) on bm = 128 / 192 / 224 / 256 / 288-row tiles; supported: >= 3 K-tiles, 32-bit offsets
 int lk_gemm1w_grouped_supported(long rows, long ldx, long x_rows, int N, int K, int swiglu, long ldo);
 int lk_gemm1w_grouped(const bf16_t* x, long ldx, const bf16_t* w, const int* seg, int E, long rows, int N, int K, int swiglu, bf16_t* out,
                       long ldo, hipStream_t st, const int* gather, long x_rows, const int* scatter, int top, int bm);

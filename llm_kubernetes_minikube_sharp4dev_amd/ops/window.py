@@ -168,7 +168,7 @@ def table_experts(h, ids, table, w_gate_up, w_down, top: int, route=None):
 
 def _grouped(T: int, pairs: int, E: int, W: int, ffp: int) -> bool:
     """Whether the expert products run as one dense product per expert (``gemm_grouped``): from GROUPED_DENSE_MIN_ROWS pairs per expert on,
-    and from GROUPED_FINE_MIN_ROWS where its 128 / 192-row tiles take both sizes (2 of 16 experts of 2048 x 2816: 600 tokens 203 -> 144
+    and from GROUPED_FINE_MIN_ROWS where its row tiles take both sizes (2 of 16 experts of 2048 x 2816: 600 tokens 203 -> 144
     us, 800 tokens 225 -> 149 us, with the same f32 activation)."""
     if pairs >= GROUPED_DENSE_MIN_ROWS * E:
         return lib().gemm_grouped_supported(2 * ffp, W, True) and lib().gemm_grouped_supported(W, ffp, False)

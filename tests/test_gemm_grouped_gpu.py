@@ -10,6 +10,19 @@ from llm_kubernetes_minikube_sharp4dev_amd import ops
 FULL192, FULL256 = [150, 192, 191, 1, 129, 193, 185, 160, 190, 170, 175, 0, 180, 188, 65, 192], [256, 250, 193, 240, 255, 257, 230, 245] * 2
 
 
+# 224 and 288 rows (and 256 at a width of 3072)
+FULL224 = [448, 449, 447, 224, 225, 223, 400, 385, 390, 672, 673, 0, 380, 370, 1, 395]
+FULL288 = [576, 575, 512, 513, 288, 289, 577, 545, 560, 0, 864, 500, 561, 1, 529, 512]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("counts,swiglu,N,K", [(FULL224, True, 4096, 192), (FULL224, False, 2048, 256), (FULL288, True, 4096, 192),
+                                               (FULL288, False, 2048, 256), (FULL288, False, 2048, 320), (FULL256, True, 3072, 192),
+                                               (FULL256, False, 3072, 256)])
+def test_rounds_of_taller_tiles(counts, swiglu, N, K):
+    test_rows_per_expert(counts, swiglu, N, K)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("counts,swiglu,N,K", [(FULL192, True, 8192, 192), (FULL192, False, 4096, 192), (FULL256, True, 4096, 192),
                                                (FULL256, False, 4096, 256)])
