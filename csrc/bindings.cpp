@@ -7,6 +7,10 @@
 #include <ATen/core/CachingHostAllocator.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/hip/HIPStream.h>
+#include <algorithm>
+#include <chrono>
+#include <memory>
+#include <thread>
 #include "kernels.h"
 
 namespace {
@@ -934,26 +938,114 @@ std::vector<at::Tensor> knn_topk(const at::Tensor& corpus, const at::Tensor& cno
 
 // The one-pass search with both results in one buffer, int32 [2, nq, K] (score bits, then row numbers), for a caller that copies
 // them to the host in one piece; an empty tensor where the one-pass search does not take the shape.
-at::Tensor knn_packed(const at::Tensor& corpus, const at::Tensor& cnorm, const at::Tensor& queries, int64_t K, bool host) {
+// Hits of a launched search in pinned memory, seen by the host as they arrive: every word holds a value that no search leaves until
+// the merge writes it, once.  A wait for an event behind the kernels costs its barrier packet and the signal's way, 13 us on an idle
+// stream; reading the words costs neither.
+struct HostHits {
+  static constexpr int kNoScore = 0x7fffdead, kNoId = (int)0x80000000;   // a NaN (rows without a comparable score are left out); ids are >= -1
+  at::Tensor out;   // [2, nq, K] int32: the scores' bits, then the indices
+  int64_t nq, K;
+  c10::hip::HIPStream stream;
+
+  HostHits(int64_t nq_, int64_t K_)
+      : out(at::empty({2, nq_, K_}, at::TensorOptions(at::kInt).pinned_memory(true))), nq(nq_), K(K_), stream(c10::hip::getCurrentHIPStream()) {
+    int* p = out.data_ptr<int>();
+    std::fill(p, p + nq * K, kNoScore);
+    std::fill(p + nq * K, p + 2 * nq * K, kNoId);
+  }
+  HostHits(const HostHits&) = delete;
+  HostHits& operator=(const HostHits&) = delete;
+  ~HostHits() {
+    if (arrived()) return;   // every word has been written: nothing is on its way to the block
+    try {   // dropped unread: the block is not given out again before the stream has passed this point
+      at::getHostAllocator(at::kCUDA)->record_event(out.data_ptr(), out.storage().data_ptr().get_context(), masquerading().unwrap());
+    } catch (...) {   // (no stream any more, at the process's end)
+    }
+  }
+  c10::hip::HIPStreamMasqueradingAsCUDA masquerading() const { return c10::hip::HIPStreamMasqueradingAsCUDA(c10::hip::HIPStreamMasqueradingAsCUDA::UNCHECKED, stream.unwrap()); }
+
+  bool arrived() const {
+    const int* p = out.data_ptr<int>();
+    for (int64_t i = 0; i < nq * K; ++i)
+      if (__atomic_load_n(p + i, __ATOMIC_RELAXED) == kNoScore || __atomic_load_n(p + nq * K + i, __ATOMIC_RELAXED) == kNoId) return false;
+    __atomic_thread_fence(__ATOMIC_ACQUIRE);
+    return true;
+  }
+  // (without the GIL) spins for 50 us, then gives the CPU away between looks; a stream that has failed or ended without a result raises
+  void wait() const {
+    const auto t0 = std::chrono::steady_clock::now();
+    double asked = 0.005;
+    for (;;) {
+      for (int i = 0; i < 64; ++i) {
+        if (arrived()) return;
+        __builtin_ia32_pause();
+      }
+      const double s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+      if (s > 50e-6) std::this_thread::yield();
+      if (s > asked) {
+        const hipError_t e = hipStreamQuery(stream.stream());
+        if (e == hipErrorNotReady) (void)hipGetLastError();
+        else if (!arrived()) TORCH_CHECK(false, "knn_hits: the search left no result: ", hipGetErrorString(e));
+        asked = s + 0.005;
+      }
+    }
+  }
+  // per query the hits in order, (index, score), without the padding behind fewer rows than K
+  std::vector<std::vector<std::pair<int64_t, double>>> rows(int64_t k) const {
+    const int *p = out.data_ptr<int>(), *ids = p + nq * K;
+    std::vector<std::vector<std::pair<int64_t, double>>> r(nq);
+    for (int64_t q = 0; q < nq; ++q)
+      for (int64_t j = 0; j < K && (int64_t)r[q].size() < k; ++j)
+        if (ids[q * K + j] >= 0) r[q].emplace_back(ids[q * K + j], (double)reinterpret_cast<const float*>(p)[q * K + j]);
+    return r;
+  }
+};
+
+// workgroups of the one-pass search (0: it does not take the shape); checks the operands
+int knn_scan_plan(const at::Tensor& corpus, const at::Tensor& cnorm, const at::Tensor& queries, int64_t K) {
   CHECK_CUDA(corpus); CHECK_BF16(corpus); CHECK_CONTIG(corpus); CHECK_F32(cnorm); CHECK_CONTIG(cnorm);
   CHECK_CUDA(queries); CHECK_BF16(queries); CHECK_CONTIG(queries);
   TORCH_CHECK(corpus.dim() == 2 && queries.dim() == 2 && corpus.size(1) == queries.size(1), "dimension mismatch");
-  const long N = corpus.size(0);
-  const int D = corpus.size(1), nq = queries.size(0);
-  TORCH_CHECK(cnorm.numel() == N, "norm shapes");
-  auto io = corpus.options().dtype(at::kInt);
+  TORCH_CHECK(cnorm.numel() == corpus.size(0), "norm shapes");
   const auto a16 = [](const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
-  const int nb = K <= N && a16(corpus) && a16(queries) ? lk_knn_scan_blocks(N, D, nq, (int)std::min<int64_t>(K, 64)) : 0;
+  return K <= corpus.size(0) && a16(corpus) && a16(queries)
+             ? lk_knn_scan_blocks(corpus.size(0), corpus.size(1), queries.size(0), (int)std::min<int64_t>(K, 64)) : 0;
+}
+void knn_scan_to(int* o, const at::Tensor& corpus, const at::Tensor& cnorm, const at::Tensor& queries, int64_t K, int nb) {
+  const long nq = queries.size(0);
+  at::Tensor part = at::empty({2, nq, nb, K}, corpus.options().dtype(at::kInt));
+  int* p = part.data_ptr<int>();
+  CHECK_RC(lk_knn_scan(bp(corpus), cnorm.data_ptr<float>(), corpus.size(0), corpus.size(1), bp(queries), nullptr, (int)nq, (int)K,
+                       reinterpret_cast<float*>(p), p + nq * nb * K, reinterpret_cast<float*>(o), o + nq * K, cur_stream()), "knn_scan");
+}
+
+at::Tensor knn_packed(const at::Tensor& corpus, const at::Tensor& cnorm, const at::Tensor& queries, int64_t K, bool host) {
+  const int nb = knn_scan_plan(corpus, cnorm, queries, K);
+  auto io = corpus.options().dtype(at::kInt);
   if (!nb) return at::empty({0}, io);
   // host: the merge writes the few hits straight into pinned memory (a copy behind it was one more launch in the caller's wait)
-  at::Tensor out = at::empty({2, nq, K}, host ? at::TensorOptions(at::kInt).pinned_memory(true) : io), part = at::empty({2, nq, nb, K}, io);
-  int *o = out.data_ptr<int>(), *p = part.data_ptr<int>();
-  const int rc = lk_knn_scan(bp(corpus), cnorm.data_ptr<float>(), N, D, bp(queries), nullptr, nq, (int)K, reinterpret_cast<float*>(p),
-                             p + (long)nq * nb * K, reinterpret_cast<float*>(o), o + (long)nq * K, cur_stream());
-  if (host)   // the pinned block is not given out again before the stream has passed this point
-    at::getHostAllocator(at::kCUDA)->record_event(o, out.storage().data_ptr().get_context(), c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().unwrap());
-  CHECK_RC(rc, "knn_scan");
+  at::Tensor out = at::empty({2, queries.size(0), K}, host ? at::TensorOptions(at::kInt).pinned_memory(true) : io);
+  int* o = out.data_ptr<int>();
+  const auto passed = [&] {   // the pinned block is not given out again before the stream has passed this point
+    if (host) at::getHostAllocator(at::kCUDA)->record_event(o, out.storage().data_ptr().get_context(), c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().unwrap());
+  };
+  try {
+    knn_scan_to(o, corpus, cnorm, queries, K, nb);
+  } catch (...) {
+    passed();
+    throw;
+  }
+  passed();
   return out;
+}
+
+// the same with the hits seen as they arrive (null: the one-pass search does not take the shape)
+std::unique_ptr<HostHits> knn_hits(const at::Tensor& corpus, const at::Tensor& cnorm, const at::Tensor& queries, int64_t K) {
+  const int nb = knn_scan_plan(corpus, cnorm, queries, K);
+  if (!nb) return nullptr;
+  auto h = std::make_unique<HostHits>(queries.size(0), K);
+  knn_scan_to(h->out.data_ptr<int>(), corpus, cnorm, queries, K, nb);
+  return h;
 }
 
 std::vector<at::Tensor> knn_merge(const at::Tensor& cand_s, const at::Tensor& cand_i, int64_t K) {
@@ -2470,6 +2562,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("knn_topk", &knn_topk, "", py::arg("corpus"), py::arg("cnorm"), py::arg("queries"), py::arg("qnorm"),
         py::arg("K"), py::arg("force_fused") = false);
   m.def("knn_packed", &knn_packed, "", py::arg("corpus"), py::arg("cnorm"), py::arg("queries"), py::arg("K"), py::arg("host") = false);
+  py::class_<HostHits>(m, "HostHits")
+      .def("query", &HostHits::arrived)
+      .def("synchronize", &HostHits::wait, py::call_guard<py::gil_scoped_release>())
+      .def("rows", &HostHits::rows);
+  m.def("knn_hits", &knn_hits);
   m.def("knn_merge", &knn_merge);
   m.def("pool_normalize", &pool_normalize, "", py::arg("hidden"), py::arg("cu"), py::arg("mode"), py::arg("normalize"),
         py::arg("out") = py::none());

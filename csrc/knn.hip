@@ -43,17 +43,21 @@ LK_DEVICE void wave_argmax(float& s, int& i) {
   }
 }
 
-template <int W>  // over groups of W lanes
-LK_DEVICE void group_argmax(float& s, int& i) {
-#pragma unroll
-  for (int o = W / 2; o > 0; o >>= 1) {
-    const float s2 = __shfl_xor(s, o, 64);
-    const int i2 = __shfl_xor(i, o, 64);
-    if (better(s2, i2, s, i)) {
-      s = s2;
-      i = i2;
-    }
+// over groups of 16 lanes, by row rotations of the vector unit (every lane ends with the same pair)
+template <int STEP>
+LK_DEVICE void rotate_argmax(float& s, int& i) {
+  const float s2 = wave_partner<STEP>(s);
+  const int i2 = __builtin_amdgcn_update_dpp(0, i, 0x120 + STEP, 0xf, 0xf, true);
+  if (better(s2, i2, s, i)) {
+    s = s2;
+    i = i2;
   }
+}
+LK_DEVICE void row_argmax(float& s, int& i) {
+  rotate_argmax<8>(s, i);
+  rotate_argmax<4>(s, i);
+  rotate_argmax<2>(s, i);
+  rotate_argmax<1>(s, i);
 }
 
 template <int D>
@@ -274,7 +278,9 @@ __global__ __launch_bounds__(256) void knn_merge_kernel(const float* __restrict_
 // 16 rows x 128 bytes (row_ring.h), walk 16-row tiles round robin without a barrier, so 120 KB of corpus are on their way
 // per CU.  A lane sees 4 rows of one query per tile and keeps its 8 best in order (rows come in ascending order, so an
 // equal score never displaces: the stable order); 16 lists per query meet in LDS at the end.
-// 16 x 485,620 x 768: scan 158 + top-k 26 + merge 10 us -> 130 + 6 (5.7 TB/s); 1 x 20,011: 11 + 12 + 5 -> 15 + 5.
+// What bounds it: the stream of rows at 485,620 x 768 (120 us, 6.2 TB/s, and 5 for the merge; 131 and 6 with a wait per number of stages
+// left, row addresses per stage and reductions through the LDS unit); at 20,011 rows a wave has one or two tiles and the chain of launch,
+// code and first loads counts (12 + 4 us; 16 + 5).  The scores' own two-pass form took 158 + 26 + 10 and 11 + 12 + 5.
 constexpr int kScanK = 8, kScanQ = 16, kScanStages = 16;
 
 // ls / li descending: s, i enters behind everything that is not smaller
@@ -315,48 +321,46 @@ __global__ __launch_bounds__(256, 1) void knn_scan_kernel(const bf16_t* __restri
 #pragma unroll
     for (int k = 0; k < 2 * SEG; ++k) qf[k] = *reinterpret_cast<const short8*>(q + 32 * k);
   }
-  float qn;
-  if (qnorm) {
-    qn = qnorm[min(r16, nq - 1)];
-  } else {
-    float p[2 * SEG], ss = 0.f;  // (eight at a time: one chain of D / 4 additions would cost the norm its last bits)
+  const float qgiven = qnorm ? qnorm[min(r16, nq - 1)] : 0.f;
+  const int tiles = (int)((N + 15) / 16), first = blockIdx.x * 4 + w, step = gridDim.x * 4;
+  const int total = first < tiles ? ((tiles - 1 - first) / step + 1) * SEG : 0;  // this wave's stages
+  unsigned char* const ring = smem + w * NS * 2048;
+  const int lrow = lane >> 3, lcol = rg_lane_col(lane);
+  const bf16_t* src[2];  // this lane's part of the tile being requested
+  int ist = 0;           // stages requested
+  auto issue = [&](int seg, long tile) {
+    if (seg == 0) {
 #pragma unroll
-    for (int k = 0; k < 2 * SEG; ++k) {
-      p[k] = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float v = bf2f((bf16_t)qf[k][e]);
-        p[k] += v * v;
-      }
+      for (int i = 0; i < 2; ++i) src[i] = corpus + min(tile * 16 + 8 * i + lrow, N - 1) * D + lcol;
     }
+    unsigned char* base = ring + (ist % NS) * 2048;
 #pragma unroll
-    for (int k = 0; k < 2 * SEG; k += 4) ss += (p[k] + p[k + 1]) + (2 * SEG - k >= 4 ? p[k + 2] + p[k + 3] : 0.f);
+    for (int i = 0; i < 2; ++i) __builtin_amdgcn_global_load_lds((rg_gptr)(src[i] + seg * 64), (rg_lptr)(base + i * 1024), 16, 0, 2);
+    ++ist;
+  };
+#pragma unroll
+  for (int p = 0; p < NS - 1; ++p)
+    if (p < total) issue(p % SEG, first + (long)(p / SEG) * step);
+  // the queries' norms: the diagonal of Q Q^T, in four chains (one chain of D / 32 sums would cost the norm its last bits; against
+  // float64 the scores of 640 queries are off by 0.85e-7 (D 128) to 1.8e-7 (1,024) rms, as with eight products at a time in the vector unit)
+  float qn = qgiven;
+  if (!qnorm) {
+    floatx4 n[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) n[c] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < 2 * SEG; ++k) n[k & 3] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qf[k], qf[k], n[k & 3], 0, 0, 0);
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (4 * g + j == r16) ss = (n[0][j] + n[1][j]) + (n[2][j] + n[3][j]);
     ss += __shfl_xor(ss, 16, 64);
     ss += __shfl_xor(ss, 32, 64);
     qn = sqrtf(ss);
   }
-  const long tiles = (N + 15) / 16, first = (long)blockIdx.x * 4 + w, step = (long)gridDim.x * 4;
-  const long mine = first < tiles ? (tiles - 1 - first) / step + 1 : 0, total = mine * SEG;  // this wave's tiles and stages
-  unsigned char* const ring = smem + w * NS * 2048;
-  const int lrow = lane >> 3, lcol = rg_lane_col(lane);
-  long it = first, ist = 0;  // the next stage to request: its tile and number
-  int iseg = 0;
-  auto issue = [&]() {
-    unsigned char* base = ring + (ist % NS) * 2048;
+  // (the compiler's wait for the queries belongs here: in the loop it would drain the ring at every tile)
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const long row = min(it * 16 + 8 * i + lrow, N - 1);
-      __builtin_amdgcn_global_load_lds((rg_gptr)(corpus + row * D + iseg * 64 + lcol), (rg_lptr)(base + i * 1024), 16, 0, 2);
-    }
-    ++ist;
-    if (++iseg == SEG) {
-      iseg = 0;
-      it += step;
-    }
-  };
-#pragma unroll
-  for (int p = 0; p < NS - 1; ++p)
-    if (p < total) issue();
+  for (int k = 0; k < 2 * SEG; ++k) asm volatile("" : "+v"(qf[k]));
   float ls[kScanK];
   int li[kScanK];
 #pragma unroll
@@ -364,7 +368,7 @@ __global__ __launch_bounds__(256, 1) void knn_scan_kernel(const bf16_t* __restri
     ls[j] = -INFINITY;
     li[j] = 0x7fffffff;
   }
-  long st = 0;
+  int st = 0;
   for (long t = first; t < tiles; t += step) {
     const long d0 = t * 16 + 4 * g;
     float cn[4];
@@ -373,9 +377,12 @@ __global__ __launch_bounds__(256, 1) void knn_scan_kernel(const bf16_t* __restri
     floatx4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int seg = 0; seg < SEG; ++seg, ++st) {
-      rg_wait_ahead<2, NS - 2>((int)min((long)(NS - 2), total - 1 - st));
+      // Two waits, not one per number of stages left: all of the last NS - 1 are waited for at once, which is 0.3 us of a wave's end, and
+      // the code of a stage is a tenth (a short scan runs it once and fetching it is what it waits for)
+      if (total - 1 - st >= NS - 2) rg_wait<2 * (NS - 2)>();
+      else rg_wait<0>();
       __builtin_amdgcn_sched_barrier(0);
-      if (ist < total) issue();
+      if (ist < total) issue((seg + NS - 1) % SEG, t + (long)((seg + NS - 1) / SEG) * step);
       __builtin_amdgcn_sched_barrier(0);
       const unsigned char* base = ring + (st % NS) * 2048;
 #pragma unroll
@@ -413,7 +420,7 @@ __global__ __launch_bounds__(256, 1) void knn_scan_kernel(const bf16_t* __restri
     for (int k = 0; k < K; ++k) {
       float bs = v[0];
       int bi = id[0];
-      group_argmax<16>(bs, bi);
+      row_argmax(bs, bi);
       if (r16 == 0 && q < nq) {
         const long o = ((long)q * gridDim.x + blockIdx.x) * K + k;
         part_s[o] = bs;
@@ -444,7 +451,7 @@ __global__ __launch_bounds__(256) void knn_merge_lists_kernel(const float* __res
   for (int k = 0; k < K; ++k) {
     float bs = s[0];
     int bi = i[0];
-    group_argmax<16>(bs, bi);
+    row_argmax(bs, bi);
     if (l16 == 0) {
       rs[grp][k] = bs;
       ri[grp][k] = bi;
@@ -461,10 +468,10 @@ __global__ __launch_bounds__(256) void knn_merge_lists_kernel(const float* __res
   for (int k = 0; k < K; ++k) {
     float bs = s[0];
     int bi = i[0];
-    group_argmax<16>(bs, bi);
-    if (l16 == 0) {
-      out_s[(long)q * K + k] = bs;
-      out_i[(long)q * K + k] = bs == -INFINITY ? -1 : bi;
+    row_argmax(bs, bi);
+    if (l16 == 0) {  // (each word once, at system scope: in pinned memory the host sees it arrive)
+      __hip_atomic_store(out_s + (long)q * K + k, bs, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      __hip_atomic_store(out_i + (long)q * K + k, bs == -INFINITY ? -1 : bi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
     if (i[0] == bi) list_pop(s, i);
   }

@@ -276,6 +276,15 @@ def knn_packed(corpus, cnorm, queries, K: int, host: bool = False):
     return r if r.numel() else None
 
 
+def knn_hits(corpus, cnorm, queries, K: int):
+    """:func:`knn_packed` into pinned memory as a handle: ``query()`` whether the hits have arrived, ``synchronize()`` waits for them
+    alone (no event behind the kernels), ``rows(k)`` then the (index, score) pairs of each query.  None where the one-pass search does
+    not take the shape."""
+    if not (use_hip(corpus) and queries.is_cuda and 1 <= K <= 64 and queries.shape[0] > 0):
+        return None
+    return lib().knn_hits(corpus, cnorm, queries, K)
+
+
 def knn_merge(cand_s, cand_i, K: int):
     if use_hip(cand_s):
         return tuple(lib().knn_merge(cand_s.contiguous(), cand_i.contiguous(), K))

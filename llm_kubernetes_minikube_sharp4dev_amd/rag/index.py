@@ -181,8 +181,8 @@ class RagIndex:
 
     def search_vectors_async(self, q: np.ndarray | torch.Tensor, top_k: int) -> "PendingSearch":
         """Launch a batched search without blocking the host: on the GPU the kNN kernels, which leave
-        (scores, ids) in pinned memory, are enqueued on the current stream before an event;
-        :meth:`PendingSearch.result` waits for that event only (an engine thread collects it after its next
+        (scores, ids) in pinned memory, are enqueued on the current stream; :meth:`PendingSearch.result`
+        waits for these words, or for an event behind the copies of a larger search (an engine thread collects it after its next
         step, when it has long completed), not for what other threads enqueue on the stream behind it.
         Elsewhere the search runs synchronously."""
         k = max(1, top_k)
@@ -202,11 +202,9 @@ class RagIndex:
             # host queries are cast on the host (a few KB) and copied once: no device cast kernel
             qt = (qt.to(torch.bfloat16).to(self.device) if qt.device.type == "cpu"
                   else qt.to(self.device, torch.bfloat16)).reshape(-1, corpus.shape[1]).contiguous()
-            host = ops.knn_packed(corpus, norms, qt, min(k, 64), host=True) if qt.is_cuda else None
-            if host is not None:
-                ev = torch.cuda.Event()
-                ev.record()
-                return PendingSearch(host=(host[0].view(torch.float32), host[1], min(k, n)), event=ev)
+            hits = ops.knn_hits(corpus, norms, qt, min(k, 64))
+            if hits is not None:
+                return PendingSearch(event=hits, rows=lambda: hits.rows(min(k, n)))
             qn = ops.row_norms(qt) if qt.is_cuda else qt.float().norm(dim=-1)
             s, i = ops.knn_topk(corpus, norms, qt, qn, min(k, 64))
         if not s.is_cuda:
@@ -328,11 +326,11 @@ def _rows(s, i, k):
 
 
 class PendingSearch:
-    """A launched :meth:`RagIndex.search_vectors_async`: ``ready()`` polls its event,
+    """A launched :meth:`RagIndex.search_vectors_async`: ``ready()`` polls its event (or the hits themselves),
     ``result()`` waits for it (not for the device) and decodes the rows once."""
 
-    def __init__(self, host=None, event=None, done=None):
-        self._host, self._event, self._done = host, event, done
+    def __init__(self, host=None, event=None, done=None, rows=None):
+        self._host, self._event, self._done, self._rows = host, event, done, rows
         self.wait_s = 0.0  # host time spent blocked in result()
 
     def ready(self) -> bool:
@@ -344,7 +342,10 @@ class PendingSearch:
             if self._event is not None:
                 self._event.synchronize()
             self.wait_s = time.perf_counter() - t0
-            hs, hi, k = self._host
-            self._done = _rows(hs.tolist(), hi.tolist(), k)
+            if self._rows is not None:
+                self._done = self._rows()
+            else:
+                hs, hi, k = self._host
+                self._done = _rows(hs.tolist(), hi.tolist(), k)
             M.KNN_LAT.observe(self.wait_s)
         return self._done

@@ -34,6 +34,36 @@ def test_scan(hip, N, D, nq, K):
         assert torch.equal(both[1], i) and ((both[0].view(torch.float32) - s).abs() <= 1e-6).all()
 
 
+@pytest.mark.parametrize("N,D,nq,K", [(150001, 128, 5, 4), (131072, 128, 1, 8), (100003, 256, 16, 8), (60007, 384, 2, 5), (49169, 512, 1, 1),
+                                      (16384, 768, 1, 5), (16385, 768, 2, 8), (33000, 1024, 3, 8)])
+def test_scan_ring(hip, N, D, nq, K):
+    """Waves of one tile to more than the ring holds, and a wave's last stages, which are waited for together."""
+    test_scan(hip, N, D, nq, K)
+
+
+def test_hits_as_they_arrive(hip):
+    """The handle of a search: rows as the packed form's, -1 and rows without a comparable score left out; handles dropped unread."""
+    g = torch.Generator(device=DEV).manual_seed(9)
+    c = torch.randn(20011, 768, device=DEV, generator=g).to(torch.bfloat16)
+    c[5:9] = float("nan")
+    few = torch.full((3, 768), float("nan"), device=DEV, dtype=torch.bfloat16)
+    few[1] = 1.0
+    for corpus in (c, few):
+        cn = ops.row_norms(corpus)
+        for nq, K in ((1, 1), (1, 3), (16, 3)):
+            q = torch.randn(nq, 768, device=DEV, generator=g).to(torch.bfloat16)
+            s, i = ops.knn_packed(corpus, cn, q, K).cpu()
+            for _ in range(20):
+                ops.knn_hits(corpus, cn, q.flip(1).contiguous(), K)      # dropped at once
+                h = ops.knn_hits(corpus, cn, q, K)
+                h.synchronize()
+                assert h.query()
+                for k in (K, 1):
+                    want = [[(int(b), float(a)) for a, b in zip(x, y) if b >= 0][:k] for x, y in zip(s.view(torch.float32), i)]
+                    assert h.rows(k) == want
+    assert ops.knn_hits(c, ops.row_norms(c), torch.randn(17, 768, device=DEV).to(torch.bfloat16), 3) is None
+
+
 def test_index_search_agrees(hip):
     """RagIndex gives the same hits whether or not the one-pass search takes the shape."""
     g = torch.Generator(device=DEV).manual_seed(3)
