@@ -1321,7 +1321,7 @@ def _cfg_of(M: int, N: int, K: int, epi: int):
             cfg = None
         elif cfg is not None and not SPLIT_ON and cfg[0] in GEMM1W_SPLIT:
             cfg = (3, 256, 1)
-    return cfg if cfg is not None else _tile_rule(M, N, K, epi)
+    return cfg if cfg is not None else _rounds_rule(M, N, K, epi) or _tile_rule(M, N, K, epi)
 
 
 # Shapes without a measured entry, more than 256 rows: gemm1w.hip's 128 / 192 / 256-row tiles against the fallback.  Its
@@ -1373,9 +1373,7 @@ def _tiled_cost(M: int, N: int, K: int, epi: int) -> Optional[float]:
 
 def _tile_rule(M: int, N: int, K: int, epi: int):
     d = _gemm_default(M, N, K, epi)
-    # (past the rows it was fitted on a launch is many waves, whose stores overlap and which this cost does not describe: the encoder's
-    # 62,500-row batches ran 1.6 % longer on its pick.  The fallback stays there, also at 4,608 - 8,192 rows, where the best tiles
-    # measured up to 1.5 times faster than it: 768 x 768 GELU at M 6500 22.9 / 15.1, 3072 x 2048 at M 5500 88.7 / 68.9)
+    # (past the rows it was fitted on a launch is several waves, whose stores overlap and which this cost does not describe: _rounds_rule)
     if not GEMM1W or not 256 < M <= 4608 or epi > 4 or K // 64 < 3 or N % 256 or d is None:
         return d
     key = (M, N, K, epi, d)
@@ -1392,6 +1390,28 @@ def _tile_rule(M: int, N: int, K: int, epi: int):
             clear = 0.8 if d[2] > 1 and K >= 5632 else 1.0
         _TILE_RULE[key] = (best, 256, 1) if cost(best) < clear * other else d
     return _TILE_RULE[key]
+
+
+def _rounds_cost(M: int, N: int, bm: int) -> float:
+    """Time of one K-tile over all rounds of ``bm`` x 256 tiles: a tile takes a + b * (share of the CUs at work beside it), with the constants
+    of grouped_tile_rows in csrc/gemm.hip."""
+    cus, f = device_cus(), bm / 256
+    a, b = 1.41 * f - 0.17, 0.69 - 0.18 * f
+    whole, part = divmod(-(-M // bm) * (N // 256), cus)
+    return whole * (a + b) + (a + b * part / cus if part else 0.0)
+
+
+def _rounds_rule(M: int, N: int, K: int, epi: int):
+    """Tile of an unsplit product past the rows that ``_tile_rule`` covers, or None: 256 or 192 rows of gemm1w.hip by their rounds over the CUs
+    alone, 192 where those take 3 % less.  Over 174 products (4,700 - 66,000 rows, N 768 - 28,672, K 768 - 5,632, four epilogues) the pick is
+    1.3 % behind the better of the two.  Where N is a multiple of 192 the fallback takes gemm.hip's 192 columns, whose kernel needs 1.1 - 1.3
+    times as long: 58,963 x 2304 x 768 248 -> 205 us, 8,925 x 2304 x 1536 70 -> 56, 44,104 x 768 x 768 65 -> 56, 5,500 x 3072 x 2048 89 -> 69."""
+    if not GEMM1W or M <= 4608 or epi > 4 or K // 64 < 3 or N % 256 or (M + 256) * max(N, K) * 2 >= 0x7FFFFFF0:   # (its 32-bit offsets)
+        return None
+    d = _gemm_default(M, N, K, epi)
+    if d is None or d[2] != 1:
+        return None
+    return (4, 256, 1) if _rounds_cost(M, N, 192) < 0.97 * _rounds_cost(M, N, 256) else (3, 256, 1)
 
 
 def _resid_cfg(M: int, N: int, K: int):

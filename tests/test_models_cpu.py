@@ -421,6 +421,21 @@ def test_tile_rule_takes_what_measured_fastest(monkeypatch, M, N, K, epi, pick):
     assert ops._tile_rule(M, N, K, epi) == (ops._gemm_default(M, N, K, epi) if pick is None else (pick, 256, 1))
 
 
+@pytest.mark.parametrize("M,N,K,epi,pick", [
+    (58963, 2304, 768, 2, 3), (35218, 1536, 768, 2, 3), (44104, 768, 768, 2, 4), (17401, 768, 768, 2, 3), (8925, 2304, 1536, 0, 4), (5500, 3072, 2048, 0, 4),
+    (62947, 6144, 2048, 0, 3), (14488, 1536, 4096, 0, 4), (4609, 768, 3072, 2, None), (4608, 2304, 768, 2, None), (9000, 192, 768, 0, None),
+    (200000, 6144, 2048, 0, None)])
+def test_rounds_rule_takes_what_measured_fastest(monkeypatch, M, N, K, epi, pick):
+    """Row tiles past 4,608 rows by their rounds over the CUs; split-K, fewer rows and widths without 256-column tiles keep their rules."""
+    from llm_kubernetes_minikube_sharp4dev_amd import ops
+
+    monkeypatch.setattr(ops, "GEMM1W", True)
+    monkeypatch.setattr(ops, "_CUS", 256)
+    assert ops._rounds_rule(M, N, K, epi) == (None if pick is None else (pick, 256, 1))
+    monkeypatch.setattr(ops, "GEMM1W", False)
+    assert ops._rounds_rule(M, N, K, epi) is None
+
+
 def test_few_row_rule_counts_the_devices_cus(monkeypatch):
     """The few-row kernel's rounds are of the device's CUs: what it wins on a whole chip (128 workgroups in half a round) it loses on a
     partition of 32 CUs, where they are four rounds."""
