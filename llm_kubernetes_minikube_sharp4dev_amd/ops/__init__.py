@@ -1403,7 +1403,7 @@ def _rounds_cost(M: int, N: int, bm: int) -> float:
 
 def _rounds_rule(M: int, N: int, K: int, epi: int):
     """Tile of an unsplit product past the rows that ``_tile_rule`` covers, or None: 256 or 192 rows of gemm1w.hip by their rounds over the CUs
-    alone, 192 where those take 3 % less.  Over 174 products (4,700 - 66,000 rows, N 768 - 28,672, K 768 - 5,632, four epilogues) the pick is
+    alone, 192 where those take 3 % less.  Over 98 products (4,700 - 66,000 rows, N 768 - 28,672, K 768 - 5,632, four epilogues) the pick is
     1.3 % behind the better of the two.  Where N is a multiple of 192 the fallback takes gemm.hip's 192 columns, whose kernel needs 1.1 - 1.3
     times as long: 58,963 x 2304 x 768 248 -> 205 us, 8,925 x 2304 x 1536 70 -> 56, 44,104 x 768 x 768 65 -> 56, 5,500 x 3072 x 2048 89 -> 69."""
     if not GEMM1W or M <= 4608 or epi > 4 or K // 64 < 3 or N % 256 or (M + 256) * max(N, K) * 2 >= 0x7FFFFFF0:   # (its 32-bit offsets)
