@@ -196,16 +196,22 @@ LK_DEVICE void load_q(const bf16_t* qrow, bool valid, uint4_t (&qf)[(RP + RDP) /
   for (int s = 0; s < (RP + RDP) / 32; ++s) qf[s] = valid ? ld16(qrow + 32 * s + 8 * g) : uint4_t{0u, 0u, 0u, 0u};
 }
 
+// a page's number and place: shifts where pages hold a power of two of rows (a division of scalars is 40 instructions)
+struct Paging {
+  int BS, shift;
+  LK_DEVICE explicit Paging(int bs) : BS(bs), shift((bs & (bs - 1)) == 0 ? __builtin_ctz(bs) : -1) {}
+  LK_DEVICE int page(int key) const { return shift >= 0 ? key >> shift : key / BS; }
+  LK_DEVICE int row(int key) const { return shift >= 0 ? key & (BS - 1) : key % BS; }
+};
 // the page of the 16-key group kg (a multiple of 16, clamped to the sequence's last group): pages hold a multiple of 16 rows, so
 // a group lies in one page
-LK_DEVICE int group_page(const int* bt, int BS, int kg, int last) { return bt[min(kg, last) / BS]; }
+LK_DEVICE int group_page(const int* bt, const Paging& pg, int kg, int last) { return bt[pg.page(min(kg, last))]; }
 
-// 64 pieces of 16 bytes (one per lane, `src`) to 1,024 consecutive bytes of LDS at `dst` (wave-uniform), without registers.  Written as
+// 64 pieces of 16 bytes (one per lane) to 1,024 consecutive bytes of LDS at `dst` (wave-uniform), without registers.  Written as
 // assembly: the builtin makes the compiler wait for it before every transposed LDS read, also of the other buffer.  The caller
 // waits (vmcnt) before the piece is read.
-LK_DEVICE void request_piece(const void* src, void* dst) {
-  const unsigned off = __builtin_amdgcn_readfirstlane((unsigned)reinterpret_cast<uintptr_t>((lds_void_ptr)dst));
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(off), "v"(src) : "memory", "m0");
+LK_DEVICE void request_piece(const void* base, unsigned at, unsigned dst) {   // (base, dst: wave-uniform; at: this lane's bytes behind base)
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(at), "s"(base) : "memory", "m0");
 }
 
 constexpr int kPreCols = 128;
@@ -215,31 +221,69 @@ constexpr int pre_groups() { return 2; }
 template <int RP>
 constexpr int pre_waves() { return kPreCols / (16 * pre_groups<RP>()); }
 
-// grid (query tiles, head blocks): tile x is found by walking the sequences (at most ceil(qlen / NQ) tiles each, a sequence's last
-// queries first: they see the most keys)
+// the tile of a prompt workgroup, found by walking the sequences (at most ceil(qlen / NQ) tiles each, a sequence's last queries first: they
+// see the most keys); false: none
+LK_DEVICE bool find_tile(const int* cu_q, int nseq, int NQ, int& b, int& q0) {
+  const int tile = blockIdx.x;
+  int acc = 0;
+  for (int i = 0; i < nseq; ++i) {
+    const int nt = (cu_q[i + 1] - cu_q[i] + NQ - 1) / NQ;
+    if (tile < acc + nt) {
+      b = i;
+      q0 = (nt - 1 - (tile - acc)) * NQ;
+      return true;
+    }
+    acc += nt;
+  }
+  return false;
+}
+
+// 32 cache rows from key kb on (pages page0, page1) to LDS at dst without registers (LDS-DMA) by W waves: 64 pieces of 16 bytes per wave
+// instruction, in the order of their places in LDS; the source piece of a place is the one the swizzle puts there
+template <int KD, int W>
+struct TileRequest {
+  static constexpr int CPR = KD / 8, NCH = 32 * CPR, NL = (NCH / 64 + W - 1) / W, STEP = 64 * W;   // NL: instructions of a wave, STEP: pieces per round of the waves
+  static_assert(16 * CPR % 64 == 0, "an instruction's pieces belong to one 16-key group");
+  const bf16_t* group[2];
+  unsigned dst;
+  int w, r, pos;   // row and place of this lane's piece, stepped from instruction to instruction (made anew per tile: registers are scarce)
+  LK_DEVICE TileRequest(const bf16_t* cache, const Paging& pg, int kb, int last, int page0, int page1, unsigned char* to) {
+    w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    group[0] = cache + ((long)__builtin_amdgcn_readfirstlane(page0) * pg.BS + pg.row(min(kb, last))) * KD;
+    group[1] = cache + ((long)__builtin_amdgcn_readfirstlane(page1) * pg.BS + pg.row(min(kb + 16, last)) - 16) * KD;
+    dst = __builtin_amdgcn_readfirstlane((unsigned)reinterpret_cast<uintptr_t>((lds_void_ptr)to));
+    const int piece0 = 64 * w + (int)(threadIdx.x & 63);
+    r = piece0 / CPR;
+    pos = piece0 % CPR;
+    asm volatile("" : "+v"(r), "+v"(pos));
+  }
+  LK_DEVICE void issue(int i) {   // the i-th, in order
+    const int blk = W * i + w;    // wave-uniform
+    if (NCH / 64 % W == 0 || blk < NCH / 64)
+      request_piece(group[blk >= 16 * CPR / 64], (unsigned)(r * (KD * 2) + ((pos & ~7) | ((pos & 7) ^ swz(r))) * 16), dst + blk * 1024);
+    r += STEP / CPR;
+    pos += STEP % CPR;
+    if (pos >= CPR) {
+      pos -= CPR;
+      ++r;
+    }
+  }
+  LK_DEVICE void all() {
+#pragma unroll
+    for (int i = 0; i < NL; ++i) issue(i);
+  }
+};
+
+// grid (query tiles, head blocks)
 template <int RP, int RDP>
 __global__ __launch_bounds__(pre_waves<RP>() * 64, RP >= 256 ? 1 : 2) void lat_prefill_kernel(LatParams p, const int* __restrict__ cu_q, const int* __restrict__ ctx_lens,
                                                                      int nseq) {
-  constexpr int KD = RP + RDP, CPR = KD / 8, VT = RP / 16, NCH = 32 * CPR, NL = (NCH / 64 + pre_waves<RP>() - 1) / pre_waves<RP>(),
-                CG = pre_groups<RP>();
+  constexpr int KD = RP + RDP, VT = RP / 16, CG = pre_groups<RP>();
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];   // two tiles of 32 rows
-  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), n16 = lane & 15, g = lane >> 4;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n16 = lane & 15, g = lane >> 4;
   const int NQ = kPreCols / p.HC;
-  int b = -1, q0 = 0;
-  {
-    const int tile = blockIdx.x;
-    int acc = 0;
-    for (int i = 0; i < nseq; ++i) {
-      const int nt = (cu_q[i + 1] - cu_q[i] + NQ - 1) / NQ;
-      if (tile < acc + nt) {
-        b = i;
-        q0 = (nt - 1 - (tile - acc)) * NQ;
-        break;
-      }
-      acc += nt;
-    }
-  }
-  if (b < 0) return;   // the whole workgroup leaves
+  int b = 0, q0 = 0;
+  if (!find_tile(cu_q, nseq, NQ, b, q0)) return;   // the whole workgroup leaves
   const int qbeg = cu_q[b], qlen = cu_q[b + 1] - qbeg, ctx = ctx_lens[b], past = ctx - qlen;
   uint4_t qf[CG][KD / 32];
   floatx4 o[CG][VT];
@@ -258,31 +302,8 @@ __global__ __launch_bounds__(pre_waves<RP>() * 64, RP >= 256 ? 1 : 2) void lat_p
   const int k1 = min(ctx, past + q0 + NQ), k0 = first_key(past + q0, p.window) & ~31, last = (k1 - 1) & ~15;
   const int* bt = p.bt + (long)b * p.bt_stride;
   const bf16_t* cache = reinterpret_cast<const bf16_t*>(p.cache);
-  // a tile travels from the cache to LDS without registers (LDS-DMA): 64 pieces of 16 bytes per wave instruction, in the order of
-  // their places in LDS; the source piece of a place is the one the swizzle puts there
-  const int piece0 = 64 * w + lane;
-  constexpr int STEP = 64 * pre_waves<RP>();   // pieces per round of the workgroup's waves
-  auto request = [&](int kb, int page0, int page1, int which) {
-    const int r0 = __builtin_amdgcn_readfirstlane(page0) * p.BS + min(kb, last) % p.BS,
-              r1 = __builtin_amdgcn_readfirstlane(page1) * p.BS + min(kb + 16, last) % p.BS;
-    unsigned char* dst = smem + which * 64 * KD;
-    int r = piece0 / CPR, pos = piece0 % CPR;   // row and place of this lane's piece, stepped from instruction to instruction
-    asm volatile("" : "+v"(r), "+v"(pos));      // (recomputed per tile: the registers are worth more than the few operations)
-#pragma unroll
-    for (int i = 0; i < NL; ++i) {
-      const int blk = pre_waves<RP>() * i + w;   // wave-uniform
-      if (NCH / 64 % pre_waves<RP>() == 0 || blk < NCH / 64) {
-        const int cc = (pos & ~7) | ((pos & 7) ^ swz(r));
-        request_piece(cache + (long)((r < 16 ? r0 : r1) + (r & 15)) * KD + cc * 8, dst + blk * 1024);
-      }
-      r += STEP / CPR;
-      pos += STEP % CPR;
-      if (pos >= CPR) {
-        pos -= CPR;
-        ++r;
-      }
-    }
-  };
+  const Paging pg(p.BS);
+  auto request = [&](int kb, int page0, int page1, int which) { TileRequest<KD, pre_waves<RP>()>(cache, pg, kb, last, page0, page1, smem + which * 64 * KD).all(); };
   for (int pass = 0; pass < 2; ++pass) {
 #pragma unroll
     for (int x = 0; x < CG; ++x) {
@@ -291,16 +312,16 @@ __global__ __launch_bounds__(pre_waves<RP>() * 64, RP >= 256 ? 1 : 2) void lat_p
 #pragma unroll
       for (int vt = 0; vt < VT; ++vt) o[x][vt] = floatx4{0.f, 0.f, 0.f, 0.f};
     }
-    request(k0, group_page(bt, p.BS, k0, last), group_page(bt, p.BS, k0 + 16, last), 0);
-    int n0 = group_page(bt, p.BS, k0 + 32, last), n1 = group_page(bt, p.BS, k0 + 48, last);   // the pages of the tile to request next
+    request(k0, group_page(bt, pg, k0, last), group_page(bt, pg, k0 + 16, last), 0);
+    int n0 = group_page(bt, pg, k0 + 32, last), n1 = group_page(bt, pg, k0 + 48, last);   // the pages of the tile to request next
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     int cur = 0;
     for (int kb = k0; kb < k1; kb += 32) {
       if (kb + 32 < k1) {
         request(kb + 32, n0, n1, cur ^ 1);
-        n0 = group_page(bt, p.BS, kb + 64, last);   // (raw: used, and waited for, in the next round)
-        n1 = group_page(bt, p.BS, kb + 80, last);
+        n0 = group_page(bt, pg, kb + 64, last);   // (raw: used, and waited for, in the next round)
+        n1 = group_page(bt, pg, kb + 80, last);
       }
       lat_tile<RP, RDP, CG, true>(reinterpret_cast<const bf16_t*>(smem + cur * 64 * KD), qf, kb, qpos, klo, s2, m, top, l, o);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the next tile has arrived (this wave's part of it)
@@ -326,6 +347,208 @@ __global__ __launch_bounds__(pre_waves<RP>() * 64, RP >= 256 ? 1 : 2) void lat_p
       bf16_t* orow = reinterpret_cast<bf16_t*>(p.out) + (long)(qbeg + qi) * p.os + (long)head * p.OH + 4 * g;
 #pragma unroll
       for (int vt = 0; vt < VT; ++vt) store_avg(p, orow + 16 * vt, {o[x][vt][0] * f, o[x][vt][1] * f, o[x][vt][2] * f, o[x][vt][3] * f});
+    }
+  }
+}
+
+// The same for latents of 512 + 64 columns, by two pairs of waves.  Four waves of 32 columns each fill a SIMD's registers alone, so nothing
+// hides what a tile's steps wait for: 10,200 cycles a tile for 2,200 of MFMAs, 2,200 of other instructions and 1,700 of LDS.  A pair has 32
+// columns: a wave takes half of the scores' dimensions and half of the latent for all of them and the softmax of its own 16.  Per tile
+// the waves exchange partial scores (f32) and weights (bf16) of 16 columns through LDS, 6 KB a wave for the 34 KB of the tile that it no
+// longer reads.  The registers halve, and two workgroups share a CU, each with its two tiles in half of the LDS to the byte, so one
+// multiplies while the other waits at a barrier (one workgroup of four pairs: 133 us for the first line).  The next tile is requested an
+// instruction per step of the scores: in one go that took 1,300 cycles in which the wave did nothing else.
+// 4,095 rows of 4 prompts, 16 heads, window 512: 144 -> 129 us; 32 heads, window 2,048: 322 -> 282; 300 rows behind 700: 68 -> 44.
+constexpr int kPairWaves = 4, kPairCols = 16 * kPairWaves;
+constexpr int pair_lds(int KD) { return 2 * 64 * KD + kPairWaves * 2048; }
+template <int RP, int RDP>
+constexpr bool in_pairs() { return RP > 256 && 2 * pair_lds(RP + RDP) <= 160 * 1024; }   // (512 + 128 columns: one workgroup a CU, 112 us for 87 by four single waves)
+template <int RP, int RDP>
+__global__ __launch_bounds__(64 * kPairWaves, 2) void lat_prefill_pair_kernel(LatParams p, const int* __restrict__ cu_q, const int* __restrict__ ctx_lens,
+                                                                             int nseq) {
+  constexpr int KD = RP + RDP, VT = RP / 16, HV = VT / 2, HS = KD / 64;   // HV, HS: c^T tiles and steps of 32 dimensions of a wave
+  static_assert(TileRequest<RP + RDP, kPairWaves>::NL <= HS, "an instruction per step");
+  constexpr int QA = 2, VA = 4;                                            // fragments requested ahead of their products
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];    // two tiles of 32 rows, the exchange
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), pr = w >> 1, hf = w & 1;
+  int lane, n16, g;
+  auto fresh = [&]() {   // addresses are made anew from these per tile: kept over the loop they would be spilled
+    lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));
+    n16 = lane & 15;
+    g = lane >> 4;
+  };
+  fresh();
+  const int NQ = kPairCols / p.HC;
+  int b = 0, q0 = 0;
+  if (!find_tile(cu_q, nseq, NQ, b, q0)) return;   // the whole workgroup leaves
+  const int qbeg = cu_q[b], qlen = cu_q[b + 1] - qbeg, ctx = ctx_lens[b], past = ctx - qlen;
+  floatx4* const xs = reinterpret_cast<floatx4*>(smem + 128 * KD) + 128 * w;                  // this wave's partial scores for its partner [2][64]
+  const floatx4* const ys = reinterpret_cast<const floatx4*>(smem + 128 * KD) + 128 * (w ^ 1);   // the partner's for this wave, then this wave's weights
+  // columns: y = 0 this wave's 16, y = 1 the partner's
+  uint4_t qf[2][HS];
+  int qpos = -1;
+#pragma unroll
+  for (int y = 0; y < 2; ++y) {
+    const int c = 16 * (2 * pr + (hf ^ y)) + n16, qi = q0 + c / p.HC, head = blockIdx.y * p.HC + c % p.HC;
+    const bool valid = c / p.HC < NQ && qi < qlen && head < p.H;
+    if (y == 0) qpos = valid ? past + qi : -1;
+    const bf16_t* qrow = reinterpret_cast<const bf16_t*>(p.q) + (long)(qbeg + min(qi, qlen - 1)) * p.qs + (long)min(head, p.H - 1) * KD;
+#pragma unroll
+    for (int s = 0; s < HS; ++s) qf[y][s] = valid ? ld16(qrow + 32 * (hf * HS + s) + 8 * g) : uint4_t{0u, 0u, 0u, 0u};
+  }
+  const int klo = first_key(qpos, p.window);
+  float m = kNegBig, top, l;
+  floatx4 o[2][HV];
+  const float s2 = p.scale * kLog2e;
+  const int k1 = min(ctx, past + q0 + NQ), k0 = first_key(past + q0, p.window) & ~31, last = (k1 - 1) & ~15;
+  const int* bt = p.bt + (long)b * p.bt_stride;
+  const bf16_t* cache = reinterpret_cast<const bf16_t*>(p.cache);
+  const Paging pg(p.BS);
+  using Request = TileRequest<KD, kPairWaves>;
+  auto handed = [&]() {   // LDS written and read as far as asked; the next tile stays on its way
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  for (int pass = 0; pass < 2; ++pass) {
+    top = kNegBig;
+    l = 0.f;
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+#pragma unroll
+      for (int vt = 0; vt < HV; ++vt) o[y][vt] = floatx4{0.f, 0.f, 0.f, 0.f};
+    Request(cache, pg, k0, last, group_page(bt, pg, k0, last), group_page(bt, pg, k0 + 16, last), smem).all();
+    int n0 = group_page(bt, pg, k0 + 32, last), n1 = group_page(bt, pg, k0 + 48, last);   // the pages of the tile to request next
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    int cur = 0;
+    for (int kb = k0; kb < k1; kb += 32) {
+      fresh();
+      const bool more = kb + 32 < k1;
+      Request next(cache, pg, kb + 32, last, n0, n1, smem + (cur ^ 1) * 64 * KD);   // (requested between the scores' products: issuing takes its time)
+      if (more) {
+        n0 = group_page(bt, pg, kb + 64, last);   // (raw: used, and waited for, in the next round)
+        n1 = group_page(bt, pg, kb + 80, last);
+      }
+      const unsigned base = (unsigned)reinterpret_cast<uintptr_t>((lds_void_ptr)(smem + cur * 64 * KD));
+      // ---- this half's scores of both column groups: steps hf HS + s; the two 16-byte chunks of a 64-column piece alternate from step to step
+      floatx4 c[2][2];
+#pragma unroll
+      for (int y = 0; y < 2; ++y) c[y][0] = c[y][1] = floatx4{0.f, 0.f, 0.f, 0.f};
+      const int sw = swz(n16), S0 = hf * HS;   // (rows n16 and 16 + n16 have the same swizzle)
+      const unsigned kc0 = base + n16 * KD * 2 + (g ^ sw) * 16, kc1 = base + n16 * KD * 2 + ((4 + g) ^ sw) * 16;
+      const unsigned ke = ((S0 & 1) ? kc1 : kc0) + 128 * (S0 / 2), ko = ((S0 & 1) ? kc0 : kc1) + 128 * ((S0 + 1) / 2);
+      uint4_t kf[QA][2];
+      static_for<QA>([&](auto sc_) {
+        constexpr int s = decltype(sc_)::value;
+        lds_read16<128 * (s / 2)>(kf[s][0], (s & 1) ? ko : ke);
+        lds_read16<128 * (s / 2) + 16 * KD * 2>(kf[s][1], (s & 1) ? ko : ke);
+      });
+      static_for<HS>([&](auto sc_) {
+        constexpr int s = decltype(sc_)::value, ahead = (s + QA < HS ? QA : HS - s) - 1;
+        lds_wait<2 * ahead>(kf[s % QA][0], kf[s % QA][1]);
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int y = 0; y < 2; ++y) c[y][t] = mma_qk<bf16_t>(kf[s % QA][t], qf[y][s], c[y][t]);
+        if constexpr (s + QA < HS) {
+          lds_read16<128 * ((s + QA) / 2)>(kf[s % QA][0], ((s + QA) & 1) ? ko : ke);
+          lds_read16<128 * ((s + QA) / 2) + 16 * KD * 2>(kf[s % QA][1], ((s + QA) & 1) ? ko : ke);
+        }
+        if constexpr (s < Request::NL) {
+          if (more) next.issue(s);
+        }
+      });
+#pragma unroll
+      for (int t = 0; t < 2; ++t) xs[t * 64 + lane] = c[1][t];
+      handed();
+      // ---- the softmax of this wave's columns, with the first c^T fragments travelling under it
+      const int qq = n16 >> 2, pp = n16 & 3, swv = swz(4 * g + qq);   // rows 4g + qq and 16 + 4g + qq have the same swizzle
+      const unsigned vr = base + (4 * g + qq) * KD * 2 + 8 * (pp & 1) + hf * (RP / 2) * 2;
+      unsigned va[4];
+#pragma unroll
+      for (int x = 0; x < 4; ++x) va[x] = vr + ((2 * x + (pp >> 1)) ^ swv) * 16;
+      const floatx4 d0 = ys[lane], d1 = ys[64 + lane];
+      float sc[2][4];
+      bool ok[2][4];
+      float mx = kNegBig;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int key = kb + 16 * t + 4 * g + j;
+          ok[t][j] = key <= qpos && key >= klo;
+          sc[t][j] = (c[0][t][j] + (t ? d1[j] : d0[j])) * s2;
+          if (ok[t][j]) mx = fmaxf(mx, sc[t][j]);
+        }
+      mx = max_groups(mx);
+      if (m == kNegBig) m = mx;
+      top = fmaxf(top, mx);
+      short8 pb[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float e = ok[t][j] ? __builtin_amdgcn_exp2f(sc[t][j] - m) : 0.f;
+          l += e;
+          pb[0][4 * t + j] = (short)f2bf(e);
+        }
+      const_cast<floatx4*>(ys)[lane] = __builtin_bit_cast(floatx4, pb[0]);   // (only this wave reads there before)
+      handed();
+      pb[1] = __builtin_bit_cast(short8, xs[lane]);
+      // ---- this half of the latent for both column groups
+      short4_t vlo[VA], vhi[VA];
+      static_for<VA>([&](auto vc_) {
+        constexpr int vt = decltype(vc_)::value;
+        lds_read_tr<128 * (vt / 4)>(vlo[vt], va[vt % 4]);
+        lds_read_tr<128 * (vt / 4) + 16 * KD * 2>(vhi[vt], va[vt % 4]);
+      });
+      static_for<HV>([&](auto vc_) {
+        constexpr int vt = decltype(vc_)::value, ahead = (vt + VA < HV ? VA : HV - vt) - 1;
+        lds_wait<2 * ahead>(vlo[vt % VA], vhi[vt % VA]);
+        const short8 a = __builtin_shufflevector(vlo[vt % VA], vhi[vt % VA], 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+        for (int y = 0; y < 2; ++y) o[y][vt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pb[y], o[y][vt], 0, 0, 0);
+        if constexpr (vt + VA < HV) {
+          lds_read_tr<128 * ((vt + VA) / 4)>(vlo[vt % VA], va[(vt + VA) % 4]);
+          lds_read_tr<128 * ((vt + VA) / 4) + 16 * KD * 2>(vhi[vt % VA], va[(vt + VA) % 4]);
+        }
+      });
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the next tile has arrived (this wave's part of it)
+      __syncthreads();
+      cur ^= 1;
+    }
+    // (a vote through the exchange's words: the library's takes LDS of its own, and then no second workgroup fits a CU)
+    const bool grew = top > m + kMaxGrowth;
+    m = pass == 0 && grew ? top : m;
+    const int any = __any(grew);
+    if (lane == 0) *reinterpret_cast<int*>(xs) = any;
+    handed();
+    int again = 0;
+#pragma unroll
+    for (int i = 0; i < kPairWaves; ++i) again |= *reinterpret_cast<const int*>(smem + 128 * KD + 2048 * i);
+    handed();
+    if (!again) break;
+  }
+  // ---- both groups' factors, then this half of the averages
+  fresh();
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  float f[2];
+  const int c0 = 16 * (2 * pr + hf) + n16, head0 = blockIdx.y * p.HC + c0 % p.HC;
+  if (p.sink && qpos >= 0) l += __builtin_amdgcn_exp2f(p.sink[head0] * kLog2e - m);   // one more term without a value
+  f[0] = qpos >= 0 && l > 0.f ? lat_gate<bf16_t>(p, qbeg + q0 + c0 / p.HC, head0) / l : 0.f;
+  reinterpret_cast<float*>(xs)[lane] = f[0];
+  handed();
+  f[1] = reinterpret_cast<const float*>(ys)[lane];
+#pragma unroll
+  for (int y = 0; y < 2; ++y) {
+    const int c = 16 * (2 * pr + (hf ^ y)) + n16, qi = q0 + c / p.HC, head = blockIdx.y * p.HC + c % p.HC;
+    if (c / p.HC < NQ && qi < qlen && head < p.H) {
+      bf16_t* orow = reinterpret_cast<bf16_t*>(p.out) + (long)(qbeg + qi) * p.os + (long)head * p.OH + hf * (RP / 2) + 4 * g;
+#pragma unroll
+      for (int vt = 0; vt < HV; ++vt) store_avg(p, orow + 16 * vt, {o[y][vt][0] * f[y], o[y][vt][1] * f[y], o[y][vt][2] * f[y], o[y][vt][3] * f[y]});
     }
   }
 }
@@ -654,10 +877,16 @@ bool mfma_shape(int RP, int KD) {
 template <int RP, int RDP>
 int launch_prefill(const LatParams& p, const int* cu_q, const int* ctx, int nseq, long rows, hipStream_t st) {
   constexpr size_t lds = 2 * 64 * (RP + RDP);
-  const int NQ = kPreCols / p.HC;
+  const int NQ = (in_pairs<RP, RDP>() ? kPairCols : kPreCols) / p.HC;
   const long tiles = (rows + NQ - 1) / NQ + nseq;   // every sequence ends with at most one partial tile
-  LK_SET_MAX_LDS((lat_prefill_kernel<RP, RDP>), lds);
-  lat_prefill_kernel<RP, RDP><<<dim3((unsigned)tiles, (unsigned)((p.H + p.HC - 1) / p.HC)), pre_waves<RP>() * 64, lds, st>>>(p, cu_q, ctx, nseq);
+  const dim3 grid((unsigned)tiles, (unsigned)((p.H + p.HC - 1) / p.HC));
+  if constexpr (in_pairs<RP, RDP>()) {
+    LK_SET_MAX_LDS((lat_prefill_pair_kernel<RP, RDP>), pair_lds(RP + RDP));
+    lat_prefill_pair_kernel<RP, RDP><<<grid, 64 * kPairWaves, pair_lds(RP + RDP), st>>>(p, cu_q, ctx, nseq);
+  } else {
+    LK_SET_MAX_LDS((lat_prefill_kernel<RP, RDP>), lds);
+    lat_prefill_kernel<RP, RDP><<<grid, pre_waves<RP>() * 64, lds, st>>>(p, cu_q, ctx, nseq);
+  }
   LK_CHECK_LAUNCH();
   return 0;
 }

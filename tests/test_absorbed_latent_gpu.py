@@ -129,6 +129,51 @@ def test_latent_query(T, H, dim, rd, qdim, K, rp, kd, adjacent, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rp,rdp", [(512, 64), (512, 128), (256, 64), (128, 128)])
+@pytest.mark.parametrize("H,lens,past,window,loud", [(16, [1, 3, 4, 5], [0, 40, 31, 32], 24, False), (16, [70, 33], [0, 7], 0, False), (5, [29, 8], [3, 64], 33, True),
+                                                    (40, [65], [17], 48, False), (1, [130, 64], [0, 1], 512, True)])
+def test_prompt_rows(rp, rdp, H, lens, past, window, loud):
+    """Prompt portions behind cached rows on both prompt kernels: queries per workgroup that do and do not divide a portion, heads that do and do not
+    fill a block, windows inside and across 32-key tiles, a sink, gates; loud: later keys so far above the first tile's that the pass is
+    repeated.  Against float64."""
+    from llm_kubernetes_minikube_sharp4dev_amd import ops
+    g = torch.Generator().manual_seed(rp + H)
+    BS, kd, T = 16, rp + rdp, sum(lens)
+    blocks = [-(-(n + p) // BS) for n, p in zip(lens, past)]
+    cache, q = q16(rnd(g, sum(blocks) + 2, BS, kd)), q16(rnd(g, T, H, kd, scale=0.3))
+    order = torch.randperm(sum(blocks) + 2, generator=g)[:sum(blocks)].int()
+    table, at = torch.zeros(len(lens), max(blocks), dtype=torch.int32), 0
+    for i, n in enumerate(blocks):
+        table[i, :n] = order[at:at + n]
+        at += n
+    if loud:   # the last keys of every sequence point along its last query's
+        for i, (n, p) in enumerate(zip(lens, past)):
+            for k in range(max(0, n + p - 6), n + p):
+                cache[table[i, k // BS].long(), k % BS] = q16(q[sum(lens[:i + 1]) - 1, 0] * 60)
+    gate, sink = q16(rnd(g, T, H)), rnd(g, H).float()
+    out = torch.full((T + 1, H, 2 * rp), 7.0, dtype=torch.bfloat16, device="cuda")
+    cu = torch.tensor([0] + lens).cumsum(0).int().cuda()
+    ctx = torch.tensor([n + p for n, p in zip(lens, past)]).int().cuda()
+    ops.latent_attention_prefill(q.bfloat16().cuda(), cache.bfloat16().cuda(), table.cuda(), cu, ctx, window, kd ** -0.5, sink.cuda(), rp, out[:T], max(lens),
+                                 gate=gate.bfloat16().cuda())
+    got, t0 = out[:T, :, :rp].double().cpu() + out[:T, :, rp:].double().cpu(), 0
+    for i, (n, p) in enumerate(zip(lens, past)):
+        rows = cache[table[i, :blocks[i]].long()].reshape(-1, kd)[:n + p].double()
+        s = torch.einsum("qhd,kd->hqk", q[t0:t0 + n].double(), rows) * kd ** -0.5
+        qi, ki = torch.arange(p, p + n)[:, None], torch.arange(n + p)[None]
+        s = s.masked_fill(((ki > qi) | ((ki <= qi - window) if window else torch.zeros_like(ki, dtype=torch.bool)))[None], float("-inf"))
+        s = torch.cat([sink.double().view(H, 1, 1).expand(H, n, 1), s], -1)
+        w = s.softmax(-1)[..., 1:]
+        want = torch.einsum("hqk,kd->qhd", w, rows[:, :rp]) * torch.sigmoid(gate[t0:t0 + n].double())[..., None]
+        size = torch.einsum("hqk,kd->qhd", w, rows[:, :rp].abs())
+        # weights rounded to bf16 (2^-9), scores in f32: up to kd products of the size of the row's largest score
+        big = float(s[s.isfinite()].abs().max())
+        assert bool(((got[t0:t0 + n] - want).abs() <= (2.0 ** -8 + big * 2.0 ** -18) * size + 1e-5).all()), float(((got[t0:t0 + n] - want).abs() / (size + 1e-9)).max())
+        t0 += n
+    assert bool((out[T] == 7.0).all())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("splits", [1, 2, 4, 5, 70])
 def test_decode_splits_agree_with_gates(splits):
     """One query row per sequence over any number of key splits, gated: against float64."""
