@@ -681,6 +681,15 @@ at::Tensor embed_rows(const at::Tensor& table, const at::Tensor& ids, int64_t lo
 }
 
 // ids[dst] = prev[src] (in-flight decode inputs of a pipelined step)
+// ids (int32, on the GPU) = the host's values; false where they are more than one launch takes
+bool set_ids(at::Tensor& ids, const at::Tensor& host) {
+  CHECK_CUDA(ids); CHECK_I32(ids); CHECK_CONTIG(ids); CHECK_I32(host); CHECK_CONTIG(host);
+  TORCH_CHECK(host.device().is_cpu() && host.numel() == ids.numel(), "set_ids: as many host values as ids");
+  if (ids.numel() > kLkFewIds) return false;
+  CHECK_RC(lk_set_ids(ids.data_ptr<int>(), host.data_ptr<int>(), (int)ids.numel(), cur_stream()), "set_ids");
+  return true;
+}
+
 void scatter_ids(at::Tensor& ids, const at::Tensor& dst, const at::Tensor& prev, const at::Tensor& src) {
   CHECK_CUDA(ids); CHECK_I32(ids); CHECK_CONTIG(ids); CHECK_I32(prev); CHECK_CONTIG(prev);
   TORCH_CHECK(dst.scalar_type() == at::kLong && src.scalar_type() == at::kLong && dst.is_contiguous() && src.is_contiguous() &&
@@ -2503,6 +2512,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("embed_errors", []() { return (int64_t)lk_embed_errors(); },
         "token ids outside the (whole) embedding table seen since the last call (resets)");
   m.def("scatter_ids", &scatter_ids);
+  m.def("set_ids", &set_ids);
   m.def("gather_rows", &gather_rows);
   m.def("argmax_key", &argmax_key, "", py::arg("logits"), py::arg("vocab_lo") = 0);
   m.def("keys_to_ids", &keys_to_ids);

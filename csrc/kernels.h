@@ -256,6 +256,8 @@ int lk_debug_invalid_launch(hipStream_t st);
 int lk_embed_rows(bf16_t* out, const bf16_t* table, const int* ids, long T, int H, long lo, long n_local,
                   hipStream_t st, int strict = 0);
 int lk_embed_errors();  // out-of-table ids seen by strict lk_embed_rows since the last call
+constexpr int kLkFewIds = 64;
+int lk_set_ids(int* ids, const int* host, int n, hipStream_t st);   // host: n <= kLkFewIds values, read before the call returns
 int lk_scatter_ids(int* ids, const long* dst, const int* prev, const long* src, int n, hipStream_t st);
 int lk_gather_rows(bf16_t* out, const bf16_t* x, long xs, const long* idx, long R, int H, hipStream_t st);
 

@@ -36,6 +36,16 @@ __global__ __launch_bounds__(256) void scatter_ids_kernel(int* __restrict__ ids,
   if (i < n) ids[dst[i]] = prev[src[i]];
 }
 
+// ids[i] = v[i], the values in the launch's own arguments: a few host ids reach the device without a pinned block and a copy (whose launch and
+// bookkeeping cost 7 us in front of a query's graph)
+struct FewIds {
+  int v[kLkFewIds];
+};
+__global__ __launch_bounds__(64) void set_ids_kernel(int* __restrict__ ids, const FewIds x, int n) {
+  const int i = blockIdx.x * 64 + threadIdx.x;
+  if (i < n) ids[i] = x.v[i];
+}
+
 // out[r, :] = x[idx[r], :]  (rows of H bf16, x row stride xs)
 __global__ __launch_bounds__(256) void gather_rows_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
                                                           long xs, const long* __restrict__ idx, long R, int H) {
@@ -76,6 +86,16 @@ int lk_scatter_ids(int* ids, const long* dst, const int* prev, const long* src, 
   if (n < 0) return -1;
   if (n == 0) return 0;
   scatter_ids_kernel<<<(n + 255) / 256, 256, 0, st>>>(ids, dst, prev, src, n);
+  return 0;
+}
+
+int lk_set_ids(int* ids, const int* host, int n, hipStream_t st) {
+  if (n < 0 || n > kLkFewIds) return -1;
+  if (n == 0) return 0;
+  FewIds x{};
+  for (int i = 0; i < n; ++i) x.v[i] = host[i];
+  set_ids_kernel<<<(n + 63) / 64, 64, 0, st>>>(ids, x, n);
+  LK_CHECK_LAUNCH();
   return 0;
 }
 

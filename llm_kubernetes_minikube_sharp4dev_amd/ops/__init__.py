@@ -1503,6 +1503,12 @@ def embed_rows(table, ids, lo: int = 0, n_local: Optional[int] = None):
     return table[local.clamp(0, max(0, n_local - 1))].masked_fill(mask[:, None], 0)
 
 
+def set_ids(ids, host):
+    """ids (int32) = host (CPU int32); on the GPU a few travel in a launch's own arguments, without a pinned copy."""
+    if not (use_hip(ids) and lib().set_ids(ids, host)):
+        ids.copy_(host.pin_memory() if ids.is_cuda else host, non_blocking=True)
+
+
 def scatter_ids(ids, dst, prev, src):
     """ids[dst] = prev[src] (the in-flight decode inputs of a pipelined step), one launch."""
     if use_hip(ids) and ids.dtype == torch.int32 and prev.dtype == torch.int32:
