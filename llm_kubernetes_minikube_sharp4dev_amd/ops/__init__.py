@@ -736,6 +736,7 @@ def gemm(x, w, b=None, epi: int = 0, out=None):
     if out is not None and (out.data_ptr() % 16 or out.stride(0) % 8 or out.stride(1) != 1):
         return None
     cfg = _cfg_of(M, N, K, epi)
+    cfg = _split_rule(M, N, K, epi, cfg, x.stride(0) if out is None else max(x.stride(0), out.stride(0)))
     if cfg is None or not lib().gemm_supported(M, N, K, epi, cfg[1], cfg[2], cfg[0]):
         return None
     return lib().gemm(x, w, b, epi, cfg[1], out, cfg[0], cfg[2])
@@ -1368,6 +1369,11 @@ def _tiled_cost(M: int, N: int, K: int, epi: int) -> Optional[float]:
         return None
     cost, other = _tile_times(M, N, K, epi, d)
     cfg = _cfg_of(M, N, K, epi)
+    split = _split_rule(M, N, K, epi, cfg, 0)
+    if split != cfg and split[2] > 1:
+        # (the few-row kernel runs 10 - 20 % ahead of its estimate at these rows, and within a forward pass the sum's launch has a gap before it:
+        # at 512 rows 2048 x 5632 28.7 split and 28.3 in it, 3072 x 2048 22.9 and 18.6)
+        return 1.2 * (_split_cost(M, N, K, split[0], split[2]) + (2.5 if epi == 3 else 0))
     return cost(cfg[0]) if cfg is not None and cfg != d and cfg[0] in _TILE_COST else other
 
 
@@ -1414,12 +1420,56 @@ def _rounds_rule(M: int, N: int, K: int, epi: int):
     return (4, 256, 1) if _rounds_cost(M, N, 192) < 0.97 * _rounds_cost(M, N, 256) else (3, 256, 1)
 
 
-def _resid_cfg(M: int, N: int, K: int):
+# A plain, bias, activation or residual product of 257 - 4,608 rows may also run as 2 - 8 ranges of K on gemm1w.hip's tiles, f32 partials
+# and a sum behind them.  Unsplit, N 2048 at 300 rows is 24 tiles of 128 rows on 256 CUs that each walk all of K; gemm.hip's
+# split has 256-row tiles, four ranges at most and twice the time per 64 columns.  A round of workgroups costs a + f b us per 64 columns of its range
+# (f: how much of the chip the launch fills), a further one c more, the launch 6.3 - 9.9 us, the sum 2.9 us and 0.46 us per range and MB of
+# bf16 output: within 5.1 % (rms) of 20,000 launches, N 512 - 10,240, K 512 - 14,336.  An unsplit tile is left where that is 5 % less,
+# gemm.hip's split for the best of all of these (it was the fastest of none).  Weights cold, before / the pick (us):
+#   4096 x 4096: M 350 39.7 / 25.7 (4 of 128 rows)   M 512 41.6 / 31.6   M 1024 45.1 / 42.1 (2)   from M 1152 on the same (unsplit)
+#   4096 x 14336: M 512 89.3 / 66.9 (4)   M 768 98.9 / 86.2 (4 of 192)   M 1024 115.2 / 106.0 (4 of 256)   M 1536 170 / 140 (2 of 192)
+#   2048 x 5632: M 300 40.6 / 21.2 (8)   M 768 44.4 / 30.1 (4)   M 2048 63.3 / 51.0 (2)   M 3072 85.6 / 64.6 (1)
+#   1024 x 4096: M 300 33.3 / 16.5 (8)   M 1024 35.8 / 22.9   M 3072 47.7 / 36.6 (2)      2048 x 2048: M 300 22.6 / 14.9 (4)   M 768 24.1 / 20.8 (3)
+# Over the 1,325 products of two sweeps (one of them of random shapes) the picks take 0.9 % more than the best of all kernels, those before 28 %.
+# v: (rows, start and end, a, b, c)
+_SPLIT_COST = {5: (128, 6.3, 0.451, 0.319, 5.0), 4: (192, 8.1, 0.658, 0.357, 6.4), 3: (256, 9.9, 0.868, 0.409, 8.1)}
+_SPLIT_RULE: dict = {}
+
+
+def _split_cost(M: int, N: int, K: int, v: int, ks: int) -> float:
+    bm, ends, a, b, c = _SPLIT_COST[v]
+    cus = device_cus()
+    wgs = -(-M // bm) * (N // 256) * ks
+    rounds = -(-wgs // cus)
+    return (ends + rounds * -(-(K // 64) // ks) * (a + b * wgs / (rounds * cus)) + (rounds - 1) * c
+            + (2.9 + 0.46e-6 * ks * M * N * 2 if ks > 1 else 0.0))
+
+
+def _split_rule(M: int, N: int, K: int, epi: int, cfg, ld: int):
+    """The pick ``cfg`` of :func:`_cfg_of`, or what the costs above take instead: (variant, 256, ranges of K).  ``ld``: the longest of the
+    operands' row strides -- a split needs them whole within 32-bit offsets, where rows further apart go in chunks unsplit and in gemm.hip.
+    (The start-up measurements pass here too: they hold no split of these tiles.)"""
+    if (not (GEMM1W and GEMM_SPLITK) or not 256 < M <= 4608 or epi not in (0, 2, 3, 4) or N % 256 or K % 64 or cfg is None
+            or cfg[0] in GEMM1W_SPLIT or max(N, ld) * (M + 256) >= 1 << 26 or N * K * 2 >= 0x7FFFFFF0):
+        return cfg
+    key = (M, N, K, cfg)
+    if key not in _SPLIT_RULE:
+        costs = {(v, 256, ks): _split_cost(M, N, K, v, ks) for v in _SPLIT_COST for ks in (1, 2, 3, 4, 6, 8)
+                 if K // 64 >= 3 * ks}
+        best = min(costs, key=costs.get, default=cfg)
+        if cfg in costs and (best[2] == 1 or costs[best] > 0.95 * costs[cfg]):
+            best = cfg
+        if len(_SPLIT_RULE) > 4096:
+            _SPLIT_RULE.clear()
+        _SPLIT_RULE[key] = best
+    return _SPLIT_RULE[key]
+
+
+def _resid_cfg(M: int, N: int, K: int, ld: int = 0):
     c = _cfg_of(M, N, K, 0)
-    if c is not None and c[0] in GEMM1W_BM:
-        return c  # (variant, 256, 1)
-    sched = c[0] if c is not None else _gemm_sched(K)
-    return sched, 256, _gemm_splits(M, N, K, 0, 256)
+    if c is None or c[0] not in GEMM1W_BM:
+        c = (c[0] if c is not None else _gemm_sched(K), 256, _gemm_splits(M, N, K, 0, 256))
+    return _split_rule(M, N, K, 0, c, ld)
 
 
 def prefill_chain_ok(x, w_qkv, w_o, w_gate_up, w_down) -> bool:
@@ -1459,7 +1509,7 @@ def linear_resid(x, w, residual, ss_out):
         return ref.linear_resid(x, w, residual, ss_out)
     M, K = x.shape
     N = w.shape[0]
-    sched, bn, ks = _resid_cfg(M, N, K)
+    sched, bn, ks = _resid_cfg(M, N, K, max(x.stride(0), residual.stride(0)))
     return lib().gemm_fused(x, w, EPI_RESID, bn, None, sched, ks, resid=residual, ss_out=ss_out)
 
 

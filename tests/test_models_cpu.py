@@ -421,6 +421,27 @@ def test_tile_rule_takes_what_measured_fastest(monkeypatch, M, N, K, epi, pick):
     assert ops._tile_rule(M, N, K, epi) == (ops._gemm_default(M, N, K, epi) if pick is None else (pick, 256, 1))
 
 
+@pytest.mark.parametrize("M,N,K,epi,cfg,pick", [
+    (300, 4096, 4096, 0, (2, 256, 4), (5, 256, 4)), (1152, 4096, 4096, 0, (5, 256, 1), (5, 256, 1)), (1536, 4096, 14336, 0, (2, 256, 2), (4, 256, 2)),
+    (300, 2048, 5632, 0, (2, 256, 4), (5, 256, 8)), (3072, 2048, 5632, 0, (2, 256, 2), (5, 256, 1)), (512, 2048, 2048, 0, (5, 256, 1), (5, 256, 4)),
+    (1024, 2048, 1024, 3, (5, 256, 1), (5, 256, 1)), (4608, 4096, 4096, 0, (3, 256, 1), (3, 256, 1)),
+    (256, 4096, 4096, 0, (2, 256, 4), None), (4609, 2048, 5632, 0, (2, 256, 2), None), (300, 2112, 4096, 0, (2, 192, 4), None),
+    (300, 4096, 4096, 1, (0, 256, 1), None), (2664, 6144, 4096, 0, (6, 256, 1), None), (300, 256, 128, 0, (0, 256, 1), None), (300, 2048, 2048, 0, None, None)])
+def test_split_rule_takes_what_measured_fastest(monkeypatch, M, N, K, epi, cfg, pick):
+    """Ranges of K on gemm1w.hip's tiles, on both sides of the line (None: the rule does not take the product, whatever its pick)."""
+    from llm_kubernetes_minikube_sharp4dev_amd import ops
+
+    for name, value in (("GEMM1W", True), ("GEMM_SPLITK", True), ("_CUS", 256), ("_SPLIT_RULE", {})):
+        monkeypatch.setattr(ops, name, value)
+    assert ops._split_rule(M, N, K, epi, cfg, K) == (pick or cfg)
+    got = ops._split_rule(M, N, K, epi, cfg, (1 << 26) // (M + 256) + 1)   # rows too far apart for 32-bit offsets
+    assert got == cfg
+    for name in ("GEMM1W", "GEMM_SPLITK"):
+        monkeypatch.setattr(ops, name, False)
+        assert ops._split_rule(M, N, K, epi, cfg, K) == cfg
+        monkeypatch.setattr(ops, name, True)
+
+
 @pytest.mark.parametrize("M,N,K,epi,pick", [
     (58963, 2304, 768, 2, 3), (35218, 1536, 768, 2, 3), (44104, 768, 768, 2, 4), (17401, 768, 768, 2, 3), (8925, 2304, 1536, 0, 4), (5500, 3072, 2048, 0, 4),
     (62947, 6144, 2048, 0, 3), (14488, 1536, 4096, 0, 4), (4609, 768, 3072, 2, None), (4608, 2304, 768, 2, None), (9000, 192, 768, 0, None),
