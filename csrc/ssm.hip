@@ -687,8 +687,8 @@ __global__ __launch_bounds__(256) void ssm_chunk_kernel(const T* __restrict__ xb
 // enters a product as three bf16 parts (8 + 8 + 8 mantissa bits, an f32), summed in the f32 accumulators.  A sequence's chunks are a
 // serial chain, so what bounds the kernel is the time of one chunk: 64 tokens take 130 products of 16 cycles per wave instead of
 // 4 x 100 of 32 (16x16x4 f32), with two barriers instead of eight.  4 x 1,024 tokens, 64 heads of [64, 128]: 351 us (f32
-// products, chunks of 16) -> 133 -> 126 us (operands filed and prefetched as below); y writes 67 MB and the
-// rows read 50.  Error against f64 9e-8 (f32 products: 2.2e-7).
+// products, chunks of 16) -> 126 us (now ssm_pipe_kernel's, which takes states of 33 - 128 columns); 4 x 512, 32 heads of [64, 256] 75 us.
+// Error against f64 9e-8 (f32 products: 2.2e-7).
 // grid (sequence, head, P / 64): wave w owns state columns p0 + 16 w .. +15 (all N rows as accumulators S[n][p]: lane p = l & 15,
 // rows 16 nt + 4 (l >> 4) + j) and computes M's rows of token tile w for everybody.  y is accumulated transposed (lane: one token,
 // four adjacent columns).  The order of n inside a 32-step is (4g + j, 16 + 4g + j), so that the accumulators are operands as they lie.
@@ -973,6 +973,321 @@ __global__ __launch_bounds__(256, 1) void ssm_chunk_bf16_kernel(const bf16_t* __
   }
 }
 
+// The same for states of 33 - 128 columns and prompts, as a pipeline of 16 waves in one workgroup.  A chunk's chain is latency, not work (with four
+// waves, one to a SIMD, 12 k cycles for 4.6 k of vector and 2 k of matrix instructions per SIMD), and half of it does not depend on the state: eight waves
+// file the next chunk's rows, its decays and then its M, eight carry the state and y behind them, so that every SIMD has four waves to take
+// turns.  Those eight hold half of N each (nh), exchange their halves of S^T C through LDS and finish two token tiles each.
+// 64 heads of [64, 128], in four waves / here (us): 4 sequences of 1,024 111 / 61 (y writes 67 MB and the rows read 50: 24), one of 2,000 203 / 99,
+// of 300 35 / 19, of 8 10.4 / 7.4, 64 of 8 133 / 95, 512 rows and 64 decode rows 189 / 126; 32 heads of [64, 64], 4 of 1,024 77 / 41.
+// Error against f64 as there: 0.9e-7.
+template <int NR>
+constexpr int ssm_pipe_lds() {
+  return 2 * 64 * (NR * 16 + 8) * 2 + 3 * 64 * 72 * 2 + 2 * (NR * 16 * 72 * 2 + 64 * 72 * 2 + 6 * 64 * 4) + 16 * 64 * 16;
+}
+
+template <int NR>
+__global__ __launch_bounds__(1024) void ssm_pipe_kernel(const bf16_t* __restrict__ xbc, long xs, const bf16_t* __restrict__ dtp, long dts,
+                                                        int heads, int P, int N, int groups, const float* __restrict__ dt_bias,
+                                                        const float* __restrict__ A_log, const float* __restrict__ Dp,
+                                                        float* __restrict__ state, const int* __restrict__ cu,
+                                                        const int* __restrict__ slots, const int* __restrict__ positions,
+                                                        float* __restrict__ y, long ys) {
+  constexpr int L = 64, NP = NR * 16, LN = NP + 8, LT = L + 8, BT = NP * LT, XT = 64 * LT, W = 6 * L, NH = NR / 2;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  bf16_t* const sB = reinterpret_cast<bf16_t*>(smem);  // [t][n]
+  bf16_t* const sC = sB + L * LN;                      // [t][n]
+  bf16_t* const sM = sC + L * LN;                      // [part][t][s]
+  bf16_t* const sBt0 = sM + 3 * L * LT;                // [chunk & 1][n][t]
+  bf16_t* const sXt0 = sBt0 + 2 * BT;                  // [chunk & 1][p][t]
+  floatx4* const sY = reinterpret_cast<floatx4*>(sXt0 + 2 * XT);   // [column tile][token tile][lane]: the other half's part of S^T C
+  float* const sw0 = reinterpret_cast<float*>(sY + 16 * 64);       // [chunk & 1][c, dt, 2^c, weight, c's low part, 2^c_L]
+  const int s = blockIdx.x, h = blockIdx.y, p0 = blockIdx.z * 64;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, g = lane >> 4;
+  const int w = wave & 3, half = (wave >> 2) & 1;
+  const bool files = wave >= 8;
+  const int row0 = cu[s], len = cu[s + 1] - row0, slot = slots[s];
+  if (len <= 0) return;
+  if (slot < 0) {
+    for (int i = threadIdx.x; i < len * 64; i += 1024)
+      if (p0 + (i & 63) < P) y[(long)(row0 + (i >> 6)) * ys + (long)h * P + p0 + (i & 63)] = 0.f;
+    return;
+  }
+  // a transposed row's groups of 8 tokens are turned by two in every second tile of 16 rows: 32 lanes file 8 rows four apart at 4 tokens each
+  auto at_t = [](int row, int t) { return row * LT + (((t >> 3) ^ ((row >> 3) & 2)) << 3) + (t & 7); };
+
+  if (files) {
+    const int inner = heads * P, grp = h / (heads / groups), q = wave - 8;
+    const bf16_t* const bx = xbc + (long)row0 * xs + (long)h * P + p0;
+    const bf16_t* const bb = xbc + (long)row0 * xs + inner + (long)grp * N;
+    const bf16_t* const bc = bb + (long)groups * N;
+    const double nA = -1.4426950408889634 * expf(A_log[h]);   // (decays as powers of two: in M one instruction where expf is 13)
+    const float db = dt_bias[h], Dh = Dp[h];
+    // what a thread files: B as 4 tokens x 4 columns (in both orders), x so too (the upper four waves), C in pieces of 16 bytes
+    constexpr int BN = NP / 32, NC = NP / 64;   // (waves across B's columns; pieces of C)
+    const bool hasb = q < 2 * BN, hasx = q >= 4;
+    const int bn = q % BN * 32 + (lane & 7) * 4, bt = q / BN % 2 * 32 + (lane >> 3) * 4;
+    const int xp = (q & 1) * 32 + (lane & 7) * 4, xt = (q >> 1 & 1) * 32 + (lane >> 3) * 4;
+    const bool vb = bn < N, vx = p0 + xp < P;
+    const int pt = threadIdx.x - 512, cn = pt % (NP / 8) * 8, ct = pt / (NP / 8);
+    constexpr int CR = 512 / (NP / 8);   // rows of C between a thread's pieces
+    const bool vc = cn < N;
+    short4_t fb[4], fx[4];
+    uint4_t fc[NC];
+    bf16_t fdt = 0;
+    // a chunk's rows, requested one chunk ahead (rows and columns that are not there: others again, and zeros when they are filed)
+    auto fetch = [&](int t0) {
+      const int last = min(len - t0, L) - 1;
+      if (q == 4) fdt = dtp[(long)(row0 + t0 + min(lane, last)) * dts + h];
+      const bf16_t *const cb = bb + (long)t0 * xs, *const cc = bc + (long)t0 * xs, *const cx = bx + (long)t0 * xs;
+      const unsigned st = (unsigned)xs;
+      if (hasb) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) fb[i] = *reinterpret_cast<const short4_t*>(cb + ((unsigned)min(bt + i, last) * st + (vb ? bn : 0)));
+      }
+      if (hasx) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) fx[i] = *reinterpret_cast<const short4_t*>(cx + ((unsigned)min(xt + i, last) * st + (vx ? xp : 0)));
+      }
+#pragma unroll
+      for (int k = 0; k < NC; ++k) fc[k] = *reinterpret_cast<const uint4_t*>(cc + ((unsigned)min(ct + k * CR, last) * st + (vc ? cn : 0)));
+    };
+    auto file = [&](int t0, int odd) {
+      const int tl = min(L, len - t0);
+      const short4_t z4 = {0, 0, 0, 0};
+      if (tl < L || N < NP || P - p0 < 64) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          fb[i] = (bt + i < tl && vb) ? fb[i] : z4;
+          fx[i] = (xt + i < tl && vx) ? fx[i] : z4;
+        }
+#pragma unroll
+        for (int k = 0; k < NC; ++k) fc[k] = (ct + k * CR < tl && vc) ? fc[k] : (uint4_t){0u, 0u, 0u, 0u};
+      }
+      if (hasb) {
+        bf16_t* const sBt = sBt0 + odd * BT;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          *reinterpret_cast<short4_t*>(sB + (bt + i) * LN + bn) = fb[i];
+          *reinterpret_cast<short4_t*>(sBt + at_t(bn + i, bt)) = (short4_t){fb[0][i], fb[1][i], fb[2][i], fb[3][i]};
+        }
+      }
+      if (hasx) {
+        bf16_t* const sXt = sXt0 + odd * XT;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) *reinterpret_cast<short4_t*>(sXt + at_t(xp + i, xt)) = (short4_t){fx[0][i], fx[1][i], fx[2][i], fx[3][i]};
+      }
+#pragma unroll
+      for (int k = 0; k < NC; ++k) *reinterpret_cast<uint4_t*>(sC + (ct + k * CR) * LN + cn) = fc[k];
+    };
+    // lane = token: c, the running sum of the log-decays (one wave, of the two that have no tile of M)
+    auto decays = [&](int t0, int odd) {
+      const int tl = min(L, len - t0);
+      float* const sw = sw0 + odd * W;
+      const float a = bf2f(fdt) + db;
+      const float dt = lane < tl ? (a > 20.f ? a : log1pf(expf(a))) : 0.f;
+      // (the sum over 64 tokens in f64 and as two floats: a difference of two of them keeps an f32's relative error, as the
+      // 16-token chunks' sums did)
+      double c = nA * dt;
+      c += dpp64<0x111, 0xf>(c);   // row_shr 1, 2, 4, 8: inside 16 lanes (by the LDS unit, 14 exchanges deep, it was a tenth of a chunk)
+      c += dpp64<0x112, 0xf>(c);
+      c += dpp64<0x114, 0xf>(c);
+      c += dpp64<0x118, 0xf>(c);
+      c += dpp64<0x142, 0xa>(c);   // row_bcast 15 to the second and fourth 16, 31 to the upper half
+      c += dpp64<0x143, 0xc>(c);
+      const int2 last = __builtin_bit_cast(int2, c);
+      const double cld = __builtin_bit_cast(double, make_int2(__builtin_amdgcn_readlane(last.x, 63), __builtin_amdgcn_readlane(last.y, 63)));
+      constexpr double kLn2 = 0.6931471805599453;
+      const float hi = (float)c;
+      sw[lane] = hi;
+      sw[L + lane] = dt;
+      sw[2 * L + lane] = exp_f64sum(c * kLn2);
+      sw[3 * L + lane] = exp_f64sum((cld - c) * kLn2) * dt;
+      sw[4 * L + lane] = (float)(c - hi);
+      sw[5 * L + lane] = exp_f64sum(cld * kLn2);
+    };
+    // M^T tiles: columns t of tile w, rows s of the half's two tiles (one tile of zeros completes a 32-step; the 32-steps behind t's are not read)
+    auto scores = [&](int odd) {
+      const float *const sc = sw0 + odd * W, *const sdt = sc + L, *const scl = sc + 4 * L;
+      const int t = 16 * w + r16;
+      const float ct = sc[t], ctl = scl[t];
+      floatx4 m[2], cs[2], cw[2], ds[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int o = 32 * half + 16 * u + 4 * g;
+        cs[u] = *reinterpret_cast<const floatx4*>(sc + o);
+        cw[u] = *reinterpret_cast<const floatx4*>(scl + o);
+        ds[u] = *reinterpret_cast<const floatx4*>(sdt + o);
+      }
+#pragma unroll
+      for (int kk = 0; kk < NR / 2; ++kk) {
+        const short8 cf = *reinterpret_cast<const short8*>(sC + t * LN + 32 * kk + 8 * g);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const short8 a = *reinterpret_cast<const short8*>(sB + (32 * half + 16 * u + r16) * LN + 32 * kk + 8 * g);
+          m[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, cf, kk == 0 ? floatx4{0.f, 0.f, 0.f, 0.f} : m[u], 0, 0, 0);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int st = 2 * half + u;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          float below = m[u][j] * (__builtin_amdgcn_exp2f((ct - cs[u][j]) + (ctl - cw[u][j])) * ds[u][j]);
+          if (st < w) {
+            m[u][j] = below;
+          } else {
+            const int sj = 16 * st + 4 * g + j;
+            asm volatile("" : "+v"(below));   // (side by side: a branch for each otherwise)
+            m[u][j] = sj < t ? below : (sj == t ? m[u][j] * ds[u][j] + Dh : 0.f);   // the skip D x on the diagonal
+          }
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          uint2 v;
+          v.x = pack_bf2(m[u][0], m[u][1]);
+          v.y = pack_bf2(m[u][2], m[u][3]);
+          *reinterpret_cast<uint2*>(sM + (k * L + t) * LT + 32 * half + 16 * u + 4 * g) = v;
+          m[u][0] -= __uint_as_float(v.x << 16);
+          m[u][1] -= __uint_as_float(v.x & 0xffff0000u);
+          m[u][2] -= __uint_as_float(v.y << 16);
+          m[u][3] -= __uint_as_float(v.y & 0xffff0000u);
+        }
+    };
+    fetch(0);
+    file(0, 0);
+    if (q == 4) decays(0, 0);
+    if (L < len) fetch(L);
+    __syncthreads();
+    int odd = 0;
+    for (int t0 = 0; t0 < len; t0 += L, odd ^= 1) {
+      if (!half || w >= 2) scores(odd);
+      else if (q == 4 && t0 + L < len) decays(t0 + L, odd ^ 1);
+      __syncthreads();  // M is complete; B and C by rows are read
+      if (t0 + L < len) {
+        file(t0 + L, odd ^ 1);
+        if (t0 + 2 * L < len) fetch(t0 + 2 * L);
+      }
+      __syncthreads();  // the next chunk is filed; M and this chunk's columns are read
+    }
+    return;
+  }
+
+  const int pcol = p0 + 16 * w + r16;
+  const bool pv = pcol < P, past = positions[row0] > 0;
+  float* const sp = state + (((long)slot * heads + h) * P + (pv ? pcol : 0)) * N;
+  floatx4 S[NH], ya[4];   // (rows 16 (NH half + j) + 4 g + ..)
+#pragma unroll
+  for (int j = 0; j < NH; ++j) {
+    const int n = (half * NH + j) * 16 + 4 * g;
+    S[j] = (past && pv && n < N) ? *reinterpret_cast<const floatx4*>(sp + n) : (floatx4){0.f, 0.f, 0.f, 0.f};
+  }
+  // y^T[p][t] from the state: 2^c_t S^T C over the half's rows; the token tiles that the other half finishes go to it
+  auto from_state = [&](int odd) {
+    const float* const sec = sw0 + odd * W + 2 * L;
+#pragma unroll
+    for (int tt = 0; tt < 4; ++tt) ya[tt] = (floatx4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kk = 0; kk < NH / 2; ++kk) {
+      float v[8];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        v[j] = S[2 * kk][j];
+        v[4 + j] = S[2 * kk + 1][j];
+      }
+      const BfParts b = bf_split3(v);
+      short8 c[4];
+#pragma unroll
+      for (int tt = 0; tt < 4; ++tt) {
+        const bf16_t* cp = sC + (16 * tt + r16) * LN + 32 * (half * (NH / 2) + kk) + 4 * g;
+        const short4_t lo = *reinterpret_cast<const short4_t*>(cp), hi = *reinterpret_cast<const short4_t*>(cp + 16);
+        c[tt] = (short8){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      }
+#pragma unroll
+      for (int k = 2; k >= 0; --k)
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) ya[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b.p[k], c[tt], ya[tt], 0, 0, 0);
+    }
+#pragma unroll
+    for (int tt = 0; tt < 4; ++tt) ya[tt] *= sec[16 * tt + r16];
+    sY[(w * 4 + 1 - half) * 64 + lane] = half ? ya[0] : ya[1];
+    sY[(w * 4 + 2 + half) * 64 + lane] = half ? ya[3] : ya[2];
+  };
+  // .. and from the chunk's own tokens, for tiles T0 and T1
+  auto finish = [&](int t0, int odd, bool both, auto T0, auto T1) {
+    const int tl = min(L, len - t0);
+    const bf16_t* const sXt = sXt0 + odd * XT;
+    constexpr int tts[2] = {decltype(T0)::value, decltype(T1)::value};
+    floatx4 a[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) a[i] = both ? ya[tts[i]] + sY[(w * 4 + tts[i]) * 64 + lane] : ya[tts[i]];
+    // (xe: without the second tile of a 32-step, whose M rows are zeros for an even token tile: an infinity or NaN among its x would
+    // reach outputs up to 31 tokens before it, not only those of its own 16 as in chunks of 16)
+    short8 xf[2], xe[2];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      xf[kk] = *reinterpret_cast<const short8*>(sXt + at_t(16 * w + r16, 32 * kk + 8 * g));
+      xe[kk] = g < 2 ? xf[kk] : (short8){0, 0, 0, 0, 0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int k = 2; k >= 0; --k)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          if (kk > tts[i] / 2) continue;
+          const short8 m = *reinterpret_cast<const short8*>(sM + (k * L + 16 * tts[i] + r16) * LT + 32 * kk + 8 * g);
+          a[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(2 * kk == tts[i] ? xe[kk] : xf[kk], m, a[i], 0, 0, 0);
+        }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int t = 16 * tts[i] + r16, p = p0 + 16 * w + 4 * g;
+      if (t < tl && p < P) *reinterpret_cast<floatx4*>(y + (long)(row0 + t0 + t) * ys + (long)h * P + p) = a[i];
+    }
+    // S' = 2^c_L S + B (w x)^T
+    const bf16_t* const sBt = sBt0 + odd * BT;
+    const float* const swv = sw0 + odd * W + 3 * L;
+    const float dec = swv[2 * L];
+#pragma unroll
+    for (int j = 0; j < NH; ++j) S[j] *= dec;
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      float v[8];
+      const floatx4 w0 = *reinterpret_cast<const floatx4*>(swv + 32 * kk + 8 * g), w1 = *reinterpret_cast<const floatx4*>(swv + 32 * kk + 8 * g + 4);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = bf2f((bf16_t)xf[kk][e]) * (e < 4 ? w0[e & 3] : w1[e & 3]);
+      const BfParts b = bf_split3(v);
+#pragma unroll
+      for (int k = 2; k >= 0; --k)
+#pragma unroll
+        for (int j = 0; j < NH; ++j) {
+          const short8 a = *reinterpret_cast<const short8*>(sBt + at_t(16 * (half * NH + j) + r16, 32 * kk + 8 * g));
+          S[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b.p[k], S[j], 0, 0, 0);
+        }
+    }
+  };
+  __syncthreads();
+  int odd = 0;
+  for (int t0 = 0; t0 < len; t0 += L, odd ^= 1) {
+    const bool both = past || t0 > 0;
+    if (both) from_state(odd);
+    else ya[0] = ya[1] = ya[2] = ya[3] = (floatx4){0.f, 0.f, 0.f, 0.f};
+    __syncthreads();
+    if (half == 0) finish(t0, odd, both, std::integral_constant<int, 0>{}, std::integral_constant<int, 3>{});
+    else finish(t0, odd, both, std::integral_constant<int, 1>{}, std::integral_constant<int, 2>{});
+    __syncthreads();
+  }
+  if (pv) {
+#pragma unroll
+    for (int j = 0; j < NH; ++j) {
+      const int n = (half * NH + j) * 16 + 4 * g;
+      if (n < N) *reinterpret_cast<floatx4*>(sp + n) = S[j];
+    }
+  }
+}
+
 // grid (row, norm group): out = (y * silu(z)) / sqrt(mean_group((y silu z)^2) + eps) * w
 template <typename T>
 __global__ __launch_bounds__(256) void gated_group_rmsnorm_kernel(const float* __restrict__ y, long ys,
@@ -1038,7 +1353,7 @@ __global__ __launch_bounds__(256) void gated_group_rmsnorm_wave_kernel(const flo
 
 // prompt portions (some sequence of the step has >= kChunkMin rows): the chunked MFMA kernel, for the step's other sequences too.  What
 // decides in short portions and decode rows is the pass over the state, so the 64-token chunks lead there as well; us, chunks of 16 ->
-// of 64, 64 heads of [64, 128]: 512 rows and 64 decode rows 322 -> 212, 8 and 64 177 -> 157, 64 portions of 8 170 -> 153, one of 8 14.4 -> 11.4.
+// of 64, 64 heads of [64, 128]: 512 rows and 64 decode rows 322 -> 126, 8 and 64 177 -> 102, 64 portions of 8 170 -> 95, one of 8 14.4 -> 7.4.
 // With up to 32 state columns that pass is short and a chunk's own work decides: there portions of up to 16 tokens stay with chunks of 16
 // (16 heads of [128, 16]: 32 portions of 16 10.3 against 15.0, 8 and 64 decode rows 17.4 / 24.8; 17 tokens 7.5 / 7.1).
 constexpr int kChunkMin = 8;
@@ -1052,18 +1367,25 @@ int scan_t(const T* xbc, long xs, const T* dtp, long dts, int S, int heads, int 
     if constexpr (sizeof(T) == 2) {
       // 16-byte loads of B, C and the state's rows, 8-byte ones of x, 16-byte stores of y
       const auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-      if (!(N <= 32 && max_len <= 16) && N % 8 == 0 && N <= 256 && P % 4 == 0 && ((long)heads * P) % 8 == 0 && xs % 8 == 0 && ys % 4 == 0 && a16(xbc) && a16(state) && a16(y)) {
+      if (!(N <= 32 && max_len <= 16) && N % 8 == 0 && N <= 256 && xs < (1L << 25) && P % 4 == 0 && ((long)heads * P) % 8 == 0 && xs % 8 == 0 && ys % 4 == 0 && a16(xbc) && a16(state) && a16(y)) {
 #define LK_CHUNK64(NR)                                                                                                             \
   do {                                                                                                                             \
     LK_SET_MAX_LDS((ssm_chunk_bf16_kernel<NR>), (ssm_chunk_lds<NR>()));                                                            \
     ssm_chunk_bf16_kernel<NR><<<cgrid, 256, ssm_chunk_lds<NR>(), st>>>(xbc, xs, dtp, dts, heads, P, N, groups, dt_bias, A_log, D,  \
                                                                       state, cu, slots, positions, y, ys);                        \
   } while (0)
+#define LK_PIPE(NR)                                                                                                            \
+  do {                                                                                                                         \
+    LK_SET_MAX_LDS((ssm_pipe_kernel<NR>), (ssm_pipe_lds<NR>()));                                                               \
+    ssm_pipe_kernel<NR><<<cgrid, 1024, ssm_pipe_lds<NR>(), st>>>(xbc, xs, dtp, dts, heads, P, N, groups, dt_bias, A_log, D,    \
+                                                                 state, cu, slots, positions, y, ys);                          \
+  } while (0)
         if (N <= 32) LK_CHUNK64(2);
-        else if (N <= 64) LK_CHUNK64(4);
-        else if (N <= 128) LK_CHUNK64(8);
-        else LK_CHUNK64(16);
+        else if (N <= 64) LK_PIPE(4);
+        else if (N <= 128) LK_PIPE(8);
+        else LK_CHUNK64(16);   // (two chunks' columns of 256 do not fit the LDS)
 #undef LK_CHUNK64
+#undef LK_PIPE
         LK_CHECK_LAUNCH();
         return 0;
       }

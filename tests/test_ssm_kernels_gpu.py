@@ -107,3 +107,13 @@ def test_step_whole_passes(hip, N, P, shift, dtype):
     y, ref, state, want = _run([1, 1, 2, 1], 4, P, N, 2, dtype, 1, 5, shift)
     assert (y.double() - ref).norm() <= 1e-6 * ref.norm()   # as above
     assert (state.double() - want).norm() <= 1e-6 * want.norm()
+
+
+@pytest.mark.parametrize("H,P,N,G", [(2, 64, 40, 1), (3, 20, 64, 3), (2, 72, 96, 1), (4, 128, 128, 2), (2, 4, 72, 2)])
+@pytest.mark.parametrize("lens", [[8, 1], [63, 64, 65], [16, 17, 32, 33, 48, 49], [127, 128, 129, 192], [1000, 2]])
+@pytest.mark.parametrize("later", [0, 5])
+def test_chunk_pipeline(hip, H, P, N, G, lens, later):
+    """Chunks of 64 tokens behind each other at the edges of their token tiles, states that fill their tiles and not, with and without one before."""
+    y, ref, state, want = _run(lens, H, P, N, G, torch.bfloat16, max(lens), later)
+    assert (y.double() - ref).norm() <= 1e-6 * ref.norm()   # as above
+    assert (state.double() - want).norm() <= 1e-6 * want.norm()
