@@ -212,6 +212,12 @@ def prefill_tiles(q_lens: Sequence[int], ctx_lens: Sequence[int], G: int, causal
     return (np.asarray(seqs, dtype=np.int32)[order], np.asarray(q0s, dtype=np.int32)[order])
 
 
+def device_tiles(q_lens: Sequence[int], ctx_lens: Sequence[int], G: int, causal: bool, D: int, device):
+    """:func:`prefill_tiles` on the device, in one copy: what a forward pass hands to all of its layers."""
+    both = torch.from_numpy(np.stack(prefill_tiles(q_lens, ctx_lens, G, causal, D))).to(device, non_blocking=True)
+    return both[0], both[1]
+
+
 def flash_prefill(q, k, v, cu_q, Hq: int, Hkv: int, D: int, scale: float, causal: bool,
                   block_tables=None, ctx_lens=None, q_lens_cpu=None, ctx_lens_cpu=None,
                   tiles=None, out=None, part=None, q_past=None):
@@ -237,9 +243,7 @@ def flash_prefill(q, k, v, cu_q, Hq: int, Hkv: int, D: int, scale: float, causal
                 need = max((int(c) + BS - 1) // BS for c in ctx_lens_cpu) if ctx_lens_cpu else 0
                 if need > block_tables.shape[1]:
                     raise ValueError("block table too narrow for the context lengths")
-            ts, tq = prefill_tiles(q_lens_cpu, ctx_lens_cpu, Hq // Hkv, causal, D)
-            tiles = (torch.from_numpy(ts).to(q.device, non_blocking=True),
-                     torch.from_numpy(tq).to(q.device, non_blocking=True))
+            tiles = device_tiles(q_lens_cpu, ctx_lens_cpu, Hq // Hkv, causal, D, q.device)
         pp_o, pp_ml = part if part is not None else (None, None)
         if out is not None and part is None and (out.data_ptr() % 16 or out.stride(0) % 8):
             # the kernel's output rows leave as 16-byte stores: stage a misaligned view
