@@ -73,6 +73,7 @@ struct PrefillParams {
   // negative or past the keys: this rank holds only a shard of the keys); null = ctx - q_len
   const int* q_past;
   int xcd;  // XCD-aware workgroup order (prefill_xcd())
+  int pairs, ntiles;  // the encoder's order on a one-dimensional grid
   int btv;  // block-table entries preloaded per lane (LK_PREFILL_BTV, default 1)
 };
 
@@ -102,7 +103,19 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void flash_prefill_kernel(PrefillP
   // each XCD takes its tiles heaviest first (LK_PREFILL_XCD=0: the plain order)
   const int nx = gridDim.x;
   const int lin = p.xcd ? xcd_remap(blockIdx.y * nx + blockIdx.x, nx * gridDim.y) : blockIdx.y * nx + blockIdx.x;
-  const int bx = lin % nx, by = lin / nx;
+  int bx = lin % nx, by = lin / nx;
+  if constexpr (!PAGED && !CAUSAL) {
+    if (p.pairs) {
+      // an encoder's rows hold all heads side by side: an XCD takes two tiles (most sequences are one or two) with all of their heads behind
+      // each other, so that the 128-byte pieces of a row are read close together and a sequence's second tile finds its keys in that L2.
+      // 543 sequences of 20 - 224, 12 heads of 64: 125 -> 117 us; heads of 32 78 -> 66; 128 of 400 - 512 156 -> 151.  A head's tiles
+      // one after the other, or one tile or four at a time, were 1 - 6 us slower in one or another.
+      const int ny = p.Hq / WH, at = blockIdx.x >> 3;
+      bx = ((at / (2 * ny)) * 8 + (blockIdx.x & 7)) * 2 + at % (2 * ny) / ny;
+      by = at % ny;
+      if (bx >= p.ntiles) return;
+    }
+  }
   const int head = by * WH + (w % WH);
   const int kvh = head / G;
   const int rg = w / WH;
@@ -531,7 +544,7 @@ int lk_flash_prefill(const bf16_t* q, long qs, const bf16_t* k, const bf16_t* v,
   while ((1 << bs_shift) < BS) ++bs_shift;
   PrefillParams pr{q, qs, k, v, ks, vs, block_tables, bt_stride, cu_q, ctx_lens, tile_seq,
                    tile_q0, out, os, Hq, Hkv, BS, bs_shift, scale * 1.4426950408889634f, part_o, part_ml,
-                   part_o ? 0.f : prefill_defer(), q_past, 0, prefill_btv()};
+                   part_o ? 0.f : prefill_defer(), q_past, 0, 0, ntiles, prefill_btv()};
   const int WH = G >= 4 ? 4 : G;
   const int NW = prefill_waves(G, D);
   dim3 grid(ntiles, Hq / WH);
@@ -539,6 +552,11 @@ int lk_flash_prefill(const bf16_t* q, long qs, const bf16_t* k, const bf16_t* v,
   // 930 keys: 69.5 / 68.4 vs 75.5 / 76.1 us); the long-prefill grids of 8192 workgroups run
   // 2-6 % faster in the plain order (profiles/r5_flash_xcd/)
   pr.xcd = prefill_xcd() && (long)ntiles * (Hq / WH) <= 2048;
+  const long paired = (long)(ntiles + 15) / 16 * 16 * (Hq / WH);
+  if (!paged && !causal && prefill_xcd() && !pr.xcd && paired < (1L << 31)) {
+    pr.pairs = 1;
+    grid = dim3((unsigned)paired);
+  }
   const bool pipe = causal && prefill_pipe();
 #define L(DD, C, PG, W, N)                                                        \
   if (pipe) flash_prefill_kernel<DD, C, PG, W, N, true><<<grid, 64 * N, 0, st>>>(pr); \
