@@ -81,8 +81,12 @@ __global__ __launch_bounds__(256) void stream_rmsnorm_kernel(float* __restrict__
   }
 }
 
-// The same with the row kept in registers and 16-byte (f32) / 8-byte (bf16) accesses: W % 4 == 0,
-// W <= 4 * 256 * MAXV, 16-byte aligned rows.  One read of every input, one write of x and of out.
+// The same with the row kept in registers and 16-byte (f32) / 8-byte (bf16) accesses: W % 4 == 0, W <= 4 * 256 * MAXV, 16-byte
+// aligned rows.  One read of every input, one write of x and of out.  A row is short, so what it costs is the trips to memory: every
+// input and the weight are requested before anything waits (columns past the row are its last again, and not used), in registers for
+// rows of up to 1,024, 2,048, 4,096 or 8,192 (with eight
+// pieces and a test for each, one after the other, whatever the width: 4,095 x 2,048 with a 20.4 -> 16.0 us, with b too 23.8 -> 18.4;
+// x 4,096 33.0 -> 29.7, x 768 11.8 -> 7.1; 949 x 2,048 6.7 -> 5.1; 117 and 134 MB at 4,095 x 2,048).
 template <typename T, int MAXV>
 __global__ __launch_bounds__(256) void stream_rmsnorm_vec_kernel(float* __restrict__ x, const T* __restrict__ a, long as,
                                                                  const float* __restrict__ ab, const T* __restrict__ b,
@@ -91,33 +95,41 @@ __global__ __launch_bounds__(256) void stream_rmsnorm_vec_kernel(float* __restri
                                                                  const float* __restrict__ w, float woff, float eps,
                                                                  const long* __restrict__ idx, T* __restrict__ out,
                                                                  long os, int W) {
+  using Raw = std::conditional_t<sizeof(T) == 2, short4_t, floatx4>;
   __shared__ float red[4];
   const long orow = blockIdx.x, row = idx ? idx[orow] : orow;
   const int nv = W >> 2;
-  floatx4 v[MAXV];
-  float ss = 0.f;
-  auto ld4 = [](const T* p) -> floatx4 {
-    if constexpr (sizeof(T) == 2) {
-      const short4_t r = *reinterpret_cast<const short4_t*>(p);
-      return floatx4{bf2f((bf16_t)r[0]), bf2f((bf16_t)r[1]), bf2f((bf16_t)r[2]), bf2f((bf16_t)r[3])};
-    } else {
-      return *reinterpret_cast<const floatx4*>(p);
-    }
+  floatx4 v[MAXV], g[MAXV], ev[MAXV], abv[MAXV];
+  Raw ra[MAXV], rb[MAXV];
+  auto wide = [](Raw r) -> floatx4 {
+    if constexpr (sizeof(T) == 2) return floatx4{bf2f((bf16_t)r[0]), bf2f((bf16_t)r[1]), bf2f((bf16_t)r[2]), bf2f((bf16_t)r[3])};
+    else return r;
   };
+  auto get = [&](auto (&to)[MAXV], auto* from) {
+#pragma unroll
+    for (int i = 0; i < MAXV; ++i) to[i] = *reinterpret_cast<const std::remove_reference_t<decltype(to[0])>*>(from + 4 * min((int)threadIdx.x + 256 * i, nv - 1));
+  };
+  get(v, x + row * W);
+  if (a) get(ra, a + row * as);
+  if (b) get(rb, b + row * bs);
+  constexpr bool kAll = MAXV <= 4;   // (more registers than the waves behind each other can spare otherwise)
+  if (kAll && e) get(ev, e + row * W);
+  if (kAll && a && ab) get(abv, ab);
+  if (kAll && w) get(g, w);
+  float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < MAXV; ++i) {
     const int c = threadIdx.x + 256 * i;
+    floatx4 d = {0.f, 0.f, 0.f, 0.f};
+    const int cc = 4 * min(c, nv - 1);
+    if (a) d += wide(ra[i]);
+    if (a && ab) d += kAll ? abv[i] : *reinterpret_cast<const floatx4*>(ab + cc);
+    if (b) d += wide(rb[i]);
+    v[i] += m * d;
+    if (e) v[i] += kAll ? ev[i] : *reinterpret_cast<const floatx4*>(e + row * W + cc);
     if (c < nv) {
-      floatx4 t = *reinterpret_cast<const floatx4*>(x + row * W + 4 * c);
-      floatx4 d = {0.f, 0.f, 0.f, 0.f};
-      if (a) d += ld4(a + row * as + 4 * c);
-      if (a && ab) d += *reinterpret_cast<const floatx4*>(ab + 4 * c);
-      if (b) d += ld4(b + row * bs + 4 * c);
-      t += m * d;
-      if (e) t += *reinterpret_cast<const floatx4*>(e + row * W + 4 * c);
-      if (!idx && (a || b || e)) *reinterpret_cast<floatx4*>(x + row * W + 4 * c) = t;
-      v[i] = t;
-      ss += t[0] * t[0] + t[1] * t[1] + t[2] * t[2] + t[3] * t[3];
+      if (!idx && (a || b || e)) *reinterpret_cast<floatx4*>(x + row * W + 4 * c) = v[i];
+      ss += v[i][0] * v[i][0] + v[i][1] * v[i][1] + v[i][2] * v[i][2] + v[i][3] * v[i][3];
     }
   }
   ss = block_sum<4>(ss, red);
@@ -126,9 +138,9 @@ __global__ __launch_bounds__(256) void stream_rmsnorm_vec_kernel(float* __restri
   for (int i = 0; i < MAXV; ++i) {
     const int c = threadIdx.x + 256 * i;
     if (c < nv) {
-      floatx4 g = {1.f, 1.f, 1.f, 1.f};
-      if (w) g = *reinterpret_cast<const floatx4*>(w + 4 * c) + woff;
-      const floatx4 r = v[i] * inv * g;
+      floatx4 gi = {1.f, 1.f, 1.f, 1.f};
+      if (w) gi = (kAll ? g[i] : *reinterpret_cast<const floatx4*>(w + 4 * c)) + woff;
+      const floatx4 r = v[i] * inv * gi;
       T* o = out + orow * os + 4 * c;
       if constexpr (sizeof(T) == 2) {
         short4_t q = {(short)f2bf(r[0]), (short)f2bf(r[1]), (short)f2bf(r[2]), (short)f2bf(r[3])};
@@ -253,12 +265,20 @@ int lk_stream_rmsnorm(float* x, const void* a, long as, const float* a_bias, con
   const int tv = esz == 2 ? 8 : 16;  // bytes of a 4-element access to the activations
   if (W % 4 == 0 && W <= 4 * 256 * kMaxV && al(x, (long)W * 4, 16) && al(e, (long)W * 4, 16) && al(w, 0, 16) && al(a_bias, 0, 16) &&
       al(a, as * (long)esz, tv) && al(b, bs * (long)esz, tv) && al(out, os * (long)esz, tv)) {
-    if (esz == 2)
-      stream_rmsnorm_vec_kernel<bf16_t, kMaxV><<<(unsigned)out_rows, 256, 0, st>>>(
-          x, (const bf16_t*)a, as, a_bias, (const bf16_t*)b, bs, e, m, w, woff, eps, idx, (bf16_t*)out, os, W);
-    else
-      stream_rmsnorm_vec_kernel<float, kMaxV><<<(unsigned)out_rows, 256, 0, st>>>(
-          x, (const float*)a, as, a_bias, (const float*)b, bs, e, m, w, woff, eps, idx, (float*)out, os, W);
+#define LK_VEC(T, V)                                                                                                                  \
+  stream_rmsnorm_vec_kernel<T, V><<<(unsigned)out_rows, 256, 0, st>>>(x, (const T*)a, as, a_bias, (const T*)b, bs, e, m, w, woff, eps, \
+                                                                      idx, (T*)out, os, W)
+#define LK_VECS(T)                      \
+  do {                                  \
+    if (W <= 1024) LK_VEC(T, 1);        \
+    else if (W <= 2048) LK_VEC(T, 2);   \
+    else if (W <= 4096) LK_VEC(T, 4);   \
+    else LK_VEC(T, kMaxV);              \
+  } while (0)
+    if (esz == 2) LK_VECS(bf16_t);
+    else LK_VECS(float);
+#undef LK_VECS
+#undef LK_VEC
     LK_CHECK_LAUNCH();
     return 0;
   }

@@ -339,3 +339,22 @@ def test_mamba2_slot_reuse_and_long_memory(device, dtype):
     other[0] = -other[0]
     seen = rel_err(oracle_mamba(spec, w, other)[200], want[200])
     assert seen > 5 * tol(dtype), seen   # the last row still depends on token 0: the comparison above sees a lost state
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("W", [4, 1020, 1024, 1028, 2048, 2052, 4096, 4100, 8192])
+def test_stream_norm_row_lengths(hip, W):
+    """Rows at the edges of what one, two, four and eight pieces per thread hold, with every input and with one."""
+    g = torch.Generator().manual_seed(W)
+    T, eps, m = 5, 1e-5, 0.37
+    x, e, w, ab = (rnd(g, *s).float() for s in ((T, W), (T, W), (W,), (W,)))
+    a, b = q16(rnd(g, T, W)), q16(rnd(g, T, W))
+    d = lambda t: t.cuda()
+    dt = torch.bfloat16 if W % 8 == 0 else torch.float32
+    for full in (True, False):
+        want = x.double() + m * (a.double() + (ab.double() + b.double() if full else 0)) + (e.double() if full else 0)
+        xd = d(x.clone())
+        h = ops.stream_rmsnorm(xd, d(a.to(dt)), d(b.to(dt)) if full else None, d(e) if full else None, m, d(w), 1.0, eps,
+                               a_bias=d(ab) if full else None, out_dtype=dt)
+        assert rel_err(xd, want) < 1e-6   # (four f32 roundings)
+        assert rel_err(h, O.offset_rmsnorm(want, w, eps)) < (1e-2 if dt == torch.bfloat16 else 3e-6)
