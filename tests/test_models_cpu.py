@@ -421,6 +421,19 @@ def test_tile_rule_takes_what_measured_fastest(monkeypatch, M, N, K, epi, pick):
     assert ops._tile_rule(M, N, K, epi) == (ops._gemm_default(M, N, K, epi) if pick is None else (pick, 256, 1))
 
 
+@pytest.mark.parametrize("M,N,cfg,pick", [
+    (257, 28672, (3, 256, 1), 4), (384, 28672, (3, 256, 1), 4), (385, 28672, (3, 256, 1), 3), (512, 28672, (3, 256, 1), 3), (1100, 28672, (3, 256, 1), 4),
+    (1153, 28672, (3, 256, 1), 3), (256, 28672, (3, 256, 1), 3), (4609, 28672, (3, 256, 1), 3), (1153, 28672, (4, 256, 1), 3), (2600, 4096, (4, 256, 1), 4)])
+def test_bucket_rule_takes_the_other_tile_below_a_buckets_top(monkeypatch, M, N, cfg, pick):
+    """Measured tiles of 256 and 192 rows inside their bucket; other variants and splits are left as they were measured."""
+    from llm_kubernetes_minikube_sharp4dev_amd import ops
+
+    monkeypatch.setattr(ops, "_CUS", 256)
+    assert ops._bucket_rule(M, N, cfg) == (pick, 256, 1)
+    for kept in ((5, 256, 1), (2, 256, 4), (6, 256, 1), (3, 256, 2), (0, 192, 1)):
+        assert ops._bucket_rule(M, N, kept) == kept
+
+
 @pytest.mark.parametrize("M,N,K,epi,cfg,pick", [
     (300, 4096, 4096, 0, (2, 256, 4), (5, 256, 4)), (1152, 4096, 4096, 0, (5, 256, 1), (5, 256, 1)), (1536, 4096, 14336, 0, (2, 256, 2), (4, 256, 2)),
     (300, 2048, 5632, 0, (2, 256, 4), (5, 256, 8)), (3072, 2048, 5632, 0, (2, 256, 2), (5, 256, 1)), (512, 2048, 2048, 0, (5, 256, 1), (5, 256, 4)),
