@@ -1326,7 +1326,7 @@ def _cfg_of(M: int, N: int, K: int, epi: int):
             cfg = None
         elif cfg is not None and not SPLIT_ON and cfg[0] in GEMM1W_SPLIT:
             cfg = (3, 256, 1)
-    return _bucket_rule(M, N, cfg) if cfg is not None else _rounds_rule(M, N, K, epi) or _tile_rule(M, N, K, epi)
+    return _fill_rule(M, N, epi, cfg if cfg is not None else _rounds_rule(M, N, K, epi) or _tile_rule(M, N, K, epi))
 
 
 # Shapes without a measured entry, more than 256 rows: gemm1w.hip's 128 / 192 / 256-row tiles against the fallback.  Its
@@ -1411,23 +1411,36 @@ def _rounds_cost(M: int, N: int, bm: int) -> float:
     return whole * (a + b) + (a + b * part / cus if part else 0.0)
 
 
-_BUCKET_RULE: dict = {}
+_FILL_RULE: dict = {}
 
 
-def _bucket_rule(M: int, N: int, cfg):
-    """A measured pick of 256 or 192-row tiles at this number of rows: it was measured at the top of a bucket of 256, and further down the other one
-    may fill the rows or the rounds better.  The other where its rounds cost 5 % less.  28,672 x 4,096 with SwiGLU: 300 rows 84.2 -> 73.5 us (two
-    tiles of either, 192 rows each), 384 89.0 -> 79.2; 57,344 x 8,192 300 rows 317 -> 270.  Of 352 products (16 measured shapes, 257 - 4,300 rows) it
-    changes 10, by 0.85 on average, and makes none slower."""
-    if cfg[0] not in (3, 4) or cfg[2] != 1 or not 256 < M <= 4608:
+def _fill_cost(M: int, N: int, epi: int, v: int) -> float:
+    """``_rounds_cost`` of a variant; of a column split the sum of its two launches, of which a short last round costs up to 0.3 more."""
+    cus = device_cus()
+    if v not in GEMM1W_SPLIT:
+        return _rounds_cost(M, N, GEMM1W_BM[v])
+    cols, bm = gemm1w_split_cols(M, N, epi, cus), GEMM1W_SPLIT[v]
+    last = -(-M // bm) * (N // 256 - cols) % cus
+    return _rounds_cost(M, cols * 256, 256) + _rounds_cost(M, N - cols * 256, bm) + (0.3 * (1 - last / cus) if last else 0.0)
+
+
+def _fill_rule(M: int, N: int, epi: int, cfg):
+    """A pick of 256 or 192-row tiles or of a column split, at this very number of rows: a table's entry was measured at the top of a bucket of
+    256, and the rules above know no column split.  Another of the four where its rounds over the CUs cost 2.5 % less.  28,672 x 4,096 with SwiGLU:
+    300 rows 84.2 -> 73.5 us (two tiles of either, 192 rows each), 949 rows 177.6 -> 167.0 (64 columns of 256 rows, the rest in 192), 1,100 rows
+    234 -> 206; 10,496 x 2,048 at 4,095 rows 142.7 -> 135.4 (32 columns, the rest in 192); 14,336 x 4,096 at 2,589 248 -> 228.  Of 587 products (22
+    shapes, 257 - 4,500 rows) it changes 34, by 0.92 on average, and makes none slower."""
+    if cfg is None or cfg[0] not in (3, 4, 6, 7) or cfg[2] != 1 or not 256 < M <= 4608 or not GEMM1W or N % 256:
         return cfg
-    key = (M, N, cfg[0], device_cus())
-    if key not in _BUCKET_RULE:
-        if len(_BUCKET_RULE) > 4096:
-            _BUCKET_RULE.clear()
-        other = 7 - cfg[0]
-        _BUCKET_RULE[key] = (other, 256, 1) if _rounds_cost(M, N, GEMM1W_BM[other]) < 0.95 * _rounds_cost(M, N, GEMM1W_BM[cfg[0]]) else cfg
-    return _BUCKET_RULE[key]
+    key = (M, N, epi, cfg[0], device_cus(), SPLIT_ON)
+    if key not in _FILL_RULE:
+        forms = (3, 4, 6, 7) if SPLIT_ON and _split_applies(M, N, epi) else (3, 4)
+        costs = {v: _fill_cost(M, N, epi, v) for v in forms}
+        best = min(costs, key=costs.get)
+        if len(_FILL_RULE) > 4096:
+            _FILL_RULE.clear()
+        _FILL_RULE[key] = (best, 256, 1) if costs[best] < 0.975 * costs.get(cfg[0], costs[3]) else cfg   # (a split that does not apply runs as 3)
+    return _FILL_RULE[key]
 
 
 def _rounds_rule(M: int, N: int, K: int, epi: int):

@@ -422,16 +422,20 @@ def test_tile_rule_takes_what_measured_fastest(monkeypatch, M, N, K, epi, pick):
 
 
 @pytest.mark.parametrize("M,N,cfg,pick", [
-    (257, 28672, (3, 256, 1), 4), (384, 28672, (3, 256, 1), 4), (385, 28672, (3, 256, 1), 3), (512, 28672, (3, 256, 1), 3), (1100, 28672, (3, 256, 1), 4),
-    (1153, 28672, (3, 256, 1), 3), (256, 28672, (3, 256, 1), 3), (4609, 28672, (3, 256, 1), 3), (1153, 28672, (4, 256, 1), 3), (2600, 4096, (4, 256, 1), 4)])
-def test_bucket_rule_takes_the_other_tile_below_a_buckets_top(monkeypatch, M, N, cfg, pick):
-    """Measured tiles of 256 and 192 rows inside their bucket; other variants and splits are left as they were measured."""
+    (257, 28672, 3, 4), (384, 28672, 3, 4), (385, 28672, 3, 3), (512, 28672, 3, 3), (949, 28672, 3, 7), (961, 28672, 3, 3), (1100, 28672, 6, 4),
+    (1100, 28672, 3, 4), (1194, 28672, 6, 6), (256, 28672, 3, 3), (4609, 28672, 3, 3), (4095, 10496, 3, 7), (2589, 14336, 3, 6), (2600, 4096, 4, 4),
+    (300, 2048, 3, 4)])
+def test_fill_rule_takes_what_measured_fastest(monkeypatch, M, N, cfg, pick):
+    """Tiles of 256 and 192 rows and column splits by the rounds of this number of rows; other variants and ranges of K are left."""
     from llm_kubernetes_minikube_sharp4dev_amd import ops
 
-    monkeypatch.setattr(ops, "_CUS", 256)
-    assert ops._bucket_rule(M, N, cfg) == (pick, 256, 1)
-    for kept in ((5, 256, 1), (2, 256, 4), (6, 256, 1), (3, 256, 2), (0, 192, 1)):
-        assert ops._bucket_rule(M, N, kept) == kept
+    for name, value in (("GEMM1W", True), ("SPLIT_ON", True), ("_CUS", 256)):
+        monkeypatch.setattr(ops, name, value)
+    assert ops._fill_rule(M, N, 1, (cfg, 256, 1)) == (pick, 256, 1)
+    for kept in ((5, 256, 1), (2, 256, 4), (3, 256, 2), (0, 192, 1), None):
+        assert ops._fill_rule(M, N, 1, kept) == kept
+    monkeypatch.setattr(ops, "SPLIT_ON", False)
+    assert ops._fill_rule(M, N, 1, (3, 256, 1))[0] in (3, 4)
 
 
 @pytest.mark.parametrize("M,N,K,epi,cfg,pick", [
