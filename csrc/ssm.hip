@@ -32,7 +32,7 @@ template <>
 LK_DEVICE void stf<float>(float* p, float v) { *p = v; }
 
 constexpr int kMaxTaps = 8;
-constexpr int kConvRows = 16;  // tokens per workgroup of the convolution
+constexpr int kConvRows = 16;  // tokens per workgroup of the convolution (at most)
 
 template <bool EXACT>
 LK_DEVICE float silu_f(float x) {
@@ -1461,9 +1461,12 @@ int lk_conv_silu(const void* u, long us, int C, int taps, const float* w, const 
   const auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
   if (taps <= 4 && C % ev == 0 && us % ev == 0 && os % ev == 0 && a16(u) && a16(out) && a16(state)) {
     const int cblocks = (C / ev + 255) / 256;
-    // tokens per workgroup (a kernel argument: tiles of 4 tokens were tried for steps of few, long sequences, where 16-token
-    // tiles leave a chip of 256 CUs a handful of waves each, and measured slower: 79 us against 61 us at 4 x 1,024 x 2,048)
-    const int rows = kConvRows;
+    // tokens per workgroup, which walks them in fours behind each other: 4 or 8 where that leaves about a workgroup or two to a CU, 16 where
+    // shorter tiles would not all be on the chip at once.  bf16 x 6,144 channels, 4 / 8 / 16 tokens (us, with the state's launch): one sequence of
+    // 60 7.8 / 9.0 / 11.8, of 300 8.9 / 9.6 / 12.2, of 900 16.5 / 14.5 / 14.2, of 2,000 30 / 22.0 / 21.2, four of 1,024 45 / 37 / 28.9; x 2,048
+    // 18.8 / 16.2 / 17.6, x 512 8.2 / 8.7 / 11.0
+    const auto groups = [&](int r) { return (long)S * cblocks * ((max_len + r - 1) / r); };
+    const int rows = groups(4) <= 300 ? 4 : groups(8) <= 600 ? 8 : kConvRows;
     const bool one = max_len == 1;
     dim3 gv(S, (max_len + rows - 1) / rows, cblocks);
     if (esz == 2)

@@ -117,3 +117,30 @@ def test_chunk_pipeline(hip, H, P, N, G, lens, later):
     y, ref, state, want = _run(lens, H, P, N, G, torch.bfloat16, max(lens), later)
     assert (y.double() - ref).norm() <= 1e-6 * ref.norm()   # as above
     assert (state.double() - want).norm() <= 1e-6 * want.norm()
+
+
+# (tiles of 4, 8 and 16 tokens at and past their edges, sequences shorter than one, a step of mixed lengths)
+@pytest.mark.parametrize("lens,C", [([1, 3, 4, 5], 2048), ([300], 6144), ([601], 6144), ([803, 7, 8, 9], 2048), ([1600, 15, 16, 17, 1], 6144)])
+@pytest.mark.parametrize("later", [0, 5])
+def test_conv_tiles(hip, lens, C, later):
+    g = torch.Generator(device=DEV).manual_seed(C + lens[0])
+    T, S, taps = sum(lens), len(lens), 4
+    u = torch.randn(T, C + 64, device=DEV, generator=g).bfloat16()
+    w, b = torch.randn(C, taps, device=DEV, generator=g), torch.randn(C, device=DEV, generator=g)
+    state = torch.randn(S + 1, taps - 1, C, device=DEV, generator=g).bfloat16()
+    cu = torch.tensor([sum(lens[:i]) for i in range(S + 1)], dtype=torch.int32, device=DEV)
+    slots = torch.arange(S, 0, -1, device=DEV).to(torch.int32)
+    pos = torch.cat([torch.arange(n) + later for n in lens]).to(torch.int32).to(DEV)
+    before = state.clone()
+    y = hip.conv_silu(u, 64, C, w, b, state, cu, slots, pos, max(lens), True).double()
+    for s, n in enumerate(lens):
+        x = u[int(cu[s]):int(cu[s + 1]), 64:]
+        x = torch.cat([before[S - s] if later else torch.zeros_like(before[S - s]), x])
+        a = sum(x[k:k + n].double() * w[:, k].double() for k in range(taps)) + b.double()
+        size = sum(x[k:k + n].double().abs() * w[:, k].double().abs() for k in range(taps)) + b.double().abs()
+        want = a * torch.sigmoid(a)
+        # bf16 rounding; the sum's five f32 roundings (SiLU's slope is below 1.1); SiLU's own exponential and division, a few 2^-24 of its argument
+        bound = 2.0 ** -8 * want.abs() + 1.1 * 5 * 2.0 ** -24 * size + 2.0 ** -19 * a.abs() + 2.0 ** -30
+        assert bool(((y[int(cu[s]):int(cu[s + 1])] - want).abs() <= bound * (1 + 2.0 ** -8)).all())
+        assert torch.equal(state[S - s], x[-(taps - 1):])
+    assert torch.equal(state[0], before[0])
