@@ -1381,25 +1381,32 @@ def _tiled_cost(M: int, N: int, K: int, epi: int) -> Optional[float]:
     return cost(cfg[0]) if cfg is not None and cfg != d and cfg[0] in _TILE_COST else other
 
 
+def _remember(table: dict, key, value):
+    """table[key] = value in a table of bounded size, and the value back: a caller never reads the table again, which another thread may empty."""
+    if len(table) > 4096:
+        table.clear()
+    table[key] = value
+    return value
+
+
 def _tile_rule(M: int, N: int, K: int, epi: int):
     d = _gemm_default(M, N, K, epi)
     # (past the rows it was fitted on a launch is several waves, whose stores overlap and which this cost does not describe: _rounds_rule)
     if not GEMM1W or not 256 < M <= 4608 or epi > 4 or K // 64 < 3 or N % 256 or d is None:
         return d
     key = (M, N, K, epi, d)
-    if key not in _TILE_RULE:
-        cost, other = _tile_times(M, N, K, epi, d)
-        best = min(_TILE_COST, key=cost)
-        if len(_TILE_RULE) > 4096:
-            _TILE_RULE.clear()
-        # (the pick has to be clear where the estimates are least sure: between two of these tiles 3 % of them, at K up to 1,024 7 %, and
-        # against split-K 20 % from K 5,632 on, where 100 - 200 tiles of deep K run up to a quarter longer than estimated)
-        if d[0] in _TILE_COST:
-            clear = 0.93 if K <= 1024 else 0.97
-        else:
-            clear = 0.8 if d[2] > 1 and K >= 5632 else 1.0
-        _TILE_RULE[key] = (best, 256, 1) if cost(best) < clear * other else d
-    return _TILE_RULE[key]
+    pick = _TILE_RULE.get(key)
+    if pick is not None:
+        return pick
+    cost, other = _tile_times(M, N, K, epi, d)
+    best = min(_TILE_COST, key=cost)
+    # (the pick has to be clear where the estimates are least sure: between two of these tiles 3 % of them, at K up to 1,024 7 %, and
+    # against split-K 20 % from K 5,632 on, where 100 - 200 tiles of deep K run up to a quarter longer than estimated)
+    if d[0] in _TILE_COST:
+        clear = 0.93 if K <= 1024 else 0.97
+    else:
+        clear = 0.8 if d[2] > 1 and K >= 5632 else 1.0
+    return _remember(_TILE_RULE, key, (best, 256, 1) if cost(best) < clear * other else d)
 
 
 def _rounds_cost(M: int, N: int, bm: int) -> float:
@@ -1433,14 +1440,14 @@ def _fill_rule(M: int, N: int, epi: int, cfg):
     if cfg is None or cfg[0] not in (3, 4, 6, 7) or cfg[2] != 1 or not 256 < M <= 4608 or not GEMM1W or N % 256:
         return cfg
     key = (M, N, epi, cfg[0], device_cus(), SPLIT_ON)
-    if key not in _FILL_RULE:
-        forms = (3, 4, 6, 7) if SPLIT_ON and _split_applies(M, N, epi) else (3, 4)
-        costs = {v: _fill_cost(M, N, epi, v) for v in forms}
-        best = min(costs, key=costs.get)
-        if len(_FILL_RULE) > 4096:
-            _FILL_RULE.clear()
-        _FILL_RULE[key] = (best, 256, 1) if costs[best] < 0.975 * costs.get(cfg[0], costs[3]) else cfg   # (a split that does not apply runs as 3)
-    return _FILL_RULE[key]
+    pick = _FILL_RULE.get(key)
+    if pick is not None:
+        return pick
+    forms = (3, 4, 6, 7) if SPLIT_ON and _split_applies(M, N, epi) else (3, 4)
+    costs = {v: _fill_cost(M, N, epi, v) for v in forms}
+    best = min(costs, key=costs.get)
+    # (a split that does not apply runs as 3)
+    return _remember(_FILL_RULE, key, (best, 256, 1) if costs[best] < 0.975 * costs.get(cfg[0], costs[3]) else cfg)
 
 
 def _rounds_rule(M: int, N: int, K: int, epi: int):
@@ -1489,16 +1496,15 @@ def _split_rule(M: int, N: int, K: int, epi: int, cfg, ld: int):
             or cfg[0] in GEMM1W_SPLIT or max(N, ld) * (M + 256) >= 1 << 26 or N * K * 2 >= 0x7FFFFFF0):
         return cfg
     key = (M, N, K, cfg)
-    if key not in _SPLIT_RULE:
-        costs = {(v, 256, ks): _split_cost(M, N, K, v, ks) for v in _SPLIT_COST for ks in (1, 2, 3, 4, 6, 8)
-                 if K // 64 >= 3 * ks}
-        best = min(costs, key=costs.get, default=cfg)
-        if cfg in costs and (best[2] == 1 or costs[best] > 0.95 * costs[cfg]):
-            best = cfg
-        if len(_SPLIT_RULE) > 4096:
-            _SPLIT_RULE.clear()
-        _SPLIT_RULE[key] = best
-    return _SPLIT_RULE[key]
+    best = _SPLIT_RULE.get(key)
+    if best is not None:
+        return best
+    costs = {(v, 256, ks): _split_cost(M, N, K, v, ks) for v in _SPLIT_COST for ks in (1, 2, 3, 4, 6, 8)
+             if K // 64 >= 3 * ks}
+    best = min(costs, key=costs.get, default=cfg)
+    if cfg in costs and (best[2] == 1 or costs[best] > 0.95 * costs[cfg]):
+        best = cfg
+    return _remember(_SPLIT_RULE, key, best)
 
 
 def _resid_cfg(M: int, N: int, K: int, ld: int = 0):

@@ -459,6 +459,27 @@ def test_split_rule_takes_what_measured_fastest(monkeypatch, M, N, K, epi, cfg, 
         monkeypatch.setattr(ops, name, True)
 
 
+@pytest.mark.parametrize("rule", ["_TILE_RULE", "_FILL_RULE", "_SPLIT_RULE"])
+def test_rules_of_tiles_survive_a_full_table(monkeypatch, rule):
+    """A rule's table of picks is shared by threads and emptied when it is full: a pick does not need its entry to be there still."""
+    from llm_kubernetes_minikube_sharp4dev_amd import ops
+
+    class Emptied(dict):   # another thread empties the table right behind every entry
+        def __setitem__(self, key, value):
+            super().__setitem__(key, value)
+            self.clear()
+
+    for name, value in (("GEMM1W", True), ("GEMM_SPLITK", True), ("SPLIT_ON", True), ("_CUS", 256)):
+        monkeypatch.setattr(ops, name, value)
+    picks = {"_TILE_RULE": lambda M: ops._tile_rule(M, 2048, 5632, 0), "_FILL_RULE": lambda M: ops._fill_rule(M, 28672, 1, (3, 256, 1)),
+             "_SPLIT_RULE": lambda M: ops._split_rule(M, 4096, 4096, 0, (3, 256, 1), 4096)}[rule]
+    monkeypatch.setattr(ops, rule, {})
+    want = [picks(M) for M in range(300, 1500, 100)]
+    assert [picks(M) for M in range(300, 1500, 100)] == want   # (from the table)
+    monkeypatch.setattr(ops, rule, Emptied())
+    assert [picks(M) for M in range(300, 1500, 100)] == want
+
+
 @pytest.mark.parametrize("M,N,K,epi,pick", [
     (58963, 2304, 768, 2, 3), (35218, 1536, 768, 2, 3), (44104, 768, 768, 2, 4), (17401, 768, 768, 2, 3), (8925, 2304, 1536, 0, 4), (5500, 3072, 2048, 0, 4),
     (62947, 6144, 2048, 0, 3), (14488, 1536, 4096, 0, 4), (4609, 768, 3072, 2, None), (4608, 2304, 768, 2, None), (9000, 192, 768, 0, None),
