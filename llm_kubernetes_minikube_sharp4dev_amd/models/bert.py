@@ -12,6 +12,7 @@ Varlen packed batches ([T, H] rows + cu_seqlens) — no padding FLOPs:
 from __future__ import annotations
 
 import math
+from typing import Optional
 
 import torch
 import torch.nn as nn
@@ -80,11 +81,13 @@ class EncoderModel(nn.Module):
         return self
 
     def forward(self, ids: torch.Tensor, cu: torch.Tensor, positions: torch.Tensor,
-                lens_cpu: list, type_ids=None, pool: bool = True, out=None, tiles=None):
+                lens_cpu: Optional[list], type_ids=None, pool: bool = True, out=None, tiles=None):
         """ids/positions [T] int32 packed; cu [B+1] int32 -> [B, H] f32 embeddings (``out``: the
         pooling kernel writes these rows instead, f32 or bf16; ``tiles``: the attention's device
-        tile list, precomputed -- a hipGraph capture cannot upload it)."""
+        tile list, precomputed -- a hipGraph capture cannot upload it).  ``lens_cpu`` None: the lengths are read from ``cu``."""
         cfg, nh, D, H = self.cfg, self.nh, self.D, self.cfg.hidden
+        if lens_cpu is None and tiles is None:
+            lens_cpu = (cu[1:] - cu[:-1]).tolist()
         h = ops.embed_layernorm(ids, None if cfg.rotary else positions, type_ids, self.tok, self.pos,
                                 self.typ, self.emb_ln_w, self.emb_ln_b, cfg.norm_eps)
         if cfg.bias and cfg.activation == "gelu" and not cfg.rotary and ops.encoder_rows_ok(h, H, cfg.intermediate):
@@ -116,7 +119,7 @@ class EncoderModel(nn.Module):
     def _few_rows(self, h, cu, lens_cpu, pool, out, tiles):
         """The layers with every norm inside the projection that reads it (and one text's attention inside its own)."""
         cfg, prev, s = self.cfg, None, None
-        if len(lens_cpu) > 1:
+        if lens_cpu is not None and len(lens_cpu) > 1:
             tiles = self._tiles(h, lens_cpu, tiles)
         for L in self.layers:
             if prev is None:

@@ -1058,8 +1058,8 @@ def attn_linear_add(qkv, cu, lens_cpu, nh: int, head_dim: int, scale: float, w, 
     """Bidirectional attention over packed rows [q | k | v], the projection of its output and the residual; one launch for one short
     text."""
     K = nh * head_dim
-    if (use_hip(qkv) and not GEMM_LIBRARY and head_dim == 64 and len(lens_cpu) == 1 and lens_cpu[0] == qkv.shape[0] and _fused_weight(w, b)
-            and lib().attn_linear_supported(qkv.shape[0], nh, w.shape[0])):
+    if (use_hip(qkv) and not GEMM_LIBRARY and head_dim == 64 and lens_cpu is not None and len(lens_cpu) == 1 and lens_cpu[0] == qkv.shape[0]
+            and _fused_weight(w, b) and lib().attn_linear_supported(qkv.shape[0], nh, w.shape[0])):
         return lib().attn_linear(qkv, nh, scale, w, b, residual)
     a = flash_prefill(qkv[:, :K], qkv[:, K:2 * K], qkv[:, 2 * K:], cu, nh, nh, head_dim, scale, False, q_lens_cpu=lens_cpu, tiles=tiles)
     return linear_add(a, w, b, residual)

@@ -162,6 +162,23 @@ def test_parameters_anywhere(hip, lens):
     assert torch.equal(m(ids, cu, pos, lens), want)
 
 
+@pytest.mark.parametrize("name", ["minilm-l6", "bert-tiny", "nomic-tiny"])
+@pytest.mark.parametrize("lens", [[9], [3, 9], [40], [30, 1, 12]])
+def test_lengths_from_the_device(hip, name, lens):
+    """``lens_cpu`` may be left out: the lengths are read from ``cu``, or only the given tiles are used."""
+    from llm_kubernetes_minikube_sharp4dev_amd import ops
+    from llm_kubernetes_minikube_sharp4dev_amd.models import build_encoder
+
+    m = build_encoder(name, device="cuda").random_init(3)
+    ids, cu, pos = _inputs(lens)
+    want = m(ids, cu, pos, lens)
+    assert torch.equal(m(ids, cu, pos, None), want)
+    got = m(ids, cu, pos, None, tiles=ops.device_tiles(lens, lens, 1, False, m.D, ids.device))
+    # (one text of heads of 64 has its attention inside a projection where its length is known: eight bf16 roundings a layer, 2^-9 of a value at
+    # most, on either way)
+    assert (got - want).norm() <= 2 * (8 * m.cfg.num_layers) ** 0.5 * 2.0 ** -9 * want.norm()
+
+
 def test_query_graphs_on_the_callers_streams(hip):
     """Replays enqueued from several streams and threads at once, with and without a priority of their own: the graphs share buffers, every
     vector is its own text's, and later work of a caller's stream finds it there."""
