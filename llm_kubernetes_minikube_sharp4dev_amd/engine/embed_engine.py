@@ -183,7 +183,7 @@ class EmbeddingEngine:
         # On the caller's own stream, unless the replays were given a priority that it does not have: waits between two streams on both sides
         # of a replay took 80 us of a query's 377.  The graphs share their buffers, so a replay waits for one enqueued on another stream before it.
         gs = cur if self._gpriority == 0 or cur.priority <= self._gpriority else self._gstream
-        with self._glock:
+        with self._glock, torch.cuda.device(self.device):   # (launches go to the current device's stream; a caller's may be another device)
             if gs != cur:
                 gs.wait_stream(cur)  # dst exists (and whatever the caller queued before it)
             with torch.cuda.stream(gs) if gs != cur else _nullctx():

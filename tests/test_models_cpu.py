@@ -688,3 +688,54 @@ def test_sums_of_two_products_where_they_pay(monkeypatch, M, N, K1, K2, pay):
 
     monkeypatch.setattr(ops, "_CUS", 256)
     assert ops.sums_pay(M, N, K1, K2) == pay
+
+
+def _query_replay(monkeypatch, current, priority):
+    """EmbeddingEngine._replay_query on a device that is only written down: what it did, in order, each with the device it was done on."""
+    import threading
+    from types import SimpleNamespace
+
+    import numpy as np
+
+    from llm_kubernetes_minikube_sharp4dev_amd import ops
+    from llm_kubernetes_minikube_sharp4dev_amd.engine.embed_engine import EmbeddingEngine
+
+    done, device, on = [], [0], [current]
+
+    class Within:
+        def __init__(self, cell, value):
+            self.cell, self.value = cell, value
+
+        def __enter__(self):
+            self.before, self.cell[0] = self.cell[0], self.value
+
+        def __exit__(self, *a):
+            self.cell[0] = self.before
+
+    def did(what):
+        return lambda *a: done.append((what, device[0], on[0]))
+
+    monkeypatch.setattr(torch.cuda, "device", lambda d: Within(device, torch.device(d).index))
+    monkeypatch.setattr(torch.cuda, "stream", lambda s: Within(on, s))
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda d=None: current)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(ops, "set_ids", did("ids"))
+    eng = object.__new__(EmbeddingEngine)
+    eng.device = torch.device("cuda", 1)
+    own = SimpleNamespace(priority=priority, wait_stream=did("wait"))
+    eng._gstream, eng._gpriority, eng._glock, eng._glast = own, priority, threading.Lock(), None
+    eng._gdone = SimpleNamespace(record=did("done"))
+    eng._qgraphs = {(3, torch.float32): (SimpleNamespace(replay=did("replay")), None, None)}
+    dst = SimpleNamespace(dtype=torch.float32, copy_=did("out"), record_stream=did("kept"))
+    assert eng._replay_query(np.array([1, 2, 3]), dst)
+    assert device == [0] and on == [current]
+    return done, own
+
+
+def test_query_replay_switches_to_its_device(monkeypatch):
+    """A caller whose current device is another one: ids, graph and result are enqueued on the engine's."""
+    from types import SimpleNamespace
+
+    cur = SimpleNamespace(priority=0, wait_stream=lambda s: None)
+    done, _ = _query_replay(monkeypatch, cur, 0)
+    assert done == [(w, 1, cur) for w in ("ids", "replay", "out", "done")]
