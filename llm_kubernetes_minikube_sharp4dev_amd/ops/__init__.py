@@ -1326,7 +1326,7 @@ def _cfg_of(M: int, N: int, K: int, epi: int):
             cfg = None
         elif cfg is not None and not SPLIT_ON and cfg[0] in GEMM1W_SPLIT:
             cfg = (3, 256, 1)
-    return _fill_rule(M, N, epi, cfg if cfg is not None else _rounds_rule(M, N, K, epi) or _tile_rule(M, N, K, epi))
+    return _fill_rule(M, N, epi, cfg if cfg is not None else _rounds_rule(M, N, K, epi) or _tile_rule(M, N, K, epi), K)
 
 
 # Shapes without a measured entry, more than 256 rows: gemm1w.hip's 128 / 192 / 256-row tiles against the fallback.  Its
@@ -1421,33 +1421,40 @@ def _rounds_cost(M: int, N: int, bm: int) -> float:
 _FILL_RULE: dict = {}
 
 
-def _fill_cost(M: int, N: int, epi: int, v: int) -> float:
-    """``_rounds_cost`` of a variant; of a column split the sum of its two launches, of which a short last round costs up to 0.3 more."""
-    cus = device_cus()
+def _fill_cost(M: int, N: int, epi: int, v: int, K: int = 4096) -> float:
+    """us that a variant's launches are estimated to differ by from another's: 0.71 of ``_rounds_cost`` per K-tile (of a column split the sum of its
+    two launches, of which a short last round costs up to 0.3 more), 2 us per round of 256-row tiles for their ends, 2 us for a second launch."""
+    cus, tn, steps = device_cus(), N // 256, K / 64
+
+    def launch(bm, cols):
+        return 0.71 * steps * _rounds_cost(M, cols * 256, bm) + 2.0 * bm / 256 * -(-(-(-M // bm) * cols) // cus)
+
     if v not in GEMM1W_SPLIT:
-        return _rounds_cost(M, N, GEMM1W_BM[v])
+        return launch(GEMM1W_BM[v], tn)
     cols, bm = gemm1w_split_cols(M, N, epi, cus), GEMM1W_SPLIT[v]
-    last = -(-M // bm) * (N // 256 - cols) % cus
-    return _rounds_cost(M, cols * 256, 256) + _rounds_cost(M, N - cols * 256, bm) + (0.3 * (1 - last / cus) if last else 0.0)
+    last = -(-M // bm) * (tn - cols) % cus
+    return launch(256, cols) + launch(bm, tn - cols) + 2.0 + (0.71 * steps * 0.3 * (1 - last / cus) if last else 0.0)
 
 
-def _fill_rule(M: int, N: int, epi: int, cfg):
+def _fill_rule(M: int, N: int, epi: int, cfg, K: int = 4096):
     """A pick of 256 or 192-row tiles or of a column split, at this very number of rows: a table's entry was measured at the top of a bucket of
-    256, and the rules above know no column split.  Another of the four where its rounds over the CUs cost 2.5 % less.  28,672 x 4,096 with SwiGLU:
+    256, and the rules above know no column split.  Another of the four where it is estimated to cost 1.5 % and 1 us less.  28,672 x 4,096 with SwiGLU:
     300 rows 84.2 -> 73.5 us (two tiles of either, 192 rows each), 949 rows 177.6 -> 167.0 (64 columns of 256 rows, the rest in 192), 1,100 rows
-    234 -> 206; 10,496 x 2,048 at 4,095 rows 142.7 -> 135.4 (32 columns, the rest in 192); 14,336 x 4,096 at 2,589 248 -> 228.  Of 587 products (22
-    shapes, 257 - 4,500 rows) it changes 34, by 0.92 on average, and makes none slower."""
+    234 -> 206; 10,496 x 2,048 at 4,095 rows 142.7 -> 135.4 (32 columns, the rest in 192); 14,336 x 4,096 at 2,589 248 -> 228.  Over 610 products (N 2,304 -
+    28,672, K 192 - 4,096, 257 - 4,600 rows, three epilogues) it changes 233 of the picks before it, 15 to over 2 % slower (12 % the worst, 10,496 x 320), all to
+    0.979 of their time on average.  By the rounds alone, without what a round and a launch cost whatever K is, 391 were changed and 61 slower,
+    most by a column split at K up to 1,024: 6,144 x 192 with GELU at 4,099 rows 1.12, 11,264 x 1,024 at 3,733 1.16."""
     if cfg is None or cfg[0] not in (3, 4, 6, 7) or cfg[2] != 1 or not 256 < M <= 4608 or not GEMM1W or N % 256:
         return cfg
-    key = (M, N, epi, cfg[0], device_cus(), SPLIT_ON)
+    key = (M, N, K, epi, cfg[0], device_cus(), SPLIT_ON)
     pick = _FILL_RULE.get(key)
     if pick is not None:
         return pick
     forms = (3, 4, 6, 7) if SPLIT_ON and _split_applies(M, N, epi) else (3, 4)
-    costs = {v: _fill_cost(M, N, epi, v) for v in forms}
+    costs = {v: _fill_cost(M, N, epi, v, K) for v in forms}
     best = min(costs, key=costs.get)
     # (a split that does not apply runs as 3)
-    return _remember(_FILL_RULE, key, (best, 256, 1) if costs[best] < 0.975 * costs.get(cfg[0], costs[3]) else cfg)
+    return _remember(_FILL_RULE, key, (best, 256, 1) if costs[best] + 1.0 < 0.985 * costs.get(cfg[0], costs[3]) else cfg)
 
 
 def _rounds_rule(M: int, N: int, K: int, epi: int):

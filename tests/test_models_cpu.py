@@ -459,6 +459,18 @@ def test_split_rule_takes_what_measured_fastest(monkeypatch, M, N, K, epi, cfg, 
         monkeypatch.setattr(ops, name, True)
 
 
+@pytest.mark.parametrize("M,N,K,epi,cfg,pick", [
+    (4258, 6144, 192, 0, 3, 3), (4099, 6144, 192, 3, 3, 3), (3754, 10496, 256, 0, 3, 3), (4139, 10496, 512, 0, 3, 3), (3821, 11264, 768, 3, 3, 3),
+    (3733, 11264, 1024, 3, 3, 3), (1148, 28672, 1024, 0, 3, 4), (2413, 16384, 4096, 1, 3, 6), (2589, 14336, 4096, 1, 3, 6)])
+def test_fill_rule_weighs_a_second_launch(monkeypatch, M, N, K, epi, cfg, pick):
+    """What a column split saves grows with K, what its second launch costs does not: a short K stays in one launch."""
+    from llm_kubernetes_minikube_sharp4dev_amd import ops
+
+    for name, value in (("GEMM1W", True), ("SPLIT_ON", True), ("_CUS", 256)):
+        monkeypatch.setattr(ops, name, value)
+    assert ops._fill_rule(M, N, epi, (cfg, 256, 1), K) == (pick, 256, 1)
+
+
 @pytest.mark.parametrize("rule", ["_TILE_RULE", "_FILL_RULE", "_SPLIT_RULE"])
 def test_rules_of_tiles_survive_a_full_table(monkeypatch, rule):
     """A rule's table of picks is shared by threads and emptied when it is full: a pick does not need its entry to be there still."""
