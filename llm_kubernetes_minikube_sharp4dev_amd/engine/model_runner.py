@@ -170,10 +170,11 @@ class ModelRunner:
         if tp is not None and tp.enabled and not getattr(tp, "simulated", False):
             import torch.distributed as dist
 
-            box = [dict(ops._GEMM_TABLE) if lead else None]
+            box = [(dict(ops._GEMM_TABLE), dict(ops._GEMM_MEASURED)) if lead else None]
             dist.broadcast_object_list(box, src=tp.ranks[0] if tp.ranks else 0, group=tp.ctrl or tp.group)
-            ops._GEMM_TABLE.clear()
-            ops._GEMM_TABLE.update(box[0])
+            for table, got in zip((ops._GEMM_TABLE, ops._GEMM_MEASURED), box[0]):
+                table.clear()
+                table.update(got)
         return res
 
     @staticmethod

@@ -568,6 +568,8 @@ def _gemm_sched(K: int) -> int:
         return GEMM_SCHED
     return 2 if K >= 4096 else 0
 _GEMM_TABLE: dict = {}
+# key -> (rows that were measured, the fastest there with ranges of K on gemm1w.hip's tiles among the candidates)
+_GEMM_MEASURED: dict = {}
 LIBRARY_FALLBACKS: dict = {}
 # measured (variant, bn, splits) per (M bucket, N, K, epilogue) for the shipped models' projections
 # (benchmarks/gemm_table.py on an MI355X; LK_GEMM_STATIC=0 ignores it)
@@ -634,6 +636,12 @@ def _static_cfg(key):
 
 def _gemm_key(M: int, N: int, K: int, epi: int):
     return ((M + 255) // 256, N, K, epi)
+
+
+def _measured(M: int, N: int, K: int, epi: int):
+    """What ``tune_gemm`` found fastest, where these rows are as many tiles of 128, 192 and 256 rows as those it measured, else None."""
+    m, best = _GEMM_MEASURED.get(_gemm_key(M, N, K, epi), (0, None))
+    return best if all(-(-M // bm) == -(-m // bm) for bm in (128, 192, 256)) else None
 
 
 # Variants 3 / 4 / 5 = csrc/gemm1w.hip, the one-wave-per-SIMD kernel with 256-wide column tiles and
@@ -761,7 +769,8 @@ def tune_gemm(weights, max_m: int, min_m: int = 512, iters: int = 6, cold_bytes:
     """Time every (schedule / variant, column tile) of the prefill kernels for each 256-row M
     bucket in [min_m, max_m] (or the row counts ``ms``) and each (weight, epilogue) pair; keep
     the fastest.  gemm.hip candidates run with the split-K the policy gives them, gemm1w.hip
-    unsplit.  As in serving, the weights arrive from HBM: each launch reads the next of enough
+    unsplit; where K may also be cut into ranges on gemm1w.hip's tiles (``_split_rule``), those that are estimated
+    within 1.3 of the best such split are measured too and kept apart (QKV and SwiGLU of a fused step take no split).  As in serving, the weights arrive from HBM: each launch reads the next of enough
     weight copies to overflow the 256 MB MALL (a warm-weight tuning picks the 2-phase schedule for
     the SwiGLU projection, which is 3 % slower in situ).  Candidates are timed round-robin so
     clock drift hits all alike.  ``weights``: [(w [N, K] bf16 CUDA tensor, epi)].  Returns
@@ -804,6 +813,9 @@ def tune_gemm(weights, max_m: int, min_m: int = 512, iters: int = 6, cold_bytes:
                     cfgs.append((v, bn, ks))
             if not cfgs:
                 continue
+            ranges = _split_costs(M, N, K) if _split_takes(M, N, K, epi, K) else {}
+            ranges = {c: t for c, t in ranges.items() if c[2] > 1 and L.gemm_supported(M, N, K, epi, c[1], c[2], c[0])}
+            unsplit, cfgs = cfgs, cfgs + [c for c, t in ranges.items() if t <= 1.3 * min(ranges.values())]
             fns = {c: (lambda c=c: L.gemm(x, wn(), bias, epi, c[1], None, c[0], c[2])) for c in cfgs}
             for f in fns.values():
                 f()
@@ -813,7 +825,7 @@ def tune_gemm(weights, max_m: int, min_m: int = 512, iters: int = 6, cold_bytes:
                     ts[c].append(once(f))
             med = {c: statistics.median(v) for c, v in ts.items()}
             key = _gemm_key(M, N, K, epi)
-            _GEMM_TABLE[key] = min(med, key=med.get)
+            _GEMM_TABLE[key], _GEMM_MEASURED[key] = min(unsplit, key=med.get), (M, min(med, key=med.get))
             out[key] = {f"v{c[0]}/{c[1]}/k{c[2]}": round(t, 1) for c, t in med.items()}
         del copies
     return out
@@ -1317,9 +1329,11 @@ EPI_RESID, EPI_QKV = 6, 7
 def _cfg_of(M: int, N: int, K: int, epi: int):
     """(schedule / variant, bn, splits) of the prefill GEMM for this shape: the start-up tuned
     table (LK_GEMM_TUNE=1), else the shipped measurements (gemm_table_mi355x.json), else the
-    fallback policy."""
+    fallback policy.  What start-up measured stays as it is for rows that make as many tiles; the rest by these very rows (``_fill_rule``)."""
     key = _gemm_key(M, N, K, epi)
     cfg = _GEMM_TABLE.get(key)
+    if cfg is not None and _measured(M, N, K, epi) is not None:
+        return cfg
     if cfg is None:
         cfg = _static_cfg(key)
         if cfg is not None and (not GEMM1W and cfg[0] in GEMM1W_BM):
@@ -1495,19 +1509,29 @@ def _split_cost(M: int, N: int, K: int, v: int, ks: int) -> float:
             + (2.9 + 0.46e-6 * ks * M * N * 2 if ks > 1 else 0.0))
 
 
+def _split_costs(M: int, N: int, K: int) -> dict:
+    return {(v, 256, ks): _split_cost(M, N, K, v, ks) for v in _SPLIT_COST for ks in (1, 2, 3, 4, 6, 8) if K // 64 >= 3 * ks}
+
+
+def _split_takes(M: int, N: int, K: int, epi: int, ld: int) -> bool:
+    return (GEMM1W and GEMM_SPLITK and 256 < M <= 4608 and epi in (0, 2, 3, 4) and N % 256 == 0 and K % 64 == 0
+            and max(N, ld) * (M + 256) < 1 << 26 and N * K * 2 < 0x7FFFFFF0)
+
+
 def _split_rule(M: int, N: int, K: int, epi: int, cfg, ld: int):
     """The pick ``cfg`` of :func:`_cfg_of`, or what the costs above take instead: (variant, 256, ranges of K).  ``ld``: the longest of the
     operands' row strides -- a split needs them whole within 32-bit offsets, where rows further apart go in chunks unsplit and in gemm.hip.
-    (The start-up measurements pass here too: they hold no split of these tiles.)"""
-    if (not (GEMM1W and GEMM_SPLITK) or not 256 < M <= 4608 or epi not in (0, 2, 3, 4) or N % 256 or K % 64 or cfg is None
-            or cfg[0] in GEMM1W_SPLIT or max(N, ld) * (M + 256) >= 1 << 26 or N * K * 2 >= 0x7FFFFFF0):
+    Where start-up has measured, that decides."""
+    if cfg is None or not _split_takes(M, N, K, epi, ld):
         return cfg
+    best = _measured(M, N, K, epi)
+    if best is not None or cfg[0] in GEMM1W_SPLIT:
+        return best or cfg
     key = (M, N, K, cfg)
     best = _SPLIT_RULE.get(key)
     if best is not None:
         return best
-    costs = {(v, 256, ks): _split_cost(M, N, K, v, ks) for v in _SPLIT_COST for ks in (1, 2, 3, 4, 6, 8)
-             if K // 64 >= 3 * ks}
+    costs = _split_costs(M, N, K)
     best = min(costs, key=costs.get, default=cfg)
     if cfg in costs and (best[2] == 1 or costs[best] > 0.95 * costs[cfg]):
         best = cfg

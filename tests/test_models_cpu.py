@@ -471,6 +471,47 @@ def test_fill_rule_weighs_a_second_launch(monkeypatch, M, N, K, epi, cfg, pick):
     assert ops._fill_rule(M, N, epi, (cfg, 256, 1), K) == (pick, 256, 1)
 
 
+@pytest.mark.parametrize("M,N,K,epi,fastest", [
+    (949, 28672, 256, 1, (3, 256, 1)), (1100, 28672, 256, 1, (6, 256, 1)), (512, 512, 4096, 0, (2, 256, 4)), (300, 512, 4096, 3, (0, 256, 2)),
+    (512, 512, 4096, 2, (5, 256, 8)), (768, 768, 2048, 0, (4, 256, 1)), (512, 512, 1024, 0, None)])
+def test_measured_products_run_as_measured(monkeypatch, M, N, K, epi, fastest):
+    """``tune_gemm`` on a clock that lets one candidate win: that one runs at the measured rows and at all that make as many tiles, and the
+    rules, which know estimates only, are not asked there."""
+    from types import SimpleNamespace
+
+    from llm_kubernetes_minikube_sharp4dev_amd import ops
+
+    ran = []
+
+    class Event:
+        def __init__(self, **kw):
+            self.record = self.synchronize = lambda: None
+
+        def elapsed_time(self, other):
+            return 1.0 if ran[-1] == fastest else 2.0 + 0.001 * len(set(ran[:ran.index(ran[-1])]))
+
+    lib = SimpleNamespace(gemm_supported=lambda M, N, K, epi, bn, ks, v: True, gemm=lambda x, w, b, epi, bn, out, v, ks: ran.append((v, bn, ks)))
+    for name, value in (("GEMM1W", True), ("GEMM_SPLITK", True), ("SPLIT_ON", True), ("_CUS", 256), ("lib", lambda: lib), ("_GEMM_TABLE", {}),
+                        ("_GEMM_MEASURED", {}), ("_gemm_splits", lambda M, N, K, epi, bn: fastest[2] if fastest and fastest[0] < 3 else 1)):
+        monkeypatch.setattr(ops, name, value, raising=False)
+    monkeypatch.setattr(torch.cuda, "Event", Event)
+    ops.tune_gemm([(torch.zeros(N, K, dtype=torch.bfloat16), epi)], 0, iters=1, cold_bytes=0, ms=[M])
+
+    def runs(m):
+        cfg = ops._cfg_of(m, N, K, epi)
+        return ops._split_rule(m, N, K, epi, cfg, K)
+
+    pick = fastest or ran[0]   # (None: the first of the candidates)
+    assert pick in ran and runs(M) == pick
+    tiles = lambda m: [-(-m // bm) for bm in (128, 192, 256)]  # noqa: E731
+    for m in range(max(257, M - 256), M + 256):
+        if tiles(m) == tiles(M):
+            assert runs(m) == pick
+    if fastest and fastest[0] >= 3 and fastest[2] > 1:   # unsplit where a split cannot run: fused QKV, rows further apart
+        assert ops._cfg_of(M, N, K, epi)[2] == 1
+        assert ops._split_rule(M, N, K, epi, ops._cfg_of(M, N, K, epi), 1 << 20) == ops._cfg_of(M, N, K, epi)
+
+
 @pytest.mark.parametrize("rule", ["_TILE_RULE", "_FILL_RULE", "_SPLIT_RULE"])
 def test_rules_of_tiles_survive_a_full_table(monkeypatch, rule):
     """A rule's table of picks is shared by threads and emptied when it is full: a pick does not need its entry to be there still."""
