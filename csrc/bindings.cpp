@@ -980,7 +980,9 @@ struct HostHits {
     __atomic_thread_fence(__ATOMIC_ACQUIRE);
     return true;
   }
-  // (without the GIL) spins for 50 us, then gives the CPU away between looks; a stream that has failed or ended without a result raises
+  // (without the GIL) looks without a pause for 50 us and between other threads' turns for 500, where most searches end; behind other
+  // work on the stream it then sleeps for a sixteenth of the time it has waited (half a millisecond at most) from look to look.  A stream
+  // that has failed or ended without a result raises
   void wait() const {
     const auto t0 = std::chrono::steady_clock::now();
     double asked = 0.005;
@@ -990,7 +992,8 @@ struct HostHits {
         __builtin_ia32_pause();
       }
       const double s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-      if (s > 50e-6) std::this_thread::yield();
+      if (s > 500e-6) std::this_thread::sleep_for(std::chrono::duration<double>(std::min(s / 16, 500e-6)));
+      else if (s > 50e-6) std::this_thread::yield();
       if (s > asked) {
         const hipError_t e = hipStreamQuery(stream.stream());
         if (e == hipErrorNotReady) (void)hipGetLastError();

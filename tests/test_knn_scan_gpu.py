@@ -64,6 +64,28 @@ def test_hits_as_they_arrive(hip):
     assert ops.knn_hits(c, ops.row_norms(c), torch.randn(17, 768, device=DEV).to(torch.bfloat16), 3) is None
 
 
+def test_a_long_wait_sleeps(hip):
+    """A search behind tens of milliseconds of other work: its waiting thread leaves the CPU to others."""
+    import time
+
+    g = torch.Generator(device=DEV).manual_seed(4)
+    c, q = (torch.randn(n, 768, device=DEV, generator=g).to(torch.bfloat16) for n in (20011, 2))
+    cn, m = ops.row_norms(c), torch.randn(8192, 8192, device=DEV, generator=g).to(torch.bfloat16)
+    want = ops.knn_packed(c, cn, q, 5)
+    m @ m
+    torch.cuda.synchronize()
+    for _ in range(40):
+        y = m @ m
+    h = ops.knn_hits(c, cn, q, 5)
+    t, cpu = time.perf_counter(), time.thread_time()
+    h.synchronize()
+    t, cpu = time.perf_counter() - t, time.thread_time() - cpu
+    assert t > 0.01, t   # (40 products of 1.1 TFLOP are 17 ms at the card's peak)
+    assert cpu < 0.3 * t, (cpu, t)
+    assert [[i for i, _ in r] for r in h.rows(5)] == want[1].tolist()
+    del y
+
+
 def test_index_search_agrees(hip):
     """RagIndex gives the same hits whether or not the one-pass search takes the shape."""
     g = torch.Generator(device=DEV).manual_seed(3)
