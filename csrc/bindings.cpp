@@ -680,7 +680,6 @@ at::Tensor embed_rows(const at::Tensor& table, const at::Tensor& ids, int64_t lo
   return out;
 }
 
-// ids[dst] = prev[src] (in-flight decode inputs of a pipelined step)
 // ids (int32, on the GPU) = the host's values; false where they are more than one launch takes
 bool set_ids(at::Tensor& ids, const at::Tensor& host) {
   CHECK_CUDA(ids); CHECK_I32(ids); CHECK_CONTIG(ids); CHECK_I32(host); CHECK_CONTIG(host);
@@ -690,6 +689,7 @@ bool set_ids(at::Tensor& ids, const at::Tensor& host) {
   return true;
 }
 
+// ids[dst] = prev[src] (in-flight decode inputs of a pipelined step)
 void scatter_ids(at::Tensor& ids, const at::Tensor& dst, const at::Tensor& prev, const at::Tensor& src) {
   CHECK_CUDA(ids); CHECK_I32(ids); CHECK_CONTIG(ids); CHECK_I32(prev); CHECK_CONTIG(prev);
   TORCH_CHECK(dst.scalar_type() == at::kLong && src.scalar_type() == at::kLong && dst.is_contiguous() && src.is_contiguous() &&
@@ -945,8 +945,6 @@ std::vector<at::Tensor> knn_topk(const at::Tensor& corpus, const at::Tensor& cno
   return {out_s, out_i};
 }
 
-// The one-pass search with both results in one buffer, int32 [2, nq, K] (score bits, then row numbers), for a caller that copies
-// them to the host in one piece; an empty tensor where the one-pass search does not take the shape.
 // Hits of a launched search in pinned memory, seen by the host as they arrive: every word holds a value that no search leaves until
 // the merge writes it, once.  A wait for an event behind the kernels costs its barrier packet and the signal's way, 13 us on an idle
 // stream; reading the words costs neither.
@@ -1031,23 +1029,12 @@ void knn_scan_to(int* o, const at::Tensor& corpus, const at::Tensor& cnorm, cons
                        reinterpret_cast<float*>(p), p + nq * nb * K, reinterpret_cast<float*>(o), o + nq * K, cur_stream()), "knn_scan");
 }
 
-at::Tensor knn_packed(const at::Tensor& corpus, const at::Tensor& cnorm, const at::Tensor& queries, int64_t K, bool host) {
+// The one-pass search with both results in one buffer, int32 [2, nq, K] (score bits, then row numbers); an empty tensor where the one-pass
+// search does not take the shape.
+at::Tensor knn_packed(const at::Tensor& corpus, const at::Tensor& cnorm, const at::Tensor& queries, int64_t K) {
   const int nb = knn_scan_plan(corpus, cnorm, queries, K);
-  auto io = corpus.options().dtype(at::kInt);
-  if (!nb) return at::empty({0}, io);
-  // host: the merge writes the few hits straight into pinned memory (a copy behind it was one more launch in the caller's wait)
-  at::Tensor out = at::empty({2, queries.size(0), K}, host ? at::TensorOptions(at::kInt).pinned_memory(true) : io);
-  int* o = out.data_ptr<int>();
-  const auto passed = [&] {   // the pinned block is not given out again before the stream has passed this point
-    if (host) at::getHostAllocator(at::kCUDA)->record_event(o, out.storage().data_ptr().get_context(), c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().unwrap());
-  };
-  try {
-    knn_scan_to(o, corpus, cnorm, queries, K, nb);
-  } catch (...) {
-    passed();
-    throw;
-  }
-  passed();
+  at::Tensor out = at::empty({nb ? 2 : 0, queries.size(0), K}, corpus.options().dtype(at::kInt));
+  if (nb) knn_scan_to(out.data_ptr<int>(), corpus, cnorm, queries, K, nb);
   return out;
 }
 
@@ -2574,7 +2561,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("flash_prefill", &flash_prefill, "", py::arg("q"), py::arg("k"), py::arg("v"), py::arg("block_tables"), py::arg("cu_q"), py::arg("ctx_lens"), py::arg("tile_seq"), py::arg("tile_q0"), py::arg("Hq"), py::arg("Hkv"), py::arg("D"), py::arg("scale"), py::arg("causal"), py::arg("out") = py::none(), py::arg("part_o") = py::none(), py::arg("part_ml") = py::none(), py::arg("q_past") = py::none());
   m.def("knn_topk", &knn_topk, "", py::arg("corpus"), py::arg("cnorm"), py::arg("queries"), py::arg("qnorm"),
         py::arg("K"), py::arg("force_fused") = false);
-  m.def("knn_packed", &knn_packed, "", py::arg("corpus"), py::arg("cnorm"), py::arg("queries"), py::arg("K"), py::arg("host") = false);
+  m.def("knn_packed", &knn_packed, "", py::arg("corpus"), py::arg("cnorm"), py::arg("queries"), py::arg("K"));
   py::class_<HostHits>(m, "HostHits")
       .def("query", &HostHits::arrived)
       .def("synchronize", &HostHits::wait, py::call_guard<py::gil_scoped_release>())

@@ -270,13 +270,12 @@ def knn_topk(corpus, cnorm, queries, qnorm, K: int):
     return ref.knn_topk(corpus, cnorm, queries, qnorm, K)
 
 
-def knn_packed(corpus, cnorm, queries, K: int, host: bool = False):
+def knn_packed(corpus, cnorm, queries, K: int):
     """:func:`knn_topk` of few queries on the GPU with both results in one int32 tensor [2, nq, K] (the scores' bits, then
-    the indices), with ``host`` in pinned memory, to be read once the stream has come there.  None where the one-pass search does
-    not take the shape."""
+    the indices).  None where the one-pass search does not take the shape."""
     if not (use_hip(corpus) and queries.is_cuda and 1 <= K <= 64 and queries.shape[0] > 0):
         return None
-    r = lib().knn_packed(corpus, cnorm, queries, K, host)
+    r = lib().knn_packed(corpus, cnorm, queries, K)
     return r if r.numel() else None
 
 
