@@ -1503,7 +1503,7 @@ at::Tensor ssm_scan(const at::Tensor& xbc, const at::Tensor& dt, int64_t heads, 
   CHECK_CUDA(state); CHECK_F32(state); CHECK_CONTIG(state);
   TORCH_CHECK(state.dim() == 4 && state.size(1) == heads && state.size(2) == P && state.size(3) == N, "state must be f32 [slots, heads, P, N]");
   at::Tensor y = at::empty({xbc.size(0), heads * P}, xbc.options().dtype(at::kFloat));
-  CHECK_RC(lk_ssm_scan(xbc.data_ptr(), xbc.stride(0), dt.data_ptr(), dt.stride(0), cu.numel() - 1, heads, P, N, groups,
+  CHECK_RC(lk_ssm_scan(xbc.data_ptr(), xbc.stride(0), dt.data_ptr(), dt.stride(0), xbc.size(0), cu.numel() - 1, heads, P, N, groups,
                        fp(dt_bias, heads, "dt_bias"), fp(A_log, heads, "A_log"), fp(D, heads, "D"), state.data_ptr<float>(),
                        ip(cu), ip(slots), ip(positions), y.data_ptr<float>(), y.stride(0), (int)max_len, esz, cur_stream()), "ssm_scan");
   return y;
@@ -2390,6 +2390,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sigattn_decode", &sigattn_decode);
   m.def("conv_silu", &conv_silu);
   m.def("ssm_scan", &ssm_scan);
+  m.def("ssm_piped", &lk_ssm_piped, "", py::arg("S"), py::arg("heads"), py::arg("P"), py::arg("N"), py::arg("max_len"), py::arg("rows"), py::arg("cus"));
   m.def("gated_group_rmsnorm", &gated_group_rmsnorm);
   m.def("embed_stream", &embed_stream);
   m.def("stream_layernorm", &stream_layernorm);

@@ -292,7 +292,8 @@ int lk_sigattn_decode(const void* q, long qs, const void* kc, const void* vc, co
 int lk_conv_silu(const void* u, long us, int C, int taps, const float* w, const float* bias, void* state, const int* cu,
                  const int* slots, const int* positions, int S, int max_len, void* out, long os, int act, int esz,
                  hipStream_t st);
-int lk_ssm_scan(const void* xbc, long xs, const void* dt, long dts, int S, int heads, int P, int N, int groups,
+int lk_ssm_piped(int S, int heads, int P, int N, int max_len, long rows, int cus);
+int lk_ssm_scan(const void* xbc, long xs, const void* dt, long dts, long rows, int S, int heads, int P, int N, int groups,
                 const float* dt_bias, const float* A_log, const float* D, float* state, const int* cu, const int* slots,
                 const int* positions, float* y, long ys, int max_len, int esz, hipStream_t st);
 int lk_gated_group_rmsnorm(const float* y, long ys, const void* z, long zs, const float* w, long rows, int inner,

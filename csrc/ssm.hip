@@ -13,6 +13,7 @@
 // A batch is a list of sequences (prefill chunks of any length, decode rows of length 1): rows
 // [cu[s], cu[s+1]) belong to sequence s, whose state lives in slot slots[s] (< 0: a padding row,
 // skipped) and starts from zero when its first row sits at position 0.
+#include <algorithm>
 #include "common.h"
 #include "kernels.h"
 
@@ -687,7 +688,7 @@ __global__ __launch_bounds__(256) void ssm_chunk_kernel(const T* __restrict__ xb
 // enters a product as three bf16 parts (8 + 8 + 8 mantissa bits, an f32), summed in the f32 accumulators.  A sequence's chunks are a
 // serial chain, so what bounds the kernel is the time of one chunk: 64 tokens take 130 products of 16 cycles per wave instead of
 // 4 x 100 of 32 (16x16x4 f32), with two barriers instead of eight.  4 x 1,024 tokens, 64 heads of [64, 128]: 351 us (f32
-// products, chunks of 16) -> 126 us (now ssm_pipe_kernel's, which takes states of 33 - 128 columns); 4 x 512, 32 heads of [64, 256] 75 us.
+// products, chunks of 16) -> 126 us (now ssm_pipe_kernel's, which takes states of 33 - 128 columns: lk_ssm_piped); 4 x 512, 32 heads of [64, 256] 75 us.
 // Error against f64 9e-8 (f32 products: 2.2e-7).
 // grid (sequence, head, P / 64): wave w owns state columns p0 + 16 w .. +15 (all N rows as accumulators S[n][p]: lane p = l & 15,
 // rows 16 nt + 4 (l >> 4) + j) and computes M's rows of token tile w for everybody.  y is accumulated transposed (lane: one token,
@@ -1358,8 +1359,17 @@ __global__ __launch_bounds__(256) void gated_group_rmsnorm_wave_kernel(const flo
 // (16 heads of [128, 16]: 32 portions of 16 10.3 against 15.0, 8 and 64 decode rows 17.4 / 24.8; 17 tokens 7.5 / 7.1).
 constexpr int kChunkMin = 8;
 
+int cu_count() {
+  static const int cus = [] {
+    int dev = 0, n = 256;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 256;
+    return n;
+  }();
+  return cus;
+}
+
 template <typename T>
-int scan_t(const T* xbc, long xs, const T* dtp, long dts, int S, int heads, int P, int N, int groups,
+int scan_t(const T* xbc, long xs, const T* dtp, long dts, long rows, int S, int heads, int P, int N, int groups,
            const float* dt_bias, const float* A_log, const float* D, float* state, const int* cu, const int* slots,
            const int* positions, float* y, long ys, int max_len, hipStream_t st) {
   if (max_len >= kChunkMin) {
@@ -1381,7 +1391,8 @@ int scan_t(const T* xbc, long xs, const T* dtp, long dts, int S, int heads, int 
                                                                  state, cu, slots, positions, y, ys);                          \
   } while (0)
         if (N <= 32) LK_CHUNK64(2);
-        else if (N <= 64) LK_PIPE(4);
+        else if (N <= 64 && lk_ssm_piped(S, heads, P, N, max_len, rows, cu_count())) LK_PIPE(4);
+        else if (N <= 64) LK_CHUNK64(4);
         else if (N <= 128) LK_PIPE(8);
         else LK_CHUNK64(16);   // (two chunks' columns of 256 do not fit the LDS)
 #undef LK_CHUNK64
@@ -1500,14 +1511,27 @@ int lk_conv_silu(const void* u, long us, int C, int taps, const float* w, const 
   return 0;
 }
 
-int lk_ssm_scan(const void* xbc, long xs, const void* dt, long dts, int S, int heads, int P, int N, int groups,
+// Whether 64-token chunks of 33 - 128 state columns run as the pipeline of 16 waves, one workgroup to a CU, or (up to 64 columns, whose
+// LDS leaves room for two) in four waves.  The pipeline shortens a sequence's chain; where workgroups queue for the CUs what decides is how long one
+// of one chunk holds its place, and that is shorter in four waves.  us: the longest sequence alone, then each further round of workgroups with
+// its average chunks; within 6 % (rms) of 126 launches (6 layouts of 33 - 64 columns, 1 - 257 sequences of 8 - 2,000 tokens), and the slower of the
+// two for two of them (10 %).  32 heads of [64, 64], four waves / pipeline: 16 x 8 tokens 10.7 / 12.9, 64 x 8 33.5 / 42.6, 64 x 64 34.0 / 43.5,
+// 64 x 128 55.4 / 62.3, 16 x 256 30.1 / 28.7, 8 x 512 42.4 / 25.9, 4 x 8 8.7 / 7.0, 8 and 256 decode rows 110 / 160, 512 and 64 65.2 / 60.8.
+int lk_ssm_piped(int S, int heads, int P, int N, int max_len, long rows, int cus) {
+  if (N > 64) return 1;
+  const long wgs = (long)S * heads * ((P + 63) / 64);
+  const double later = (max_len + 63) / 64 - 1, each = std::min(later, rows / 64.0 / S), queue = (double)((wgs + cus - 1) / cus - 1);
+  return 7.0 + 2.2 * later + queue * (4.9 + 2.6 * each) < 8.1 + 4.4 * later + queue * (3.3 + 2.3 * each);
+}
+
+int lk_ssm_scan(const void* xbc, long xs, const void* dt, long dts, long rows, int S, int heads, int P, int N, int groups,
                 const float* dt_bias, const float* A_log, const float* D, float* state, const int* cu, const int* slots,
                 const int* positions, float* y, long ys, int max_len, int esz, hipStream_t st) {
   if (S <= 0) return 0;
   if (heads <= 0 || groups <= 0 || heads % groups || P <= 0 || N <= 0) return -1;
-  return esz == 2 ? scan_t<bf16_t>((const bf16_t*)xbc, xs, (const bf16_t*)dt, dts, S, heads, P, N, groups, dt_bias,
+  return esz == 2 ? scan_t<bf16_t>((const bf16_t*)xbc, xs, (const bf16_t*)dt, dts, rows, S, heads, P, N, groups, dt_bias,
                                    A_log, D, state, cu, slots, positions, y, ys, max_len, st)
-                  : scan_t<float>((const float*)xbc, xs, (const float*)dt, dts, S, heads, P, N, groups, dt_bias, A_log,
+                  : scan_t<float>((const float*)xbc, xs, (const float*)dt, dts, rows, S, heads, P, N, groups, dt_bias, A_log,
                                   D, state, cu, slots, positions, y, ys, max_len, st);
 }
 

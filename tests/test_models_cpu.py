@@ -512,6 +512,19 @@ def test_measured_products_run_as_measured(monkeypatch, M, N, K, epi, fastest):
         assert ops._split_rule(M, N, K, epi, ops._cfg_of(M, N, K, epi), 1 << 20) == ops._cfg_of(M, N, K, epi)
 
 
+@pytest.mark.parametrize("S,heads,P,N,max_len,rows,piped", [
+    (4, 32, 64, 64, 8, 32, 1), (16, 32, 64, 64, 8, 128, 0), (64, 32, 64, 64, 64, 4096, 0), (256, 8, 64, 64, 16, 4096, 0), (64, 16, 128, 64, 128, 8192, 0),
+    (8, 32, 64, 64, 512, 4096, 1), (4, 128, 64, 64, 1024, 4096, 1), (1, 128, 64, 64, 8, 8, 1), (65, 32, 64, 64, 8, 72, 0), (65, 32, 64, 64, 512, 576, 1),
+    (65, 128, 64, 64, 512, 576, 0), (257, 24, 64, 40, 8, 264, 0), (16, 16, 32, 48, 64, 1024, 1), (64, 80, 64, 72, 8, 512, 1), (256, 64, 64, 128, 8, 2048, 1)])
+def test_state_space_pipeline_takes_what_it_is_faster_at(S, heads, P, N, max_len, rows, piped):
+    """33 - 64 state columns: many short portions stay with the kernel of two workgroups to a CU."""
+    from llm_kubernetes_minikube_sharp4dev_amd.ops import _ext
+
+    if not _ext.available():
+        pytest.skip("the kernel library is not built")
+    assert _ext.lib().ssm_piped(S, heads, P, N, max_len, rows, 256) == piped
+
+
 @pytest.mark.parametrize("rule", ["_TILE_RULE", "_FILL_RULE", "_SPLIT_RULE"])
 def test_rules_of_tiles_survive_a_full_table(monkeypatch, rule):
     """A rule's table of picks is shared by threads and emptied when it is full: a pick does not need its entry to be there still."""

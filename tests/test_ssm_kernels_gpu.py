@@ -119,6 +119,16 @@ def test_chunk_pipeline(hip, H, P, N, G, lens, later):
     assert (state.double() - want).norm() <= 1e-6 * want.norm()
 
 
+@pytest.mark.parametrize("H,P,N,lens,piped", [(8, 64, 64, [8, 64, 33, 17] * 16, False), (8, 64, 64, [64, 9] * 16, True), (16, 72, 40, [65, 8, 70, 64] * 8, False),
+                                              (8, 20, 48, [300, 1, 129] + [1] * 31, True), (24, 64, 56, [8] + [1] * 79, False)])
+def test_chunks_of_many_sequences(hip, H, P, N, lens, piped):
+    """States of 33 - 64 columns on both sides of the line between the pipeline and four waves."""
+    assert bool(hip.ssm_piped(len(lens), H, P, N, max(lens), sum(lens), 256)) == piped
+    y, ref, state, want = _run(lens, H, P, N, 1, torch.bfloat16, max(lens), 5)
+    assert (y.double() - ref).norm() <= 1e-6 * ref.norm()   # as above
+    assert (state.double() - want).norm() <= 1e-6 * want.norm()
+
+
 # (tiles of 4, 8 and 16 tokens at and past their edges, sequences shorter than one, a step of mixed lengths)
 @pytest.mark.parametrize("lens,C", [([1, 3, 4, 5], 2048), ([300], 6144), ([601], 6144), ([803, 7, 8, 9], 2048), ([1600, 15, 16, 17, 1], 6144)])
 @pytest.mark.parametrize("later", [0, 5])
