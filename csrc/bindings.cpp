@@ -2390,6 +2390,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sigattn_decode", &sigattn_decode);
   m.def("conv_silu", &conv_silu);
   m.def("ssm_scan", &ssm_scan);
+  m.def("conv_rows", &lk_conv_rows, "", py::arg("S"), py::arg("cblocks"), py::arg("max_len"), py::arg("cus"));
   m.def("ssm_piped", &lk_ssm_piped, "", py::arg("S"), py::arg("heads"), py::arg("P"), py::arg("N"), py::arg("max_len"), py::arg("rows"), py::arg("cus"));
   m.def("gated_group_rmsnorm", &gated_group_rmsnorm);
   m.def("embed_stream", &embed_stream);

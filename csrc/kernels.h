@@ -289,6 +289,7 @@ int lk_sigattn_decode(const void* q, long qs, const void* kc, const void* vc, co
                       hipStream_t st);
 
 // csrc/ssm.hip: selective state-space mixer (sequences = rows [cu[s], cu[s+1]), state slot slots[s])
+int lk_conv_rows(int S, int cblocks, int max_len, int cus);
 int lk_conv_silu(const void* u, long us, int C, int taps, const float* w, const float* bias, void* state, const int* cu,
                  const int* slots, const int* positions, int S, int max_len, void* out, long os, int act, int esz,
                  hipStream_t st);

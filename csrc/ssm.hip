@@ -1462,6 +1462,15 @@ int scan_t(const T* xbc, long xs, const T* dtp, long dts, long rows, int S, int 
 
 }  // namespace
 
+// Tokens per workgroup of the convolution, which walks them in fours behind each other: 4 or 8 where that leaves about a workgroup or two to a CU, 16
+// where shorter tiles would not all be on the chip at once.  bf16 x 6,144 channels, 4 / 8 / 16 tokens (us, with the state's launch): one sequence of
+// 60 7.8 / 9.0 / 11.8, of 300 8.9 / 9.6 / 12.2, of 900 16.5 / 14.5 / 14.2, of 2,000 30 / 22.0 / 21.2, four of 1,024 45 / 37 / 28.9; x 2,048
+// 18.8 / 16.2 / 17.6, x 512 8.2 / 8.7 / 11.0
+int lk_conv_rows(int S, int cblocks, int max_len, int cus) {
+  const auto groups = [&](int r) { return (long)S * cblocks * ((max_len + r - 1) / r); };
+  return groups(4) * 256 <= 300L * cus ? 4 : groups(8) * 256 <= 600L * cus ? 8 : kConvRows;
+}
+
 int lk_conv_silu(const void* u, long us, int C, int taps, const float* w, const float* bias, void* state, const int* cu,
                  const int* slots, const int* positions, int S, int max_len, void* out, long os, int act, int esz,
                  hipStream_t st) {
@@ -1472,12 +1481,7 @@ int lk_conv_silu(const void* u, long us, int C, int taps, const float* w, const 
   const auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
   if (taps <= 4 && C % ev == 0 && us % ev == 0 && os % ev == 0 && a16(u) && a16(out) && a16(state)) {
     const int cblocks = (C / ev + 255) / 256;
-    // tokens per workgroup, which walks them in fours behind each other: 4 or 8 where that leaves about a workgroup or two to a CU, 16 where
-    // shorter tiles would not all be on the chip at once.  bf16 x 6,144 channels, 4 / 8 / 16 tokens (us, with the state's launch): one sequence of
-    // 60 7.8 / 9.0 / 11.8, of 300 8.9 / 9.6 / 12.2, of 900 16.5 / 14.5 / 14.2, of 2,000 30 / 22.0 / 21.2, four of 1,024 45 / 37 / 28.9; x 2,048
-    // 18.8 / 16.2 / 17.6, x 512 8.2 / 8.7 / 11.0
-    const auto groups = [&](int r) { return (long)S * cblocks * ((max_len + r - 1) / r); };
-    const int rows = groups(4) <= 300 ? 4 : groups(8) <= 600 ? 8 : kConvRows;
+    const int rows = lk_conv_rows(S, cblocks, max_len, cu_count());
     const bool one = max_len == 1;
     dim3 gv(S, (max_len + rows - 1) / rows, cblocks);
     if (esz == 2)

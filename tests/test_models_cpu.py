@@ -525,6 +525,20 @@ def test_state_space_pipeline_takes_what_it_is_faster_at(S, heads, P, N, max_len
     assert _ext.lib().ssm_piped(S, heads, P, N, max_len, rows, 256) == piped
 
 
+@pytest.mark.parametrize("S,cblocks,max_len,rows", [(1, 3, 60, 4), (1, 3, 400, 4), (1, 3, 401, 8), (1, 3, 1600, 8), (1, 3, 1601, 16), (4, 3, 1024, 16), (300, 1, 1, 4),
+                                                    (600, 1, 2, 8), (601, 1, 8, 16)])
+def test_convolution_tiles_count_the_devices_cus(S, cblocks, max_len, rows):
+    """The convolution's tiles fill the CUs of the device: a partition of 32 picks what the whole chip does at eight times the workgroups."""
+    from llm_kubernetes_minikube_sharp4dev_amd.ops import _ext
+
+    if not _ext.available():
+        pytest.skip("the kernel library is not built")
+    pick = _ext.lib().conv_rows
+    assert pick(S, cblocks, max_len, 256) == rows
+    assert pick(S, 8 * cblocks, max_len, 2048) == rows
+    assert pick(S, cblocks, max_len, 32) >= rows and pick(S, cblocks, max_len, 32) == pick(S, 8 * cblocks, max_len, 256)
+
+
 @pytest.mark.parametrize("rule", ["_TILE_RULE", "_FILL_RULE", "_SPLIT_RULE"])
 def test_rules_of_tiles_survive_a_full_table(monkeypatch, rule):
     """A rule's table of picks is shared by threads and emptied when it is full: a pick does not need its entry to be there still."""
