@@ -526,6 +526,13 @@ static float prefill_defer() {
 // the query rows one workgroup covers: must use the launch's prefill_waves(G, D)
 int lk_prefill_rows_per_tile(int G, int D) { return G >= 4 ? 32 * (prefill_waves(G, D) / 4) : 32 * (4 / G); }
 
+// workgroups of the encoder's one-dimensional order over `groups` head groups, 0 where a launch does not take as many: the threads of one
+// dimension are counted in 32 bits, and the two-dimensional grid has the groups in another
+long lk_prefill_pairs(long ntiles, int groups, int threads) {
+  const long n = (ntiles + 15) / 16 * 16 * groups;
+  return n * threads < (1L << 32) ? n : 0;
+}
+
 int lk_flash_prefill(const bf16_t* q, long qs, const bf16_t* k, const bf16_t* v, long ks, long vs,
                      const int* block_tables, int bt_stride, const int* cu_q, const int* ctx_lens,
                      const int* tile_seq, const int* tile_q0, int ntiles, bf16_t* out, long os,
@@ -552,8 +559,8 @@ int lk_flash_prefill(const bf16_t* q, long qs, const bf16_t* k, const bf16_t* v,
   // 930 keys: 69.5 / 68.4 vs 75.5 / 76.1 us); the long-prefill grids of 8192 workgroups run
   // 2-6 % faster in the plain order (profiles/r5_flash_xcd/)
   pr.xcd = prefill_xcd() && (long)ntiles * (Hq / WH) <= 2048;
-  const long paired = (long)(ntiles + 15) / 16 * 16 * (Hq / WH);
-  if (!paged && !causal && prefill_xcd() && !pr.xcd && paired < (1L << 31)) {
+  const long paired = !paged && !causal && prefill_xcd() && !pr.xcd ? lk_prefill_pairs(ntiles, Hq / WH, 64 * NW) : 0;
+  if (paired) {
     pr.pairs = 1;
     grid = dim3((unsigned)paired);
   }

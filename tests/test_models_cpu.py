@@ -525,6 +525,17 @@ def test_state_space_pipeline_takes_what_it_is_faster_at(S, heads, P, N, max_len
     assert _ext.lib().ssm_piped(S, heads, P, N, max_len, rows, 256) == piped
 
 
+@pytest.mark.parametrize("ntiles,groups,workgroups", [(1, 1, 16), (796, 12, 9600), ((1 << 20) - 16, 16, (1 << 24) - 256),
+                                                      ((1 << 20) - 15, 16, 0), (1 << 20, 16, 0), (8 << 20, 2, 0)])
+def test_encoder_attention_grid_stays_in_a_launch(ntiles, groups, workgroups):
+    """One dimension of a launch holds fewer than 2^32 threads: past that the attention over many short texts keeps its two-dimensional grid."""
+    from llm_kubernetes_minikube_sharp4dev_amd.ops import _ext
+
+    if not _ext.available():
+        pytest.skip("the kernel library is not built")
+    assert _ext.lib().prefill_pairs(ntiles, groups, 256) == workgroups
+
+
 @pytest.mark.parametrize("S,cblocks,max_len,rows", [(1, 3, 60, 4), (1, 3, 400, 4), (1, 3, 401, 8), (1, 3, 1600, 8), (1, 3, 1601, 16), (4, 3, 1024, 16), (300, 1, 1, 4),
                                                     (600, 1, 2, 8), (601, 1, 8, 16)])
 def test_convolution_tiles_count_the_devices_cus(S, cblocks, max_len, rows):
