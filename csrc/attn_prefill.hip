@@ -107,9 +107,9 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void flash_prefill_kernel(PrefillP
   if constexpr (!PAGED && !CAUSAL) {
     if (p.pairs) {
       // an encoder's rows hold all heads side by side: an XCD takes two tiles (most sequences are one or two) with all of their heads behind
-      // each other, so that the 128-byte pieces of a row are read close together and a sequence's second tile finds its keys in that L2.
-      // 543 sequences of 20 - 224, 12 heads of 64: 125 -> 117 us; heads of 32 78 -> 66; 128 of 400 - 512 156 -> 151.  A head's tiles
-      // one after the other, or one tile or four at a time, were 1 - 6 us slower in one or another.
+      // each other, so that the 128-byte pieces of a row are read close together and a sequence's second tile finds its keys in that L2
+      // (where that pays: lk_prefill_order).  543 sequences of 20 - 224, 12 heads of 64: 125 -> 117 us; heads of 32 78 -> 66; 128 of 400 - 512
+      // 156 -> 151.  A head's tiles one after the other, or one tile or four at a time, were 1 - 6 us slower in one or another.
       const int ny = p.Hq / WH, at = blockIdx.x >> 3;
       bx = ((at / (2 * ny)) * 8 + (blockIdx.x & 7)) * 2 + at % (2 * ny) / ny;
       by = at % ny;
@@ -526,6 +526,18 @@ static float prefill_defer() {
 // the query rows one workgroup covers: must use the launch's prefill_waves(G, D)
 int lk_prefill_rows_per_tile(int G, int D) { return G >= 4 ? 32 * (prefill_waves(G, D) / 4) : 32 * (4 / G); }
 
+// Whether an encoder's grid of more than 2,048 workgroups runs in the order of two tiles with all of their heads (see the kernel).  It pays where
+// texts have a second tile that reads the same keys, up to about 2,048 rows, from where on a head's keys fill an L2 by themselves; of texts of one
+// tile, where rows leave the 256 MB behind the L2s or a head's piece of a row is half a line, and not while there is little to read in a tile,
+// whose start two more divisions lengthen.  Plain / this order (us): 12 heads of 64, 4,096 x 10 rows 210 / 225, 260 x 96 30.5 / 32.2, 500 x 128
+// 84.7 / 83.5, 496 x 129 139 / 131, 320 of 100 - 300 126 / 121, 64 x 1,024 302 / 297, 8 x 8,192 2,044 / 2,076; of 32, 2,500 x 10 87 / 93,
+// 260 x 96 25.9 / 21.2, 250 x 256 81 / 55; 16 heads of 128, 260 x 96 110 / 95, 16 x 4,096 2,593 / 2,665.
+int lk_prefill_order(long ntiles, long seqs, long rows, int heads, int D) {
+  if (rows >= 2048 * seqs) return 0;
+  if (10 * ntiles > 11 * seqs) return 1;   // (one text in ten has a second tile)
+  return rows >= 40 * ntiles && (D <= 32 || rows * heads * D * 8 >= 256L << 20);   // (q, k, v and the output)
+}
+
 // workgroups of the encoder's one-dimensional order over `groups` head groups, 0 where a launch does not take as many: the threads of one
 // dimension are counted in 32 bits, and the two-dimensional grid has the groups in another
 long lk_prefill_pairs(long ntiles, int groups, int threads) {
@@ -537,7 +549,7 @@ int lk_flash_prefill(const bf16_t* q, long qs, const bf16_t* k, const bf16_t* v,
                      const int* block_tables, int bt_stride, const int* cu_q, const int* ctx_lens,
                      const int* tile_seq, const int* tile_q0, int ntiles, bf16_t* out, long os,
                      int Hq, int Hkv, int D, int BS, float scale, int causal, int paged,
-                     float* part_o, float* part_ml, const int* q_past, hipStream_t st) {
+                     float* part_o, float* part_ml, const int* q_past, long rows, long seqs, hipStream_t st) {
   if (ntiles == 0) return 0;
   if (Hq % Hkv) return -1;
   // 16-B output stores (permlane-paired epilogue): 16-B aligned output rows
@@ -559,7 +571,8 @@ int lk_flash_prefill(const bf16_t* q, long qs, const bf16_t* k, const bf16_t* v,
   // 930 keys: 69.5 / 68.4 vs 75.5 / 76.1 us); the long-prefill grids of 8192 workgroups run
   // 2-6 % faster in the plain order (profiles/r5_flash_xcd/)
   pr.xcd = prefill_xcd() && (long)ntiles * (Hq / WH) <= 2048;
-  const long paired = !paged && !causal && prefill_xcd() && !pr.xcd ? lk_prefill_pairs(ntiles, Hq / WH, 64 * NW) : 0;
+  const long paired = !paged && !causal && prefill_xcd() && !pr.xcd && lk_prefill_order(ntiles, seqs, rows, Hq, D)
+                          ? lk_prefill_pairs(ntiles, Hq / WH, 64 * NW) : 0;
   if (paired) {
     pr.pairs = 1;
     grid = dim3((unsigned)paired);

@@ -879,7 +879,7 @@ at::Tensor flash_prefill(const at::Tensor& q, const at::Tensor& k, const at::Ten
                             bt_stride, ip(cu_q), ipo(ctx_lens), ip(tile_seq), ip(tile_q0), tile_seq.numel(),
                             partial ? nullptr : bp(out), partial ? 0 : out.stride(0), Hq, Hkv, D, BS, (float)scale,
                             causal ? 1 : 0, paged ? 1 : 0, partial ? part_o->data_ptr<float>() : nullptr,
-                            partial ? part_ml->data_ptr<float>() : nullptr, ipo(q_past), cur_stream());
+                            partial ? part_ml->data_ptr<float>() : nullptr, ipo(q_past), T, cu_q.numel() - 1, cur_stream());
   CHECK_RC(rc, "flash_prefill");
   return out;
 }
@@ -2561,6 +2561,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   }, "weight-streaming GEMM kernel for this (M bucket, N, K, swiglu): 0 ring, 1 loader waves, -1 default",
         py::arg("M"), py::arg("N"), py::arg("K"), py::arg("swiglu"), py::arg("variant"));
   m.def("prefill_pairs", &lk_prefill_pairs, "", py::arg("ntiles"), py::arg("groups"), py::arg("threads"));
+  m.def("prefill_order", &lk_prefill_order, "", py::arg("ntiles"), py::arg("seqs"), py::arg("rows"), py::arg("heads"), py::arg("D"));
   m.def("flash_prefill", &flash_prefill, "", py::arg("q"), py::arg("k"), py::arg("v"), py::arg("block_tables"), py::arg("cu_q"), py::arg("ctx_lens"), py::arg("tile_seq"), py::arg("tile_q0"), py::arg("Hq"), py::arg("Hkv"), py::arg("D"), py::arg("scale"), py::arg("causal"), py::arg("out") = py::none(), py::arg("part_o") = py::none(), py::arg("part_ml") = py::none(), py::arg("q_past") = py::none());
   m.def("knn_topk", &knn_topk, "", py::arg("corpus"), py::arg("cnorm"), py::arg("queries"), py::arg("qnorm"),
         py::arg("K"), py::arg("force_fused") = false);

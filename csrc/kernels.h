@@ -205,11 +205,12 @@ int lk_paged_decode(const bf16_t* q, long qs, const bf16_t* kc, const bf16_t* vc
 // attn_prefill.hip
 int lk_prefill_rows_per_tile(int G, int D);
 long lk_prefill_pairs(long ntiles, int groups, int threads);
+int lk_prefill_order(long ntiles, long seqs, long rows, int heads, int D);
 int lk_flash_prefill(const bf16_t* q, long qs, const bf16_t* k, const bf16_t* v, long ks, long vs,
                      const int* block_tables, int bt_stride, const int* cu_q, const int* ctx_lens,
                      const int* tile_seq, const int* tile_q0, int ntiles, bf16_t* out, long os,
                      int Hq, int Hkv, int D, int BS, float scale, int causal, int paged,
-                     float* part_o, float* part_ml, const int* q_past, hipStream_t st);
+                     float* part_o, float* part_ml, const int* q_past, long rows, long seqs, hipStream_t st);
 
 // knn.hip
 int lk_knn_scan_blocks(long N, int D, int nq, int K);

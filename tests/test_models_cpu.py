@@ -536,6 +536,21 @@ def test_encoder_attention_grid_stays_in_a_launch(ntiles, groups, workgroups):
     assert _ext.lib().prefill_pairs(ntiles, groups, 256) == workgroups
 
 
+@pytest.mark.parametrize("texts,rows,heads,D,order", [
+    (4096, 10, 12, 64, 0), (2500, 10, 12, 32, 0), (260, 96, 12, 64, 0), (384, 65, 16, 64, 0), (500, 128, 12, 64, 1), (260, 96, 12, 32, 1), (260, 96, 16, 128, 1),
+    (496, 129, 12, 64, 1), (69, 129, 16, 128, 1), (128, 450, 12, 64, 1), (64, 1024, 12, 64, 1), (43, 1500, 16, 64, 1), (32, 2048, 12, 64, 0),
+    (8, 8192, 12, 64, 0), (16, 4096, 16, 128, 0)])
+def test_encoder_attention_order_by_its_texts(texts, rows, heads, D, order):
+    """Pairs of tiles with all of their heads where that measured faster: not for many texts of a few rows, nor for long ones."""
+    from llm_kubernetes_minikube_sharp4dev_amd import ops
+    from llm_kubernetes_minikube_sharp4dev_amd.ops import _ext
+
+    if not _ext.available():
+        pytest.skip("the kernel library is not built")
+    tiles = len(ops.prefill_tiles([rows] * texts, [rows] * texts, 1, False, D)[0])
+    assert _ext.lib().prefill_order(tiles, texts, rows * texts, heads, D) == order
+
+
 @pytest.mark.parametrize("S,cblocks,max_len,rows", [(1, 3, 60, 4), (1, 3, 400, 4), (1, 3, 401, 8), (1, 3, 1600, 8), (1, 3, 1601, 16), (4, 3, 1024, 16), (300, 1, 1, 4),
                                                     (600, 1, 2, 8), (601, 1, 8, 16)])
 def test_convolution_tiles_count_the_devices_cus(S, cblocks, max_len, rows):
