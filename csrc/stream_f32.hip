@@ -257,7 +257,7 @@ int lk_embed_pos(const int* ids, const int* positions, const void* tok, int voca
 int lk_stream_rmsnorm(float* x, const void* a, long as, const float* a_bias, const void* b, long bs, const float* e, float m, const float* w,
                       float woff, float eps, const long* idx, long out_rows, void* out, long os, int W, int esz,
                       hipStream_t st) {
-  if (out_rows <= 0) return 0;
+  if (out_rows <= 0 || W <= 0) return 0;   // (rows of no columns: nothing to read in the place of columns past the last)
   const auto al = [](const void* p, long stride_bytes, int vec_bytes) {
     return p == nullptr || (reinterpret_cast<uintptr_t>(p) % vec_bytes == 0 && stride_bytes % vec_bytes == 0);
   };

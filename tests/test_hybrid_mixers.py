@@ -342,6 +342,15 @@ def test_mamba2_slot_reuse_and_long_memory(device, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_stream_norm_rows_of_no_columns(hip, dtype):
+    x, a, idx = torch.zeros(3, 0, device="cuda"), torch.zeros(3, 0, device="cuda", dtype=dtype), torch.tensor([2, 0], device="cuda")
+    assert ops.stream_rmsnorm(x, a, out_dtype=dtype).shape == (3, 0)
+    assert ops.stream_rmsnorm(x, a, w=torch.zeros(0, device="cuda"), idx=idx, out_dtype=dtype).shape == (2, 0)
+    torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("W", [4, 1020, 1024, 1028, 2048, 2052, 4096, 4100, 8192])
 def test_stream_norm_row_lengths(hip, W):
     """Rows at the edges of what one, two, four and eight pieces per thread hold, with every input and with one."""
