@@ -180,8 +180,8 @@ def test_lengths_from_the_device(hip, name, lens):
 
 
 def test_query_graphs_on_the_callers_streams(hip):
-    """Replays enqueued from several streams and threads at once, with and without a priority of their own: the graphs share buffers, every
-    vector is its own text's, and later work of a caller's stream finds it there."""
+    """Replays enqueued from several streams and threads at once: the graphs share buffers, every vector is its own text's, and later work of
+    a caller's stream finds it there."""
     import threading
 
     from llm_kubernetes_minikube_sharp4dev_amd.engine.embed_engine import EmbeddingEngine
@@ -191,30 +191,29 @@ def test_query_graphs_on_the_callers_streams(hip):
     eager, g = EmbeddingEngine(m, None, "e"), torch.Generator().manual_seed(2)
     texts = [torch.randint(1000, 30000, (n,), generator=g).tolist() for n in (3, 9, 9, 14, 20)]
     want = [eager.embed_ids([t]) for t in texts]
-    for priority in (0, -1):
-        eng = EmbeddingEngine(m, None, "g")
-        assert eng.capture_queries(max_len=16, dtypes=(torch.float32,), priority=priority) == 16
-        got = {}
+    eng = EmbeddingEngine(m, None, "g")
+    assert eng.capture_queries(max_len=16, dtypes=(torch.float32,)) == 16
+    got = {}
 
-        def caller(i, eng=eng, got=got):
-            with torch.cuda.stream(torch.cuda.Stream()):
-                for r in range(20):
-                    for k, t in enumerate(texts):
-                        got[i, r, k] = eng.embed_ids([t]).clone()
-                torch.cuda.current_stream().synchronize()
+    def caller(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for r in range(20):
+                for k, t in enumerate(texts):
+                    got[i, r, k] = eng.embed_ids([t]).clone()
+            torch.cuda.current_stream().synchronize()
 
-        threads = [threading.Thread(target=caller, args=(i,)) for i in range(3)]
-        for t in threads:
-            t.start()
-        for r in range(20):
-            for k, t in enumerate(texts):
-                got["main", r, k] = eng.embed_ids([t]) * 1.0
-        for t in threads:
-            t.join()
-        torch.cuda.synchronize()
-        assert len(got) == 4 * 20 * len(texts)
-        for (_, _, k), v in got.items():
-            assert torch.equal(v, want[k])
+    threads = [threading.Thread(target=caller, args=(i,)) for i in range(3)]
+    for t in threads:
+        t.start()
+    for r in range(20):
+        for k, t in enumerate(texts):
+            got["main", r, k] = eng.embed_ids([t]) * 1.0
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert len(got) == 4 * 20 * len(texts)
+    for (_, _, k), v in got.items():
+        assert torch.equal(v, want[k])
 
 
 @pytest.mark.parametrize("n", [1, 63, 64, 65])

@@ -796,8 +796,9 @@ def test_sums_of_two_products_where_they_pay(monkeypatch, M, N, K1, K2, pay):
     assert ops.sums_pay(M, N, K1, K2) == pay
 
 
-def _query_replay(monkeypatch, current, priority):
-    """EmbeddingEngine._replay_query on a device that is only written down: what it did, in order, each with the device it was done on."""
+def _query_replay(monkeypatch, current, priority, last=None):
+    """EmbeddingEngine._replay_query on a device that is only written down: what it did, in order, each with the device and stream it was
+    done on (``last``: the stream of the replay before, or "own", the engine's)."""
     import threading
     from types import SimpleNamespace
 
@@ -828,8 +829,8 @@ def _query_replay(monkeypatch, current, priority):
     monkeypatch.setattr(ops, "set_ids", did("ids"))
     eng = object.__new__(EmbeddingEngine)
     eng.device = torch.device("cuda", 1)
-    own = SimpleNamespace(priority=priority, wait_stream=did("wait"))
-    eng._gstream, eng._gpriority, eng._glock, eng._glast = own, priority, threading.Lock(), None
+    own = SimpleNamespace(priority=priority, wait_stream=did("wait"), wait_event=did("event"))
+    eng._gstream, eng._gpriority, eng._glock, eng._glast = own, priority, threading.Lock(), own if last == "own" else last
     eng._gdone = SimpleNamespace(record=did("done"))
     eng._qgraphs = {(3, torch.float32): (SimpleNamespace(replay=did("replay")), None, None)}
     dst = SimpleNamespace(dtype=torch.float32, copy_=did("out"), record_stream=did("kept"))
@@ -845,3 +846,22 @@ def test_query_replay_switches_to_its_device(monkeypatch):
     cur = SimpleNamespace(priority=0, wait_stream=lambda s: None)
     done, _ = _query_replay(monkeypatch, cur, 0)
     assert done == [(w, 1, cur) for w in ("ids", "replay", "out", "done")]
+
+
+@pytest.mark.parametrize("current,priority,mine", [(0, 0, True), (-1, 0, True), (-1, -1, True), (0, -1, False)])
+def test_query_replay_stream(monkeypatch, current, priority, mine):
+    """Replays run on the caller's stream, or on the engine's where that has a priority that the caller's has not; behind a replay on another stream."""
+    from types import SimpleNamespace
+
+    joined, events = [], []
+    cur = SimpleNamespace(priority=current, wait_stream=joined.append, wait_event=events.append)
+    for last in (None, "own", cur, SimpleNamespace()):
+        done, own = _query_replay(monkeypatch, cur, priority, last)
+        on = cur if mine else own
+        other = last is not None and (own if last == "own" else last) is not on
+        work = [(w, 1, on) for w in ("ids", "replay", "out", "done")]
+        if mine:
+            assert done == work and len(events) == other and not joined
+        else:   # (waits for the caller's work before, and the caller for it behind; the result is kept for this stream)
+            assert done == [("wait", 1, cur)] + [("event", 1, own)] * other + work + [("kept", 0, cur)] and joined == [own]
+        joined.clear(), events.clear()
