@@ -358,7 +358,8 @@ __global__ __launch_bounds__(pre_waves<RP>() * 64, RP >= 256 ? 1 : 2) void lat_p
 // longer reads.  The registers halve, and two workgroups share a CU, each with its two tiles in half of the LDS to the byte, so one
 // multiplies while the other waits at a barrier (one workgroup of four pairs: 133 us for the first line).  The next tile is requested an
 // instruction per step of the scores: in one go that took 1,300 cycles in which the wave did nothing else.
-// 4,095 rows of 4 prompts, 16 heads, window 512: 144 -> 129 us; 32 heads, window 2,048: 322 -> 282; 300 rows behind 700: 68 -> 44.
+// 4,095 rows of 4 prompts, 16 heads, window 512: 144 -> 129 us; 32 heads, window 2,048: 322 -> 282; 300 rows behind 700: 68 -> 44.  Many portions of
+// little to read are where twice the workgroups, each of which walks the sequences for its tile, cost more: 200 of 16 rows behind 100, 93 -> 101.
 constexpr int kPairWaves = 4, kPairCols = 16 * kPairWaves;
 constexpr int pair_lds(int KD) { return 2 * 64 * KD + kPairWaves * 2048; }
 template <int RP, int RDP>
@@ -463,7 +464,7 @@ __global__ __launch_bounds__(64 * kPairWaves, 2) void lat_prefill_pair_kernel(La
 #pragma unroll
       for (int t = 0; t < 2; ++t) xs[t * 64 + lane] = c[1][t];
       handed();
-      // ---- the softmax of this wave's columns, with the first c^T fragments travelling under it
+      // ---- the softmax of this wave's columns (the c^T fragments are requested behind it: before the second hand-over they would have to be waited for)
       const int qq = n16 >> 2, pp = n16 & 3, swv = swz(4 * g + qq);   // rows 4g + qq and 16 + 4g + qq have the same swizzle
       const unsigned vr = base + (4 * g + qq) * KD * 2 + 8 * (pp & 1) + hf * (RP / 2) * 2;
       unsigned va[4];

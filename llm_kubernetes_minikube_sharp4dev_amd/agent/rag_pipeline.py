@@ -61,7 +61,7 @@ class RagAgentPipeline:
     def plan_launch(self, prompts: list[str]) -> dict:
         """Enqueue retrieval for a batch of user prompts without waiting on the device: the
         query encoder and the kNN kernel run on the current stream, the top-k lands in
-        pinned memory behind an event (:meth:`RagIndex.search_vectors_async`)."""
+        pinned memory (:meth:`RagIndex.search_vectors_async`)."""
         t0 = time.perf_counter()
         r = self.cfg.rag
         embedder = self.index.embedder

@@ -117,7 +117,8 @@ class EmbeddingEngine:
         """Capture one hipGraph of the encoder per single-query length 1..max_len (and output
         dtype), sharing one memory pool; returns the number captured.  Call once at start-up,
         while nothing else runs on the device (capture is thread-local: other threads' launches
-        stay legal).  ``priority``: of the stream the replays run on (-1: a serving process's
+        stay legal).  Replays run on the caller's stream, unless its priority is below ``priority``:
+        then on a stream of this engine that has it (-1: a serving process's
         query embeddings go ahead of the LLM engine's queued kernels, as embed_cpu's do)."""
         if self.device.type != "cuda" or not QUERY_GRAPHS:
             return 0

@@ -374,7 +374,7 @@ def test_bulk_embedding_two_streams_bit_identical(monkeypatch):
 def test_query_encoder_graphs_equal_eager():
     """Single-query embeddings replayed from the per-length encoder hipGraphs
     (EmbeddingEngine.capture_queries) equal the eager encoder's, f32 and bf16 rows, also from
-    several threads at once (replays are serialised on the engine's graph stream)."""
+    several threads at once (a replay on another stream waits for the one before it)."""
     import threading
 
     from llm_kubernetes_minikube_sharp4dev_amd.engine.embed_engine import EmbeddingEngine
