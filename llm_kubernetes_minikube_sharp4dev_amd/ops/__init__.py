@@ -639,6 +639,8 @@ def _gemm_key(M: int, N: int, K: int, epi: int):
 
 def _measured(M: int, N: int, K: int, epi: int):
     """What ``tune_gemm`` found fastest, where these rows are as many tiles of 128, 192 and 256 rows as those it measured, else None."""
+    if not _GEMM_MEASURED:   # (asked for every product of a pass)
+        return None
     m, best = _GEMM_MEASURED.get(_gemm_key(M, N, K, epi), (0, None))
     return best if all(-(-M // bm) == -(-m // bm) for bm in (128, 192, 256)) else None
 
@@ -1521,7 +1523,7 @@ def _split_rule(M: int, N: int, K: int, epi: int, cfg, ld: int):
     """The pick ``cfg`` of :func:`_cfg_of`, or what the costs above take instead: (variant, 256, ranges of K).  ``ld``: the longest of the
     operands' row strides -- a split needs them whole within 32-bit offsets, where rows further apart go in chunks unsplit and in gemm.hip.
     Where start-up has measured, that decides."""
-    if cfg is None or not _split_takes(M, N, K, epi, ld):
+    if cfg is None or not 256 < M <= 4608 or not _split_takes(M, N, K, epi, ld):
         return cfg
     best = _measured(M, N, K, epi)
     if best is not None or cfg[0] in GEMM1W_SPLIT:
