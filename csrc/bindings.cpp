@@ -158,9 +158,16 @@ at::Tensor skinny_linear(const at::Tensor& x, const at::Tensor& w, bool swiglu, 
   return out;
 }
 
+// the weight-streaming kernels reach X's rows by 32-bit offsets: rows further apart than those hold are copied together first
+static at::Tensor ws_near(const at::Tensor& x) {
+  const bool far = x.dim() == 2 && x.stride(1) == 1 && x.stride(0) % 8 == 0 && x.size(0) * x.stride(0) * 2 >= 0xFFFFFF00L;
+  return far ? x.contiguous() : x;
+}
+
 // Weight-streaming GEMM for 64 < M <= 256 (LDS-DMA staged, csrc/skinny_gemm.hip wsgemm)
-at::Tensor ws_linear(const at::Tensor& x, const at::Tensor& w, bool swiglu, int64_t bn, int64_t splits,
+at::Tensor ws_linear(const at::Tensor& x_, const at::Tensor& w, bool swiglu, int64_t bn, int64_t splits,
                      const c10::optional<at::Tensor>& out_) {
+  const at::Tensor x = ws_near(x_);
   CHECK_CUDA(x); CHECK_BF16(x); CHECK_BF16(w); CHECK_LASTDIM(x); CHECK_CONTIG(w);
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1), "x [M,K], w [N,K]");
   check_rows16(x, "x"); check_rows16(w, "w");
@@ -314,9 +321,10 @@ WsSplit ws_split(const at::Tensor& x, const at::Tensor& w, int64_t bn, int64_t s
 }  // namespace
 
 // out = RMSNorm(x W^T + residual) * norm_w, residual += x W^T (bf16, in place)
-at::Tensor ws_linear_rmsnorm(const at::Tensor& x, const at::Tensor& w, at::Tensor& residual,
+at::Tensor ws_linear_rmsnorm(const at::Tensor& x_, const at::Tensor& w, at::Tensor& residual,
                              const at::Tensor& norm_w, double eps, int64_t bn, int64_t splits,
                              const c10::optional<at::Tensor>& tickets) {
+  const at::Tensor x = ws_near(x_);
   const WsSplit p = ws_split(x, w, bn, splits, "ws_linear_rmsnorm");
   CHECK_CUDA(residual); CHECK_BF16(residual); CHECK_LASTDIM(residual); check_rows16(residual, "residual");
   TORCH_CHECK(residual.dim() == 2 && residual.size(0) == p.M && residual.size(1) == p.N, "residual shape");
@@ -341,11 +349,12 @@ at::Tensor ws_linear_rmsnorm(const at::Tensor& x, const at::Tensor& w, at::Tenso
 }
 
 // qkv = x W^T with RoPE applied and K/V scattered into the paged cache (as rope_kv_)
-at::Tensor ws_linear_rope_kv(const at::Tensor& x, const at::Tensor& w, const at::Tensor& positions,
+at::Tensor ws_linear_rope_kv(const at::Tensor& x_, const at::Tensor& w, const at::Tensor& positions,
                              const at::Tensor& cos_sin, int64_t Hq, int64_t Hkv, int64_t D,
                              const c10::optional<at::Tensor>& k_cache, const c10::optional<at::Tensor>& v_cache,
                              const c10::optional<at::Tensor>& slots, bool neox, bool write_k_inplace, int64_t bn,
                              int64_t splits, const c10::optional<at::Tensor>& tickets) {
+  const at::Tensor x = ws_near(x_);
   const WsSplit p = ws_split(x, w, bn, splits, "ws_linear_rope_kv");
   TORCH_CHECK(p.N == (Hq + 2 * Hkv) * D, "w must be the fused [(Hq + 2 Hkv) * D, K] projection");
   CHECK_I32(positions); CHECK_F32(cos_sin); CHECK_CONTIG(cos_sin); CHECK_CONTIG(positions);

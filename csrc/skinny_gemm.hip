@@ -29,6 +29,8 @@
 #include <cstdlib>
 #include <map>
 #include <mutex>
+#include <type_traits>
+#include <utility>
 
 #include "common.h"
 #include "kernels.h"
@@ -491,17 +493,21 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
 // Weight-streaming GEMM for 64 < M <= 256 rows ("wsgemm").  The fragment-shaped loads
 // of skinny_gemm_kernel touch 16 rows x 64 B per wave instruction, which caps the
 // per-CU load rate once X (re-read by every column block) grows with M.  Here both
-// operands are staged through LDS with 16-B global_load_lds (LDS-DMA): every wave
+// operands are staged through LDS by 16-B LDS-DMA: every wave
 // instruction moves 8 rows x one full 128-B line, lane-linear into LDS, with the
 // (row>>1)&7 XOR chunk swizzle applied on the SOURCE address so the MFMA fragment
 // reads (ds_read_b128, 16 rows x 16 B per lane group) are bank-conflict free.
-//   * block = 4 waves, tile = all M rows (16*MT) x BN columns, BK = 64 per stage,
-//     3-stage LDS ring, ONE raw s_barrier per stage, counted vmcnt (the DMA of the
-//     next stage stays in flight across the barrier and under the MFMAs);
-//   * waves split M (each 4*MT rows x BN columns: acc = MT/4 x BN/16 tiles);
-//   * W rows are streamed once with the non-temporal policy (aux = 2);
+//   * block = 4 waves, tile = all M rows (16*MT) x BN columns, BK = 64 per stage, as many stages as 160 KB of LDS hold, the walk below;
+//   * W rows are streamed once with the non-temporal policy;
 //   * split-K over blocks (S) when N/BN leaves CUs idle; partial slabs -> the same
 //     reduce / SwiGLU kernel as skinny_gemm; S = 1 writes bf16 (or SwiGLU) directly.
+// What bounds it: at 128 rows the chip's matrix rate (20 us for 28672 x 4096) is half of the weight's stream (38 us at 6.1 TB/s), so
+// neither hides a wait that the other has.  A CU takes 125 - 150 KB/us out of its L2 (X) and, with 256 of them at it, 24 from memory (W);
+// four waves with 8 KB each in flight reach that.  Waves that each took all columns of a quarter of the rows read 20 fragments a stage in three
+// groups, each waited for before its MFMAs, 0.64 us a stage with W out of L2; a 2 x 2 grid of waves reads 16, under the MFMAs of the stage
+// before: 0.5.  Cold, us (one ring / loader waves before -> now): 120 rows: gate / up 28672 x 4096 47.9 / 48.4 -> 46.7, 32768 x 4096
+// 51.0 / 48.8 -> 47.7, 6144 x 4096 15.6 / 16.2 -> 14.5, 4096 x 4096 12.5 / 13.2 -> 11.7, 4096 x 14336 27.9 / 27.7 -> 27.5; 256 rows:
+// 77 / 71 -> 59, 82 / 77 -> 62, 22.5 / 23.0 -> 20.0, 18.0 / 19.6 -> 17.5, 40.5 / 38.7 -> 34.7.
 template <int N>
 LK_DEVICE void wait_vmcnt() {
   static_assert(N >= 0 && N < 64, "vmcnt range");
@@ -509,31 +515,26 @@ LK_DEVICE void wait_vmcnt() {
 }
 
 typedef __attribute__((address_space(3))) void* lds_void_ptr;
-typedef const __attribute__((address_space(1))) void* gbl_void_ptr;
+
+typedef const __attribute__((address_space(3))) short8* lds_frag_t;
+typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 
 LK_DEVICE int wsz(int row) { return (row >> 1) & 7; }
-
-// ring depth: the in-flight DMA bytes per CU set the per-CU load rate (latency-bound
-// at one block per CU), so fill the 160 KB LDS
-constexpr int ws_stages(int MT, int BN) {
-  const int sb = (16 * MT + BN) * 128;
-  const int n = 163840 / sb;
-  return n > 8 ? 8 : (n < 3 ? 3 : n);
+template <class Fn, int... I>
+LK_DEVICE void ws_unroll_impl(Fn&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class Fn>
+LK_DEVICE void ws_unroll(Fn&& f) {
+  ws_unroll_impl(f, std::make_integer_sequence<int, N>{});
+}
+LK_DEVICE unsigned ws_rfl(unsigned v) { return (unsigned)__builtin_amdgcn_readfirstlane((int)v); }
+LK_DEVICE u32x4_t ws_srd(const void* p, long bytes) {  // buffer descriptor words, wave-uniform
+  const unsigned long a = reinterpret_cast<unsigned long>(p);
+  return u32x4_t{ws_rfl((unsigned)a), ws_rfl((unsigned)(a >> 32)), ws_rfl((unsigned)max(0L, min(bytes, 0xFFFFFFF0L))), 0x00020000u};
 }
 
-template <int L, int NS>
-LK_DEVICE void wait_ahead(int ahead) {  // vmcnt(ahead * L), ahead in [0, NS-2]
-  if constexpr (NS > 2) {
-    if (ahead >= NS - 2) {
-      wait_vmcnt<L * (NS - 2)>();
-      return;
-    }
-    wait_ahead<L, NS - 1>(ahead);
-  } else {
-    wait_vmcnt<0>();
-  }
-}
-
+// ring depth: as many stages as 160 KB of LDS hold
 // (PRO: a WsPro prologue computes X first -- the LDS ring leaves room for its static scratch)
 constexpr int ws_stages_pro(int MT, int BN, int PRO) {
   const int sb = (16 * MT + BN) * 128;
@@ -541,161 +542,217 @@ constexpr int ws_stages_pro(int MT, int BN, int PRO) {
   return n > 8 ? 8 : (n < 3 ? 3 : n);
 }
 
-template <int MT, int BN, bool SWIGLU, bool TAIL, int PRO = 0>
-__global__ __launch_bounds__(256, 1) void wsgemm_kernel(const bf16_t* __restrict__ X, long ldx,
-                                                        const bf16_t* __restrict__ W, int M, int K, int ks,
-                                                        int n_tiles, int swiglu_I, bf16_t* __restrict__ out,
-                                                        long ldo, float* __restrict__ part, long part_ld,
-                                                        long n_rows, int rot_mul, WsTail tl, WsPro pr) {
-  // n_rows: valid W rows (the last column tile may be partial: kNN over a corpus of
-  // any size); loads clamp to the last row, stores are masked
-  constexpr int ROWS = 16 * MT;          // padded M
-  constexpr int MTW = MT / 4;            // row tiles per wave
-  constexpr int NT = BN / 16;            // column tiles per wave
-  constexpr int XB = ROWS * 128;         // X stage bytes
-  constexpr int WB = BN * 128;           // W stage bytes
-  constexpr int SB = XB + WB;            // stage bytes
-  constexpr int NS = ws_stages_pro(MT, BN, PRO);  // ring depth: as many stages as 160 KB of LDS holds
-  constexpr int LX = ROWS / 32;          // X glds per wave per stage (8 rows each, 4 waves)
-  constexpr int LW = BN / 32;            // W glds per wave per stage
-  constexpr int L = LX + LW;
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+// The walk of one workgroup over its stages (64 columns of K): four waves in a 2 x 2 grid, a wave (ROWS / 2) rows x (BN / 2) columns.
+// The fragments of the next stage go to a second set of registers under this stage's MFMAs, so a stage is one barrier that says at once
+// "the next stage has landed" and "everyone holds this one in registers: its slot may be requested again", and no MFMA waits for LDS.
+// Stages past the last come from a descriptor without range (zeros nobody uses), so that every stage is the same code.
+// NSX / NSW: stages of X's and of W's ring.  LOADERS waves more than the four request W (0: the four do).
+template <int MT, int BN, bool SWIGLU, int NSX, int NSW, int LOADERS>
+struct WsWalk {
+  static constexpr int MW = MT / 2, NW = BN / 32;                     // 16 x 16 tiles of a wave; also the four waves' LDS-DMA pieces (8 rows) per stage
+  static constexpr int PW = LOADERS ? BN / 8 / LOADERS : NW;          // W pieces per stage of a wave that requests them
+  static constexpr int WSTEP = LOADERS ? LOADERS : 4;                 // its pieces are so many apart
+  static constexpr int XB = 16 * MT * 128, WB = BN * 128, L = MW + NW;
+  static constexpr int NM = 2 * MW * NW, NR = 2 * L;                  // MFMAs and fragment reads of a wave and stage
+  static constexpr int OPS = LOADERS ? MW : L;                        // requests per stage of one of the four
+  static_assert(LOADERS || NSX == NSW, "one ring");
+  static_assert((NSX - 1) * OPS < 64 && (NSW - 1) * PW < 64, "vmcnt");
+  unsigned xo[MW], wo[PW];
+  unsigned ldsx, ldsw, bx[2], bw[2];
+  u32x4_t xs, ws[2];
+  int nst, last, at, kofs;      // at: the next stage to request; kofs: its byte offset in a row
+  floatx4 acc[MW][NW];
+  short8 fx[2][2][MW], fw[2][2][NW];
 
-  const int t = blockIdx.x % n_tiles, s = blockIdx.x / n_tiles;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int r = lane & 15, g = lane >> 4;
-  const long kbase = (long)s * ks;
-  const int nst = ks / 64;
-  // K-step rotation: column tile t starts its K walk at step (t * rot_mul) % nst, so the
-  // blocks streaming at the same moment read different 128-B columns of X (every block
-  // reads all of X: in lockstep they would all hit the same few L2 channels)
-  const int rot = rot_mul ? (int)(((long)t * rot_mul) % nst) : 0;
+  // first row of column tile n in the tile's W rows as they lie in LDS, from the wave's first; SwiGLU: gate rows, then up rows
+  static constexpr int col(int n) { return SWIGLU ? (n < NW / 2 ? 16 * n : BN / 2 + 16 * (n - NW / 2)) : 16 * n; }
+  // piece i of a wave that requests W is one of up rows
+  static constexpr bool up(int i) { return SWIGLU && i >= PW / 2; }
 
-  auto wrow = [&](int row) -> long {  // tile row -> global W row (output column)
-    if constexpr (SWIGLU) {
-      return row < BN / 2 ? (long)t * (BN / 2) + row : (long)swiglu_I + (long)t * (BN / 2) + row - BN / 2;
-    } else {
-      return (long)t * BN + row;
-    }
-  };
-
-  // per-lane source pointers of this wave's glds instructions (k offset added per stage)
-  const bf16_t* xsrc[LX];
-  const bf16_t* wsrc[LW];
-  const int lrow = lane >> 3, lch = lane & 7;
+  // wave q of those that request W
+  LK_DEVICE void begin(const unsigned char* smem, const bf16_t* X, long ldx, const bf16_t* W, const bf16_t* W2, long wrows, int M, int K,
+                       long kbase, int stages, int rot) {
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, g = lane >> 4, lrow = lane >> 3, q = LOADERS ? w - 4 : w;
+    xs = ws_srd(X + kbase, (long)M * ldx * 2 - kbase * 2);            // rows past M: zeros
+    ws[0] = ws_srd(W + kbase, wrows * K * 2 - kbase * 2);
+    ws[1] = SWIGLU ? ws_srd(W2 + kbase, wrows * K * 2 - kbase * 2) : ws[0];
+    nst = stages;
+    at = 0;
+    last = stages * 128;
+    kofs = rot * 128;
+    // piece p: rows 8 p .., lane l the chunk (l & 7) ^ ((row >> 1) & 7) of row l >> 3; a wave's pieces are an even number apart
+    const int ch = (lane & 7) ^ (lrow >> 1);
 #pragma unroll
-  for (int i = 0; i < LX; ++i) {
-    const int row = (w * LX + i) * 8 + lrow;
-    xsrc[i] = X + (long)min(row, M - 1) * ldx + kbase + ((lch ^ wsz(row)) * 8);
-  }
+    for (int i = 0; i < MW; ++i) xo[i] = (unsigned)(8 * (4 * i + w) + lrow) * (unsigned)(ldx * 2) + (unsigned)((ch ^ (4 * (w & 1))) * 16);
 #pragma unroll
-  for (int i = 0; i < LW; ++i) {
-    const int row = (w * LW + i) * 8 + lrow;
-    wsrc[i] = W + min(wrow(row), n_rows - 1) * K + kbase + ((lch ^ wsz(row)) * 8);
-  }
-  auto issue_x = [&](int st) {
-    unsigned char* base = smem + (st % NS) * SB;
-    const int k = (st + rot < nst ? st + rot : st + rot - nst) * 64;
-#pragma unroll
-    for (int i = 0; i < LX; ++i)
-      __builtin_amdgcn_global_load_lds((gbl_void_ptr)(xsrc[i] + k),
-                                       (lds_void_ptr)(base + (w * LX + i) * 8 * 128), 16, 0, 0);
-  };
-  auto issue_w = [&](int st) {
-    unsigned char* base = smem + (st % NS) * SB;
-    const int k = (st + rot < nst ? st + rot : st + rot - nst) * 64;
-#pragma unroll
-    for (int i = 0; i < LW; ++i)
-      __builtin_amdgcn_global_load_lds((gbl_void_ptr)(wsrc[i] + k),
-                                       (lds_void_ptr)(base + XB + (w * LW + i) * 8 * 128), 16, 0, 2);
-  };
-  auto issue = [&](int st) {
-    issue_x(st);
-    issue_w(st);
-  };
-
-  floatx4 acc[MTW][NT];
-#pragma unroll
-  for (int m = 0; m < MTW; ++m)
-#pragma unroll
-    for (int n = 0; n < NT; ++n) acc[m][n] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-  auto compute = [&](int st) {
-    const unsigned char* base = smem + (st % NS) * SB;
+    for (int i = 0; i < PW; ++i)
+      wo[i] = (unsigned)(8 * (WSTEP * (SWIGLU ? i % (PW / 2) : i) + q) + lrow) * (unsigned)(K * 2) + (unsigned)((ch ^ (4 * (q & 1))) * 16);
+    const unsigned lds0 = (unsigned)reinterpret_cast<uintptr_t>((lds_void_ptr)smem);
+    ldsx = lds0 + w * 1024;
+    ldsw = lds0 + NSX * XB + q * 1024;
+    const int wr = w >> 1, wc = w & 1;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const int c = 4 * h + g;
-      short8 a[MTW], b[NT];
-#pragma unroll
-      for (int m = 0; m < MTW; ++m) {
-        const int row = w * (4 * MT) + 16 * m + r;
-        a[m] = *reinterpret_cast<const short8*>(base + row * 128 + ((c ^ wsz(row)) << 4));
-      }
-#pragma unroll
-      for (int n = 0; n < NT; ++n) {
-        const int row = 16 * n + r;
-        b[n] = *reinterpret_cast<const short8*>(base + XB + row * 128 + ((c ^ wsz(row)) << 4));
-      }
-      // W fragment as the MFMA's A operand: the lane ends with ONE output row and 4
-      // consecutive columns, so the epilogue writes 16 B (f32 partials) / 8 B (bf16) per lane
-      // -- a quarter of the store instructions of a column-per-lane image (the store tail
-      // of a short weight-streaming kernel is issue-bound)
-#pragma unroll
-      for (int m = 0; m < MTW; ++m)
-#pragma unroll
-        for (int n = 0; n < NT; ++n)
-          acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[n], a[m], acc[m][n], 0, 0, 0);
+      const unsigned b = lds0 + (((4 * h + g) ^ wsz(r)) << 4) + r * 128;
+      bx[h] = b + wr * (8 * MT) * 128;
+      bw[h] = b + NSX * XB + wc * (SWIGLU ? BN / 4 : BN / 2) * 128;
     }
-  };
-
-  if constexpr (PRO != 0) {
-    // W of the first stages streams in while the workgroup computes its X slice; then X's
-    // first stages come from the rows just written (every wave waits for its own DMAs, the
-    // loop's barrier for everyone's)
 #pragma unroll
-    for (int p = 0; p < NS - 1; ++p)
-      if (p < nst) issue_w(p);
-    ws_prologue<PRO>(pr, M, K, kbase, ks);
-    wait_vmcnt<0>();
-    __syncthreads();
+    for (int m = 0; m < MW; ++m)
 #pragma unroll
-    for (int p = 0; p < NS - 1; ++p)
-      if (p < nst) issue_x(p);
-    wait_vmcnt<0>();
-  } else {
-#pragma unroll
-    for (int p = 0; p < NS - 1; ++p)
-      if (p < nst) issue(p);
+      for (int n = 0; n < NW; ++n) acc[m][n] = floatx4{0.f, 0.f, 0.f, 0.f};
   }
-  for (int st = 0; st < nst; ++st) {
-    // stage st landed (this wave's DMAs); later stages may stay in flight
-    wait_ahead<L, NS>(min(NS - 2, nst - 1 - st));
-    __builtin_amdgcn_s_barrier();  // ... for every wave; and buffer (st-1)%NS is free
-    __builtin_amdgcn_sched_barrier(0);
-    if (st + NS - 1 < nst) issue(st + NS - 1);
-    __builtin_amdgcn_sched_barrier(0);
-    compute(st);
+  // piece i of the stage to request next, into the ring slot at `slot`
+  template <int I>
+  LK_DEVICE void dma_x(unsigned slot) {
+    asm volatile("s_add_u32 m0, %3, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+                 ::"v"(xo[I]), "s"(xs), "s"(kofs), "s"(ldsx + slot), "i"(I * 4096) : "memory", "scc");
   }
+  template <int I>
+  LK_DEVICE void dma_w(unsigned slot) {
+    asm volatile("s_add_u32 m0, %3, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen nt lds"
+                 ::"v"(wo[I]), "s"(ws[up(I)]), "s"(kofs), "s"(ldsw + slot), "i"(I * WSTEP * 1024) : "memory", "scc");
+  }
+  LK_DEVICE void advance() {   // to the stage after `at`: past the last no descriptor has a range
+    kofs = kofs + 128 == last ? 0 : kofs + 128;
+    if (++at == nst) xs.z = ws[0].z = ws[1].z = 0;
+  }
+  template <bool X, bool W>
+  LK_DEVICE void request(unsigned xslot, unsigned wslot) {
+    if constexpr (X) ws_unroll<MW>([&](auto j_t) { dma_x<decltype(j_t)::value>(xslot); });
+    if constexpr (W) ws_unroll<PW>([&](auto j_t) { dma_w<decltype(j_t)::value>(wslot); });
+  }
+  // fragment j of the stage whose reads start at ax / aw: the first half of K, then the second; X, then W
+  template <int P>
+  LK_DEVICE void read(int j, const unsigned (&ax)[2], const unsigned (&aw)[2]) {
+    const int h = j / L, q = j % L;
+    if (q < MW) fx[P][h][q] = *reinterpret_cast<lds_frag_t>(ax[h] + q * 2048);
+    else fw[P][h][q - MW] = *reinterpret_cast<lds_frag_t>(aw[h] + col(q - MW) * 128);
+  }
+  struct Slots { unsigned x, w; };
+  LK_DEVICE static void step(Slots& s) {
+    s.x = s.x + XB == (unsigned)(NSX * XB) ? 0 : s.x + XB;
+    s.w = s.w + WB == (unsigned)(NSW * WB) ? 0 : s.w + WB;
+  }
+  LK_DEVICE void addresses(Slots s, unsigned (&ax)[2], unsigned (&aw)[2]) const {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {   // (opaque: the rest of every address stays the instruction's immediate)
+      ax[h] = bx[h] + s.x;
+      aw[h] = bw[h] + s.w;
+      asm volatile("" : "+v"(ax[h]), "+v"(aw[h]));
+    }
+  }
+  // stage in register set P; cur: its slots, requested again; nxt: the next one's, read into the other set
+  template <int P>
+  LK_DEVICE void stage(Slots cur, Slots nxt) {
+    unsigned ax[2], aw[2];
+    addresses(nxt, ax, aw);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0xF | (0x3 << 14) | (0x7 << 4));   // lgkmcnt(0)
+    wait_vmcnt<(NSX - 2) * OPS>();
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    ws_unroll<NM>([&](auto i_t) {
+      constexpr int i = decltype(i_t)::value, h = i / (MW * NW), m = i % MW, n = i / MW % NW;
+      // the reads over the first two thirds of the MFMAs, the requests over all
+#pragma unroll
+      for (int j = 0; j < NR; ++j)
+        if (j * NM * 2 / (NR * 3) == i) read<P ^ 1>(j, ax, aw);
+      ws_unroll<OPS>([&](auto j_t) {
+        constexpr int j = decltype(j_t)::value;
+        if constexpr (j * NM / OPS + (NM > OPS ? 1 : 0) == i) {
+          if constexpr (j < MW) dma_x<j>(cur.x);
+          else dma_w<j - MW>(cur.w);
+        }
+      });
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (LOADERS) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc[m][n]) : "v"(fw[P][h][n]), "v"(fx[P][h][m]));
+      else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[m][n]) : "v"(fw[P][h][n]), "v"(fx[P][h][m]));
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    advance();
+  }
+  // the first NSX stages have been requested, in order, into the slots from 0 on (W's by the loaders)
+  LK_DEVICE void walk() {
+    wait_vmcnt<(NSX - 1) * OPS>();
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    Slots cur{0, 0}, nxt{0, 0};
+    unsigned ax[2], aw[2];
+    addresses(cur, ax, aw);
+#pragma unroll
+    for (int j = 0; j < NR; ++j) read<0>(j, ax, aw);
+    step(nxt);
+    for (int st = 0;; st += 2) {
+      stage<0>(cur, nxt);
+      cur = nxt;
+      step(nxt);
+      if (st + 1 >= nst) break;
+      stage<1>(cur, nxt);
+      cur = nxt;
+      step(nxt);
+      if (st + 2 >= nst) break;
+    }
+    wait_vmcnt<0>();   // the last requests land before the workgroup's LDS is used again or released
+    // (the MFMAs are asm: the wait between the last ones and the first use of their results is ours)
+    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" ::: "memory");
+#pragma unroll
+    for (int m = 0; m < MW; ++m)
+#pragma unroll
+      for (int n = 0; n < NW; ++n) {
+        if constexpr (LOADERS) asm volatile("" : "+v"(acc[m][n]));
+        else asm volatile("" : "+a"(acc[m][n]));
+      }
+  }
+  // a loader wave's part: as many barriers as walk() has
+  LK_DEVICE void load() {
+    for (int p = 0; p < NSW; ++p) {
+      request<false, true>(0, p * WB);
+      advance();
+    }
+    wait_vmcnt<(NSW - 1) * PW>();
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    unsigned slot = 0;
+    for (int st = 0; st < nst; ++st) {
+      wait_vmcnt<(NSW - 2) * PW>();   // the next stage has landed
+      __builtin_amdgcn_s_barrier();   // ... and this one is in everyone's registers
+      __builtin_amdgcn_sched_barrier(0);
+      request<false, true>(0, slot);
+      advance();
+      slot = slot + WB == (unsigned)(NSW * WB) ? 0 : slot + WB;
+    }
+    wait_vmcnt<0>();
+  }
+};
 
-  // ---- epilogue straight from the accumulators: lane holds row 16m + r of its wave's rows,
-  // tile columns 16n + 4g .. +3
+// The epilogue of tile t (split s of `splits`), straight from the accumulators (W fragment as the MFMA's A operand): a lane holds row
+// 16 m + r of its wave's rows, 4 consecutive columns 16 n + 4 g .. + 3, so it writes 16 B (f32 partials) / 8 B (bf16).
+template <int MT, int BN, bool SWIGLU, bool TAIL>
+LK_DEVICE void ws_store(const floatx4 (&acc)[MT / 2][BN / 32], int t, int s, int M, int splits, int swiglu_I, bf16_t* __restrict__ out, long ldo,
+                        float* __restrict__ part, long part_ld, long n_rows) {
+  constexpr int MW = MT / 2, NW = BN / 32;
+  const long first = (long)t * (SWIGLU ? BN / 2 : BN);
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, g = lane >> 4, wr = w >> 1, wc = w & 1;
   const bool split = part != nullptr;
   const bool part_vec = split && part_ld % 4 == 0 && reinterpret_cast<uintptr_t>(part) % 16 == 0;
   // (fused tail: the partial slabs through a buffer resource, written past L1 / L2)
   const __amdgpu_buffer_rsrc_t tprs = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)part, (short)0, (int)min((long)(K / ks) * M * part_ld * 4, 0x7FFFFFF0L), 0x00020000);
+      (void*)part, (short)0, (int)min((long)splits * M * part_ld * 4, 0x7FFFFFF0L), 0x00020000);
   const bool out_vec = ldo % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0;
 #pragma unroll
-  for (int m = 0; m < MTW; ++m) {
-    const int row = w * (4 * MT) + 16 * m + r;
+  for (int m = 0; m < MW; ++m) {
+    const int row = wr * (8 * MT) + 16 * m + r;
     if (row >= M) continue;
     if (SWIGLU && !split) {
 #pragma unroll
-      for (int n = 0; n < NT / 2; ++n) {
+      for (int n = 0; n < NW / 2; ++n) {
         float y[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) y[i] = rbf(silu_f(rbf(acc[m][n][i]))) * rbf(acc[m][n + NT / 2][i]);
-        bf16_t* dst = out + (long)row * ldo + (long)t * (BN / 2) + 16 * n + 4 * g;
+        for (int i = 0; i < 4; ++i) y[i] = rbf(silu_f(rbf(acc[m][n][i]))) * rbf(acc[m][n + NW / 2][i]);
+        bf16_t* dst = out + (long)row * ldo + first + wc * (BN / 4) + 16 * n + 4 * g;
         if (out_vec) {
           uint2 pk;
           pk.x = pack_bf2(y[0], y[1]);
@@ -706,54 +763,102 @@ __global__ __launch_bounds__(256, 1) void wsgemm_kernel(const bf16_t* __restrict
           for (int i = 0; i < 4; ++i) dst[i] = f2bf(y[i]);
         }
       }
-    } else if (split) {
-#pragma unroll
-      for (int n = 0; n < NT; ++n) {
-        // 4 consecutive tile rows stay inside one half of a SwiGLU tile: contiguous W rows
-        const long col = wrow(16 * n + 4 * g);
-        float* dst = part + (long)s * M * part_ld + (long)row * part_ld + col;
-        if (TAIL) {  // fused tail: through to memory (full 16-B tiles: checked on the host)
-          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4_t, acc[m][n]), tprs,
-                                                 (unsigned)(((long)s * M + row) * part_ld + col) * 4u, 0, kSysCoherent);
-        } else if (part_vec && col + 3 < n_rows) {
-          *reinterpret_cast<floatx4*>(dst) = acc[m][n];
-        } else {
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (col + i < n_rows) dst[i] = acc[m][n][i];
-        }
-      }
     } else {
 #pragma unroll
-      for (int n = 0; n < NT; ++n) {
-        const long col = (long)t * BN + 16 * n + 4 * g;
-        bf16_t* dst = out + (long)row * ldo + col;
-        if (out_vec && col + 3 < n_rows) {
-          uint2 pk;
-          pk.x = pack_bf2(acc[m][n][0], acc[m][n][1]);
-          pk.y = pack_bf2(acc[m][n][2], acc[m][n][3]);
-          *reinterpret_cast<uint2*>(dst) = pk;
-        } else {
+      for (int n = 0; n < NW; ++n) {
+        // first of this lane's 4 columns (W rows): a SwiGLU tile's second half are the up rows
+        const long col = first + (SWIGLU ? wc * (BN / 4) + 16 * (n % (NW / 2)) + (n < NW / 2 ? 0 : swiglu_I) : wc * (BN / 2) + 16 * n) + 4 * g;
+        const floatx4 v = acc[m][n];
+        if (split) {
+          float* dst = part + (long)s * M * part_ld + (long)row * part_ld + col;
+          if (TAIL) {  // fused tail: through to memory (full 16-B tiles: checked on the host)
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4_t, v), tprs,
+                                                   (unsigned)(((long)s * M + row) * part_ld + col) * 4u, 0, kSysCoherent);
+          } else if (part_vec && col + 3 < n_rows) {
+            *reinterpret_cast<floatx4*>(dst) = v;
+          } else {
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (col + i < n_rows) dst[i] = f2bf(acc[m][n][i]);
+            for (int i = 0; i < 4; ++i)
+              if (col + i < n_rows) dst[i] = v[i];
+          }
+        } else {
+          bf16_t* dst = out + (long)row * ldo + col;
+          if (out_vec && col + 3 < n_rows) {
+            uint2 pk;
+            pk.x = pack_bf2(v[0], v[1]);
+            pk.y = pack_bf2(v[2], v[3]);
+            *reinterpret_cast<uint2*>(dst) = pk;
+          } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              if (col + i < n_rows) dst[i] = f2bf(v[i]);
+          }
         }
       }
     }
   }
+}
+
+template <int MT, int BN, bool SWIGLU, bool TAIL, int PRO = 0>
+__global__ __launch_bounds__(256, 1) void wsgemm_kernel(const bf16_t* __restrict__ X, long ldx,
+                                                        const bf16_t* __restrict__ W, int M, int K, int ks,
+                                                        int n_tiles, int swiglu_I, bf16_t* __restrict__ out,
+                                                        long ldo, float* __restrict__ part, long part_ld,
+                                                        long n_rows, int rot_mul, WsTail tl, WsPro pr) {
+  // n_rows: valid W rows (the last column tile may be partial: kNN over a corpus of
+  // any size); rows past them read as zeros, stores are masked
+  constexpr int NS = ws_stages_pro(MT, BN, PRO);  // ring depth: as many stages as 160 KB of LDS holds
+  using Walk = WsWalk<MT, BN, SWIGLU, NS, NS, 0>;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+
+  const int t = blockIdx.x % n_tiles, s = blockIdx.x / n_tiles;
+  const long kbase = (long)s * ks;
+  const int nst = ks / 64;
+  // K-step rotation: column tile t starts its K walk at step (t * rot_mul) % nst, so the
+  // blocks streaming at the same moment read different 128-B columns of X (every block
+  // reads all of X: in lockstep they would all hit the same few L2 channels)
+  const int rot = rot_mul ? (int)(((long)t * rot_mul) % nst) : 0;
+  const long first = (long)t * (SWIGLU ? BN / 2 : BN);   // the tile's first W row (SwiGLU: gate row; up: + I)
+  Walk k;
+  k.begin(smem, X, ldx, W + first * K, W + (first + swiglu_I) * K, SWIGLU ? (long)BN / 2 : min(n_rows - first, (long)BN), M, K, kbase, nst, rot);
+  if constexpr (PRO != 0) {
+    // W of the first stages streams in while the workgroup computes its X slice; then X's
+    // first stages come from the rows just written (every wave waits for its own DMAs, the
+    // walk's barrier for everyone's)
+    const Walk k0 = k;
+    for (int p = 0; p < NS; ++p) {
+      k.template request<false, true>(0, p * Walk::WB);
+      k.advance();
+    }
+    ws_prologue<PRO>(pr, M, K, kbase, ks);
+    wait_vmcnt<0>();
+    __syncthreads();
+    k = k0;
+    for (int p = 0; p < NS; ++p) {
+      k.template request<true, false>(p * Walk::XB, 0);
+      k.advance();
+    }
+    wait_vmcnt<0>();
+  } else {
+    for (int p = 0; p < NS; ++p) {
+      k.template request<true, true>(p * Walk::XB, p * Walk::WB);
+      k.advance();
+    }
+  }
+  k.walk();
+
+  ws_store<MT, BN, SWIGLU, TAIL>(k.acc, t, s, M, K / ks, swiglu_I, out, ldo, part, part_ld, n_rows);
   if constexpr (TAIL) ws_tail(tl, part, M, part_ld, K / ks, t, n_tiles, smem);
 }
 
 // ---------------------------------------------------------------------------------
-// Loader-wave variant of the weight-streaming GEMM ("lw").  s_waitcnt vmcnt retires a wave's
-// vector-memory ops in issue order, so in wsgemm_kernel -- X and W of a stage issued together by
-// the same waves -- the W prefetch can run only as far ahead as the shared ring, and at M 192-256
-// (X stages twice the W stages) that is 1-2 stages: the W stream ran 3.0-3.9 TB/s, in proportion
-// to the W bytes in flight per CU.  Here the W stream has waves of its own (2 loader waves, their
-// own vmcnt): 4 compute waves stage X through a short ring (L2-resident, 2-3 stages) and compute;
-// the loader waves keep NSW - 1 W stages (all the remaining LDS) in flight; one s_barrier per
-// stage joins them.  Same tile, swizzles, K rotation and epilogue as wsgemm_kernel.
-constexpr int lw_nsx(int MT) { return MT <= 8 ? 3 : 2; }
+// Loader-wave variant of the weight-streaming GEMM ("lw").  s_waitcnt vmcnt retires a wave's vector-memory ops in issue order, so where the
+// same waves request X and W, the W prefetch runs only as far ahead as their common ring.  Here the W stream has waves of its own (2 loader
+// waves, their own vmcnt): 4 compute waves stage X through a short ring (L2-resident, 3 stages) and compute;
+// the loader waves keep the remaining LDS of W stages in flight.  Same walk, tile, K rotation and epilogue, so the same bits.  Up to 128 rows: it is
+// the faster one by up to 3 % where few workgroups of 128 columns leave CUs idle (120 x 4096 x 4096 in 4 parts of K 15.0 -> 14.7 us), and
+// beyond, two sets of fragments for six waves do not fit the registers (the one ring runs).
+constexpr int lw_nsx(int) { return 3; }
 constexpr int lw_nsw(int MT, int BN) {
   const int n = (163840 - lw_nsx(MT) * 16 * MT * 128) / (BN * 128);
   return n > 12 ? 12 : n;
@@ -765,186 +870,25 @@ __global__ __launch_bounds__(384, 1) void wsgemm_lw_kernel(const bf16_t* __restr
                                                            int n_tiles, int swiglu_I, bf16_t* __restrict__ out,
                                                            long ldo, float* __restrict__ part, long part_ld,
                                                            long n_rows, int rot_mul, WsTail tl) {
-  constexpr int ROWS = 16 * MT;
-  constexpr int MTW = MT / 4;
-  constexpr int NT = BN / 16;
-  constexpr int XB = ROWS * 128;
-  constexpr int WB = BN * 128;
-  constexpr int NSX = lw_nsx(MT);
-  constexpr int NSW = lw_nsw(MT, BN);
-  constexpr int LX = ROWS / 32;  // X glds per compute wave per stage (4 waves x 8 rows)
-  constexpr int LW = BN / 16;    // W glds per loader wave per stage (2 waves x 8 rows)
-  static_assert(NSW >= 3, "W ring");
+  using Walk = WsWalk<MT, BN, SWIGLU, lw_nsx(MT), lw_nsw(MT, BN), 2>;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  unsigned char* xring = smem;
-  unsigned char* wring = smem + NSX * XB;
-
   const int t = blockIdx.x % n_tiles, s = blockIdx.x / n_tiles;
-  const int lane = threadIdx.x & 63;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const bool loader = w >= 4;
-  const int r = lane & 15, g = lane >> 4;
   const long kbase = (long)s * ks;
   const int nst = ks / 64;
   const int rot = rot_mul ? (int)(((long)t * rot_mul) % nst) : 0;
-  auto kof = [&](int st) { return (st + rot < nst ? st + rot : st + rot - nst) * 64; };
-
-  auto wrow = [&](int row) -> long {
-    if constexpr (SWIGLU) {
-      return row < BN / 2 ? (long)t * (BN / 2) + row : (long)swiglu_I + (long)t * (BN / 2) + row - BN / 2;
-    } else {
-      return (long)t * BN + row;
-    }
-  };
-  const int lrow = lane >> 3, lch = lane & 7;
-
-  floatx4 acc[MTW][NT];
-#pragma unroll
-  for (int m = 0; m < MTW; ++m)
-#pragma unroll
-    for (int n = 0; n < NT; ++n) acc[m][n] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-  if (loader) {
-    const int lw = w - 4;
-    const bf16_t* wsrc[LW];
-#pragma unroll
-    for (int i = 0; i < LW; ++i) {
-      const int row = (lw * LW + i) * 8 + lrow;
-      wsrc[i] = W + min(wrow(row), n_rows - 1) * K + kbase + ((lch ^ wsz(row)) * 8);
-    }
-    auto issue_w = [&](int st) {
-      unsigned char* base = wring + (st % NSW) * WB;
-#pragma unroll
-      for (int i = 0; i < LW; ++i)
-        __builtin_amdgcn_global_load_lds((gbl_void_ptr)(wsrc[i] + kof(st)),
-                                         (lds_void_ptr)(base + (lw * LW + i) * 8 * 128), 16, 0, 2);
-    };
-#pragma unroll
-    for (int p = 0; p < NSW - 1; ++p)
-      if (p < nst) issue_w(p);
-    for (int st = 0; st < nst; ++st) {
-      wait_ahead<LW, NSW>(min(NSW - 2, nst - 1 - st));  // W(st) landed, later stages in flight
-      __builtin_amdgcn_s_barrier();                      // ... and ring slot (st - 1) % NSW is free
-      __builtin_amdgcn_sched_barrier(0);
-      if (st + NSW - 1 < nst) issue_w(st + NSW - 1);
-    }
-    // the epilogue is the compute waves' (no barrier after the loop); a fused tail needs
-    // every wave again
+  const long first = (long)t * (SWIGLU ? BN / 2 : BN);
+  Walk k;
+  k.begin(smem, X, ldx, W + first * K, W + (first + swiglu_I) * K, SWIGLU ? (long)BN / 2 : min(n_rows - first, (long)BN), M, K, kbase, nst, rot);
+  if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) >= 4) {
+    k.load();
   } else {
-
-  const bf16_t* xsrc[LX];
-#pragma unroll
-  for (int i = 0; i < LX; ++i) {
-    const int row = (w * LX + i) * 8 + lrow;
-    xsrc[i] = X + (long)min(row, M - 1) * ldx + kbase + ((lch ^ wsz(row)) * 8);
-  }
-  auto issue_x = [&](int st) {
-    unsigned char* base = xring + (st % NSX) * XB;
-#pragma unroll
-    for (int i = 0; i < LX; ++i)
-      __builtin_amdgcn_global_load_lds((gbl_void_ptr)(xsrc[i] + kof(st)),
-                                       (lds_void_ptr)(base + (w * LX + i) * 8 * 128), 16, 0, 0);
-  };
-  auto compute = [&](int st) {
-    const unsigned char* xb = xring + (st % NSX) * XB;
-    const unsigned char* wb = wring + (st % NSW) * WB;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int c = 4 * h + g;
-      short8 a[MTW], b[NT];
-#pragma unroll
-      for (int m = 0; m < MTW; ++m) {
-        const int row = w * (4 * MT) + 16 * m + r;
-        a[m] = *reinterpret_cast<const short8*>(xb + row * 128 + ((c ^ wsz(row)) << 4));
-      }
-#pragma unroll
-      for (int n = 0; n < NT; ++n) {
-        const int row = 16 * n + r;
-        b[n] = *reinterpret_cast<const short8*>(wb + row * 128 + ((c ^ wsz(row)) << 4));
-      }
-#pragma unroll
-      for (int m = 0; m < MTW; ++m)
-#pragma unroll
-        for (int n = 0; n < NT; ++n)
-          acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[n], a[m], acc[m][n], 0, 0, 0);
+    for (int p = 0; p < lw_nsx(MT); ++p) {
+      k.template request<true, false>(p * Walk::XB, 0);
+      k.advance();
     }
-  };
-#pragma unroll
-  for (int p = 0; p < NSX - 1; ++p)
-    if (p < nst) issue_x(p);
-  for (int st = 0; st < nst; ++st) {
-    wait_ahead<LX, NSX>(min(NSX - 2, nst - 1 - st));  // X(st) landed (the W side waits in the loaders)
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    if (st + NSX - 1 < nst) issue_x(st + NSX - 1);
-    __builtin_amdgcn_sched_barrier(0);
-    compute(st);
+    k.walk();
+    ws_store<MT, BN, SWIGLU, TAIL>(k.acc, t, s, M, K / ks, swiglu_I, out, ldo, part, part_ld, n_rows);
   }
-
-  // ---- epilogue (as wsgemm_kernel): lane holds row 16m + r of its wave's rows, tile columns
-  // 16n + 4g .. +3
-  const bool split = part != nullptr;
-  const bool part_vec = split && part_ld % 4 == 0 && reinterpret_cast<uintptr_t>(part) % 16 == 0;
-  // (fused tail: the partial slabs through a buffer resource, written past L1 / L2)
-  const __amdgpu_buffer_rsrc_t tprs = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)part, (short)0, (int)min((long)(K / ks) * M * part_ld * 4, 0x7FFFFFF0L), 0x00020000);
-  const bool out_vec = ldo % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0;
-#pragma unroll
-  for (int m = 0; m < MTW; ++m) {
-    const int row = w * (4 * MT) + 16 * m + r;
-    if (row >= M) continue;
-    if (SWIGLU && !split) {
-#pragma unroll
-      for (int n = 0; n < NT / 2; ++n) {
-        float y[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) y[i] = rbf(silu_f(rbf(acc[m][n][i]))) * rbf(acc[m][n + NT / 2][i]);
-        bf16_t* dst = out + (long)row * ldo + (long)t * (BN / 2) + 16 * n + 4 * g;
-        if (out_vec) {
-          uint2 pk;
-          pk.x = pack_bf2(y[0], y[1]);
-          pk.y = pack_bf2(y[2], y[3]);
-          *reinterpret_cast<uint2*>(dst) = pk;
-        } else {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) dst[i] = f2bf(y[i]);
-        }
-      }
-    } else if (split) {
-#pragma unroll
-      for (int n = 0; n < NT; ++n) {
-        const long col = wrow(16 * n + 4 * g);
-        float* dst = part + (long)s * M * part_ld + (long)row * part_ld + col;
-        if (TAIL) {  // fused tail: through to memory
-          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4_t, acc[m][n]), tprs,
-                                                 (unsigned)(((long)s * M + row) * part_ld + col) * 4u, 0, kSysCoherent);
-        } else if (part_vec && col + 3 < n_rows) {
-          *reinterpret_cast<floatx4*>(dst) = acc[m][n];
-        } else {
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (col + i < n_rows) dst[i] = acc[m][n][i];
-        }
-      }
-    } else {
-#pragma unroll
-      for (int n = 0; n < NT; ++n) {
-        const long col = (long)t * BN + 16 * n + 4 * g;
-        bf16_t* dst = out + (long)row * ldo + col;
-        if (out_vec && col + 3 < n_rows) {
-          uint2 pk;
-          pk.x = pack_bf2(acc[m][n][0], acc[m][n][1]);
-          pk.y = pack_bf2(acc[m][n][2], acc[m][n][3]);
-          *reinterpret_cast<uint2*>(dst) = pk;
-        } else {
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (col + i < n_rows) dst[i] = f2bf(acc[m][n][i]);
-        }
-      }
-    }
-  }
-  }  // (compute waves)
   if constexpr (TAIL) ws_tail(tl, part, M, part_ld, K / ks, t, n_tiles, smem);  // every wave: it has barriers
 }
 
@@ -956,7 +900,7 @@ int g_ws_rot_mul = -1;
 template <int MT, int BN, bool SWIGLU>
 void launch_ws(const bf16_t* x, long ldx, const bf16_t* w, int M, int K, int ks, int S, int n_tiles, int I,
                bf16_t* out, long ldo, float* part, long part_ld, long n_rows, hipStream_t st, const WsTail& tl) {
-  constexpr size_t lds = (size_t)ws_stages(MT, BN) * (16 * MT * 128 + BN * 128);
+  constexpr size_t lds = (size_t)ws_stages_pro(MT, BN, 0) * (16 * MT * 128 + BN * 128);
   // (the fused-tail instantiation only where a tail runs: the plain kernel keeps its registers)
   auto kern = tl.kind ? wsgemm_kernel<MT, BN, SWIGLU, true> : wsgemm_kernel<MT, BN, SWIGLU, false>;
   if (tl.kind) LK_SET_MAX_LDS((wsgemm_kernel<MT, BN, SWIGLU, true>), (int)lds);
@@ -991,16 +935,23 @@ void launch_ws_lw(const bf16_t* x, long ldx, const bf16_t* w, int M, int K, int 
   kern<<<n_tiles * S, 384, lds, st>>>(x, ldx, w, M, K, ks, n_tiles, I, out, ldo, part, part_ld, n_rows, rot_mul, tl);
 }
 
+// a tile's rows are reached by 32-bit offsets from its first: up to 256 of X, up to 128 of W
+bool ws_too_far(int M, long ldx, int K) { return M * ldx * 2 >= 0xFFFFFF00L || (long)K * 256 >= 0xFFFFFF00L; }
+
 template <bool SWIGLU>
 int dispatch_ws(int MT, int BN, const bf16_t* x, long ldx, const bf16_t* w, int M, int K, int ks, int S,
                 int n_tiles, int I, bf16_t* out, long ldo, float* part, long part_ld, hipStream_t st,
                 long n_rows = 1L << 40, int variant = 0, const WsTail& tl = WsTail{}) {
+  if (ws_too_far(M, ldx, K)) return -1;
 #define LK_WS(mt, bn)                                                                                          \
   if (MT == mt && BN == bn) {                                                                                  \
-    if (variant == 1)                                                                                          \
-      launch_ws_lw<mt, bn, SWIGLU>(x, ldx, w, M, K, ks, S, n_tiles, I, out, ldo, part, part_ld, n_rows, st, tl); \
-    else                                                                                                       \
-      launch_ws<mt, bn, SWIGLU>(x, ldx, w, M, K, ks, S, n_tiles, I, out, ldo, part, part_ld, n_rows, st, tl);    \
+    if constexpr (mt <= 8) {                                                                                   \
+      if (variant == 1) {                                                                                      \
+        launch_ws_lw<mt, bn, SWIGLU>(x, ldx, w, M, K, ks, S, n_tiles, I, out, ldo, part, part_ld, n_rows, st, tl); \
+        return 0;                                                                                              \
+      }                                                                                                        \
+    }                                                                                                          \
+    launch_ws<mt, bn, SWIGLU>(x, ldx, w, M, K, ks, S, n_tiles, I, out, ldo, part, part_ld, n_rows, st, tl);    \
     return 0;                                                                                                  \
   }
   LK_WS(4, 64) LK_WS(4, 128) LK_WS(8, 64) LK_WS(8, 128) LK_WS(12, 64) LK_WS(12, 128) LK_WS(16, 64) LK_WS(16, 128)
@@ -1155,7 +1106,7 @@ int lk_wsgemm_pro(int kind, bf16_t* x, const bf16_t* w, int M, int N, int K, int
                   bf16_t* out, long ldo, float* part, const float* pp, int pS, const bf16_t* res, bf16_t* res_out,
                   long rs, const bf16_t* gamma, float eps, const float* po, const float* pml, const int* ctx, int Hq,
                   int D, int max_splits, int split, hipStream_t st) {
-  if (M < 1 || M > 64 || S < 1 || K % (S * 64) || !x || (BN != 64 && BN != 128 && (BN != 96 || swiglu))) return -1;
+  if (M < 1 || M > 64 || S < 1 || K % (S * 64) || !x || ws_too_far(M, K, K) || (BN != 64 && BN != 128 && (BN != 96 || swiglu))) return -1;
   const int per = swiglu ? BN / 2 : BN;
   if (swiglu ? (N % 2 || (N / 2) % per) : N % BN) return -1;
   if ((S > 1 && !part) || (S == 1 && !out)) return -1;

@@ -1169,6 +1169,32 @@ def test_ws_loader_wave_variant_bit_identical(hip, M, NK, swiglu):
         hip.ws_set_variant(M, N, K, swiglu, -1)
 
 
+@pytest.mark.parametrize("M,N,K,swiglu,bn,S", [(1, 256, 64, False, 64, 1), (33, 384, 128, False, 96, 2), (64, 256, 320, True, 128, 1),
+                                              (65, 384, 192, False, 128, 1), (128, 512, 704, True, 64, 1), (129, 192, 512, False, 96, 4),
+                                              (192, 512, 576, True, 128, 3), (193, 256, 1088, False, 128, 1), (256, 256, 384, False, 64, 3)])
+@pytest.mark.parametrize("variant", [0, 1])
+def test_ws_walk_edges(hip, M, N, K, swiglu, bn, S, variant):
+    """The weight-streaming walk where it can go wrong: one stage, fewer stages than the ring has, odd and even numbers of them, every
+    row tile's first and last rows, rows far apart.  bf16 inputs, f32 sums: one rounding of the result, at most 2^-9 of it; SwiGLU
+    also rounds its factors g, u and silu(g), and g's rounding moves silu(g) by at most 1.1 times as much (twice that allowed)."""
+    torch.manual_seed(M + N + K)
+    x = torch.randn(M, K, device=DEV, dtype=torch.bfloat16)
+    w = torch.randn(N, K, device=DEV, dtype=torch.bfloat16) / K ** 0.5
+    far = torch.empty(M * 17_000_000 if M == 129 else M * (K + 64), device=DEV, dtype=torch.bfloat16)
+    strided = far.as_strided((M, K), (far.numel() // M, 1)).copy_(x)
+    y = x.double() @ w.double().t()
+    want = torch.nn.functional.silu(y[:, :N // 2]) * y[:, N // 2:] if swiglu else y
+    try:
+        hip.ws_set_variant(M, N, K, swiglu, variant)
+        for a in (x, strided):
+            got = hip.ws_linear(a, w, swiglu, bn, S)
+            err = (got.double() - want).abs()
+            bound = 3 * want.abs() + 1.1 * (y[:, :N // 2] * y[:, N // 2:]).abs() if swiglu else want.abs()
+            assert (err <= 2.0 ** -8 * bound + 1e-5).all(), float(err.max())
+    finally:
+        hip.ws_set_variant(M, N, K, swiglu, -1)
+
+
 def test_invalid_launch_raises(hip):
     """A launch the runtime rejects (2048 threads per workgroup) raises with the HIP error
     instead of returning as if it had run; the next op on the stream still works."""
