@@ -192,6 +192,19 @@ at::Tensor ws_linear(const at::Tensor& x_, const at::Tensor& w, bool swiglu, int
   return out;
 }
 
+// (x w1^T, silu(x wg^T) * (x wu^T)) for w2 = [wg; wu] in one launch (csrc/skinny_gemm.hip ws_beside_kernel)
+std::vector<at::Tensor> ws_beside(const at::Tensor& x_, const at::Tensor& w1, const at::Tensor& w2, int64_t bn) {
+  const at::Tensor x = ws_near(x_);
+  CHECK_CUDA(x); CHECK_BF16(x); CHECK_BF16(w1); CHECK_BF16(w2); CHECK_LASTDIM(x); CHECK_CONTIG(w1); CHECK_CONTIG(w2);
+  TORCH_CHECK(x.dim() == 2 && w1.dim() == 2 && w2.dim() == 2 && x.size(1) == w1.size(1) && x.size(1) == w2.size(1), "x [M,K], w1 [N,K], w2 [2I,K]");
+  check_rows16(x, "x"); check_rows16(w1, "w1"); check_rows16(w2, "w2");
+  const int M = x.size(0), K = x.size(1), N1 = w1.size(0), I = w2.size(0) / 2;
+  TORCH_CHECK(w2.size(0) % 2 == 0, "w2 [2I,K]");
+  at::Tensor out1 = at::empty({M, N1}, x.options()), out2 = at::empty({M, I}, x.options());
+  CHECK_RC(lk_ws_beside(bp(x), x.stride(0), M, K, bp(w1), N1, bp(out1), N1, bp(w2), I, bp(out2), I, (int)bn, cur_stream()), "ws_beside");
+  return {out1, out2};
+}
+
 // few-row GEMM (csrc/rows_gemm.hip): M <= 4,096 rows, any epilogue, one launch.  epi: 0 none, 1 SwiGLU, 2 bias, 3 bias + GELU,
 // 4 bias + ReLU, 5 bias + residual; wide: columns of a workgroup, 0: 16, 1: 32, 2: 64
 at::Tensor rows_linear(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, int64_t epi, int64_t wide,
@@ -2525,6 +2538,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("silu_mul", &silu_mul, "", py::arg("x"), py::arg("out") = py::none());
   m.def("activation_", &activation_);
   m.def("rope_kv_", &rope_kv_);
+  m.def("ws_beside", &ws_beside, "", py::arg("x"), py::arg("w1"), py::arg("w2"), py::arg("bn"));
   m.def("ws_set_rot", [](int64_t r) { lk_wsgemm_set_rot((int)r); });
   m.def("ws_linear_rmsnorm", &ws_linear_rmsnorm, "", py::arg("x"), py::arg("w"), py::arg("residual"),
         py::arg("norm_w"), py::arg("eps"), py::arg("bn") = 0, py::arg("splits") = 0, py::arg("tickets") = py::none());

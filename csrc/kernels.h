@@ -86,6 +86,10 @@ int lk_ws_rmsnorm_fused(const bf16_t* x, long ldx, const bf16_t* w, int M, int N
                         int* tickets, bf16_t* out, long os, bf16_t* residual, long rs, const bf16_t* norm_w, float eps,
                         hipStream_t st);
 
+// out1 [M, N1] = x w1^T and out2 [M, I] = silu(x wg^T) * (x wu^T), w2 = [wg; wu], in one launch; bn: 64 or 128 W rows per workgroup, which
+// N1 and 2 I are multiples of; M <= 128
+int lk_ws_beside(const bf16_t* x, long ldx, int M, int K, const bf16_t* w1, int N1, bf16_t* out1, long ld1, const bf16_t* w2, int I,
+                 bf16_t* out2, long ld2, int bn, hipStream_t st);
 void lk_wsgemm_set_rot(int rot_mul);  // K-step rotation per column tile (0 = off, -1 = policy)
 
 int lk_ws_scores_f32(const bf16_t* x, long ldx, const bf16_t* w, int M, long N, int K, float* out, long ldo,

@@ -851,6 +851,33 @@ __global__ __launch_bounds__(256, 1) void wsgemm_kernel(const bf16_t* __restrict
   if constexpr (TAIL) ws_tail(tl, part, M, part_ld, K / ks, t, n_tiles, smem);
 }
 
+// Two products of one X in one launch: tiles of BN output columns of x w1^T, then tiles of BN / 2 columns of silu(x wg^T) * (x wu^T), each
+// the whole of K.
+template <int MT, int BN, int NS>
+__global__ __launch_bounds__(256, BN == 64 ? 2 : 1) void ws_beside_kernel(const bf16_t* __restrict__ X, long ldx, int M, int K,
+                                                                          const bf16_t* __restrict__ W1, bf16_t* __restrict__ out1, long ld1,
+                                                                          int tiles1, const bf16_t* __restrict__ W2, int I,
+                                                                          bf16_t* __restrict__ out2, long ld2) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  auto tile = [&](auto swiglu_t, int t) {
+    constexpr bool SW = decltype(swiglu_t)::value;
+    using Walk = WsWalk<MT, BN, SW, NS, NS, 0>;
+    const int nst = K / 64;
+    const long first = (long)t * (SW ? BN / 2 : BN);
+    const bf16_t* W = SW ? W2 : W1;
+    Walk k;
+    k.begin(smem, X, ldx, W + first * K, W + (first + I) * K, SW ? BN / 2 : BN, M, K, 0, nst, (int)((long)t * 5 % nst));
+    for (int p = 0; p < NS; ++p) {
+      k.template request<true, true>(p * Walk::XB, p * Walk::WB);
+      k.advance();
+    }
+    k.walk();
+    ws_store<MT, BN, SW, false>(k.acc, t, 0, M, 1, I, SW ? out2 : out1, SW ? ld2 : ld1, nullptr, 0, 1L << 40);
+  };
+  if ((int)blockIdx.x < tiles1) tile(std::false_type{}, blockIdx.x);
+  else tile(std::true_type{}, blockIdx.x - tiles1);
+}
+
 // ---------------------------------------------------------------------------------
 // Loader-wave variant of the weight-streaming GEMM ("lw").  s_waitcnt vmcnt retires a wave's vector-memory ops in issue order, so where the
 // same waves request X and W, the W prefetch runs only as far ahead as their common ring.  Here the W stream has waves of its own (2 loader
@@ -986,6 +1013,25 @@ int dispatch_mt(int MT, const bf16_t* x, long ldx, const bf16_t* w, int M, int K
 
 }  // namespace
 
+template <int MT, int BN>
+static int launch_beside(const bf16_t* x, long ldx, int M, int K, const bf16_t* w1, int N1, bf16_t* out1, long ld1, const bf16_t* w2, int I,
+                         bf16_t* out2, long ld2, hipStream_t st) {
+  // 64 columns: two workgroups per CU
+  constexpr int SB = (16 * MT + BN) * 128, FIT = (BN == 64 ? 81920 : 163840) / SB, NS = FIT > 8 ? 8 : FIT;
+  LK_SET_MAX_LDS((ws_beside_kernel<MT, BN, NS>), NS * SB);
+  ws_beside_kernel<MT, BN, NS><<<N1 / BN + I / (BN / 2), 256, NS * SB, st>>>(x, ldx, M, K, w1, out1, ld1, N1 / BN, w2, I, out2, ld2);
+  LK_CHECK_LAUNCH();
+  return 0;
+}
+
+int lk_ws_beside(const bf16_t* x, long ldx, int M, int K, const bf16_t* w1, int N1, bf16_t* out1, long ld1, const bf16_t* w2, int I,
+                 bf16_t* out2, long ld2, int bn, hipStream_t st) {
+  if (M < 1 || M > 128 || K < 64 || K % 64 || N1 < bn || N1 % bn || I < bn / 2 || I % (bn / 2) || ws_too_far(M, ldx, K)) return -1;
+  if (bn == 64) return (M <= 64 ? launch_beside<4, 64> : launch_beside<8, 64>)(x, ldx, M, K, w1, N1, out1, ld1, w2, I, out2, ld2, st);
+  if (bn == 128) return (M <= 64 ? launch_beside<4, 128> : launch_beside<8, 128>)(x, ldx, M, K, w1, N1, out1, ld1, w2, I, out2, ld2, st);
+  return -1;
+}
+
 // padded row tiles of the weight-streaming GEMM: 16-row MFMA tiles, 4 waves splitting M
 // (the X bytes every column block stages grow with the padding: 192 rows for M 129-192
 // instead of 256)
@@ -997,7 +1043,9 @@ void lk_wsgemm_plan(int M, int N, int K, int swiglu, int* bn_out, int* s_out) {
   // Rule fitted to the exhaustive (BN, S) sweep on MI355X (profiles/r1_ws_sweep.md):
   // one block per CU, so fill <= 256 CUs in ONE round; prefer BN = 128 (half the X
   // re-reads through L2) and split K only while every block keeps >= 16 stages;
-  // fall back to BN = 64 when BN = 128 leaves more than 30 % of the CUs idle.
+  // fall back to BN = 64 when BN = 128 leaves more than 30 % of the CUs idle, and no
+  // fewer than 64-column tiles do without a sum behind them (64 x 10496 x 2048, SwiGLU
+  // 11264 x 2048: 16.6 and 17.1 us in two parts of 128 columns, 13.7 and 13.6 whole).
   (void)M;
   auto plan = [&](int BN, int* S_out) -> double {
     const int cols = swiglu ? N / 2 : N, per = swiglu ? BN / 2 : BN;
@@ -1012,7 +1060,7 @@ void lk_wsgemm_plan(int M, int N, int K, int swiglu, int* bn_out, int* s_out) {
   int s128 = 1, s64 = 1;
   const double o128 = plan(128, &s128), o64 = plan(64, &s64);
   double occ;
-  if (o128 >= 0.7 || (o128 >= 0 && o64 <= o128)) {
+  if (o128 >= 0.7 || (o128 >= 0 && (o64 < o128 || (o64 == o128 && s64 >= s128)))) {
     *bn_out = 128;
     *s_out = s128;
     occ = o128;

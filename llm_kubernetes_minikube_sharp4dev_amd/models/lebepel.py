@@ -7,7 +7,7 @@
 A configurable span of layers runs several times with the same weights; every pass has its own
 KV cache or recurrent state, and the embedding output is added to the stream once before each
 pass after the first.  Mixers: ``models.attention.sigmoid_paged_attention`` (paged K/V) and
-``models.ssm.mamba2_mixed`` (per-sequence state slots).
+``models.ssm.mamba2_projected`` (per-sequence state slots).
 
 MI355X layout decisions:
   * the residual stream is f32 and never leaves one fused kernel per block: the scaled sum of the
@@ -36,7 +36,7 @@ from .. import ops
 from ..parallel.tp import SINGLE, TPGroup
 from .attention import AttnMeta, SigmoidAttnSpec, sigmoid_paged_attention
 from .configs import LebepelConfig, pad_vocab
-from .ssm import Mamba2Spec, mamba2_mixed
+from .ssm import Mamba2Spec, mamba2_projected
 
 
 # The q|k|v bias either rides in the projection GEMM's epilogue (False) or is added in f32 by the
@@ -307,18 +307,25 @@ class LebepelModel(nn.Module):
         return self.cache_block_bytes(1)
 
     # ------------------------------------------------------------------ forward
-    def _mixed(self, L: LebepelLayer, h, meta: AttnMeta, cache):
-        """-> (what the mixer's output projection L.o reads, the projection's bias or None)."""
+    def _projected(self, L: LebepelLayer, h):
+        """-> (the mixer's input projection, the feed-forward up to its down projection): both read h, and steps of few rows
+        run them in one launch.  The second is None elsewhere (prompts run it behind the mixer: 1.5 % of a pass)."""
+        if L.type == "attention" and not FUSE_QKV_BIAS:
+            return ops.linear(h, L.qkv, L.qkv_b), None
+        w = L.qkv if L.type == "attention" else L.in_proj
+        both = ops.linear_beside(h, w, L.gate_up) if L.ff else None
+        return both if both is not None else (ops.linear(h, w), None)
+
+    def _mixed(self, L: LebepelLayer, u, meta: AttnMeta, cache):
+        """The mixer behind its input projection -> (what its output projection L.o reads, that projection's bias or None)."""
         if L.type == "attention":
             # the output projection runs bias-free (decode-sized steps then take the weight-streaming GEMMs):
             # its bias is added by the stream update in f32; the q|k|v bias: see FUSE_QKV_BIAS
-            fuse = FUSE_QKV_BIAS
-            qkv = ops.linear(h, L.qkv) if fuse else ops.linear(h, L.qkv, L.qkv_b)
-            att = sigmoid_paged_attention(qkv, cache[0], cache[1], meta, L.spec, L.r1, L.r2, L.pb, self.cfg.norm_eps,
-                                          qkv_bias=L.qkv_b if fuse else None)
+            att = sigmoid_paged_attention(u, cache[0], cache[1], meta, L.spec, L.r1, L.r2, L.pb, self.cfg.norm_eps,
+                                          qkv_bias=L.qkv_b if FUSE_QKV_BIAS else None)
             return att, L.o_b
-        return mamba2_mixed(h, L.in_proj, L.conv_w, L.conv_b, L.dt_bias, L.A_log, L.D, L.mix_norm, L.spec,
-                            self.cfg.norm_eps, cache, meta), None
+        return mamba2_projected(u, L.conv_w, L.conv_b, L.dt_bias, L.A_log, L.D, L.mix_norm, L.spec,
+                                self.cfg.norm_eps, cache, meta), None
 
     def forward(self, ids: torch.Tensor, meta: AttnMeta, caches, taps: list = None) -> torch.Tensor:
         """-> normed hidden rows [R, W] that feed the LM head (``meta.logits_idx``, or every row).
@@ -334,8 +341,10 @@ class LebepelModel(nn.Module):
                                    a_bias=ab, sums=sums)
             if taps is not None and run:  # the stream after the previous run, before this pass's re-injection
                 taps.append(x - emb if add_emb else x.clone())
-            y, ab = self._mixed(L, h, meta, caches[run])
-            f = ops.linear_swiglu_any(h, L.gate_up) if L.ff else None
+            u, f = self._projected(L, h)
+            y, ab = self._mixed(L, u, meta, caches[run])
+            if f is None and L.ff:
+                f = ops.linear_swiglu_any(h, L.gate_up)
             # (decode-sized steps: both projections as f32 parts that the next norm adds up)
             fused = (L.ff and taps is None and self.dtype == torch.bfloat16
                      and ops.sums_pay(y.shape[0], L.o.shape[0], L.o.shape[1], L.down.shape[1]))

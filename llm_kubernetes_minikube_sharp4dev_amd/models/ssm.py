@@ -64,8 +64,12 @@ def mamba2_mixer(h, w_in, conv_w, conv_b, dt_bias, A_log, D, norm_w, w_out, spec
 
 def mamba2_mixed(h, w_in, conv_w, conv_b, dt_bias, A_log, D, norm_w, spec: Mamba2Spec, eps: float, state, meta):
     """The mixer up to its output projection."""
+    return mamba2_projected(ops.linear(h, w_in), conv_w, conv_b, dt_bias, A_log, D, norm_w, spec, eps, state, meta)
+
+
+def mamba2_projected(u, conv_w, conv_b, dt_bias, A_log, D, norm_w, spec: Mamba2Spec, eps: float, state, meta):
+    """The mixer between its two projections."""
     conv_state, ssm_state = state
-    u = ops.linear(h, w_in)
     inner, C = spec.inner, spec.conv_channels
     xbc = ops.conv_silu(u, inner, C, conv_w, conv_b, conv_state, meta.seq_cu, meta.state_slots, meta.positions,
                         meta.max_seq_len)

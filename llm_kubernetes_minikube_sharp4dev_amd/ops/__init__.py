@@ -423,8 +423,10 @@ _ROWS_RULE: dict = {}
 
 
 def _ws_cost(M: int, N: int, K: int, swiglu: bool) -> float:
-    """us of the weight-streaming kernel: its workgroups' bytes at 32 KB/us, 1.2 us for each further round of them, the weight at
-    5.1 TB/s at least, and the sum of its parts of K behind it.  Within 7 % of 600 measured products."""
+    """us of the weight-streaming kernel: 3.8 ns for each of a workgroup's columns and 2.5 ns for each row per 64 of K, 6 us for each
+    further round of workgroups, the weight at 6.4 TB/s at least, and the sum of its parts of K behind it: within 20 % of 510 products
+    of 1 - 256 rows (32 shapes, 1024 - 128256 x 768 - 14336).  Given on the scale of the few-row kernel's estimate, which lies 10 % above its
+    own times, 16 % up to 64 rows and 25 % up to 16: the picks of the two take 0.3 / 0.9 / 1.3 % more than the better one."""
     def plan(bn):   # (filled share of the CUs, parts of K), as csrc/skinny_gemm.hip lays a launch out
         cols, per = (N // 2, bn // 2) if swiglu else (N, bn)
         if cols % per:
@@ -435,12 +437,14 @@ def _ws_cost(M: int, N: int, K: int, swiglu: bool) -> float:
         return cols // per * s / (256 * -(-cols // per * s // 256)), s
 
     full, half, mid = plan(128), plan(64), (-1.0, 1) if swiglu else plan(96)
-    (fill, parts), bn = (full, 128) if full[0] >= 0.7 or 0 <= half[0] <= full[0] else (half, 64)
+    whole = full[0] >= 0.7 or half[0] < full[0] or (half[0] == full[0] and half[1] >= full[1])
+    (fill, parts), bn = (full, 128) if full[0] >= 0 and whole else (half, 64)
     if mid[0] > fill + 1e-9:
         parts, bn = mid[1], 96
     rounds = -(-(N // bn * parts) // 256)
-    chain = 3.1 + rounds * (K / parts) * 2 * (bn + 0.54 * 64 * -(-M // 64)) / 32300 + 1.25 * (rounds - 1)
-    return max(chain, 4 + N * K * 2 / 5.07e6) + (2.1 + 2.3e-6 * parts * M * N if parts > 1 else 0)
+    chain = 3.0 + rounds * (K / parts) / 64 * (0.0038 * bn + 0.0025 * 64 * -(-M // 64) - 0.16) + 6.3 * (rounds - 1)
+    us = max(chain, 3.3 + N * K * 2 / 6.35e6) + (2.0 + 2.4e-6 * parts * M * N if parts > 1 else 0)
+    return us * (1.1 if M > 64 else 1.16 if M > 16 else 1.25)
 
 
 def _rows_cost(M: int, N: int, K: int, epi: int, products: int = 1):
@@ -998,6 +1002,40 @@ def linear_pair(x1, w1, x2, w2):
             if wide is not None:
                 return lib().rows_pair(x1, w1, x2, w2, wide)
     return linear(x1, w1), linear(x2, w2)
+
+
+# Two products of one x in one launch (csrc/skinny_gemm.hip ws_beside_kernel): a product of a few rows that does not fill the chip leaves CUs and
+# the memory idle at its start and its end, and both of these once.  64 W rows per workgroup where all of them run in one round of the CUs
+# (two fit a CU's LDS), else 128 where those do: 64 re-read x twice as often, and past one round the CUs with two workgroups hold up the launch.
+# Beyond, each product fills the chip by itself and the launch gains nothing; at few rows 128 pay from two thirds of the CUs on (fewer take in
+# less than the memory gives).  Plain + SwiGLU apart -> together, us, weights cold, 1 / 4 / 16 / 64 / 128 rows:
+#    3072 + 2 x 5632, K 2048   64: 13.3 / 14.4 / 15.2 / 21.4 / 32.0 -> 11.3 / 11.3 / 11.5 / 13.9 / 18.5
+#   10496 + 2 x 5632, K 2048  128: 18.2 / 19.2 / 20.3 / 27.6 / 42.7 -> 18.2 / 17.3 / 17.6 / 20.8 / 25.6   (with 64: 20.7 / 19.7 / 20.0 / 24.3 / 31.6)
+#    1536 + 2 x 2048, K 1024   64:  7.2 /  7.7 /  7.9 /  9.3 / 11.5 ->  6.2 /  6.3 /  6.4 /  8.0 / 10.5
+#    4096 + 2 x 8192, K 4096  128: 30.2 / 29.7 / 30.1 / 38.7 / 54.8 -> 29.8 / 30.1 / 30.8 / 36.0 / 44.9   (taken from 49 rows on)
+#    5120 + 2 x 13824, K 5120 128: 57.1 / 57.9 / 60.7 / 75.3 / 90.5 -> 52.3 / 52.1 / 52.3 / 56.6 / 66.7
+#    6144 + 2 x 14336, K 4096   -: 47.6 / 49.5 / 49.8 / 57.1 / 70.5    (64: 54.1 / 54.4 / 55.1 / 66.2 / 87.8; 128: 62.9 / 63.3 / 64.2 / 70.9 / 85.6)
+BESIDE_MAX_M = 128
+
+
+def _beside_rule(M: int, N: int, I: int, K: int) -> int:
+    """W rows per workgroup for N plain and I SwiGLU output columns in one launch; 0: two launches."""
+    if not 1 <= M <= BESIDE_MAX_M or K < 64 or K % 64:
+        return 0
+    cus = device_cus()
+    if N % 64 == 0 and I % 32 == 0 and N > 0 and I > 0 and N // 64 + I // 32 <= cus:
+        return 64
+    tiles = N // 128 + I // 64
+    return 128 if N % 128 == 0 and I % 64 == 0 and N > 0 and I > 0 and tiles <= cus and (M > 48 or tiles >= 0.65 * cus) else 0
+
+
+def linear_beside(x, w, w_gate_up):
+    """(x w^T, silu(x wg^T) * (x wu^T)) for a fused [wg; wu] weight in one launch; None where two pay."""
+    if not GEMM_LIBRARY and _gemm_ok(x, w) and _gemm_ok(x, w_gate_up) and w.data_ptr() % 16 == 0 and w_gate_up.data_ptr() % 16 == 0:
+        bn = _beside_rule(x.shape[0], w.shape[0], w_gate_up.shape[0] // 2, w.shape[1])
+        if bn and w.shape[1] == w_gate_up.shape[1] == x.shape[1] and w_gate_up.shape[0] % 2 == 0:
+            return tuple(lib().ws_beside(x, w, w_gate_up, bn))
+    return None
 
 
 def sums_pay(M: int, N: int, K1: int, K2: int) -> bool:

@@ -110,3 +110,44 @@ def test_measured_routes_win(monkeypatch, N, K, swiglu):
         spy.ran.clear()
         run(x, w)
         assert (spy.ran == ["rows_linear"]) == (ops._rows_rule(m - 3, N, K, 1 if swiglu else 0) is not None)
+
+
+@pytest.mark.parametrize("M,N,I,K,bn", [(1, 64, 32, 64, 64), (3, 192, 96, 128, 64), (64, 3072, 5632, 512, 64), (65, 128, 64, 320, 128), (128, 384, 192, 704, 128),
+                                        (48, 10496, 5632, 256, 128), (128, 192, 32, 1088, 64)])
+def test_two_products_beside(hip, M, N, I, K, bn):
+    """A plain and a SwiGLU product of one x in one launch, both tile widths, fewer K stages than the rings have, rows apart: one bf16
+    rounding of the plain result (2^-9 of it), SwiGLU also of g, u and silu(g), g's moving silu(g) by at most 1.1 times as much (twice that allowed)."""
+    torch.manual_seed(M + N + K)
+    rows = torch.randn(M, K + 64, device="cuda", dtype=torch.bfloat16)
+    w, wgu = (torch.randn(n, K, device="cuda", dtype=torch.bfloat16) / K ** 0.5 for n in (N, 2 * I))
+    for x in (rows[:, :K], rows[:, :K].contiguous()):
+        got, f = hip.ws_beside(x, w, wgu, bn)
+        y, gu = x.double() @ w.double().t(), x.double() @ wgu.double().t()
+        g, u = gu[:, :I], gu[:, I:]
+        assert ((got.double() - y).abs() <= 2.0 ** -8 * y.abs() + 1e-5).all()
+        want = torch.nn.functional.silu(g) * u
+        assert ((f.double() - want).abs() <= 2.0 ** -8 * (3 * want.abs() + 1.1 * (g * u).abs()) + 1e-5).all()
+
+
+def test_two_products_beside_takes_what_apart_takes(hip):
+    """ops.linear_beside returns what the two calls return, to the roundings of their sums' orders, or leaves the operands to them: rows and
+    widths inside and outside the rule, an x of transposed memory, f32."""
+    torch.manual_seed(0)
+    big = torch.randn(300, 1024, device="cuda", dtype=torch.bfloat16)
+    wn, wgu = (torch.randn(n, 256, device="cuda", dtype=torch.bfloat16) / 16 for n in (192, 256))
+    cases = [(big[:m, :256], wn, wgu) for m in (1, 2, 17, 128, 129, 300)]
+    cases += [(big[:256, :64].t(), wn, wgu), (big[:5, 8:264], wn, wgu), (big[:40, :256], wn[:40], wgu[:48]),
+              (big[:40, :256].float(), wn.float(), wgu.float())]
+    for x, w, gu in cases:
+        if x.dtype == torch.bfloat16:
+            a, b = ops.linear(x, w), ops.linear_swiglu_any(x, gu)
+        else:
+            a, b = torch.nn.functional.linear(x, w), ops.linear_swiglu_any(x, gu)
+        both = ops.linear_beside(x, w, gu)
+        assert (both is not None) == (x.dtype == torch.bfloat16 and x.stride(1) == 1 and x.shape[0] <= 128 and w.shape[0] == 192)
+        if both is None:
+            continue
+        y, f = both
+        assert y.shape == a.shape and f.shape == b.shape and y.dtype == a.dtype
+        for p, q in ((y, a), (f, b)):
+            assert (p.float() - q.float()).abs().max() <= 2.0 ** -6 * q.float().abs().max()
