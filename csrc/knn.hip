@@ -274,14 +274,14 @@ __global__ __launch_bounds__(256) void knn_merge_kernel(const float* __restrict_
 
 // One pass for up to 16 queries and K <= 8.  The corpus is read once (746 MB at 485,620 x 768) and nothing of its size is
 // written: the two-pass form wrote and re-read f32 scores of every row (31 MB at 16 queries) and paid two more launches.
-// 4 waves per CU, each with the queries' fragments in registers (D / 32 of them) and a private LDS ring of 16 stages of
-// 16 rows x 128 bytes (row_ring.h), walk 16-row tiles round robin without a barrier, so 120 KB of corpus are on their way
+// 8 waves per CU, each with the queries' fragments in registers (D / 32 of them) and a private LDS ring of 10 stages of
+// 16 rows x 128 bytes (row_ring.h), walk 16-row tiles round robin without a barrier, so 144 KB of corpus are on their way
 // per CU.  A lane sees 4 rows of one query per tile and keeps its 8 best in order (rows come in ascending order, so an
-// equal score never displaces: the stable order); 16 lists per query meet in LDS at the end.
+// equal score never displaces: the stable order); 32 lists per query meet in LDS at the end.
 // What bounds it: the stream of rows at 485,620 x 768 (120 us, 6.2 TB/s, and 5 for the merge; 131 and 6 with a wait per number of stages
 // left, row addresses per stage and reductions through the LDS unit); at 20,011 rows a wave has one or two tiles and the chain of launch,
 // code and first loads counts (12 + 4 us; 16 + 5).  The scores' own two-pass form took 158 + 26 + 10 and 11 + 12 + 5.
-constexpr int kScanK = 8, kScanQ = 16, kScanStages = 16;
+constexpr int kScanK = 8, kScanQ = 16, kScanStages = 10, kScanWaves = 8, kScanLists = 4 * kScanWaves;
 
 // ls / li descending: s, i enters behind everything that is not smaller
 LK_DEVICE void list_insert(float s, int i, float (&ls)[kScanK], int (&li)[kScanK]) {
@@ -309,7 +309,7 @@ LK_DEVICE void list_pop(float (&ls)[kScanK], int (&li)[kScanK]) {
 }
 
 template <int SEG>
-__global__ __launch_bounds__(256, 1) void knn_scan_kernel(const bf16_t* __restrict__ corpus, const float* __restrict__ cnorm, long N,
+__global__ __launch_bounds__(64 * kScanWaves, 1) void knn_scan_kernel(const bf16_t* __restrict__ corpus, const float* __restrict__ cnorm, long N,
                                                           const bf16_t* __restrict__ queries, const float* __restrict__ qnorm, int nq,
                                                           int K, float* __restrict__ part_s, int* __restrict__ part_i) {
   constexpr int D = SEG * 64, NS = kScanStages;
@@ -322,21 +322,22 @@ __global__ __launch_bounds__(256, 1) void knn_scan_kernel(const bf16_t* __restri
     for (int k = 0; k < 2 * SEG; ++k) qf[k] = *reinterpret_cast<const short8*>(q + 32 * k);
   }
   const float qgiven = qnorm ? qnorm[min(r16, nq - 1)] : 0.f;
-  const int tiles = (int)((N + 15) / 16), first = blockIdx.x * 4 + w, step = gridDim.x * 4;
+  // (a workgroup's waves are a grid apart: where there are fewer tiles than waves, every CU has as many)
+  const int tiles = (int)((N + 15) / 16), first = w * gridDim.x + blockIdx.x, step = gridDim.x * kScanWaves;
   const int total = first < tiles ? ((tiles - 1 - first) / step + 1) * SEG : 0;  // this wave's stages
   unsigned char* const ring = smem + w * NS * 2048;
   const int lrow = lane >> 3, lcol = rg_lane_col(lane);
   const bf16_t* src[2];  // this lane's part of the tile being requested
-  int ist = 0;           // stages requested
+  int ist = 0, to = 0;   // stages requested; where the next goes
   auto issue = [&](int seg, long tile) {
     if (seg == 0) {
 #pragma unroll
       for (int i = 0; i < 2; ++i) src[i] = corpus + min(tile * 16 + 8 * i + lrow, N - 1) * D + lcol;
     }
-    unsigned char* base = ring + (ist % NS) * 2048;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) __builtin_amdgcn_global_load_lds((rg_gptr)(src[i] + seg * 64), (rg_lptr)(base + i * 1024), 16, 0, 2);
+    for (int i = 0; i < 2; ++i) __builtin_amdgcn_global_load_lds((rg_gptr)(src[i] + seg * 64), (rg_lptr)(ring + to + i * 1024), 16, 0, 2);
     ++ist;
+    to = to + 2048 == NS * 2048 ? 0 : to + 2048;
   };
 #pragma unroll
   for (int p = 0; p < NS - 1; ++p)
@@ -368,7 +369,7 @@ __global__ __launch_bounds__(256, 1) void knn_scan_kernel(const bf16_t* __restri
     ls[j] = -INFINITY;
     li[j] = 0x7fffffff;
   }
-  int st = 0;
+  int st = 0, from = 0;
   for (long t = first; t < tiles; t += step) {
     const long d0 = t * 16 + 4 * g;
     float cn[4];
@@ -384,7 +385,8 @@ __global__ __launch_bounds__(256, 1) void knn_scan_kernel(const bf16_t* __restri
       __builtin_amdgcn_sched_barrier(0);
       if (ist < total) issue((seg + NS - 1) % SEG, t + (long)((seg + NS - 1) / SEG) * step);
       __builtin_amdgcn_sched_barrier(0);
-      const unsigned char* base = ring + (st % NS) * 2048;
+      const unsigned char* base = ring + from;
+      from = from + 2048 == NS * 2048 ? 0 : from + 2048;
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const short8 a = *reinterpret_cast<const short8*>(base + r16 * 128 + (((4 * h + g) ^ (r16 & 7)) << 4));
@@ -397,31 +399,42 @@ __global__ __launch_bounds__(256, 1) void knn_scan_kernel(const bf16_t* __restri
       if (s > ls[kScanK - 1]) list_insert(s, (int)(d0 + j), ls, li);
     }
   }
-  // [query][4 waves x 4 lane groups][kScanK]
+  // [kScanK][kScanLists: 8 waves x 4 lane groups][query], a query's words 17 apart: neither side meets a bank twice, and lanes without a
+  // query write nothing (lists of 8 words each behind the other met one bank 16 at a time: 2.1 us of a scan for 0.9)
   __syncthreads();
+  constexpr int LQ = kScanQ + 1;
   float* ms = reinterpret_cast<float*>(smem);
-  int* mi = reinterpret_cast<int*>(smem) + kScanQ * 16 * kScanK;
+  int* mi = reinterpret_cast<int*>(smem) + kScanK * kScanLists * LQ;
+  if (r16 < nq) {
 #pragma unroll
-  for (int j = 0; j < kScanK; ++j) {
-    ms[(r16 * 16 + w * 4 + g) * kScanK + j] = ls[j];
-    mi[(r16 * 16 + w * 4 + g) * kScanK + j] = li[j];
+    for (int j = 0; j < kScanK; ++j) {
+      ms[(j * kScanLists + w * 4 + g) * LQ + r16] = ls[j];
+      mi[(j * kScanLists + w * 4 + g) * LQ + r16] = li[j];
+    }
   }
   __syncthreads();
-  // a wave takes four queries at once, a lane one of their 16 lists: K rounds over the lists' heads
-  {
-    const int q = w * 4 + g;
+  // a wave takes two queries at once, a lane one of their 32 lists: K rounds over the lists' heads
+  if (w * 2 < nq) {
+    const int q = min(w * 2 + (lane >> 5), nq - 1), l = lane & 31;
+    const bool mine = w * 2 + (lane >> 5) < nq;
     float v[kScanK];
     int id[kScanK];
 #pragma unroll
     for (int j = 0; j < kScanK; ++j) {
-      v[j] = ms[(q * 16 + r16) * kScanK + j];
-      id[j] = mi[(q * 16 + r16) * kScanK + j];
+      v[j] = ms[(j * kScanLists + l) * LQ + q];
+      id[j] = mi[(j * kScanLists + l) * LQ + q];
     }
     for (int k = 0; k < K; ++k) {
       float bs = v[0];
       int bi = id[0];
       row_argmax(bs, bi);
-      if (r16 == 0 && q < nq) {
+      const float s2 = __shfl_xor(bs, 16, 64);
+      const int i2 = __shfl_xor(bi, 16, 64);
+      if (better(s2, i2, bs, bi)) {
+        bs = s2;
+        bi = i2;
+      }
+      if (l == 0 && mine) {
         const long o = ((long)q * gridDim.x + blockIdx.x) * K + k;
         part_s[o] = bs;
         part_i[o] = bs == -INFINITY ? -1 : bi;
@@ -480,9 +493,10 @@ __global__ __launch_bounds__(256) void knn_merge_lists_kernel(const float* __res
 template <int SEG>
 int launch_scan(const bf16_t* corpus, const float* cnorm, long N, const bf16_t* queries, const float* qnorm, int nq, int K, int nb,
                 float* part_s, int* part_i, hipStream_t st) {
-  constexpr int lds = 4 * kScanStages * 2048;  // (the lists at the end need 16 KB of it)
+  constexpr int lds = kScanWaves * kScanStages * 2048;
+  static_assert(lds >= 2 * 4 * kScanK * kScanLists * (kScanQ + 1), "the lists at the end");
   LK_SET_MAX_LDS((knn_scan_kernel<SEG>), lds);
-  knn_scan_kernel<SEG><<<nb, 256, lds, st>>>(corpus, cnorm, N, queries, qnorm, nq, K, part_s, part_i);
+  knn_scan_kernel<SEG><<<nb, 64 * kScanWaves, lds, st>>>(corpus, cnorm, N, queries, qnorm, nq, K, part_s, part_i);
   LK_CHECK_LAUNCH();
   return 0;
 }
