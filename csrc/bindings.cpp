@@ -924,14 +924,14 @@ std::vector<at::Tensor> knn_topk(const at::Tensor& corpus, const at::Tensor& cno
   at::Tensor out_i = at::empty({nq, (long)K}, io);
   const auto a16 = [](const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
   if (const int nb = force_fused || !a16(corpus) || !a16(queries) ? 0 : lk_knn_scan_blocks(N, D, nq, kk)) {
-    at::Tensor ps = at::empty({nq, nb, kk}, fo), pi = at::empty({nq, nb, kk}, io);
+    at::Tensor part = at::empty({2, nq, nb, kk}, io);
     if (kk < K) {
       out_s.fill_(-INFINITY);
       out_i.fill_(-1);
     }
     at::Tensor ks = kk < K ? at::empty({nq, kk}, fo) : out_s, ki = kk < K ? at::empty({nq, kk}, io) : out_i;
-    CHECK_RC(lk_knn_scan(bp(corpus), cnorm.data_ptr<float>(), N, D, bp(queries), qnorm.data_ptr<float>(), nq, kk, ps.data_ptr<float>(),
-                         pi.data_ptr<int>(), ks.data_ptr<float>(), ki.data_ptr<int>(), cur_stream()), "knn_scan");
+    CHECK_RC(lk_knn_scan(bp(corpus), cnorm.data_ptr<float>(), N, D, bp(queries), qnorm.data_ptr<float>(), nq, kk,
+                         part.data_ptr<int>(), ks.data_ptr<float>(), ki.data_ptr<int>(), cur_stream()), "knn_scan");
     if (kk < K) {
       out_s.slice(1, 0, kk).copy_(ks);
       out_i.slice(1, 0, kk).copy_(ki);
@@ -1046,9 +1046,8 @@ int knn_scan_plan(const at::Tensor& corpus, const at::Tensor& cnorm, const at::T
 void knn_scan_to(int* o, const at::Tensor& corpus, const at::Tensor& cnorm, const at::Tensor& queries, int64_t K, int nb) {
   const long nq = queries.size(0);
   at::Tensor part = at::empty({2, nq, nb, K}, corpus.options().dtype(at::kInt));
-  int* p = part.data_ptr<int>();
   CHECK_RC(lk_knn_scan(bp(corpus), cnorm.data_ptr<float>(), corpus.size(0), corpus.size(1), bp(queries), nullptr, (int)nq, (int)K,
-                       reinterpret_cast<float*>(p), p + nq * nb * K, reinterpret_cast<float*>(o), o + nq * K, cur_stream()), "knn_scan");
+                       part.data_ptr<int>(), reinterpret_cast<float*>(o), o + nq * K, cur_stream()), "knn_scan");
 }
 
 // The one-pass search with both results in one buffer, int32 [2, nq, K] (score bits, then row numbers); an empty tensor where the one-pass

@@ -219,7 +219,7 @@ int lk_flash_prefill(const bf16_t* q, long qs, const bf16_t* k, const bf16_t* v,
 // knn.hip
 int lk_knn_scan_blocks(long N, int D, int nq, int K);
 int lk_knn_scan(const bf16_t* corpus, const float* cnorm, long N, int D, const bf16_t* queries, const float* qnorm, int nq, int K,
-                float* part_s, int* part_i, float* out_s, int* out_i, hipStream_t st);
+                void* part, float* out_s, int* out_i, hipStream_t st);
 int lk_knn_nblocks(long N);
 int lk_knn_partial(const bf16_t* corpus, const float* cnorm, long N, int D, const bf16_t* queries,
                    const float* qnorm, int nq, int K, float* part_s, int* part_i, hipStream_t st);

@@ -43,21 +43,36 @@ LK_DEVICE void wave_argmax(float& s, int& i) {
   }
 }
 
-// over groups of 16 lanes, by row rotations of the vector unit (every lane ends with the same pair)
-template <int STEP>
-LK_DEVICE void rotate_argmax(float& s, int& i) {
-  const float s2 = wave_partner<STEP>(s);
-  const int i2 = __builtin_amdgcn_update_dpp(0, i, 0x120 + STEP, 0xf, 0xf, true);
-  if (better(s2, i2, s, i)) {
-    s = s2;
-    i = i2;
-  }
+// A hit as one number that orders as (score desc, index asc) does: the score's bits made monotonic, then the index's complement; 0: none.
+// (Both zeros are one score.)
+typedef unsigned long long hit_t;
+LK_DEVICE hit_t hit_of(float s, int i) {
+  const unsigned u = __float_as_uint(s + 0.f);
+  return s == -INFINITY ? 0 : (hit_t)(u ^ ((unsigned)((int)u >> 31) | 0x80000000u)) << 32 | (unsigned)~i;
 }
-LK_DEVICE void row_argmax(float& s, int& i) {
-  rotate_argmax<8>(s, i);
-  rotate_argmax<4>(s, i);
-  rotate_argmax<2>(s, i);
-  rotate_argmax<1>(s, i);
+LK_DEVICE float hit_score(hit_t h) {
+  const unsigned u = (unsigned)(h >> 32);
+  return h == 0 ? -INFINITY : __uint_as_float(u >> 31 ? u ^ 0x80000000u : ~u);
+}
+LK_DEVICE int hit_index(hit_t h) { return h == 0 ? -1 : (int)~(unsigned)h; }
+
+// the best of groups of 16 lanes, by row rotations of the vector unit (every lane ends with it)
+template <int STEP>
+LK_DEVICE hit_t rotate_best(hit_t h) {
+  const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)h, 0x120 + STEP, 0xf, 0xf, true);
+  const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(h >> 32), 0x120 + STEP, 0xf, 0xf, true);
+  const hit_t o = (hit_t)hi << 32 | lo;
+  return o > h ? o : h;
+}
+LK_DEVICE hit_t row_best(hit_t h) { return rotate_best<1>(rotate_best<2>(rotate_best<4>(rotate_best<8>(h)))); }
+// ... of pairs of them (lanes l and l ^ 16)
+LK_DEVICE hit_t rows_best(hit_t h) {
+  h = row_best(h);
+  const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)h, (unsigned)h, false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(h >> 32), (unsigned)(h >> 32), false, false);
+  const unsigned l0 = lo[0], l1 = lo[1], h0 = hi[0], h1 = hi[1];
+  const hit_t a = (hit_t)h0 << 32 | l0, b = (hit_t)h1 << 32 | l1;
+  return a > b ? a : b;
 }
 
 template <int D>
@@ -278,9 +293,11 @@ __global__ __launch_bounds__(256) void knn_merge_kernel(const float* __restrict_
 // 16 rows x 128 bytes (row_ring.h), walk 16-row tiles round robin without a barrier, so 144 KB of corpus are on their way
 // per CU.  A lane sees 4 rows of one query per tile and keeps its 8 best in order (rows come in ascending order, so an
 // equal score never displaces: the stable order); 32 lists per query meet in LDS at the end.
-// What bounds it: the stream of rows at 485,620 x 768 (120 us, 6.2 TB/s, and 5 for the merge; 131 and 6 with a wait per number of stages
-// left, row addresses per stage and reductions through the LDS unit); at 20,011 rows a wave has one or two tiles and the chain of launch,
-// code and first loads counts (12 + 4 us; 16 + 5).  The scores' own two-pass form took 158 + 26 + 10 and 11 + 12 + 5.
+// What bounds it: the stream of rows at 485,620 x 768 (118 us, 6.3 TB/s, and 4 for the merge; 131 and 6 with a wait per number of stages
+// left, row addresses per stage and reductions through the LDS unit); at 20,011 rows the chain of launch, code and first loads: of 10 us the
+// rows come between the third and the ninth, the lists and the merge of a workgroup take the rest.  Four waves per CU had a quarter of their
+// tiles behind another and met one LDS bank with all lists (13.2 us), and hits in two words compared in three steps (11.2); one question in
+// all 29.0 -> 26.5 us, 16 over 485,620 150 -> 145.  The scores' own two-pass form took 158 + 26 + 10 and 11 + 12 + 5.
 constexpr int kScanK = 8, kScanQ = 16, kScanStages = 10, kScanWaves = 8, kScanLists = 4 * kScanWaves;
 
 // ls / li descending: s, i enters behind everything that is not smaller
@@ -298,20 +315,16 @@ LK_DEVICE void list_insert(float s, int i, float (&ls)[kScanK], int (&li)[kScanK
 }
 
 // the head leaves (of the padding behind a short list, all heads do: nothing follows it)
-LK_DEVICE void list_pop(float (&ls)[kScanK], int (&li)[kScanK]) {
+LK_DEVICE void list_pop(hit_t (&l)[kScanK]) {
 #pragma unroll
-  for (int j = 0; j + 1 < kScanK; ++j) {
-    ls[j] = ls[j + 1];
-    li[j] = li[j + 1];
-  }
-  ls[kScanK - 1] = -INFINITY;
-  li[kScanK - 1] = 0x7fffffff;
+  for (int j = 0; j + 1 < kScanK; ++j) l[j] = l[j + 1];
+  l[kScanK - 1] = 0;
 }
 
 template <int SEG>
 __global__ __launch_bounds__(64 * kScanWaves, 1) void knn_scan_kernel(const bf16_t* __restrict__ corpus, const float* __restrict__ cnorm, long N,
                                                           const bf16_t* __restrict__ queries, const float* __restrict__ qnorm, int nq,
-                                                          int K, float* __restrict__ part_s, int* __restrict__ part_i) {
+                                                          int K, hit_t* __restrict__ part) {
   constexpr int D = SEG * 64, NS = kScanStages;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, g = lane >> 4;
@@ -400,103 +413,65 @@ __global__ __launch_bounds__(64 * kScanWaves, 1) void knn_scan_kernel(const bf16
     }
   }
   // [kScanK][kScanLists: 8 waves x 4 lane groups][query], a query's words 17 apart: neither side meets a bank twice, and lanes without a
-  // query write nothing (lists of 8 words each behind the other met one bank 16 at a time: 2.1 us of a scan for 0.9)
+  // query write nothing (lists of 8 words each behind the other met one bank 16 at a time)
   __syncthreads();
   constexpr int LQ = kScanQ + 1;
-  float* ms = reinterpret_cast<float*>(smem);
-  int* mi = reinterpret_cast<int*>(smem) + kScanK * kScanLists * LQ;
+  hit_t* ml = reinterpret_cast<hit_t*>(smem);
   if (r16 < nq) {
 #pragma unroll
-    for (int j = 0; j < kScanK; ++j) {
-      ms[(j * kScanLists + w * 4 + g) * LQ + r16] = ls[j];
-      mi[(j * kScanLists + w * 4 + g) * LQ + r16] = li[j];
-    }
+    for (int j = 0; j < kScanK; ++j) ml[(j * kScanLists + w * 4 + g) * LQ + r16] = hit_of(ls[j], li[j]);
   }
   __syncthreads();
   // a wave takes two queries at once, a lane one of their 32 lists: K rounds over the lists' heads
   if (w * 2 < nq) {
     const int q = min(w * 2 + (lane >> 5), nq - 1), l = lane & 31;
     const bool mine = w * 2 + (lane >> 5) < nq;
-    float v[kScanK];
-    int id[kScanK];
+    hit_t v[kScanK];
 #pragma unroll
-    for (int j = 0; j < kScanK; ++j) {
-      v[j] = ms[(j * kScanLists + l) * LQ + q];
-      id[j] = mi[(j * kScanLists + l) * LQ + q];
-    }
+    for (int j = 0; j < kScanK; ++j) v[j] = ml[(j * kScanLists + l) * LQ + q];
     for (int k = 0; k < K; ++k) {
-      float bs = v[0];
-      int bi = id[0];
-      row_argmax(bs, bi);
-      const float s2 = __shfl_xor(bs, 16, 64);
-      const int i2 = __shfl_xor(bi, 16, 64);
-      if (better(s2, i2, bs, bi)) {
-        bs = s2;
-        bi = i2;
-      }
-      if (l == 0 && mine) {
-        const long o = ((long)q * gridDim.x + blockIdx.x) * K + k;
-        part_s[o] = bs;
-        part_i[o] = bs == -INFINITY ? -1 : bi;
-      }
-      if (id[0] == bi) list_pop(v, id);
+      const hit_t best = rows_best(v[0]);
+      if (l == 0 && mine) part[((long)q * gridDim.x + blockIdx.x) * K + k] = best;
+      if (v[0] == best) list_pop(v);
     }
   }
 }
 
 // merge of at most 256 lists of K <= 8, each in order: one workgroup per query, a list per thread; every 16 lanes take the
 // K best of their lists by the lists' heads, then 16 lanes those of the 16 groups
-__global__ __launch_bounds__(256) void knn_merge_lists_kernel(const float* __restrict__ cs, const int* __restrict__ ci, int lists, int K,
-                                                              float* __restrict__ out_s, int* __restrict__ out_i) {
-  __shared__ float rs[16][kScanK];
-  __shared__ int ri[16][kScanK];
+__global__ __launch_bounds__(256) void knn_merge_lists_kernel(const hit_t* __restrict__ part, int lists, int K, float* __restrict__ out_s,
+                                                              int* __restrict__ out_i) {
+  __shared__ hit_t rl[16][kScanK];
   const int q = blockIdx.x, tid = threadIdx.x, l16 = tid & 15, grp = tid >> 4;
-  float s[kScanK];
-  int i[kScanK];
+  hit_t v[kScanK];
 #pragma unroll
-  for (int j = 0; j < kScanK; ++j) {
-    const long o = ((long)q * lists + tid) * K + j;
-    const bool on = tid < lists && j < K;
-    s[j] = on ? cs[o] : -INFINITY;
-    const int v = on ? ci[o] : -1;
-    i[j] = v < 0 ? 0x7fffffff : v;
-  }
+  for (int j = 0; j < kScanK; ++j) v[j] = tid < lists && j < K ? part[((long)q * lists + tid) * K + j] : 0;
   for (int k = 0; k < K; ++k) {
-    float bs = s[0];
-    int bi = i[0];
-    row_argmax(bs, bi);
-    if (l16 == 0) {
-      rs[grp][k] = bs;
-      ri[grp][k] = bi;
-    }
-    if (i[0] == bi) list_pop(s, i);
+    const hit_t best = row_best(v[0]);
+    if (l16 == 0) rl[grp][k] = best;
+    if (v[0] == best) list_pop(v);
   }
   __syncthreads();
   if (grp) return;
 #pragma unroll
-  for (int j = 0; j < kScanK; ++j) {
-    s[j] = j < K ? rs[l16][j] : -INFINITY;
-    i[j] = j < K ? ri[l16][j] : 0x7fffffff;
-  }
+  for (int j = 0; j < kScanK; ++j) v[j] = j < K ? rl[l16][j] : 0;
   for (int k = 0; k < K; ++k) {
-    float bs = s[0];
-    int bi = i[0];
-    row_argmax(bs, bi);
+    const hit_t best = row_best(v[0]);
     if (l16 == 0) {  // (each word once, at system scope: in pinned memory the host sees it arrive)
-      __hip_atomic_store(out_s + (long)q * K + k, bs, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      __hip_atomic_store(out_i + (long)q * K + k, bs == -INFINITY ? -1 : bi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      __hip_atomic_store(out_s + (long)q * K + k, hit_score(best), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      __hip_atomic_store(out_i + (long)q * K + k, hit_index(best), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
-    if (i[0] == bi) list_pop(s, i);
+    if (v[0] == best) list_pop(v);
   }
 }
 
 template <int SEG>
 int launch_scan(const bf16_t* corpus, const float* cnorm, long N, const bf16_t* queries, const float* qnorm, int nq, int K, int nb,
-                float* part_s, int* part_i, hipStream_t st) {
+                hit_t* part, hipStream_t st) {
   constexpr int lds = kScanWaves * kScanStages * 2048;
-  static_assert(lds >= 2 * 4 * kScanK * kScanLists * (kScanQ + 1), "the lists at the end");
+  static_assert(lds >= 8 * kScanK * kScanLists * (kScanQ + 1), "the lists at the end");
   LK_SET_MAX_LDS((knn_scan_kernel<SEG>), lds);
-  knn_scan_kernel<SEG><<<nb, 64 * kScanWaves, lds, st>>>(corpus, cnorm, N, queries, qnorm, nq, K, part_s, part_i);
+  knn_scan_kernel<SEG><<<nb, 64 * kScanWaves, lds, st>>>(corpus, cnorm, N, queries, qnorm, nq, K, part);
   LK_CHECK_LAUNCH();
   return 0;
 }
@@ -550,22 +525,22 @@ int lk_knn_scan_blocks(long N, int D, int nq, int K) {
   return (int)(b < 256 ? b : 256);
 }
 
-// out_s / out_i [nq, K]; qnorm null: the queries' norms are taken here; part_*: [nq, blocks, K]
+// out_s / out_i [nq, K]; qnorm null: the queries' norms are taken here; part: [nq, blocks, K] of 8 bytes
 int lk_knn_scan(const bf16_t* corpus, const float* cnorm, long N, int D, const bf16_t* queries, const float* qnorm, int nq, int K,
-                float* part_s, int* part_i, float* out_s, int* out_i, hipStream_t st) {
+                void* part, float* out_s, int* out_i, hipStream_t st) {
   const int nb = lk_knn_scan_blocks(N, D, nq, K);
   if (!nb) return -1;
   int rc;
   switch (D) {
-    case 128: rc = launch_scan<2>(corpus, cnorm, N, queries, qnorm, nq, K, nb, part_s, part_i, st); break;
-    case 256: rc = launch_scan<4>(corpus, cnorm, N, queries, qnorm, nq, K, nb, part_s, part_i, st); break;
-    case 384: rc = launch_scan<6>(corpus, cnorm, N, queries, qnorm, nq, K, nb, part_s, part_i, st); break;
-    case 512: rc = launch_scan<8>(corpus, cnorm, N, queries, qnorm, nq, K, nb, part_s, part_i, st); break;
-    case 768: rc = launch_scan<12>(corpus, cnorm, N, queries, qnorm, nq, K, nb, part_s, part_i, st); break;
-    default: rc = launch_scan<16>(corpus, cnorm, N, queries, qnorm, nq, K, nb, part_s, part_i, st); break;
+    case 128: rc = launch_scan<2>(corpus, cnorm, N, queries, qnorm, nq, K, nb, (hit_t*)part, st); break;
+    case 256: rc = launch_scan<4>(corpus, cnorm, N, queries, qnorm, nq, K, nb, (hit_t*)part, st); break;
+    case 384: rc = launch_scan<6>(corpus, cnorm, N, queries, qnorm, nq, K, nb, (hit_t*)part, st); break;
+    case 512: rc = launch_scan<8>(corpus, cnorm, N, queries, qnorm, nq, K, nb, (hit_t*)part, st); break;
+    case 768: rc = launch_scan<12>(corpus, cnorm, N, queries, qnorm, nq, K, nb, (hit_t*)part, st); break;
+    default: rc = launch_scan<16>(corpus, cnorm, N, queries, qnorm, nq, K, nb, (hit_t*)part, st); break;
   }
   if (rc) return rc;
-  knn_merge_lists_kernel<<<nq, 256, 0, st>>>(part_s, part_i, nb, K, out_s, out_i);
+  knn_merge_lists_kernel<<<nq, 256, 0, st>>>((const hit_t*)part, nb, K, out_s, out_i);
   LK_CHECK_LAUNCH();
   return 0;
 }

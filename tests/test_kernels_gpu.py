@@ -1195,6 +1195,32 @@ def test_ws_walk_edges(hip, M, N, K, swiglu, bn, S, variant):
         hip.ws_set_variant(M, N, K, swiglu, -1)
 
 
+@pytest.mark.parametrize("N,nq,K", [(1, 1, 1), (5, 3, 8), (16, 16, 8), (17, 2, 5), (4097, 16, 8), (40000, 1, 3)])
+def test_knn_scan_orders_signs_and_ties(hip, N, nq, K):
+    """The one-pass search's hits as ordered numbers: negative scores, zero rows (a zero of either sign is one score), equal rows in order
+    of their numbers, fewer rows than K, fewer tiles than waves and more.  Rows of small whole numbers: dots and norms are exact."""
+    g = torch.Generator().manual_seed(N + nq)
+    c = torch.randint(-2, 3, (N, 128), generator=g)
+    c[::3] = c[0].clone()                           # equal rows
+    c[1::7] = 0
+    q = -c[torch.arange(nq) % N] if N < 64 else torch.randint(-2, 3, (nq, 128), generator=g)   # (few rows: no positive score)
+    q[0, 0] += 1
+    corpus, queries = (t.to(torch.bfloat16).to(DEV) for t in (c, q))
+    cn, qn = (t.double().norm(dim=1) for t in (c, q))
+    s, i = (t.cpu() for t in hip.knn_topk(corpus, cn.float().to(DEV), queries, qn.float().to(DEV), K))
+    want = (q.double() @ c.double().t()) / (qn[:, None] * cn[None] + 1e-9)
+    # f32 scores tie where the exact ones do: order by the kernel's own arithmetic
+    f = (q.float() @ c.float().t()) / (qn.float()[:, None] * cn.float()[None] + 1e-9)
+    for r in range(nq):
+        order = sorted(range(N), key=lambda j: (-float(f[r, j]) + 0.0, j))[:K]
+        n = len(order)
+        assert torch.isfinite(s[r, :n]).all() and (i[r, n:] == -1).all() and (s[r, n:] == -float("inf")).all()
+        assert (s[r, :n].double() - want[r, order]).abs().max() <= 2.0 ** -22
+        got = i[r, :n].tolist()
+        assert len(set(got)) == n and all((float(f[r, a]), -a) > (float(f[r, b]), -b) or abs(float(f[r, a] - f[r, b])) <= 2.0 ** -22 and want[r, a] != want[r, b]
+                                          for a, b in zip(got, got[1:]))
+
+
 def test_invalid_launch_raises(hip):
     """A launch the runtime rejects (2048 threads per workgroup) raises with the HIP error
     instead of returning as if it had run; the next op on the stream still works."""
