@@ -4,13 +4,15 @@
 // norms of 19 rows and 12 attentions of 12 workgroups.  Both read little, so every workgroup of the following product can afford to
 // compute all of it again from L2 while its weight rows are on their way:
 //   * ln_rows_kernel:   h = LN(s) for the workgroup's rows in LDS, in the order that the fragment reads want, then
-//     Y = act(h W^T + b).  Row tiles of 64; each row of h is stored by one of the workgroups (it is the next residual).
+//     Y = act(h W^T + b).  Each row of h is stored by one of the workgroups (it is the next residual).  Row tiles of 64; up to 32 rows two
+//     tiles of half the rows and 32 columns: a workgroup's norms are arithmetic of 12 waves on 4 SIMDs (1.3 - 1.9 us of 4.6 with all 19 rows,
+//     24 rows at once, between 2.2 us of loads and 0.9 of sums and stores), and half of them half as much.
 //   * attn_rows_kernel: bidirectional attention of ONE text of up to 32 tokens and heads of 64, then Y = bf16(A W^T + b) + R.  A
 //     wave computes one head: S^T = K Q^T leaves each lane four adjacent keys of one query, O^T = V^T P^T takes them as they are
 //     (its K order is permuted alike on both sides), and O^T, rounded to bf16 as the attention alone stores it, is the product's X
 //     fragment of the head's 64 columns in registers (W is read from LDS in the same permuted order).
-// Measured in a pass (19 tokens): norm and QKV 3.6 + 3.8 -> 6.1 us, norm and first projection 3.6 + 3.7 -> 6.4 us, attention and its
-// projection 3.8 + 3.7 -> 6.3 us, and a third fewer launches: a pass with cold weights 518 -> 410 us.
+// Measured in a pass (19 tokens): launches apart 314 us, fused 295, with two tiles of half the rows 275 (behind a pass over 512 MB 357 -> 300);
+// of a launch's 5.6 us 1.5 are the gap before it, 2.2 its first loads.
 // One wave per 64 columns of K in both: every load of a workgroup is requested at its start, so a launch waits for memory once.
 // The arithmetic and the roundings are those of layernorm_kernel, of flash_prefill (f32 scores and sums, P and A in bf16) and
 // of rows_gemm_kernel.
@@ -21,16 +23,20 @@
 namespace {
 
 constexpr int kErRows = 64;      // rows of a workgroup
+// Beyond this many rows and up to 32: two tiles of half the rows.  12 layers of 768 (384), cold weights, 8 / 9 / 16 / 19 / 24 / 32 tokens, one tile ->
+// two: 250 / 256 / 275 / 295 / 304 / 333 (194 / 199 / 219 / 230 / 246 / 259) -> 255 / 256 / 273 / 271 / 281 / 296 (197 / 197 / 208 / 210 / 216 / 233) us
+constexpr int kErHalve = 8;
 constexpr int kErWaves = 12;     // 64 columns of K each: a 64-row tile of h and the weight rows in 160 KB
 
 enum { ER_BIAS = 2, ER_GELU = 3, ER_ADD = 5 };
 
-// 16 weight rows x this wave's 64 columns
+// 16 NT weight rows x this wave's 64 columns
+template <int NT = 1>
 LK_DEVICE void er_load_w(const bf16_t* W, int n0, int K, int wave, unsigned char* wl) {
   const int lane = threadIdx.x & 63;
   const bf16_t* w = W + (long)(n0 + (lane >> 3)) * K + wave * 64 + rg_lane_col(lane);
 #pragma unroll
-  for (int i = 0; i < 2; ++i) __builtin_amdgcn_global_load_lds((rg_gptr)(w + (long)i * 8 * K), (rg_lptr)(wl + i * 1024), 16, 0, 2);
+  for (int i = 0; i < 2 * NT; ++i) __builtin_amdgcn_global_load_lds((rg_gptr)(w + (long)i * 8 * K), (rg_lptr)(wl + i * 1024), 16, 0, 2);
 }
 
 // The waves' partial tiles through LDS: wave m, m + waves, .. gets tile row m from total(m, sum)
@@ -74,26 +80,26 @@ LK_DEVICE void er_store(bf16_t* y, const bf16_t* b, const bf16_t* r, floatx4 t) 
   *reinterpret_cast<uint2*>(y) = pk;
 }
 
-// grid (N / 16, row tiles), K / 64 waves; LDS: the tile of s, then of h: K / 64 pieces of [16 MT rows][128 bytes]; the weight rows
-template <int MT, int EPI>
+// grid (N / (16 NT), tiles of `rows` rows), K / 64 waves; LDS: the tile of s, then of h: K / 64 pieces of [16 MT rows][128 bytes]; the weight rows
+template <int MT, int NT, int EPI>
 __global__ __launch_bounds__(64 * kErWaves, 1) void ln_rows_kernel(const bf16_t* __restrict__ S, long ss, const bf16_t* __restrict__ lw,
                                                                    const bf16_t* __restrict__ lb, float eps, bf16_t* __restrict__ H,
                                                                    const bf16_t* __restrict__ W, const bf16_t* __restrict__ bias,
-                                                                   bf16_t* __restrict__ Y, int M, int N, int K) {
+                                                                   bf16_t* __restrict__ Y, int M, int N, int K, int rows) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = K / 64;
-  const int n0 = blockIdx.x * 16, m0 = blockIdx.y * kErRows;
-  M = min(M - m0, kErRows);
+  const int n0 = blockIdx.x * (16 * NT), m0 = blockIdx.y * rows;
+  M = min(M - m0, rows);
   S += (long)m0 * ss;
   H += (long)m0 * K;
   Y += (long)m0 * N;
-  unsigned char* wl = smem + (long)waves * MT * 2048 + wave * 2048;
+  unsigned char* wl = smem + (long)waves * MT * 2048 + wave * (NT * 2048);
   unsigned char* sl = smem + (long)wave * MT * 2048;
 #pragma unroll
   for (int i = 0; i < 2 * MT; ++i)   // rows past M repeat the last one
     __builtin_amdgcn_global_load_lds((rg_gptr)(S + (long)min(8 * i + (lane >> 3), M - 1) * ss + wave * 64 + rg_lane_col(lane)),
                                      (rg_lptr)(sl + i * 1024), 16, 0, 0);
-  er_load_w(W, n0, K, wave, wl);
+  er_load_w<NT>(W, n0, K, wave, wl);
 
   // Half a wave per row; lane l holds the row's 16-byte chunks l, l + 32, l + 64 (K <= 768: 96).  The loop stays rolled: unrolled over
   // the rows it is 12 KB of code that a launch runs once, and fetching that took longer than the arithmetic.
@@ -147,46 +153,55 @@ __global__ __launch_bounds__(64 * kErWaves, 1) void ln_rows_kernel(const bf16_t*
   }
   __syncthreads();   // everyone's rows of h
 
-  floatx4 acc[MT];
+  floatx4 acc[MT * NT];
 #pragma unroll
-  for (int m = 0; m < MT; ++m) acc[m] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int m = 0; m < MT * NT; ++m) acc[m] = floatx4{0.f, 0.f, 0.f, 0.f};
   const int r16 = lane & 15, g4 = lane >> 4;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const int at = r16 * 128 + (((4 * h + g4) ^ (r16 & 7)) << 4);
-    const short8 b = *reinterpret_cast<const short8*>(wl + at);
+    short8 b[NT];
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
-      acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, *reinterpret_cast<const short8*>(sl + m * 2048 + at), acc[m], 0, 0, 0);
+    for (int n = 0; n < NT; ++n) b[n] = *reinterpret_cast<const short8*>(wl + n * 2048 + at);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      const short8 a = *reinterpret_cast<const short8*>(sl + m * 2048 + at);
+#pragma unroll
+      for (int n = 0; n < NT; ++n) acc[m * NT + n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[n], a, acc[m * NT + n], 0, 0, 0);
+    }
   }
-  er_sums<MT>(smem, acc, wave, waves, [&](int m, floatx4 t) {
-    const int row = m * 16 + r16, col = n0 + 4 * g4;
+  er_sums<MT * NT>(smem, acc, wave, waves, [&](int i, floatx4 t) {
+    const int row = i / NT * 16 + r16, col = n0 + i % NT * 16 + 4 * g4;
     if (row < M) er_store<EPI>(Y + (long)row * N + col, bias + col, nullptr, t);
   });
 }
 
-// grid (N / 16), nh waves; QKV rows [q | k | v] of nh heads of 64 each; LDS: V [head][16 MT rows][128 bytes], the weight rows
-template <int MT>
+// grid (N / 16, tiles of `rows` queries), nh waves; QKV rows [q | k | v] of nh heads of 64 each; LDS: V [head][16 MT rows][128 bytes], the
+// weight rows.  Texts of 9 - 32 tokens as two tiles of half the queries (beyond 16, MQ 1 of MT 2): the softmax and the products of all 19
+// queries were 2.4 us of the workgroup's 4.6, and 48 workgroups leave CUs for as many more.
+template <int MQ, int MT>
 __global__ __launch_bounds__(64 * kErWaves, 1) void attn_rows_kernel(const bf16_t* __restrict__ QKV, long qs, int nh, float scale_log2,
                                                                      const bf16_t* __restrict__ W, const bf16_t* __restrict__ bias,
                                                                      const bf16_t* __restrict__ R, long rs, bf16_t* __restrict__ Y, int M,
-                                                                     int N) {
+                                                                     int N, int rows) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   typedef __attribute__((address_space(3))) short4_t* s4_ptr;
   constexpr int KS = (MT + 1) / 2;   // steps of 32 keys
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, g = lane >> 4;
-  const int K = nh * 64, n0 = blockIdx.x * 16;
+  const int K = nh * 64, n0 = blockIdx.x * 16, q0 = blockIdx.y * rows, MR = min(M - q0, rows);
+  R += (long)q0 * rs;
+  Y += (long)q0 * N;
   unsigned char* vl = smem + (long)wave * MT * 2048;
   unsigned char* wl = smem + (long)nh * MT * 2048 + wave * 2048;
   // this head's q and k as fragments (16 rows x 64 bytes), V and W through LDS-DMA
-  uint4_t qf[MT][2], kf[MT][2];
+  uint4_t qf[MQ][2], kf[MT][2];
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
-    const bf16_t* p = QKV + (long)min(16 * m + r16, M - 1) * qs + wave * 64 + 8 * g;   // rows past M repeat the last one
+    const bf16_t *p = QKV + wave * 64 + 8 * g, *k = p + K + (long)min(16 * m + r16, M - 1) * qs;   // rows past the last repeat it
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      qf[m][s] = *reinterpret_cast<const uint4_t*>(p + 32 * s);
-      kf[m][s] = *reinterpret_cast<const uint4_t*>(p + K + 32 * s);
+      if (m < MQ) qf[m < MQ ? m : 0][s] = *reinterpret_cast<const uint4_t*>(p + (long)(q0 + min(16 * m + r16, MR - 1)) * qs + 32 * s);
+      kf[m][s] = *reinterpret_cast<const uint4_t*>(k + 32 * s);
     }
   }
 #pragma unroll
@@ -195,10 +210,10 @@ __global__ __launch_bounds__(64 * kErWaves, 1) void attn_rows_kernel(const bf16_
                                      (rg_lptr)(vl + i * 1024), 16, 0, 0);
   er_load_w(W, n0, K, wave, wl);
 
-  short8 p[MT][KS];
-  float l[MT];
+  short8 p[MQ][KS];
+  float l[MQ];
 #pragma unroll
-  for (int m = 0; m < MT; ++m) {   // 16 queries: column r16; keys 16 t + 4 g + j
+  for (int m = 0; m < MQ; ++m) {   // 16 queries: column r16; keys 16 t + 4 g + j
     floatx4 s[MT];
     float mx = -INFINITY;
 #pragma unroll
@@ -238,11 +253,11 @@ __global__ __launch_bounds__(64 * kErWaves, 1) void attn_rows_kernel(const bf16_
   rg_wait<0>();   // this wave's V and W
   __builtin_amdgcn_sched_barrier(0);
   // O^T tile n: dims 16 n + 4 g + j of query r16
-  floatx4 o[4][MT], acc[MT];
+  floatx4 o[4][MQ], acc[MQ];
 #pragma unroll
   for (int n = 0; n < 4; ++n) {
 #pragma unroll
-    for (int m = 0; m < MT; ++m) o[n][m] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int m = 0; m < MQ; ++m) o[n][m] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int c = 0; c < KS; ++c) {
       const int r0 = 32 * c + 4 * g + (r16 >> 2), r1 = 2 * c + 1 < MT ? r0 + 16 : r0;   // (no second tile: P is zero there, V any row of the text)
@@ -251,12 +266,12 @@ __global__ __launch_bounds__(64 * kErWaves, 1) void attn_rows_kernel(const bf16_
       const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s4_ptr)(vl + r1 * 128 + ((ch ^ (r1 & 7)) << 4) + half));
       const short8 a = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
 #pragma unroll
-      for (int m = 0; m < MT; ++m) o[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, p[m][c], o[n][m], 0, 0, 0);
+      for (int m = 0; m < MQ; ++m) o[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, p[m][c], o[n][m], 0, 0, 0);
     }
   }
   // the product's two steps of 32 columns of this head, columns in O^T's order: 32 s + 4 g + j, then 32 s + 16 + 4 g + j
 #pragma unroll
-  for (int m = 0; m < MT; ++m) acc[m] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int m = 0; m < MQ; ++m) acc[m] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     const unsigned char* wr = wl + r16 * 128 + (g & 1) * 8;
@@ -264,7 +279,7 @@ __global__ __launch_bounds__(64 * kErWaves, 1) void attn_rows_kernel(const bf16_
     const short4_t hi = *reinterpret_cast<const short4_t*>(wr + (((4 * s + 2 + (g >> 1)) ^ (r16 & 7)) << 4));
     const short8 b = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
+    for (int m = 0; m < MQ; ++m) {
       uint4_t a;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
@@ -272,20 +287,20 @@ __global__ __launch_bounds__(64 * kErWaves, 1) void attn_rows_kernel(const bf16_
       acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, __builtin_bit_cast(short8, a), acc[m], 0, 0, 0);
     }
   }
-  er_sums<MT>(smem, acc, wave, nh, [&](int m, floatx4 t) {
+  er_sums<MQ>(smem, acc, wave, nh, [&](int m, floatx4 t) {
     const int row = m * 16 + r16, col = n0 + 4 * g;
-    if (row < M) er_store<ER_ADD>(Y + (long)row * N + col, bias + col, R + (long)row * rs + col, t);
+    if (row < MR) er_store<ER_ADD>(Y + (long)row * N + col, bias + col, R + (long)row * rs + col, t);
   });
 }
 
-constexpr int er_lds(int MT, int waves) { return waves * (MT + 1) * 2048; }   // (the sums' MT KB per wave lie over it)
+constexpr int er_lds(int MT, int waves, int NT = 1) { return waves * (MT + NT) * 2048; }   // (the sums' MT NT KB per wave lie over it)
 
-template <int MT, int EPI>
-int launch_ln(const void* s, long ss, const void* lw, const void* lb, float eps, void* h, const void* w, const void* b, void* y, int M, int N,
+template <int MT, int NT, int EPI>
+int launch_ln(int rows, const void* s, long ss, const void* lw, const void* lb, float eps, void* h, const void* w, const void* b, void* y, int M, int N,
               int K, hipStream_t st) {
-  LK_SET_MAX_LDS((ln_rows_kernel<MT, EPI>), er_lds(MT, kErWaves));
-  ln_rows_kernel<MT, EPI><<<dim3(N / 16, (M + kErRows - 1) / kErRows), K, er_lds(MT, K / 64), st>>>(
-      (const bf16_t*)s, ss, (const bf16_t*)lw, (const bf16_t*)lb, eps, (bf16_t*)h, (const bf16_t*)w, (const bf16_t*)b, (bf16_t*)y, M, N, K);
+  LK_SET_MAX_LDS((ln_rows_kernel<MT, NT, EPI>), er_lds(MT, kErWaves, NT));
+  ln_rows_kernel<MT, NT, EPI><<<dim3(N / (16 * NT), (M + rows - 1) / rows), K, er_lds(MT, K / 64, NT), st>>>(
+      (const bf16_t*)s, ss, (const bf16_t*)lw, (const bf16_t*)lb, eps, (bf16_t*)h, (const bf16_t*)w, (const bf16_t*)b, (bf16_t*)y, M, N, K, rows);
   LK_CHECK_LAUNCH();
   return 0;
 }
@@ -293,18 +308,19 @@ int launch_ln(const void* s, long ss, const void* lw, const void* lb, float eps,
 template <int EPI>
 int ln_by_rows(const void* s, long ss, const void* lw, const void* lb, float eps, void* h, const void* w, const void* b, void* y, int M, int N,
                int K, hipStream_t st) {
-  if (M <= 16) return launch_ln<1, EPI>(s, ss, lw, lb, eps, h, w, b, y, M, N, K, st);
-  if (M <= 32) return launch_ln<2, EPI>(s, ss, lw, lb, eps, h, w, b, y, M, N, K, st);
-  if (M <= 48) return launch_ln<3, EPI>(s, ss, lw, lb, eps, h, w, b, y, M, N, K, st);
-  return launch_ln<4, EPI>(s, ss, lw, lb, eps, h, w, b, y, M, N, K, st);
+  if (M > kErHalve && M <= 32 && N % 32 == 0) return launch_ln<1, 2, EPI>((M + 1) / 2, s, ss, lw, lb, eps, h, w, b, y, M, N, K, st);
+  if (M <= 16) return launch_ln<1, 1, EPI>(kErRows, s, ss, lw, lb, eps, h, w, b, y, M, N, K, st);
+  if (M <= 32) return launch_ln<2, 1, EPI>(kErRows, s, ss, lw, lb, eps, h, w, b, y, M, N, K, st);
+  if (M <= 48) return launch_ln<3, 1, EPI>(kErRows, s, ss, lw, lb, eps, h, w, b, y, M, N, K, st);
+  return launch_ln<4, 1, EPI>(kErRows, s, ss, lw, lb, eps, h, w, b, y, M, N, K, st);
 }
 
-template <int MT>
-int launch_attn(const void* qkv, long qs, int nh, float scale_log2, const void* w, const void* b, const void* r, long rs, void* y, int M, int N,
+template <int MQ, int MT>
+int launch_attn(int rows, const void* qkv, long qs, int nh, float scale_log2, const void* w, const void* b, const void* r, long rs, void* y, int M, int N,
                 hipStream_t st) {
-  LK_SET_MAX_LDS((attn_rows_kernel<MT>), er_lds(MT, kErWaves));
-  attn_rows_kernel<MT><<<dim3(N / 16), 64 * nh, er_lds(MT, nh), st>>>((const bf16_t*)qkv, qs, nh, scale_log2, (const bf16_t*)w, (const bf16_t*)b,
-                                                                      (const bf16_t*)r, rs, (bf16_t*)y, M, N);
+  LK_SET_MAX_LDS((attn_rows_kernel<MQ, MT>), er_lds(MT, kErWaves));
+  attn_rows_kernel<MQ, MT><<<dim3(N / 16, (M + rows - 1) / rows), 64 * nh, er_lds(MT, nh), st>>>((const bf16_t*)qkv, qs, nh, scale_log2, (const bf16_t*)w, (const bf16_t*)b,
+                                                                      (const bf16_t*)r, rs, (bf16_t*)y, M, N, rows);
   LK_CHECK_LAUNCH();
   return 0;
 }
@@ -331,6 +347,6 @@ int lk_attn_rows(const void* qkv, long qs, int nh, float scale, const void* w, c
                  hipStream_t st) {
   if (!lk_attn_rows_supported(M, nh, N)) return -1;
   const float s2 = scale * 1.4426950408889634f;
-  if (M <= 16) return launch_attn<1>(qkv, qs, nh, s2, w, b, r, rs, y, M, N, st);
-  return launch_attn<2>(qkv, qs, nh, s2, w, b, r, rs, y, M, N, st);
+  if (M <= 16) return launch_attn<1, 1>(M > kErHalve ? (M + 1) / 2 : 16, qkv, qs, nh, s2, w, b, r, rs, y, M, N, st);
+  return launch_attn<1, 2>((M + 1) / 2, qkv, qs, nh, s2, w, b, r, rs, y, M, N, st);
 }

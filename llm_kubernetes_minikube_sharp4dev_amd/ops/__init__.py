@@ -1067,12 +1067,12 @@ def linear_sums(x1, w1, x2, w2):
 
 
 # Encoder passes of few rows: the layer norms and the attention run inside the projections behind them (csrc/encoder_rows.hip).  Every
-# workgroup normalises all rows, so what a launch saves is lost again with more of them, sooner where the layers are narrow and each of
-# their launches is short: up to 32 rows at width 768, 16 below.  A captured pass, launches apart -> fused, us (cold: everything evicted before):
-#   12 layers of 768, one text of 8 / 16 / 19 / 32 / 48 / 64 tokens: 312 / 326 / 310 / 349 / 358 / 369 -> 256 / 278 / 300 / 337 / 389 / 415,
-#     cold 353 / 367 / 357 / 379 / 382 / 389 -> 281 / 302 / 323 / 356 / 397 / 423; 8 texts of 2 / of 4 tokens 325 / 351 -> 302 / 339
-#   6 layers of 384, one text of 8 / 16 / 22 / 32 / 64 tokens: 131 / 136 / 137 / 144 / 152 -> 127 / 137 / 145 / 152 / 196,
-#     cold 156 / 162 / 161 / 165 / 177 -> 143 / 154 / 160 / 168 / 211
+# workgroup normalises its tile's rows, so what a launch saves is lost again with more of them, sooner where the layers are narrow and each of
+# their launches is short: up to 32 rows at width 768, 16 below.  A captured pass, launches apart -> fused, us (cold: 512 MB read before):
+#   12 layers of 768, one text of 8 / 16 / 19 / 32 / 40 tokens: 299 / 316 / 314 / 344 / 343 -> 255 / 277 / 275 / 299 / 351,
+#     cold 350 / 365 / 357 / 376 / 373 -> 280 / 301 / 300 / 323 / 369; 8 texts of 2 / of 4 tokens 316 / 347 -> 306 / 324
+#   6 layers of 384, heads of 64, one text of 8 / 16 / 22 / 32 / 40 tokens: 131 / 133 / 133 / 134 / 136 -> 110 / 115 / 118 / 126 / 156,
+#     cold 155 / 158 / 156 / 158 / 158 -> 124 / 128 / 130 / 138 / 173; 8 texts of 2 / 3 / 4 tokens 134 / 134 / 136 -> 132 / 134 / 139
 ENCODER_ROWS = 32
 
 

@@ -225,3 +225,12 @@ def test_host_ids(hip, n):
     keep = host.clone()
     host.zero_()   # (the values have been taken)
     assert torch.equal(buf[:n].cpu(), keep) and int(buf[n]) == -7
+
+
+@pytest.mark.parametrize("M", [8, 9, 10, 31, 32])
+def test_two_row_tiles(hip, M):
+    """Both sides of the lines where a workgroup takes half the rows, even and odd numbers of them, and widths that the wider column tile does not divide."""
+    for K, N, gelu in ((768, 3072, True), (384, 1152, False), (64, 32, True), (320, 48, False)):
+        test_ln_linear(hip, M, K, N, gelu)
+    for nh, N in ((12, 768), (7, 448), (1, 16)):
+        test_attn_linear(hip, M, nh, N)
