@@ -1824,6 +1824,34 @@ c10::optional<at::Tensor> stream_gated_norm(at::Tensor& x, const at::Tensor& y, 
   return out;
 }
 
+// (the same's out, the causal convolution over each sequence's rows of it); one row per sequence.  Empty: the launch does not take the shapes
+std::vector<at::Tensor> stream_gated_norm_conv(at::Tensor& x, const at::Tensor& y, int64_t parts, const at::Tensor& g, const at::Tensor& gb,
+                                               const at::Tensor& wpost, const at::Tensor& wnext, double eps, const at::Tensor& cw, at::Tensor& state,
+                                               const at::Tensor& slots, const at::Tensor& positions) {
+  CHECK_CUDA(x); CHECK_F32(x); CHECK_CONTIG(x); CHECK_CUDA(y); CHECK_LASTDIM(y); CHECK_CUDA(g); CHECK_LASTDIM(g);
+  const int esz = esz_of(y, "y");
+  same_type(g, y, "g"); same_type(state, y, "state");
+  TORCH_CHECK(x.dim() == 2 && y.dim() == 2 && g.dim() == 2 && parts >= 1, "x, y, g must be 2-d");
+  const long T = x.size(0);
+  const int W = x.size(1);
+  TORCH_CHECK(y.size(0) == T * parts && y.size(1) == W && g.size(0) == T && g.size(1) == W, "y must be [T * parts, W], g [T, W]");
+  CHECK_CUDA(cw); CHECK_CUDA(state); CHECK_CONTIG(state); CHECK_I32(slots); CHECK_I32(positions); CHECK_CONTIG(slots); CHECK_CONTIG(positions);
+  TORCH_CHECK(cw.dim() == 2 && cw.size(0) == W && slots.numel() == T && positions.numel() >= T, "convolution operands");
+  const int taps = cw.size(1);
+  TORCH_CHECK(taps < 2 || (state.dim() == 3 && state.size(1) == taps - 1 && state.size(2) == W), "conv state must be [slots, taps - 1, W]");
+  const auto al = [](const at::Tensor& t, int bytes) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % bytes == 0 && (t.dim() < 2 || t.stride(0) * t.element_size() % bytes == 0); };
+  if (taps < 1 || taps > 4 || !lk_gated_norm_row(T, W, (int)parts, esz) || !al(x, 16) || !al(y, 8) || !al(g, 8) || !al(gb, 16) || !al(wpost, 16) ||
+      !al(wnext, 16) || !al(state, 8))
+    return {};
+  at::Tensor out = at::empty({T, W}, y.options()), hc = at::empty({T, W}, y.options());
+  CHECK_RC(lk_stream_gated_norm(x.data_ptr<float>(), y.data_ptr(), y.stride(0), (int)parts, g.data_ptr(), g.stride(0), fp(gb, W, "gate bias"),
+                                fp(wpost, W, "post norm weight"), fp(wnext, W, "next norm weight"), (float)eps, out.data_ptr(), out.stride(0), T, W,
+                                esz, cur_stream(), fp(cw, W * taps, "conv weight"), taps, state.data_ptr(), slots.data_ptr<int>(),
+                                positions.data_ptr<int>(), hc.data_ptr(), hc.stride(0)),
+           "stream_gated_norm_conv");
+  return {out, hc};
+}
+
 at::Tensor rms_cols(const at::Tensor& u, int64_t col0, int64_t n, const at::Tensor& w, double eps) {
   CHECK_CUDA(u); CHECK_LASTDIM(u);
   const int esz = esz_of(u, "u");
@@ -2427,6 +2455,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sinkattn_prefill", &sinkattn_prefill);
   m.def("sinkattn_decode", &sinkattn_decode);
   m.def("stream_gated_norm", &stream_gated_norm);
+  m.def("stream_gated_norm_conv", &stream_gated_norm_conv);
   m.def("rms_cols", &rms_cols);
   m.def("rot_kv_write", &rot_kv_write);
   m.def("pool_kv_write", &pool_kv_write);

@@ -349,7 +349,10 @@ int lk_sinkattn_decode(const void* q, long qs, const void* kc, const void* vc, c
 // csrc/window_ops.hip: gated + normed sublayer result into the f32 stream (+ the next norm), RMS norm of a column block,
 // pair rotation + key assembly + paged K / V write, pooled (mean) keys / values of finished blocks
 int lk_stream_gated_norm(float* x, const void* y, long ys, int parts, const void* g, long gs, const float* gb, const float* wpost,
-                         const float* wnext, float eps, void* out, long os, long rows, int W, int esz, hipStream_t st);
+                         const float* wnext, float eps, void* out, long os, long rows, int W, int esz, hipStream_t st,
+                         const float* cw = nullptr, int taps = 0, void* cstate = nullptr, const int* slots = nullptr,
+                         const int* positions = nullptr, void* cout = nullptr, long cos = 0);
+bool lk_gated_norm_row(long rows, int W, int parts, int esz);   // the convolution (cout) can ride in the launch
 int lk_rms_cols(const void* u, long us, int n, const float* w, float eps, void* out, long os, long rows, int esz, hipStream_t st);
 int lk_rot_kv_write(void* q, long qs, int H, int qdim, const void* k, long ks, int G, int kdim, const void* sh, long shs, int sdim,
                     const void* v, long vs, int vdim, int rot_off, int rot, const float* freq, float mag, const int* positions,

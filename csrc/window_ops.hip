@@ -126,6 +126,120 @@ __global__ __launch_bounds__(256) void stream_gated_norm_kernel(float* __restric
   }
 }
 
+// The same for steps of few rows (bf16), whose time is the trips to memory behind each other: everything that a row reads is requested
+// before anything waits (columns past the row are its last again, and not used).  With many rows the registers cost more waves than the trips.  CONV: the causal convolution over each sequence's rows
+// that the next sublayer opens with (conv_silu_vec_kernel of csrc/ssm.hip with one token per sequence, without activation and bias; the
+// normed row as it rounds is its input): its columns are this thread's, so only the weights and the state's rows come on top and a launch less.
+struct GatedConv {
+  const float* w;     // [W][taps]
+  int taps;
+  bf16_t* state;      // [slots][taps - 1][W]
+  const int* slots;   // per row; < 0: zeros, and no state
+  const int* positions;
+  bf16_t* out;
+  long os;
+};
+template <int MAXI, int PARTS, bool CONV>
+__global__ __launch_bounds__(512) void gated_norm_row_kernel(float* __restrict__ x, const bf16_t* __restrict__ y, long ys,
+                                                             const bf16_t* __restrict__ g, long gs, const float* __restrict__ gb,
+                                                             const float* __restrict__ wpost, const float* __restrict__ wnext, float eps,
+                                                             bf16_t* __restrict__ out, long os, int W, GatedConv cv) {
+  __shared__ float red[8];
+  const long row = blockIdx.x;
+  const int ng = W / 4;
+  int col[MAXI];
+  bool on[MAXI];
+#pragma unroll
+  for (int i = 0; i < MAXI; ++i) {
+    on[i] = (int)threadIdx.x + 512 * i < ng;
+    col[i] = 4 * min((int)threadIdx.x + 512 * i, ng - 1);
+  }
+  short4_t yr[MAXI][PARTS], gr[MAXI], sr[MAXI][3];
+  floatx4 bv[MAXI], xv[MAXI], wp[MAXI], wn[MAXI];
+  float wk[MAXI][4][4];   // [tap, of four][column]
+  int slot = -1, pos = 0;
+  const bool w4 = CONV && cv.taps == 4 && (reinterpret_cast<uintptr_t>(cv.w) & 15) == 0;   // a column's taps in one 16-byte load
+  if constexpr (CONV) slot = cv.slots[row], pos = cv.positions[row];
+#pragma unroll
+  for (int i = 0; i < MAXI; ++i) {
+#pragma unroll
+    for (int p = 0; p < PARTS; ++p) yr[i][p] = *reinterpret_cast<const short4_t*>(y + (row * PARTS + p) * ys + col[i]);
+    gr[i] = *reinterpret_cast<const short4_t*>(g + row * gs + col[i]);
+    bv[i] = *reinterpret_cast<const floatx4*>(gb + col[i]);
+    xv[i] = *reinterpret_cast<const floatx4*>(x + row * W + col[i]);
+    wp[i] = *reinterpret_cast<const floatx4*>(wpost + col[i]);
+    if (out) wn[i] = *reinterpret_cast<const floatx4*>(wnext + col[i]);
+    if constexpr (CONV) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (w4) {
+          const floatx4 t = *reinterpret_cast<const floatx4*>(cv.w + (long)(col[i] + e) * 4);
+#pragma unroll
+          for (int k = 0; k < 4; ++k) wk[i][k][e] = t[k];
+        } else {
+#pragma unroll
+          for (int k = 0; k < 4; ++k) wk[i][k][e] = k >= 4 - cv.taps ? cv.w[(long)(col[i] + e) * cv.taps + (k - (4 - cv.taps))] : 0.f;
+        }
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {   // the input 3 - d tokens ago: row taps - 4 + d of the state
+        const int si = cv.taps - 4 + d;
+        sr[i][d] = short4_t{0, 0, 0, 0};
+        if (si >= 0 && slot >= 0) sr[i][d] = *reinterpret_cast<const short4_t*>(cv.state + ((long)slot * (cv.taps - 1) + si) * W + col[i]);
+      }
+    }
+  }
+  float ss = 0.f, s2 = 0.f;
+  floatx4 v[MAXI];
+#pragma unroll
+  for (int i = 0; i < MAXI; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float a = bf2f((bf16_t)yr[i][0][e]);
+#pragma unroll
+      for (int p = 1; p < PARTS; ++p) a += bf2f((bf16_t)yr[i][p][e]);
+      const float val = PARTS > 1 ? a * (1.f / (float)PARTS) : a;
+      v[i][e] = val / (1.f + expf(-(bf2f((bf16_t)gr[i][e]) + bv[i][e])));
+      if (on[i]) ss += v[i][e] * v[i][e];
+    }
+  ss = block_sum<8>(ss, red);
+  const float inv1 = 1.f / sqrtf(ss / (float)W + eps);
+#pragma unroll
+  for (int i = 0; i < MAXI; ++i) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      v[i][e] = xv[i][e] + v[i][e] * inv1 * wp[i][e];
+      if (on[i]) s2 += v[i][e] * v[i][e];
+    }
+    if (on[i]) *reinterpret_cast<floatx4*>(x + row * W + col[i]) = v[i];
+  }
+  if (!out) return;
+  s2 = block_sum<8>(s2, red);
+  const float inv2 = 1.f / sqrtf(s2 / (float)W + eps);
+#pragma unroll
+  for (int i = 0; i < MAXI; ++i) {
+    if (!on[i]) continue;
+    const floatx4 r = v[i] * inv2 * wn[i];
+    const short4_t h = {(short)f2bf(r[0]), (short)f2bf(r[1]), (short)f2bf(r[2]), (short)f2bf(r[3])};
+    *reinterpret_cast<short4_t*>(out + row * os + col[i]) = h;
+    if constexpr (CONV) {
+      short4_t c = {0, 0, 0, 0};
+      if (slot >= 0) {
+        if (pos <= 0) sr[i][0] = sr[i][1] = sr[i][2] = c;   // no past
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          c[e] = (short)f2bf(wk[i][0][e] * bf2f((bf16_t)sr[i][0][e]) + wk[i][1][e] * bf2f((bf16_t)sr[i][1][e]) + wk[i][2][e] * bf2f((bf16_t)sr[i][2][e]) +
+                             wk[i][3][e] * bf2f((bf16_t)h[e]));
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+          const int si = cv.taps - 4 + d;
+          if (si >= 0) *reinterpret_cast<short4_t*>(cv.state + ((long)slot * (cv.taps - 1) + si) * W + col[i]) = d < 2 ? sr[i][d < 2 ? d + 1 : 2] : h;
+        }
+      }
+      *reinterpret_cast<short4_t*>(cv.out + row * cv.os + col[i]) = c;
+    }
+  }
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void rms_cols_kernel(const T* __restrict__ u, long us, int n, const float* __restrict__ w, float eps,
                                                        T* __restrict__ out, long os) {
@@ -446,8 +560,16 @@ int gated_norm_t(float* x, const void* y, long ys, int parts, const void* g, lon
 
 }  // namespace
 
+// Whether a step of this many rows takes the row kernel.  us before / with it, 2,048 columns in two parts: 64 rows 4.3 / 3.1, 256 4.7 / 3.5, 512 5.3 / 4.7,
+// 1,024 7.4 / 6.9, 2,048 12.2 / 12.4; 8,192 columns: 64 9.9 / 6.2, 1,024 23.3 / 22.3, 2,048 40.5 / 40.4.  Up to 1,024 columns, where half of the
+// threads or more idle: 64 rows 3.4 / 3.0, 256 3.6 / 3.3, 512 4.1 / 4.3, 1,024 4.8 / 5.7.
+bool lk_gated_norm_row(long rows, int W, int parts, int esz) {
+  return esz == 2 && rows <= (W > 1024 ? 1024 : 256) && W % 4 == 0 && W >= 4 && W <= 4 * 512 * 4 && (parts == 1 || parts == 2);
+}
+
 int lk_stream_gated_norm(float* x, const void* y, long ys, int parts, const void* g, long gs, const float* gb, const float* wpost,
-                         const float* wnext, float eps, void* out, long os, long rows, int W, int esz, hipStream_t st) {
+                         const float* wnext, float eps, void* out, long os, long rows, int W, int esz, hipStream_t st, const float* cw, int taps,
+                         void* cstate, const int* slots, const int* positions, void* cout, long cos) {
   if (rows <= 0) return 0;
   if (parts < 1 || W < 1 || !y || !g || !gb || !wpost || (out && !wnext)) return -1;
   const auto al = [](const void* p, long stride_bytes, int vec_bytes) {
@@ -456,6 +578,29 @@ int lk_stream_gated_norm(float* x, const void* y, long ys, int parts, const void
   const int tv = esz == 2 ? 8 : 16;
   const bool vec = W % 4 == 0 && al(x, (long)W * 4, 16) && al(gb, 0, 16) && al(wpost, 0, 16) && al(wnext, 0, 16) &&
                    al(y, ys * (long)esz, tv) && al(g, gs * (long)esz, tv) && al(out, os * (long)esz, tv);
+  const bool conv = cout != nullptr;
+  if (conv && (!out || !cw || !slots || !positions || taps < 1 || taps > 4 || (taps > 1 && !cstate) || !al(cstate, (long)W * 2, 8) ||
+               !al(cout, cos * 2, 8)))
+    return -1;
+  if (vec && lk_gated_norm_row(rows, W, parts, esz)) {
+    const GatedConv cv{cw, taps, (bf16_t*)cstate, slots, positions, (bf16_t*)cout, cos};
+#define LK_ROW(I, P, C)                                                                                                                  \
+  gated_norm_row_kernel<I, P, C><<<(unsigned)rows, 512, 0, st>>>(x, (const bf16_t*)y, ys, (const bf16_t*)g, gs, gb, wpost, wnext, eps,   \
+                                                                 (bf16_t*)out, os, W, cv)
+#define LK_ROWS(I)                                              \
+  do {                                                          \
+    if (parts == 1) { if (conv) LK_ROW(I, 1, true); else LK_ROW(I, 1, false); } \
+    else { if (conv) LK_ROW(I, 2, true); else LK_ROW(I, 2, false); }       \
+  } while (0)
+    if (W <= 2048) LK_ROWS(1);
+    else if (W <= 4096) LK_ROWS(2);
+    else LK_ROWS(4);
+#undef LK_ROWS
+#undef LK_ROW
+    LK_CHECK_LAUNCH();
+    return 0;
+  }
+  if (conv) return -1;
   return esz == 2 ? gated_norm_t<bf16_t>(x, y, ys, parts, g, gs, gb, wpost, wnext, eps, out, os, rows, W, vec, st)
                   : gated_norm_t<float>(x, y, ys, parts, g, gs, gb, wpost, wnext, eps, out, os, rows, W, vec, st);
 }

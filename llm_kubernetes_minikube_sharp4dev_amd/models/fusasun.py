@@ -331,11 +331,12 @@ class FusasunModel(nn.Module):
         return self.cache_block_bytes(1)
 
     # ------------------------------------------------------------------ forward
-    def _attended(self, L: FusasunLayer, h, meta: AttnMeta, cache):
-        """The mixer's heads; its output projection runs beside the layer's first gate."""
+    def _attended(self, L: FusasunLayer, h, meta: AttnMeta, cache, hc=None):
+        """The mixer's heads; its output projection runs beside the layer's first gate.  ``hc``: the convolution's rows, where they exist."""
         W = self.cfg.hidden
-        hc = ops.conv_silu(h, 0, W, L.canon, None, cache[-1], meta.seq_cu, meta.state_slots, meta.positions, meta.max_seq_len,
-                           act=False)
+        if hc is None:
+            hc = ops.conv_silu(h, 0, W, L.canon, None, cache[-1], meta.seq_cu, meta.state_slots, meta.positions, meta.max_seq_len,
+                               act=False)
         M = L.mix
         u = ops.linear(hc, M.w_in)
         if L.type == "attention":
@@ -363,18 +364,27 @@ class FusasunModel(nn.Module):
         eps = cfg.norm_eps
         x, _ = ops.embed_stream(ids, self.embed, self.dtype, cfg.embed_scale)
         h = ops.stream_rmsnorm(x, w=self.layers[0].norm1, eps=eps, out_dtype=self.dtype)
-        n, routes = len(self.layers), self._routes(ids)
+        n, routes, hc = len(self.layers), self._routes(ids), None
+
+        def normed(y, g, gb, post, i, parts=1):
+            """The stream takes y, gated, in; -> (the norm that opens layer i, the convolution behind it)."""
+            if i == n:
+                return ops.stream_gated_norm(x, y, g, gb, post, None, eps, self.dtype, parts=parts), None
+            L = self.layers[i]
+            return ops.stream_gated_norm_conv(x, y, g, gb, post, L.norm1, eps, self.dtype, parts, L.canon, caches[i][-1], meta.seq_cu, meta.state_slots,
+                                              meta.positions, meta.max_seq_len)
+
         for i, L in enumerate(self.layers):
             # the first gate reads h and is as large as the output projection: one launch for both
-            g, y = ops.linear_pair(h, L.rg1, self._attended(L, h, meta, caches[i]), L.mix.o)
-            nxt = L.norm2 if L.mlp is not None else (self.layers[i + 1].norm1 if i + 1 < n else None)
-            h = ops.stream_gated_norm(x, y, g, L.rg1_b, L.norm1b, nxt, eps, self.dtype)
-            if L.mlp is not None:
+            g, y = ops.linear_pair(h, L.rg1, self._attended(L, h, meta, caches[i], hc), L.mix.o)
+            if L.mlp is None:
+                h, hc = normed(y, g, L.rg1_b, L.norm1b, i + 1)
+            else:
+                h = ops.stream_gated_norm(x, y, g, L.rg1_b, L.norm1b, L.norm2, eps, self.dtype)
                 X = L.mlp
                 g = ops.linear(h, L.rg2)
                 y = ops.table_experts(h, ids, X.table, X.gate_up, X.down, X.top, routes[i])
-                nxt = self.layers[i + 1].norm1 if i + 1 < n else None
-                h = ops.stream_gated_norm(x, y, g, L.rg2_b, L.norm2b, nxt, eps, self.dtype, parts=X.top)
+                h, hc = normed(y, g, L.rg2_b, L.norm2b, i + 1, X.top)
             if taps is not None:
                 taps.append(x.clone())
         idx = meta.logits_idx

@@ -20,12 +20,13 @@ import torch
 import torch.nn.functional as F
 
 from ._ext import lib, use_hip
+from .mixers import conv_silu
 
 # from this many (token, choice) pairs per expert on average the experts run on the dense GEMM's tiles (_grouped)
 GROUPED_DENSE_MIN_ROWS = 128
 GROUPED_FINE_MIN_ROWS = 64
 
-__all__ = ["stream_gated_norm", "rms_cols", "rot_kv_write", "pool_kv_write", "table_experts", "run_experts", "moe_route", "moe_routes"]
+__all__ = ["stream_gated_norm", "stream_gated_norm_conv", "rms_cols", "rot_kv_write", "pool_kv_write", "table_experts", "run_experts", "moe_route", "moe_routes"]
 
 
 def stream_gated_norm(x, y, g, g_bias, w_post, w_next, eps: float, out_dtype=torch.bfloat16, parts: int = 1):
@@ -43,6 +44,17 @@ def stream_gated_norm(x, y, g, g_bias, w_post, w_next, eps: float, out_dtype=tor
     if w_next is None:
         return None
     return (x / torch.sqrt(x.pow(2).mean(-1, keepdim=True) + eps) * w_next).to(out_dtype)
+
+
+def stream_gated_norm_conv(x, y, g, g_bias, w_post, w_next, eps: float, out_dtype, parts: int, conv_w, state, cu, slots, positions, max_len: int):
+    """(h, hc): :func:`stream_gated_norm`'s rows h and their causal convolution ``conv_silu(h, ..., act=False)`` per sequence;
+    one launch where every sequence has one row."""
+    if use_hip(x) and max_len == 1 and slots.numel() == x.shape[0] and y.dtype == out_dtype == state.dtype == torch.bfloat16:
+        both = lib().stream_gated_norm_conv(x, y, int(parts), g, g_bias, w_post, w_next, float(eps), conv_w, state, slots, positions)
+        if both:
+            return tuple(both)
+    h = stream_gated_norm(x, y, g, g_bias, w_post, w_next, eps, out_dtype, parts)
+    return h, conv_silu(h, 0, h.shape[1], conv_w, None, state, cu, slots, positions, max_len, act=False)
 
 
 def rms_cols(u, col0: int, n: int, w, eps: float):

@@ -306,6 +306,32 @@ def test_gated_stream_update_and_column_norm(W, parts, device, dtype):
     assert rel_err(got, O.rms(u[:, 5:W + 2], eps) * w.double()) < (3e-6 if dtype == torch.float32 else 1e-2)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("W,parts,taps,T", [(4, 1, 4, 1), (100, 2, 4, 5), (2048, 2, 4, 64), (2052, 1, 3, 1024), (4100, 2, 2, 7), (8192, 1, 1, 3),
+                                            (2048, 1, 4, 1025), (1024, 2, 4, 256), (1024, 2, 4, 257), (64, 3, 4, 9), (2048, 2, 5, 4)])
+def test_gated_norm_with_the_next_convolution(W, parts, taps, T):
+    """The row kernel's widths around its column tiles (2,048, 4,096, 8,192), the fewest and most taps, rows without a slot and without a past, and
+    past each limit the general kernels: the stream within the two orders' rounding, the convolution the bits of its own
+    kernel on the same rows (the same expression; bf16 may round the other way where a product is contracted: 1 part in 256)."""
+    g = torch.Generator().manual_seed(W + T)
+    d = lambda t: t.cuda()
+    x, y, gate = rnd(g, T, W).float(), d(rnd(g, T * parts, W).bfloat16()), d(rnd(g, T, W + 8).bfloat16())[:, :W]
+    gb, wp, wn = d(rnd(g, W).float()), d(rnd(g, W).float() + 1), d(rnd(g, W).float() + 1)
+    cw, state = d(rnd(g, W, taps).float()), d(rnd(g, T + 2, max(taps - 1, 1), W).bfloat16())
+    slots = torch.randperm(T + 2, generator=g)[:T].int()
+    slots[1::7] = -1
+    pos = torch.arange(T, dtype=torch.int32) % 3
+    cu, slots, pos = d(torch.arange(T + 1, dtype=torch.int32)), d(slots), d(pos)
+    xd, s1, s2 = d(x.clone()), state.clone(), state.clone()
+    h, hc = ops.stream_gated_norm_conv(xd, y, gate, gb, wp, wn, 1e-5, torch.bfloat16, parts, cw, s1, cu, slots, pos, 1)
+    v = y.double().view(T, parts, W).mean(1) * torch.sigmoid(gate.double() + gb)
+    wx = d(x).double() + O.rms(v, 1e-5) * wp.double()
+    assert rel_err(xd, wx.cpu()) < 3e-6 and rel_err(h, (O.rms(wx, 1e-5) * wn.double()).cpu()) < 1e-2
+    want = ops.conv_silu(h, 0, W, cw, None, s2, cu, slots, pos, 1, act=False)
+    assert torch.equal(s1, s2)
+    assert ((hc.float() - want.float()).abs() <= want.float().abs() / 128 + 1e-6).all()
+
+
 @pytest.mark.parametrize("device,dtype", ALL)
 @pytest.mark.parametrize("W,ff,E,top,T", [(48, 20, 5, 2, 37), (36, 13, 1, 1, 5), (50, 24, 7, 3, 70), (256, 128, 8, 2, 130),
                                           (64, 40, 2, 2, 150), (72, 100, 3, 1, 333), (44, 12, 2, 2, 100), (64, 24, 2, 2, 300), (128, 128, 2, 1, 700), (192, 256, 3, 2, 600)])
