@@ -82,12 +82,16 @@ __global__ __launch_bounds__(256) void conv_silu_kernel(const T* __restrict__ u,
 // The same for taps <= 4 with 16-byte accesses: a thread owns EV adjacent channels and walks its `rows`
 // tokens with the three previous inputs in registers (weights right-aligned in a 4-tap window, the
 // unused leading taps zero), so every input row is read once per tile instead of once per tap.
-// Needs C % EV == 0 and 16-byte aligned rows of u, out and the state.  new_state != null (steps of single tokens): the thread also
-// leaves its channels' last inputs there (the same tensor as `state`: it has read them before).
-template <typename T>
+// Needs C % EV == 0 and 16-byte aligned rows of u, out and the state.  The sequence's first tile also leaves the channels' last inputs
+// in the state (nobody else reads it), without a launch of its own.  GR: rows requested together, a group ahead of the one in use (1: steps of
+// single tokens; 8 are level, 16 slower by half, from registers).  A thread's weights are 128 bytes from its neighbour's, so that loading them
+// cost as much as 8 rows: a tile's come in one sweep and are turned round in LDS.  bf16 x 6,144 channels, before / now, us: four sequences of 1,024
+// tokens 28.2 / 23.1 (100 MB: 4.4 TB/s), 32 of 200 45.7 / 37.8, one of 900 15.1 / 11.0, of 60 6.9 / 5.5, 64 single tokens 4.7 / 4.4; x 2,048
+// 16.1 / 13.0, 20.2 / 16.9, 8.5 / 5.8, 6.9 / 5.5, 4.2 / 4.1.
+template <typename T, int GR>
 __global__ __launch_bounds__(256) void conv_silu_vec_kernel(const T* __restrict__ u, long us, int C, int taps,
                                                             const float* __restrict__ w, const float* __restrict__ bias,
-                                                            const T* state, T* new_state, const int* __restrict__ cu,
+                                                            T* state, const int* __restrict__ cu,
                                                             const int* __restrict__ slots,
                                                             const int* __restrict__ positions, T* __restrict__ out,
                                                             long os, int act, int rows) {
@@ -95,16 +99,16 @@ __global__ __launch_bounds__(256) void conv_silu_vec_kernel(const T* __restrict_
   const int s = blockIdx.x, c0 = (blockIdx.z * 256 + threadIdx.x) * EV;
   const int row0 = cu[s], len = cu[s + 1] - row0, slot = slots[s];
   const int i0 = blockIdx.y * rows;
-  if (c0 >= C || i0 >= len) return;
+  if (i0 >= len) return;   // (the whole workgroup)
   const int i1 = min(len, i0 + rows);
-  auto ldrow = [&](const T* p, float (&f)[EV]) {
-    if constexpr (sizeof(T) == 2) {
-      load8(p, f);
-    } else {
-      const floatx4 v = *reinterpret_cast<const floatx4*>(p);
+  const bool on = c0 < C;
+  using Row = std::conditional_t<sizeof(T) == 2, short8, floatx4>;
+  auto ldrow = [&](const T* p) { return *reinterpret_cast<const Row*>(p); };
+  auto flt = [&](const Row& v, float (&f)[EV]) {
 #pragma unroll
-      for (int e = 0; e < EV; ++e) f[e] = v[e];
-    }
+    for (int e = 0; e < EV; ++e)
+      if constexpr (sizeof(T) == 2) f[e] = bf2f((bf16_t)v[e]);
+      else f[e] = v[e];
   };
   auto strow = [&](T* p, const float (&f)[EV]) {
     if constexpr (sizeof(T) == 2) {
@@ -117,59 +121,105 @@ __global__ __launch_bounds__(256) void conv_silu_vec_kernel(const T* __restrict_
     float z[EV];
 #pragma unroll
     for (int e = 0; e < EV; ++e) z[e] = 0.f;
-    for (int i = i0; i < i1; ++i) strow(out + (long)(row0 + i) * os + c0, z);
+    for (int i = i0; i < i1 && on; ++i) strow(out + (long)(row0 + i) * os + c0, z);
     return;
   }
   const bool past = positions[row0] > 0;
+  Row cur[GR], old[3], last[3];   // old[3 - d] = the input d tokens before the tile's first; last: the sequence's new state
+  const Row zero = {};
   float wk[4][EV], b[EV], win[3][EV];
   const bool w4 = taps == 4 && (reinterpret_cast<uintptr_t>(w) & 15) == 0;   // a channel's taps in one 16-byte load
+  auto rows_of = [&](int i) {
+#pragma unroll
+    for (int x = 0; x < GR; ++x) cur[x] = ldrow(u + (long)(row0 + min(i + x, i1 - 1)) * us + c0);
+  };
+  if constexpr (GR == 1)
+    if (on && w4)
+#pragma unroll
+      for (int e = 0; e < EV; ++e) {
+        const floatx4 v = *reinterpret_cast<const floatx4*>(w + (long)(c0 + e) * 4);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) wk[k][e] = v[k];
+      }
+  if (on) {
+    rows_of(i0);
+#pragma unroll
+    for (int d = 3; d >= 1; --d) {
+      const int idx = i0 - d, si = taps - 1 + idx, at = len - d;
+      old[3 - d] = last[3 - d] = zero;
+      if (d <= taps - 1) {
+        if (idx >= 0) old[3 - d] = ldrow(u + (long)(row0 + idx) * us + c0);
+        else if (si >= 0) old[3 - d] = ldrow(state + ((long)slot * (taps - 1) + si) * C + c0);   // (the position may be on its way)
+        if (GR > 1 && i0 == 0 && at >= 0) last[3 - d] = ldrow(u + (long)(row0 + at) * us + c0);
+      }
+    }
+  }
+  if constexpr (GR > 1) {
+    // the block's weights in one sweep, turned round in LDS (9 places for 8, so that the threads' reads, 128 bytes apart, meet different banks)
+    __shared__ floatx4 sw[256 * EV + 256 * EV / 8];
+    if (w4) {
+      const int b0 = blockIdx.z * 256 * EV;
+      for (int c = threadIdx.x; c < min(256 * EV, C - b0); c += 256) sw[c + c / 8] = *reinterpret_cast<const floatx4*>(w + (long)(b0 + c) * 4);
+      __syncthreads();
+#pragma unroll
+      for (int e = 0; e < EV; ++e) {
+        const int c = threadIdx.x * EV + e;
+        const floatx4 v = sw[on ? c + c / 8 : 0];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) wk[k][e] = v[k];
+      }
+    }
+  }
+  if (!on) return;
 #pragma unroll
   for (int e = 0; e < EV; ++e) {
     b[e] = bias ? bias[c0 + e] : 0.f;
-    if (w4) {
-      const floatx4 v = *reinterpret_cast<const floatx4*>(w + (long)(c0 + e) * 4);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) wk[k][e] = v[k];
-    } else {
+    if (!w4)
 #pragma unroll
       for (int k = 0; k < 4; ++k) wk[k][e] = k >= 4 - taps ? w[(long)(c0 + e) * taps + (k - (4 - taps))] : 0.f;
-    }
   }
 #pragma unroll
-  for (int d = 3; d >= 1; --d) {  // win[3 - d] = the input d tokens before the tile's first
-    const int idx = i0 - d, si = taps - 1 + idx;
+  for (int x = 0; x < 3; ++x) {
+    if (i0 - 3 + x < 0 && !past) old[x] = zero;
+    flt(old[x], win[x]);
+  }
+  if (i0 == 0) {   // the first tile has read the old state, so it writes the new one: the last taps - 1 of [state, inputs]
 #pragma unroll
-    for (int e = 0; e < EV; ++e) win[3 - d][e] = 0.f;
-    if (d <= taps - 1) {
-      if (idx >= 0) ldrow(u + (long)(row0 + idx) * us + c0, win[3 - d]);
-      else if (past && si >= 0) ldrow(state + ((long)slot * (taps - 1) + si) * C + c0, win[3 - d]);
+    for (int x = 0; x < 3; ++x) {
+      const int si = taps - 4 + x;   // row of the state: the input 3 - x tokens before the end
+      if (si < 0) continue;
+      Row v = last[x];
+      if (GR == 1) {                 // (one token)
+        v = x < 2 ? old[x < 2 ? x + 1 : 2] : cur[0];
+      } else if (len - 3 + x < 0) {  // of the old state (len is 1 or 2): old[x + len], a token earlier per input
+        v = zero;
+#pragma unroll
+        for (int n = 1; n < 3; ++n)
+          if (len == n && x + n < 3) v = old[x + n < 3 ? x + n : 2];
+      }
+      *reinterpret_cast<Row*>(state + ((long)slot * (taps - 1) + si) * C + c0) = v;
     }
   }
-  // (rows in groups of four, requested together: the window slides over values in registers)
-  for (int i = i0; i < i1; i += 4) {
-    float cur[4][EV];
+  // (rows in groups, the next group's requested before this one's are used: the window slides over values in registers)
+  for (int i = i0; i < i1; i += GR) {
+    Row now[GR];
 #pragma unroll
-    for (int x = 0; x < 4; ++x) ldrow(u + (long)(row0 + min(i + x, i1 - 1)) * us + c0, cur[x]);
+    for (int x = 0; x < GR; ++x) now[x] = cur[x];
+    if (i + GR < i1) rows_of(i + GR);
 #pragma unroll
-    for (int x = 0; x < 4; ++x) {
+    for (int x = 0; x < GR; ++x) {
       if (i + x >= i1) break;
-      float r[EV];
+      float r[EV], in[EV];
+      flt(now[x], in);
 #pragma unroll
       for (int e = 0; e < EV; ++e) {
-        const float acc = b[e] + wk[0][e] * win[0][e] + wk[1][e] * win[1][e] + wk[2][e] * win[2][e] + wk[3][e] * cur[x][e];
+        const float acc = b[e] + wk[0][e] * win[0][e] + wk[1][e] * win[1][e] + wk[2][e] * win[2][e] + wk[3][e] * in[e];
         r[e] = act ? silu_f<sizeof(T) == 4>(acc) : acc;
         win[0][e] = win[1][e];
         win[1][e] = win[2][e];
-        win[2][e] = cur[x][e];
+        win[2][e] = in[e];
       }
       strow(out + (long)(row0 + i + x) * os + c0, r);
-    }
-  }
-  if (new_state) {
-#pragma unroll
-    for (int x = 0; x < 3; ++x) {   // win[x] is the input 3 - x - 1 tokens before the last one
-      const int si = taps - 4 + x;
-      if (si >= 0) strow(new_state + ((long)slot * (taps - 1) + si) * C + c0, win[x]);
     }
   }
 }
@@ -1463,9 +1513,9 @@ int scan_t(const T* xbc, long xs, const T* dtp, long dts, long rows, int S, int 
 }  // namespace
 
 // Tokens per workgroup of the convolution, which walks them in fours behind each other: 4 or 8 where that leaves about a workgroup or two to a CU, 16
-// where shorter tiles would not all be on the chip at once.  bf16 x 6,144 channels, 4 / 8 / 16 tokens (us, with the state's launch): one sequence of
-// 60 7.8 / 9.0 / 11.8, of 300 8.9 / 9.6 / 12.2, of 900 16.5 / 14.5 / 14.2, of 2,000 30 / 22.0 / 21.2, four of 1,024 45 / 37 / 28.9; x 2,048
-// 18.8 / 16.2 / 17.6, x 512 8.2 / 8.7 / 11.0
+// where shorter tiles would not all be on the chip at once.  bf16 x 6,144 channels, us, what is taken / 8 / 32 tokens: one sequence of 60
+// 5.5 / 6.6 / 13.5, of 300 5.9 / 7.0 / 13.8, of 900 11.0 / 11.0 / 15.1, of 2,000 16.1 / 16.5 / 17.1, four of 1,024 23.1 / 26.3 / 24.4, 32 of 200
+// 37.8 / 40.8 / 35.9; x 2,048, four of 1,024 13.0 / 13.1 / 16.2; x 512 5.9 / 5.9 / 12.4
 int lk_conv_rows(int S, int cblocks, int max_len, int cus) {
   const auto groups = [&](int r) { return (long)S * cblocks * ((max_len + r - 1) / r); };
   return groups(4) * 256 <= 300L * cus ? 4 : groups(8) * 256 <= 600L * cus ? 8 : kConvRows;
@@ -1482,22 +1532,17 @@ int lk_conv_silu(const void* u, long us, int C, int taps, const float* w, const 
   if (taps <= 4 && C % ev == 0 && us % ev == 0 && os % ev == 0 && a16(u) && a16(out) && a16(state)) {
     const int cblocks = (C / ev + 255) / 256;
     const int rows = lk_conv_rows(S, cblocks, max_len, cu_count());
-    const bool one = max_len == 1;
     dim3 gv(S, (max_len + rows - 1) / rows, cblocks);
-    if (esz == 2)
-      conv_silu_vec_kernel<bf16_t><<<gv, 256, 0, st>>>((const bf16_t*)u, us, C, taps, w, bias, (const bf16_t*)state,
-                                                       one && taps > 1 ? (bf16_t*)state : nullptr, cu, slots, positions, (bf16_t*)out, os,
-                                                       act, rows);
-    else
-      conv_silu_vec_kernel<float><<<gv, 256, 0, st>>>((const float*)u, us, C, taps, w, bias, (const float*)state,
-                                                      one && taps > 1 ? (float*)state : nullptr, cu, slots, positions, (float*)out, os, act,
-                                                      rows);
-    LK_CHECK_LAUNCH();
-    if (taps > 1 && !one) {
-      if (esz == 2) conv_state_kernel<bf16_t><<<g2, 256, 0, st>>>((const bf16_t*)u, us, C, taps, (bf16_t*)state, cu, slots, positions);
-      else conv_state_kernel<float><<<g2, 256, 0, st>>>((const float*)u, us, C, taps, (float*)state, cu, slots, positions);
-      LK_CHECK_LAUNCH();
+#define LK_CONV(T, GR) conv_silu_vec_kernel<T, GR><<<gv, 256, 0, st>>>((const T*)u, us, C, taps, w, bias, (T*)state, cu, slots, positions, (T*)out, os, act, rows)
+    if (max_len == 1) {
+      if (esz == 2) LK_CONV(bf16_t, 1);
+      else LK_CONV(float, 1);
+    } else {
+      if (esz == 2) LK_CONV(bf16_t, 4);
+      else LK_CONV(float, 4);
     }
+#undef LK_CONV
+    LK_CHECK_LAUNCH();
     return 0;
   }
   if (esz == 2) {

@@ -154,3 +154,38 @@ def test_conv_tiles(hip, lens, C, later):
         assert bool(((y[int(cu[s]):int(cu[s + 1])] - want).abs() <= bound * (1 + 2.0 ** -8)).all())
         assert torch.equal(state[S - s], x[-(taps - 1):])
     assert torch.equal(state[0], before[0])
+
+
+@pytest.mark.parametrize("C", [8, 1024, 2040, 2056, 4104])
+@pytest.mark.parametrize("taps", [1, 2, 3, 4])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("lens", [[1, 1, 1], [2, 1, 3, 9, 0]])
+def test_conv_channel_blocks(hip, C, taps, dtype, lens):
+    """Channels that end inside a block of the weights' sweep (2,048 in bf16, 1,024 in f32), every window, portions shorter than the state with a
+    past and without, a sequence without a slot and one without rows: the state is the bits of the last inputs."""
+    g = torch.Generator(device=DEV).manual_seed(C + taps)
+    T, S = sum(lens), len(lens)
+    u, w = torch.randn(T, C, device=DEV, generator=g).to(dtype), torch.randn(C, taps, device=DEV, generator=g)
+    state = torch.randn(S + 1, max(taps - 1, 1), C, device=DEV, generator=g).to(dtype)
+    cu = torch.tensor([sum(lens[:i]) for i in range(S + 1)], dtype=torch.int32, device=DEV)
+    slots = torch.arange(S, 0, -1, device=DEV).to(torch.int32)
+    slots[1] = -1
+    pos = torch.cat([torch.arange(n) + 3 * (i % 2 == 0) * (i < 3) for i, n in enumerate(lens)]).to(torch.int32).to(DEV)
+    before = state.clone()
+    y = hip.conv_silu(u, 0, C, w, None, state, cu, slots, pos, max(lens), False).double()
+    for s, n in enumerate(lens):
+        if s == 1:
+            assert not y[int(cu[s]):int(cu[s + 1])].any()
+            continue
+        past = before[S - s][:taps - 1]
+        x = torch.cat([past if n and int(pos[int(cu[s])]) else torch.zeros_like(past), u[int(cu[s]):int(cu[s + 1])]])
+        want = sum((x[k:k + n].double() * w[:, k].double() for k in range(taps)), torch.zeros(n, C, dtype=torch.float64, device=DEV))
+        size = sum((x[k:k + n].double().abs() * w[:, k].double().abs() for k in range(taps)), torch.zeros(n, C, dtype=torch.float64, device=DEV))
+        # the result's rounding, the sum's five f32 roundings
+        bound = (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -24) * want.abs() + 5 * 2.0 ** -24 * size
+        assert bool(((y[int(cu[s]):int(cu[s + 1])] - want).abs() <= bound * (1 + 2.0 ** -8)).all())
+        if n and taps > 1:
+            assert torch.equal(state[S - s], x[-(taps - 1):])
+        else:
+            assert torch.equal(state[S - s], before[S - s])
+    assert torch.equal(state[S - 1], before[S - 1]) and torch.equal(state[0], before[0])
