@@ -80,9 +80,15 @@ struct PrefillParams {
 // NW waves per workgroup (4 or 8): WH of them share a row group (one head each), and
 // NW / WH row groups of 32 queries sit on top of each other, all fed by the same staged
 // K/V tile -- with NW = 8 each K/V byte brought into LDS serves 2x the MFMA work.
-template <int D, bool CAUSAL, bool PAGED, int WH, int NW, bool PIPE>
-__global__ __launch_bounds__(64 * NW, 8 / NW) void flash_prefill_kernel(PrefillParams p) {
-  constexpr int NT = 64 * NW;      // threads
+// KS = 2: two such sets of waves with LDS of their own take every other key tile of the same rows and add their sums up at the end.  Alone on
+// its CU a workgroup waits for every link of a tile's chain (scores, maximum, exponentials, values: 2 us, of which the matrix units work
+// 0.5), so where the grid leaves a CU to one workgroup the most key tiles of any are the time.  32 / 8 heads of 128, us: 949 rows 32.2 -> 26.6,
+// 1,500 51.4 -> 38.0, 512 rows over 4,096 keys 124 -> 88; 8 heads of a 64-column model, 700 rows, 16.6 -> 13.9.
+template <int D, bool CAUSAL, bool PAGED, int WH, int NW, bool PIPE, int KS = 1>
+__global__ __launch_bounds__(64 * NW * KS, 8 / (NW * KS)) void flash_prefill_kernel(PrefillParams p) {
+  static_assert(KS == 1 || (KS == 2 && PIPE && NW == 4), "two sets of four waves");
+  constexpr int NT = 64 * NW;      // threads of a set
+  constexpr int NB = PIPE ? 2 : 1;  // tiles of K and of V in LDS
   constexpr int KK = D / 16;       // QK k-steps
   constexpr int ND = D / 32;       // O^T d tiles
   constexpr int CPR = D / 8;       // 16-byte chunks per row
@@ -92,9 +98,11 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void flash_prefill_kernel(PrefillP
   constexpr int QB = 32 * WR;
   static_assert(CPT >= 1 && NCH % NT == 0, "tile too small for the workgroup");
 
-  __shared__ __attribute__((aligned(16))) bf16_t lds[2 * KT * D];
+  __shared__ __attribute__((aligned(16))) bf16_t lds_all[KS * NB * 2 * KT * D];
 
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int set = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / NT);
+  const int tid = threadIdx.x - set * NT, lane = tid & 63, w = tid >> 6;
+  bf16_t* lds = lds_all + set * NB * 2 * KT * D;
   const int r = lane & 31, h = lane >> 5;
   const int G = p.Hq / p.Hkv;
   // XCD-aware order: the hardware deals workgroups round-robin over the 8 XCDs (each with its own
@@ -351,8 +359,10 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void flash_prefill_kernel(PrefillP
   };
 
   bf16_t* Ks = lds;
-  bf16_t* Vs = lds + KT * D;
+  bf16_t* Vs = lds + NB * KT * D;
   const int ntiles = (kend + KT - 1) / KT;
+  const int nt = KS == 1 ? ntiles : (ntiles - set + 1) / 2;  // this set's: the keys from key(t) on, 0 <= t < nt (set 0 has the most)
+  auto key = [&](int t) __attribute__((always_inline)) { return (KS * t + set) * KT; };
   floatx16 s[2];
   short8 pf[2][2];
   if constexpr (!PIPE) {
@@ -380,54 +390,98 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void flash_prefill_kernel(PrefillP
   } else if (ntiles > 0) {
     // Software-pipelined by one tile: iteration t runs QK(t), then PV(t-1) in the same basic
     // block as the exponentials of tile t (independent work the scheduler interleaves: MFMA
-    // next to VALU within the wave), then O <- (O + P(t-1) V(t-1)) * alpha(t).  The LDS holds
-    // K(t) and V(t-1); after each tile K(t+1) and V(t) are written and K(t+2) / V(t+1) issued.
-    auto stage = [&](int t) __attribute__((always_inline)) {
-      __syncthreads();  // K(t) and V(t-1) read by everyone
-      if (t + 1 < ntiles) swrite_k(Ks);
-      swrite_v(Vs);
-      __syncthreads();
-      if (t + 2 < ntiles) gload_k((t + 2) * KT);
-      if (t + 1 < ntiles) gload_v((t + 1) * KT);
+    // next to VALU within the wave), then O <- (O + P(t-1) V(t-1)) * alpha(t).  LDS holds two tiles
+    // of each: in iteration t K(t+1) and V(t), requested in the one before, are written beside K(t) and
+    // V(t-1), which are being read, and K(t+2) / V(t+1) requested; one barrier ends it.
+    constexpr int kTile = KT * D;
+    auto refill = [&](int t) __attribute__((always_inline)) {
+      if (t + 1 < nt) swrite_k(Ks + ((t + 1) & 1) * kTile);
+      if (KS == 1 || t < nt) swrite_v(Vs + (t & 1) * kTile);
+      if (t + 2 < nt) gload_k(key(t + 2));
+      if (t + 1 < nt) gload_v(key(t + 1));
     };
-    gload_k(0);
-    gload_v(0);
-    swrite_k(Ks);
-    if (ntiles > 1) gload_k(KT);
-    __syncthreads();
     short8 pfp[2][2];
-    {
-      qk(Ks, s);
-      float base;
-      const float alpha = stats(0, s, &base, std::true_type{});
-      exp_pack(s, base, alpha, pfp);
-      stage(0);
+    if (KS == 1 || nt > 0) {
+      gload_k(key(0));
+      gload_v(key(0));
+      swrite_k(Ks);
+      if (nt > 1) gload_k(key(1));
     }
-    auto step = [&](int t, auto may_mask) __attribute__((always_inline)) {
+    __syncthreads();
+    if (KS == 1 || nt > 0) {
       qk(Ks, s);
+      refill(0);
       float base;
-      const float alpha = stats(t * KT, s, &base, may_mask);
-      pv(Vs, pfp);
+      const float alpha = stats(key(0), s, &base, std::true_type{});
+      exp_pack(s, base, alpha, pfp);
+    }
+    __syncthreads();
+    auto step = [&](int t, auto may_mask) __attribute__((always_inline)) {
+      qk(Ks + (t & 1) * kTile, s);
+      refill(t);
+      float base;
+      const float alpha = stats(key(t), s, &base, may_mask);
+      pv(Vs + ((t - 1) & 1) * kTile, pfp);
       exp_pack(s, base, alpha, pf);
       rescale(alpha);
 #pragma unroll
       for (int m = 0; m < 2; ++m)
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2) pfp[m][s2] = pf[m][s2];
-      stage(t);
+      __syncthreads();
     };
     // leading tiles that no row of the workgroup masks: a branch-free body, so the row max
     // is scheduled next to PV(t-1) too.  (Unrolling by two to swap pf / pfp instead of
     // copying them takes the kernel to 256 VGPRs and spills.)
-    const int nfree = min(ntiles, min(ctx / KT, CAUSAL ? (past + q0 + 1) / KT : ntiles));
+    const int whole = min(ctx / KT, CAUSAL ? (past + q0 + 1) / KT : ntiles);
+    const int nfree = min(nt, KS == 1 ? whole : (whole - set + 1) / 2);
     int t = 1;
     for (; t < nfree; ++t) step(t, std::false_type{});
-    for (; t < ntiles; ++t) step(t, std::true_type{});
-    pv(Vs, pfp);
+    for (; t < nt; ++t) step(t, std::true_type{});
+    if constexpr (KS > 1) {
+      if (set == 1 && t < (ntiles + 1) / 2) __syncthreads();  // set 0 has a tile more: its barrier
+    }
+    if (KS == 1 || nt > 0) pv(Vs + ((nt - 1) & 1) * kTile, pfp);
   }
 
+  // ---- two sets: both take the larger base and the whole sum, each hands the other half of its columns over and keeps the rest
+  if constexpr (KS > 1) {
+    float* x = reinterpret_cast<float*>(lds_all);
+    __syncthreads();  // (K and V read)
+    x[set * 2 * NT + tid] = m_run;
+    x[set * 2 * NT + NT + tid] = l_run;
+    __syncthreads();
+    const float mo = x[(set ^ 1) * 2 * NT + tid], lo = x[(set ^ 1) * 2 * NT + NT + tid];
+    const float m = fmaxf(m_run, mo), base = m == -INFINITY ? 0.f : m;
+    const float mine = __builtin_amdgcn_exp2f(m_run - base), other = __builtin_amdgcn_exp2f(mo - base);
+    l_run = set == 0 ? l_run * mine + lo * other : lo * other + l_run * mine;
+    __syncthreads();
+    floatx4* xo = reinterpret_cast<floatx4*>(lds_all) + set * (ND / 2) * 4 * NT + tid;
+#pragma unroll
+    for (int n = 0; n < ND / 2; ++n)
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4) {
+        floatx4 v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = (set == 0 ? o[ND / 2 + n][4 * g4 + i] : o[n][4 * g4 + i]) * mine;
+        xo[(4 * n + g4) * NT] = v;
+      }
+    __syncthreads();
+    xo = reinterpret_cast<floatx4*>(lds_all) + (set ^ 1) * (ND / 2) * 4 * NT + tid;
+#pragma unroll
+    for (int n = 0; n < ND / 2; ++n)
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4) {
+        const floatx4 v = xo[(4 * n + g4) * NT];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[n][4 * g4 + i] = (set == 0 ? o[n][4 * g4 + i] : o[ND / 2 + n][4 * g4 + i]) * mine + v[i];
+      }
+  }
+  constexpr int NO = ND / KS;               // the columns that this set writes
+  const int n0 = KS == 1 ? 0 : set * NO;
+
   // ---- epilogue: O^T lane layout: d = 32n + (i&3) + 8(i>>2) + 4h, query row = qrow
-  if (qvalid && p.part_o) {
+  if (KS == 1 && qvalid && p.part_o) {
     const long pr = (long)(qbeg + qrow) * p.Hq + head;
     float* po = p.part_o + pr * D;
 #pragma unroll
@@ -446,9 +500,9 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void flash_prefill_kernel(PrefillP
     // 2k+1 whole, so the row is written with 16-B stores (half the store instructions of the
     // issue-bound tail: CDNA playbook T21).  The swap runs on every lane (the pair shares qvalid).
     const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
-    bf16_t* op = p.out + (long)(qbeg + qrow) * p.os + (long)head * D;
+    bf16_t* op = p.out + (long)(qbeg + qrow) * p.os + (long)head * D + 32 * n0;
 #pragma unroll
-    for (int n = 0; n < ND; ++n)
+    for (int n = 0; n < NO; ++n)
 #pragma unroll
       for (int g2 = 0; g2 < 2; ++g2) {
         unsigned a[2], b[2];
@@ -545,6 +599,24 @@ long lk_prefill_pairs(long ntiles, int groups, int threads) {
   return n * threads < (1L << 32) ? n : 0;
 }
 
+static int cu_count() {
+  static const int n = [] {
+    int dev = 0, v = 0;
+    return hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0 ? v : 256;
+  }();
+  return n;
+}
+
+// Whether `groups` workgroups over paged keys run as two sets of waves each (causal, heads of 64 or 128).  Up to one workgroup per CU that pays
+// from about three key tiles in a chain on (us, plain / two sets: 100 rows 9.3 / 9.4, 130 9.7 / 9.7, 200 11.6 / 11.2, 8 x 100 9.7 / 10.5,
+// 2 x 500 20.6 / 18.6); up to two, which the plain kernel runs side by side, only where few long chains outlast the rest: 1,500 51.4 / 38.0,
+// 2,000 68 / 57, 2 x 600 24.3 / 20.9, 2 x 1,000 39.1 / 37.6, but 3 x 400 19.2 / 19.7, 4 x 500 25.4 / 28.6.  Past that it is the slower one
+// (3,000 105 / 117).  The keys before the rows are not known here; a short piece of a long prompt runs plain.
+int lk_prefill_split_keys(long groups, long rows, long seqs, int cus) {
+  if (groups <= cus) return rows >= 160 * seqs;
+  return groups <= 2 * cus && 4 * rows >= 7 * groups * seqs;
+}
+
 int lk_flash_prefill(const bf16_t* q, long qs, const bf16_t* k, const bf16_t* v, long ks, long vs,
                      const int* block_tables, int bt_stride, const int* cu_q, const int* ctx_lens,
                      const int* tile_seq, const int* tile_q0, int ntiles, bf16_t* out, long os,
@@ -578,6 +650,15 @@ int lk_flash_prefill(const bf16_t* q, long qs, const bf16_t* k, const bf16_t* v,
     grid = dim3((unsigned)paired);
   }
   const bool pipe = causal && prefill_pipe();
+  if (pipe && paged && D >= 64 && NW == 4 && !part_o && lk_prefill_split_keys((long)ntiles * (Hq / WH), rows, seqs, cu_count())) {
+#define LS(DD, W) flash_prefill_kernel<DD, true, true, W, 4, true, 2><<<grid, 512, 0, st>>>(pr)
+#define LS_W(DD) if (WH == 4) LS(DD, 4); else if (WH == 2) LS(DD, 2); else LS(DD, 1)
+    if (D == 128) { LS_W(128); }
+    else { LS_W(64); }
+#undef LS_W
+#undef LS
+    return 0;
+  }
 #define L(DD, C, PG, W, N)                                                        \
   if (pipe) flash_prefill_kernel<DD, C, PG, W, N, true><<<grid, 64 * N, 0, st>>>(pr); \
   else flash_prefill_kernel<DD, C, PG, W, N, false><<<grid, 64 * N, 0, st>>>(pr)

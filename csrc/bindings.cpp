@@ -2613,6 +2613,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("M"), py::arg("N"), py::arg("K"), py::arg("swiglu"), py::arg("variant"));
   m.def("prefill_pairs", &lk_prefill_pairs, "", py::arg("ntiles"), py::arg("groups"), py::arg("threads"));
   m.def("prefill_order", &lk_prefill_order, "", py::arg("ntiles"), py::arg("seqs"), py::arg("rows"), py::arg("heads"), py::arg("D"));
+  m.def("prefill_split_keys", &lk_prefill_split_keys, "", py::arg("groups"), py::arg("rows"), py::arg("seqs"), py::arg("cus"));
   m.def("flash_prefill", &flash_prefill, "", py::arg("q"), py::arg("k"), py::arg("v"), py::arg("block_tables"), py::arg("cu_q"), py::arg("ctx_lens"), py::arg("tile_seq"), py::arg("tile_q0"), py::arg("Hq"), py::arg("Hkv"), py::arg("D"), py::arg("scale"), py::arg("causal"), py::arg("out") = py::none(), py::arg("part_o") = py::none(), py::arg("part_ml") = py::none(), py::arg("q_past") = py::none());
   m.def("knn_topk", &knn_topk, "", py::arg("corpus"), py::arg("cnorm"), py::arg("queries"), py::arg("qnorm"),
         py::arg("K"), py::arg("force_fused") = false);

@@ -210,6 +210,7 @@ int lk_paged_decode(const bf16_t* q, long qs, const bf16_t* kc, const bf16_t* vc
 int lk_prefill_rows_per_tile(int G, int D);
 long lk_prefill_pairs(long ntiles, int groups, int threads);
 int lk_prefill_order(long ntiles, long seqs, long rows, int heads, int D);
+int lk_prefill_split_keys(long groups, long rows, long seqs, int cus);
 int lk_flash_prefill(const bf16_t* q, long qs, const bf16_t* k, const bf16_t* v, long ks, long vs,
                      const int* block_tables, int bt_stride, const int* cu_q, const int* ctx_lens,
                      const int* tile_seq, const int* tile_q0, int ntiles, bf16_t* out, long os,

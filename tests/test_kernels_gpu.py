@@ -266,6 +266,30 @@ def test_flash_prefill_paged(G, D, BS):
     _close(y, y_ref, 0.02, 0.0, "flash prefill paged")
 
 
+@pytest.mark.parametrize("G,D,BS", [(1, 64, 16), (2, 128, 16), (4, 64, 128), (4, 128, 8), (8, 128, 16)])
+@pytest.mark.parametrize("q_lens,past", [([160], [0]), ([193], [0]), ([320, 1], [0, 700]), ([257], [63]), ([180], [129])])
+def test_flash_prefill_two_sets_of_waves(hip, G, D, BS, q_lens, past):
+    """Few long rows: two sets of waves take every other key tile, among them chains of one tile (none for the second set), of even and odd
+    numbers, with a partly masked last one in either set.  The bound is the plain kernel's: P and the result in bf16."""
+    torch.manual_seed(11)
+    Hkv = 2
+    Hq = Hkv * G
+    ctx = [a + b for a, b in zip(q_lens, past)]
+    T = sum(q_lens)
+    rows = ops.prefill_rows_per_tile(G, D)
+    groups = sum(-(-n // rows) for n in q_lens) * Hq // min(G, 4)
+    assert hip.prefill_split_keys(groups, T, len(q_lens), 256)
+    kc, vc, bt = _paged_setup(len(ctx), ctx, Hkv, D, BS, seed=12)
+    q = torch.randn(T, Hq * D, device=DEV, dtype=torch.bfloat16)
+    q[T // 2] *= 8  # (a row whose maximum jumps from tile to tile)
+    cu = torch.tensor([0] + list(torch.tensor(q_lens).cumsum(0)), dtype=torch.int32, device=DEV)
+    cl = torch.tensor(ctx, dtype=torch.int32, device=DEV)
+    scale = 1 / math.sqrt(D)
+    y = ops.flash_prefill(q, kc, vc, cu, Hq, Hkv, D, scale, True, block_tables=bt, ctx_lens=cl, q_lens_cpu=q_lens, ctx_lens_cpu=ctx)
+    y_ref = ref.flash_prefill(q, kc, vc, bt, cu.cpu(), cl.cpu(), Hq, Hkv, D, scale, True)
+    _close(y, y_ref, 0.02, 0.0, "flash prefill, two sets")
+
+
 @pytest.mark.parametrize("D", [32, 64, 128])
 def test_flash_encoder_dense(D):
     torch.manual_seed(9)

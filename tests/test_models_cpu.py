@@ -551,6 +551,19 @@ def test_encoder_attention_order_by_its_texts(texts, rows, heads, D, order):
     assert _ext.lib().prefill_order(tiles, texts, rows * texts, heads, D) == order
 
 
+@pytest.mark.parametrize("lens,Hq,Hkv,two", [([159], 32, 8, 0), ([160], 32, 8, 1), ([100] * 8, 32, 8, 0), ([1024], 32, 8, 1), ([2048], 32, 8, 1), ([2049], 32, 8, 0),
+                                             ([400] * 3, 32, 8, 0), ([600] * 2, 32, 8, 1), ([500] * 4, 32, 8, 0), ([1500], 32, 32, 1)])
+def test_prompt_attention_splits_keys_where_few_chains_are_long(lens, Hq, Hkv, two):
+    from llm_kubernetes_minikube_sharp4dev_amd.ops import _ext
+
+    if not _ext.available():
+        pytest.skip("the kernel library is not built")
+    G = Hq // Hkv
+    rows = 32 if G >= 4 else 32 * (4 // G)
+    groups = sum(-(-n // rows) for n in lens) * Hq // min(G, 4)
+    assert _ext.lib().prefill_split_keys(groups, sum(lens), len(lens), 256) == two
+
+
 @pytest.mark.parametrize("S,cblocks,max_len,rows", [(1, 3, 60, 4), (1, 3, 400, 4), (1, 3, 401, 8), (1, 3, 1600, 8), (1, 3, 1601, 16), (4, 3, 1024, 16), (300, 1, 1, 4),
                                                     (600, 1, 2, 8), (601, 1, 8, 16)])
 def test_convolution_tiles_count_the_devices_cus(S, cblocks, max_len, rows):
