@@ -73,6 +73,13 @@ LK_DEVICE void dot8(const uint4_t wv, const uint4_t xv, float& acc) {
   }
 }
 
+// a barrier that leaves loads to registers in flight
+LK_DEVICE void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// What bounds it: the weights' stream, and before it the prologue (two or three trips to memory and LDS, 1 - 2 us), under which the first
+// chunks' requests now fly: 16 KB a wave, what a CU takes in in 5 us.  Cold, us, one row / two: 6144 x 4096 with the norm 11.1 -> 10.8 / 12.6 ->
+// 11.6, 4096 x 4096 8.0 -> 7.5 / 8.7 -> 8.5, 28672 x 4096 SwiGLU 41.1 -> 39.8 / 43.2 -> 41.2, 4096 x 14336 21.7 (as before) / 24.3 -> 23.7,
+// 2048 x 2048 3.7 -> 3.4.  Requests for the next pair ahead of a pair's sums were slower (11.5, 41.1, 23.2): half the waves fit.
 template <int MR, int PRO, int MODE, int U, int KW>
 __global__ __launch_bounds__(256) void gemv_decode_kernel(GemvArgs g) {
   constexpr bool NORM = PRO == 1;
@@ -126,6 +133,31 @@ __global__ __launch_bounds__(256) void gemv_decode_kernel(GemvArgs g) {
     if constexpr (NORM)
       __builtin_amdgcn_global_load_lds((gemv_gptr)(g.gamma + (c0 + lane) * 8), (gemv_lptr)(gs + c0 * 8), 16, 0, 0);
   }
+  // the first U chunks of this wave's first pair, behind the requests for X (loads return in order) and ahead of all that waits for it;
+  // PRO 2's merge loads come later, and would wait for these
+  constexpr int PPW = 4 / KW;  // pairs per workgroup per round
+  const int ps = wv / KW, kh = wv % KW;
+  const int kc_w = kc_lane / KW;  // chunks per lane of this wave's part of K
+  const int jb = kh * kc_w;
+  long ra = 0, rb = 0;
+  int hd = 0, head = 0, ip = 0;
+  uint4_t va[U], vb[U];
+  auto load_w = [&](int j0) __attribute__((always_inline)) {
+    const uint4_t* wa = reinterpret_cast<const uint4_t*>(g.w + ra * K) + lane;
+    const uint4_t* wb = reinterpret_cast<const uint4_t*>(g.w + rb * K) + lane;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      va[u] = __builtin_nontemporal_load(wa + (j0 + u) * 64);
+      vb[u] = __builtin_nontemporal_load(wb + (j0 + u) * 64);
+    }
+  };
+  constexpr bool EARLY = PRO != 2;
+  if constexpr (EARLY) {
+    __builtin_amdgcn_sched_barrier(0);
+    pair_rows(min((int)blockIdx.x * PPW + ps, g.npairs - 1), ra, rb, hd, head, ip);  // (a wave without a pair: a load that nobody uses)
+    load_w(jb);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   if constexpr (PRO == 2) {
 #pragma unroll
     for (int m = 0; m < MR; ++m) {
@@ -157,8 +189,9 @@ __global__ __launch_bounds__(256) void gemv_decode_kernel(GemvArgs g) {
       }
     }
   }
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0) (lgkmcnt / expcnt untouched)
-  __syncthreads();
+  constexpr int NEWER = EARLY ? 2 * U : 0;
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (NEWER & 15) | (NEWER >> 4) << 14);  // vmcnt(NEWER) (lgkmcnt / expcnt untouched)
+  lds_barrier();
   if constexpr (NORM) {
     // RMSNorm with rmsnorm_kernel's rounding: y = bf16(bf16(v * inv) * g), in place in LDS
 #pragma unroll
@@ -175,7 +208,7 @@ __global__ __launch_bounds__(256) void gemv_decode_kernel(GemvArgs g) {
       ss = wave_sum(ss);
       if (lane == 0) red[m * 4 + wv] = ss;
     }
-    __syncthreads();
+    lds_barrier();
 #pragma unroll
     for (int m = 0; m < MR; ++m) {
       const float tot = red[m * 4] + red[m * 4 + 1] + red[m * 4 + 2] + red[m * 4 + 3];
@@ -193,37 +226,24 @@ __global__ __launch_bounds__(256) void gemv_decode_kernel(GemvArgs g) {
         *reinterpret_cast<uint4_t*>(xs + m * K + c * 8) = o;
       }
     }
-    __syncthreads();
+    lds_barrier();
   }
 
   // ---- stream W: one pair of rows per KW waves at a time (KW = 2: the two waves take one half of
   // K each and their sums meet in LDS -- twice the loads in flight for the long-K projections).
   // The round loop is uniform over the workgroup (its barriers), a wave past the last pair idles.
-  constexpr int PPW = 4 / KW;  // pairs per workgroup per round
-  const int ps = wv / KW, kh = wv % KW;
-  const int kc_w = kc_lane / KW;  // chunks per lane of this wave's part of K
-  const int jb = kh * kc_w;
   __shared__ float red2[KW > 1 ? PPW : 1][MR][2];
   for (int pb = blockIdx.x * PPW; pb < g.npairs; pb += gridDim.x * PPW) {
     const int p = pb + ps;
     const bool valid = p < g.npairs;
-    long ra = 0, rb = 0;
-    int hd = 0, head = 0, ip = 0;
     float acc_a[MR], acc_b[MR];
 #pragma unroll
     for (int m = 0; m < MR; ++m) acc_a[m] = acc_b[m] = 0.f;
     if (valid) {
       pair_rows(p, ra, rb, hd, head, ip);
-      const uint4_t* wa = reinterpret_cast<const uint4_t*>(g.w + ra * K) + lane;
-      const uint4_t* wb = reinterpret_cast<const uint4_t*>(g.w + rb * K) + lane;
       const uint4_t* xl = reinterpret_cast<const uint4_t*>(xs) + lane;
       for (int j0 = jb; j0 < jb + kc_w; j0 += U) {
-        uint4_t va[U], vb[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          va[u] = __builtin_nontemporal_load(wa + (j0 + u) * 64);
-          vb[u] = __builtin_nontemporal_load(wb + (j0 + u) * 64);
-        }
+        if (!EARLY || j0 != jb || pb != (int)blockIdx.x * PPW) load_w(j0);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
 #pragma unroll
