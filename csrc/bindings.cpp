@@ -1557,6 +1557,33 @@ std::vector<at::Tensor> embed_stream(const at::Tensor& ids, const at::Tensor& to
   return {x, copy};
 }
 
+// {x, norm, copy}: embed_pos (with positions) or embed_stream, then stream_rmsnorm, in one launch where the sizes allow it
+std::vector<at::Tensor> embed_norm(const at::Tensor& ids, const at::Tensor& tok, const at::Tensor& w, double woff, double eps, double scale,
+                                   const c10::optional<at::Tensor>& positions, const c10::optional<at::Tensor>& pos, bool keep_copy) {
+  CHECK_CUDA(ids); CHECK_I32(ids); CHECK_CONTIG(ids); CHECK_CUDA(tok); CHECK_CONTIG(tok);
+  const int esz = esz_of(tok, "tok");
+  TORCH_CHECK(tok.dim() == 2 && positions.has_value() == pos.has_value() && (!positions || scale == 1.0) && (positions || !keep_copy), "embed_norm");
+  const long T = ids.numel();
+  const int W = tok.size(1);
+  if (positions) {
+    CHECK_CUDA(*positions); CHECK_I32(*positions); CHECK_CONTIG(*positions);
+    same_type(tok, *pos, "pos");
+    TORCH_CHECK(pos->dim() == 2 && pos->is_contiguous() && pos->size(1) == W && positions->numel() == T, "tables");
+  }
+  at::Tensor x = at::empty({T, W}, tok.options().dtype(at::kFloat)), h = at::empty({T, W}, tok.options());
+  at::Tensor copy = keep_copy ? at::empty({T, W}, x.options()) : at::Tensor();
+  const int rc = lk_embed_norm(ip(ids), positions ? ip(*positions) : nullptr, tok.data_ptr(), tok.size(0), pos ? pos->data_ptr() : nullptr,
+                               pos ? pos->size(0) : 0, (float)scale, T, W, x.data_ptr<float>(), keep_copy ? copy.data_ptr<float>() : nullptr,
+                               fp(w, W, "w"), (float)woff, (float)eps, h.data_ptr(), esz, cur_stream());
+  if (rc == 1) {
+    auto r = positions ? embed_pos(ids, *positions, tok, *pos, keep_copy) : embed_stream(ids, tok, tok.scalar_type(), scale);
+    h = stream_rmsnorm(r[0], c10::nullopt, c10::nullopt, c10::nullopt, c10::nullopt, 1.0, w, woff, eps, c10::nullopt, tok.scalar_type());
+    return {r[0], h, keep_copy ? r[1] : at::Tensor()};
+  }
+  CHECK_RC(rc, "embed_norm");
+  return {x, h, copy};
+}
+
 at::Tensor stream_layernorm(at::Tensor& x, const c10::optional<at::Tensor>& y, const c10::optional<at::Tensor>& ls, double alpha,
                             const at::Tensor& w, const at::Tensor& b, double eps, const c10::optional<at::Tensor>& idx,
                             at::ScalarType out_dtype) {
@@ -2443,6 +2470,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("ssm_piped", &lk_ssm_piped, "", py::arg("S"), py::arg("heads"), py::arg("P"), py::arg("N"), py::arg("max_len"), py::arg("rows"), py::arg("cus"));
   m.def("gated_group_rmsnorm", &gated_group_rmsnorm);
   m.def("embed_stream", &embed_stream);
+  m.def("embed_norm", &embed_norm);
   m.def("stream_layernorm", &stream_layernorm);
   m.def("gelu_tanh_mul", &gelu_tanh_mul);
   m.def("dual_rmsnorm_mean", &dual_rmsnorm_mean);

@@ -269,6 +269,8 @@ int lk_scatter_ids(int* ids, const long* dst, const int* prev, const long* src, 
 int lk_gather_rows(bf16_t* out, const bf16_t* x, long xs, const long* idx, long R, int H, hipStream_t st);
 
 // csrc/stream_f32.hip: f32 residual stream (esz = element size of the bf16 / f32 activations)
+int lk_embed_norm(const int* ids, const int* positions, const void* tok, long vocab, const void* pos, int max_pos, float scale, long rows, int W,
+                  float* x, float* copy, const float* w, float woff, float eps, void* out, int esz, hipStream_t st);
 int lk_embed_pos(const int* ids, const int* positions, const void* tok, int vocab, const void* pos, int max_pos, long rows,
                  int W, float* x, float* copy, int esz, hipStream_t st);
 int lk_stream_embed_errors();  // ids / positions outside their tables seen by lk_embed_pos (their rows are zero)

@@ -152,6 +152,64 @@ __global__ __launch_bounds__(256) void stream_rmsnorm_vec_kernel(float* __restri
   }
 }
 
+// The stream's first rows and their norm: x f32 = token row (+ position row) * scale (kept twice with `copy`), out = the norm of it, as
+// embed_pos_kernel / the embedding of stream_ln.hip and then the kernel above give them, to the bit.  W % 4 == 0, W <= 1024 MAXV, aligned
+// rows.  A row was two launches, the first with a trip to memory for every 256 columns: 64 x 2,048 8.4 (with a copy that nobody read) + 4.3 ->
+// 5.2 us, with positions 7.4 + 3.7 -> 7.0; 4,095 x 2,048 23.5 + 9.2 -> 18.2, with positions 20.7 + 9.0 -> 20.5.  positions: an id or position outside its table gives zeros and is counted; without, ids are clamped.
+template <typename T, int MAXV>
+__global__ __launch_bounds__(256) void embed_norm_kernel(const int* __restrict__ ids, const int* __restrict__ positions, const T* __restrict__ tok, long vocab,
+                                                         const T* __restrict__ pos, int max_pos, float scale, float* __restrict__ x,
+                                                         float* __restrict__ copy, const float* __restrict__ w, float woff, float eps,
+                                                         T* __restrict__ out, int W) {
+  using Raw = std::conditional_t<sizeof(T) == 2, short4_t, floatx4>;
+  __shared__ float red[4];
+  const long row = blockIdx.x;
+  const int id = ids[row], ps = positions ? positions[row] : 0, nv = W >> 2;
+  const bool ok = !positions || (id >= 0 && id < vocab && ps >= 0 && ps < max_pos);
+  if (!ok && threadIdx.x == 0) atomicAdd(&g_stream_embed_errors, 1);
+  const T* tr = tok + min(max((long)id, 0L), vocab - 1) * W;
+  const T* pr = positions ? pos + (long)min(max(ps, 0), max_pos - 1) * W : nullptr;
+  auto wide = [](Raw r) -> floatx4 {
+    if constexpr (sizeof(T) == 2) return floatx4{bf2f((bf16_t)r[0]), bf2f((bf16_t)r[1]), bf2f((bf16_t)r[2]), bf2f((bf16_t)r[3])};
+    else return r;
+  };
+  floatx4 v[MAXV], g[MAXV];
+  Raw rt[MAXV], rp[MAXV];
+#pragma unroll
+  for (int i = 0; i < MAXV; ++i) {
+    const int c = 4 * min((int)threadIdx.x + 256 * i, nv - 1);
+    rt[i] = *reinterpret_cast<const Raw*>(tr + c);
+    if (positions) rp[i] = *reinterpret_cast<const Raw*>(pr + c);
+    g[i] = *reinterpret_cast<const floatx4*>(w + c);
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < MAXV; ++i) {
+    const int c = threadIdx.x + 256 * i;
+    v[i] = positions ? wide(rt[i]) + wide(rp[i]) : wide(rt[i]) * scale;
+    if (!ok) v[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    if (c < nv) {
+      *reinterpret_cast<floatx4*>(x + row * W + 4 * c) = v[i];
+      if (copy) *reinterpret_cast<floatx4*>(copy + row * W + 4 * c) = v[i];
+      ss += v[i][0] * v[i][0] + v[i][1] * v[i][1] + v[i][2] * v[i][2] + v[i][3] * v[i][3];
+    }
+  }
+  ss = block_sum<4>(ss, red);
+  const float inv = 1.f / sqrtf(ss / (float)W + eps);
+#pragma unroll
+  for (int i = 0; i < MAXV; ++i) {
+    const int c = threadIdx.x + 256 * i;
+    if (c >= nv) continue;
+    const floatx4 r = v[i] * inv * (g[i] + woff);
+    if constexpr (sizeof(T) == 2) {
+      const short4_t q = {(short)f2bf(r[0]), (short)f2bf(r[1]), (short)f2bf(r[2]), (short)f2bf(r[3])};
+      *reinterpret_cast<short4_t*>(out + row * W + 4 * c) = q;
+    } else {
+      *reinterpret_cast<floatx4*>(out + row * W + 4 * c) = r;
+    }
+  }
+}
+
 // The same where a and b are products that come as f32 parts [n, rows, W] (s1 of them a's): each is summed and rounded as the product
 // itself would be.  W % 4 == 0, W <= 1024 MAXV; SP >= n parts are requested together.
 template <int MAXV, int SP>
@@ -250,6 +308,27 @@ int lk_embed_pos(const int* ids, const int* positions, const void* tok, int voca
   else
     embed_pos_kernel<float><<<(unsigned)rows, 256, 0, st>>>(ids, positions, (const float*)tok, vocab, (const float*)pos,
                                                             max_pos, W, x, copy);
+  LK_CHECK_LAUNCH();
+  return 0;
+}
+
+// 0: done, 1: not for these sizes or addresses (two launches then)
+int lk_embed_norm(const int* ids, const int* positions, const void* tok, long vocab, const void* pos, int max_pos, float scale, long rows, int W,
+                  float* x, float* copy, const float* w, float woff, float eps, void* out, int esz, hipStream_t st) {
+  const auto al = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  if (W <= 0 || W % 4 || W > 4096 || vocab <= 0 || (positions && max_pos <= 0) || !al(tok) || !al(pos) || !al(w) || !al(x) || !al(copy) || !al(out)) return 1;
+  if (rows <= 0) return 0;
+#define LK_EN(T, V) embed_norm_kernel<T, V><<<(unsigned)rows, 256, 0, st>>>(ids, positions, (const T*)tok, vocab, (const T*)pos, max_pos, scale, x, copy, w, woff, eps, (T*)out, W)
+#define LK_ENS(T)                 \
+  do {                            \
+    if (W <= 1024) LK_EN(T, 1);   \
+    else if (W <= 2048) LK_EN(T, 2); \
+    else LK_EN(T, 4);             \
+  } while (0)
+  if (esz == 2) LK_ENS(bf16_t);
+  else LK_ENS(float);
+#undef LK_ENS
+#undef LK_EN
   LK_CHECK_LAUNCH();
   return 0;
 }

@@ -362,8 +362,7 @@ class FusasunModel(nn.Module):
         ``taps``: a list that receives a copy of the f32 stream after every layer (debugging and tests)."""
         cfg = self.cfg
         eps = cfg.norm_eps
-        x, _ = ops.embed_stream(ids, self.embed, self.dtype, cfg.embed_scale)
-        h = ops.stream_rmsnorm(x, w=self.layers[0].norm1, eps=eps, out_dtype=self.dtype)
+        x, h, _ = ops.embed_norm(ids, self.embed, self.layers[0].norm1, 0.0, eps, cfg.embed_scale)
         n, routes, hc = len(self.layers), self._routes(ids), None
 
         def normed(y, g, gb, post, i, parts=1):
@@ -387,10 +386,7 @@ class FusasunModel(nn.Module):
                 h, hc = normed(y, g, L.rg2_b, L.norm2b, i + 1, X.top)
             if taps is not None:
                 taps.append(x.clone())
-        idx = meta.logits_idx
-        if idx is None:
-            idx = torch.arange(x.shape[0], dtype=torch.long, device=x.device)
-        return ops.stream_rmsnorm(x, w=self.final_norm, eps=eps, idx=idx, out_dtype=self.dtype)
+        return ops.stream_rmsnorm(x, w=self.final_norm, eps=eps, idx=meta.logits_idx, out_dtype=self.dtype)
 
     def head(self, hidden):
         return ops.linear(hidden, self.lm_head)[:, : self.cfg.vocab_size]

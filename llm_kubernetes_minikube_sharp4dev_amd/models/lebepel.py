@@ -333,12 +333,14 @@ class LebepelModel(nn.Module):
         and tests; costs one extra pass per layer)."""
         cfg = self.cfg
         m, eps = cfg.residual_mult, cfg.norm_eps
-        x, emb = ops.embed_pos(ids, meta.positions, self.embed, self.pos, keep_copy=self.reinject)
+        first = self.layers[self.runs[0][0]].norm1 if self.runs else self.final_norm
+        x, h, emb = ops.embed_norm(ids, self.embed, first, 1.0, eps, positions=meta.positions, pos=self.pos, keep_copy=self.reinject)
         a = b = ab = sums = None
         for run, (li, add_emb) in enumerate(self.runs):
             L = self.layers[li]
-            h = ops.stream_rmsnorm(x, a, b, emb if add_emb else None, m, L.norm1, 1.0, eps, out_dtype=self.dtype,
-                                   a_bias=ab, sums=sums)
+            if run or add_emb:
+                h = ops.stream_rmsnorm(x, a, b, emb if add_emb else None, m, L.norm1, 1.0, eps, out_dtype=self.dtype,
+                                       a_bias=ab, sums=sums)
             if taps is not None and run:  # the stream after the previous run, before this pass's re-injection
                 taps.append(x - emb if add_emb else x.clone())
             u, f = self._projected(L, h)

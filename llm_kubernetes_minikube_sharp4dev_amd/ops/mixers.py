@@ -22,7 +22,7 @@ import torch.nn.functional as F
 
 from ._ext import lib, use_hip
 
-__all__ = ["embed_pos", "stream_rmsnorm", "softcap", "linear_swiglu_any", "unitnorm_kv_write", "sig_prefill_tiles", "sig_decode_splits",
+__all__ = ["embed_pos", "embed_norm", "stream_rmsnorm", "softcap", "linear_swiglu_any", "unitnorm_kv_write", "sig_prefill_tiles", "sig_decode_splits",
            "sigmoid_attention_prefill", "sigmoid_attention_decode", "sigattn_supported", "conv_silu", "ssm_scan",
            "gated_group_rmsnorm", "embed_stream", "stream_layernorm", "stream_sandwich_layernorm", "gelu_tanh_mul", "dual_rmsnorm_mean", "normrope_kv_write",
            "sink_attention_prefill", "sink_attention_decode", "mask_first_key", "pooled_blocks_seen", "MASK_CAUSAL", "MASK_CHUNK",
@@ -295,6 +295,15 @@ def embed_stream(ids, tok, out_dtype=torch.bfloat16, scale: float = 1.0):
     if scale != 1.0:
         x = x * scale
     return x, (x if out_dtype == torch.float32 else x.to(out_dtype))
+
+
+def embed_norm(ids, tok, w, w_offset: float, eps: float, scale: float = 1.0, positions=None, pos=None, keep_copy: bool = False):
+    """(x, h, copy): ``embed_pos`` where ``positions`` and ``pos`` are given, else ``embed_stream``, and ``stream_rmsnorm`` of the new
+    stream in the table's dtype."""
+    if use_hip(tok):
+        return tuple(lib().embed_norm(ids, tok, w, float(w_offset), float(eps), float(scale), positions, pos, keep_copy))
+    x, copy = embed_pos(ids, positions, tok, pos, keep_copy) if positions is not None else (embed_stream(ids, tok, tok.dtype, scale)[0], None)
+    return x, stream_rmsnorm(x, w=w, w_offset=w_offset, eps=eps, out_dtype=tok.dtype), copy
 
 
 def stream_layernorm(x, y, ls, alpha: float, w, b, eps: float, out_dtype=torch.bfloat16, idx=None):

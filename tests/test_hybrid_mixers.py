@@ -69,6 +69,32 @@ def test_embed_stream_norm_softcap(W, device, dtype):
 
 
 @pytest.mark.parametrize("device,dtype", ALL)
+@pytest.mark.parametrize("W", [4, 70, 1024, 1028, 2052, 4096, 4100])   # (70 and 4,100: two launches)
+def test_embed_norm_is_embedding_then_norm(W, device, dtype):
+    g = torch.Generator().manual_seed(4)
+    V, P, T = 50, 40, 9
+    tok, pos = (q16(rnd(g, n, W)).to(dtype).to(device) for n in (V, P))
+    w = rnd(g, W, scale=0.1).float().to(device)
+    ids, ps = (torch.randint(0, n, (T,), generator=g, dtype=torch.int32).to(device) for n in (V, P))
+    for keep in (False, True):
+        x, h, e = ops.embed_norm(ids, tok, w, 1.0, 1e-3, positions=ps, pos=pos, keep_copy=keep)
+        xr, _ = ops.embed_pos(ids, ps, tok, pos)
+        assert torch.equal(x, xr) and torch.equal(h, ops.stream_rmsnorm(xr, w=w, w_offset=1.0, eps=1e-3, out_dtype=dtype))
+        assert (e is None) if not keep else torch.equal(e, xr) and e.data_ptr() != x.data_ptr()
+    x, h, e = ops.embed_norm(ids, tok, w, 0.0, 1e-3, scale=0.3)
+    xr, _ = ops.embed_stream(ids, tok, dtype, 0.3)
+    assert e is None and torch.equal(x, xr) and torch.equal(h, ops.stream_rmsnorm(xr, w=w, eps=1e-3, out_dtype=dtype))
+    if device != "cpu":   # ids and positions outside their tables: zeros, and counted; clamped without positions
+        bad = ids.clone()
+        bad[2], bad[5] = V, -1
+        n = ops.lib().stream_embed_errors()
+        x, h, _ = ops.embed_norm(bad, tok, w, 1.0, 1e-3, positions=ps, pos=pos)
+        assert ops.lib().stream_embed_errors() == n + 2 and not x[[2, 5]].any() and not h[[2, 5]].any()
+        x, _, _ = ops.embed_norm(bad, tok, w, 0.0, 1e-3)
+        assert torch.equal(x[2], tok[V - 1].float()) and torch.equal(x[5], tok[0].float())
+
+
+@pytest.mark.parametrize("device,dtype", ALL)
 def test_swiglu_any_dtype(device, dtype):
     g = torch.Generator().manual_seed(2)
     h, wgu = q16(rnd(g, 5, 64)), q16(rnd(g, 2 * 48, 64, scale=0.2))
