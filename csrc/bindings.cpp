@@ -2090,6 +2090,22 @@ at::Tensor moe_gemm(const at::Tensor& x, const at::Tensor& order, const at::Tens
   return out;
 }
 
+// moe_gemm(act) of tokens x and, beside it, x w2^T: {experts' rows, product}
+std::vector<at::Tensor> moe_gemm_beside(const at::Tensor& x, const at::Tensor& order, const at::Tensor& seg, const at::Tensor& w, int64_t top,
+                                        const at::Tensor& w2) {
+  CHECK_CUDA(x); CHECK_LASTDIM(x); CHECK_CUDA(w); CHECK_CONTIG(w); CHECK_CUDA(order); CHECK_I32(order); CHECK_CONTIG(order);
+  CHECK_CUDA(seg); CHECK_I32(seg); CHECK_CONTIG(seg); CHECK_CUDA(w2); CHECK_CONTIG(w2);
+  TORCH_CHECK(x.scalar_type() == at::kBFloat16, "moe_gemm_beside: bf16");
+  same_type(w, x, "w");
+  same_type(w2, x, "w2");
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 3 && w.size(2) == x.size(1) && seg.numel() == w.size(0) + 1 && top >= 1, "x [rows, K], w [E, N, K]");
+  TORCH_CHECK(w2.dim() == 2 && w2.size(1) == x.size(1) && order.numel() == x.size(0) * top, "w2 [N2, K], order [rows * top]");
+  at::Tensor out = at::empty({order.numel(), w.size(1) / 2}, x.options()), y2 = at::empty({x.size(0), w2.size(0)}, x.options());
+  CHECK_RC(lk_moe_gemm_beside(bp(x), x.stride(0), ip(order), ip(seg), (int)w.size(0), (int)top, x.size(0), bp(w), (int)w.size(1), (int)w.size(2),
+                              out.data_ptr(), out.stride(0), bp(w2), (int)w2.size(0), y2.data_ptr(), y2.stride(0), cur_stream()), "moe_gemm_beside");
+  return {out, y2};
+}
+
 // ---------------------------------------------------------------------------------------------
 // mixed residual streams, skinny f32 projections, matrix memory, attention over a cached latent
 std::vector<c10::optional<at::Tensor>> stream_hyper_norm(at::Tensor& x, int64_t S, const c10::optional<at::Tensor>& a,
@@ -2501,6 +2517,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     return lk_gemm1w_grouped_supported(rows, K, x_rows, (int)N, (int)K, swiglu ? 1 : 0, swiglu ? N / 2 : N) != 0;
   });
   m.def("moe_gemm", &moe_gemm);
+  m.def("moe_gemm_beside", &moe_gemm_beside);
+  m.def("moe_beside_ok", [](int64_t T, int64_t top, int64_t E, int64_t N, int64_t K, int64_t N2) {
+    return lk_moe_beside_ok(T, (int)top, (int)E, (int)N, (int)K, (int)N2) != 0;
+  });
   m.def("stream_hyper_norm", &stream_hyper_norm);
   m.def("relu_sq_", &relu_sq_);
   m.def("gate_proj", &gate_proj);

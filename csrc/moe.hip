@@ -371,19 +371,58 @@ int launch_moe(const void* x, long xs, const int* order, const int* seg, int E, 
   return 0;
 }
 
+// A product of the same rows beside the experts' (moe_rows_kernel): y = x w^T [M, N], in the first nb workgroups of the launch.
+struct Beside {
+  const bf16_t* w = nullptr;
+  bf16_t* y = nullptr;
+  long ldy = 0;
+  int M = 0, N = 0, nb = 0;
+};
+
 // The same product for decode-sized steps of bf16 rows: a stream of the experts' weights, each read once.  One workgroup
 // takes 16 columns (act: 16 gate and their up columns; else 2 x 16) of ONE expert and all of its pairs, MT x 16 at a
 // time (more than that is a second walk over the same weight rows, out of L2); the four waves split K through private
 // LDS rings (row_ring.h), so up to 64 KB of weight rows are on their way per CU and no wave waits for another inside the walk.
 // 64 tokens x 2 of 16 experts of 2048 x 2816: gate / up 110 us (3.4 TB/s) -> 56 us (6.6 TB/s), down 67 us (2.7 TB/s) -> 30 us.
-template <bool ACT, int MT>
+// BESIDE: the stream's gate is a product of the rows that the experts read, and on its own a launch of 5.7 us for 8 MB (64 x 2,048 x 2,048) before
+// theirs, which is bound by the weights' stream; in it the three products take 23.5 -> 20.0 us with one row, 59.5 ->
+// 55.9 with 8, 92.3 -> 89.5 with 32, 93.3 -> 91.6 with 64 (spread over the launch instead of in front: 22.5, 70.8 for 73.8, 87.9, 90.9).  Its workgroups take what the experts' take in,
+// (MT + 2) 16-row tiles of K, as MT + 1 tiles of rows by 16 columns; the row tiles of a column follow one another on one XCD.
+template <bool ACT, int MT, bool BESIDE = false>
 __global__ __launch_bounds__(256) void moe_rows_kernel(const bf16_t* __restrict__ x, long xs, const int* __restrict__ order,
                                                        const int* __restrict__ seg, int top, const bf16_t* __restrict__ w, int N, int K,
-                                                       bf16_t* __restrict__ out, long os, int blocks) {
+                                                       bf16_t* __restrict__ out, long os, int blocks, Beside p) {
   constexpr int NT = 2, NS = 3;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int e = blockIdx.x / blocks, cb = blockIdx.x % blocks;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int at = blockIdx.x;
+  if constexpr (BESIDE) {
+    if (at < p.nb) {
+      constexpr int BT = MT + 1;
+      const int tiles = (p.M + 16 * BT - 1) / (16 * BT), column = (at >> 3) / tiles * 8 + (at & 7), m0 = (at >> 3) % tiles * (16 * BT);
+      if (column * 16 >= p.N) return;
+      const int all = K / 64, first = wave * all / kRgWaves, nst = (wave + 1) * all / kRgWaves - first, lrow = lane >> 3;
+      const long k = (long)first * 64 + rg_lane_col(lane);
+      const bf16_t *xp[2 * BT], *wp[2];
+#pragma unroll
+      for (int i = 0; i < 2 * BT; ++i) xp[i] = x + (long)min(m0 + 8 * i + lrow, p.M - 1) * xs + k;  // rows past M repeat the last one
+#pragma unroll
+      for (int i = 0; i < 2; ++i) wp[i] = p.w + (long)(column * 16 + 8 * i + lrow) * K + k;
+      floatx4 acc[BT][1];
+      rg_walk<BT, 1, NS>(xp, wp, nst, smem + wave * NS * rg_stage(BT, 1), acc);
+      rg_sums<BT, 1>(smem, acc, [&](int m, const floatx4 (&t)[1]) {
+        const int row = m0 + m * 16 + (lane & 15);
+        if (row >= p.M) return;
+        uint2 pk;
+        pk.x = pack_bf2(t[0][0], t[0][1]);
+        pk.y = pack_bf2(t[0][2], t[0][3]);
+        *reinterpret_cast<uint2*>(p.y + (long)row * p.ldy + column * 16 + 4 * (lane >> 4)) = pk;
+      });
+      return;
+    }
+    at -= p.nb;
+  }
+  const int e = at / blocks, cb = at % blocks;
   const int end = seg[e + 1], F = ACT ? N / 2 : N, c0 = cb * (ACT ? 16 : 32);
   const int all = K / 64, first = wave * all / kRgWaves, nst = (wave + 1) * all / kRgWaves - first;
   const int lrow = lane >> 3;
@@ -420,6 +459,19 @@ __global__ __launch_bounds__(256) void moe_rows_kernel(const bf16_t* __restrict_
   }
 }
 
+template <int MT>
+int launch_moe_beside(const void* x, long xs, const int* order, const int* seg, int E, int top, const void* w, int N, int K, void* out,
+                      long os, Beside p, hipStream_t st) {
+  constexpr int lds = rg_lds(MT, 2, 3);
+  static_assert(rg_lds(MT + 1, 1, 3) <= lds, "both tiles in one workgroup's LDS");
+  LK_SET_MAX_LDS((moe_rows_kernel<true, MT, true>), lds);
+  p.nb = (p.N / 16 + 7) / 8 * 8 * ((p.M + 16 * (MT + 1) - 1) / (16 * (MT + 1)));
+  moe_rows_kernel<true, MT, true><<<(unsigned)(p.nb + (long)E * (N / 32)), 256, lds, st>>>((const bf16_t*)x, xs, order, seg, top, (const bf16_t*)w, N, K,
+                                                                                      (bf16_t*)out, os, N / 32, p);
+  LK_CHECK_LAUNCH();
+  return 0;
+}
+
 template <bool ACT, int MT>
 int launch_moe_rows(const void* x, long xs, const int* order, const int* seg, int E, int top, const void* w, int N, int K, void* out,
                     long os, hipStream_t st) {
@@ -427,7 +479,7 @@ int launch_moe_rows(const void* x, long xs, const int* order, const int* seg, in
   constexpr int lds = rg_lds(MT, 2, 3);
   LK_SET_MAX_LDS((moe_rows_kernel<ACT, MT>), lds);
   moe_rows_kernel<ACT, MT><<<(unsigned)((long)E * blocks), 256, lds, st>>>((const bf16_t*)x, xs, order, seg, top, (const bf16_t*)w, N, K,
-                                                                          (bf16_t*)out, os, blocks);
+                                                                          (bf16_t*)out, os, blocks, Beside{});
   LK_CHECK_LAUNCH();
   return 0;
 }
@@ -473,6 +525,22 @@ int lk_moe_route(const int* ids, const int* const* tables, int n, int vocab, int
   else moe_route_kernel<kRouteU><<<n, kRouteThreads, 0, st>>>(ids, rt, vocab, top, E, T, seg, order);
   LK_CHECK_LAUNCH();
   return 0;
+}
+
+// Whether the gate of T rows runs beside the experts' first product: the few-row kernel for both, and so few rows that reading X again for
+// every 16 columns costs less than a launch (2,048 x 2,048 beside 16 experts of 2,048 x 2,816, both and the second product: 88 rows
+// 111.7 -> 109.8 us, 96 rows 112.9 -> 112.0)
+int lk_moe_beside_ok(long T, int top, int E, int N, int K, int N2) {
+  return T >= 1 && T <= 96 && top >= 1 && E >= 1 && T * top <= 22L * E && K % 64 == 0 && N % 32 == 0 && N2 > 0 && N2 % 16 == 0 && (long)E * (N / 32) <= 1 << 30;
+}
+
+int lk_moe_gemm_beside(const void* x, long xs, const int* order, const int* seg, int E, int top, long T, const void* w, int N, int K,
+                       void* out, long os, const void* w2, int N2, void* y2, long ldy, hipStream_t st) {
+  const auto al = [](const void* p, int n) { return reinterpret_cast<uintptr_t>(p) % n == 0; };
+  if (!lk_moe_beside_ok(T, top, E, N, K, N2) || xs % 8 || os % 4 || ldy % 4 || !al(x, 16) || !al(w, 16) || !al(w2, 16) || !al(out, 8) || !al(y2, 8)) return -1;
+  const Beside p{(const bf16_t*)w2, (bf16_t*)y2, ldy, (int)T, N2, 0};
+  return T * top / E <= 10 ? launch_moe_beside<1>(x, xs, order, seg, E, top, w, N, K, out, os, p, st)
+                           : launch_moe_beside<2>(x, xs, order, seg, E, top, w, N, K, out, os, p, st);
 }
 
 int lk_moe_gemm(const void* x, long xs, const int* order, const int* seg, int E, int top, long pairs, const void* w, int N, int K,

@@ -381,8 +381,7 @@ class FusasunModel(nn.Module):
             else:
                 h = ops.stream_gated_norm(x, y, g, L.rg1_b, L.norm1b, L.norm2, eps, self.dtype)
                 X = L.mlp
-                g = ops.linear(h, L.rg2)
-                y = ops.table_experts(h, ids, X.table, X.gate_up, X.down, X.top, routes[i])
+                g, y = ops.linear_table_experts(h, L.rg2, ids, X.table, X.gate_up, X.down, X.top, routes[i])
                 h, hc = normed(y, g, L.rg2_b, L.norm2b, i + 1, X.top)
             if taps is not None:
                 taps.append(x.clone())

@@ -178,6 +178,21 @@ def table_experts(h, ids, table, w_gate_up, w_down, top: int, route=None):
     return run_experts(h, ids, table, w_gate_up, w_down, top, route)
 
 
+def linear_table_experts(h, w, ids, table, w_gate_up, w_down, top: int, route=None):
+    """(``linear(h, w)``, ``table_experts(h, ..)``): the product beside the experts' first one where the step is small."""
+    from . import linear
+
+    T, W = h.shape
+    E, N = w_gate_up.shape[:2]
+    if (use_hip(h) and h.dtype == torch.bfloat16 and w.dtype == h.dtype and w.is_contiguous() and h.stride(1) == 1 and h.stride(0) % 8 == 0
+            and (h.data_ptr() | w.data_ptr() | w_gate_up.data_ptr()) % 16 == 0 and not _grouped(T, T * top, E, W, w_down.shape[2])
+            and lib().moe_beside_ok(T, top, E, N, W, w.shape[0])):
+        seg, order = route if route is not None else moe_route(ids, table, E)
+        mid, y = lib().moe_gemm_beside(h, order, seg, w_gate_up, int(top), w)
+        return y, lib().moe_gemm(mid, order, seg, w_down, int(top), False)
+    return linear(h, w), run_experts(h, ids, table, w_gate_up, w_down, top, route)
+
+
 def _grouped(T: int, pairs: int, E: int, W: int, ffp: int) -> bool:
     """Whether the expert products run as one dense product per expert (``gemm_grouped``): from GROUPED_DENSE_MIN_ROWS pairs per expert on,
     and from GROUPED_FINE_MIN_ROWS where its row tiles take both sizes (2 of 16 experts of 2048 x 2816: 600 tokens 203 -> 144

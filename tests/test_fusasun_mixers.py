@@ -366,6 +366,26 @@ def test_table_routed_experts(W, ff, E, top, T, device, dtype):
 
 
 @pytest.mark.parametrize("device,dtype", ALL)
+@pytest.mark.parametrize("T,W,N,E,top,ffp", [(1, 64, 16, 4, 2, 32), (32, 128, 48, 8, 2, 48), (33, 192, 144, 8, 2, 16), (64, 2048, 2048, 16, 2, 64), (96, 256, 64, 16, 3, 32),
+                                             (88, 64, 80, 8, 2, 16), (97, 64, 64, 16, 2, 32), (20, 64, 24, 8, 1, 32), (5, 40, 16, 4, 1, 16)])
+def test_product_beside_the_experts(T, W, N, E, top, ffp, device, dtype):
+    """A product of the rows that the experts read, in their launch (the last three: apart): one to four row tiles, the last short, column tiles
+    that 8 does not divide.  The experts' rows are the same bits as without."""
+    g = torch.Generator().manual_seed(T)
+    V = 31
+    d = lambda t: t.to(dtype).to(device)
+    h, w = q16(rnd(g, T, W)), q16(rnd(g, N, W, scale=W ** -0.5))
+    gu, dn = q16(rnd(g, E, 2 * ffp, W, scale=W ** -0.5)), q16(rnd(g, E, W, ffp, scale=ffp ** -0.5))
+    table = torch.rand(V, E, generator=g).argsort(1)[:, :top].to(torch.int32).to(device)
+    ids = torch.randint(0, V, (T,), generator=g, dtype=torch.int32).to(device)
+    if device != "cpu" and dtype == torch.bfloat16:
+        assert ops.lib().moe_beside_ok(T, top, E, 2 * ffp, W, N) == (T <= 96 and W % 64 == 0 and N % 16 == 0)
+    y, m = ops.linear_table_experts(d(h), d(w), ids, table, d(gu), d(dn), top)
+    assert y.shape == (T, N) and rel_err(y, h @ w.t()) < (1e-5 if dtype == torch.float32 else 4e-3)   # bf16: one rounding, 2^-9
+    assert torch.equal(m, ops.table_experts(d(h), ids, table, d(gu), d(dn), top))
+
+
+@pytest.mark.parametrize("device,dtype", ALL)
 @pytest.mark.parametrize("taps,W", [(1, 36), (3, 48), (4, 40), (8, 50)])
 def test_convolution_added_to_its_input_over_cuts(taps, W, device, dtype):
     """h + conv(h) as one convolution whose last tap carries the identity, its state kept per slot across
