@@ -1968,7 +1968,8 @@ at::Tensor gemm_grouped(const at::Tensor& x, const at::Tensor& seg, const at::Te
 
 // ids absent: the table has one row per token of the step (a router's choice)
 // seg [n, E + 1] and order [n, T * top] of n tables of the same sizes
-std::vector<at::Tensor> moe_routes(const c10::optional<at::Tensor>& ids, const std::vector<at::Tensor>& tables, int64_t E) {
+std::vector<at::Tensor> moe_routes(const c10::optional<at::Tensor>& ids, const std::vector<at::Tensor>& tables, int64_t E,
+                                   const c10::optional<at::Tensor>& live) {
   if (ids) { CHECK_CUDA(*ids); CHECK_I32(*ids); CHECK_CONTIG(*ids); }
   const int n = tables.size();
   TORCH_CHECK(n >= 1 && n <= kMaxRouteTables && E >= 1, "tables");
@@ -1983,13 +1984,14 @@ std::vector<at::Tensor> moe_routes(const c10::optional<at::Tensor>& ids, const s
   const int top = tables[0].size(1);
   at::Tensor seg = at::empty({n, E + 1}, tables[0].options());
   at::Tensor order = at::empty({n, T * top}, tables[0].options());
-  CHECK_RC(lk_moe_route(ipo(ids), ptr, n, (int)tables[0].size(0), top, (int)E, (int)T, seg.data_ptr<int>(), order.data_ptr<int>(),
+  if (live) { CHECK_CUDA(*live); CHECK_I32(*live); CHECK_CONTIG(*live); TORCH_CHECK(live->numel() == T, "live: one word per row"); }
+  CHECK_RC(lk_moe_route(ipo(ids), ipo(live), ptr, n, (int)tables[0].size(0), top, (int)E, (int)T, seg.data_ptr<int>(), order.data_ptr<int>(),
                         cur_stream()), "moe_route");
   return {seg, order};
 }
 
 std::vector<at::Tensor> moe_route(const c10::optional<at::Tensor>& ids, const at::Tensor& table, int64_t E) {
-  const auto r = moe_routes(ids, {table}, E);
+  const auto r = moe_routes(ids, {table}, E, c10::nullopt);
   return {r[0][0], r[1][0]};
 }
 
@@ -2504,7 +2506,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rot_kv_write", &rot_kv_write);
   m.def("pool_kv_write", &pool_kv_write);
   m.def("moe_route", &moe_route);
-  m.def("moe_routes", &moe_routes);
+  m.def("moe_routes", &moe_routes, py::arg("ids"), py::arg("tables"), py::arg("E"), py::arg("live") = py::none());
+  m.def("moe_rows_ok", [](int64_t T, int64_t top, int64_t E, int64_t W, int64_t ff) { return lk_moe_rows_ok(T, (int)top, (int)E, (int)W, (int)ff) != 0; });
   m.def("stream_parallel_norm", &stream_parallel_norm);
   m.def("router_topk", &router_topk);
   m.def("clamped_glu", &clamped_glu);

@@ -378,7 +378,8 @@ int lk_sigmoid_mul_(void* x, long xs, const void* g, long gs, long rows, int n, 
 
 // csrc/moe.hip: experts chosen by a table of token ids: pairs sorted by expert on the device, grouped MFMA products
 constexpr int kMaxRouteTables = 64;
-int lk_moe_route(const int* ids, const int* const* tables, int n, int vocab, int top, int E, int T, int* seg, int* order, hipStream_t st);
+int lk_moe_rows_ok(long T, int top, int E, int W, int ff);
+int lk_moe_route(const int* ids, const int* live, const int* const* tables, int n, int vocab, int top, int E, int T, int* seg, int* order, hipStream_t st);
 int lk_moe_beside_ok(long T, int top, int E, int N, int K, int N2);
 int lk_moe_gemm_beside(const void* x, long xs, const int* order, const int* seg, int E, int top, long T, const void* w, int N, int K,
                        void* out, long os, const void* w2, int N2, void* y2, long ldy, hipStream_t st);

@@ -49,18 +49,18 @@ struct RouteTables {
 
 // one workgroup per table (the layers of a model whose tables are indexed by the token ids know their routing at the step's start)
 template <int U>
-__global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(const int* __restrict__ ids, RouteTables tables, int vocab,
-                                                                  int top, int E, int T, int* __restrict__ seg,
+__global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(const int* __restrict__ ids, const int* __restrict__ live, RouteTables tables,
+                                                                  int vocab, int top, int E, int T, int* __restrict__ seg,
                                                                   int* __restrict__ order) {
   const int* __restrict__ table = tables.t[blockIdx.x];
   seg += (long)blockIdx.x * (E + 1);
   order += (long)blockIdx.x * T * top;
   __shared__ int cnt[kMaxExperts];
-  __shared__ int nxt[kMaxExperts];
+  __shared__ int nxt[kMaxExperts + 1];   // the last: the pairs of rows that are not live
   const int n = T * top, tid = threadIdx.x;
   for (int e = tid; e < E; e += kRouteThreads) cnt[e] = 0;
   __syncthreads();
-  int ex[U];
+  int ex[U], lv[U];
   auto experts = [&](int p0) {   // of pairs p0 + tid + 1024 u (behind the end: the last pair's)
     int id[U], at[U];
 #pragma unroll
@@ -69,6 +69,7 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(const int* __r
       const int p = (int)min((long)p0 + u * kRouteThreads + tid, (long)n - 1), t = p / top;
       at[u] = p - t * top;
       id[u] = ids ? ids[t] : t;                 // no ids: the table has one row per token of the step
+      lv[u] = live ? live[t] : 0;
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -78,14 +79,14 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(const int* __r
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if ((long)p0 + u * kRouteThreads >= n) break;
-      ex[u] = min(max(ex[u], 0), E - 1);
+      ex[u] = lv[u] < 0 ? E : min(max(ex[u], 0), E - 1);
     }
   };
   for (long p0 = 0; p0 < n; p0 += U * kRouteThreads) {
     experts((int)p0);
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (p0 + u * kRouteThreads + tid < n) atomicAdd(&cnt[ex[u]], 1);
+      if (p0 + u * kRouteThreads + tid < n && ex[u] < E) atomicAdd(&cnt[ex[u]], 1);
   }
   __syncthreads();
   if (tid < 64) {   // running sums of the counts, 64 experts at a time
@@ -96,7 +97,7 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(const int* __r
       if (e0 + tid < E) seg[e0 + tid] = nxt[e0 + tid] = acc + v - c;
       acc += __builtin_amdgcn_readlane(v, 63);
     }
-    if (tid == 0) seg[E] = acc;
+    if (tid == 0) seg[E] = nxt[E] = acc;
   }
   __syncthreads();
   for (long p0 = 0; p0 < n; p0 += U * kRouteThreads) {
@@ -391,7 +392,7 @@ struct Beside {
 template <bool ACT, int MT, bool BESIDE = false>
 __global__ __launch_bounds__(256) void moe_rows_kernel(const bf16_t* __restrict__ x, long xs, const int* __restrict__ order,
                                                        const int* __restrict__ seg, int top, const bf16_t* __restrict__ w, int N, int K,
-                                                       bf16_t* __restrict__ out, long os, int blocks, Beside p) {
+                                                       bf16_t* __restrict__ out, long os, int blocks, long pairs, int E, Beside p) {
   constexpr int NT = 2, NS = 3;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -423,6 +424,11 @@ __global__ __launch_bounds__(256) void moe_rows_kernel(const bf16_t* __restrict_
     at -= p.nb;
   }
   const int e = at / blocks, cb = at % blocks;
+  if constexpr (!ACT) {   // the pairs of rows that are not live, behind the experts' (lk_moe_route): zeros
+    if (e == 0)
+      for (long place = seg[E] + (threadIdx.x >> 3); place < pairs; place += 32)
+        *reinterpret_cast<uint2*>(out + (long)order[place] * os + cb * 32 + 4 * (threadIdx.x & 7)) = make_uint2(0, 0);
+  }
   const int end = seg[e + 1], F = ACT ? N / 2 : N, c0 = cb * (ACT ? 16 : 32);
   const int all = K / 64, first = wave * all / kRgWaves, nst = (wave + 1) * all / kRgWaves - first;
   const int lrow = lane >> 3;
@@ -467,19 +473,19 @@ int launch_moe_beside(const void* x, long xs, const int* order, const int* seg, 
   LK_SET_MAX_LDS((moe_rows_kernel<true, MT, true>), lds);
   p.nb = (p.N / 16 + 7) / 8 * 8 * ((p.M + 16 * (MT + 1) - 1) / (16 * (MT + 1)));
   moe_rows_kernel<true, MT, true><<<(unsigned)(p.nb + (long)E * (N / 32)), 256, lds, st>>>((const bf16_t*)x, xs, order, seg, top, (const bf16_t*)w, N, K,
-                                                                                      (bf16_t*)out, os, N / 32, p);
+                                                                                      (bf16_t*)out, os, N / 32, 0, E, p);
   LK_CHECK_LAUNCH();
   return 0;
 }
 
 template <bool ACT, int MT>
-int launch_moe_rows(const void* x, long xs, const int* order, const int* seg, int E, int top, const void* w, int N, int K, void* out,
+int launch_moe_rows(const void* x, long xs, const int* order, const int* seg, int E, int top, long pairs, const void* w, int N, int K, void* out,
                     long os, hipStream_t st) {
   const int blocks = N / 32;  // 16 output columns of two weight rows each, or 32
   constexpr int lds = rg_lds(MT, 2, 3);
   LK_SET_MAX_LDS((moe_rows_kernel<ACT, MT>), lds);
   moe_rows_kernel<ACT, MT><<<(unsigned)((long)E * blocks), 256, lds, st>>>((const bf16_t*)x, xs, order, seg, top, (const bf16_t*)w, N, K,
-                                                                          (bf16_t*)out, os, blocks, Beside{});
+                                                                          (bf16_t*)out, os, blocks, pairs, E, Beside{});
   LK_CHECK_LAUNCH();
   return 0;
 }
@@ -501,8 +507,8 @@ int moe_gemm_t(const void* x, long xs, const int* order, const int* seg, int E, 
     if (vec && K % 64 == 0 && N % 32 == 0 && os % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0 && (long)E * (N / 32) <= 2147483647L) {
       const long avg = pairs / E;
 #define LK_MOE_ROWS(MT)                                                                           \
-  (act ? launch_moe_rows<true, MT>(x, xs, order, seg, E, top, w, N, K, out, os, st)               \
-       : launch_moe_rows<false, MT>(x, xs, order, seg, E, top, w, N, K, out, os, st))
+  (act ? launch_moe_rows<true, MT>(x, xs, order, seg, E, top, pairs, w, N, K, out, os, st)        \
+       : launch_moe_rows<false, MT>(x, xs, order, seg, E, top, pairs, w, N, K, out, os, st))
       return avg <= 10 ? LK_MOE_ROWS(1) : avg <= 22 ? LK_MOE_ROWS(2) : LK_MOE_ROWS(4);
 #undef LK_MOE_ROWS
     }
@@ -515,14 +521,22 @@ int moe_gemm_t(const void* x, long xs, const int* order, const int* seg, int E, 
 
 }  // namespace
 
-// seg [tables][E + 1], order [tables][T * top]
-int lk_moe_route(const int* ids, const int* const* tables, int n, int vocab, int top, int E, int T, int* seg, int* order, hipStream_t st) {
+// Whether both products of T rows run as moe_rows_kernel (aligned operands), which gives zeros for the rows that are not live
+int lk_moe_rows_ok(long T, int top, int E, int W, int ff) {
+  return T >= 1 && top >= 1 && E >= 1 && T * top < 64L * E && W % 64 == 0 && ff % 64 == 0 && (long)E * (max(2 * ff, W) / 32) <= 2147483647L;
+}
+
+// seg [tables][E + 1], order [tables][T * top].  live (or null): the pairs of a row with live < 0 are no expert's and stand behind all others, from
+// seg[E] on.  A step captured for 48 rows that has 33 ran its 15 empty ones as token 0, all through the same experts: a second walk over their
+// weights (16 experts of 2,048 x 2,816, gate / up 64 us for 57), or experts that nobody else needs.  Four steps of eight such layers, us, with the
+// gate beside the experts: 3 sequences 3,291 -> 2,741, 5 3,747 -> 3,144, 17 4,742 -> 4,384, 33 5,525 -> 4,889, 64 5,410 -> 5,068.
+int lk_moe_route(const int* ids, const int* live, const int* const* tables, int n, int vocab, int top, int E, int T, int* seg, int* order, hipStream_t st) {
   if (T <= 0) return 0;
   if (E < 1 || E > kMaxExperts || top < 1 || vocab < 1 || n < 1 || n > kMaxRouteTables) return -1;
   RouteTables rt = {};
   for (int i = 0; i < n; ++i) rt.t[i] = tables[i];
-  if ((long)T * top <= kRouteThreads) moe_route_kernel<1><<<n, kRouteThreads, 0, st>>>(ids, rt, vocab, top, E, T, seg, order);
-  else moe_route_kernel<kRouteU><<<n, kRouteThreads, 0, st>>>(ids, rt, vocab, top, E, T, seg, order);
+  if ((long)T * top <= kRouteThreads) moe_route_kernel<1><<<n, kRouteThreads, 0, st>>>(ids, live, rt, vocab, top, E, T, seg, order);
+  else moe_route_kernel<kRouteU><<<n, kRouteThreads, 0, st>>>(ids, live, rt, vocab, top, E, T, seg, order);
   LK_CHECK_LAUNCH();
   return 0;
 }

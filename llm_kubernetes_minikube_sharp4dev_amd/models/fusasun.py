@@ -344,16 +344,20 @@ class FusasunModel(nn.Module):
         return latent_window_attention(u, M.rows, M.up_rows.off["uv"], M.w_uq, M.w_ukv, M.dq_norm, M.dkv_norm, cache, meta, M.spec, M.freq,
                                        M.hscale, self.cfg.norm_eps, w_heads=M.w_heads)
 
-    def _routes(self, ids) -> list:
-        """Every layer's expert routing (None: no experts), known from the token ids."""
+    def _routes(self, ids, meta: AttnMeta) -> list:
+        """Every layer's expert routing (None: no experts), known from the token ids.  The padding rows of a decode step, whose slots are
+        negative, run through none."""
         out = [None] * len(self.layers)
         if self.embed.is_cuda:
             groups = {}
             for i, L in enumerate(self.layers):
                 if L.mlp is not None:
-                    groups.setdefault((L.mlp.gate_up.shape[0], tuple(L.mlp.table.shape)), []).append(i)
-            for (experts, _), at in groups.items():
-                for i, r in zip(at, ops.moe_routes(ids, [self.layers[i].mlp.table for i in at], experts)):
+                    groups.setdefault((L.mlp.gate_up.shape[0], tuple(L.mlp.table.shape), L.mlp.down.shape[2]), []).append(i)
+            T = ids.numel()
+            for (experts, (_, top), ffp), at in groups.items():
+                skip = (meta.num_decode == T and meta.slots is not None and self.dtype == torch.bfloat16
+                        and ops.moe_skips_rows(T, top, experts, self.cfg.hidden, ffp))
+                for i, r in zip(at, ops.moe_routes(ids, [self.layers[i].mlp.table for i in at], experts, meta.slots if skip else None)):
                     out[i] = r
         return out
 
@@ -363,7 +367,7 @@ class FusasunModel(nn.Module):
         cfg = self.cfg
         eps = cfg.norm_eps
         x, h, _ = ops.embed_norm(ids, self.embed, self.layers[0].norm1, 0.0, eps, cfg.embed_scale)
-        n, routes, hc = len(self.layers), self._routes(ids), None
+        n, routes, hc = len(self.layers), self._routes(ids, meta), None
 
         def normed(y, g, gb, post, i, parts=1):
             """The stream takes y, gated, in; -> (the norm that opens layer i, the convolution behind it)."""

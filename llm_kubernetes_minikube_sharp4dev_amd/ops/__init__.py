@@ -20,7 +20,7 @@ from .mixers import (conv_silu, embed_norm, embed_pos, gated_group_rmsnorm, line
                      softcap, ssm_scan, stream_rmsnorm, unitnorm_kv_write, embed_stream, stream_layernorm, gelu_tanh_mul,
                      dual_rmsnorm_mean, normrope_kv_write, sink_attention_prefill, sink_attention_decode, mask_first_key,
                      pooled_blocks_seen, stream_sandwich_layernorm, MASK_CAUSAL, MASK_CHUNK, MASK_WINDOW, SIG_TILE_ROWS)
-from .window import moe_route, moe_routes, pool_kv_write, rms_cols, rot_kv_write, linear_table_experts, run_experts, stream_gated_norm, stream_gated_norm_conv, table_experts  # noqa: F401
+from .window import moe_route, moe_routes, moe_skips_rows, pool_kv_write, rms_cols, rot_kv_write, linear_table_experts, run_experts, stream_gated_norm, stream_gated_norm_conv, table_experts  # noqa: F401
 from .routed import clamped_glu, routed_experts, router_topk, sigmoid_mul_, silu_, stream_parallel_norm  # noqa: F401
 from .hyper import (GROUP_MAX, GROUP_TOP2, MAX_STREAMS, SCORE_SIGMOID, SCORE_SOFTMAX, gate_proj, relu_sq_, router_choice,  # noqa: F401
                     stream_hyper_norm)

@@ -26,7 +26,7 @@ from .mixers import conv_silu
 GROUPED_DENSE_MIN_ROWS = 128
 GROUPED_FINE_MIN_ROWS = 64
 
-__all__ = ["stream_gated_norm", "stream_gated_norm_conv", "rms_cols", "rot_kv_write", "pool_kv_write", "table_experts", "run_experts", "moe_route", "moe_routes"]
+__all__ = ["stream_gated_norm", "stream_gated_norm_conv", "rms_cols", "rot_kv_write", "pool_kv_write", "table_experts", "run_experts", "moe_route", "moe_routes", "moe_skips_rows", "linear_table_experts"]
 
 
 def stream_gated_norm(x, y, g, g_bias, w_post, w_next, eps: float, out_dtype=torch.bfloat16, parts: int = 1):
@@ -157,16 +157,22 @@ def moe_route(ids, table, experts: int):
     return seg, order
 
 
-def moe_routes(ids, tables, experts: int) -> list:
+def moe_routes(ids, tables, experts: int, live=None) -> list:
     """:func:`moe_route` of several layers' tables of the same sizes, [(seg, order)] in their order: on the GPU one launch per
-    64 of them (8 layers, 64 tokens x 2 of 16 experts: 8 launches of 4.5 us behind each other before)."""
+    64 of them (8 layers, 64 tokens x 2 of 16 experts: 8 launches of 4.5 us behind each other before).  ``live`` (int32 [T], GPU only): rows with
+    a negative word belong to no expert (their pairs stand behind the others); see :func:`moe_skips_rows`."""
     if tables and use_hip(tables[0]):
         out = []
         for a in range(0, len(tables), 64):
-            seg, order = lib().moe_routes(ids, list(tables[a:a + 64]), int(experts))
+            seg, order = lib().moe_routes(ids, list(tables[a:a + 64]), int(experts), live)
             out += list(zip(seg.unbind(0), order.unbind(0)))
         return out
     return [moe_route(ids, t, experts) for t in tables]
+
+
+def moe_skips_rows(T: int, top: int, E: int, W: int, ffp: int) -> bool:
+    """Whether the experts' products of T bf16 rows may leave rows out (``moe_routes(live=)``): their results are zeros."""
+    return lib().moe_rows_ok(T, top, E, W, ffp) and not _grouped(T, T * top, E, W, ffp)
 
 
 def table_experts(h, ids, table, w_gate_up, w_down, top: int, route=None):

@@ -116,3 +116,31 @@ def test_pooled_means(hip, dim, vdim, P, BS):
         out.append((pk.cpu().float(), pv.cpu().float()))
     for a, b in zip(*out):   # f32 means in another order may round to the other neighbour: one bf16 step
         assert ((a - b).abs() <= 2.0 ** -7 * a.abs() + 1e-6).all() and ((a != 0) == (b != 0)).all()
+
+
+@pytest.mark.parametrize("T,top,E,dead", [(1, 2, 4, 1), (48, 2, 16, 15), (48, 2, 16, 0), (64, 2, 16, 64), (17, 3, 8, 9), (600, 2, 128, 31)])
+def test_rows_that_are_not_live_run_through_no_expert(T, top, E, dead):
+    """The pairs of rows without a live word are no expert's and stand behind the others; their results are zeros, the others' the same bits."""
+    W, ff, V = 128, 64, 40
+    g = torch.Generator().manual_seed(T + dead)
+    bf = lambda *s: (torch.randn(*s, generator=g) * 0.1).to(torch.bfloat16).cuda()
+    h, gu, dn = bf(T, W), bf(E, 2 * ff, W), bf(E, W, ff)
+    table = torch.rand(V, E, generator=g).argsort(1)[:, :top].to(torch.int32).contiguous().cuda()
+    ids = torch.randint(0, V, (T,), generator=g, dtype=torch.int32).cuda()
+    live = torch.arange(T, dtype=torch.int32)
+    live[torch.randperm(T, generator=g)[:dead]] = -1
+    live = live.cuda()
+    assert ops.moe_skips_rows(T, top, E, W, ff)
+    (seg, order), = ops.moe_routes(ids, [table], E, live)
+    seg, order_h = seg.tolist(), order.tolist()
+    assert seg[-1] == (T - dead) * top and sorted(order_h) == list(range(T * top))
+    assert all(live[p // top] >= 0 for p in order_h[:seg[-1]]) and all(live[p // top] < 0 for p in order_h[seg[-1]:])
+    route = ops.moe_routes(ids, [table], E, live)[0]
+    got = ops.table_experts(h, ids, table, gu, dn, top, route).view(T, top, W)
+    want = ops.table_experts(h, ids, table, gu, dn, top).view(T, top, W).clone()
+    want[(live < 0)] = 0
+    assert torch.equal(got, want)
+    y, got = ops.linear_table_experts(h, gu[0].contiguous(), ids, table, gu, dn, top, route)
+    assert torch.equal(got.view(T, top, W), want)
+    exact = h.double() @ gu[0].double().t()
+    assert ((y.double() - exact).norm() / exact.norm()).item() < 4e-3   # (one rounding to bf16: 2^-9)
