@@ -18,8 +18,17 @@ _mod = None
 _err: Exception | None = None
 
 
+# Every op asks for the switch, one to three times, and os.environ's look-up of a name that is not there takes 0.9 us: it encodes the name and
+# raises inside.  Whether the name is there at all is asked of the mapping below it, at every call, in 0.2 us.  A pass over 5 texts of 60 - 120
+# tokens 695 - 730 -> 671 - 687 us, over 2 of 9 - 12 565 - 585 -> 548 - 556; a prompt of 60 tokens through the state-space hybrid 525 -> 512.
+_ENV, _ENV_NAMES, _FORCE = os.environ, getattr(os.environ, "_data", None), "LK_FORCE_REFERENCE"
+_FORCE_KEY = os.fsencode(_FORCE) if os.name == "posix" else None
+
+
 def force_reference() -> bool:
-    return os.environ.get("LK_FORCE_REFERENCE", "0") not in ("", "0", "false", "False")
+    if os.environ is _ENV and _ENV_NAMES is not None and _FORCE_KEY is not None and _FORCE_KEY not in _ENV_NAMES:
+        return False
+    return os.environ.get(_FORCE, "0") not in ("", "0", "false", "False")
 
 
 def try_lib():

@@ -551,6 +551,23 @@ def test_encoder_attention_order_by_its_texts(texts, rows, heads, D, order):
     assert _ext.lib().prefill_order(tiles, texts, rows * texts, heads, D) == order
 
 
+def test_reference_switch_follows_the_environment(monkeypatch):
+    """Set, changed and taken away while the process runs, and in a mapping put in the environment's place."""
+    import os
+
+    from llm_kubernetes_minikube_sharp4dev_amd.ops import _ext
+
+    monkeypatch.delenv("LK_FORCE_REFERENCE", raising=False)
+    assert not _ext.force_reference()
+    for value, on in (("1", True), ("0", False), ("", False), ("false", False), ("yes", True)):
+        monkeypatch.setenv("LK_FORCE_REFERENCE", value)
+        assert _ext.force_reference() == on
+    monkeypatch.delenv("LK_FORCE_REFERENCE")
+    assert not _ext.force_reference()
+    monkeypatch.setattr(os, "environ", {"LK_FORCE_REFERENCE": "1"})
+    assert _ext.force_reference()
+
+
 @pytest.mark.parametrize("lens,Hq,Hkv,two", [([159], 32, 8, 0), ([160], 32, 8, 1), ([100] * 8, 32, 8, 0), ([1024], 32, 8, 1), ([2048], 32, 8, 1), ([2049], 32, 8, 0),
                                              ([400] * 3, 32, 8, 0), ([600] * 2, 32, 8, 1), ([500] * 4, 32, 8, 0), ([1500], 32, 32, 1)])
 def test_prompt_attention_splits_keys_where_few_chains_are_long(lens, Hq, Hkv, two):
