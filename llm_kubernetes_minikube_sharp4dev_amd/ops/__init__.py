@@ -1222,9 +1222,9 @@ _GEMV_OK: dict = {}
 
 # The long-K projections (K split into an even number >= 2 of streaming blocks: down at K 14,336,
 # the 70B QKV / gate_up at K 8,192) take two waves per pair of W rows, a K half each, their sums
-# joined in LDS (LK_GEMV_KSPLIT=0: one wave per pair).  Tried and removed: the first W block
-# prefetched before the X prologue, in registers (batch-1 decode step 3.199 vs 3.17 ms) and by
-# LDS-DMA (3.31 vs 3.10; profiles/r6_gemv/).  Workgroup target (LK_GEMV_WGS, 0: 512)
+# joined in LDS (LK_GEMV_KSPLIT=0: one wave per pair).  The first W block is requested behind X's
+# LDS-DMA and ahead of the prologue's waits; requested before X it held X up (loads return in order:
+# 3.199 vs 3.17 ms; by LDS-DMA 3.31 vs 3.10, profiles/r6_gemv/).  Workgroup target (LK_GEMV_WGS, 0: 512)
 GEMV_KSPLIT = os.environ.get("LK_GEMV_KSPLIT", "1") != "0"
 GEMV_WGS = int(os.environ.get("LK_GEMV_WGS", "0") or 0)
 
