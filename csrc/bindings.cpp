@@ -160,7 +160,7 @@ at::Tensor skinny_linear(const at::Tensor& x, const at::Tensor& w, bool swiglu, 
 
 // the weight-streaming kernels reach X's rows by 32-bit offsets: rows further apart than those hold are copied together first
 static at::Tensor ws_near(const at::Tensor& x) {
-  const bool far = x.dim() == 2 && x.stride(1) == 1 && x.stride(0) % 8 == 0 && x.size(0) * x.stride(0) * 2 >= 0xFFFFFF00L;
+  const bool far = x.dim() == 2 && x.stride(1) == 1 && x.stride(0) % 8 == 0 && ((x.size(0) - 1) * x.stride(0) + x.size(1)) * 2 > 0xFC000000L;
   return far ? x.contiguous() : x;
 }
 

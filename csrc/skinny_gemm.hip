@@ -534,6 +534,9 @@ LK_DEVICE u32x4_t ws_srd(const void* p, long bytes) {  // buffer descriptor word
   return u32x4_t{ws_rfl((unsigned)a), ws_rfl((unsigned)(a >> 32)), ws_rfl((unsigned)max(0L, min(bytes, 0xFFFFFFF0L))), 0x00020000u};
 }
 
+// A byte offset behind every operand's range, also with an offset along K (less than 32 MB) on top of it.  Host: ws_too_far.
+constexpr unsigned kWsPast = 0xFC000000u;
+
 // ring depth: as many stages as 160 KB of LDS hold
 // (PRO: a WsPro prologue computes X first -- the LDS ring leaves room for its static scratch)
 constexpr int ws_stages_pro(int MT, int BN, int PRO) {
@@ -574,7 +577,8 @@ struct WsWalk {
                        long kbase, int stages, int rot) {
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15, g = lane >> 4, lrow = lane >> 3, q = LOADERS ? w - 4 : w;
-    xs = ws_srd(X + kbase, (long)M * ldx * 2 - kbase * 2);            // rows past M: zeros
+    // from the first row's start to the last one's end, whatever lies between two rows' starts (0: one row M times; less than K: windows)
+    xs = ws_srd(X + kbase, ((long)(M - 1) * ldx + K - kbase) * 2);
     ws[0] = ws_srd(W + kbase, wrows * K * 2 - kbase * 2);
     ws[1] = SWIGLU ? ws_srd(W2 + kbase, wrows * K * 2 - kbase * 2) : ws[0];
     nst = stages;
@@ -584,7 +588,10 @@ struct WsWalk {
     // piece p: rows 8 p .., lane l the chunk (l & 7) ^ ((row >> 1) & 7) of row l >> 3; a wave's pieces are an even number apart
     const int ch = (lane & 7) ^ (lrow >> 1);
 #pragma unroll
-    for (int i = 0; i < MW; ++i) xo[i] = (unsigned)(8 * (4 * i + w) + lrow) * (unsigned)(ldx * 2) + (unsigned)((ch ^ (4 * (w & 1))) * 16);
+    for (int i = 0; i < MW; ++i) {
+      const int row = 8 * (4 * i + w) + lrow;   // rows past M: zeros
+      xo[i] = row < M ? (unsigned)row * (unsigned)(ldx * 2) + (unsigned)((ch ^ (4 * (w & 1))) * 16) : kWsPast;
+    }
 #pragma unroll
     for (int i = 0; i < PW; ++i)
       wo[i] = (unsigned)(8 * (WSTEP * (SWIGLU ? i % (PW / 2) : i) + q) + lrow) * (unsigned)(K * 2) + (unsigned)((ch ^ (4 * (q & 1))) * 16);
@@ -963,7 +970,7 @@ void launch_ws_lw(const bf16_t* x, long ldx, const bf16_t* w, int M, int K, int 
 }
 
 // a tile's rows are reached by 32-bit offsets from its first: up to 256 of X, up to 128 of W
-bool ws_too_far(int M, long ldx, int K) { return M * ldx * 2 >= 0xFFFFFF00L || (long)K * 256 >= 0xFFFFFF00L; }
+bool ws_too_far(int M, long ldx, int K) { return ((M - 1) * ldx + K) * 2 > (long)kWsPast || (long)K * 256 > (long)kWsPast; }
 
 template <bool SWIGLU>
 int dispatch_ws(int MT, int BN, const bf16_t* x, long ldx, const bf16_t* w, int M, int K, int ks, int S,

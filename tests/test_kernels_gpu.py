@@ -1219,6 +1219,45 @@ def test_ws_walk_edges(hip, M, N, K, swiglu, bn, S, variant):
         hip.ws_set_variant(M, N, K, swiglu, -1)
 
 
+@pytest.mark.parametrize("M,N,K,swiglu,bn,S", [(2, 256, 64, False, 64, 1), (33, 384, 128, False, 96, 2), (64, 256, 320, True, 128, 1), (100, 512, 704, True, 64, 1),
+                                              (129, 192, 512, False, 96, 4), (256, 256, 384, False, 64, 3)])
+@pytest.mark.parametrize("step", [0, 8, 64])
+@pytest.mark.parametrize("variant", [0, 1])
+def test_ws_rows_closer_together_than_k(hip, M, N, K, swiglu, bn, S, step, variant):
+    """One row M times (step 0) and overlapping windows: the same bits as their copy, whatever the loads' order."""
+    torch.manual_seed(M + N + step)
+    x = torch.randn((M - 1) * step + K, device=DEV, dtype=torch.bfloat16).as_strided((M, K), (step, 1))
+    w = torch.randn(N, K, device=DEV, dtype=torch.bfloat16) / K ** 0.5
+    try:
+        hip.ws_set_variant(M, N, K, swiglu, variant)
+        assert torch.equal(hip.ws_linear(x, w, swiglu, bn, S), hip.ws_linear(x.contiguous(), w, swiglu, bn, S))
+    finally:
+        hip.ws_set_variant(M, N, K, swiglu, -1)
+    if not swiglu and bn == 64 and M <= 128:
+        wgu = torch.randn(128, K, device=DEV, dtype=torch.bfloat16) / K ** 0.5
+        for a, b in zip(hip.ws_beside(x, w, wgu, bn), hip.ws_beside(x.contiguous(), w, wgu, bn)):
+            assert torch.equal(a, b)
+    if S == 4:   # (the norm sums 2, 4 or 8 parts)
+        res, nw = torch.randn(M, N, device=DEV, dtype=torch.bfloat16), torch.randn(N, device=DEV, dtype=torch.bfloat16)
+        r1, r2 = res.clone(), res.clone()
+        assert torch.equal(hip.ws_linear_rmsnorm(x, w, r1, nw, 1e-5, bn, S), hip.ws_linear_rmsnorm(x.contiguous(), w, r2, nw, 1e-5, bn, S))
+        assert torch.equal(r1, r2)
+
+
+@pytest.mark.parametrize("variant", [0, 1])
+def test_ws_rows_as_far_apart_as_offsets_hold(hip, variant):
+    """65 rows whose 32-bit offsets just fit: the tile's other 63 rows have offsets past 2^32 and come as zeros."""
+    M, N, K, step = 65, 128, 256, 33_000_000
+    x = torch.randn(M, K, device=DEV, dtype=torch.bfloat16)
+    w = torch.randn(N, K, device=DEV, dtype=torch.bfloat16) / K ** 0.5
+    far = torch.empty((M - 1) * step + K, device=DEV, dtype=torch.bfloat16).as_strided((M, K), (step, 1)).copy_(x)
+    try:
+        hip.ws_set_variant(M, N, K, False, variant)
+        assert torch.equal(hip.ws_linear(far, w, False, 128, 1), hip.ws_linear(x, w, False, 128, 1))
+    finally:
+        hip.ws_set_variant(M, N, K, False, -1)
+
+
 @pytest.mark.parametrize("N,nq,K", [(1, 1, 1), (5, 3, 8), (16, 16, 8), (17, 2, 5), (4097, 16, 8), (40000, 1, 3)])
 def test_knn_scan_orders_signs_and_ties(hip, N, nq, K):
     """The one-pass search's hits as ordered numbers: negative scores, zero rows (a zero of either sign is one score), equal rows in order
