@@ -54,6 +54,13 @@ void check_rows16(const at::Tensor& t, const char* name) {
   if (t.dim() >= 2) TORCH_CHECK((t.stride(0) * t.element_size()) % 16 == 0, name, " row stride must be a multiple of 16 bytes");
 }
 
+// The prefill products reach X through a buffer of rows times their distance: rows closer together than their length (one row
+// expanded, overlapping windows) are copied apart first.
+at::Tensor rows_apart(const at::Tensor& x) {
+  const bool close = x.dim() == 2 && x.size(0) > 0 && x.stride(1) == 1 && x.stride(0) % 8 == 0 && x.stride(0) < x.size(1);
+  return close ? x.clone(at::MemoryFormat::Contiguous) : x;
+}
+
 at::Tensor rmsnorm(const at::Tensor& x, const at::Tensor& w, double eps,
                    const c10::optional<at::Tensor>& residual, const c10::optional<at::Tensor>& out_) {
   CHECK_CUDA(x); CHECK_BF16(x); CHECK_BF16(w); CHECK_LASTDIM(x);
@@ -587,8 +594,9 @@ at::Tensor gemv_decode(int64_t mode, const at::Tensor& x, const at::Tensor& w, c
 
 // Prefill / encoder-regime linear (csrc/gemm.hip): epi(x [M, K] . w[N, K]^T (+ bias)).
 // epi 0 none, 1 SwiGLU (w = [Wg; Wu], out [M, N/2]), 2 bias, 3 bias+GELU(erf), 4 bias+ReLU.
-at::Tensor gemm(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, int64_t epi,
+at::Tensor gemm(const at::Tensor& x_, const at::Tensor& w, const c10::optional<at::Tensor>& bias, int64_t epi,
                 int64_t bn, const c10::optional<at::Tensor>& out_, int64_t variant, int64_t splits) {
+  const at::Tensor x = rows_apart(x_);
   CHECK_CUDA(x); CHECK_BF16(x); CHECK_BF16(w); CHECK_LASTDIM(x); CHECK_CONTIG(w);
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1), "x [M,K], w [N,K]");
   check_rows16(x, "x"); check_rows16(w, "w");
@@ -618,12 +626,13 @@ at::Tensor gemm(const at::Tensor& x, const at::Tensor& w, const c10::optional<at
 // The fused prefill chain (csrc/gemm.hip LkEpi): epi 0 / 1 / 7 with an optional folded-RMSNorm
 // row scale from ss_in [nt, ld] f32, epi 6 (RESID) updating `resid` in place and writing the
 // per-256-column partial sums of squares into ss_out [N / 256, ld].  Returns `out` (RESID: resid).
-at::Tensor gemm_fused(const at::Tensor& x, const at::Tensor& w, int64_t epi, int64_t bn, const c10::optional<at::Tensor>& out_,
+at::Tensor gemm_fused(const at::Tensor& x_, const at::Tensor& w, int64_t epi, int64_t bn, const c10::optional<at::Tensor>& out_,
                       int64_t variant, int64_t splits, const c10::optional<at::Tensor>& ss_in, double eps,
                       const c10::optional<at::Tensor>& resid, const c10::optional<at::Tensor>& ss_out,
                       const c10::optional<at::Tensor>& positions, const c10::optional<at::Tensor>& cos_sin,
                       const c10::optional<at::Tensor>& slots, const c10::optional<at::Tensor>& k_cache,
                       const c10::optional<at::Tensor>& v_cache, int64_t hq, int64_t hkv, int64_t hd) {
+  const at::Tensor x = rows_apart(x_);
   CHECK_CUDA(x); CHECK_BF16(x); CHECK_BF16(w); CHECK_LASTDIM(x); CHECK_CONTIG(w);
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1), "x [M,K], w [N,K]");
   check_rows16(x, "x"); check_rows16(w, "w");
@@ -1950,8 +1959,9 @@ void pool_kv_write(const at::Tensor& kc, const at::Tensor& vc, at::Tensor& pkc, 
 
 // x [rows, K] sorted by expert -- or, with `gather` int32 [rows], any x whose row gather[r] is sorted row r's input; the
 // result's rows are sorted, or with `scatter` int32 [rows] sorted row r lands in out row scatter[r] (a permutation)
-at::Tensor gemm_grouped(const at::Tensor& x, const at::Tensor& seg, const at::Tensor& w, bool swiglu,
+at::Tensor gemm_grouped(const at::Tensor& x_, const at::Tensor& seg, const at::Tensor& w, bool swiglu,
                         const c10::optional<at::Tensor>& gather, const c10::optional<at::Tensor>& scatter, int64_t top) {
+  const at::Tensor x = rows_apart(x_);
   CHECK_CUDA(x); CHECK_BF16(x); CHECK_LASTDIM(x); CHECK_CUDA(w); CHECK_BF16(w); CHECK_CONTIG(w); CHECK_CUDA(seg); CHECK_I32(seg);
   CHECK_CONTIG(seg);
   TORCH_CHECK(x.dim() == 2 && w.dim() == 3 && w.size(2) == x.size(1) && seg.numel() == w.size(0) + 1, "x [rows, K], w [E, N, K], seg [E + 1]");

@@ -572,6 +572,29 @@ def test_gemm1w_persistent_walk(hip, M, N, K, epi):
     _close(hip.gemm(x, w, b, epi, 256, None, 3, 1), y, 0.03, 0.01, f"persistent epi{epi} M{M} N{N} K{K}")
 
 
+@pytest.mark.parametrize("step", [0, 8, 256])
+@pytest.mark.parametrize("M,variant,splits", [(1, 0, 1), (300, 0, 1), (300, 1, 2), (513, 2, 1), (300, 3, 1), (300, 4, 2), (130, 5, 1)])
+def test_gemm_rows_closer_together_than_k(hip, M, variant, splits, step):
+    """One row M times (step 0) and overlapping windows: the same bits as their copy, in every form of the prefill product."""
+    K, N = 768, 512
+    torch.manual_seed(M + step)
+    x = torch.randn((M - 1) * step + K, device=DEV, dtype=torch.bfloat16).as_strided((M, K), (step, 1))
+    y, w = torch.empty(M, K, device=DEV, dtype=torch.bfloat16).copy_(x), torch.randn(N, K, device=DEV, dtype=torch.bfloat16) / K ** 0.5
+    b = torch.randn(N, device=DEV, dtype=torch.bfloat16)
+    for epi in (0, 1, 3) if splits == 1 else (0, 3):
+        assert torch.equal(*(hip.gemm(a, w, b if epi == 3 else None, epi, 256, None, variant, splits) for a in (x, y)))
+    r = [torch.ones(M, N, device=DEV, dtype=torch.bfloat16) for _ in range(2)]
+    ss = [torch.empty(N // 256, M, device=DEV) for _ in range(2)]
+    for a, ri, si in zip((x, y), r, ss):
+        hip.gemm_fused(a, w, 6, 256, None, variant, splits, resid=ri, ss_out=si)
+    assert torch.equal(*r) and torch.equal(*ss)
+    seg, we = torch.tensor([0, M // 3, M], dtype=torch.int32, device=DEV), torch.stack([w, -w])
+    gather = torch.arange(M - 1, -1, -1, dtype=torch.int32, device=DEV)
+    for g in (None, gather):
+        assert torch.equal(*(hip.gemm_grouped(a, seg, we, True, g, None) for a in (x, y)))
+    assert torch.equal(ops.linear(x, w), ops.linear(y, w))
+
+
 @pytest.mark.parametrize("MNK", [(2048, 4096, 4096), (300, 1280, 8192), (1000, 768, 3072), (4096, 1280, 8192)])
 @pytest.mark.parametrize("splits", [2, 3, 4])
 @pytest.mark.parametrize("epi", [0, 2, 3, 4])
