@@ -614,12 +614,12 @@ struct WsWalk {
   template <int I>
   LK_DEVICE void dma_x(unsigned slot) {
     asm volatile("s_add_u32 m0, %3, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
-                 ::"v"(xo[I]), "s"(xs), "s"(kofs), "s"(ldsx + slot), "i"(I * 4096) : "memory", "scc");
+                 ::"v"(xo[I]), "s"(xs), "s"(kofs), "s"(ldsx + slot), "i"(I * 4096) : "memory", "m0", "scc");
   }
   template <int I>
   LK_DEVICE void dma_w(unsigned slot) {
     asm volatile("s_add_u32 m0, %3, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen nt lds"
-                 ::"v"(wo[I]), "s"(ws[up(I)]), "s"(kofs), "s"(ldsw + slot), "i"(I * WSTEP * 1024) : "memory", "scc");
+                 ::"v"(wo[I]), "s"(ws[up(I)]), "s"(kofs), "s"(ldsw + slot), "i"(I * WSTEP * 1024) : "memory", "m0", "scc");
   }
   LK_DEVICE void advance() {   // to the stage after `at`: past the last no descriptor has a range
     kofs = kofs + 128 == last ? 0 : kofs + 128;

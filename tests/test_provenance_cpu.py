@@ -77,3 +77,16 @@ def test_native_runtime_stamp_matches():
     if not runtime.so_path().exists():
         pytest.skip("runtime not built")
     assert provenance.read_stamp(runtime.so_path()) == runtime.tree_hash()
+
+
+def test_asm_that_writes_m0_says_so():
+    """The compiler keeps values of its own in M0 (LDS-DMA builtins): a statement that writes the register names it."""
+    import re
+
+    found = 0
+    for f in _build_mod().sources():
+        for body in re.findall(r'\basm(?:\s+volatile)?\s*\((.*?)\);', f.read_text(), re.S):
+            if re.search(r"\bs_\w+ m0,", body):
+                found += 1
+                assert '"m0"' in body, f"{f.name}: {body}"
+    assert found
