@@ -345,8 +345,8 @@ class FusasunModel(nn.Module):
                                        M.hscale, self.cfg.norm_eps, w_heads=M.w_heads)
 
     def _routes(self, ids, meta: AttnMeta) -> list:
-        """Every layer's expert routing (None: no experts), known from the token ids.  The padding rows of a decode step, whose slots are
-        negative, run through none."""
+        """Every layer's expert routing (None: no experts), known from the token ids.  The padding rows of a decode step, whose state slots
+        are negative (a row that only files no key has a negative ``slots`` word), run through none."""
         out = [None] * len(self.layers)
         if self.embed.is_cuda:
             groups = {}
@@ -355,9 +355,10 @@ class FusasunModel(nn.Module):
                     groups.setdefault((L.mlp.gate_up.shape[0], tuple(L.mlp.table.shape), L.mlp.down.shape[2]), []).append(i)
             T = ids.numel()
             for (experts, (_, top), ffp), at in groups.items():
-                skip = (meta.num_decode == T and meta.slots is not None and self.dtype == torch.bfloat16
+                # (one sequence, and so one state slot, per row)
+                skip = (meta.num_decode == T and meta.state_slots is not None and meta.state_slots.numel() == T and self.dtype == torch.bfloat16
                         and ops.moe_skips_rows(T, top, experts, self.cfg.hidden, ffp))
-                for i, r in zip(at, ops.moe_routes(ids, [self.layers[i].mlp.table for i in at], experts, meta.slots if skip else None)):
+                for i, r in zip(at, ops.moe_routes(ids, [self.layers[i].mlp.table for i in at], experts, meta.state_slots if skip else None)):
                     out[i] = r
         return out
 

@@ -385,6 +385,29 @@ def test_product_beside_the_experts(T, W, N, E, top, ffp, device, dtype):
     assert torch.equal(m, ops.table_experts(d(h), ids, table, d(gu), d(dn), top))
 
 
+@pytest.mark.gpu
+def test_a_row_that_files_no_key_still_runs_its_experts(monkeypatch):
+    """A negative ``slots`` word keeps a row's key out of the cache and nothing else; a padding row has no state slot."""
+    att = {"heads": 4, "kv_heads": 2, "dim": 64, "vdim": 64, "scale": 0.125, "mask": {"size": 48, "pool": 16}, "rot": {"base": 10000.0, "dims": 64}}
+    cfg = FusasunConfig.from_json({"architecture": "Fusasun", "vocab": 61, "width": 256, "norm": {"eps": 1e-5}, "embedding": {"scale": 1.0}, "canon": {"taps": 4},
+                                   "layers": [{"type": "attention", "mixer": att, "mlp": {"kind": "moe", "expert": {"ff": 128}, "router": {"experts": 8, "top": 2}}}] * 2})
+    m = build_decoder(cfg, device="cuda", dtype=torch.bfloat16, seed=2)
+    ids = torch.tensor([7, 30, 0, 12], dtype=torch.int32, device="cuda")
+
+    def step():
+        meta = step_meta([(0, 1, [i], slot, True) for i, slot in enumerate([2, 0, -1, 1])], "cuda")
+        meta.slots[1] = meta.slots[2] = -1
+        with torch.inference_mode():
+            return m(ids, meta, m.make_caches(8, BS, 3)).float()
+
+    assert ops.moe_skips_rows(4, 2, 8, 256, m.layers[0].mlp.down.shape[2])
+    got = step()
+    monkeypatch.setattr(ops, "moe_skips_rows", lambda *a: False)
+    want = step()
+    live = [0, 1, 3]
+    assert torch.equal(got[live], want[live]) and not torch.equal(got[2], want[2])
+
+
 @pytest.mark.parametrize("device,dtype", ALL)
 @pytest.mark.parametrize("taps,W", [(1, 36), (3, 48), (4, 40), (8, 50)])
 def test_convolution_added_to_its_input_over_cuts(taps, W, device, dtype):
