@@ -19,7 +19,7 @@ from __future__ import annotations
 import torch
 import torch.nn.functional as F
 
-from ._ext import lib, use_hip
+from ._ext import force_reference, lib, use_hip
 from .mixers import conv_silu
 
 # from this many (token, choice) pairs per expert on average the experts run on the dense GEMM's tiles (_grouped)
@@ -171,8 +171,9 @@ def moe_routes(ids, tables, experts: int, live=None) -> list:
 
 
 def moe_skips_rows(T: int, top: int, E: int, W: int, ffp: int) -> bool:
-    """Whether the experts' products of T bf16 rows may leave rows out (``moe_routes(live=)``): their results are zeros."""
-    return lib().moe_rows_ok(T, top, E, W, ffp) and not _grouped(T, T * top, E, W, ffp)
+    """Whether the experts' products of T bf16 rows may leave rows out (``moe_routes(live=)``): their results are zeros.  The reference
+    runs all rows."""
+    return not force_reference() and lib().moe_rows_ok(T, top, E, W, ffp) and not _grouped(T, T * top, E, W, ffp)
 
 
 def table_experts(h, ids, table, w_gate_up, w_down, top: int, route=None):

@@ -568,6 +568,19 @@ def test_reference_switch_follows_the_environment(monkeypatch):
     assert _ext.force_reference()
 
 
+def test_reference_switch_asks_no_library(monkeypatch):
+    """What chooses a kernel asks the library only where kernels run: with the switch on it need not be there."""
+    from llm_kubernetes_minikube_sharp4dev_amd import ops
+    from llm_kubernetes_minikube_sharp4dev_amd.ops import window
+
+    def absent():
+        raise RuntimeError("no library")
+
+    monkeypatch.setattr(window, "lib", absent)
+    monkeypatch.setenv("LK_FORCE_REFERENCE", "1")
+    assert not ops.moe_skips_rows(4, 2, 8, 256, 128)
+
+
 @pytest.mark.parametrize("lens,Hq,Hkv,two", [([159], 32, 8, 0), ([160], 32, 8, 1), ([100] * 8, 32, 8, 0), ([1024], 32, 8, 1), ([2048], 32, 8, 1), ([2049], 32, 8, 0),
                                              ([400] * 3, 32, 8, 0), ([600] * 2, 32, 8, 1), ([500] * 4, 32, 8, 0), ([1500], 32, 32, 1)])
 def test_prompt_attention_splits_keys_where_few_chains_are_long(lens, Hq, Hkv, two):
