@@ -355,9 +355,10 @@ class FusasunModel(nn.Module):
                     groups.setdefault((L.mlp.gate_up.shape[0], tuple(L.mlp.table.shape), L.mlp.down.shape[2]), []).append(i)
             T = ids.numel()
             for (experts, (_, top), ffp), at in groups.items():
-                # (one sequence, and so one state slot, per row)
+                # (one sequence, and so one state slot, per row; weights that lie elsewhere run on a kernel that knows nothing of left out rows)
                 skip = (meta.num_decode == T and meta.state_slots is not None and meta.state_slots.numel() == T and self.dtype == torch.bfloat16
-                        and ops.moe_skips_rows(T, top, experts, self.cfg.hidden, ffp))
+                        and ops.moe_skips_rows(T, top, experts, self.cfg.hidden, ffp)
+                        and not any((self.layers[i].mlp.gate_up.data_ptr() | self.layers[i].mlp.down.data_ptr()) % 16 for i in at))
                 for i, r in zip(at, ops.moe_routes(ids, [self.layers[i].mlp.table for i in at], experts, meta.state_slots if skip else None)):
                     out[i] = r
         return out

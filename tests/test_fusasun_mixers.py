@@ -408,6 +408,29 @@ def test_a_row_that_files_no_key_still_runs_its_experts(monkeypatch):
     assert torch.equal(got[live], want[live]) and not torch.equal(got[2], want[2])
 
 
+@pytest.mark.gpu
+def test_padding_rows_run_where_the_weights_are_not_aligned(monkeypatch):
+    """Weights off a 16-byte line take the general kernel, which writes every row: no row of a step is left as its memory was."""
+    att = {"heads": 4, "kv_heads": 2, "dim": 64, "vdim": 64, "scale": 0.125, "mask": {"size": 48, "pool": 16}, "rot": {"base": 10000.0, "dims": 64}}
+    cfg = FusasunConfig.from_json({"architecture": "Fusasun", "vocab": 61, "width": 256, "norm": {"eps": 1e-5}, "embedding": {"scale": 1.0}, "canon": {"taps": 4},
+                                   "layers": [{"type": "attention", "mixer": att, "mlp": {"kind": "moe", "expert": {"ff": 128}, "router": {"experts": 8, "top": 2}}}]})
+    m = build_decoder(cfg, device="cuda", dtype=torch.bfloat16, seed=2)
+    down = m.layers[0].mlp.down
+    down.data = torch.empty(down.numel() + 4, dtype=torch.bfloat16, device="cuda")[4:].view(down.shape).copy_(down)
+    ids = torch.tensor([7, 30, 0, 12], dtype=torch.int32, device="cuda")
+
+    def step():
+        meta = step_meta([(0, 1, [i], slot, True) for i, slot in enumerate([2, 0, -1, 1])], "cuda")
+        keep = [torch.full((8, 256), math.nan, dtype=torch.bfloat16, device="cuda") for _ in range(64)]
+        del keep   # (what the next allocations of the step's size start as)
+        with torch.inference_mode():
+            return m(ids, meta, m.make_caches(8, BS, 3)).float()
+
+    got = step()
+    monkeypatch.setattr(ops, "moe_skips_rows", lambda *a: False)
+    assert torch.equal(got, step())
+
+
 @pytest.mark.parametrize("device,dtype", ALL)
 @pytest.mark.parametrize("taps,W", [(1, 36), (3, 48), (4, 40), (8, 50)])
 def test_convolution_added_to_its_input_over_cuts(taps, W, device, dtype):
