@@ -26,7 +26,7 @@ SHAPES = [("QKV", 6144, 4096, False), ("O", 4096, 4096, False), ("gate_up+SwiGLU
 
 def main():
     ap = argparse.ArgumentParser()
-    ap.add_argument("--ms", default="64,128,192,256")
+    ap.add_argument("--ms", default="64,128")
     ap.add_argument("--rounds", type=int, default=7)
     ap.add_argument("--md", default=None)
     a = ap.parse_args()

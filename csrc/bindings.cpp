@@ -2670,8 +2670,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   });
   m.def("ws_set_variant", [](int64_t M, int64_t N, int64_t K, bool swiglu, int64_t v) {
     CHECK_RC(lk_wsgemm_set_variant((int)M, (int)N, (int)K, swiglu ? 1 : 0, (int)v), "ws_set_variant");
-  }, "weight-streaming GEMM kernel for this (M bucket, N, K, swiglu): 0 ring, 1 loader waves, -1 default",
+  }, "weight-streaming GEMM kernel for this (M bucket, N, K, swiglu): 0 ring, 1 loader waves (up to 128 rows), -1 default",
         py::arg("M"), py::arg("N"), py::arg("K"), py::arg("swiglu"), py::arg("variant"));
+  m.def("ws_variant", [](int64_t M, int64_t N, int64_t K, bool swiglu) { return lk_wsgemm_variant((int)M, (int)N, (int)K, swiglu ? 1 : 0); },
+        "the kernel that runs", py::arg("M"), py::arg("N"), py::arg("K"), py::arg("swiglu"));
   m.def("prefill_pairs", &lk_prefill_pairs, "", py::arg("ntiles"), py::arg("groups"), py::arg("threads"));
   m.def("prefill_order", &lk_prefill_order, "", py::arg("ntiles"), py::arg("seqs"), py::arg("rows"), py::arg("heads"), py::arg("D"));
   m.def("prefill_split_keys", &lk_prefill_split_keys, "", py::arg("groups"), py::arg("rows"), py::arg("seqs"), py::arg("cus"));

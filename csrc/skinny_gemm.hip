@@ -892,6 +892,7 @@ __global__ __launch_bounds__(256, BN == 64 ? 2 : 1) void ws_beside_kernel(const 
 // the loader waves keep the remaining LDS of W stages in flight.  Same walk, tile, K rotation and epilogue, so the same bits.  Up to 128 rows: it is
 // the faster one by up to 3 % where few workgroups of 128 columns leave CUs idle (120 x 4096 x 4096 in 4 parts of K 15.0 -> 14.7 us), and
 // beyond, two sets of fragments for six waves do not fit the registers (the one ring runs).
+constexpr int kWsLoaderRows = 128;
 constexpr int lw_nsx(int) { return 3; }
 constexpr int lw_nsw(int MT, int BN) {
   const int n = (163840 - lw_nsx(MT) * 16 * MT * 128) / (BN * 128);
@@ -979,7 +980,7 @@ int dispatch_ws(int MT, int BN, const bf16_t* x, long ldx, const bf16_t* w, int 
   if (ws_too_far(M, ldx, K)) return -1;
 #define LK_WS(mt, bn)                                                                                          \
   if (MT == mt && BN == bn) {                                                                                  \
-    if constexpr (mt <= 8) {                                                                                   \
+    if constexpr (16 * mt <= kWsLoaderRows) {                                                                  \
       if (variant == 1) {                                                                                      \
         launch_ws_lw<mt, bn, SWIGLU>(x, ldx, w, M, K, ks, S, n_tiles, I, out, ldo, part, part_ld, n_rows, st, tl); \
         return 0;                                                                                              \
@@ -1095,13 +1096,14 @@ void lk_wsgemm_plan(int M, int N, int K, int swiglu, int* bn_out, int* s_out) {
 
 // per-shape kernel variant of the weight-streaming GEMM: 0 = one LDS ring (wsgemm_kernel),
 // 1 = loader waves (wsgemm_lw_kernel); keyed by (row tile MT, N, K, swiglu), set by the decode
-// tuner's measurement (ops.tune_decode), default LK_WS_LOADER (0)
+// tuner's measurement (ops.tune_decode), default LK_WS_LOADER (0).  Past kWsLoaderRows there is the ring only, whatever was set.
 static std::mutex g_ws_var_mu;
 static std::map<long, int> g_ws_var;
 static long ws_var_key(int MT, int N, int K, int swiglu) {
   return (((long)MT * 1000003L + N) * 1000003L + K) * 2 + (swiglu ? 1 : 0);
 }
-static int ws_variant(int M, int N, int K, int swiglu) {
+int lk_wsgemm_variant(int M, int N, int K, int swiglu) {
+  if (M > kWsLoaderRows) return 0;
   static const int dflt = [] {
     const char* e = getenv("LK_WS_LOADER");
     return e ? (atoi(e) != 0) : 0;
@@ -1130,7 +1132,7 @@ int lk_wsgemm(const bf16_t* x, long ldx, const bf16_t* w, int M, int N, int K, i
   const int MT = ws_mt(M);
   const int ks = K / S;
   float* p = S > 1 ? part : nullptr;
-  const int var = ws_variant(M, N, K, swiglu);
+  const int var = lk_wsgemm_variant(M, N, K, swiglu);
   const int rc = swiglu ? dispatch_ws<true>(MT, BN, x, ldx, w, M, K, ks, S, n_tiles, I, out, ldo, p, N, st,
                                             1L << 40, var)
                         : dispatch_ws<false>(MT, BN, x, ldx, w, M, K, ks, S, n_tiles, I, out, ldo, p, N, st,
@@ -1221,7 +1223,7 @@ int lk_wsgemm_part(const bf16_t* x, long ldx, const bf16_t* w, int M, int N, int
     return -1;
   const int MT = ws_mt(M);
   const int rc = dispatch_ws<false>(MT, BN, x, ldx, w, M, K, K / S, S, N / BN, 0, nullptr, 0, part, N, st,
-                                    1L << 40, ws_variant(M, N, K, 0));
+                                    1L << 40, lk_wsgemm_variant(M, N, K, 0));
   LK_CHECK_LAUNCH();
   return rc;
 }
@@ -1254,7 +1256,7 @@ int lk_ws_rope_kv_fused(const bf16_t* x, long ldx, const bf16_t* w, int M, int K
   tl.neox = neox;
   tl.write_k_inplace = write_k_inplace;
   const int rc = dispatch_ws<false>(ws_mt(M), BN, x, ldx, w, M, K, K / S, S, N / BN, 0, nullptr, 0, part, N, st,
-                                    1L << 40, ws_variant(M, N, K, 0), tl);
+                                    1L << 40, lk_wsgemm_variant(M, N, K, 0), tl);
   LK_CHECK_LAUNCH();
   return rc;
 }
@@ -1277,7 +1279,7 @@ int lk_ws_rmsnorm_fused(const bf16_t* x, long ldx, const bf16_t* w, int M, int N
   tl.norm_w = norm_w;
   tl.eps = eps;
   const int rc = dispatch_ws<false>(ws_mt(M), BN, x, ldx, w, M, K, K / S, S, N / BN, 0, nullptr, 0, part, N, st,
-                                    1L << 40, ws_variant(M, N, K, 0), tl);
+                                    1L << 40, lk_wsgemm_variant(M, N, K, 0), tl);
   LK_CHECK_LAUNCH();
   return rc;
 }

@@ -861,7 +861,7 @@ def tune_decode(weights, ms: Sequence[int] = DECODE_TUNE_MS, iters: int = 3, col
     (`_ROWS_TABLE`: what `linear` chooses by).  The few-row rule's answer stands unless another arm is 5 %
     faster, so that near ties do not change from one start to the next.  Returns
     {(M, N, K, swiglu): {"ws" / "gemm": us}}, {(M, N, K, swiglu, "few", "rows"): {arm: us}} of all arms and,
-    per measured row tile, {(M, N, K, swiglu, "ws_variant"): {"ring" / "loader": us}}."""
+    per row tile that has two kernels (64 and 128 rows), {(M, N, K, swiglu, "ws_variant"): {"ring" / "loader": us}}."""
     import statistics
 
     L = lib()
@@ -904,11 +904,11 @@ def tune_decode(weights, ms: Sequence[int] = DECODE_TUNE_MS, iters: int = 3, col
                     ts[k].append(a.elapsed_time(b) * 1e3 / len(copies))
             return {k: statistics.median(v) for k, v in ts.items()}
 
-        # the weight-streaming kernel's variant per row tile (64 / 128 / 192 / 256 rows): one LDS
-        # ring vs loader waves (csrc/skinny_gemm.hip wsgemm_lw_kernel), measured at the tile's
-        # largest M, before the routing below times the ws arm with it
+        # the weight-streaming kernel's variant per row tile (64 / 128 rows; past those there is the
+        # ring only): one LDS ring vs loader waves (csrc/skinny_gemm.hip wsgemm_lw_kernel), measured
+        # at the tile's largest M, before the routing below times the ws arm with it
         if WS_VARIANT_TUNE and _decode_static_ok(N, K, swiglu):
-            for M in [m for m in (64, 128, 192, 256) if m in ms]:
+            for M in [m for m in (64, 128) if m in ms]:
                 x = torch.randn(M, K, device=w.device, dtype=torch.bfloat16)
                 fns = {}
                 for v in (0, 1):
