@@ -378,6 +378,8 @@ LM_HEAD_SKINNY_MAX_M = 16
 WS_LM_HEAD = os.environ.get("LK_WS_LM_HEAD", "0") == "1"
 WS_MAX_M = int(os.environ.get("LK_WS_MAX_M", "256"))
 WS_SWIGLU_MAX_M = 160
+# 256 rows of X and a tile's of W within 32-bit offsets (csrc/skinny_gemm.hip ws_too_far); beyond, the fragment-load kernel
+WS_MAX_K = 8_000_000
 
 
 # Measured per-shape choice between the weight-streaming kernel and the prefill GEMM for
@@ -528,7 +530,7 @@ def _decode_gemm_kind(x, w, swiglu: bool) -> Optional[str]:
             return None
     elif N % 128:
         return None
-    if M <= SKINNY_MAX_M:
+    if M <= SKINNY_MAX_M or (K > WS_MAX_K and M <= WS_MAX_M):
         return "skinny"
     if _DECODE_TABLE and M > LM_HEAD_SKINNY_MAX_M:
         b = _decode_bucket(M)
@@ -952,7 +954,7 @@ def tune_decode(weights, ms: Sequence[int] = DECODE_TUNE_MS, iters: int = 3, col
 
 
 def _decode_static_ok(N: int, K: int, swiglu: bool) -> bool:
-    if K % 256:
+    if K % 256 or K > WS_MAX_K:
         return False
     return (N % 2 == 0 and (N // 2) % 64 == 0) if swiglu else N % 128 == 0
 
@@ -1020,7 +1022,7 @@ BESIDE_MAX_M = 128
 
 def _beside_rule(M: int, N: int, I: int, K: int) -> int:
     """W rows per workgroup for N plain and I SwiGLU output columns in one launch; 0: two launches."""
-    if not 1 <= M <= BESIDE_MAX_M or K < 64 or K % 64:
+    if not 1 <= M <= BESIDE_MAX_M or not 64 <= K <= WS_MAX_K or K % 64:
         return 0
     cus = device_cus()
     if N % 64 == 0 and I % 32 == 0 and N > 0 and I > 0 and N // 64 + I // 32 <= cus:

@@ -1284,6 +1284,20 @@ def test_ws_rows_as_far_apart_as_offsets_hold(hip, variant):
         hip.ws_set_variant(M, N, K, False, -1)
 
 
+@pytest.mark.parametrize("K", [8_000_000, 8_388_608])
+def test_products_of_millions_of_columns(hip, K):
+    """256 rows that 32-bit offsets hold and that they do not: 0, 1 and -1 in X and W keep every partial sum a whole number below 2^24."""
+    g = torch.Generator(device=DEV).manual_seed(1)
+    M, N = 256, 128
+    x = torch.randint(-1, 2, (M, K), device=DEV, generator=g, dtype=torch.int8).to(torch.bfloat16)
+    w = torch.randint(-1, 2, (N, K), device=DEV, generator=g, dtype=torch.int8).to(torch.bfloat16)
+    assert ops._decode_gemm_kind(x, w, False) == ("ws" if K == 8_000_000 else "skinny")
+    want = torch.zeros(M, N, device=DEV, dtype=torch.float64)
+    for a in range(0, K, 1 << 20):
+        want += x[:, a:a + (1 << 20)].float() @ w[:, a:a + (1 << 20)].float().t()
+    assert torch.equal(ops.linear(x, w), want.to(torch.bfloat16))
+
+
 @pytest.mark.parametrize("N,nq,K", [(1, 1, 1), (5, 3, 8), (16, 16, 8), (17, 2, 5), (4097, 16, 8), (40000, 1, 3)])
 def test_knn_scan_orders_signs_and_ties(hip, N, nq, K):
     """The one-pass search's hits as ordered numbers: negative scores, zero rows (a zero of either sign is one score), equal rows in order
