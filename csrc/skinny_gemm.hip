@@ -1034,10 +1034,10 @@ static int launch_beside(const bf16_t* x, long ldx, int M, int K, const bf16_t* 
 
 int lk_ws_beside(const bf16_t* x, long ldx, int M, int K, const bf16_t* w1, int N1, bf16_t* out1, long ld1, const bf16_t* w2, int I,
                  bf16_t* out2, long ld2, int bn, hipStream_t st) {
-  if (M < 1 || M > 128 || K < 64 || K % 64 || N1 < bn || N1 % bn || I < bn / 2 || I % (bn / 2) || ws_too_far(M, ldx, K)) return -1;
+  if ((bn != 64 && bn != 128) || M < 1 || M > 128 || K < 64 || K % 64 || N1 < bn || N1 % bn || I < bn / 2 || I % (bn / 2) || ws_too_far(M, ldx, K))
+    return -1;
   if (bn == 64) return (M <= 64 ? launch_beside<4, 64> : launch_beside<8, 64>)(x, ldx, M, K, w1, N1, out1, ld1, w2, I, out2, ld2, st);
-  if (bn == 128) return (M <= 64 ? launch_beside<4, 128> : launch_beside<8, 128>)(x, ldx, M, K, w1, N1, out1, ld1, w2, I, out2, ld2, st);
-  return -1;
+  return (M <= 64 ? launch_beside<4, 128> : launch_beside<8, 128>)(x, ldx, M, K, w1, N1, out1, ld1, w2, I, out2, ld2, st);
 }
 
 // padded row tiles of the weight-streaming GEMM: 16-row MFMA tiles, 4 waves splitting M

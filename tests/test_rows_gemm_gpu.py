@@ -129,6 +129,15 @@ def test_two_products_beside(hip, M, N, I, K, bn):
         assert ((f.double() - want).abs() <= 2.0 ** -8 * (3 * want.abs() + 1.1 * (g * u).abs()) + 1e-5).all()
 
 
+@pytest.mark.parametrize("M,N,I,bn", [(4, 128, 128, 0), (4, 128, 128, -64), (4, 128, 128, 1), (4, 128, 128, 32), (4, 128, 128, 256), (129, 128, 128, 64), (4, 96, 128, 64),
+                                      (4, 128, 48, 64)])
+def test_two_products_beside_refuses(hip, M, N, I, bn):
+    """Tile widths that there are none of, none among them, and sizes that they do not divide: an error, not the end of the process."""
+    x, w, wgu = (torch.zeros(n, 64, device="cuda", dtype=torch.bfloat16) for n in (M, N, 2 * I))
+    with pytest.raises(RuntimeError, match="ws_beside"):
+        hip.ws_beside(x, w, wgu, bn)
+
+
 def test_two_products_beside_takes_what_apart_takes(hip):
     """ops.linear_beside returns what the two calls return, to the roundings of their sums' orders, or leaves the operands to them: rows and
     widths inside and outside the rule, an x of transposed memory, f32."""
