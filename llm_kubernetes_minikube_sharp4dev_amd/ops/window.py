@@ -49,7 +49,8 @@ def stream_gated_norm(x, y, g, g_bias, w_post, w_next, eps: float, out_dtype=tor
 def stream_gated_norm_conv(x, y, g, g_bias, w_post, w_next, eps: float, out_dtype, parts: int, conv_w, state, cu, slots, positions, max_len: int):
     """(h, hc): :func:`stream_gated_norm`'s rows h and their causal convolution ``conv_silu(h, ..., act=False)`` per sequence;
     one launch where every sequence has one row."""
-    if use_hip(x) and max_len == 1 and slots.numel() == x.shape[0] and y.dtype == out_dtype == state.dtype == torch.bfloat16:
+    if (use_hip(x) and max_len == 1 and cu.numel() - 1 == slots.numel() == x.shape[0]
+            and y.dtype == out_dtype == state.dtype == torch.bfloat16):
         both = lib().stream_gated_norm_conv(x, y, int(parts), g, g_bias, w_post, w_next, float(eps), conv_w, state, slots, positions)
         if both:
             return tuple(both)

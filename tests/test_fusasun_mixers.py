@@ -332,6 +332,21 @@ def test_gated_norm_with_the_next_convolution(W, parts, taps, T):
     assert ((hc.float() - want.float()).abs() <= want.float().abs() / 128 + 1e-6).all()
 
 
+@pytest.mark.gpu
+def test_rows_of_no_sequence_leave_their_slots_alone():
+    """Fewer sequences than rows and slots: the convolution's state changes for the sequences there are, as in its own launch."""
+    g = torch.Generator().manual_seed(4)
+    T, W, taps = 5, 64, 4
+    x, y, gate = rnd(g, T, W).float().cuda(), rnd(g, T, W).bfloat16().cuda(), rnd(g, T, W).bfloat16().cuda()
+    gb, wp, wn, cw = (rnd(g, *s).float().cuda() for s in ((W,), (W,), (W,), (W, taps)))
+    state = rnd(g, 7, taps - 1, W).bfloat16().cuda()
+    cu, slots, pos = (torch.tensor(v, dtype=torch.int32, device="cuda") for v in ([0, 1, 2, 3], [5, 0, 2, 4, 1], [3, 0, 1, 2, 5]))
+    s1, s2 = state.clone(), state.clone()
+    h, hc = ops.stream_gated_norm_conv(x, y, gate, gb, wp, wn, 1e-5, torch.bfloat16, 1, cw, s1, cu, slots, pos, 1)
+    want = ops.conv_silu(h, 0, W, cw, None, s2, cu, slots, pos, 1, act=False)
+    assert torch.equal(s1, s2) and torch.equal(hc[:3], want[:3]) and torch.equal(s1[[4, 1]], state[[4, 1]])
+
+
 @pytest.mark.parametrize("device,dtype", ALL)
 @pytest.mark.parametrize("W,ff,E,top,T", [(48, 20, 5, 2, 37), (36, 13, 1, 1, 5), (50, 24, 7, 3, 70), (256, 128, 8, 2, 130),
                                           (64, 40, 2, 2, 150), (72, 100, 3, 1, 333), (44, 12, 2, 2, 100), (64, 24, 2, 2, 300), (128, 128, 2, 1, 700), (192, 256, 3, 2, 600)])
