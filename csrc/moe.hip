@@ -541,11 +541,20 @@ int lk_moe_route(const int* ids, const int* live, const int* const* tables, int 
   return 0;
 }
 
-// Whether the gate of T rows runs beside the experts' first product: the few-row kernel for both, and so few rows that reading X again for
-// every 16 columns costs less than a launch (2,048 x 2,048 beside 16 experts of 2,048 x 2,816, both and the second product: 88 rows
-// 111.7 -> 109.8 us, 96 rows 112.9 -> 112.0)
+// 16-row tiles of an expert's pairs per walk where the gate runs beside; a workgroup of the gate takes one more of rows
+static int beside_tiles(long T, int top, int E) { return T * top / E <= 10 ? 1 : 2; }
+
+// Whether the gate of T rows runs beside the experts' first product: the few-row kernel for both, and the launch that it saves worth more than X
+// and W read again out of the L2s, X for every 16 columns and W for every tile of rows.  Those bytes come at 16 MB/us beside the experts' stream;
+// on its own the gate takes 2.7 us and its weight at 6.6 MB/us.  Over 456 products (width 512 - 7,168, gates of 256 columns to twice the
+// width, 4 - 64 experts of 512 - 14,336, 1 - 96 rows) 0.903 of the time apart, 0.2 % more than the better of both; all of them beside, 0.915.
+// Apart / beside, us, 8 / 40 / 80 rows: 2,048 x 2,048 with 16 experts of 2,816 37.9 / 60.5 / 72.1 -> 34.0 / 58.4 / 71.2, 4,096 x 4,096 with 16 of 1,536
+// 45.4 / 71.4 / 74.0 -> 43.1 / 74.7 / 81.4, 7,168 x 7,168 with 16 of 2,048 96.7 / 159.7 / 169.0 -> 98.2 / 184.4 / 204.7.
 int lk_moe_beside_ok(long T, int top, int E, int N, int K, int N2) {
-  return T >= 1 && T <= 96 && top >= 1 && E >= 1 && T * top <= 22L * E && K % 64 == 0 && N % 32 == 0 && N2 > 0 && N2 % 16 == 0 && (long)E * (N / 32) <= 1 << 30;
+  if (T < 1 || T > 96 || top < 1 || E < 1 || T * top > 22L * E || K < 1 || K % 64 || N < 1 || N % 32 || N2 < 1 || N2 % 16 || (long)E * (N / 32) > 1 << 30) return 0;
+  const int rows = beside_tiles(T, top, E) + 1;   // 16-row tiles of one workgroup
+  const double again = (double)(N2 / 16) * ((T + 16 * rows - 1) / (16 * rows)) * (rows + 1) * 16 * K * 2e-6;
+  return again / 16 + 0.5 < 2.7 + (double)N2 * K * 2e-6 / 6.6;
 }
 
 int lk_moe_gemm_beside(const void* x, long xs, const int* order, const int* seg, int E, int top, long T, const void* w, int N, int K,
@@ -553,8 +562,8 @@ int lk_moe_gemm_beside(const void* x, long xs, const int* order, const int* seg,
   const auto al = [](const void* p, int n) { return reinterpret_cast<uintptr_t>(p) % n == 0; };
   if (!lk_moe_beside_ok(T, top, E, N, K, N2) || xs % 8 || os % 4 || ldy % 4 || !al(x, 16) || !al(w, 16) || !al(w2, 16) || !al(out, 8) || !al(y2, 8)) return -1;
   const Beside p{(const bf16_t*)w2, (bf16_t*)y2, ldy, (int)T, N2, 0};
-  return T * top / E <= 10 ? launch_moe_beside<1>(x, xs, order, seg, E, top, w, N, K, out, os, p, st)
-                           : launch_moe_beside<2>(x, xs, order, seg, E, top, w, N, K, out, os, p, st);
+  return beside_tiles(T, top, E) == 1 ? launch_moe_beside<1>(x, xs, order, seg, E, top, w, N, K, out, os, p, st)
+                                      : launch_moe_beside<2>(x, xs, order, seg, E, top, w, N, K, out, os, p, st);
 }
 
 int lk_moe_gemm(const void* x, long xs, const int* order, const int* seg, int E, int top, long pairs, const void* w, int N, int K,

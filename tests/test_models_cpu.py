@@ -581,6 +581,17 @@ def test_reference_switch_asks_no_library(monkeypatch):
     assert not ops.moe_skips_rows(4, 2, 8, 256, 128)
 
 
+@pytest.mark.parametrize("T,W,N2,E,ff,top,beside", [(1, 2048, 2048, 16, 2816, 2, 1), (64, 2048, 2048, 16, 2816, 2, 1), (40, 4096, 4096, 16, 1536, 2, 0), (16, 4096, 4096, 16, 1536, 2, 1),
+                                                    (40, 7168, 7168, 16, 2048, 2, 0), (80, 2048, 4096, 16, 2816, 2, 0), (80, 1024, 1024, 16, 1408, 2, 1), (96, 2048, 256, 16, 2816, 2, 1),
+                                                    (97, 1024, 1024, 16, 1408, 2, 0), (0, 1024, 1024, 16, 1408, 2, 0), (8, 1000, 1024, 16, 1408, 2, 0), (8, 1024, 1000, 16, 1408, 2, 0)])
+def test_gate_beside_the_experts_by_its_bytes(T, W, N2, E, ff, top, beside):
+    from llm_kubernetes_minikube_sharp4dev_amd.ops import _ext
+
+    if not _ext.available():
+        pytest.skip("the kernel library is not built")
+    assert _ext.lib().moe_beside_ok(T, top, E, 2 * ff, W, N2) == bool(beside)
+
+
 @pytest.mark.parametrize("lens,Hq,Hkv,two", [([159], 32, 8, 0), ([160], 32, 8, 1), ([100] * 8, 32, 8, 0), ([1024], 32, 8, 1), ([2048], 32, 8, 1), ([2049], 32, 8, 0),
                                              ([400] * 3, 32, 8, 0), ([600] * 2, 32, 8, 1), ([500] * 4, 32, 8, 0), ([1500], 32, 32, 1)])
 def test_prompt_attention_splits_keys_where_few_chains_are_long(lens, Hq, Hkv, two):
