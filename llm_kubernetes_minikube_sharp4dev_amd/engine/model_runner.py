@@ -188,12 +188,14 @@ class ModelRunner:
         if tp is not None and tp.enabled and not getattr(tp, "simulated", False):
             import torch.distributed as dist
 
-            box = [(dict(ops._DECODE_TABLE), dict(ops._WS_VARIANTS), dict(ops._ROWS_TABLE)) if lead else None]
+            box = [(dict(ops._DECODE_TABLE), dict(ops._WS_VARIANTS), dict(ops._ROWS_TABLE), dict(ops._DECODE_US)) if lead else None]
             dist.broadcast_object_list(box, src=tp.ranks[0] if tp.ranks else 0, group=tp.ctrl or tp.group)
             ops._DECODE_TABLE.clear()
             ops._DECODE_TABLE.update(box[0][0])
             ops._ROWS_TABLE.clear()
             ops._ROWS_TABLE.update(box[0][2])
+            ops._DECODE_US.clear()
+            ops._DECODE_US.update(box[0][3])
             if not lead:
                 ops.apply_ws_variants(box[0][1])
         picks = {}

@@ -446,7 +446,12 @@ def _ws_cost(M: int, N: int, K: int, swiglu: bool) -> float:
     rounds = -(-(N // bn * parts) // 256)
     chain = 3.0 + rounds * (K / parts) / 64 * (0.0038 * bn + 0.0025 * 64 * -(-M // 64) - 0.16) + 6.3 * (rounds - 1)
     us = max(chain, 3.3 + N * K * 2 / 6.35e6) + (2.0 + 2.4e-6 * parts * M * N if parts > 1 else 0)
-    return us * (1.1 if M > 64 else 1.16 if M > 16 else 1.25)
+    return us * _few_scale(M)
+
+
+def _few_scale(M: int) -> float:
+    """How far the few-row kernel's estimate lies above its times."""
+    return 1.1 if M > 64 else 1.16 if M > 16 else 1.25
 
 
 def _rows_cost(M: int, N: int, K: int, epi: int, products: int = 1):
@@ -492,6 +497,20 @@ def _rows_rule(M: int, N: int, K: int, epi: int, products: int = 1) -> Optional[
 # What ``tune_decode`` measured of the few-row kernel for a plain or SwiGLU projection, {(M bucket, N, K, swiglu): wide, or None
 # where another kernel (``_DECODE_TABLE``) was faster}; the rule above holds for shapes and rows that were not measured.
 _ROWS_TABLE: dict = {}
+# The us of the kernel that those picks run, {(M bucket, N, K, swiglu): us}
+_DECODE_US: dict = {}
+
+
+def _alone_us(M: int, N: int, K: int, swiglu: bool):
+    """us of a plain or SwiGLU product as :func:`linear` runs it: what start-up measured, else the estimate; None without one."""
+    if M > LM_HEAD_SKINNY_MAX_M and (_decode_bucket(M), N, K, swiglu) in _DECODE_US:
+        return _DECODE_US[(_decode_bucket(M), N, K, swiglu)]
+    if GEMV and M <= GEMV_MAX_M and gemv_supported(M, N, K, 2 if swiglu else 0):
+        return 1.9 + 0.4 * M + N * K * 2 / 6.4e6
+    est = _rows_cost(M, N, K, int(swiglu))
+    if est is not None:
+        return min(est[0], est[2]) / _few_scale(M)
+    return _ws_cost(M, N, K, swiglu) / _few_scale(M) if _decode_static_ok(N, K, swiglu) else None
 
 
 def _rows_choice(M: int, N: int, K: int, epi: int, products: int = 1) -> Optional[int]:
@@ -943,12 +962,16 @@ def tune_decode(weights, ms: Sequence[int] = DECODE_TUNE_MS, iters: int = 3, col
             if len(arms) > 1:
                 _DECODE_TABLE[key] = min(arms, key=med.get)
                 out[key] = {k: round(med[k], 1) for k in arms}
+            run = min(arms, key=med.get) if arms else None
             if rows and arms:
                 best = min(med, key=med.get)
                 stay = next(iter(rows)) if est[0] < est[2] else min(arms, key=med.get)
                 pick = best if med[best] < 0.95 * med[stay] else stay
                 _ROWS_TABLE[key] = est[1] if pick in rows else None
+                run = pick
                 out[key + ("few", "rows")] = {k: round(v, 1) for k, v in med.items()}
+            if run is not None:
+                _DECODE_US[key] = med[run]
         del copies
     return out
 
@@ -1010,7 +1033,11 @@ def linear_pair(x1, w1, x2, w2):
 # the memory idle at its start and its end, and both of these once.  64 W rows per workgroup where all of them run in one round of the CUs
 # (two fit a CU's LDS), else 128 where those do: 64 re-read x twice as often, and past one round the CUs with two workgroups hold up the launch.
 # Beyond, each product fills the chip by itself and the launch gains nothing; at few rows 128 pay from two thirds of the CUs on (fewer take in
-# less than the memory gives).  Plain + SwiGLU apart -> together, us, weights cold, 1 / 4 / 16 / 64 / 128 rows:
+# less than the memory gives).  A workgroup walks the whole of K, which the launches apart cut into ranges: where that chain by itself is as long
+# as they are, few workgroups wait for it, and the products stay apart (1 / 128 rows: 384 + 2 x 512, K 8192 8.9 / 25.0 apart, 25.5 / 52.3
+# together; 2048 + 2 x 2048, K 2048 8.2 / 16.7, 9.5 / 17.0).  Over 1,172 products (N 64 - 16384, I 64 - 13824, K 256 - 8192, 1 - 128 rows) 0.851 of the
+# time apart, 8 of them slower by 3 % or more, 1.105 at most; without the chain in the rule 0.902, 230 and 2.9.
+# Plain + SwiGLU apart -> together, us, weights cold, 1 / 4 / 16 / 64 / 128 rows:
 #    3072 + 2 x 5632, K 2048   64: 13.3 / 14.4 / 15.2 / 21.4 / 32.0 -> 11.3 / 11.3 / 11.5 / 13.9 / 18.5
 #   10496 + 2 x 5632, K 2048  128: 18.2 / 19.2 / 20.3 / 27.6 / 42.7 -> 18.2 / 17.3 / 17.6 / 20.8 / 25.6   (with 64: 20.7 / 19.7 / 20.0 / 24.3 / 31.6)
 #    1536 + 2 x 2048, K 1024   64:  7.2 /  7.7 /  7.9 /  9.3 / 11.5 ->  6.2 /  6.3 /  6.4 /  8.0 / 10.5
@@ -1024,11 +1051,21 @@ def _beside_rule(M: int, N: int, I: int, K: int) -> int:
     """W rows per workgroup for N plain and I SwiGLU output columns in one launch; 0: two launches."""
     if not 1 <= M <= BESIDE_MAX_M or not 64 <= K <= WS_MAX_K or K % 64:
         return 0
-    cus = device_cus()
-    if N % 64 == 0 and I % 32 == 0 and N > 0 and I > 0 and N // 64 + I // 32 <= cus:
-        return 64
-    tiles = N // 128 + I // 64
-    return 128 if N % 128 == 0 and I % 64 == 0 and N > 0 and I > 0 and tiles <= cus and (M > 48 or tiles >= 0.65 * cus) else 0
+    if N < 1 or I < 1:
+        return 0
+    cus, tiles = device_cus(), N // 128 + I // 64
+    if N % 64 == 0 and I % 32 == 0 and N // 64 + I // 32 <= cus:
+        bn = 64
+    elif N % 128 == 0 and I % 64 == 0 and tiles <= cus and (M > 48 or tiles >= 0.65 * cus):
+        bn = 128
+    else:
+        return 0
+    # the chain of one workgroup: per 64 of K the tile's columns, the row tile and the rows in it
+    chain = 4.0 + K / 64 * ((0.14 if bn == 64 else 0.32) + 0.056 * (-(-M // 64) - 1) + 0.034 * -(-M // 16))
+    alone = _alone_us(M, N, K, False), _alone_us(M, 2 * I, K, True)
+    # (one or two rows stream at the matrix-vector kernel's rate, to which a chain has to leave room)
+    gemv = GEMV and M <= GEMV_MAX_M and gemv_supported(M, N, K, 0) and gemv_supported(M, 2 * I, K, 2)
+    return bn if None not in alone and chain < (0.82 if gemv else 1.0) * sum(alone) else 0
 
 
 def linear_beside(x, w, w_gate_up):

@@ -592,6 +592,25 @@ def test_gate_beside_the_experts_by_its_bytes(T, W, N2, E, ff, top, beside):
     assert _ext.lib().moe_beside_ok(T, top, E, 2 * ff, W, N2) == bool(beside)
 
 
+@pytest.mark.parametrize("M,N,I,K,bn", [(64, 3072, 5632, 2048, 64), (64, 10496, 5632, 2048, 128), (4, 3072, 5632, 2048, 64), (64, 4096, 8192, 4096, 128), (16, 4096, 8192, 4096, 0),
+                                       (1, 384, 512, 8192, 0), (64, 384, 512, 8192, 0), (128, 384, 512, 8192, 0), (128, 2048, 2048, 2048, 0), (1, 2048, 2048, 2048, 0),
+                                       (48, 2048, 2048, 2048, 64), (128, 128, 128, 2560, 0), (64, 3072, 512, 12288, 0), (129, 3072, 5632, 2048, 0), (64, 3072, 5632, 2000, 0),
+                                       (0, 3072, 5632, 2048, 0), (4, 0, 5632, 2048, 0)])
+def test_products_beside_by_their_chain(monkeypatch, M, N, I, K, bn):
+    """Long K on few workgroups stays apart; where start-up measured the products alone, that is what the chain is held against."""
+    from llm_kubernetes_minikube_sharp4dev_amd import ops
+
+    if not ops.available():
+        pytest.skip("the kernel library is not built")
+    monkeypatch.setattr(ops, "_DECODE_US", {})
+    monkeypatch.setattr(ops, "_CUS", 256)
+    assert ops._beside_rule(M, N, I, K) == bn
+    if bn and M > ops.LM_HEAD_SKINNY_MAX_M:
+        b = ops._decode_bucket(M)
+        ops._DECODE_US.update({(b, N, K, False): 0.5, (b, 2 * I, K, True): 0.5})
+        assert ops._beside_rule(M, N, I, K) == 0
+
+
 @pytest.mark.parametrize("lens,Hq,Hkv,two", [([159], 32, 8, 0), ([160], 32, 8, 1), ([100] * 8, 32, 8, 0), ([1024], 32, 8, 1), ([2048], 32, 8, 1), ([2049], 32, 8, 0),
                                              ([400] * 3, 32, 8, 0), ([600] * 2, 32, 8, 1), ([500] * 4, 32, 8, 0), ([1500], 32, 32, 1)])
 def test_prompt_attention_splits_keys_where_few_chains_are_long(lens, Hq, Hkv, two):
