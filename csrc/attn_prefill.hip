@@ -650,7 +650,7 @@ int lk_flash_prefill(const bf16_t* q, long qs, const bf16_t* k, const bf16_t* v,
     grid = dim3((unsigned)paired);
   }
   const bool pipe = causal && prefill_pipe();
-  if (pipe && paged && D >= 64 && NW == 4 && !part_o && lk_prefill_split_keys((long)ntiles * (Hq / WH), rows, seqs, cu_count())) {
+  if (pipe && paged && (D == 64 || D == 128) && NW == 4 && !part_o && lk_prefill_split_keys((long)ntiles * (Hq / WH), rows, seqs, cu_count())) {
 #define LS(DD, W) flash_prefill_kernel<DD, true, true, W, 4, true, 2><<<grid, 512, 0, st>>>(pr)
 #define LS_W(DD) if (WH == 4) LS(DD, 4); else if (WH == 2) LS(DD, 2); else LS(DD, 1)
     if (D == 128) { LS_W(128); }

@@ -290,6 +290,17 @@ def test_flash_prefill_two_sets_of_waves(hip, G, D, BS, q_lens, past):
     _close(y, y_ref, 0.02, 0.0, "flash prefill, two sets")
 
 
+@pytest.mark.parametrize("D", [96, 192, 256])
+@pytest.mark.parametrize("n", [100, 400])
+def test_flash_prefill_refuses_other_head_sizes(hip, D, n):
+    """Heads of 32, 64 and 128 have kernels; others raise, whatever the rows would choose."""
+    kc, vc, bt = _paged_setup(1, [n], 2, D, 16, seed=3)
+    q = torch.zeros(n, 8 * D, device=DEV, dtype=torch.bfloat16)
+    cu, cl, tile = (torch.tensor(v, dtype=torch.int32, device=DEV) for v in ([0, n], [n], [0]))
+    with pytest.raises(RuntimeError, match="flash_prefill"):
+        hip.flash_prefill(q, kc, vc, bt, cu, cl, tile, tile, 8, 2, D, D ** -0.5, True)
+
+
 @pytest.mark.parametrize("D", [32, 64, 128])
 def test_flash_encoder_dense(D):
     torch.manual_seed(9)
