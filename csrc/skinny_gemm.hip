@@ -1051,10 +1051,14 @@ void lk_wsgemm_plan(int M, int N, int K, int swiglu, int* bn_out, int* s_out) {
   // Rule fitted to the exhaustive (BN, S) sweep on MI355X (profiles/r1_ws_sweep.md):
   // one block per CU, so fill <= 256 CUs in ONE round; prefer BN = 128 (half the X
   // re-reads through L2) and split K only while every block keeps >= 16 stages;
-  // fall back to BN = 64 when BN = 128 leaves more than 30 % of the CUs idle, and no
-  // fewer than 64-column tiles do without a sum behind them (64 x 10496 x 2048, SwiGLU
-  // 11264 x 2048: 16.6 and 17.1 us in two parts of 128 columns, 13.7 and 13.6 whole).
-  (void)M;
+  // fall back to BN = 64 when BN = 128 leaves more than 30 % of the CUs idle and 64 fewer,
+  // and where as many 64-column tiles do without a sum behind them, of short K: the chain of
+  // the whole K has to stay below that of two parts and the sum (2.5 us).  Two parts of 128
+  // columns / 64 whole, us, 16 / 64 / 128 / 256 rows: SwiGLU 11008 x 2048 13.7 / 17.9 / 23.3 / 29.9
+  // -> 11.4 / 14.6 / 18.1 / 26.3, 10240 x 3072 17.3 / 22.2 / 29.2 / 35.9 -> 15.7 / 20.1 / 27.2 / 37.6, 8960 x 4096
+  // 20.8 / 25.2 / 31.9 / 39.0 -> 18.3 / 23.8 / 30.7 / 46.2, 9472 x 7168 29.6 / 36.9 / 47.2 / 57.6 -> 30.8 / 40.1 / 52.8 /
+  // 78.1, 11008 x 14336 55.6 / 68.7 / 85.2 / 102.8 -> 57.8 / 77.2 / 102.6 / 188; with parts on both sides
+  // (5120 x 11008, four of 128 / two of 64) 27.2 / 33.2 / 39.6 / 49.7 -> 30.4 / 37.1 / 49.8 / 66.5.
   auto plan = [&](int BN, int* S_out) -> double {
     const int cols = swiglu ? N / 2 : N, per = swiglu ? BN / 2 : BN;
     if (cols % per) return -1.0;
@@ -1067,8 +1071,9 @@ void lk_wsgemm_plan(int M, int N, int K, int swiglu, int* bn_out, int* s_out) {
   };
   int s128 = 1, s64 = 1;
   const double o128 = plan(128, &s128), o64 = plan(64, &s64);
+  const bool whole = o64 == o128 && s64 == 1 && s128 > 1 && (K <= 3072 || (K <= 4096 && M <= 128));
   double occ;
-  if (o128 >= 0.7 || (o128 >= 0 && (o64 < o128 || (o64 == o128 && s64 >= s128)))) {
+  if (o128 >= 0.7 || (o128 >= 0 && o64 <= o128 && !whole)) {
     *bn_out = 128;
     *s_out = s128;
     occ = o128;

@@ -439,8 +439,8 @@ def _ws_cost(M: int, N: int, K: int, swiglu: bool) -> float:
         return cols // per * s / (256 * -(-cols // per * s // 256)), s
 
     full, half, mid = plan(128), plan(64), (-1.0, 1) if swiglu else plan(96)
-    whole = full[0] >= 0.7 or half[0] < full[0] or (half[0] == full[0] and half[1] >= full[1])
-    (fill, parts), bn = (full, 128) if full[0] >= 0 and whole else (half, 64)
+    whole = half[0] == full[0] and half[1] == 1 < full[1] and (K <= 3072 or (K <= 4096 and M <= 128))   # 64 columns of all of K
+    (fill, parts), bn = (full, 128) if full[0] >= 0.7 or (0 <= full[0] and half[0] <= full[0] and not whole) else (half, 64)
     if mid[0] > fill + 1e-9:
         parts, bn = mid[1], 96
     rounds = -(-(N // bn * parts) // 256)

@@ -611,6 +611,18 @@ def test_products_beside_by_their_chain(monkeypatch, M, N, I, K, bn):
         assert ops._beside_rule(M, N, I, K) == 0
 
 
+@pytest.mark.parametrize("M,N,K,swiglu,plan", [(64, 10496, 2048, False, (64, 1)), (256, 11264, 2048, True, (64, 1)), (128, 8960, 4096, False, (64, 1)), (129, 8960, 4096, False, (128, 2)),
+                                              (16, 9472, 7168, False, (128, 2)), (16, 9472, 7168, True, (128, 2)), (192, 5120, 5120, False, (128, 4)), (8, 2560, 14336, False, (128, 8)),
+                                              (120, 4096, 14336, False, (128, 8)), (120, 28672, 4096, True, (128, 1)), (120, 6144, 4096, False, (96, 4))])
+def test_streaming_plans_by_k_and_rows(M, N, K, swiglu, plan):
+    """Whole K on 64-column tiles only where it is short; otherwise as many parts of 128 columns."""
+    from llm_kubernetes_minikube_sharp4dev_amd.ops import _ext
+
+    if not _ext.available():
+        pytest.skip("the kernel library is not built")
+    assert tuple(_ext.lib().ws_plan(M, N, K, swiglu)) == plan
+
+
 @pytest.mark.parametrize("lens,Hq,Hkv,two", [([159], 32, 8, 0), ([160], 32, 8, 1), ([100] * 8, 32, 8, 0), ([1024], 32, 8, 1), ([2048], 32, 8, 1), ([2049], 32, 8, 0),
                                              ([400] * 3, 32, 8, 0), ([600] * 2, 32, 8, 1), ([500] * 4, 32, 8, 0), ([1500], 32, 32, 1)])
 def test_prompt_attention_splits_keys_where_few_chains_are_long(lens, Hq, Hkv, two):
