@@ -806,7 +806,7 @@ LK_DEVICE void ws_store(const floatx4 (&acc)[MT / 2][BN / 32], int t, int s, int
   }
 }
 
-template <int MT, int BN, bool SWIGLU, bool TAIL, int PRO = 0>
+template <int MT, int BN, bool SWIGLU, bool TAIL, int PRO = 0, int DEPTH = ws_stages_pro(MT, BN, PRO)>
 __global__ __launch_bounds__(256, 1) void wsgemm_kernel(const bf16_t* __restrict__ X, long ldx,
                                                         const bf16_t* __restrict__ W, int M, int K, int ks,
                                                         int n_tiles, int swiglu_I, bf16_t* __restrict__ out,
@@ -814,7 +814,7 @@ __global__ __launch_bounds__(256, 1) void wsgemm_kernel(const bf16_t* __restrict
                                                         long n_rows, int rot_mul, WsTail tl, WsPro pr) {
   // n_rows: valid W rows (the last column tile may be partial: kNN over a corpus of
   // any size); rows past them read as zeros, stores are masked
-  constexpr int NS = ws_stages_pro(MT, BN, PRO);  // ring depth: as many stages as 160 KB of LDS holds
+  constexpr int NS = DEPTH;  // stages of the ring
   using Walk = WsWalk<MT, BN, SWIGLU, NS, NS, 0>;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
@@ -1289,6 +1289,19 @@ int lk_ws_rmsnorm_fused(const bf16_t* x, long ldx, const bf16_t* w, int M, int N
   return rc;
 }
 
+// Scores of a corpus: thousands of tiles with few K stages each, so what counts is that one workgroup's start and end hide behind another's:
+// a ring of DEPTH stages leaves room for two or three on a CU, and requests nothing that a short row does not have.  One ring of
+// 160 KB / this, us, 485,620 rows, 17 / 40 / 100 queries with their top 5: 128 columns 92.4 / 120.8 / 194.6 -> 67.7 / 100.8 / 174.7 (2 stages), 384 129.5 /
+// 159.7 / 243.5 -> 110.5 / 143.6 / 235.8 (3), 768 189.6 / 225.8 / 318.2 -> 174.3 / 212.4 / 314.4 (3); 20,011 rows level.  2 stages of longer rows
+// were ahead for a large corpus (17: 172.6) and behind for 1,000 and 20,011 rows (28.4 -> 31.6); past 128 queries there is no room for two.
+template <int MT, int DEPTH>
+static int launch_scores(const bf16_t* x, long ldx, const bf16_t* w, int M, int K, int tiles, float* out, long ldo, long N, hipStream_t st) {
+  constexpr int lds = DEPTH * (16 * MT + 128) * 128;
+  LK_SET_MAX_LDS((wsgemm_kernel<MT, 128, false, false, 0, DEPTH>), lds);
+  wsgemm_kernel<MT, 128, false, false, 0, DEPTH><<<tiles, 256, lds, st>>>(x, ldx, w, M, K, K, tiles, 0, nullptr, 0, out, ldo, N, 0, WsTail{}, WsPro{});
+  return 0;
+}
+
 // f32 X W^T for a W of any row count (kNN scores: X = queries, W = corpus rows):
 // out[M, N] with row stride ldo; one pass over W, no split-K.
 int lk_ws_scores_f32(const bf16_t* x, long ldx, const bf16_t* w, int M, long N, int K, float* out, long ldo,
@@ -1298,7 +1311,18 @@ int lk_ws_scores_f32(const bf16_t* x, long ldx, const bf16_t* w, int M, long N, 
   const long tiles = (N + BN - 1) / BN;
   if (tiles > (1L << 30)) return -1;
   const int MT = ws_mt(M);
-  const int rc = dispatch_ws<false>(MT, BN, x, ldx, w, M, K, K, 1, (int)tiles, 0, nullptr, 0, out, ldo, st, N);
+  if (ws_too_far(M, ldx, K)) return -1;
+  const int deep = K <= 192 ? 2 : MT <= 8 ? 3 : 0;
+  int rc = 0;
+  switch (MT + 100 * deep) {
+    case 204: rc = launch_scores<4, 2>(x, ldx, w, M, K, (int)tiles, out, ldo, N, st); break;
+    case 208: rc = launch_scores<8, 2>(x, ldx, w, M, K, (int)tiles, out, ldo, N, st); break;
+    case 212: rc = launch_scores<12, 2>(x, ldx, w, M, K, (int)tiles, out, ldo, N, st); break;
+    case 216: rc = launch_scores<16, 2>(x, ldx, w, M, K, (int)tiles, out, ldo, N, st); break;
+    case 304: rc = launch_scores<4, 3>(x, ldx, w, M, K, (int)tiles, out, ldo, N, st); break;
+    case 308: rc = launch_scores<8, 3>(x, ldx, w, M, K, (int)tiles, out, ldo, N, st); break;
+    default: rc = dispatch_ws<false>(MT, BN, x, ldx, w, M, K, K, 1, (int)tiles, 0, nullptr, 0, out, ldo, st, N);
+  }
   LK_CHECK_LAUNCH();
   return rc;
 }

@@ -1345,6 +1345,22 @@ def test_invalid_launch_raises(hip):
     _close(hip.rmsnorm(x, w, 1e-5, None, None), ref.rmsnorm(x, w, 1e-5, None), 0.05, 0.01, "after a failed launch")
 
 
+@pytest.mark.parametrize("D", [64, 128, 192, 256, 320, 768])
+@pytest.mark.parametrize("nq", [17, 64, 65, 128, 129, 193, 256])
+def test_knn_scores_of_many_queries(hip, nq, D):
+    """The two-pass search at every row tile and ring depth, one stage and fewer stages than the ring, a last column tile of 41 rows: dots of
+    small whole numbers are exact, and a score's division and norm round three times (f32)."""
+    g = torch.Generator().manual_seed(nq + D)
+    c, q = (torch.randint(-2, 3, (n, D), generator=g) for n in (1065, nq))
+    q[:, 0] += 4
+    corpus, queries = (t.to(torch.bfloat16).to(DEV) for t in (c, q))
+    cn, qn = (t.double().norm(dim=1) for t in (c, q))
+    s, i = (t.cpu() for t in hip.knn_topk(corpus, cn.float().to(DEV), queries, qn.float().to(DEV), 7))
+    want = (q.double() @ c.double().t()) / (qn[:, None] * cn[None] + 1e-9)
+    assert (s.double() - want.topk(7).values).abs().max() <= 2.0 ** -22
+    assert (want.gather(1, i.long()) - s.double()).abs().max() <= 2.0 ** -22 and all(len(set(r)) == 7 for r in i.tolist())
+
+
 @pytest.mark.parametrize("fused", [False, True])
 def test_knn_topk_config4_scale(hip, fused):
     """BASELINE config 4's index size: 1M runbook documents -> ~4.86M chunks x 768 (7.5 GB bf16,
