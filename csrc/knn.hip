@@ -328,16 +328,16 @@ __global__ __launch_bounds__(64 * kScanWaves, 1) void knn_scan_kernel(const bf16
   constexpr int D = SEG * 64, NS = kScanStages;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, g = lane >> 4;
-  short8 qf[2 * SEG];
-  {
+  // (a workgroup's waves are a grid apart: where there are fewer tiles than waves, every CU has as many)
+  const int tiles = (int)((N + 15) / 16), first = w * gridDim.x + blockIdx.x, step = gridDim.x * kScanWaves;
+  const int total = first < tiles ? ((tiles - 1 - first) / step + 1) * SEG : 0;  // this wave's stages
+  short8 qf[2 * SEG] = {};
+  if (total > 0) {   // (a wave without a tile asks for nothing: 16 queries are up to 32 KB that the other waves would wait behind)
     const bf16_t* q = queries + (long)min(r16, nq - 1) * D + 8 * g;
 #pragma unroll
     for (int k = 0; k < 2 * SEG; ++k) qf[k] = *reinterpret_cast<const short8*>(q + 32 * k);
   }
   const float qgiven = qnorm ? qnorm[min(r16, nq - 1)] : 0.f;
-  // (a workgroup's waves are a grid apart: where there are fewer tiles than waves, every CU has as many)
-  const int tiles = (int)((N + 15) / 16), first = w * gridDim.x + blockIdx.x, step = gridDim.x * kScanWaves;
-  const int total = first < tiles ? ((tiles - 1 - first) / step + 1) * SEG : 0;  // this wave's stages
   unsigned char* const ring = smem + w * NS * 2048;
   const int lrow = lane >> 3, lcol = rg_lane_col(lane);
   const bf16_t* src[2];  // this lane's part of the tile being requested
@@ -517,7 +517,8 @@ int lk_knn_merge(const float* cand_s, const int* cand_i, int nq, int ncand, int 
   return 0;
 }
 
-// workgroups of the one-pass scan (0: it does not take this shape): one per CU, a tile of 16 rows per wave at least
+// workgroups of the one-pass scan (0: it does not take this shape): one per four tiles of 16 rows, up to one per CU (up to 16,384 rows half of
+// the waves have no tile)
 int lk_knn_scan_blocks(long N, int D, int nq, int K) {
   if (N <= 0 || N >= 0x7fffffffL - 16 || nq < 1 || nq > kScanQ || K < 1 || K > kScanK) return 0;
   if (D != 128 && D != 256 && D != 384 && D != 512 && D != 768 && D != 1024) return 0;
