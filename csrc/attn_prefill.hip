@@ -611,7 +611,8 @@ static int cu_count() {
 // from about three key tiles in a chain on (us, plain / two sets: 100 rows 9.3 / 9.4, 130 9.7 / 9.7, 200 11.6 / 11.2, 8 x 100 9.7 / 10.5,
 // 2 x 500 20.6 / 18.6); up to two, which the plain kernel runs side by side, only where few long chains outlast the rest: 1,500 51.4 / 38.0,
 // 2,000 68 / 57, 2 x 600 24.3 / 20.9, 2 x 1,000 39.1 / 37.6, but 3 x 400 19.2 / 19.7, 4 x 500 25.4 / 28.6.  Past that it is the slower one
-// (3,000 105 / 117).  The keys before the rows are not known here; a short piece of a long prompt runs plain.
+// (3,000 105 / 117).  The rule sees rows and sequences and neither the longest chain nor the keys before the rows: a long prompt beside short
+// ones, and a short piece over many keys, run plain (as fast as they did), though the split would shorten their chain.
 int lk_prefill_split_keys(long groups, long rows, long seqs, int cus) {
   if (groups <= cus) return rows >= 160 * seqs;
   return groups <= 2 * cus && 4 * rows >= 7 * groups * seqs;

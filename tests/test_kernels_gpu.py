@@ -290,6 +290,60 @@ def test_flash_prefill_two_sets_of_waves(hip, G, D, BS, q_lens, past):
     _close(y, y_ref, 0.02, 0.0, "flash prefill, two sets")
 
 
+@pytest.mark.parametrize("G,D,BS", [(1, 64, 8), (4, 128, 8), (4, 64, 16)])
+@pytest.mark.parametrize("past", [1000, 2100])
+def test_flash_prefill_two_sets_over_long_block_tables(hip, G, D, BS, past):
+    """More cache blocks per sequence than a wave keeps at hand: the same bound as for short tables."""
+    torch.manual_seed(5)
+    Hkv, n = 2, 200
+    Hq, ctx = Hkv * G, past + n
+    assert -(-ctx // BS) > 128 or past == 1000
+    assert hip.prefill_split_keys(-(-n // ops.prefill_rows_per_tile(G, D)) * Hq // min(G, 4), n, 1, 256)
+    kc, vc, bt = _paged_setup(1, [ctx], Hkv, D, BS, seed=12)
+    q = torch.randn(n, Hq * D, device=DEV, dtype=torch.bfloat16)
+    cu, cl = (torch.tensor(v, dtype=torch.int32, device=DEV) for v in ([0, n], [ctx]))
+    y = ops.flash_prefill(q, kc, vc, cu, Hq, Hkv, D, D ** -0.5, True, block_tables=bt, ctx_lens=cl, q_lens_cpu=[n], ctx_lens_cpu=[ctx])
+    _close(y, ref.flash_prefill(q, kc, vc, bt, cu.cpu(), cl.cpu(), Hq, Hkv, D, D ** -0.5, True), 0.02, 0.0, "flash prefill, long tables")
+
+
+@pytest.mark.parametrize("at", [3, 70, 130, 200])
+@pytest.mark.parametrize("value", [math.inf, -math.inf, math.nan])
+def test_flash_prefill_two_sets_with_a_key_out_of_range(hip, at, value):
+    """An infinite or NaN score in one set's keys only: rows before it are the bits of the clean result, rows that see +inf or NaN are NaN,
+    rows that see -inf are those without the key."""
+    torch.manual_seed(6)
+    D, Hkv, G, n, BS = 128, 2, 4, 256, 16
+    Hq = Hkv * G
+    assert hip.prefill_split_keys(-(-n // ops.prefill_rows_per_tile(G, D)) * Hkv, n, 1, 256)
+    kc, vc, bt = _paged_setup(1, [n], Hkv, D, BS, seed=13)
+    q = torch.randn(n, Hq * D, device=DEV, dtype=torch.bfloat16)
+    cu, cl = (torch.tensor(v, dtype=torch.int32, device=DEV) for v in ([0, n], [n]))
+
+    def run():
+        return ops.flash_prefill(q, kc, vc, cu, Hq, Hkv, D, D ** -0.5, True, block_tables=bt, ctx_lens=cl, q_lens_cpu=[n], ctx_lens_cpu=[n]).view(n, Hq, D)
+
+    clean = run()
+    block = int(bt[0, at // BS])
+    kc[block, :, at % BS] = 0
+    kc[block, :, at % BS, 0] = value
+    got = run()
+    assert torch.equal(got[:at], clean[:at])
+    k = kc[bt[0].long()].transpose(1, 2).reshape(-1, Hkv, D)[:n].double().repeat_interleave(G, 1)
+    v = vc[bt[0].long()].transpose(1, 2).reshape(-1, Hkv, D)[:n].double().repeat_interleave(G, 1)
+    qd = q.view(n, Hq, D).double()
+    s = torch.stack([qd[:, h, :] @ k[:, h, :].t() for h in range(Hq)]) * D ** -0.5
+    if not math.isnan(value):   # (zero times infinity in the other columns of the product)
+        s[:, :, at] = qd[:, :, 0].t() * value
+    s.masked_fill_(torch.ones(n, n, dtype=torch.bool, device=DEV).triu(1), -math.inf)
+    lost = torch.isnan(s[:, :, at]) | (s[:, :, at] == math.inf)          # [Hq, n]
+    assert torch.isnan(got.transpose(0, 1)[lost]).all() and int(lost.sum()) >= (n - at) * Hq // 4
+    p = torch.softmax(s, -1)
+    want = torch.stack([p[h] @ v[:, h] for h in range(Hq)])
+    keep = ~lost
+    assert torch.isfinite(got.transpose(0, 1)[keep]).all()
+    _close(got.transpose(0, 1)[keep].contiguous(), want[keep].float(), 0.02, 0.0, "rows without the key")
+
+
 @pytest.mark.parametrize("D", [96, 192, 256])
 @pytest.mark.parametrize("n", [100, 400])
 def test_flash_prefill_refuses_other_head_sizes(hip, D, n):
