@@ -428,7 +428,8 @@ def _ws_cost(M: int, N: int, K: int, swiglu: bool) -> float:
     """us of the weight-streaming kernel: 3.8 ns for each of a workgroup's columns and 2.5 ns for each row per 64 of K, 6 us for each
     further round of workgroups, the weight at 6.4 TB/s at least, and the sum of its parts of K behind it: within 20 % of 510 products
     of 1 - 256 rows (32 shapes, 1024 - 128256 x 768 - 14336).  Given on the scale of the few-row kernel's estimate, which lies 10 % above its
-    own times, 16 % up to 64 rows and 25 % up to 16: the picks of the two take 0.3 / 0.9 / 1.3 % more than the better one."""
+    own times, 16 % up to 64 rows and 25 % up to 16: over 1,100 products (4 - 160 rows, N 256 - 23040, K 512 - 8192) the picks of the two
+    take 0.4 % more than the better one, 20 % at most, and 28 of them more than 5 %."""
     def plan(bn):   # (filled share of the CUs, parts of K), as csrc/skinny_gemm.hip lays a launch out
         cols, per = (N // 2, bn // 2) if swiglu else (N, bn)
         if cols % per:
@@ -445,7 +446,8 @@ def _ws_cost(M: int, N: int, K: int, swiglu: bool) -> float:
         parts, bn = mid[1], 96
     rounds = -(-(N // bn * parts) // 256)
     chain = 3.0 + rounds * (K / parts) / 64 * (0.0038 * bn + 0.0025 * 64 * -(-M // 64) - 0.16) + 6.3 * (rounds - 1)
-    us = max(chain, 3.3 + N * K * 2 / 6.35e6) + (2.0 + 2.4e-6 * parts * M * N if parts > 1 else 0)
+    # (of few workgroups the sum's launch is not hidden: 56 x 1280 x 6400 14.7 us, 11.9 without the last term, 12.3 on the few-row kernel)
+    us = max(chain, 3.3 + N * K * 2 / 6.35e6) + (2.0 + 2.4e-6 * parts * M * N + (N // bn * parts <= 128) if parts > 1 else 0)
     return us * _few_scale(M)
 
 

@@ -623,6 +623,18 @@ def test_streaming_plans_by_k_and_rows(M, N, K, swiglu, plan):
     assert tuple(_ext.lib().ws_plan(M, N, K, swiglu)) == plan
 
 
+@pytest.mark.parametrize("M,N,K,swiglu,few", [(56, 1280, 6400, True, True), (64, 1152, 5888, False, True), (56, 768, 7168, True, True), (64, 512, 5120, True, True),
+                                             (40, 3456, 6656, False, False), (80, 14080, 4352, True, False), (160, 6144, 6400, True, False), (120, 28672, 4096, True, False)])
+def test_narrow_products_of_long_k_take_the_few_row_kernel(monkeypatch, M, N, K, swiglu, few):
+    from llm_kubernetes_minikube_sharp4dev_amd import ops
+
+    if not ops.available():
+        pytest.skip("the kernel library is not built")
+    monkeypatch.setattr(ops, "_ROWS_TABLE", {})
+    monkeypatch.setattr(ops, "_ROWS_RULE", {})
+    assert (ops._rows_choice(M, N, K, int(swiglu)) is not None) == few
+
+
 @pytest.mark.parametrize("lens,Hq,Hkv,two", [([159], 32, 8, 0), ([160], 32, 8, 1), ([100] * 8, 32, 8, 0), ([1024], 32, 8, 1), ([2048], 32, 8, 1), ([2049], 32, 8, 0),
                                              ([400] * 3, 32, 8, 0), ([600] * 2, 32, 8, 1), ([500] * 4, 32, 8, 0), ([1500], 32, 32, 1)])
 def test_prompt_attention_splits_keys_where_few_chains_are_long(lens, Hq, Hkv, two):
