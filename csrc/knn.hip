@@ -293,7 +293,7 @@ __global__ __launch_bounds__(256) void knn_merge_kernel(const float* __restrict_
 // 16 rows x 128 bytes (row_ring.h), walk 16-row tiles round robin without a barrier, so 144 KB of corpus are on their way
 // per CU.  A lane sees 4 rows of one query per tile and keeps its 8 best in order (rows come in ascending order, so an
 // equal score never displaces: the stable order); 32 lists per query meet in LDS at the end.
-// What bounds it: the stream of rows at 485,620 x 768 (118 us, 6.3 TB/s, and 4 for the merge; 131 and 6 with a wait per number of stages
+// What bounds it: the stream of rows at 485,620 x 768 (116 us, 6.4 TB/s, and 4 for the merge; 131 and 6 with a wait per number of stages
 // left, row addresses per stage and reductions through the LDS unit); at 20,011 rows the chain of launch, code and first loads: of 10 us the
 // rows come between the third and the ninth, the lists and the merge of a workgroup take the rest.  Four waves per CU had a quarter of their
 // tiles behind another and met one LDS bank with all lists (13.2 us), and hits in two words compared in three steps (11.2); one question in
